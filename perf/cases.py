@@ -84,8 +84,9 @@ def draw(rng):
         high = rng.randint(140, 510)
         return dict(kind=kind, batch=log(2, 61), low=rng.randint(40, high), high=high, questions=False)
     if kind == "search":
-        return dict(kind=kind, queries=log(1, 300), rows=log(5_000, 250_007), dim=rng.choice((384, 768, 1024)),
-                    k=rng.choice((1, 3, 4, 4, 8, 10, 20, 40, 50)), metric=rng.choice(("cosine", "cosine", "ip", "l2")))
+        k = rng.choice((1, 3, 4, 4, 8, 10, 20, 40, 50))     # long candidate lists belong to the wide embedder's index
+        return dict(kind=kind, queries=log(1, 300), rows=log(5_000, 250_007), dim=1024 if k > 16 else rng.choice((384, 768, 1024)),
+                    k=k, metric=rng.choice(("cosine", "cosine", "ip", "l2")))
     if kind == "prefill":
         n, low, high = split(log(17, 14000), 6)
         return dict(kind=kind, batch=n, low=low, high=min(high, 8000))
