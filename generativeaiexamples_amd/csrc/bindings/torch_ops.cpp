@@ -372,9 +372,14 @@ void sim_topk(const Tensor& Q, const Tensor& X, const Tensor& bias, int64_t n_ro
   TORCH_CHECK(n_rows <= X.size(0) && n_rows <= bias.numel(), "sim_topk: n_rows exceeds storage");
   TORCH_CHECK(rows_per_wg % 128 == 0, "sim_topk: rows_per_wg must be a multiple of 128");
   const int cap = gai_topk_cap(k);
-  TORCH_CHECK(ws_v.numel() >= nwg * nq * cap && ws_i.numel() >= nwg * nq * cap, "sim_topk: workspace too small");
+  TORCH_CHECK(n_rows >= 1 && k >= 1 && k <= 64 && nwg * rows_per_wg >= n_rows, "sim_topk: rows or k out of range");
+  TORCH_CHECK(out_v.numel() >= nq * k && out_i.numel() >= nq * k && out_i.scalar_type() == at::kLong, "sim_topk: outputs");
+  const bool groups = ws_i.numel() == 0;  // the group form: ws_v holds a maximum per query and 16 rows
+  TORCH_CHECK(groups ? ws_v.numel() >= nq * ((n_rows + 15) / 16)
+                     : cap <= 8 && ws_v.numel() >= nwg * nq * cap && ws_i.numel() >= nwg * nq * cap,
+              "sim_topk: workspace too small");
   gai_sim_topk(Q.data_ptr(), X.data_ptr(), bias.data_ptr<float>(), nq, n_rows, D, k, ws_v.data_ptr<float>(),
-               ws_i.data_ptr<int>(), nwg, rows_per_wg, out_v.data_ptr<float>(), out_i.data_ptr<int64_t>(),
+               groups ? nullptr : ws_i.data_ptr<int>(), nwg, rows_per_wg, out_v.data_ptr<float>(), out_i.data_ptr<int64_t>(),
                cur_stream());
 }
 

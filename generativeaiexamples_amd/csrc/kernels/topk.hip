@@ -3,16 +3,15 @@
 // scores[q, x] = Q[q] . X[x] + bias[x]  with bias = 0 (inner product / cosine on
 // normalised vectors), -0.5*|x|^2 (L2 ranking) or -inf (deleted row), so one
 // kernel serves IP / cosine / L2 and tombstones. The [nq, N] score matrix is
-// never materialised:
-//   stage 1: a 512-thread workgroup keeps a tile of up to 64 queries in LDS
-//   (XOR-swizzled rows), each wave streams 16-row groups of X straight to VGPRs
-//   (X is read once from HBM per query tile: the index is bandwidth-bound),
-//   v_mfma_f32_16x16x32_bf16 produces the 16x(16*MT) score block, the block is
-//   transposed through a per-wave LDS scratch so each lane owns one query, and
-//   every lane keeps a sorted top-K list in registers (statically indexed
-//   insertion; after warm-up almost every candidate is rejected by one compare).
-//   The workgroup's lists are merged through LDS into one list per query.
-//   stage 2: one workgroup per query merges the per-workgroup lists.
+// never materialised. Both paths stream X once per 64-query tile through
+// v_mfma_f32_16x16x32_bf16 (sim_topk_stream):
+//   short lists (k <= 4, or k <= 8 for one query tile): every lane keeps a sorted list of its best rows in registers;
+//   the lists of a workgroup are merged in LDS and the workgroups' lists by sim_topk_stage2;
+//   else only the largest score of every 16-row group is kept (sim_topk_stream<.., 0, ..>), and one workgroup per
+//   query picks the k best groups - which hold the k best rows - and scores their rows again (sim_topk_select).
+// us, lists / groups (first form of k > 8: a 64-entry list per lane): 1M x 1024, k = 4: 1 query 353 / 417, 300 queries
+// 1280 / 1314; k = 8: 64 queries 422 / 510, 300 queries 1375 / 1314, 100k x 384 and 100 queries 140 / 56; k = 40: 1 query
+// 1M x 1024 (18263) / 454, 100 queries 100k x 384 (20901) / 67, 300 queries 250k x 1024 (144700) / 509.
 #include <algorithm>
 
 #include "gai_common.h"
@@ -51,166 +50,71 @@ struct TopK {
   }
 };
 
-// LDS layout: [Q image: NQ*D*2 bytes][score scratch: 8 waves * NQ * 17 floats]; the merge
-// buffer (64 lanes * K * 8 bytes) aliases the Q image after the main loop.
-template <int MT, int K>
-__global__ __launch_bounds__(512) void sim_topk_stage1(const bf16* __restrict__ Q, const bf16* __restrict__ X,
-                                                       const float* __restrict__ bias, int nq, int N, int D,
-                                                       int rows_per_wg, float* __restrict__ ws_v,
-                                                       int* __restrict__ ws_i) {
-  constexpr int NQ = 16 * MT;
-  constexpr int LPQ = 64 / NQ;  // lanes per query
-  constexpr int XPL = 16 / LPQ;  // x-columns per lane per group
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* qimg = smem;
-  float* scratch = reinterpret_cast<float*>(smem + (size_t)NQ * D * 2);
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int q0 = blockIdx.y * NQ;
-  const int ncols = D / 8;  // 16-B units per row
-
-  // stage the query tile (zero rows beyond nq)
-  for (int e = tid; e < NQ * ncols; e += 512) {
-    const int r = e / ncols, u = e % ncols;
-    bf16x8 v = (q0 + r < nq) ? load8(Q + (size_t)(q0 + r) * D + u * 8) : bf16x8{};
-    *reinterpret_cast<bf16x8*>(qimg + (size_t)r * D * 2 + ((u ^ (r & 15)) << 4)) = v;
-  }
-  __syncthreads();
-
-  const int my_q = lane % NQ, my_sub = lane / NQ;
-  TopK<K> tk;
-  tk.init();
-  float* scr = scratch + wid * NQ * 17;
-  const int wg_row0 = blockIdx.x * rows_per_wg;
-  const int wave_rows = rows_per_wg / 8;
-  const int r_begin = wg_row0 + wid * wave_rows;
-  const int r_end = min(N, r_begin + wave_rows);
-
-  for (int rb = r_begin; rb < r_end; rb += 16) {
-    const int xr = min(rb + (lane & 15), N - 1);
-    const bf16* xp = X + (size_t)xr * D + 8 * (lane >> 4);
-    f32x4 acc[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int t = 0; t < D / 32; ++t) {
-      const bf16x8 xf = load8(xp + 32 * t);
-      const int u = 4 * t + (lane >> 4);
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int qr = 16 * i + (lane & 15);
-        const bf16x8 qf = *reinterpret_cast<const bf16x8*>(qimg + (size_t)qr * D * 2 + ((u ^ (qr & 15)) << 4));
-        // D[row = query][col = x row]
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf, xf, acc[i], 0, 0, 0);
-      }
-    }
-    // transpose through LDS: scr[q][x]
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) scr[(16 * i + 4 * (lane >> 4) + r) * 17 + (lane & 15)] = acc[i][r];
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-#pragma unroll
-    for (int c = 0; c < XPL; ++c) {
-      const int xc = my_sub * XPL + c;
-      const int row = rb + xc;
-      if (row < r_end) tk.insert(scr[my_q * 17 + xc] + bias[row], row);
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  }
-
-  // merge: owner of query q = wave 0, lane q (sub 0). Buffer aliases the Q image.
-  __syncthreads();
-  float* mv = reinterpret_cast<float*>(qimg);
-  int* mi = reinterpret_cast<int*>(qimg + 64 * K * 4);
-#pragma unroll 1
-  for (int w = 0; w < 8; ++w) {
-    if (wid == w && !(w == 0 && my_sub == 0)) {
-#pragma unroll
-      for (int j = 0; j < K; ++j) {
-        mv[lane * K + j] = tk.v[j];
-        mi[lane * K + j] = tk.i[j];
-      }
-    }
-    __syncthreads();
-    if (wid == 0 && my_sub == 0) {
-#pragma unroll 1
-      for (int s = (w == 0 ? 1 : 0); s < LPQ; ++s) {
-        const int src = s * NQ + my_q;
-        for (int j = 0; j < K; ++j) {
-          const float v = mv[src * K + j];
-          if (!(v > tk.v[K - 1])) break;
-          tk.insert(v, mi[src * K + j]);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (wid == 0 && my_sub == 0 && q0 + my_q < nq) {
-    const size_t base = ((size_t)blockIdx.x * nq + q0 + my_q) * K;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-      ws_v[base + j] = tk.v[j];
-      ws_i[base + j] = tk.i[j];
-    }
-  }
-}
-
-
 // ------------------------------------------------------------------------------------------------
-// Streaming stage 1 for k <= 8 (the RAG path: top-4 of 1M-10M rows): one workgroup per CU-sized row
-// range, X streamed at HBM rate.
-//  * operands swapped (MFMA A = 16 X rows, B = 16 queries): lane l ends a 16-row group owning query
-//    l&15 (+16i) and rows 4(l>>4)..+3 - it inserts its 4 candidates straight from the accumulator, no LDS
-//    transpose, no wave barrier per group;
+// Streaming stage 1: X at HBM rate, one workgroup per row range (about one per CU) and 16 * MT queries.
+//  * MFMA A = 16 X rows, B = 16 queries: lane l ends a 16-row group owning query l&15 (+16i) and rows 4(l>>4)..+3, so
+//    the group is finished straight from the accumulator, no LDS transpose;
 //  * X fragments flow through a 16-deep register ring (16 KiB in flight per wave) that runs across
 //    group boundaries: the two 64-B halves of every 128-B X line are issued back to back;
-//  * per-lane register top-K lists; the 32 lists of a query (8 waves x 4 row-lanes) are merged in LDS
-//    once at the end.
+//  * K > 0: per-lane register top-K lists; the 32 lists of a query (8 waves x 4 row-lanes) are merged in LDS
+//    once at the end;
+//  * K = 0: the largest score of each group goes to gmax[query][group], 16-byte runs of four groups. Keeping 64 sorted
+//    entries per lane instead (the first form of k > 8) made nearly every insertion a divergent 64-step chain: 300
+//    queries x 250k rows x 1024, k = 40, took 144 ms; group maxima are 1/16 of the scores at 3 + 2/4 instructions each;
+//  * several query tiles read the same X rows: the tiles of one row range run one after the other on one XCD, so all but
+//    the first find the rows in its L2 (300 queries x 1M x 1024, k = 4: 1749 -> 1276 us).
 // ------------------------------------------------------------------------------------------------
 template <int MT, int K, int RING>
 __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ Q, const bf16* __restrict__ X,
                                                        const float* __restrict__ bias, int nq, int N, int D,
-                                                       int rows_per_wg, float* __restrict__ ws_v,
-                                                       int* __restrict__ ws_i) {
+                                                       int rows_per_wg, int qtiles, float* __restrict__ ws_v,
+                                                       int* __restrict__ ws_i, float* __restrict__ gmax, int ngr) {
   constexpr int NQ = 16 * MT;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* qimg = smem;
   float* bsm = reinterpret_cast<float*>(smem + (size_t)NQ * D * 2);  // this workgroup's bias rows
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int q0 = blockIdx.y * NQ;
+  const int seq = blockIdx.x >> 3;                              // position in its XCD's order
+  const int wgx = seq / qtiles * 8 + (blockIdx.x & 7);          // row range
+  const int q0 = seq % qtiles * NQ;                             // query tile
+  if (wgx * rows_per_wg >= N) return;                           // the grid is rounded up to whole XCD rounds
   const int ncols = D / 8;
-  const int wg_row0 = blockIdx.x * rows_per_wg;
+  const int sw = ncols & 15 ? (ncols & 7 ? 3 : 7) : 15;  // the XOR swizzle stays inside a row (D is a multiple of 32)
+  const int wg_row0 = wgx * rows_per_wg;
   for (int e = tid; e < NQ * ncols; e += 512) {
     const int r = e / ncols, u = e % ncols;
     bf16x8 v = (q0 + r < nq) ? load8(Q + (size_t)(q0 + r) * D + u * 8) : bf16x8{};
-    *reinterpret_cast<bf16x8*>(qimg + (size_t)r * D * 2 + ((u ^ (r & 15)) << 4)) = v;
+    *reinterpret_cast<bf16x8*>(qimg + (size_t)r * D * 2 + ((u ^ (r & sw)) << 4)) = v;
   }
   // bias through LDS: a global load inside the X stream would make every wait drain the ring
   for (int r = tid; r < rows_per_wg; r += 512) bsm[r] = wg_row0 + r < N ? bias[wg_row0 + r] : -INFINITY;
   __syncthreads();
 
-  TopK<K> tk[MT];
+  TopK<(K > 0 ? K : 1)> tk[MT];
+  float best[MT];  // K = 0: this lane's share of the last four groups' maxima
 #pragma unroll
-  for (int i = 0; i < MT; ++i) tk[i].init();
+  for (int i = 0; i < MT; ++i) {
+    tk[i].init();
+    best[i] = -INFINITY;
+  }
   const int wave_rows = rows_per_wg / 8;  // multiple of 16
   const int r_begin = wg_row0 + wid * wave_rows;
   const int r_end = min(N, r_begin + wave_rows);
   const int ngroups = r_end > r_begin ? (r_end - r_begin + 15) / 16 : 0;
   const int nk = D / 32;             // k-steps per 16-row group; RING divides it
   const int total = ngroups * nk;    // a multiple of RING: no tail guard inside the stream
-  // the stream position advances by RING k-steps per chunk; pointers are stepped, never divided
-  const bf16* const xlast = X + (size_t)(N - 1) * D + (D - 32) + 8 * (lane >> 4);
-  const bf16* xrow = X + (size_t)min(r_begin + (lane & 15), N - 1) * D + 8 * (lane >> 4);  // group g row
-  const size_t gstep = (size_t)16 * D;                                                    // next group
+  // the stream position advances by RING k-steps per chunk; pointers are stepped, and set once per group: rows past the
+  // wave's range (the prefetch's last chunk, a partial last group of the index) re-read the index's last row
+  int prow = r_begin + (lane & 15);
+  auto row_ptr = [&]() { return X + (size_t)(prow < r_end ? prow : N - 1) * D + 8 * (lane >> 4); };
   int pf_t = 0;                  // k-step of the prefetch pointer within its group
-  const bf16* pf = xrow;         // prefetch pointer (k-step j0 + RING)
+  const bf16* pf = row_ptr();    // prefetch pointer (k-step j0 + RING)
   auto advance_pf = [&]() {      // RING k-steps ahead
     pf_t += RING;
     if (pf_t == nk) {
       pf_t = 0;
-      pf += gstep - (size_t)32 * (nk - RING);
+      prow += 16;
+      pf = row_ptr();
     } else {
       pf += 32 * RING;
     }
@@ -224,15 +128,13 @@ __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ 
   for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   int g = 0, t0 = 0;
   for (int j0 = 0; j0 < total; j0 += RING) {
-    // past the stream's end the prefetch re-reads the last row (clamped, harmless)
-    const bf16* p = j0 + RING < total ? pf : xlast - 32 * (RING - 1);
     // query fragments one k-step ahead (LDS latency hides under the previous step's MFMAs)
     auto rdq = [&](bf16x8* qf, int t) {
       const int uu = 4 * t + (lane >> 4);
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
         const int qr = 16 * i + (lane & 15);
-        qf[i] = *reinterpret_cast<const bf16x8*>(qimg + (size_t)qr * D * 2 + ((uu ^ (qr & 15)) << 4));
+        qf[i] = *reinterpret_cast<const bf16x8*>(qimg + (size_t)qr * D * 2 + ((uu ^ (qr & sw)) << 4));
       }
     };
     bf16x8 qa[MT], qb[MT];
@@ -245,19 +147,41 @@ __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ 
 #pragma unroll
       for (int i = 0; i < MT; ++i)
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[u], qc[i], acc[i], 0, 0, 0);  // D[x row][query]
-      ring[u] = load8(p + 32 * u);  // consumed first, then refilled: the slot keeps its registers
+      ring[u] = load8(pf + 32 * u);  // consumed first, then refilled: the slot keeps its registers
     }
     advance_pf();
     t0 += RING;
     if (t0 == nk) {  // a 16-row group is complete: 4 candidate rows per lane and query tile
       const int rl = r_begin - wg_row0 + 16 * g + 4 * (lane >> 4);
       const f32x4 bv = *reinterpret_cast<const f32x4*>(bsm + rl);
+      if constexpr (K > 0) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = wg_row0 + rl + r;
-        if (row < r_end) {
+        for (int r = 0; r < 4; ++r) {
+          const int row = wg_row0 + rl + r;
+          if (row < r_end) {
 #pragma unroll
-          for (int i = 0; i < MT; ++i) tk[i].insert(acc[i][r] + bv[r], row);
+            for (int i = 0; i < MT; ++i) tk[i].insert(acc[i][r] + bv[r], row);
+          }
+        }
+      } else {  // rows past N have bias -inf; fmaxf passes NaN scores over
+        const int gr = r_begin / 16 + g;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          float m = fmaxf(fmaxf(fmaxf(-INFINITY, acc[i][0] + bv[0]), acc[i][1] + bv[1]),
+                          fmaxf(fmaxf(-INFINITY, acc[i][2] + bv[2]), acc[i][3] + bv[3]));
+          m = fmaxf(m, __shfl_xor(m, 16, 64));
+          m = fmaxf(m, __shfl_xor(m, 32, 64));
+          if ((lane >> 4) == (gr & 3)) best[i] = m;
+        }
+        if ((gr & 3) == 3 || g + 1 == ngroups) {  // this lane's group: the one of the last four with its number
+          const int mine = (gr & ~3) + (lane >> 4);
+          if (mine >= r_begin / 16 && mine <= gr) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+              const int q = q0 + 16 * i + (lane & 15);
+              if (q < nq) gmax[(size_t)q * ngr + mine] = best[i];
+            }
+          }
         }
       }
 #pragma unroll
@@ -267,37 +191,167 @@ __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ 
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (K > 0) {
+    // merge the 32 lists of every query (list = 4 * wave + row-lane group) in LDS (aliases the Q image)
+    __syncthreads();
+    float* mv = reinterpret_cast<float*>(smem);
+    int* mi = reinterpret_cast<int*>(smem + (size_t)NQ * 32 * K * 4);
+    const int list = wid * 4 + (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int q = 16 * i + (lane & 15);
+#pragma unroll
+      for (int jj = 0; jj < K; ++jj) {
+        mv[(q * 32 + list) * K + jj] = tk[i].v[jj];
+        mi[(q * 32 + list) * K + jj] = tk[i].i[jj];
+      }
+    }
+    __syncthreads();
+    if (tid < NQ && q0 + tid < nq) {
+      TopK<K> m;
+      m.init();
+      for (int l = 0; l < 32; ++l)
+        for (int jj = 0; jj < K; ++jj) {
+          const float v = mv[(tid * 32 + l) * K + jj];
+          if (!(v > m.v[K - 1])) break;
+          m.insert(v, mi[(tid * 32 + l) * K + jj]);
+        }
+      const size_t base = ((size_t)wgx * nq + q0 + tid) * K;
+#pragma unroll
+      for (int jj = 0; jj < K; ++jj) {
+        ws_v[base + jj] = m.v[jj];
+        ws_i[base + jj] = m.i[jj];
+      }
+    }
+  }
+}
 
-  // merge the 32 lists of every query (list = 4 * wave + row-lane group) in LDS (aliases the Q image)
+// ------------------------------------------------------------------------------------------------
+// k > 8, second pass: one workgroup per query. A key is (score, lowest row first) as one unsigned number, 0 = none.
+// The k groups with the largest maxima hold the k best rows: a row of another group has at least k rows before it, the
+// maxima of those groups. The same argument picks the groups: thread t's strided maximum over the group maxima, the k
+// best of those 1024 threads, and of their entries the k best. The rows of the k groups (<= 1024) are scored again with
+// the stream's own instruction order and sorted. Bound by latency: 250 KB of maxima at 1M rows, k x 32 KB of X at
+// D = 1024, three 45-step selections across lanes; 300 queries run side by side on the chip.
+// ------------------------------------------------------------------------------------------------
+typedef unsigned long long u64;
+
+__device__ __forceinline__ u64 make_key(float v, int id) {
+  if (!(v > -INFINITY)) return 0;  // deleted, absent or NaN
+  const uint32_t u = __float_as_uint(v == 0.f ? 0.f : v);
+  return ((u64)(u & 0x80000000u ? ~u : u | 0x80000000u) << 32) | (uint32_t)~id;
+}
+__device__ __forceinline__ int key_id(u64 k) { return (int)~(uint32_t)k; }
+__device__ __forceinline__ float key_value(u64 k) {
+  const uint32_t u = (uint32_t)(k >> 32);
+  return __uint_as_float(u & 0x80000000u ? u & 0x7fffffffu : ~u);
+}
+
+// lanes' keys -> descending over the lanes (bitonic; `first` = the smallest merge left to do)
+__device__ __forceinline__ u64 wave_sort(u64 x, int first = 2) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int size = 2; size <= 64; size <<= 1) {
+    if (size < first) continue;
+#pragma unroll
+    for (int d = size >> 1; d > 0; d >>= 1) {
+      const u64 y = __shfl_xor(x, d, 64);
+      const bool high = ((lane & size) == 0) == ((lane & d) == 0);  // this lane keeps the larger key
+      x = (x > y) == high ? x : y;
+    }
+  }
+  return x;
+}
+
+// The 64 largest of 1024 threads' keys (distinct or 0), descending, in list[0..63]; buf: 1024 keys. Each wave sorts its
+// own, then pairs of waves merge: the elementwise maximum of one list and the other reversed holds the 64 largest.
+__device__ __forceinline__ void top64(u64 x, u64* buf, u64* list) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  x = wave_sort(x);
+  for (int half = 8; half > 0; half >>= 1) {
+    __syncthreads();
+    if (wid >= half && wid < 2 * half) buf[tid] = x;
+    __syncthreads();
+    if (wid < half) {
+      const u64 y = buf[(wid + half) * 64 + 63 - lane];
+      x = wave_sort(x > y ? x : y, 64);
+    }
+  }
+  if (wid == 0) list[lane] = x;
   __syncthreads();
-  float* mv = reinterpret_cast<float*>(smem);
-  int* mi = reinterpret_cast<int*>(smem + (size_t)NQ * 32 * K * 4);
-  const int list = wid * 4 + (lane >> 4);
+}
+
+__global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__ Q, const bf16* __restrict__ X,
+                                                        const float* __restrict__ bias, const float* __restrict__ gmax,
+                                                        int ngr, int N, int D, int k, float* __restrict__ out_v,
+                                                        int64_t* __restrict__ out_i) {
+  __shared__ u64 buf[1024], cand[1024], list[64];
+  __shared__ int pick[64], cnt;
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const float* gm = gmax + (size_t)q * ngr;
+  u64 m = 0;
+  for (int i = tid; i < ngr; i += 1024) {
+    const u64 x = make_key(gm[i], i);
+    m = x > m ? x : m;
+  }
+  top64(m, buf, list);
+  if (ngr > 1024) {
+    if (tid < k) pick[tid] = list[tid] ? key_id(list[tid]) & 1023 : -1;
+    if (tid == 0) cnt = 0;
+    u64 bar = list[k - 1];  // the k-th best thread's maximum: nothing below it can be among the k best groups
+    __syncthreads();
+    const int per = (ngr + 1023) / 1024, all = k * per;
+    for (int base = 0; base < all; base += 960) {
+      const int e = base + tid;
+      if (tid < 960 && e < all) {
+        const int c = pick[e / per], i = c + 1024 * (e % per);
+        if (c >= 0 && i < ngr) {
+          const u64 x = make_key(gm[i], i);
+          if (x && x >= bar) cand[atomicAdd(&cnt, 1)] = x;  // <= 64 held + 960 of this round
+        }
+      }
+      __syncthreads();
+      const int n = cnt;
+      __syncthreads();  // every thread has read it before the next round adds to it
+      if (n > 64 || base + 960 >= all) {  // keep the k best
+        top64(tid < n ? cand[tid] : 0, buf, list);
+        if (tid < k) cand[tid] = list[tid];
+        if (tid == 0) cnt = n < k ? n : k;
+        if (n >= k) bar = list[k - 1];
+        __syncthreads();
+      }
+    }
+  }
+  if (tid < k) pick[tid] = list[tid] ? key_id(list[tid]) : -1;
+  cand[tid] = 0;
+  __syncthreads();
+  const bf16* qp = Q + (size_t)q * D + 8 * (lane >> 4);  // every column of the product is this query
+  auto rows = [&](int j) { return X + (size_t)min(16 * max(pick[min(j, k - 1)], 0) + (lane & 15), N - 1) * D + 8 * (lane >> 4); };
+  for (int j = wid; j < k; j += 32) {  // two groups a wave
+    const bf16 *xa = rows(j), *xb = rows(j + 16);
+    f32x4 acc[2] = {};
+#pragma unroll 8
+    for (int t = 0; t < D / 32; ++t) {
+      const bf16x8 qf = load8(qp + 32 * t);
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), qf, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xb + 32 * t), qf, acc[1], 0, 0, 0);
+    }
+    const int r = lane & 15;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int q = 16 * i + (lane & 15);
-#pragma unroll
-    for (int jj = 0; jj < K; ++jj) {
-      mv[(q * 32 + list) * K + jj] = tk[i].v[jj];
-      mi[(q * 32 + list) * K + jj] = tk[i].i[jj];
+    for (int h = 0; h < 2; ++h) {
+      const int jj = j + 16 * h;
+      if (jj >= k || pick[jj] < 0 || r >= 4) continue;
+      const int row = 16 * pick[jj] + 4 * (lane >> 4) + r;
+      const float v = r == 0 ? acc[h][0] : r == 1 ? acc[h][1] : r == 2 ? acc[h][2] : acc[h][3];
+      if (row < N) cand[16 * jj + 4 * (lane >> 4) + r] = make_key(v + bias[row], row);
     }
   }
   __syncthreads();
-  if (tid < NQ && q0 + tid < nq) {
-    TopK<K> m;
-    m.init();
-    for (int l = 0; l < 32; ++l)
-      for (int jj = 0; jj < K; ++jj) {
-        const float v = mv[(tid * 32 + l) * K + jj];
-        if (!(v > m.v[K - 1])) break;
-        m.insert(v, mi[(tid * 32 + l) * K + jj]);
-      }
-    const size_t base = ((size_t)blockIdx.x * nq + q0 + tid) * K;
-#pragma unroll
-    for (int jj = 0; jj < K; ++jj) {
-      ws_v[base + jj] = m.v[jj];
-      ws_i[base + jj] = m.i[jj];
-    }
+  top64(cand[tid], buf, list);
+  if (tid < k) {
+    const u64 x = list[tid];
+    out_v[(size_t)q * k + tid] = x ? key_value(x) : -INFINITY;
+    out_i[(size_t)q * k + tid] = x ? key_id(x) : -1;
   }
 }
 
@@ -354,75 +408,58 @@ void set_max_lds(F* f, int bytes) {
   hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
-template <int MT, int K>
-void run_topk(const void* Q, const void* X, const float* bias, int nq, int N, int D, int k, float* ws_v, int* ws_i,
-              int nwg, int rows_per_wg, float* out_v, int64_t* out_i, hipStream_t st) {
-  constexpr int NQ = 16 * MT;
-  const size_t lds = (size_t)NQ * D * 2 + (size_t)8 * NQ * 17 * 4;
-  auto k1 = sim_topk_stage1<MT, K>;
-  static bool once = false;
-  if (!once) {
-    set_max_lds(k1, 160 * 1024);
-    once = true;
-  }
-  const int qtiles = (nq + NQ - 1) / NQ;
-  k1<<<dim3(nwg, qtiles), 512, lds, st>>>((const bf16*)Q, (const bf16*)X, bias, nq, N, D, rows_per_wg, ws_v, ws_i);
-  GAI_LAUNCH_CHECK();
-  sim_topk_stage2<K><<<nq, 256, 0, st>>>(ws_v, ws_i, nwg, nq, k, out_v, out_i);
-  GAI_LAUNCH_CHECK();
-}
+struct TopkArgs {
+  const void *Q, *X;
+  const float* bias;
+  int nq, N, D, k, nwg, rows_per_wg;
+  float* ws_v;
+  int* ws_i;
+  float* out_v;
+  int64_t* out_i;
+  hipStream_t st;
+};
 
 template <int MT, int K, int RING>
-void run_stream_r(const void* Q, const void* X, const float* bias, int nq, int N, int D, int k, float* ws_v,
-                  int* ws_i, int nwg, int rows_per_wg, float* out_v, int64_t* out_i, hipStream_t st) {
+void run_stream_r(const TopkArgs& a) {
   constexpr int NQ = 16 * MT;
-  const size_t lds = std::max((size_t)NQ * D * 2 + (size_t)rows_per_wg * 4, (size_t)NQ * 32 * K * 8);
+  const size_t lds = std::max((size_t)NQ * a.D * 2 + (size_t)a.rows_per_wg * 4, (size_t)NQ * 32 * K * 8);
   auto k1 = sim_topk_stream<MT, K, RING>;
   static bool once = false;
   if (!once) {
     set_max_lds(k1, 160 * 1024);
     once = true;
   }
-  const int qtiles = (nq + NQ - 1) / NQ;
-  k1<<<dim3(nwg, qtiles), 512, lds, st>>>((const bf16*)Q, (const bf16*)X, bias, nq, N, D, rows_per_wg, ws_v, ws_i);
+  const int qtiles = (a.nq + NQ - 1) / NQ, ngr = (a.N + 15) / 16;
+  k1<<<(a.nwg + 7) / 8 * 8 * qtiles, 512, lds, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.nq, a.N, a.D, a.rows_per_wg, qtiles,
+                                         a.ws_v, a.ws_i, a.ws_v, ngr);
   GAI_LAUNCH_CHECK();
-  sim_topk_stage2<K><<<nq, 256, 0, st>>>(ws_v, ws_i, nwg, nq, k, out_v, out_i);
+  if constexpr (K > 0)
+    sim_topk_stage2<K><<<a.nq, 256, 0, a.st>>>(a.ws_v, a.ws_i, a.nwg, a.nq, a.k, a.out_v, a.out_i);
+  else
+    sim_topk_select<<<a.nq, 1024, 0, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, ngr, a.N, a.D, a.k, a.out_v,
+                                             a.out_i);
   GAI_LAUNCH_CHECK();
 }
 
 template <int MT, int K>
-void run_stream(const void* Q, const void* X, const float* bias, int nq, int N, int D, int k, float* ws_v, int* ws_i,
-                int nwg, int rows_per_wg, float* out_v, int64_t* out_i, hipStream_t st) {
-  const int nk = D / 32;
-  if (nk % 16 == 0) return run_stream_r<MT, K, 16>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-  if (nk % 8 == 0) return run_stream_r<MT, K, 8>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-  if (nk % 4 == 0) return run_stream_r<MT, K, 4>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-  return run_stream_r<MT, K, 1>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
+void run_stream(const TopkArgs& a) {
+  const int nk = a.D / 32;
+  // several query tiles: X comes from L2 for most of them, half the ring is enough (300 queries x 1M x 1024: 1355 -> 1314 us)
+  if constexpr (K == 0 && MT == 4)
+    if (a.nq > 64 && nk % 8 == 0) return run_stream_r<MT, K, 8>(a);
+  if (nk % 16 == 0) return run_stream_r<MT, K, 16>(a);
+  if (nk % 8 == 0) return run_stream_r<MT, K, 8>(a);
+  if (nk % 4 == 0) return run_stream_r<MT, K, 4>(a);
+  return run_stream_r<MT, K, 1>(a);
 }
 
 template <int K>
-void run_topk_k(const void* Q, const void* X, const float* bias, int nq, int N, int D, int k, float* ws_v, int* ws_i,
-                int nwg, int rows_per_wg, float* out_v, int64_t* out_i, hipStream_t st) {
-  if constexpr (K <= 8) {
-    // streaming kernel (host sizes rows_per_wg as a multiple of 128 for it)
-    if (rows_per_wg % 128 == 0 && rows_per_wg <= 8192) {
-      auto fits = [&](int nq_tile) { return (size_t)nq_tile * D * 2 + (size_t)rows_per_wg * 4 <= 160 * 1024; };
-      if (nq > 32 && fits(64))
-        return run_stream<4, K>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-      if (nq > 16 && fits(32))
-        return run_stream<2, K>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-      if (fits(16))
-        return run_stream<1, K>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-    }
-  }
-  // largest query tile that fits LDS (Q image + scratch, with room for the K-merge buffer)
-  auto fits = [&](int mt) {
-    const size_t lds = (size_t)16 * mt * D * 2 + (size_t)8 * 16 * mt * 17 * 4;
-    return lds <= 160 * 1024 && (size_t)16 * mt * D * 2 >= (size_t)64 * K * 8;
-  };
-  if (nq > 16 && fits(4)) return run_topk<4, K>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-  if (nq > 16 && fits(2)) return run_topk<2, K>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-  if (fits(1)) return run_topk<1, K>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
+void run_topk_k(const TopkArgs& a) {
+  // the largest query tile whose image fits LDS beside the bias rows
+  auto fits = [&](int nq_tile) { return (size_t)nq_tile * a.D * 2 + (size_t)a.rows_per_wg * 4 <= 160 * 1024; };
+  if (a.nq > 32 && fits(64)) return run_stream<4, K>(a);
+  if (a.nq > 16 && fits(32)) return run_stream<2, K>(a);
+  if (fits(16)) return run_stream<1, K>(a);
   gai_launch_error(__FILE__, __LINE__, "sim_topk: dimension too large for the LDS query tile");
 }
 
@@ -449,11 +486,11 @@ void gai_sim_topk(const void* Q, const void* X, const float* bias, int nq, int N
                   int* ws_i, int nwg, int rows_per_wg, float* out_v, int64_t* out_i, hipStream_t st) {
   if (nq == 0) return;
   if (D % 32) gai_launch_error(__FILE__, __LINE__, "sim_topk: D must be a multiple of 32");
+  const TopkArgs a{Q, X, bias, nq, N, D, k, nwg, rows_per_wg, ws_v, ws_i, out_v, out_i, st};
+  if (!ws_i) return run_topk_k<0>(a);  // ws_v: the group maxima [nq][ceil(N / 16)]
   switch (gai_topk_cap(k)) {
-    case 4: return run_topk_k<4>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-    case 8: return run_topk_k<8>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-    case 16: return run_topk_k<16>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-    case 32: return run_topk_k<32>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
-    default: return run_topk_k<64>(Q, X, bias, nq, N, D, k, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i, st);
+    case 4: return run_topk_k<4>(a);
+    case 8: return run_topk_k<8>(a);
+    default: gai_launch_error(__FILE__, __LINE__, "sim_topk: lists of more than 8 take the group form");
   }
 }

@@ -762,6 +762,9 @@ def apply_penalties(logits, tok_ids, tok_cnt, n, freq, pres, rep):
 # ---------------------------------------------------------------------------------------------
 # vector search
 # ---------------------------------------------------------------------------------------------
+_LDS_BYTES = 160 * 1024
+
+
 def topk_cap(k: int) -> int:
     return 4 if k <= 4 else 8 if k <= 8 else 16 if k <= 16 else 32 if k <= 32 else 64
 
@@ -773,20 +776,27 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
     k_eff = min(k, n_rows)
     if not Q.is_cuda or n_rows == 0:
         return ref.sim_topk(Q, X, bias, n_rows, k_eff)
-    nq = Q.shape[0]
-    if topk_cap(k_eff) <= 8:
-        # streaming kernel: ~one workgroup per CU, its bias rows staged in LDS (<= 4096 rows)
-        rows_per_wg = min(4096, max(128, ((n_rows + 255) // 256 + 127) // 128 * 128))
-    else:
-        rows_per_wg = max(128, ((n_rows + 1023) // 1024 + 127) // 128 * 128)
-        rows_per_wg = min(rows_per_wg, 8192)
+    nq, D = Q.shape
+    # ~one workgroup per CU, its bias rows staged in LDS beside at least 16 queries (<= 4096 rows)
+    rows_per_wg = min(4096, max(128, ((n_rows + 255) // 256 + 127) // 128 * 128),
+                      max(128, (_LDS_BYTES - 32 * D) // 4 // 128 * 128))
     nwg = (n_rows + rows_per_wg - 1) // rows_per_wg
-    cap = topk_cap(k_eff)
-    ws_v = torch.empty(nwg * nq * cap, dtype=torch.float32, device=Q.device)
-    ws_i = torch.empty(nwg * nq * cap, dtype=torch.int32, device=Q.device)
     out_v = torch.empty(nq, k_eff, dtype=torch.float32, device=Q.device)
     out_i = torch.empty(nq, k_eff, dtype=torch.int64, device=Q.device)
-    native().sim_topk(Q.contiguous(), X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i)
+    Q, cap = Q.contiguous(), topk_cap(k_eff)
+    if cap == 4 or (cap == 8 and nq <= 64):  # short lists in registers (topk.hip: both forms measured)
+        ws_v = torch.empty(nwg * nq * cap, dtype=torch.float32, device=Q.device)
+        ws_i = torch.empty(nwg * nq * cap, dtype=torch.int32, device=Q.device)
+        native().sim_topk(Q, X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i)
+        return out_v, out_i
+    # the largest score of every 16 rows and query, for at most 256 MB of (query, group) pairs at a time
+    groups = (n_rows + 15) // 16
+    step = min(nq, max(64, (64 << 20) // groups // 64 * 64))
+    ws_v = torch.empty(max(1, step * groups), dtype=torch.float32, device=Q.device)
+    ws_i = torch.empty(0, dtype=torch.int32, device=Q.device)
+    for s in range(0, nq, max(1, step)):
+        e = min(nq, s + step)
+        native().sim_topk(Q[s:e], X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v[s:e], out_i[s:e])
     return out_v, out_i
 
 

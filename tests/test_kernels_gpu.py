@@ -489,6 +489,36 @@ def test_sim_topk_stream_large(cuda, nq):
         assert ((i % 11) != 5).all() and (i < N).all()
 
 
+@pytest.mark.parametrize("nq,N,D,k,kind", [
+    (1, 9, 64, 9, "plain"), (2, 40, 384, 33, "plain"), (17, 16 * 1024, 96, 64, "plain"), (3, 16 * 1024 + 1, 384, 17, "plain"),
+    (130, 70_001, 128, 40, "plain"), (33, 300_000, 32, 64, "equal"), (70, 20_000, 64, 7, "plain"), (2, 400_003, 32, 64, "strided"), (5, 2000, 64, 12, "odd")])
+def test_sim_topk_long_lists(cuda, nq, N, D, k, kind):
+    """k > 8 (group maxima + second pass): small whole numbers, so every sum is exact and the order among equal scores
+    (lowest row first) can be compared too. equal: every row the same; strided: the best rows share one thread of the
+    selection; odd: NaN, infinite and deleted rows."""
+    g = torch.Generator().manual_seed(N + k)
+    X = torch.randint(-2, 3, (N, D), generator=g).float()
+    Q = torch.randint(-2, 3, (nq, D), generator=g).float()
+    bias = torch.zeros(N)
+    if kind == "equal":
+        X[:] = X[0]
+    if kind == "strided":
+        bias[7 * 16::16 * 1024] = 1000.0
+        bias[7 * 16 + 1::16 * 1024] = 1000.0
+        bias[3 * 16:20_000 * 16:16] = torch.arange(bias[3 * 16:20_000 * 16:16].numel()).flip(0) / 64
+    if kind == "odd":
+        bias[::3] = float("-inf")
+        bias[10], bias[11], bias[13] = float("nan"), float("inf"), float("inf")
+        bias[16:] = float("-inf")   # nine live rows
+    s = Q @ X.t() + bias
+    v, i = ops.sim_topk(Q.to(cuda, torch.bfloat16), X.to(cuda, torch.bfloat16), bias.to(cuda), N, k)
+    s = torch.where(s.isnan(), torch.full_like(s, float("-inf")), s)
+    vr, ir = torch.sort(s, dim=-1, descending=True, stable=True)
+    vr, ir = vr[:, :k], ir[:, :k]
+    assert torch.equal(v.cpu(), vr)
+    assert torch.equal(i.cpu(), torch.where(vr == float("-inf"), torch.full_like(ir, -1), ir))
+
+
 def test_embedding_pool_act(cuda):
     torch.manual_seed(10)
     table = torch.randn(1000, 256, device=cuda, dtype=torch.bfloat16)
