@@ -734,6 +734,49 @@ void mlstm(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& ig, 
             (float)den_eps, y.data_ptr(), wsp, dt, cur_stream());
 }
 
+// proj [T, 2 Hk DK + 2 Hv DV + 2 Hv] (q | k | v | z | b | a), conv weight [C, 4], conv state [slots, 3, C]
+void gdn_prep(const Tensor& proj, const Tensor& cw, const Tensor& cstate, const Tensor& cu, const Tensor& slots,
+              const Tensor& A_log, const Tensor& dt_bias, Tensor& q, Tensor& k, Tensor& v, Tensor& g, Tensor& beta) {
+  const int dt = act_dt(proj, "proj"), ld = row_stride(proj, "proj");
+  TORCH_CHECK(q.dim() == 3 && k.sizes() == q.sizes() && v.dim() == 3, "gdn_prep: q / k [T, Hk, DK], v [T, Hv, DV]");
+  const int T = proj.size(0), S = slots.numel(), Hk = q.size(1), DK = q.size(2), Hv = v.size(1), DV = v.size(2);
+  const int64_t C = 2 * (int64_t)Hk * DK + (int64_t)Hv * DV;
+  TORCH_CHECK(proj.size(1) == C + (int64_t)Hv * DV + 2 * Hv && q.size(0) == T && v.size(0) == T, "gdn_prep: projection width");
+  TORCH_CHECK(cw.dim() == 2 && cw.size(0) == C && cw.size(1) == 4 && cstate.dim() == 3 && cstate.size(1) == 3 &&
+                  cstate.size(2) == C, "gdn_prep: convolution of 4 taps, state [slots, 3, C]");
+  TORCH_CHECK(S >= 1 && cu.numel() == S + 1 && A_log.numel() == Hv && dt_bias.numel() == Hv &&
+                  g.numel() == (int64_t)T * Hv && beta.numel() == g.numel(), "gdn_prep: cu / gates");
+  gai_gdn_prep(proj.data_ptr(), ld, f32(cw, "cw"), f32(cstate, "cstate"), i32(cu, "cu"), i32(slots, "slots"), S, T, Hk, Hv,
+               DK, DV, f32(A_log, "A_log"), f32(dt_bias, "dt_bias"), f32w(q, "q"), f32w(k, "k"), f32w(v, "v"), f32w(g, "g"),
+               f32w(beta, "beta"), dt, cur_stream());
+}
+
+void gdn_chunks(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta, const Tensor& chunks,
+                const Tensor& chunk0, const Tensor& slots, Tensor& ws, Tensor& state, Tensor& out) {
+  TORCH_CHECK(q.dim() == 3 && k.sizes() == q.sizes() && v.dim() == 3 && state.dim() == 4, "gdn_chunks: shapes");
+  const int64_t T = q.size(0), Hk = q.size(1), DK = q.size(2), Hv = v.size(1), DV = v.size(2);
+  const int64_t nc = chunks.numel() / 2, S = slots.numel(), ch = nc * Hv * 64;
+  TORCH_CHECK(v.size(0) == T && g.numel() == T * Hv && beta.numel() == T * Hv && out.numel() == T * Hv * DV && Hk > 0 &&
+                  Hv % Hk == 0 && DV % 16 == 0, "gdn_chunks: v / g / beta / out shapes");
+  TORCH_CHECK(state.size(1) == Hv && state.size(2) == DK && state.size(3) == DV && chunk0.numel() == S + 1,
+              "gdn_chunks: state / chunk shapes");
+  TORCH_CHECK(ws.numel() >= ch * (2 * 64 + 3), "gdn_chunks: workspace too small");
+  float* W = f32w(ws, "ws");
+  gai_gdn_chunks(f32(q, "q"), f32(k, "k"), f32(v, "v"), f32(g, "g"), f32(beta, "beta"), i32(chunks, "chunks"),
+                 i32(chunk0, "chunk0"), i32(slots, "slots"), (int)nc, (int)S, (int)Hk, (int)Hv, (int)DK, (int)DV, W,
+                 W + ch * 64, W + ch * 2 * 64, f32w(state, "state"), f32w(out, "out"), cur_stream());
+}
+
+void gdn_out(const Tensor& o, const Tensor& z, const Tensor& w, double eps, Tensor& y) {
+  const int dt = act_dt(z, "z");
+  same_dt(w, dt, "w");
+  same_dt(y, dt, "y");
+  TORCH_CHECK(o.dim() == 3 && w.numel() == o.size(2) && w.is_contiguous() && y.is_contiguous() && y.numel() == o.numel() &&
+                  z.size(0) == o.size(0) && z.size(1) == o.size(1) * o.size(2), "gdn_out: shapes");
+  gai_gdn_out(f32(o, "o"), z.data_ptr(), row_stride(z, "z"), w.data_ptr(), y.data_ptr(), o.size(0), o.size(1), o.size(2),
+              (float)eps, dt, cur_stream());
+}
+
 }  // namespace
 
 void gai_bind_seq_ops(pybind11::module_& m) {
@@ -768,6 +811,9 @@ void gai_bind_seq_ops(pybind11::module_& m) {
   m.def("state_tail_write", &state_tail_write);
   m.def("conv_silu", &conv_silu);
   m.def("wkv_scan", &wkv_scan);
+  m.def("gdn_prep", &gdn_prep);
+  m.def("gdn_chunks", &gdn_chunks);
+  m.def("gdn_out", &gdn_out);
   m.def("delta_prep", &delta_prep);
   m.def("delta_scan", &delta_scan);
   m.def("gated_norm_add_f32", &gated_norm_add_f32);

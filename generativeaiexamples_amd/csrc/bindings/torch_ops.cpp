@@ -957,13 +957,14 @@ void gdn_decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
   check_f32(out, "out");
   check_i32(slots, "slots");
   TORCH_CHECK(q.dim() == 3 && k.sizes() == q.sizes() && v.dim() == 3 && state.dim() == 4, "gdn_decode: shapes");
-  const int B = q.size(0), Hv = q.size(1), DK = q.size(2), DV = v.size(2);
+  const int B = q.size(0), Hk = q.size(1), Hv = v.size(1), DK = q.size(2), DV = v.size(2);
+  TORCH_CHECK(Hk > 0 && Hv % Hk == 0, "gdn_decode: value heads must be a multiple of the key heads");
   TORCH_CHECK(v.size(0) == B && v.size(1) == Hv && g.numel() == (int64_t)B * Hv && beta.numel() == (int64_t)B * Hv,
               "gdn_decode: v / g / beta shapes");
   TORCH_CHECK(state.size(1) == Hv && state.size(2) == DK && state.size(3) == DV && slots.numel() == B &&
                   out.numel() == (int64_t)B * Hv * DV, "gdn_decode: state / slots / out shapes");
   gai_gdn_decode(q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), g.data_ptr<float>(),
-                 beta.data_ptr<float>(), state.data_ptr<float>(), slots.data_ptr<int>(), out.data_ptr<float>(), B, Hv,
+                 beta.data_ptr<float>(), state.data_ptr<float>(), slots.data_ptr<int>(), out.data_ptr<float>(), B, Hk, Hv,
                  DK, DV, cur_stream());
 }
 

@@ -209,9 +209,18 @@ int gai_gemm_splitk_fusable_norm(int M, int N, int K);
 void gai_gemm_splitk_add_rmsnorm(const void* A, const void* B, const void* bias, void* res, const void* g, void* out,
                                  int M, int N, int K, float eps, float* ws, int psw, hipStream_t st);
 
-// gdn.hip (Qwen3-Next gated DeltaNet decode step; state pool [slots, Hv, DK, DV] fp32, updated in place)
+// gdn.hip (Qwen3-Next gated DeltaNet; state pool [slots, Hv, DK, DV] fp32, updated in place; Hv a multiple of Hk).
+// chunks [nc, 2]: first row and length of every 64-row chunk, chunk0 [S + 1]: first chunk of every sequence
 void gai_gdn_decode(const float* q, const float* k, const float* v, const float* g, const float* beta, float* state,
-                    const int* slots, float* out, int B, int Hv, int DK, int DV, hipStream_t st);
+                    const int* slots, float* out, int B, int Hk, int Hv, int DK, int DV, hipStream_t st);
+void gai_gdn_prep(const void* proj, int ld, const float* cw, const float* cstate, const int* cu, const int* slots, int S,
+                  int T, int Hk, int Hv, int DK, int DV, const float* A_log, const float* dt_bias, float* q, float* k,
+                  float* v, float* g, float* beta, int dt, hipStream_t st);
+void gai_gdn_chunks(const float* q, const float* k, const float* v, const float* g, const float* beta, const int* chunks,
+                    const int* chunk0, const int* slots, int nc, int S, int Hk, int Hv, int DK, int DV, float* Ti, float* M,
+                    float* F, float* state, float* out, hipStream_t st);
+void gai_gdn_out(const float* o, const void* z, int ldz, const void* w, void* y, int T, int Hv, int DV, float eps, int dt,
+                 hipStream_t st);
 
 // ---- sequence mixers with fp32 residual / state (hybrid decoders: window attention, WKV, channel-decay delta rule) ----
 // dt: 0 = bf16 activations, 1 = fp32 activations (weights of the small per-channel tables are always fp32).

@@ -22,8 +22,9 @@ MI355X mapping:
     rotation (cos 1, sin 0) on the pass-through dims;
   * linear-attention layers keep per-sequence fp32 states (conv window + [Hv, dk, dv] recurrent state)
     in a slot pool; decode steps update them in place with the ``gdn_decode`` HIP kernel (graph
-    capturable: slot vector is a static graph input); prefill chunks run the chunked (WY-form) gated
-    delta rule as batched fp32 GEMMs, resuming from the slot state across chunked-prefill steps;
+    capturable: slot vector is a static graph input); prefill portions run the chunked (WY-form) gated
+    delta rule on the fp32 matrix cores (gdn.hip gdn_chunk / gdn_carry), resuming from the slot state across
+    chunked-prefill steps; head sizes those kernels are not built for take batched fp32 products (gdn_chunk_prefill);
   * MoE reuses the Mixtral route / dispatch / grouped-GEMM / combine kernels; the shared-expert gate
     is one extra row of the router GEMM.
 """
@@ -401,11 +402,20 @@ class Qwen3NextModel:
         dec = [self._slot(sid, False) for sid in fb.seq_ids[P:]]
         fb.extra = dict(prefill_slots=pre,
                         decode_slots=torch.tensor(dec, dtype=torch.int32).to(self.device, non_blocking=True))
+        if self._gdn_kernels:
+            cu = [0]
+            for n in list(fb.prefill_qlen) + [1] * len(dec):
+                cu.append(cu[-1] + n)
+            fb.extra["cu"] = torch.tensor(cu, dtype=torch.int32).to(self.device, non_blocking=True)
+            fb.extra["slots"] = torch.tensor(pre + dec, dtype=torch.int32).to(self.device, non_blocking=True)
+            if P:
+                fb.extra["chunks"], fb.extra["chunk0"] = ops.gdn_chunk_plan(fb.prefill_qlen, self.device)
 
     def graph_static_inputs(self, bs: int) -> dict:
         self._ensure_pool()
-        return dict(prefill_slots=[], decode_slots=torch.full((bs,), self.pad_slot, dtype=torch.int32,
-                                                              device=self.device))
+        ds = torch.full((bs,), self.pad_slot, dtype=torch.int32, device=self.device)
+        return dict(prefill_slots=[], decode_slots=ds, slots=ds,
+                    cu=torch.arange(bs + 1, dtype=torch.int32, device=self.device))
 
     def fill_graph_inputs(self, extra: dict, seq_ids, n: int):
         ids = torch.tensor([self._slot(s, False) for s in seq_ids], dtype=torch.int32)
@@ -434,11 +444,38 @@ class Qwen3NextModel:
         a = attn.view(T, -1) * torch.sigmoid(gate)
         return ops.linear(a, w[p + "o"])
 
+    @property
+    def _gdn_kernels(self) -> bool:
+        c = self.cfg
+        return self.device.type == "cuda" and ops.gdn_ok(c.linear_key_head_dim, c.linear_value_head_dim,
+                                                         c.linear_conv_kernel_dim, c.linear_num_key_heads,
+                                                         c.linear_num_value_heads)
+
+    def _linear_attention_kernels(self, proj, i, fb, T, P):
+        """The mixer on the gfx950 kernels: inputs, chunked rule over the prompt portions, recurrent step of the decoded
+        tokens, gated norm."""
+        c, w, p, extra = self.cfg, self.w, f"l{i}.", fb.extra
+        Hk, Hv, dk, dv = c.linear_num_key_heads, c.linear_num_value_heads, c.linear_key_head_dim, c.linear_value_head_dim
+        li, cd, vd = self.lin_index[i], self.conv_dim, self.vd
+        cs, ss = self.conv_state[li], self.ssm_state[li]
+        q, k, v, g, beta = ops.gdn_prep(proj, w[p + "conv"], cs, extra["cu"], extra["slots"], w[p + "A_log"],
+                                        w[p + "dt_bias"], Hk, dk, Hv, dv)
+        ops.state_tail_write(proj[:, :cd], cs, extra["cu"], extra["slots"])
+        core = torch.empty(T, Hv, dv, device=proj.device)
+        if P > 0:
+            ops.gdn_chunks(q[:P], k[:P], v[:P], g[:P], beta[:P], extra["chunks"], extra["chunk0"],
+                           extra["slots"][: len(fb.prefill_qlen)], ss, core[:P])
+        if T > P:
+            ops.native().gdn_decode(q[P:], k[P:], v[P:], g[P:], beta[P:], ss, extra["decode_slots"][: T - P], core[P:])
+        return ops.linear(ops.gdn_out(core, proj[:, cd:cd + vd], w[p + "gnorm"], c.rms_eps), w[p + "out"])
+
     def _linear_attention(self, x, i, fb, T, P):
         c, w, p = self.cfg, self.w, f"l{i}."
         Hk, Hv, dk, dv = c.linear_num_key_heads, c.linear_num_value_heads, c.linear_key_head_dim, c.linear_value_head_dim
         Kc, li = c.linear_conv_kernel_dim, self.lin_index[i]
         proj = ops.linear(x, w[p + "in_proj"])
+        if self._gdn_kernels:
+            return self._linear_attention_kernels(proj, i, fb, T, P)
         cd, vd = self.conv_dim, self.vd
         mixed = proj[:, :cd].float()
         z = proj[:, cd:cd + vd]

@@ -1373,6 +1373,50 @@ def wkv_scan(r, k, v, wpre, w0, u, state, cu, slots):
     return out
 
 
+GDN_CHUNK = 64
+
+
+def gdn_ok(DK: int, DV: int, taps: int, Hk: int, Hv: int) -> bool:
+    """Head sizes the gated-DeltaNet kernels (gdn.hip) are built for."""
+    return DK in (64, 128, 256) and DV % 16 == 0 and taps == 4 and Hv % Hk == 0
+
+
+def gdn_prep(proj, conv_w, conv_state, cu, slots, A_log, dt_bias, Hk: int, DK: int, Hv: int, DV: int):
+    """Gated-DeltaNet inputs of projected rows (q | k | v | z | b | a): causal convolution + SiLU (history before a
+    sequence's first row from conv_state[slot], which is only read), unit q (x DK^-1/2) and k [T, Hk, DK], v [T, Hv, DV],
+    log decay and write strength [T, Hv]; all fp32."""
+    T, e = proj.shape[0], lambda *s: torch.empty(*s, dtype=torch.float32, device=proj.device)  # noqa: E731
+    q, k, v, g, beta = e(T, Hk, DK), e(T, Hk, DK), e(T, Hv, DV), e(T, Hv), e(T, Hv)
+    native().gdn_prep(proj, conv_w, conv_state, cu, slots, A_log, dt_bias, q, k, v, g, beta)
+    return q, k, v, g, beta
+
+
+def gdn_chunk_plan(lens: Sequence[int], device):
+    """(chunks [nc, 2], chunk0 [S + 1]) of packed prompt portions: first row and length of every 64-row chunk, and the
+    first chunk of every portion."""
+    chunks, first, at = [], [0], 0
+    for n in lens:
+        chunks += [(at + c, min(GDN_CHUNK, n - c)) for c in range(0, n, GDN_CHUNK)]
+        first.append(len(chunks))
+        at += n
+    flat = torch.tensor([x for c in chunks for x in c] + first, dtype=torch.int32).to(device, non_blocking=True)
+    return flat[:2 * len(chunks)], flat[2 * len(chunks):]
+
+
+def gdn_chunks(q, k, v, g, beta, chunks, chunk0, slots, state, out) -> None:
+    """Gated delta rule over prompt portions: out [T, Hv, DV], state[slots] updated in place (fp32 throughout)."""
+    nc, Hv = chunks.numel() // 2, v.shape[1]
+    ws = torch.empty(nc * Hv * GDN_CHUNK * (2 * GDN_CHUNK + 3), dtype=torch.float32, device=q.device)
+    native().gdn_chunks(q, k, v, g, beta, chunks, chunk0, slots, ws, state, out)
+
+
+def gdn_out(o, z, w, eps: float):
+    """silu(z) * (w * norm(o)) per head, rounded to z's type after each step -> [T, Hv * DV]."""
+    y = torch.empty(o.shape[0], o.shape[1] * o.shape[2], dtype=z.dtype, device=z.device)
+    native().gdn_out(o, z, w, float(eps), y)
+    return y
+
+
 def delta_prep(qkv, a, b, A_log, dt_bias, H: int, G: int, DK: int):
     """Delta-rule inputs: unit q (x DK^-1/2) / k [T, G, DK], decay [T, H, DK], beta [T, H] (all fp32)."""
     if not qkv.is_cuda:

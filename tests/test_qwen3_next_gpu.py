@@ -33,6 +33,71 @@ def test_gdn_decode_kernel(cuda, dk, dv):
     assert torch.equal(state[untouched], before[untouched])
 
 
+@pytest.mark.parametrize("lens,Hk,Hv,dk,dv", [([1], 1, 1, 64, 16), ([63, 1, 65], 2, 4, 128, 128), ([200, 64], 2, 2, 64, 48),
+                                              ([3, 129], 1, 3, 256, 32), ([1000], 2, 4, 128, 128)])
+def test_gdn_chunks_against_float64(cuda, lens, Hk, Hv, dk, dv):
+    """Chunked rule on the matrix cores, resumed from a non-zero state, against the token-by-token recurrence in float64.
+    Bound: the running sum of the log decay reaches -40 in a chunk of these inputs, so a factor e^(G_t - G_s) carries a
+    relative error of up to 2 x 40 x 2^-24 = 4.8e-6 however it is computed from fp32 sums; the products' own rounding is
+    below it."""
+    g_ = torch.Generator().manual_seed(sum(lens))
+    T, S = sum(lens), len(lens)
+    rn = lambda *s: torch.randn(*s, generator=g_, dtype=torch.float64)  # noqa: E731
+    q, k = (torch.nn.functional.normalize(rn(T, Hk, dk), dim=-1) for _ in range(2))
+    q, v = q * dk ** -0.5, rn(T, Hv, dv)
+    g, beta = -torch.rand(T, Hv, generator=g_, dtype=torch.float64) ** 4 * 3, torch.sigmoid(rn(T, Hv))
+    state, slots = rn(S + 2, Hv, dk, dv) * 0.1, list(range(S + 1, 1, -1))
+    ins = [t.float() for t in (q, k, v, g, beta)]
+    q, k, v, g, beta = (t.double() for t in ins)
+    s32 = state.float().to(cuda)
+    want, Sw, at = torch.empty(T, Hv, dv, dtype=torch.float64), state.float().double(), 0
+    r = Hv // Hk
+    for n, slot in zip(lens, slots):
+        St = Sw[slot][None].clone()
+        for t in range(at, at + n):
+            o, St = gdn_recurrent_step(q[t:t + 1].repeat_interleave(r, 1), k[t:t + 1].repeat_interleave(r, 1), v[t:t + 1],
+                                       g[t:t + 1], beta[t:t + 1], St)
+            want[t] = o[0]
+        Sw[slot] = St[0]
+        at += n
+    out = torch.full((T, Hv, dv), float("nan"), device=cuda)
+    chunks, chunk0 = ops.gdn_chunk_plan(lens, cuda)
+    ops.gdn_chunks(*(t.to(cuda) for t in ins), chunks, chunk0, torch.tensor(slots, dtype=torch.int32, device=cuda), s32, out)
+    for a, b in ((out, want), (s32, Sw)):
+        assert (a.cpu().double() - b).norm() <= 4.8e-6 * b.norm()
+
+
+@pytest.mark.parametrize("lens,Hk,Hv,dk,dv,dt", [([1, 2, 5], 2, 4, 64, 64, torch.bfloat16), ([700, 1, 3, 0, 9], 1, 3, 128, 48, torch.bfloat16),
+                                                 ([1] * 5, 2, 2, 256, 16, torch.float32)])
+def test_gdn_prep_matches_torch(cuda, lens, Hk, Hv, dk, dv, dt):
+    """Convolution over sequence starts (history from the slot), unit q / k, gates; then the history that is kept."""
+    torch.manual_seed(1)
+    T, S, kd, vd = sum(lens), len(lens), Hk * dk, Hv * dv
+    cd = 2 * kd + vd
+    proj = torch.randn(T, cd + vd + 2 * Hv, device=cuda).to(dt)
+    cw, cs = torch.randn(cd, 4, device=cuda), torch.randn(S + 3, 3, cd, device=cuda)
+    A_log, dt_bias = torch.randn(Hv, device=cuda), torch.randn(Hv, device=cuda)
+    slots = torch.randperm(S + 3)[:S].to(cuda, torch.int32)
+    cu = torch.tensor([0] + lens).cumsum(0).to(cuda, torch.int32)
+    q, k, v, g, beta = ops.gdn_prep(proj, cw, cs, cu, slots, A_log, dt_bias, Hk, dk, Hv, dv)
+    x, at, conv, kept = proj[:, :cd].double(), 0, [], cs.double()
+    for s, n in enumerate(lens):
+        xs = torch.cat([kept[slots[s]], x[at:at + n]])
+        if n:
+            conv.append((xs.unfold(0, 4, 1) * cw.double()).sum(-1))
+            kept[slots[s]] = xs[-3:]
+        at += n
+    conv = torch.nn.functional.silu(torch.cat(conv))
+    unit = lambda t: t * torch.rsqrt(t.pow(2).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    b, a = proj[:, cd + vd:cd + vd + Hv].double(), proj[:, cd + vd + Hv:].double()
+    want = (unit(conv[:, :kd].view(T, Hk, dk)) * dk ** -0.5, unit(conv[:, kd:2 * kd].view(T, Hk, dk)), conv[:, 2 * kd:].view(T, Hv, dv),
+            -torch.exp(A_log.double()) * torch.nn.functional.softplus(a + dt_bias.double()), torch.sigmoid(b))
+    for got, w in zip((q, k, v, g, beta), want):
+        assert torch.allclose(got.double(), w, rtol=2e-6, atol=2e-6)
+    ops.state_tail_write(proj[:, :cd], cs, cu, slots)
+    assert torch.allclose(cs.double(), kept, rtol=1e-6, atol=0)
+
+
 def _pair(cuda):
     cfg = Qwen3NextConfig.tiny()
     g = Qwen3NextModel(cfg, device=cuda).random_init(3)
