@@ -9,6 +9,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "gai_gemm_mid.h"
 #include "gai_kernels.h"
 
 void gai_launch_error(const char* file, int line, const char* msg) {
@@ -164,6 +165,18 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
   if (R) {
     check_bf16(*R, "residual");
     TORCH_CHECK(R->numel() == (int64_t)M * N, "gemm: residual has wrong size");
+  }
+  if (M > 0 && N > 0 && (force == 0 || force == 14 || force >= 1000)) {  // a few hundred rows, where it pays
+    GaiMidPlan plan;
+    if (gai_gemm_mid_plan(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi,
+                          f32 ? 1 : 0, (int)force, bfrag ? 1 : 0, cur_stream(), &plan)) {
+      Tensor ws;
+      if (plan.ws_floats) ws = at::empty({(int64_t)plan.ws_floats}, A.options().dtype(at::kFloat));
+      gai_gemm_mid(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f32 ? 1 : 0,
+                   plan, plan.ws_floats ? ws.data_ptr<float>() : nullptr, cur_stream(), bfrag ? 1 : 0);
+      return;
+    }
+    TORCH_CHECK(force == 0, "gemm: the mid-size kernel needs K % 128 == 0, N % 16 == 0 and aligned operands");
   }
   gai_gemm(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f32 ? 1 : 0,
            (int)force, cur_stream(), bfrag ? 1 : 0);

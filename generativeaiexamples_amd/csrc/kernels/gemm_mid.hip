@@ -1,0 +1,384 @@
+// bf16 GEMM for a few hundred rows (64 < M <= 2048: short prompts, prompt portions, batches of questions):
+// C[M, N] = A[M, K] . B[N, K]^T with the fused epilogues of gemm_impl.h, B row-major or in fragment order.
+//
+// At these sizes the weights are read once and bound the product (Llama-3-8B down projection, M = 187: 117 MB, 20 us at
+// 5.8 TB/s); what keeps a tiled kernel from that rate is latency (a load from HBM takes over 2 us) and the few tiles there
+// are. So:
+//  * a workgroup takes 16 * MT rows x 64 * NG columns: 128 x 64 (two workgroups share a CU), 128 x 128 or, so that up to
+//    192 rows still fetch the weights once, 192 x 128;
+//  * the weights go straight to registers in operand layout, DB 128-deep K steps ahead (wave = 16 * NG columns x half of
+//    the K step: nothing is fetched twice, and in whole 128-byte lines); the rows of A, which sit in L2, pass through registers into LDS (two buffers, one
+//    barrier per step) and are read by all waves. All loads are ordinary ones, so their waits are counted. Both operands by
+//    DMA through a five-step LDS ring instead held 80 KB of weights per CU in flight and took 0.52 us a step, whatever the
+//    rest of the step looked like;
+//  * K is cut into S parts, so tile x part items fill the CUs;
+//  * measured on one card, weights from HBM, fragment order (row-major about 15 % slower), N x K: 187 rows 4096 x 14336
+//    200 -> 49 us, 4096 x 4096 66 -> 24 us, 6144 x 4096 57 -> 29 us, 28672 x 4096 (SwiGLU) 73 -> 61 us; 512 rows 67 -> 33,
+//    59 -> 41, 1024 x 4096 62 -> 19, 3072 x 1024 21 -> 11, 2048 x 5632 78 -> 28 us.
+//  * MFMA operands swapped (rows = weights), so a lane ends with four consecutive columns of a row: 8-byte stores;
+//  * S > 1: every wave stores its fp32 share (write-through) and draws the (tile, wave) ticket; the one that draws the last
+//    sums the parts in part order - the same result whichever it is - and runs the epilogue. Nobody waits, and a wave that
+//    sees all others done keeps its share in registers.
+#include "gai_common.h"
+#include "gai_epilogue.h"
+#include "gai_gemm_mid.h"
+#include "gai_kernels.h"
+
+#include <algorithm>
+#include <map>
+#include <mutex>
+#include <utility>
+
+using namespace gai;
+
+namespace {
+
+constexpr int kBK = 128;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+
+template <int EPI, bool OUTF32>
+__device__ __forceinline__ void store4(void* C, const bf16* bias, const bf16* R, int ldc, int m, int n, f32x4 v) {
+  const size_t o = (size_t)m * ldc + n;
+  constexpr bool kBias = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_BIAS_RESIDUAL || EPI == EPI_BIAS_RELU ||
+                         EPI == EPI_BIAS_QUICKGELU;
+  constexpr bool kRes = EPI == EPI_RESIDUAL || EPI == EPI_BIAS_RESIDUAL;
+  if constexpr (kBias) {
+    const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + n);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] += (float)b[r];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if constexpr (EPI == EPI_BIAS_GELU) v[r] = gelu_erf(v[r]);
+    if constexpr (EPI == EPI_BIAS_RELU) v[r] = fmaxf(v[r], 0.f);
+    if constexpr (EPI == EPI_BIAS_QUICKGELU) v[r] = quick_gelu(v[r]);
+  }
+  if constexpr (kRes) {
+    const bf16x4 x = *reinterpret_cast<const bf16x4*>(R + o);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = (OUTF32 ? v[r] : (float)(bf16)v[r]) + (float)x[r];
+  }
+  if constexpr (OUTF32) {
+    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + o) = v;
+  } else {
+    bf16x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = (bf16)v[r];
+    *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(C) + o) = y;
+  }
+}
+
+template <int MT, int NG, int EPI, bool OUTF32>
+__global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B, void* C,
+                                                          const bf16* __restrict__ bias, const bf16* R, int M, int N, int K,
+                                                          int ldc, int bfrag, int S, float* ws, int* cnt) {
+  constexpr int BM = 16 * MT, BN = 64 * NG, NA = MT / 2, NF = MT / 2 * NG;
+  constexpr int DB = NG == 2 ? 3 : 4, U = NG == 2 ? 6 : 4;  // steps the weights are ahead; unrolled steps (even)
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // 2 x BM x 256 B; at the end the k halves' exchange
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tm_n = (M + BM - 1) / BM, tiles = tm_n * ((N + BN - 1) / BN);
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int part = id / tiles, tile = id - part * tiles;
+  const int m0 = tile % tm_n * BM, n0 = tile / tm_n * BN;
+  const int nk = K / kBK, k0 = (int)((long long)nk * part / S), n = (int)((long long)nk * (part + 1) / S) - k0;
+  const int g = wid & 3, h = wid >> 2;  // column group, k half
+
+  const bf16* ap[NA];  // row tid / 16 (+ 32 per piece), 16-B piece tid & 15
+  int a_wr[NA];
+#pragma unroll
+  for (int q = 0; q < NA; ++q) {
+    const int row = q * 32 + (tid >> 4), c = tid & 15;
+    ap[q] = A + (size_t)min(m0 + row, M - 1) * K + (size_t)k0 * kBK + c * 8;
+    a_wr[q] = row * 256 + ((c ^ (row & 15)) << 4);
+  }
+  const bf16* bp[NG];
+#pragma unroll
+  for (int f = 0; f < NG; ++f) {
+    const int col = n0 + (g * NG + f) * 16;
+    bp[f] = bfrag ? B + ((size_t)min(col / 16, N / 16 - 1) * (K / 32) + 4 * (size_t)k0 + 2 * h) * 512 + lane * 8
+                  : B + (size_t)min(col + (lane & 15), N - 1) * K + (size_t)k0 * kBK + 64 * h + 8 * (lane >> 4);
+  }
+  const int bstep = bfrag ? 2048 : kBK, bhalf = bfrag ? 512 : 32;
+  bf16x8 ar[NA], br[DB][NG][2];
+  // past the end the last step is read again (from L2): the count of loads stays what the code says
+  auto load_a = [&](int t, bf16x8(&d)[NA]) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) d[q] = load8(ap[q] + (size_t)min(t, n - 1) * kBK);
+  };
+  auto load_b = [&](int t, bf16x8(&d)[NG][2]) {
+#pragma unroll
+    for (int f = 0; f < NG; ++f)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) d[f][e] = load8(bp[f] + (size_t)min(t, n - 1) * bstep + e * bhalf);
+  };
+  auto put_a = [&](int buf, const bf16x8(&d)[NA]) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) *reinterpret_cast<bf16x8*>(smem + buf * (BM * 256) + a_wr[q]) = d[q];
+  };
+  int a_rd[2];  // + 4096 per 16 rows
+#pragma unroll
+  for (int e = 0; e < 2; ++e) a_rd[e] = (lane & 15) * 256 + (((8 * h + 4 * e + (lane >> 4)) ^ (lane & 15)) << 4);
+  f32x4 acc[MT][NG];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int f = 0; f < NG; ++f) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  load_a(0, ar);
+#pragma unroll
+  for (int d = 0; d < DB; ++d) load_b(d, br[d]);
+  put_a(0, ar);
+  load_a(1, ar);
+  for (int t = 0;; t += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // A of this step is in LDS and everybody has left the other buffer
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      put_a((u + 1) & 1, ar);
+      load_a(t + u + 2, ar);
+      const char* s = smem + (u & 1) * (BM * 256);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        bf16x8 af[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const bf16x8*>(s + a_rd[e] + i * 4096);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int f = 0; f < NG; ++f)
+            acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(br[u % DB][f][e], af[i], acc[i][f], 0, 0, 0);
+      }
+      load_b(t + u + DB, br[u % DB]);
+      if (t + u + 1 >= n) goto done;
+    }
+  }
+done:
+  // the k halves: this wave keeps row tiles h * MT / 2 .. of its columns and adds what its partner has of them
+  __syncthreads();
+  f32x4 v[NF];
+  {
+    f32x4* x = reinterpret_cast<f32x4*>(smem) + g * 2 * NF * 64 + lane;  // [group][half][NF][64]
+#pragma unroll
+    for (int i = 0; i < MT / 2; ++i)
+#pragma unroll
+      for (int f = 0; f < NG; ++f) {
+        v[i * NG + f] = h ? acc[MT / 2 + i][f] : acc[i][f];
+        x[((h ^ 1) * NF + i * NG + f) * 64] = h ? acc[i][f] : acc[MT / 2 + i][f];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < NF; ++e) {
+      const f32x4 y = x[(h * NF + e) * 64];
+      v[e] = h ? y + v[e] : v[e] + y;  // first half + second half
+    }
+  }
+  if (S > 1) {
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(ws, (short)0, 0x7fffffff, 0x00020000);
+    auto woff = [&](int p, int e) {
+      return (unsigned)__builtin_amdgcn_readfirstlane(((p * tiles + tile) * 8 + wid) * (NF * 1024) + e * 1024);
+    };
+    int* ctr = cnt + tile * 8 + wid;
+    bool stored = false;
+    if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != S - 1) {
+#pragma unroll
+      for (int e = 0; e < NF; ++e)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[e]), rw, lane * 16, woff(part, e), 16);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share has landed
+      int tk = 0;
+      if (lane == 0) tk = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__builtin_amdgcn_readfirstlane(tk) != S - 1) return;
+      stored = true;
+    }
+    if (lane == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // no instruction: keeps the loads below the ticket
+    f32x4 sum[NF], nx[4][NF];  // four parts' loads at a time
+#pragma unroll
+    for (int e = 0; e < NF; ++e) sum[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < S; p += 4) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int e = 0; e < NF; ++e)
+          nx[d][e] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, woff(min(p + d, S - 1), e), 16));
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        if (p + d >= S) break;
+        const bool own = p + d == part && !stored;
+#pragma unroll
+        for (int e = 0; e < NF; ++e) sum[e] += own ? v[e] : nx[d][e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < NF; ++e) v[e] = sum[e];
+  }
+  // lane: row m of C, columns n .. n + 3 of each 16 x 16 tile
+#pragma unroll
+  for (int i = 0; i < MT / 2; ++i) {
+    const int m = m0 + 16 * (h * (MT / 2) + i) + (lane & 15);
+    if (m >= M) continue;
+    const int nn = n0 + g * NG * 16;
+    if constexpr (epi_glu(EPI)) {
+      static_assert(NG == 2, "a gated pair of column tiles belongs to one wave");
+      if (nn >= N) continue;
+      f32x4 y;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = glu_act<EPI>(v[i * NG][r], v[i * NG + NG - 1][r]);
+      store4<EPI_NONE, OUTF32>(C, nullptr, nullptr, ldc, m, nn / 2 + 4 * (lane >> 4), y);
+    } else {
+#pragma unroll
+      for (int f = 0; f < NG; ++f)
+        if (nn + 16 * f < N) store4<EPI, OUTF32>(C, bias, R, ldc, m, nn + 16 * f + 4 * (lane >> 4), v[i * NG + f]);
+    }
+  }
+}
+
+int mid_cus() {
+  static int ncu = 0;
+  if (!ncu) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
+      gai_launch_error(__FILE__, __LINE__, "gemm_mid: cannot query the CU count");
+  }
+  return ncu;
+}
+
+int mid_tiles(int M, int N, int mt, int ng) { return ((M + 16 * mt - 1) / (16 * mt)) * ((N + 64 * ng - 1) / (64 * ng)); }
+
+// Tickets of a (device, stream): kCnt zeros, zero again after every launch. Never freed or grown: at most 64 KB a stream.
+constexpr int kCnt = 16384;
+int* mid_counters(hipStream_t st) {
+  static std::mutex mu;
+  static std::map<std::pair<int, hipStream_t>, int*> pool;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lk(mu);
+  int*& c = pool[{dev, st}];
+  if (!c) {
+    if (hipMalloc(&c, kCnt * sizeof(int)) != hipSuccess) return c = nullptr;
+    if (hipMemsetAsync(c, 0, kCnt * sizeof(int), st) != hipSuccess) {
+      (void)hipFree(c);
+      c = nullptr;
+    }
+  }
+  return c;
+}
+
+// Modelled times in us, fitted to eleven N x K from 1024 x 1024 to 28672 x 4096 at 80 - 2048 rows (most within 15 %).
+// This kernel: launch, first loads and epilogue; K steps of a workgroup (slower when the chip is full) or the weights at the
+// rate HBM gives; storing and summing the parts.
+double mid_cost(int M, int N, int K, int mt, int ng, int S, int bfrag) {
+  const int items = mid_tiles(M, N, mt, ng) * S, steps = (K / kBK + S - 1) / S, G = mid_cus(), rounds = (items + G - 1) / G;
+  const double base = mt == 12 ? 8.6 : ng == 2 ? 6.3 : 4.7, alone = mt == 12 ? 1.35 : ng == 2 ? 1.0 : 0.71;
+  const double full = mt == 12 ? 1.65 : ng == 2 ? 1.2 : 0.73, fill = std::min(1.0, (double)items / G);
+  const double step = (alone + (full - alone) * fill) * (bfrag ? 1.0 : 1.17);
+  return base + std::max(rounds * steps * step, (double)N * K * 2 / 5.0e6) + (S > 1 ? 2.3 + 1.2 * S : 0.0);
+}
+// the kernels of gemm_impl.h, with its own rules: skinny (M <= 128), 128 x 128 tiles, 256 x 256 tiles, stream-K
+double other_cost(int M, int N, int K) {
+  if (M <= 128 && K % 256 == 0) return K <= 1024 && N <= 4096 ? 0.0 : 1e9;
+  const int G = mid_cus() & ~7, t1 = ((M + 127) / 128) * ((N + 127) / 128), t2 = ((M + 255) / 256) * ((N + 255) / 256);
+  if (M >= 256 && N >= 256 && 2 * t2 >= G) return 12.0 + (t2 + G - 1) / G * (K / 64) * (t2 < 200 ? 1.15 : 1.4);
+  if (M >= 256 && N >= 256 && K >= 8192) return 70.0 + 0.05 * M;
+  return 8.0 + (t1 + 2 * G - 1) / (2 * G) * (K / 64) * 1.0;
+}
+
+template <int MT, int NG, int EPI, bool OUTF32>
+void launch_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int S,
+                float* ws, int* cnt, hipStream_t st, int bfrag) {
+  constexpr int lds = MT * 8192;  // two A buffers; the exchange takes MT * NG * 4096
+  static bool once = false;
+  if (!once) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mid_kernel<MT, NG, EPI, OUTF32>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+      gai_launch_error(__FILE__, __LINE__, "gemm_mid: LDS size");
+    once = true;
+  }
+  gemm_mid_kernel<MT, NG, EPI, OUTF32><<<mid_tiles(M, N, MT, NG) * S, 512, lds, st>>>(
+      (const bf16*)A, (const bf16*)B, C, (const bf16*)bias, (const bf16*)R, M, N, K, ldc, bfrag, S, ws, cnt);
+  GAI_LAUNCH_CHECK();
+}
+
+}  // namespace
+
+bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K,
+                       int ldc, int epi, int out_f32, int force, int bfrag, hipStream_t st, GaiMidPlan* plan) {
+  if (M < 1 || K % kBK || N % 16 || ldc % 4 || (out_f32 && epi != EPI_NONE)) return false;
+  if (force == 0 && (M <= 64 || M > 2048 || N < 256)) return false;
+  const bool glu = epi == EPI_SWIGLU || epi == EPI_GEGLU;
+  if ((!(epi >= EPI_NONE && epi <= EPI_BIAS_QUICKGELU) && !glu) || (glu && N % 32)) return false;
+  // 4-column loads and stores, 16-byte loads of the operands
+  auto off = [](const void* p, unsigned a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
+  if (off(A, 16) || off(B, 16) || off(C, out_f32 ? 16 : 8) || off(bias, 8) || off(R, 8)) return false;
+  GaiMidPlan best{8, 2, 1, 0};
+  if (force >= 1000) {
+    best = {force / 1000, glu ? 2 : force / 100 % 10, std::max(1, std::min(force % 100, K / kBK)), 0};
+  } else {
+    double bc = 1e30;
+    for (int v = glu ? 1 : 0; v < 3; ++v) {
+      const int mt = v == 2 ? 12 : 8, ng = v == 0 ? 1 : 2;
+      for (int S = 1; S <= std::min(16, std::max(1, K / kBK / 4)); ++S) {
+        if (S > 1 && mid_tiles(M, N, mt, ng) * 8 > kCnt) break;
+        const double c = mid_cost(M, N, K, mt, ng, S, bfrag);
+        if (c < bc) {
+          bc = c;
+          best = {mt, ng, S, 0};
+        }
+      }
+    }
+    if (force == 0 && bc >= other_cost(M, N, K)) return false;
+  }
+  if (best.parts > 1) {
+    // a captured launch may replay beside another one on this stream: tickets cannot be shared with it
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const int tiles = mid_tiles(M, N, best.mt, best.ng);
+    const size_t bytes = (size_t)tiles * best.parts * 8 * (best.mt / 2 * best.ng) * 1024;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone || bytes >= (1ull << 31) ||
+        tiles * 8 > kCnt || !mid_counters(st))
+      best.parts = 1;
+    else
+      best.ws_floats = bytes / 4;
+    if (best.parts == 1 && force == 0 && mid_cost(M, N, K, best.mt, best.ng, 1, bfrag) >= other_cost(M, N, K)) return false;
+  }
+  *plan = best;
+  return true;
+}
+
+void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,
+                  int out_f32, const GaiMidPlan& p, float* ws, hipStream_t st, int bfrag) {
+  int* cnt = p.parts > 1 ? mid_counters(st) : nullptr;
+#define GAI_MID(MT, NG, E, F32)                                                                         \
+  if (p.mt == MT && p.ng == NG)                                                                         \
+    return launch_mid<MT, NG, E, F32>(A, B, C, bias, R, M, N, K, ldc, p.parts, ws, cnt, st, bfrag);
+#define GAI_MID_EPI(E, F32)         \
+  {                                 \
+    GAI_MID(8, 1, E, F32)           \
+    GAI_MID(8, 2, E, F32)           \
+    GAI_MID(12, 2, E, F32)          \
+    break;                          \
+  }
+#define GAI_MID_GLU(E)              \
+  {                                 \
+    GAI_MID(8, 2, E, false)         \
+    GAI_MID(12, 2, E, false)        \
+    break;                          \
+  }
+  switch (epi) {
+    case EPI_NONE:
+      if (out_f32) GAI_MID_EPI(EPI_NONE, true) else GAI_MID_EPI(EPI_NONE, false)
+      break;
+    case EPI_BIAS: GAI_MID_EPI(EPI_BIAS, false)
+    case EPI_BIAS_GELU: GAI_MID_EPI(EPI_BIAS_GELU, false)
+    case EPI_RESIDUAL: GAI_MID_EPI(EPI_RESIDUAL, false)
+    case EPI_SWIGLU: GAI_MID_GLU(EPI_SWIGLU)
+    case EPI_BIAS_RESIDUAL: GAI_MID_EPI(EPI_BIAS_RESIDUAL, false)
+    case EPI_BIAS_RELU: GAI_MID_EPI(EPI_BIAS_RELU, false)
+    case EPI_BIAS_QUICKGELU: GAI_MID_EPI(EPI_BIAS_QUICKGELU, false)
+    case EPI_GEGLU: GAI_MID_GLU(EPI_GEGLU)
+    default: break;
+  }
+#undef GAI_MID_GLU
+#undef GAI_MID_EPI
+#undef GAI_MID
+  gai_launch_error(__FILE__, __LINE__, "gemm_mid: no kernel for this plan");
+}

@@ -188,3 +188,31 @@ def test_prefill_qkv_rope_kv_narrow_declines(cuda):
     assert (q.float().cpu() - q2).abs().max().item() < 5e-2
     assert (kc.float().cpu() - k2).abs().max().item() < 5e-2
     assert (vc.float().cpu() - v2).abs().max().item() < 5e-2
+
+
+@pytest.mark.parametrize("plan", [8101, 8103, 8202, 8204, 12201, 12203])  # 1000 * rows / 16 + 100 * columns / 64 + parts of K
+@pytest.mark.parametrize("M,N,K", [(1, 64, 128), (65, 272, 256), (128, 1040, 640), (193, 320, 1152), (700, 2304, 512), (192, 512, 4224)])
+@pytest.mark.parametrize("act", [None, "bias", "gelu", "relu", "residual", "bias_residual", "swiglu", "f32"])
+def test_mid_gemm(cuda, M, N, K, act, plan):
+    """The kernel for a few hundred rows: partial row / column tiles, one to 33 K steps of uneven parts, row-major and
+    fragment-ordered weights (same sums), launch after launch the same bits."""
+    if act == "swiglu" and N % 32:
+        pytest.skip("SwiGLU weights interleave in 32-row groups")
+    torch.manual_seed(M + 3 * N + K)
+    x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    w = (torch.randn(N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
+    bias = torch.randn(N, device=cuda, dtype=torch.bfloat16) if act in ("bias", "gelu", "relu", "bias_residual") else None
+    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16) if act in ("residual", "bias_residual") else None
+    a = act if act in ("gelu", "relu", "swiglu") else None
+    dt = torch.float32 if act == "f32" else torch.bfloat16
+    y = _run(x, w, bias, res, a, dt, force=plan)
+    y_ref = ref.linear(x.cpu(), w.cpu(), None if bias is None else bias.cpu(), None if res is None else res.cpu(), a, dt)
+    err = (y.float().cpu() - y_ref.float()).abs()
+    assert not torch.isnan(y).any(), "unwritten output elements"
+    tol = 1e-4 if act == "f32" else 3e-2 + 2e-2 * y_ref.float().abs()   # f32: sums of up to 4224 products of unit size / sqrt(K)
+    assert (err <= tol).all(), f"{M}x{N}x{K} {act}: max err {err.max():.4g}"
+    f = ops.shuffle_fragments(w)
+    out = torch.full_like(y, float("nan"))
+    for _ in range(3):
+        ops.native().gemm(x, f, out, bias, res, {"f32": 0, None: 0}.get(act, ops.EPI.get(act, 0)), plan, True)
+        assert torch.equal(out, y)
