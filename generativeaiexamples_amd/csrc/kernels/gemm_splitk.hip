@@ -17,6 +17,7 @@
 
 #include "gai_common.h"
 #include "gai_epilogue.h"
+#include "gai_gemm_slim.h"
 #include "gai_kernels.h"
 #include "gai_rope.h"
 
@@ -935,6 +936,11 @@ void gai_gemm_splitk(const void* A, const void* B, void* C, const void* bias, co
   // natural weight layout: the LDS-staged decode kernel (gemm_decode.hip) when the shape fits - single
   // pass for the wide projections, K-split slabs for the deep ones
   if (gai_gemm_dec2(A, B, C, bias, R, M, N, K, ldc, epi, out_f32, st, psw)) return;
+  // narrow and shallow: one launch with all of K in a workgroup (gemm_slim.hip)
+  if (const int nf = gai_gemm_slim_nf(M, N, K, epi_glu(epi))) {
+    gai_gemm_slim(A, B, C, bias, R, M, N, K, ldc, epi, out_f32, nf, psw, st);
+    return;
+  }
   const int ks2 = gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw);
   const int KS = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
   if (KS == 0) gai_launch_error(__FILE__, __LINE__, "gemm_splitk: K must be a multiple of 512");

@@ -47,6 +47,49 @@ def test_splitk_epilogues(cuda, act):
     torch.testing.assert_close(y.float().cpu(), r, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("M,N,K,epi", [
+    (1, 16, 512, "bias"), (16, 1040, 1024, "gelu"), (17, 64, 1536, "residual"), (31, 96, 2560, "swiglu"),
+    (32, 1024, 4096, "bias_residual"), (33, 2064, 512, None), (64, 4096, 2560, "relu"), (64, 2048, 2048, "quick_gelu"),
+    (49, 3104, 1024, "geglu"), (5, 6160, 1024, None), (24, 5136, 1536, "bias")])
+@pytest.mark.parametrize("frag,f32", [(False, False), (True, False), (False, True)])
+def test_one_launch_gemm(cuda, M, N, K, epi, frag, f32):
+    """Narrow decode projections in one launch (all of K in a workgroup): row tiles 16 / 32 / 64 with ragged M, one and
+    two column fragments with a half-empty last pair, 1 to 8 activation stages with a short last one. Bound per element:
+    K fp32 products in any order, K 2^-24 sum |x w|, then what the epilogue's own steps can move, and one bf16 rounding."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g).to(torch.bfloat16) if epi in ("bias", "gelu", "relu", "quick_gelu", "bias_residual") \
+        else None
+    res = torch.randn(M, N, generator=g).to(torch.bfloat16) if epi in ("residual", "bias_residual") else None
+    dev = [None if t is None else t.cuda() for t in (x, ops.shuffle_fragments(w) if frag else w, bias, res)]
+    ncol = N // 2 if epi in ("swiglu", "geglu") else N
+    out = torch.full((M, ncol), float("nan"), device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+    nat = ops.native()
+    ws = torch.empty(nat.gemm_splitk_ws_floats(M, N, K), device="cuda", dtype=torch.float32)
+    nat.gemm_splitk(dev[0], dev[1], out, dev[2], dev[3], ops.EPI[epi] if epi else 0, ws, frag)
+    y = x.double() @ w.double().t()
+    if bias is not None:
+        y = y + bias.double()
+    e = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    if epi in ("swiglu", "geglu"):
+        y, e = (t.view(M, N // 32, 2, 16) for t in (y, e))
+        a, u = y[:, :, 0], y[:, :, 1]
+        act = torch.nn.functional.silu(a) if epi == "swiglu" else torch.nn.functional.gelu(a, approximate="tanh")
+        # both gates have slopes below 1.13; the hardware exp / tanh forms stay within 2^-18 of the value
+        e = 1.13 * e[:, :, 0] * u.abs() + act.abs() * e[:, :, 1] + 2.0 ** -18 * (act * u).abs() + 1e-6
+        y, e = (act * u).reshape(M, ncol), e.reshape(M, ncol)
+    elif epi in ("gelu", "quick_gelu", "relu"):
+        y = {"gelu": torch.nn.functional.gelu, "relu": torch.relu, "quick_gelu": lambda t: t * torch.sigmoid(1.702 * t)}[epi](y)
+        e = 1.13 * e + 2.0 ** -18 * y.abs() + 1e-6
+    if res is not None:
+        e = e + (0 if f32 else 2.0 ** -8 * y.abs())  # bf16 product, then the sum rounded again
+        y = y + res.double()
+    e = e + (2.0 ** -23 if f32 else 2.0 ** -8) * y.abs()
+    d = (out.double().cpu() - y).abs()
+    assert (d <= e).all(), (d / e).max()
+
+
 def test_linear_routes_decode_to_splitk(cuda):
     """ops.linear for M <= 64 uses the decode kernels and matches the reference."""
     x = torch.randn(64, 4096, device="cuda", dtype=torch.bfloat16)
