@@ -216,3 +216,33 @@ def test_mid_gemm(cuda, M, N, K, act, plan):
     for _ in range(3):
         ops.native().gemm(x, f, out, bias, res, {"f32": 0, None: 0}.get(act, ops.EPI.get(act, 0)), plan, True)
         assert torch.equal(out, y)
+
+
+def test_gelu_whole_range(cuda):
+    """Every bf16 value through the erf GELU: the 1.5e-7 of the erfc formula (7.1.26) times |x| / 2 and one bf16 rounding;
+    the limits at the infinities, NaN kept. The formula is a1 t exp(-z^2) far out, 0.778 / z against erfc's 0.564 / z, so a
+    negative x also stays within 0.38 of the (vanishing) value itself."""
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    y = ops.gelu(x.view(64, 1024).to(cuda)).cpu().flatten().double()
+    xd = x.double()
+    fin = torch.isfinite(xd)
+    r = xd[fin] * 0.5 * torch.erfc(-xd[fin] / math.sqrt(2))
+    # denormals may be flushed: 1e-37
+    tail = torch.where(xd[fin] < 0, torch.minimum(0.75e-7 * xd[fin].abs(), 0.39 * r.abs()), 0.75e-7 * xd[fin])
+    assert ((y[fin] - r).abs() <= 2.0 ** -8 * r.abs() + tail + 1e-37).all()
+    assert (y[xd == math.inf] == math.inf).all() and (y[xd == -math.inf] == 0).all()
+    assert y[torch.isnan(xd)].isnan().all()
+
+
+@pytest.mark.parametrize("kern", ["w4d", "w4r", "w4d192", "w4x"])
+@pytest.mark.parametrize("M,N,K,bias", [(1100, 272, 256, True), (8192, 8448, 256, False), (700, 4096, 1024, True)])
+def test_ring_residual_in_place(cuda, M, N, K, bias, kern):
+    """The residual may be the output: it is read ahead of the stores, each lane only what it stores itself."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    w = (torch.randn(N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
+    b = torch.randn(N, device=cuda, dtype=torch.bfloat16) if bias else None
+    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16)
+    y = _run(x, w, b, res, None, force=KERNELS[kern])
+    ops.native().gemm(x, w, res, b, res, ops.EPI["bias_residual" if bias else "residual"], KERNELS[kern])
+    assert torch.equal(res, y)
