@@ -166,19 +166,31 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
     check_bf16(*R, "residual");
     TORCH_CHECK(R->numel() == (int64_t)M * N, "gemm: residual has wrong size");
   }
-  if (M > 0 && N > 0 && (force == 0 || force == 14 || force >= 1000)) {  // a few hundred rows, where it pays
+  int rows = M;  // of the kernels of gemm_impl.h; the rest, if any, by the mid-size kernel
+  if (M > 0 && N > 0 && (force == 0 || force == 14 || force >= 1000)) {
     GaiMidPlan plan;
-    if (gai_gemm_mid_plan(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi,
-                          f32 ? 1 : 0, (int)force, bfrag ? 1 : 0, cur_stream(), &plan)) {
+    const int f = f32 ? 1 : 0, frag = bfrag ? 1 : 0;
+    int mid = 0;
+    if (gai_gemm_mid_plan(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f,
+                          (int)force, frag, cur_stream(), &plan))
+      mid = M;
+    else if (force == 0)
+      mid = gai_gemm_mid_tail(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f,
+                              frag, cur_stream(), &plan);
+    TORCH_CHECK(mid || force == 0, "gemm: the mid-size kernel needs K % 128 == 0, N % 16 == 0 and aligned operands");
+    if (mid) {
+      rows = M - mid;
       Tensor ws;
       if (plan.ws_floats) ws = at::empty({(int64_t)plan.ws_floats}, A.options().dtype(at::kFloat));
-      gai_gemm_mid(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f32 ? 1 : 0,
-                   plan, plan.ws_floats ? ws.data_ptr<float>() : nullptr, cur_stream(), bfrag ? 1 : 0);
-      return;
+      const void* r = opt_ptr(R);
+      gai_gemm_mid(static_cast<char*>(A.data_ptr()) + (size_t)rows * K * 2, B.data_ptr(),
+                   static_cast<char*>(C.data_ptr()) + (size_t)rows * ldc * (f32 ? 4 : 2), opt_ptr(bias),
+                   r ? static_cast<const char*>(r) + (size_t)rows * ldc * 2 : nullptr, mid, N, K, ldc, (int)epi, f, plan,
+                   plan.ws_floats ? ws.data_ptr<float>() : nullptr, cur_stream(), frag);
+      if (!rows) return;
     }
-    TORCH_CHECK(force == 0, "gemm: the mid-size kernel needs K % 128 == 0, N % 16 == 0 and aligned operands");
   }
-  gai_gemm(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f32 ? 1 : 0,
+  gai_gemm(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), rows, N, K, ldc, (int)epi, f32 ? 1 : 0,
            (int)force, cur_stream(), bfrag ? 1 : 0);
 }
 

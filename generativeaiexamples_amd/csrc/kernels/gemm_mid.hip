@@ -310,9 +310,9 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
   // 4-column loads and stores, 16-byte loads of the operands
   auto off = [](const void* p, unsigned a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
   if (off(A, 16) || off(B, 16) || off(C, out_f32 ? 16 : 8) || off(bias, 8) || off(R, 8)) return false;
-  GaiMidPlan best{8, 2, 1, 0};
+  GaiMidPlan best{8, 2, 1, 0, 0.0};
   if (force >= 1000) {
-    best = {force / 1000, glu ? 2 : force / 100 % 10, std::max(1, std::min(force % 100, K / kBK)), 0};
+    best = {force / 1000, glu ? 2 : force / 100 % 10, std::max(1, std::min(force % 100, K / kBK)), 0, 0.0};
   } else {
     double bc = 1e30;
     for (int v = glu ? 1 : 0; v < 3; ++v) {
@@ -322,7 +322,7 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
         const double c = mid_cost(M, N, K, mt, ng, S, bfrag);
         if (c < bc) {
           bc = c;
-          best = {mt, ng, S, 0};
+          best = {mt, ng, S, 0, c};
         }
       }
     }
@@ -338,10 +338,36 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
       best.parts = 1;
     else
       best.ws_floats = bytes / 4;
-    if (best.parts == 1 && force == 0 && mid_cost(M, N, K, best.mt, best.ng, 1, bfrag) >= other_cost(M, N, K)) return false;
+    if (best.parts == 1) best.cost = mid_cost(M, N, K, best.mt, best.ng, 1, bfrag);
+    if (best.parts == 1 && force == 0 && best.cost >= other_cost(M, N, K)) return false;
   }
   *plan = best;
   return true;
+}
+
+// The 256 x 256 kernels work in rounds of one tile per CU, 6 us + 1.42 us per 64 of K each (M 16384, N 4096: 28.5, 49, 94 us at
+// K 1024, 2048, 4096; 9 more with a residual), however few tiles the last one has. Its rows go to this kernel where the
+// model says so with 15 % to spare (its own error) and a launch, and the saving is 5 % of the whole. N 1024 with a residual:
+// 18337 rows (288 tiles on 256 CUs) K 1024 56.7 -> 48.3 us, K 4096 167.6 -> 134.2; 18480 rows 58.7 -> 56.8, 171.7 -> 150.8.
+// At N 3072 and 4096, K 1024 the remainder costs as much as the round it saves; after many rounds (Llama-3-8B gate_up at
+// 14500 rows: 25) the tiles have drifted apart and there is no empty round left to save (167.2 ms with, 166.1 without).
+int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
+                      int epi, int out_f32, int bfrag, hipStream_t st, GaiMidPlan* plan) {
+  if (M <= 2048 || N < 256 || N % 16 || ldc % 8 || K % kBK || K < 256) return 0;
+  const int G = mid_cus() & ~7, tn = (N + 255) / 256, tm = (M + 255) / 256;
+  const long long tiles = (long long)tm * tn;
+  if (tiles % G == 0) return 0;
+  const int m1 = (int)(tiles / G * G / tn) * 256, m2 = M - m1;  // whole rounds, whole row tiles
+  if (m1 <= 0 || m2 <= 0 || m2 > 3072) return 0;
+  auto at = [&](const void* p, size_t row, size_t size) {
+    return p ? reinterpret_cast<const char*>(p) + (size_t)m1 * row * size : nullptr;
+  };
+  if (!gai_gemm_mid_plan(at(A, K, 2), B, at(C, ldc, out_f32 ? 4 : 2), bias, at(R, ldc, 2), m2, N, K, ldc, epi, out_f32, 14, bfrag,
+                         st, plan))
+    return 0;
+  const double round = 6.0 + K / 64 * 1.42 + (R ? 9.0 : 0.0);
+  const double saved = round - plan->cost * 1.15 - 3.0;
+  return saved > 0.05 * round * ((tiles + G - 1) / G) ? m2 : 0;
 }
 
 void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,

@@ -246,3 +246,28 @@ def test_ring_residual_in_place(cuda, M, N, K, bias, kern):
     y = _run(x, w, b, res, None, force=KERNELS[kern])
     ops.native().gemm(x, w, res, b, res, ops.EPI["bias_residual" if bias else "residual"], KERNELS[kern])
     assert torch.equal(res, y)
+
+
+@pytest.mark.parametrize("M,N,K,act", [(18337, 1024, 1024, "bias_residual"), (16500, 1024, 4096, "bias_residual"),
+                                       (2306, 28672, 1024, "swiglu"), (17000, 1040, 2048, "gelu"), (9000, 2048, 4096, "f32")])
+@pytest.mark.parametrize("frag", [False, True])
+def test_tail_rows_of_a_large_gemm(cuda, M, N, K, act, frag):
+    """Rows past the last whole round of 256x256 tiles go to the mid-size kernel: against the 256x256 kernel alone, which
+    rounds the same fp32 sums taken in another order (K 2^-24 sum |x w| apart, then at most one bf16 step and, with a
+    residual, one more)."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    w = (torch.randn(N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
+    b = torch.randn(N, device=cuda, dtype=torch.bfloat16) if act in ("gelu", "bias_residual") else None
+    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16) if act == "bias_residual" else None
+    a = act if act in ("gelu", "swiglu") else None
+    dt = torch.float32 if act == "f32" else torch.bfloat16
+    one = _run(x, w, b, res, a, dt, force=10)
+    epi = 0 if act == "f32" else ops.EPI[act]
+    out = torch.full_like(one, float("nan"))
+    ops.native().gemm(x, ops.shuffle_fragments(w) if frag else w, out, b, res, epi, 0, frag)
+    assert not torch.isnan(out).any(), "unwritten rows"
+    # |x| . |w| <= K E|x| E|w| (1 + small): 0.64 sqrt(K); the gates have slopes below 1.13 and multiply by |up| < 6
+    e = K * 2.0 ** -24 * 0.75 * math.sqrt(K) * (8 if act == "swiglu" else 1.13)
+    d = (out.float() - one.float()).abs()
+    assert (d <= 2 * e + (0 if act == "f32" else 2.0 ** -6) * one.float().abs().clamp_min(1 if res is not None else 0)).all(), d.max()
