@@ -9,6 +9,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "gai_gemm_grouped.h"
 #include "gai_gemm_mid.h"
 #include "gai_kernels.h"
 
@@ -604,6 +605,22 @@ void moe_gemm(const Tensor& A, const optional<Tensor>& a_rows, const Tensor& W, 
                (float)act_param);
 }
 
+// Prefill-sized expert products in one launch; false (nothing launched) where the shape does not fit.
+bool moe_gemm_large(const Tensor& A, const Tensor& W, Tensor& C, const Tensor& offs, bool swiglu) {
+  check_bf16(A, "A");
+  check_bf16(W, "W");
+  check_bf16(C, "C");
+  check_i32(offs, "expert offsets");
+  TORCH_CHECK(A.dim() == 2 && W.dim() == 3 && W.size(2) == A.size(1), "moe_gemm_large: A [rows, K], W [E, N, K]");
+  TORCH_CHECK(offs.numel() >= W.size(0) + 1 && C.dim() == 2 && C.size(0) == A.size(0) &&
+                  C.size(1) == (swiglu ? W.size(1) / 2 : W.size(1)), "moe_gemm_large: row / offset shapes");
+  if (reinterpret_cast<uintptr_t>(A.data_ptr()) % 16 || reinterpret_cast<uintptr_t>(W.data_ptr()) % 16 ||
+      reinterpret_cast<uintptr_t>(C.data_ptr()) % 16)
+    return false;
+  return gai_gemm_grouped(A.data_ptr(), W.data_ptr(), C.data_ptr(), offs.data_ptr<int>(), W.size(0), A.size(0), W.size(1),
+                          W.size(2), swiglu ? 1 : 0, cur_stream());
+}
+
 void moe_dispatch(const Tensor& ids, int64_t E, Tensor& a_rows, Tensor& offs, Tensor& pos) {
   check_i32(ids, "expert ids");
   check_i32(a_rows, "a_rows");
@@ -1081,6 +1098,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_route", &moe_route);
   m.def("moe_router", &moe_router);
   m.def("moe_scale_rows", &moe_scale_rows);
+  m.def("moe_gemm_large", &moe_gemm_large);
   m.def("moe_gemm", &moe_gemm);
   m.def("moe_route_chosen", &moe_route_chosen);
   m.def("moe_route_grouped", &moe_route_grouped);

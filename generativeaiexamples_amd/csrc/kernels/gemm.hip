@@ -2,6 +2,7 @@
 // RoPE + paged-KV write in its epilogue. The kernels and launchers are in gemm_impl.h; the per-epilogue
 // instantiations in gemm_epi_*.hip.
 #include "gemm_impl.h"
+#include "gai_gemm_grouped.h"
 
 #ifndef GAI_GEMM_KERNELS_ONLY
 bool gai_sk_workspace(hipStream_t st, size_t ws_bytes, size_t cnt_n, float** ws_out, int** cnt_out) {
@@ -78,3 +79,8 @@ int gai_gemm_prefill_rope_kv(const void* A, const void* B, const void* bias, con
   return 1;
 }
 #endif  // GAI_GEMM_KERNELS_ONLY
+
+bool gai_gemm_grouped(const void* A, const void* B, void* C, const int* offs, int E, int M, int N, int K, int swiglu,
+                      hipStream_t st) {
+  return swiglu ? gai_gemm_grouped4(A, B, C, offs, E, M, N, K, N / 2, st) : gai_gemm_grouped0(A, B, C, offs, E, M, N, K, N, st);
+}

@@ -2,4 +2,5 @@
 #include "gemm_impl.h"
 
 GAI_GEMM_RUN(0)
+GAI_GEMM_GROUPED(0)
 GAI_GEMM_RUN(1)

@@ -2,4 +2,5 @@
 #include "gemm_impl.h"
 
 GAI_GEMM_RUN(4)
+GAI_GEMM_GROUPED(4)
 GAI_GEMM_RUN(7)

@@ -962,16 +962,23 @@ constexpr int kPart = 256 * 64 * 2;  // one operand of a double unit
 
 constexpr int kSkQuad = 128 * 128;  // fp32 of one wave's quadrant partial
 
+// WALK 3 (grouped): A's rows sorted by expert, expert e's in [offs[e], offs[e + 1]), B [E, N, K]: the tile walk over all
+// experts' tiles in one launch (M = all rows; tiles counted from offs on the device, so the host waits for nothing).
 template <int EPI, bool OUTF32, int WALK = 0>
 __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
                                                           void* C, const bf16* bias, const bf16* R, int M, int N,
-                                                          int K, int ldc, float* ws, int* cnt, int S, int bfrag) {
+                                                          int K, int ldc, float* ws, int* cnt, int S, int bfrag,
+                                                          const int* __restrict__ offs = nullptr, int E = 0) {
   constexpr bool SK = WALK == 1;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // 5 parts x 32 KiB
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_m = (M + LBM - 1) / LBM, tiles_n = (N + LBN - 1) / LBN;
-  const int tiles = tiles_m * tiles_n;
+  int tiles = tiles_m * tiles_n;
+  if constexpr (WALK == 3) {
+    tiles = 0;
+    for (int e = 0; e < E; ++e) tiles += (offs[e + 1] - offs[e] + LBM - 1) / LBM * tiles_n;
+  }
   const int G = gridDim.x;
   const int nd = K / 64;  // host guarantees K % 64 == 0, nd >= 2 (WALK 1 / 2: K % 128 == 0; WALK 2: S <= nd / 2)
   const int hp = nd / 2;
@@ -1001,27 +1008,42 @@ __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict
       len = nd;
     }
   };
-  auto raster = [&](int t, int& m0, int& n0) {
+  // mend: the end of the tile's rows (its expert's), be: its expert
+  auto raster = [&](int t, int& m0, int& n0, int& mend, int& be) {
     constexpr int GM = 4;
+    int tm = tiles_m, lo = 0;
+    mend = M;
+    be = 0;
+    if constexpr (WALK == 3) {
+      for (;; ++be) {
+        lo = offs[be];
+        mend = min(offs[be + 1], M);
+        tm = (mend - lo + LBM - 1) / LBM;
+        if (t < tm * tiles_n || be == E - 1) break;
+        t -= tm * tiles_n;
+      }
+    }
     const int group = t / (GM * tiles_n);
     const int first_m = group * GM;
-    const int gsz = min(tiles_m - first_m, GM);
+    const int gsz = min(tm - first_m, GM);
     const int pin = t % (GM * tiles_n);
-    m0 = (first_m + pin % gsz) * LBM;
+    m0 = lo + (first_m + pin % gsz) * LBM;
     n0 = (pin / gsz) * LBN;
   };
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(A), (short)0, 0x7fffffff, 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(B), (short)0, 0x7fffffff, 0x00020000);
   // bfrag: B in MFMA fragment order (as gemm_w4d_kernel): B load j of wave w = fragment (n-tile 4w + j / 2, half j & 1)
   const int bks = bfrag ? 2048 : 128;  // B bytes per k-double step
-  auto offsets = [&](int m0, int n0, int* oa, int* ob) {
+  auto offsets = [&](int m0, int n0, int mend, int be, int* oa, int* ob) {
+    const int eb = WALK == 3 ? be * N * K * 2 : 0;  // (host: E N K < 2 GiB)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int row = (wid * 8 + j) * 8 + (lane >> 3);
       const int gc = (lane & 7) ^ ((row >> 1) & 7);
-      oa[j] = min(m0 + row, M - 1) * K * 2 + gc * 16;
+      oa[j] = min(m0 + row, mend - 1) * K * 2 + gc * 16;
       ob[j] = bfrag ? (min(n0 / 16 + wid * 4 + (j >> 1), N / 16 - 1) * (K / 32) + (j & 1)) * 1024 + lane * 16
                     : min(n0 + row, N - 1) * K * 2 + gc * 16;
+      ob[j] += eb;
     }
   };
   const int wm = wid >> 1, wn = wid & 1;
@@ -1074,11 +1096,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict
 
   int s = s_beg;
   if (s >= s_end) return;  // (the host sizes the grid so that every run is non-empty)
-  int t, kb, len, m0, n0, pt = 0;
+  int t, kb, len, m0, n0, mend, be, pt = 0;
   segment(s, t, kb, len, pt);
-  raster(t, m0, n0);
+  raster(t, m0, n0, mend, be);
   int ca[8], cb[8], xa[8], xb[8];
-  offsets(m0, n0, ca, cb);
+  offsets(m0, n0, mend, be, ca, cb);
   asm volatile(GAI_AGPR_ZERO "s_nop 7\n\ts_nop 7\n" ::: GAI_AGPR_CLOBBERS);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {  // parts A(kb) B(kb) A(kb+1) B(kb+1) -> slots 0..3
@@ -1101,12 +1123,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict
     // next segment's sources; past the last one, dummy re-loads of this segment's first double pair into a
     // slot no later phase reads
     const int sn = SK ? s + len : s + 1;
-    int tn = t, kbn = kb, lenn = len, nm0 = m0, nn0 = n0, ptn = pt;
+    int tn = t, kbn = kb, lenn = len, nm0 = m0, nn0 = n0, nmend = mend, nbe = be, ptn = pt;
     if (sn < s_end) {
       segment(sn, tn, kbn, lenn, ptn);
-      raster(tn, nm0, nn0);
+      raster(tn, nm0, nn0, nmend, nbe);
     }
-    offsets(nm0, nn0, xa, xb);
+    offsets(nm0, nn0, nmend, nbe, xa, xb);
     int D = 0;
     for (; D < len - 2; ++D) {
       const int q = 2 * (gd + D);
@@ -1121,7 +1143,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict
     }
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");  // last MFMAs retire
     bool epi = true;
-    if constexpr (WALK != 0) {
+    if constexpr (WALK == 1 || WALK == 2) {
       if (SK ? (kb != 0 || len != nd) : S > 1) {  // split tile: hand the partial over, or (last ticket) sum them
         // contributors cf..cl (stream-K: logical workgroups, this one = lg; split: the parts, this one = pt)
         const int cf = SK ? owner(t * hp) : 0, cl = SK ? owner(t * hp + hp - 1) : S - 1;
@@ -1204,15 +1226,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict
     }
     if (epi) {
       EpiOperands<EPI, OUTF32> pre;
-      pre.start(bias, R, M, N, ldc, m0 + wm * 128, n0 + wn * 128, lane);
+      pre.start(bias, R, mend, N, ldc, m0 + wm * 128, n0 + wn * 128, lane);
       for_each_const<8>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         f32x4 row[8];
         read_acc_row<i>(row, std::make_integer_sequence<int, 8>{});
-        epilogue_rows<EPI, OUTF32, 8>(row, C, bias, R, pre, i % pre.kAhead, M, N, ldc, m0 + wm * 128 + 16 * i,
+        epilogue_rows<EPI, OUTF32, 8>(row, C, bias, R, pre, i % pre.kAhead, mend, N, ldc, m0 + wm * 128 + 16 * i,
                                       n0 + wn * 128, lane);
         if constexpr (i + pre.kAhead < 8)
-          pre.load_res(i % pre.kAhead, R, M, N, ldc, m0 + wm * 128 + 16 * (i + pre.kAhead), n0 + wn * 128, lane);
+          pre.load_res(i % pre.kAhead, R, mend, N, ldc, m0 + wm * 128 + 16 * (i + pre.kAhead), n0 + wn * 128, lane);
       });
     }
     asm volatile(GAI_AGPR_ZERO "s_nop 7\n\ts_nop 7\n" ::: GAI_AGPR_CLOBBERS);
@@ -1224,6 +1246,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4r_kernel(const bf16* __restrict
     pt = ptn;
     m0 = nm0;
     n0 = nn0;
+    mend = nmend;
+    be = nbe;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       ca[j] = xa[j];
@@ -1414,6 +1438,30 @@ void launch_w4r(const void* A, const void* B, void* C, const void* bias, const v
   gemm_w4r_kernel<EPI, OUTF32><<<grid, 256, 5 * kPart, st>>>((const bf16*)A, (const bf16*)B, C, (const bf16*)bias,
                                                              (const bf16*)R, M, N, K, ldc, nullptr, nullptr, 1, bfrag);
   GAI_LAUNCH_CHECK();
+}
+
+// Every expert's product in one persistent launch (WALK 3). The 256-row tiles of all experts share the rounds: 8 experts of
+// about 750 rows at N 28672 are 3 x 112 tiles each, 1.31 rounds of 256 CUs run as 2 when each expert is launched by itself,
+// and 12.3 run as 13 together. Both products
+// of a layer (N 28672, K 4096 with SwiGLU, and back) 2541 -> 1872 us, the host's wait for the row counts included.
+template <int EPI>
+bool launch_w4r_grouped(const void* A, const void* B, void* C, const int* offs, int E, int M, int N, int K, int ldc,
+                        hipStream_t st) {
+  if (E < 1 || M < 1 || N % 16 || (epi_glu(EPI) && N % 32) || K % 64 || K < 128 || ldc % 8 ||
+      (size_t)M * K * 2 >= (1ull << 31) || (size_t)E * N * K * 2 >= (1ull << 31))  // 32-bit buffer offsets
+    return false;
+  static int ncu = 0;
+  if (!ncu) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
+      gai_launch_error(__FILE__, __LINE__, "gemm_w4r_grouped: cannot query the CU count");
+    set_max_lds(gemm_w4r_kernel<EPI, false, 3>);
+  }
+  gemm_w4r_kernel<EPI, false, 3><<<ncu & ~7, 256, 5 * kPart, st>>>((const bf16*)A, (const bf16*)B, C, nullptr, nullptr, M, N,
+                                                                  K, ldc, nullptr, nullptr, 1, 0, offs, E);
+  GAI_LAUNCH_CHECK();
+  return true;
 }
 
 // Stream-K workspace of one (device, stream): partial quadrants [G][2][4][16384] fp32 and per-(tile, wave)
@@ -1618,3 +1666,11 @@ void gai_gemm_run5(GAI_GEMM_RUN_ARGS);
 void gai_gemm_run6(GAI_GEMM_RUN_ARGS);
 void gai_gemm_run7(GAI_GEMM_RUN_ARGS);
 void gai_gemm_run10(GAI_GEMM_RUN_ARGS);
+
+// per-epilogue entry points of the grouped walk, called by gai_gemm_grouped (gemm.hip)
+#define GAI_GEMM_GROUPED_ARGS \
+  const void *A, const void *B, void *C, const int *offs, int E, int M, int N, int K, int ldc, hipStream_t st
+#define GAI_GEMM_GROUPED(EP) \
+  bool gai_gemm_grouped##EP(GAI_GEMM_GROUPED_ARGS) { return launch_w4r_grouped<EP>(A, B, C, offs, E, M, N, K, ldc, st); }
+bool gai_gemm_grouped0(GAI_GEMM_GROUPED_ARGS);
+bool gai_gemm_grouped4(GAI_GEMM_GROUPED_ARGS);

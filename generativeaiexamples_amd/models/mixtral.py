@@ -62,6 +62,10 @@ class MixtralConfig(LlamaConfig):
 # MoE steps with at least this many (token, expert) rows run each expert on the dense prefill GEMMs
 # (GAI_MOE_DENSE_PREFILL_ROWS; a huge value keeps every step on the grouped kernel)
 _DENSE_PREFILL_MIN_ROWS = int(os.environ.get("GAI_MOE_DENSE_PREFILL_ROWS", "2048"))
+# ... all of them in one launch from this many rows an expert on. 8 experts, N 28672, K 4096, both products, us, one launch
+# each | one launch: 150 rows an expert 1158 | 838, 256 1379 | 1063, 748 2541 | 1872, 2048 5303 | 4605. Below it the 256-row
+# tiles are mostly padding and each expert takes the kernel for its own row count.
+_GROUPED_MIN_ROWS = 128
 
 
 class MixtralModel(LlamaModel):
@@ -160,10 +164,16 @@ class MixtralModel(LlamaModel):
     def _moe_dense_prefill(x, a_rows, offs, w13, w2, rows: int) -> torch.Tensor:
         """Prefill-sized steps: the expert-sorted rows are gathered once and every expert's slice runs on the
         dense persistent 256x256 GEMMs (SwiGLU epilogue on the interleaved w1|w3), ~1.6 vs ~1.0 PF/s for the
-        128x128 grouped kernel at Mixtral widths. Reads the expert row ranges on the host: one sync per layer,
-        prefill only (decode steps keep the graph-capturable grouped path)."""
-        bounds = offs.tolist()
+        128x128 grouped kernel at Mixtral widths: all experts in one launch from _GROUPED_MIN_ROWS rows an expert on, else
+        one launch each, which reads the expert row ranges on the host: one sync per layer, prefill only (decode steps
+        keep the graph-capturable grouped path)."""
         xs = x.index_select(0, a_rows.long())
+        if rows >= _GROUPED_MIN_ROWS * w13.shape[0] and x.dtype == w13.dtype == torch.bfloat16 and ops._GEMM_FORCE == 0:
+            h1 = ops.moe_gemm_large(xs, w13, offs, swiglu=True)
+            y = None if h1 is None else ops.moe_gemm_large(h1, w2, offs)
+            if y is not None:
+                return y
+        bounds = offs.tolist()
         h1 = torch.empty(rows, w13.shape[1] // 2, dtype=x.dtype, device=x.device)
         y = torch.empty(rows, w2.shape[1], dtype=x.dtype, device=x.device)
         for e in range(w13.shape[0]):

@@ -1018,6 +1018,14 @@ def ep_combine(back, ids, pos, offs, w, residual, e_local: int, capacity: int):
 _MOE_ACT = {None: 0, "swiglu": 1, "relu2": 2, "clamp_glu": 3}
 
 
+def moe_gemm_large(A, W, offs, swiglu: bool = False):
+    """``A`` [rows, K] sorted by expert (expert e's rows in [offs[e], offs[e + 1]), offs on the device) times W [E, N, K]:
+    every expert on the 256x256 kernel in one launch, without a look at offs from the host. None where the shape does not
+    fit (operands of 2 GiB, K off 64, N off 16 / 32)."""
+    C = torch.empty(A.shape[0], W.shape[1] // 2 if swiglu else W.shape[1], dtype=A.dtype, device=A.device)
+    return C if native().moe_gemm_large(A, W, C, offs, swiglu) else None
+
+
 def moe_gemm(A, a_rows, W, offs, rows_total: int, swiglu: bool = False, act: Optional[str] = None,
              act_param: float = 0.0):
     """Grouped expert GEMM over expert-sorted rows (A rows gathered through a_rows when given). act: None, "swiglu"

@@ -271,3 +271,38 @@ def test_tail_rows_of_a_large_gemm(cuda, M, N, K, act, frag):
     e = K * 2.0 ** -24 * 0.75 * math.sqrt(K) * (8 if act == "swiglu" else 1.13)
     d = (out.float() - one.float()).abs()
     assert (d <= 2 * e + (0 if act == "f32" else 2.0 ** -6) * one.float().abs().clamp_min(1 if res is not None else 0)).all(), d.max()
+
+
+@pytest.mark.parametrize("sizes", [[300, 0, 1, 700, 256, 0, 257, 40], [0, 0, 5], [1025], [0, 513, 255, 0]])
+@pytest.mark.parametrize("N,K", [(64, 128), (1056, 320), (4128, 192)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_grouped_experts(cuda, sizes, N, K, swiglu):
+    """Rows sorted by expert in one launch: empty experts, one row, partial row and column tiles, the shortest K, more and
+    fewer tiles than CUs. The same bits as each expert by itself on the same kernel: a tile's sums do not depend on its
+    neighbours."""
+    torch.manual_seed(sum(sizes) + N + K)
+    E, rows = len(sizes), sum(sizes)
+    x = torch.randn(rows, K, device=cuda, dtype=torch.bfloat16)
+    w = (torch.randn(E, N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
+    offs = torch.tensor([0] + sizes, dtype=torch.int32).cumsum(0).to(torch.int32).to(cuda)
+    y = torch.full((rows, N // 2 if swiglu else N), float("nan"), device=cuda, dtype=torch.bfloat16)
+    for _ in range(2):
+        assert ops.native().moe_gemm_large(x, w, y, offs, swiglu)
+    lo = 0
+    for e, n in enumerate(sizes):
+        if n:
+            part = x[lo:lo + n].contiguous()
+            r = ref.linear(part.cpu(), w[e].cpu(), act="swiglu" if swiglu else None).float()
+            d = (y[lo:lo + n].float().cpu() - r).abs()
+            assert (d <= 3e-2 + 2e-2 * r.abs()).all(), (e, d.max())  # the bound of the walks above: bf16 rounding of both
+            if K >= 192:
+                assert torch.equal(y[lo:lo + n], _run(part, w[e].contiguous(), None, None, "swiglu" if swiglu else None,
+                                                      force=10)), e
+        lo += n
+
+
+def test_grouped_experts_declines(cuda):
+    x = torch.zeros(64, 96, device=cuda, dtype=torch.bfloat16)
+    w = torch.zeros(2, 64, 96, device=cuda, dtype=torch.bfloat16)
+    offs = torch.tensor([0, 30, 64], dtype=torch.int32, device=cuda)
+    assert ops.moe_gemm_large(x, w, offs) is None  # K % 64
