@@ -777,6 +777,8 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
     if not Q.is_cuda or n_rows == 0:
         return ref.sim_topk(Q, X, bias, n_rows, k_eff)
     nq, D = Q.shape
+    if k_eff == 0:
+        return Q.new_empty(nq, 0, dtype=torch.float32), Q.new_empty(nq, 0, dtype=torch.int64)
     # ~one workgroup per CU, its bias rows staged in LDS beside at least 16 queries (<= 4096 rows)
     rows_per_wg = min(4096, max(128, ((n_rows + 255) // 256 + 127) // 128 * 128),
                       max(128, (_LDS_BYTES - 32 * D) // 4 // 128 * 128))

@@ -519,6 +519,17 @@ def test_sim_topk_long_lists(cuda, nq, N, D, k, kind):
     assert torch.equal(i.cpu(), torch.where(vr == float("-inf"), torch.full_like(ir, -1), ir))
 
 
+def test_sim_topk_no_candidates(cuda):
+    """k = 0 asks for nothing and gets empty lists, from the kernel's entry point and from the index."""
+    from generativeaiexamples_amd.index.hbm_index import HBMIndex
+    X = torch.randn(300, 64, device=cuda)
+    v, i = ops.sim_topk(X[:3].bfloat16(), X.bfloat16(), torch.zeros(300, device=cuda), 300, 0)
+    assert v.shape == (3, 0) and v.dtype == torch.float32 and i.shape == (3, 0) and i.dtype == torch.int64
+    index = HBMIndex(64, "cosine", device=cuda, capacity=300)
+    index.add(X)
+    assert index.search_raw(X[:3], 0)[1].shape == (3, 0) and index.search(X[:3], 0) == [[], [], []]
+
+
 def test_embedding_pool_act(cuda):
     torch.manual_seed(10)
     table = torch.randn(1000, 256, device=cuda, dtype=torch.bfloat16)
