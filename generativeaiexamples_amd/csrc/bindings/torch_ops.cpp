@@ -177,7 +177,7 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
       mid = M;
     else if (force == 0)
       mid = gai_gemm_mid_tail(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f,
-                              frag, cur_stream(), &plan);
+                              frag, &plan);
     TORCH_CHECK(mid || force == 0, "gemm: the mid-size kernel needs K % 128 == 0, N % 16 == 0 and aligned operands");
     if (mid) {
       rows = M - mid;
@@ -193,6 +193,19 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
   }
   gai_gemm(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), rows, N, K, ldc, (int)epi, f32 ? 1 : 0,
            (int)force, cur_stream(), bfrag ? 1 : 0);
+}
+
+// rows at the end of gemm's product that the mid-size kernel computes (all, some or none), for the tests of that rule
+int64_t gemm_mid_rows(const Tensor& A, const Tensor& B, const Tensor& C, const optional<Tensor>& bias,
+                      const optional<Tensor>& R, int64_t epi, bool bfrag) {
+  GaiMidPlan plan;
+  const int K = A.size(-1), M = A.numel() / K, N = B.size(0), ldc = epi == 4 || epi == 10 ? N / 2 : N;
+  const int f = C.scalar_type() == at::kFloat ? 1 : 0, frag = bfrag ? 1 : 0;
+  if (gai_gemm_mid_plan(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f, 0, frag,
+                        cur_stream(), &plan))
+    return M;
+  return gai_gemm_mid_tail(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi, f, frag,
+                           &plan);
 }
 
 void attn_prefill(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
@@ -1019,6 +1032,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm);
   m.def("layernorm", &layernorm);
   m.def("rope_kv_write", &rope_kv_write);
+  m.def("gemm_mid_rows", &gemm_mid_rows);
   m.def("gemm", &gemm, pybind11::arg("A"), pybind11::arg("B"), pybind11::arg("C"), pybind11::arg("bias"),
         pybind11::arg("R"), pybind11::arg("epi"), pybind11::arg("force"), pybind11::arg("bfrag") = false);
   m.def("gemm_fp8", &gemm_fp8);

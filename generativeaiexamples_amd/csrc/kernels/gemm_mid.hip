@@ -18,7 +18,12 @@
 //  * MFMA operands swapped (rows = weights), so a lane ends with four consecutive columns of a row: 8-byte stores;
 //  * S > 1: every wave stores its fp32 share (write-through) and draws the (tile, wave) ticket; the one that draws the last
 //    sums the parts in part order - the same result whichever it is - and runs the epilogue. Nobody waits, and a wave that
-//    sees all others done keeps its share in registers.
+//    sees all others done keeps its share in registers;
+//  * ORD, for the last rows of a large product (gai_gemm_mid_tail): a wave takes all of K for half the columns, one sum in
+//    the order of the 256 x 256 kernels, so equal rows give equal bits wherever they stand. 64 x 128 or 128 x 128 tiles:
+//    no weight is fetched twice in a workgroup, A is read from LDS twice as often as with k halves. 1953 rows, N 1024,
+//    residual, row-major | fragment order: K 1024 16.1 | 11.5 us (64 rows), K 4096 44.6 | 30.0 (k halves, 128 x 64 tiles
+//    14.8 | 12.5, 34.7 | 30.0; sharing a fetch between two row halves 18.4 | 13.6, 54.2 | 39.1).
 #include "gai_common.h"
 #include "gai_epilogue.h"
 #include "gai_gemm_mid.h"
@@ -68,11 +73,13 @@ __device__ __forceinline__ void store4(void* C, const bf16* bias, const bf16* R,
   }
 }
 
-template <int MT, int NG, int EPI, bool OUTF32>
+template <int MT, int NG, int EPI, bool OUTF32, bool ORD>
 __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B, void* C,
                                                           const bf16* __restrict__ bias, const bf16* R, int M, int N, int K,
                                                           int ldc, int bfrag, int S, float* ws, int* cnt) {
   constexpr int BM = 16 * MT, BN = 64 * NG, NA = MT / 2, NF = MT / 2 * NG;
+  constexpr int FW = ORD ? NG / 2 : NG, KF = ORD ? 4 : 2, RW = ORD ? MT : MT / 2;  // a wave's columns / 16, k32 fragments of a
+                                                                                   // step, rows / 16 that it stores
   constexpr int DB = NG == 2 ? 3 : 4, U = NG == 2 ? 6 : 4;  // steps the weights are ahead; unrolled steps (even)
   extern __shared__ __attribute__((aligned(16))) char smem[];  // 2 x BM x 256 B; at the end the k halves' exchange
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -81,7 +88,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
   const int part = id / tiles, tile = id - part * tiles;
   const int m0 = tile % tm_n * BM, n0 = tile / tm_n * BN;
   const int nk = K / kBK, k0 = (int)((long long)nk * part / S), n = (int)((long long)nk * (part + 1) / S) - k0;
-  const int g = wid & 3, h = wid >> 2;  // column group, k half
+  const int g = ORD ? wid : wid & 3, h = ORD ? 0 : wid >> 2;  // column group, k half
 
   const bf16* ap[NA];  // row tid / 16 (+ 32 per piece), 16-B piece tid & 15
   int a_wr[NA];
@@ -91,38 +98,38 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
     ap[q] = A + (size_t)min(m0 + row, M - 1) * K + (size_t)k0 * kBK + c * 8;
     a_wr[q] = row * 256 + ((c ^ (row & 15)) << 4);
   }
-  const bf16* bp[NG];
+  const bf16* bp[FW];
 #pragma unroll
-  for (int f = 0; f < NG; ++f) {
-    const int col = n0 + (g * NG + f) * 16;
+  for (int f = 0; f < FW; ++f) {
+    const int col = n0 + (g * FW + f) * 16;
     bp[f] = bfrag ? B + ((size_t)min(col / 16, N / 16 - 1) * (K / 32) + 4 * (size_t)k0 + 2 * h) * 512 + lane * 8
                   : B + (size_t)min(col + (lane & 15), N - 1) * K + (size_t)k0 * kBK + 64 * h + 8 * (lane >> 4);
   }
   const int bstep = bfrag ? 2048 : kBK, bhalf = bfrag ? 512 : 32;
-  bf16x8 ar[NA], br[DB][NG][2];
+  bf16x8 ar[NA], br[DB][FW][KF];
   // past the end the last step is read again (from L2): the count of loads stays what the code says
   auto load_a = [&](int t, bf16x8(&d)[NA]) {
 #pragma unroll
     for (int q = 0; q < NA; ++q) d[q] = load8(ap[q] + (size_t)min(t, n - 1) * kBK);
   };
-  auto load_b = [&](int t, bf16x8(&d)[NG][2]) {
+  auto load_b = [&](int t, bf16x8(&d)[FW][KF]) {
 #pragma unroll
-    for (int f = 0; f < NG; ++f)
+    for (int f = 0; f < FW; ++f)
 #pragma unroll
-      for (int e = 0; e < 2; ++e) d[f][e] = load8(bp[f] + (size_t)min(t, n - 1) * bstep + e * bhalf);
+      for (int e = 0; e < KF; ++e) d[f][e] = load8(bp[f] + (size_t)min(t, n - 1) * bstep + e * bhalf);
   };
   auto put_a = [&](int buf, const bf16x8(&d)[NA]) {
 #pragma unroll
     for (int q = 0; q < NA; ++q) *reinterpret_cast<bf16x8*>(smem + buf * (BM * 256) + a_wr[q]) = d[q];
   };
-  int a_rd[2];  // + 4096 per 16 rows
+  int a_rd[KF];  // + 4096 per 16 rows
 #pragma unroll
-  for (int e = 0; e < 2; ++e) a_rd[e] = (lane & 15) * 256 + (((8 * h + 4 * e + (lane >> 4)) ^ (lane & 15)) << 4);
-  f32x4 acc[MT][NG];
+  for (int e = 0; e < KF; ++e) a_rd[e] = (lane & 15) * 256 + (((8 * h + 4 * e + (lane >> 4)) ^ (lane & 15)) << 4);
+  f32x4 acc[MT][FW];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int f = 0; f < NG; ++f) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int f = 0; f < FW; ++f) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   load_a(0, ar);
 #pragma unroll
@@ -138,14 +145,14 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
       load_a(t + u + 2, ar);
       const char* s = smem + (u & 1) * (BM * 256);
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
+      for (int e = 0; e < KF; ++e) {
         bf16x8 af[MT];
 #pragma unroll
         for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const bf16x8*>(s + a_rd[e] + i * 4096);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-          for (int f = 0; f < NG; ++f)
+          for (int f = 0; f < FW; ++f)
             acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(br[u % DB][f][e], af[i], acc[i][f], 0, 0, 0);
       }
       load_b(t + u + DB, br[u % DB]);
@@ -153,10 +160,15 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
     }
   }
 done:
-  // the k halves: this wave keeps row tiles h * MT / 2 .. of its columns and adds what its partner has of them
-  __syncthreads();
-  f32x4 v[NF];
-  {
+  f32x4 v[NF];  // [RW][FW]
+  if constexpr (ORD) {
+#pragma unroll
+    for (int i = 0; i < RW; ++i)
+#pragma unroll
+      for (int f = 0; f < FW; ++f) v[i * FW + f] = acc[i][f];
+  } else {
+    // the k halves: this wave keeps row tiles h * MT / 2 .. of its columns and adds what its partner has of them
+    __syncthreads();
     f32x4* x = reinterpret_cast<f32x4*>(smem) + g * 2 * NF * 64 + lane;  // [group][half][NF][64]
 #pragma unroll
     for (int i = 0; i < MT / 2; ++i)
@@ -172,7 +184,7 @@ done:
       v[e] = h ? y + v[e] : v[e] + y;  // first half + second half
     }
   }
-  if (S > 1) {
+  if (!ORD && S > 1) {
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(ws, (short)0, 0x7fffffff, 0x00020000);
     auto woff = [&](int p, int e) {
       return (unsigned)__builtin_amdgcn_readfirstlane(((p * tiles + tile) * 8 + wid) * (NF * 1024) + e * 1024);
@@ -213,12 +225,12 @@ done:
   }
   // lane: row m of C, columns n .. n + 3 of each 16 x 16 tile
 #pragma unroll
-  for (int i = 0; i < MT / 2; ++i) {
-    const int m = m0 + 16 * (h * (MT / 2) + i) + (lane & 15);
+  for (int i = 0; i < RW; ++i) {
+    const int m = m0 + 16 * (h * RW + i) + (lane & 15);
     if (m >= M) continue;
-    const int nn = n0 + g * NG * 16;
+    const int nn = n0 + g * FW * 16;
     if constexpr (epi_glu(EPI)) {
-      static_assert(NG == 2, "a gated pair of column tiles belongs to one wave");
+      static_assert(FW == 2, "a gated pair of column tiles belongs to one wave");
       if (nn >= N) continue;
       f32x4 y;
 #pragma unroll
@@ -226,8 +238,8 @@ done:
       store4<EPI_NONE, OUTF32>(C, nullptr, nullptr, ldc, m, nn / 2 + 4 * (lane >> 4), y);
     } else {
 #pragma unroll
-      for (int f = 0; f < NG; ++f)
-        if (nn + 16 * f < N) store4<EPI, OUTF32>(C, bias, R, ldc, m, nn + 16 * f + 4 * (lane >> 4), v[i * NG + f]);
+      for (int f = 0; f < FW; ++f)
+        if (nn + 16 * f < N) store4<EPI, OUTF32>(C, bias, R, ldc, m, nn + 16 * f + 4 * (lane >> 4), v[i * FW + f]);
     }
   }
 }
@@ -283,18 +295,35 @@ double other_cost(int M, int N, int K) {
   return 8.0 + (t1 + 2 * G - 1) / (2 * G) * (K / 64) * 1.0;
 }
 
-template <int MT, int NG, int EPI, bool OUTF32>
+// the ordered form, fitted to 320 shapes of up to 3072 rows (19 of 20 within 15 %)
+double ordered_cost(int M, int N, int K, int mt, int bfrag) {
+  const int items = mid_tiles(M, N, mt, 2), G = mid_cus(), rounds = (items + G - 1) / G;
+  const double fill = std::min(1.0, (double)items / G), step = mt == 4 ? 0.66 + 0.09 * fill : 1.05;
+  const double row = mt == 4 ? 1.63 : 1.35;  // row-major weights
+  return (mt == 4 ? 3.6 : 5.6) + rounds * ((mt == 4 ? 2.5 : 2.1) + K / kBK * step * (bfrag ? 1.0 : row));
+}
+
+// operands of the kernel: whole k steps and column tiles, 4-column loads and stores, 16-byte loads of A and B
+bool mid_fits(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,
+              int out_f32) {
+  if (M < 1 || K % kBK || N % 16 || ldc % 4 || (out_f32 && epi != EPI_NONE)) return false;
+  if (!(epi >= EPI_NONE && epi <= EPI_BIAS_QUICKGELU) && !(epi_glu(epi) && N % 32 == 0)) return false;
+  auto off = [](const void* p, unsigned a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
+  return !(off(A, 16) || off(B, 16) || off(C, out_f32 ? 16 : 8) || off(bias, 8) || off(R, 8));
+}
+
+template <int MT, int NG, int EPI, bool OUTF32, bool ORD = false>
 void launch_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int S,
                 float* ws, int* cnt, hipStream_t st, int bfrag) {
   constexpr int lds = MT * 8192;  // two A buffers; the exchange takes MT * NG * 4096
   static bool once = false;
   if (!once) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mid_kernel<MT, NG, EPI, OUTF32>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mid_kernel<MT, NG, EPI, OUTF32, ORD>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       gai_launch_error(__FILE__, __LINE__, "gemm_mid: LDS size");
     once = true;
   }
-  gemm_mid_kernel<MT, NG, EPI, OUTF32><<<mid_tiles(M, N, MT, NG) * S, 512, lds, st>>>(
+  gemm_mid_kernel<MT, NG, EPI, OUTF32, ORD><<<mid_tiles(M, N, MT, NG) * S, 512, lds, st>>>(
       (const bf16*)A, (const bf16*)B, C, (const bf16*)bias, (const bf16*)R, M, N, K, ldc, bfrag, S, ws, cnt);
   GAI_LAUNCH_CHECK();
 }
@@ -303,15 +332,14 @@ void launch_mid(const void* A, const void* B, void* C, const void* bias, const v
 
 bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K,
                        int ldc, int epi, int out_f32, int force, int bfrag, hipStream_t st, GaiMidPlan* plan) {
-  if (M < 1 || K % kBK || N % 16 || ldc % 4 || (out_f32 && epi != EPI_NONE)) return false;
+  if (!mid_fits(A, B, C, bias, R, M, N, K, ldc, epi, out_f32)) return false;
   if (force == 0 && (M <= 64 || M > 2048 || N < 256)) return false;
-  const bool glu = epi == EPI_SWIGLU || epi == EPI_GEGLU;
-  if ((!(epi >= EPI_NONE && epi <= EPI_BIAS_QUICKGELU) && !glu) || (glu && N % 32)) return false;
-  // 4-column loads and stores, 16-byte loads of the operands
-  auto off = [](const void* p, unsigned a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0; };
-  if (off(A, 16) || off(B, 16) || off(C, out_f32 ? 16 : 8) || off(bias, 8) || off(R, 8)) return false;
+  const bool glu = epi_glu(epi);
   GaiMidPlan best{8, 2, 1, 0, 0.0};
-  if (force >= 1000) {
+  if (force >= 100000) {
+    if (glu) return false;
+    best = {force == 104201 ? 4 : 8, 2, 1, 0, 0.0, true};
+  } else if (force >= 1000) {
     best = {force / 1000, glu ? 2 : force / 100 % 10, std::max(1, std::min(force % 100, K / kBK)), 0, 0.0};
   } else {
     double bc = 1e30;
@@ -347,24 +375,23 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
 
 // The 256 x 256 kernels work in rounds of one tile per CU, 6 us + 1.42 us per 64 of K each (M 16384, N 4096: 28.5, 49, 94 us at
 // K 1024, 2048, 4096; 9 more with a residual), however few tiles the last one has. Its rows go to this kernel where the
-// model says so with 15 % to spare (its own error) and a launch, and the saving is 5 % of the whole. N 1024 with a residual:
-// 18337 rows (288 tiles on 256 CUs) K 1024 56.7 -> 48.3 us, K 4096 167.6 -> 134.2; 18480 rows 58.7 -> 56.8, 171.7 -> 150.8.
+// model says so with 15 % to spare (its own error) and a launch, and the saving is 5 % of the whole. N 1024 with a residual,
+// 18337 rows (288 tiles on 256 CUs): K 1024 57.5 -> 54.4 us, K 4096 167.3 -> 145.0. Over 320 products of 2100 to 60000 rows
+// (N 256 to 9000, K 256 to 14336) the rule splits 127, one of them 3 % slower for it; all in all 3.6 % faster, 3.9 % at best.
 // At N 3072 and 4096, K 1024 the remainder costs as much as the round it saves; after many rounds (Llama-3-8B gate_up at
-// 14500 rows: 25) the tiles have drifted apart and there is no empty round left to save (167.2 ms with, 166.1 without).
+// 14500 rows: 25) the tiles have drifted apart and there is no empty round left to save.
 int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
-                      int epi, int out_f32, int bfrag, hipStream_t st, GaiMidPlan* plan) {
-  if (M <= 2048 || N < 256 || N % 16 || ldc % 8 || K % kBK || K < 256) return 0;
+                      int epi, int out_f32, int bfrag, GaiMidPlan* plan) {
+  if (M <= 2048 || N < 256 || ldc % 8 || K < 256 || epi_glu(epi) || !mid_fits(A, B, C, bias, R, M, N, K, ldc, epi, out_f32))
+    return 0;
+  if ((size_t)M * K * 2 >= (1ull << 31) || (size_t)N * K * 2 >= (1ull << 31)) return 0;  // not the 256 x 256 kernels
   const int G = mid_cus() & ~7, tn = (N + 255) / 256, tm = (M + 255) / 256;
   const long long tiles = (long long)tm * tn;
   if (tiles % G == 0) return 0;
   const int m1 = (int)(tiles / G * G / tn) * 256, m2 = M - m1;  // whole rounds, whole row tiles
   if (m1 <= 0 || m2 <= 0 || m2 > 3072) return 0;
-  auto at = [&](const void* p, size_t row, size_t size) {
-    return p ? reinterpret_cast<const char*>(p) + (size_t)m1 * row * size : nullptr;
-  };
-  if (!gai_gemm_mid_plan(at(A, K, 2), B, at(C, ldc, out_f32 ? 4 : 2), bias, at(R, ldc, 2), m2, N, K, ldc, epi, out_f32, 14, bfrag,
-                         st, plan))
-    return 0;
+  const double c4 = ordered_cost(m2, N, K, 4, bfrag), c8 = ordered_cost(m2, N, K, 8, bfrag);
+  *plan = {c4 <= c8 ? 4 : 8, 2, 1, 0, std::min(c4, c8), true};
   const double round = 6.0 + K / 64 * 1.42 + (R ? 9.0 : 0.0);
   const double saved = round - plan->cost * 1.15 - 3.0;
   return saved > 0.05 * round * ((tiles + G - 1) / G) ? m2 : 0;
@@ -376,8 +403,13 @@ void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const
 #define GAI_MID(MT, NG, E, F32)                                                                         \
   if (p.mt == MT && p.ng == NG)                                                                         \
     return launch_mid<MT, NG, E, F32>(A, B, C, bias, R, M, N, K, ldc, p.parts, ws, cnt, st, bfrag);
+#define GAI_MID_ORD(MT, E, F32)                                                                           \
+  if (p.ordered && p.mt == MT)                                                                            \
+    return launch_mid<MT, 2, E, F32, true>(A, B, C, bias, R, M, N, K, ldc, 1, nullptr, nullptr, st, bfrag);
 #define GAI_MID_EPI(E, F32)         \
   {                                 \
+    GAI_MID_ORD(4, E, F32)          \
+    GAI_MID_ORD(8, E, F32)          \
     GAI_MID(8, 1, E, F32)           \
     GAI_MID(8, 2, E, F32)           \
     GAI_MID(12, 2, E, F32)          \
@@ -405,6 +437,7 @@ void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const
   }
 #undef GAI_MID_GLU
 #undef GAI_MID_EPI
+#undef GAI_MID_ORD
 #undef GAI_MID
   gai_launch_error(__FILE__, __LINE__, "gemm_mid: no kernel for this plan");
 }

@@ -248,29 +248,31 @@ def test_ring_residual_in_place(cuda, M, N, K, bias, kern):
     assert torch.equal(res, y)
 
 
-@pytest.mark.parametrize("M,N,K,act", [(18337, 1024, 1024, "bias_residual"), (16500, 1024, 4096, "bias_residual"),
-                                       (2306, 28672, 1024, "swiglu"), (17000, 1040, 2048, "gelu"), (9000, 2048, 4096, "f32")])
+@pytest.mark.parametrize("M,N,K,act,tail", [
+    (18337, 1024, 1024, "bias_residual", 1953), (16385, 1024, 4096, "bias_residual", 1), (18484, 1024, 4096, "residual", 2100),
+    (13100, 1040, 2048, "gelu", 44), (22000, 720, 1152, "bias", 240), (14500, 1200, 2048, "relu", 1444), (9000, 2048, 4096, "f32", 808),
+    (65600, 256, 512, None, 64), (9300, 1792, 1536, "quick_gelu", 84)])
 @pytest.mark.parametrize("frag", [False, True])
-def test_tail_rows_of_a_large_gemm(cuda, M, N, K, act, frag):
-    """Rows past the last whole round of 256x256 tiles go to the mid-size kernel: against the 256x256 kernel alone, which
-    rounds the same fp32 sums taken in another order (K 2^-24 sum |x w| apart, then at most one bf16 step and, with a
-    residual, one more)."""
+def test_tail_rows_of_a_large_gemm(cuda, M, N, K, act, tail, frag):
+    """Rows past the last whole round of 256x256 tiles go to the mid-size kernel (64- and 128-row tiles), which takes the
+    same sums in the same order: the bits of the 256x256 kernel alone, and of equal rows further up."""
     torch.manual_seed(M + N)
     x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    x[-5:] = x[:5] if tail >= 5 else x[-5:]
     w = (torch.randn(N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
-    b = torch.randn(N, device=cuda, dtype=torch.bfloat16) if act in ("gelu", "bias_residual") else None
-    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16) if act == "bias_residual" else None
-    a = act if act in ("gelu", "swiglu") else None
+    b = torch.randn(N, device=cuda, dtype=torch.bfloat16) if act in ("gelu", "bias", "relu", "quick_gelu", "bias_residual") else None
+    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16) if act in ("residual", "bias_residual") else None
+    if res is not None:
+        res[-5:] = res[:5]
     dt = torch.float32 if act == "f32" else torch.bfloat16
-    one = _run(x, w, b, res, a, dt, force=10)
     epi = 0 if act == "f32" else ops.EPI[act]
-    out = torch.full_like(one, float("nan"))
-    ops.native().gemm(x, ops.shuffle_fragments(w) if frag else w, out, b, res, epi, 0, frag)
-    assert not torch.isnan(out).any(), "unwritten rows"
-    # |x| . |w| <= K E|x| E|w| (1 + small): 0.64 sqrt(K); the gates have slopes below 1.13 and multiply by |up| < 6
-    e = K * 2.0 ** -24 * 0.75 * math.sqrt(K) * (8 if act == "swiglu" else 1.13)
-    d = (out.float() - one.float()).abs()
-    assert (d <= 2 * e + (0 if act == "f32" else 2.0 ** -6) * one.float().abs().clamp_min(1 if res is not None else 0)).all(), d.max()
+    one, out = (torch.full((M, N), float("nan"), device=cuda, dtype=dt) for _ in range(2))
+    ops.native().gemm(x, w, one, b, res, epi, KERNELS["w4r"])
+    wf = ops.shuffle_fragments(w) if frag else w
+    assert ops.native().gemm_mid_rows(x, wf, out, b, res, epi, frag) == tail
+    ops.native().gemm(x, wf, out, b, res, epi, 0, frag)
+    assert torch.equal(out, one)
+    assert tail < 5 or torch.equal(out[-5:], out[:5])
 
 
 @pytest.mark.parametrize("sizes", [[300, 0, 1, 700, 256, 0, 257, 40], [0, 0, 5], [1025], [0, 513, 255, 0]])
