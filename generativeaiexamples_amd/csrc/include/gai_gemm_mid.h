@@ -7,14 +7,17 @@ struct GaiMidPlan {
   int mt, ng, parts;  // rows / 16 and columns / 64 of a workgroup's tile, parts of K
   size_t ws_floats;   // fp32 workspace of the parts (0 for one part)
   double cost;        // modelled time, us
+  int tickets = 0;    // of the parts: ints, 0 before a launch and 0 again after it
   bool ordered = false;  // every output is one sum over K in order, as in the 256 x 256 kernels (mt 4 or 8, one part)
 };
 // force 0: false where another kernel is expected to be faster; 14: this kernel, plan chosen; else 1000 mt + 100 ng +
 // parts, 104201 / 108201: the ordered form
 bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K,
-                       int ldc, int epi, int out_f32, int force, int bfrag, hipStream_t st, GaiMidPlan* plan);
+                       int ldc, int epi, int out_f32, int force, int bfrag, GaiMidPlan* plan);
+// tickets: plan.tickets zeros of the caller's, or null for the stream's own, which a captured launch must not use: its replays
+// may run beside other launches on that stream
 void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,
-                  int out_f32, const GaiMidPlan& plan, float* ws, hipStream_t st, int bfrag);
+                  int out_f32, const GaiMidPlan& plan, float* ws, int* tickets, hipStream_t st, int bfrag);
 // rows at the end of a large product that this kernel should compute instead of the 256 x 256 kernels' last, partly filled
 // round of tiles (0: none), with the same sums; *plan is for those rows
 int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K, int ldc,

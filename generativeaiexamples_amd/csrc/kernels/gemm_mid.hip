@@ -257,6 +257,10 @@ int mid_cus() {
 
 int mid_tiles(int M, int N, int mt, int ng) { return ((M + 16 * mt - 1) / (16 * mt)) * ((N + 64 * ng - 1) / (64 * ng)); }
 
+size_t part_bytes(int M, int N, int mt, int ng, int S) {
+  return (size_t)mid_tiles(M, N, mt, ng) * S * 8 * (mt / 2 * ng) * 1024;
+}
+
 // Tickets of a (device, stream): kCnt zeros, zero again after every launch. Never freed or grown: at most 64 KB a stream.
 constexpr int kCnt = 16384;
 int* mid_counters(hipStream_t st) {
@@ -274,6 +278,11 @@ int* mid_counters(hipStream_t st) {
     }
   }
   return c;
+}
+
+// 32-bit workspace offsets, and the tickets of a stream
+bool parts_fit(int M, int N, int mt, int ng, int S) {
+  return mid_tiles(M, N, mt, ng) * 8 <= kCnt && part_bytes(M, N, mt, ng, S) < (1ull << 31);
 }
 
 // Modelled times in us, fitted to eleven N x K from 1024 x 1024 to 28672 x 4096 at 80 - 2048 rows (most within 15 %).
@@ -331,14 +340,14 @@ void launch_mid(const void* A, const void* B, void* C, const void* bias, const v
 }  // namespace
 
 bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K,
-                       int ldc, int epi, int out_f32, int force, int bfrag, hipStream_t st, GaiMidPlan* plan) {
+                       int ldc, int epi, int out_f32, int force, int bfrag, GaiMidPlan* plan) {
   if (!mid_fits(A, B, C, bias, R, M, N, K, ldc, epi, out_f32)) return false;
   if (force == 0 && (M <= 64 || M > 2048 || N < 256)) return false;
   const bool glu = epi_glu(epi);
   GaiMidPlan best{8, 2, 1, 0, 0.0};
   if (force >= 100000) {
     if (glu) return false;
-    best = {force == 104201 ? 4 : 8, 2, 1, 0, 0.0, true};
+    best = {force == 104201 ? 4 : 8, 2, 1, 0, 0.0, 0, true};
   } else if (force >= 1000) {
     best = {force / 1000, glu ? 2 : force / 100 % 10, std::max(1, std::min(force % 100, K / kBK)), 0, 0.0};
   } else {
@@ -346,7 +355,7 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
     for (int v = glu ? 1 : 0; v < 3; ++v) {
       const int mt = v == 2 ? 12 : 8, ng = v == 0 ? 1 : 2;
       for (int S = 1; S <= std::min(16, std::max(1, K / kBK / 4)); ++S) {
-        if (S > 1 && mid_tiles(M, N, mt, ng) * 8 > kCnt) break;
+        if (S > 1 && !parts_fit(M, N, mt, ng, S)) break;
         const double c = mid_cost(M, N, K, mt, ng, S, bfrag);
         if (c < bc) {
           bc = c;
@@ -356,18 +365,10 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
     }
     if (force == 0 && bc >= other_cost(M, N, K)) return false;
   }
+  if (best.parts > 1 && !parts_fit(M, N, best.mt, best.ng, best.parts)) best.parts = 1;
   if (best.parts > 1) {
-    // a captured launch may replay beside another one on this stream: tickets cannot be shared with it
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const int tiles = mid_tiles(M, N, best.mt, best.ng);
-    const size_t bytes = (size_t)tiles * best.parts * 8 * (best.mt / 2 * best.ng) * 1024;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone || bytes >= (1ull << 31) ||
-        tiles * 8 > kCnt || !mid_counters(st))
-      best.parts = 1;
-    else
-      best.ws_floats = bytes / 4;
-    if (best.parts == 1) best.cost = mid_cost(M, N, K, best.mt, best.ng, 1, bfrag);
-    if (best.parts == 1 && force == 0 && best.cost >= other_cost(M, N, K)) return false;
+    best.ws_floats = part_bytes(M, N, best.mt, best.ng, best.parts) / 4;
+    best.tickets = 8 * mid_tiles(M, N, best.mt, best.ng);
   }
   *plan = best;
   return true;
@@ -391,15 +392,16 @@ int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* b
   const int m1 = (int)(tiles / G * G / tn) * 256, m2 = M - m1;  // whole rounds, whole row tiles
   if (m1 <= 0 || m2 <= 0 || m2 > 3072) return 0;
   const double c4 = ordered_cost(m2, N, K, 4, bfrag), c8 = ordered_cost(m2, N, K, 8, bfrag);
-  *plan = {c4 <= c8 ? 4 : 8, 2, 1, 0, std::min(c4, c8), true};
+  *plan = {c4 <= c8 ? 4 : 8, 2, 1, 0, std::min(c4, c8), 0, true};
   const double round = 6.0 + K / 64 * 1.42 + (R ? 9.0 : 0.0);
   const double saved = round - plan->cost * 1.15 - 3.0;
   return saved > 0.05 * round * ((tiles + G - 1) / G) ? m2 : 0;
 }
 
 void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,
-                  int out_f32, const GaiMidPlan& p, float* ws, hipStream_t st, int bfrag) {
-  int* cnt = p.parts > 1 ? mid_counters(st) : nullptr;
+                  int out_f32, const GaiMidPlan& p, float* ws, int* tickets, hipStream_t st, int bfrag) {
+  int* cnt = p.parts == 1 ? nullptr : tickets ? tickets : mid_counters(st);
+  if (p.parts > 1 && !(cnt && ws)) gai_launch_error(__FILE__, __LINE__, "gemm_mid: no workspace for the parts of K");
 #define GAI_MID(MT, NG, E, F32)                                                                         \
   if (p.mt == MT && p.ng == NG)                                                                         \
     return launch_mid<MT, NG, E, F32>(A, B, C, bias, R, M, N, K, ldc, p.parts, ws, cnt, st, bfrag);

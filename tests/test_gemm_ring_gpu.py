@@ -9,6 +9,7 @@ import torch
 
 from generativeaiexamples_amd import ops
 from generativeaiexamples_amd.ops import reference as ref
+from generativeaiexamples_amd.utils.graphs import hip_graph_capture
 
 pytestmark = pytest.mark.gpu
 # force codes in gai_gemm: persistent 4-wave ring (tile walk per CU), persistent full-line double-unit kernel, and
@@ -216,6 +217,42 @@ def test_mid_gemm(cuda, M, N, K, act, plan):
     for _ in range(3):
         ops.native().gemm(x, f, out, bias, res, {"f32": 0, None: 0}.get(act, ops.EPI.get(act, 0)), plan, True)
         assert torch.equal(out, y)
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 1024, 4096), (192, 1024, 4096), (1536, 1024, 4096), (300, 2048, 5632)])
+def test_mid_gemm_captured_equals_eager(cuda, M, N, K):
+    """A captured product with parts of K takes the eager one's plan, sums and bits, whatever runs between the replays or
+    beside them on the capture stream and on another one."""
+    torch.manual_seed(M + K)
+    x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    w1, w2 = (torch.randn(n, k, device=cuda).div_(math.sqrt(k)).to(torch.bfloat16) for n, k in ((N, K), (K, N)))
+    gemm = ops.native().gemm
+
+    def chain(out, mid):
+        gemm(x, w1, mid, None, None, 0, 0)
+        gemm(mid, w2, out, None, x, ops.EPI["residual"], 0)
+        gemm(out, w1, mid, None, None, 0, 0)
+
+    want, mid = torch.empty_like(x), torch.empty(M, N, device=cuda, dtype=torch.bfloat16)
+    assert ops.native().gemm_mid_rows(x, w1, mid, None, None, 0, False) == M
+    chain(want, mid)
+    want_mid = mid.clone()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    out, gmid = torch.empty_like(x), torch.empty_like(mid)
+    s.wait_stream(torch.cuda.current_stream())
+    with hip_graph_capture(g, s):
+        chain(out, gmid)
+    for _ in range(4):
+        for t in (out, gmid):
+            t.fill_(float("nan"))
+        e, emid = torch.empty_like(x), torch.empty_like(mid)
+        s.wait_stream(torch.cuda.current_stream())
+        g.replay()
+        with torch.cuda.stream(s):
+            chain(e, emid)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(gmid, want_mid)
+        assert torch.equal(e, want) and torch.equal(emid, want_mid)
 
 
 def test_gelu_whole_range(cuda):
