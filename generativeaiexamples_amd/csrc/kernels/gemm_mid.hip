@@ -285,24 +285,67 @@ bool parts_fit(int M, int N, int mt, int ng, int S) {
   return mid_tiles(M, N, mt, ng) * 8 <= kCnt && part_bytes(M, N, mt, ng, S) < (1ull << 31);
 }
 
-// Modelled times in us, fitted to eleven N x K from 1024 x 1024 to 28672 x 4096 at 80 - 2048 rows (most within 15 %).
-// This kernel: launch, first loads and epilogue; K steps of a workgroup (slower when the chip is full) or the weights at the
-// rate HBM gives; storing and summing the parts.
-double mid_cost(int M, int N, int K, int mt, int ng, int S, int bfrag) {
+// Modelled times in us, fitted to 1376 products of 65 to 2048 rows, N 256 to 32000, K 128 to 16384, every epilogue and both
+// weight layouts, each with the kernels below and with some 13 plans of this one (19 of 20 plans within 15 %, 9 of 10 of the
+// others). A product is taken where the model says 10 % less (25 % at K >= 8192): two of those taken are then slower than the
+// kernel replaced, by 4 %, and the choice as a whole is 1.6 % above the best one; of 719 products not used for the fit, 6
+// above 10 us measured 4 to 12 % slower. At equality 22 of the 1376 are slower, by up to 19 %; the first form of the model, without the bytes of the parts, the epilogues and the
+// rounds of short K, lost up to 54 % (1535 x 2176 x 384: 9.4 -> 14.4 us; with 150 MB of parts 1536 x 11264 x 2048: 90 -> 258).
+struct MidFit {
+  double base, round, alone, full;  // launch; of a round of workgroups; of a 128-deep K step, few workgroups / full chip
+  double weights, row_major;        // GB/s / 1000 of the weights; a step's factor for row-major ones
+  double part0, part1, parts;       // parts of K: once, each, GB/s / 1000 of the sums written and read
+  double out, bias, gelu;           // GB/s / 1000 of residual and result; epilogues
+};
+constexpr MidFit kFit[3] = {{4.2, 0.4, 0.62, 0.66, 3.6, 1.30, 1.0, 0.73, 6.3, 2.5, 0.6, 0.9},    // 128 x 64
+                            {3.5, 2.4, 0.89, 0.97, 4.4, 1.39, 1.5, 0.85, 6.8, 3.0, 1.35, 1.8},   // 128 x 128
+                            {3.3, 3.6, 1.33, 1.36, 4.1, 1.22, 1.4, 1.13, 7.4, 3.3, 1.7, 2.8}};   // 192 x 128
+constexpr double kTicketFill = 1.6;  // a captured launch clears its tickets: counted always, the plan is the same
+
+// MB written and read by the epilogue; 0 none, 1 bias / residual, 2 GELU and the like
+double out_mb(int M, int N, int epi) {
+  const bool res = epi == EPI_RESIDUAL || epi == EPI_BIAS_RESIDUAL;
+  return (double)M * (epi_glu(epi) ? N / 2 : N) * (res ? 4 : 2) / 1e6;
+}
+int epi_class(int epi) {
+  return epi == EPI_NONE || epi_glu(epi) ? 0 : epi == EPI_BIAS_GELU || epi == EPI_BIAS_QUICKGELU ? 2 : 1;
+}
+
+double mid_cost(int M, int N, int K, int epi, int mt, int ng, int S, int bfrag) {
+  const MidFit& f = kFit[mt == 12 ? 2 : ng - 1];
   const int items = mid_tiles(M, N, mt, ng) * S, steps = (K / kBK + S - 1) / S, G = mid_cus(), rounds = (items + G - 1) / G;
-  const double base = mt == 12 ? 8.6 : ng == 2 ? 6.3 : 4.7, alone = mt == 12 ? 1.35 : ng == 2 ? 1.0 : 0.71;
-  const double full = mt == 12 ? 1.65 : ng == 2 ? 1.2 : 0.73, fill = std::min(1.0, (double)items / G);
-  const double step = (alone + (full - alone) * fill) * (bfrag ? 1.0 : 1.17);
-  return base + std::max(rounds * steps * step, (double)N * K * 2 / 5.0e6) + (S > 1 ? 2.3 + 1.2 * S : 0.0);
+  const double fill = std::min(1.0, (double)items / G), step = (f.alone + (f.full - f.alone) * fill) * (bfrag ? 1.0 : f.row_major);
+  const int ec = epi_class(epi);
+  return f.base + std::max(rounds * (f.round + steps * step), (double)N * K * 2 / 1e6 / f.weights) + out_mb(M, N, epi) / f.out +
+         (ec == 1 ? f.bias : ec == 2 ? f.gelu : 0.0) +
+         (S > 1 ? f.part0 + f.part1 * S + 2 * part_bytes(M, N, mt, ng, S) / 1e6 / f.parts + kTicketFill : 0.0);
 }
-// the kernels of gemm_impl.h, with its own rules: skinny (M <= 128), 128 x 128 tiles, 256 x 256 tiles, stream-K
-double other_cost(int M, int N, int K) {
-  if (M <= 128 && K % 256 == 0) return K <= 1024 && N <= 4096 ? 0.0 : 1e9;
-  const int G = mid_cus() & ~7, t1 = ((M + 127) / 128) * ((N + 127) / 128), t2 = ((M + 255) / 256) * ((N + 255) / 256);
-  if (M >= 256 && N >= 256 && 2 * t2 >= G) return 12.0 + (t2 + G - 1) / G * (K / 64) * (t2 < 200 ? 1.15 : 1.4);
-  if (M >= 256 && N >= 256 && K >= 8192) return 70.0 + 0.05 * M;
-  return 8.0 + (t1 + 2 * G - 1) / (2 * G) * (K / 64) * 1.0;
+// the kernels of gemm_impl.h, by its own rules: skinny, stream-K, 256 x 256 tiles, 128 x 128 tiles
+double other_cost(int M, int N, int K, int epi) {
+  const int G = mid_cus() & ~7, ec = epi_class(epi), kt = K / 64;
+  const int t1 = ((M + 127) / 128) * ((N + 127) / 128), t2 = ((M + 255) / 256) * ((N + 255) / 256), r2 = (t2 + G - 1) / G;
+  const double wmb = (double)N * K * 2 / 1e6, out = out_mb(M, N, epi);
+  if (M <= 128 && K % 256 == 0) {
+    const bool two = epi_glu(epi) || N / 32 >= 512;
+    const int r = ((two ? (N + 31) / 32 : (N + 15) / 16) + G - 1) / G;
+    return two ? 0.9 + std::max(r * (2.0 + K / 256 * (1.38 + 0.14 * M / 16)), wmb / 3.15) + out / 1.3 + (ec ? 0.7 : 0.0)
+               : 3.0 + std::max(r * (0.14 + K / 256 * (0.89 + 0.16 * M / 16)), wmb / 5.0) + out / 4.2;
+  }
+  if (N >= 256 && K >= 192 && M >= 256) {
+    if (K >= 8192 && 2 * t2 < G)  // a tile's sums of G / t2 workgroups are added by one
+      return 25.7 + 2.05 * t2 * kt / G + 2.04 * G / t2 + 9.2 * std::max(0.0, 1.0 - t2 * kt / (20.0 * G));
+    if (2 * t2 >= G) {
+      const double fill = std::min(1.0, (double)t2 / G);
+      return N >= 16384 ? 4.9 + r2 * (2.3 + kt * (1.30 + 0.06 * fill)) + out / 9.5 + (ec == 2 ? 10.0 : ec ? 2.5 : 0.0)
+                        : 6.7 + r2 * kt * (0.93 + 0.41 * fill) + out / 7.4 + (ec == 2 ? 6.1 : ec ? 0.5 : 0.0);
+    }
+  }
+  const double fill = (double)t1 / G, step = 0.65 + 0.11 * std::min(1.0, fill) + 0.13 * std::min(1.0, std::max(0.0, fill - 1.0)) +
+                                             0.25 * std::min(1.0, wmb / 64);
+  return 3.6 + (t1 + 2 * G - 1) / (2 * G) * (0.73 + kt * step) + out / 4.0 + (ec == 2 ? 10.1 : ec ? 7.0 : 0.0);
 }
+// (the 256 x 256 kernels at K >= 8192 are up to a fifth faster than their model where the tiles divide the chip evenly)
+double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.25 : 1.1; }
 
 // the ordered form, fitted to 320 shapes of up to 3072 rows (19 of 20 within 15 %)
 double ordered_cost(int M, int N, int K, int mt, int bfrag) {
@@ -356,14 +399,14 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
       const int mt = v == 2 ? 12 : 8, ng = v == 0 ? 1 : 2;
       for (int S = 1; S <= std::min(16, std::max(1, K / kBK / 4)); ++S) {
         if (S > 1 && !parts_fit(M, N, mt, ng, S)) break;
-        const double c = mid_cost(M, N, K, mt, ng, S, bfrag);
+        const double c = mid_cost(M, N, K, epi, mt, ng, S, bfrag);
         if (c < bc) {
           bc = c;
           best = {mt, ng, S, 0, c};
         }
       }
     }
-    if (force == 0 && bc >= other_cost(M, N, K)) return false;
+    if (force == 0 && bc * margin(M, K) >= other_cost(M, N, K, epi)) return false;
   }
   if (best.parts > 1 && !parts_fit(M, N, best.mt, best.ng, best.parts)) best.parts = 1;
   if (best.parts > 1) {

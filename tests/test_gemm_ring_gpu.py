@@ -219,6 +219,23 @@ def test_mid_gemm(cuda, M, N, K, act, plan):
         assert torch.equal(out, y)
 
 
+@pytest.mark.parametrize("M,N,K,act,frag,mid", [
+    # the kernels it would replace are the faster ones: short K, sums of the parts past the caches, K deep and tiles even
+    (1535, 2176, 384, None, False, False), (2048, 4096, 512, None, True, False), (252, 13936, 128, None, False, False),
+    (1536, 11264, 2048, "swiglu", False, False),
+    (2048, 4096, 14336, "residual", True, False), (1024, 4096, 14336, "residual", True, False), (128, 1024, 1024, "bias", False, False),
+    # and here they are not
+    (187, 4096, 14336, "residual", True, True), (65, 1024, 4096, "bias", False, True), (1024, 1024, 1024, "bias_residual", False, True), (768, 6144, 4096, None, True, True),
+    (2048, 2048, 2048, "residual", False, True)])
+def test_mid_gemm_choice(cuda, M, N, K, act, frag, mid):
+    """Where products of 65 - 2048 rows go, at shapes measured with both kernels (the model's comment has the sweep)."""
+    x, w = (torch.empty(n, K, device=cuda, dtype=torch.bfloat16) for n in (M, N))
+    b = torch.empty(N, device=cuda, dtype=torch.bfloat16) if act in ("bias", "bias_residual") else None
+    out = torch.empty(M, N // 2 if act == "swiglu" else N, device=cuda, dtype=torch.bfloat16)
+    res = out if act in ("residual", "bias_residual") else None
+    assert ops.native().gemm_mid_rows(x, w, out, b, res, ops.EPI[act], frag) == (M if mid else 0)
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 1024, 4096), (192, 1024, 4096), (1536, 1024, 4096), (300, 2048, 5632)])
 def test_mid_gemm_captured_equals_eager(cuda, M, N, K):
     """A captured product with parts of K takes the eager one's plan, sums and bits, whatever runs between the replays or
