@@ -6,8 +6,11 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include <map>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 
 #include "gai_gemm_grouped.h"
 #include "gai_gemm_mid.h"
@@ -150,7 +153,32 @@ static void check_epi_operands(int64_t epi, const optional<Tensor>& bias, const 
 // true also where the question cannot be answered: a launch that shares nothing with others is right in any case
 bool capturing() {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(cur_stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(cur_stream(), &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // or the next launch check reports it
+  return true;
+}
+
+// Scratch of a gemm_mid plan with several parts of K: their sums, and tickets. The eager launches of a (device, stream) share
+// its tickets, 64 KB kept for good (each launch leaves zeros behind); a captured launch has its own, cleared by every replay.
+// All of it is the allocator's, which takes care of captures in other threads. False where it has no memory: the launch then
+// takes one part, which needs none.
+bool mid_scratch(const GaiMidPlan& plan, const at::TensorOptions& o, Tensor& ws, Tensor& tickets) {
+  static std::mutex mu;
+  static auto* kept = new std::map<std::pair<int, hipStream_t>, Tensor>;  // (not destroyed: the device may be gone by then)
+  try {
+    ws = at::empty({(int64_t)plan.ws_floats}, o.dtype(at::kFloat));
+    if (capturing()) {
+      tickets = at::zeros({plan.tickets}, o.dtype(at::kInt));
+    } else {
+      std::lock_guard<std::mutex> lock(mu);
+      Tensor& t = (*kept)[{o.device().index(), cur_stream()}];
+      if (!t.defined()) t = at::zeros({kGaiMidTickets}, o.dtype(at::kInt));
+      tickets = t;
+    }
+    return true;
+  } catch (const c10::OutOfMemoryError&) {
+    return false;
+  }
 }
 
 void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& bias, const optional<Tensor>& R,
@@ -188,15 +216,12 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
     if (mid) {
       rows = M - mid;
       Tensor ws, tickets;
-      if (plan.parts > 1) {
-        ws = at::empty({(int64_t)plan.ws_floats}, A.options().dtype(at::kFloat));
-        if (capturing()) tickets = at::zeros({plan.tickets}, A.options().dtype(at::kInt));  // cleared by every replay
-      }
+      if (plan.parts > 1 && !mid_scratch(plan, A.options(), ws, tickets)) plan.parts = 1;
       const void* r = opt_ptr(R);
       gai_gemm_mid(static_cast<char*>(A.data_ptr()) + (size_t)rows * K * 2, B.data_ptr(),
                    static_cast<char*>(C.data_ptr()) + (size_t)rows * ldc * (f32 ? 4 : 2), opt_ptr(bias),
                    r ? static_cast<const char*>(r) + (size_t)rows * ldc * 2 : nullptr, mid, N, K, ldc, (int)epi, f, plan,
-                   ws.defined() ? ws.data_ptr<float>() : nullptr, tickets.defined() ? tickets.data_ptr<int>() : nullptr,
+                   plan.parts > 1 ? ws.data_ptr<float>() : nullptr, plan.parts > 1 ? tickets.data_ptr<int>() : nullptr,
                    cur_stream(), frag);
       if (!rows) return;
     }

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+constexpr int kGaiMidTickets = 16384;  // the most that a plan asks for
 struct GaiMidPlan {
   int mt, ng, parts;  // rows / 16 and columns / 64 of a workgroup's tile, parts of K
   size_t ws_floats;   // fp32 workspace of the parts (0 for one part)
@@ -14,8 +15,8 @@ struct GaiMidPlan {
 // parts, 104201 / 108201: the ordered form
 bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K,
                        int ldc, int epi, int out_f32, int force, int bfrag, GaiMidPlan* plan);
-// tickets: plan.tickets zeros of the caller's, or null for the stream's own, which a captured launch must not use: its replays
-// may run beside other launches on that stream
+// ws and tickets of the plan for more than one part; any plan may be run with parts = 1 instead. Launches that may run side by
+// side (streams, replays of captured ones) need tickets of their own.
 void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,
                   int out_f32, const GaiMidPlan& plan, float* ws, int* tickets, hipStream_t st, int bfrag);
 // rows at the end of a large product that this kernel should compute instead of the 256 x 256 kernels' last, partly filled

@@ -30,9 +30,6 @@
 #include "gai_kernels.h"
 
 #include <algorithm>
-#include <map>
-#include <mutex>
-#include <utility>
 
 using namespace gai;
 
@@ -261,28 +258,9 @@ size_t part_bytes(int M, int N, int mt, int ng, int S) {
   return (size_t)mid_tiles(M, N, mt, ng) * S * 8 * (mt / 2 * ng) * 1024;
 }
 
-// Tickets of a (device, stream): kCnt zeros, zero again after every launch. Never freed or grown: at most 64 KB a stream.
-constexpr int kCnt = 16384;
-int* mid_counters(hipStream_t st) {
-  static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, int*> pool;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lk(mu);
-  int*& c = pool[{dev, st}];
-  if (!c) {
-    if (hipMalloc(&c, kCnt * sizeof(int)) != hipSuccess) return c = nullptr;
-    if (hipMemsetAsync(c, 0, kCnt * sizeof(int), st) != hipSuccess) {
-      (void)hipFree(c);
-      c = nullptr;
-    }
-  }
-  return c;
-}
-
-// 32-bit workspace offsets, and the tickets of a stream
+// 32-bit workspace offsets, and the caller's tickets
 bool parts_fit(int M, int N, int mt, int ng, int S) {
-  return mid_tiles(M, N, mt, ng) * 8 <= kCnt && part_bytes(M, N, mt, ng, S) < (1ull << 31);
+  return mid_tiles(M, N, mt, ng) * 8 <= kGaiMidTickets && part_bytes(M, N, mt, ng, S) < (1ull << 31);
 }
 
 // Modelled times in us, fitted to 1376 products of 65 to 2048 rows, N 256 to 32000, K 128 to 16384, every epilogue and both
@@ -443,11 +421,10 @@ int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* b
 
 void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,
                   int out_f32, const GaiMidPlan& p, float* ws, int* tickets, hipStream_t st, int bfrag) {
-  int* cnt = p.parts == 1 ? nullptr : tickets ? tickets : mid_counters(st);
-  if (p.parts > 1 && !(cnt && ws)) gai_launch_error(__FILE__, __LINE__, "gemm_mid: no workspace for the parts of K");
+  if (p.parts > 1 && !(tickets && ws)) gai_launch_error(__FILE__, __LINE__, "gemm_mid: no workspace for the parts of K");
 #define GAI_MID(MT, NG, E, F32)                                                                         \
   if (p.mt == MT && p.ng == NG)                                                                         \
-    return launch_mid<MT, NG, E, F32>(A, B, C, bias, R, M, N, K, ldc, p.parts, ws, cnt, st, bfrag);
+    return launch_mid<MT, NG, E, F32>(A, B, C, bias, R, M, N, K, ldc, p.parts, ws, tickets, st, bfrag);
 #define GAI_MID_ORD(MT, E, F32)                                                                           \
   if (p.ordered && p.mt == MT)                                                                            \
     return launch_mid<MT, 2, E, F32, true>(A, B, C, bias, R, M, N, K, ldc, 1, nullptr, nullptr, st, bfrag);

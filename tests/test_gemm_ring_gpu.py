@@ -272,6 +272,29 @@ def test_mid_gemm_captured_equals_eager(cuda, M, N, K):
         assert torch.equal(e, want) and torch.equal(emid, want_mid)
 
 
+def test_mid_gemm_without_memory_for_its_parts(cuda):
+    """A full card: the product takes one part of K, which needs no workspace, and nothing is left to fail later."""
+    M, N, K = 512, 2048, 4096
+    x, w = torch.randn(M, K, device=cuda).bfloat16(), torch.randn(N, K, device=cuda).div_(64).bfloat16()
+    one, out = (torch.empty(M, N, device=cuda, dtype=torch.bfloat16) for _ in range(2))
+    ops.native().gemm(x, w, one, None, None, 0, 8101)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total, held = torch.cuda.get_device_properties(0).total_memory, []
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(32 << 20, device=cuda, dtype=torch.uint8))
+        ops.native().gemm(x, w, out, None, None, 0, 8116)   # 64 MB of partial sums
+        assert torch.equal(out, one)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    out.fill_(float("nan"))
+    ops.native().gemm(x, w, out, None, None, 0, 8116)
+    assert (out.float() - one.float()).abs().max() <= 2.0 ** -6 * one.float().abs().max()
+
+
 def test_gelu_whole_range(cuda):
     """Every bf16 value through the erf GELU: the 1.5e-7 of the erfc formula (7.1.26) times |x| / 2 and one bf16 rounding;
     the limits at the infinities, NaN kept. The formula is a1 t exp(-z^2) far out, 0.778 / z against erfc's 0.564 / z, so a
