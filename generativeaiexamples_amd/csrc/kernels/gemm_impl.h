@@ -1365,12 +1365,12 @@ void launch_w4p(const void* A, const void* B, void* C, const void* bias, const v
                 hipStream_t st) {
   const int tiles = ((M + LBM - 1) / LBM) * ((N + LBN - 1) / LBN);
   static int ncu = 0;
-  if (!ncu) {
+  if (!ncu) {  // the kernel's limit before ncu, which tells other threads that both are there
+    set_max_lds(gemm_w4p_kernel<EPI, OUTF32>);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
       gai_launch_error(__FILE__, __LINE__, "gemm_w4p: cannot query the CU count");
-    set_max_lds(gemm_w4p_kernel<EPI, OUTF32>);
   }
   // one workgroup per CU (160 KiB LDS each), a multiple of 8 so that walk index % 8 stays the XCD
   const int grid = tiles <= ncu ? tiles : (ncu & ~7);
@@ -1400,13 +1400,13 @@ template <int EPI, bool OUTF32>
 void launch_w4d(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
                 hipStream_t st, RopeKvArgs rk, int rows, int bfrag) {
   static int ncu = 0;
-  if (!ncu) {
+  if (!ncu) {  // the kernel's limit before ncu, which tells other threads that both are there
+    set_max_lds(gemm_w4d_kernel<EPI, OUTF32>);
+    set_max_lds(gemm_w4d_kernel<EPI, OUTF32, 0, 6>);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
       gai_launch_error(__FILE__, __LINE__, "gemm_w4d: cannot query the CU count");
-    set_max_lds(gemm_w4d_kernel<EPI, OUTF32>);
-    set_max_lds(gemm_w4d_kernel<EPI, OUTF32, 0, 6>);
   }
   const int bm = rows ? rows : w4d_rows(M, N, ncu);
   const int tiles = ((M + bm - 1) / bm) * ((N + LBN - 1) / LBN);
@@ -1427,12 +1427,12 @@ void launch_w4r(const void* A, const void* B, void* C, const void* bias, const v
                 hipStream_t st, int bfrag) {
   const int tiles = ((M + LBM - 1) / LBM) * ((N + LBN - 1) / LBN);
   static int ncu = 0;
-  if (!ncu) {
+  if (!ncu) {  // the kernel's limit before ncu, which tells other threads that both are there
+    set_max_lds(gemm_w4r_kernel<EPI, OUTF32>);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
       gai_launch_error(__FILE__, __LINE__, "gemm_w4r: cannot query the CU count");
-    set_max_lds(gemm_w4r_kernel<EPI, OUTF32>);
   }
   const int grid = tiles <= ncu ? tiles : (ncu & ~7);
   gemm_w4r_kernel<EPI, OUTF32><<<grid, 256, 5 * kPart, st>>>((const bf16*)A, (const bf16*)B, C, (const bf16*)bias,
@@ -1440,25 +1440,33 @@ void launch_w4r(const void* A, const void* B, void* C, const void* bias, const v
   GAI_LAUNCH_CHECK();
 }
 
+int sk_grid() {
+  static int ncu = 0;
+  if (!ncu) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
+      gai_launch_error(__FILE__, __LINE__, "gemm_w4r: cannot query the CU count");
+  }
+  return ncu & ~7;
+}
+
 // Every expert's product in one persistent launch (WALK 3). The 256-row tiles of all experts share the rounds: 8 experts of
 // about 750 rows at N 28672 are 3 x 112 tiles each, 1.31 rounds of 256 CUs run as 2 when each expert is launched by itself,
-// and 12.3 run as 13 together. Both products
-// of a layer (N 28672, K 4096 with SwiGLU, and back) 2541 -> 1872 us, the host's wait for the row counts included.
+// and 12.3 run as 13 together. Both products of a layer (N 28672, K 4096 with SwiGLU, and back) 2541 -> 1872 us, the host's
+// wait for the row counts included.
 template <int EPI>
 bool launch_w4r_grouped(const void* A, const void* B, void* C, const int* offs, int E, int M, int N, int K, int ldc,
                         hipStream_t st) {
   if (E < 1 || M < 1 || N % 16 || (epi_glu(EPI) && N % 32) || K % 64 || K < 128 || ldc % 8 ||
       (size_t)M * K * 2 >= (1ull << 31) || (size_t)E * N * K * 2 >= (1ull << 31))  // 32-bit buffer offsets
     return false;
-  static int ncu = 0;
-  if (!ncu) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
-      gai_launch_error(__FILE__, __LINE__, "gemm_w4r_grouped: cannot query the CU count");
+  static bool once = false;
+  if (!once) {
     set_max_lds(gemm_w4r_kernel<EPI, false, 3>);
+    once = true;
   }
-  gemm_w4r_kernel<EPI, false, 3><<<ncu & ~7, 256, 5 * kPart, st>>>((const bf16*)A, (const bf16*)B, C, nullptr, nullptr, M, N,
+  gemm_w4r_kernel<EPI, false, 3><<<sk_grid(), 256, 5 * kPart, st>>>((const bf16*)A, (const bf16*)B, C, nullptr, nullptr, M, N,
                                                                   K, ldc, nullptr, nullptr, 1, 0, offs, E);
   GAI_LAUNCH_CHECK();
   return true;
@@ -1478,17 +1486,6 @@ bool gai_sk_workspace(hipStream_t st, size_t ws_bytes, size_t cnt_n, float** ws,
 namespace {
 bool sk_workspace(hipStream_t st, size_t ws_bytes, size_t cnt_n, SkWorkspace& out) {
   return gai_sk_workspace(st, ws_bytes, cnt_n, &out.ws, &out.cnt);
-}
-
-int sk_grid() {
-  static int ncu = 0;
-  if (!ncu) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8)
-      gai_launch_error(__FILE__, __LINE__, "gemm_w4s: cannot query the CU count");
-  }
-  return ncu & ~7;
 }
 
 int ring_tiles(int M, int N) { return ((M + LBM - 1) / LBM) * ((N + LBN - 1) / LBN); }
