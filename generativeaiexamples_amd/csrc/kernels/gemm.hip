@@ -78,9 +78,9 @@ int gai_gemm_prefill_rope_kv(const void* A, const void* B, const void* bias, con
   launch_w4d<EPI_ROPE_KV, false>(A, B, nullptr, bias, nullptr, M, N, K, N, st, rk, 0, bfrag);
   return 1;
 }
-#endif  // GAI_GEMM_KERNELS_ONLY
 
 bool gai_gemm_grouped(const void* A, const void* B, void* C, const int* offs, int E, int M, int N, int K, int swiglu,
                       hipStream_t st) {
   return swiglu ? gai_gemm_grouped4(A, B, C, offs, E, M, N, K, N / 2, st) : gai_gemm_grouped0(A, B, C, offs, E, M, N, K, N, st);
 }
+#endif  // GAI_GEMM_KERNELS_ONLY
