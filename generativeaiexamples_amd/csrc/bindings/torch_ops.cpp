@@ -432,13 +432,14 @@ void token_mask(Tensor& logits, const Tensor& rows, const Tensor& mask) {
                  reinterpret_cast<const uint32_t*>(mask.data_ptr<int>()), W, cur_stream());
 }
 
+// ws_i none: the group form, ws_v holds a maximum per query and 16 rows; else both hold a list per query and row range
 void sim_topk(const Tensor& Q, const Tensor& X, const Tensor& bias, int64_t n_rows, int64_t k, Tensor& ws_v,
-              Tensor& ws_i, int64_t nwg, int64_t rows_per_wg, Tensor& out_v, Tensor& out_i) {
+              const optional<Tensor>& ws_i, int64_t nwg, int64_t rows_per_wg, Tensor& out_v, Tensor& out_i) {
   check_bf16(Q, "Q");
   check_bf16(X, "X");
   check_f32(bias, "bias");
   check_f32(ws_v, "ws_v");
-  check_i32(ws_i, "ws_i");
+  if (ws_i) check_i32(*ws_i, "ws_i");
   check_f32(out_v, "out_v");
   check_dev(out_i, "out_i");
   const int nq = Q.size(0), D = Q.size(1);
@@ -448,12 +449,11 @@ void sim_topk(const Tensor& Q, const Tensor& X, const Tensor& bias, int64_t n_ro
   const int cap = gai_topk_cap(k);
   TORCH_CHECK(n_rows >= 1 && k >= 1 && k <= 64 && nwg * rows_per_wg >= n_rows, "sim_topk: rows or k out of range");
   TORCH_CHECK(out_v.numel() >= nq * k && out_i.numel() >= nq * k && out_i.scalar_type() == at::kLong, "sim_topk: outputs");
-  const bool groups = ws_i.numel() == 0;  // the group form: ws_v holds a maximum per query and 16 rows
-  TORCH_CHECK(groups ? ws_v.numel() >= nq * ((n_rows + 15) / 16)
-                     : cap <= 8 && ws_v.numel() >= nwg * nq * cap && ws_i.numel() >= nwg * nq * cap,
+  TORCH_CHECK(ws_i ? cap <= 8 && ws_v.numel() >= nwg * nq * cap && ws_i->numel() >= nwg * nq * cap
+                   : ws_v.numel() >= nq * ((n_rows + 15) / 16),
               "sim_topk: workspace too small");
   gai_sim_topk(Q.data_ptr(), X.data_ptr(), bias.data_ptr<float>(), nq, n_rows, D, k, ws_v.data_ptr<float>(),
-               groups ? nullptr : ws_i.data_ptr<int>(), nwg, rows_per_wg, out_v.data_ptr<float>(), out_i.data_ptr<int64_t>(),
+               ws_i ? ws_i->data_ptr<int>() : nullptr, nwg, rows_per_wg, out_v.data_ptr<float>(), out_i.data_ptr<int64_t>(),
                cur_stream());
 }
 

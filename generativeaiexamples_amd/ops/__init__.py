@@ -763,6 +763,7 @@ def apply_penalties(logits, tok_ids, tok_cnt, n, freq, pres, rep):
 # vector search
 # ---------------------------------------------------------------------------------------------
 _LDS_BYTES = 160 * 1024
+_TOPK_MAXIMA = 64 << 20  # group maxima (fp32) held at a time, if that is enough for 64 queries
 
 
 def topk_cap(k: int) -> int:
@@ -791,14 +792,14 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
         ws_i = torch.empty(nwg * nq * cap, dtype=torch.int32, device=Q.device)
         native().sim_topk(Q, X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i)
         return out_v, out_i
-    # the largest score of every 16 rows and query, for at most 256 MB of (query, group) pairs at a time
+    # the largest score of every 16 rows and query, in slices of queries: 256 MB of maxima at a time up to 16.8 M rows, past
+    # that those of one 64-query tile (16 bytes a row: 1.6 GB at 100 M rows, beside 205 GB of index at 1024 columns)
     groups = (n_rows + 15) // 16
-    step = min(nq, max(64, (64 << 20) // groups // 64 * 64))
+    step = min(nq, max(64, _TOPK_MAXIMA // groups // 64 * 64))
     ws_v = torch.empty(max(1, step * groups), dtype=torch.float32, device=Q.device)
-    ws_i = torch.empty(0, dtype=torch.int32, device=Q.device)
     for s in range(0, nq, max(1, step)):
         e = min(nq, s + step)
-        native().sim_topk(Q[s:e], X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v[s:e], out_i[s:e])
+        native().sim_topk(Q[s:e], X, bias, n_rows, k_eff, ws_v, None, nwg, rows_per_wg, out_v[s:e], out_i[s:e])
     return out_v, out_i
 
 

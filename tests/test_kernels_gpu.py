@@ -519,6 +519,17 @@ def test_sim_topk_long_lists(cuda, nq, N, D, k, kind):
     assert torch.equal(i.cpu(), torch.where(vr == float("-inf"), torch.full_like(ir, -1), ir))
 
 
+@pytest.mark.parametrize("nq,k", [(130, 40), (200, 7), (64, 9)])
+def test_sim_topk_long_lists_in_slices(cuda, monkeypatch, nq, k):
+    """More group maxima than the budget: 64 queries at a time, the last slice shorter; whole numbers, so exact."""
+    g = torch.Generator().manual_seed(nq)
+    X, Q = torch.randint(-2, 3, (5003, 64), generator=g).float(), torch.randint(-2, 3, (nq, 64), generator=g).float()
+    monkeypatch.setattr(ops, "_TOPK_MAXIMA", 1000)
+    v, i = ops.sim_topk(Q.to(cuda, torch.bfloat16), X.to(cuda, torch.bfloat16), torch.zeros(5003, device=cuda), 5003, k)
+    vr, ir = torch.sort(Q @ X.t(), dim=-1, descending=True, stable=True)
+    assert torch.equal(v.cpu(), vr[:, :k]) and torch.equal(i.cpu(), ir[:, :k])
+
+
 def test_sim_topk_no_candidates(cuda):
     """k = 0 asks for nothing and gets empty lists, from the kernel's entry point and from the index."""
     from generativeaiexamples_amd.index.hbm_index import HBMIndex
