@@ -233,6 +233,9 @@ __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ 
 // best of those 1024 threads, and of their entries the k best. The rows of the k groups (<= 1024) are scored again with
 // the stream's own instruction order and sorted. Bound by latency: 250 KB of maxima at 1M rows, k x 32 KB of X at
 // D = 1024, three 45-step selections across lanes; 300 queries run side by side on the chip.
+// With at most k groups (an index, or a filter's rows, of 16 k rows) all are taken: no stream, one selection. 300 queries, 60
+// rows of 1024, k = 16: 20 us, 89 with the stream and with second groups read for nothing (lists 57); 200 rows, k = 8: 48, 61
+// (lists 55).
 // ------------------------------------------------------------------------------------------------
 typedef unsigned long long u64;
 
@@ -289,12 +292,14 @@ __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__
   __shared__ int pick[64], cnt;
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const float* gm = gmax + (size_t)q * ngr;
-  u64 m = 0;
-  for (int i = tid; i < ngr; i += 1024) {
-    const u64 x = make_key(gm[i], i);
-    m = x > m ? x : m;
+  if (ngr > k) {  // else every group is taken, and gmax was not written
+    u64 m = 0;
+    for (int i = tid; i < ngr; i += 1024) {
+      const u64 x = make_key(gm[i], i);
+      m = x > m ? x : m;
+    }
+    top64(m, buf, list);
   }
-  top64(m, buf, list);
   if (ngr > 1024) {
     if (tid < k) pick[tid] = list[tid] ? key_id(list[tid]) & 1023 : -1;
     if (tid == 0) cnt = 0;
@@ -322,19 +327,25 @@ __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__
       }
     }
   }
-  if (tid < k) pick[tid] = list[tid] ? key_id(list[tid]) : -1;
+  if (tid < k) pick[tid] = ngr <= k ? (tid < ngr ? tid : -1) : list[tid] ? key_id(list[tid]) : -1;
   cand[tid] = 0;
   __syncthreads();
   const bf16* qp = Q + (size_t)q * D + 8 * (lane >> 4);  // every column of the product is this query
   auto rows = [&](int j) { return X + (size_t)min(16 * max(pick[min(j, k - 1)], 0) + (lane & 15), N - 1) * D + 8 * (lane >> 4); };
-  for (int j = wid; j < k; j += 32) {  // two groups a wave
+  for (int j = wid; j < k && pick[j] >= 0; j += 32) {  // (the picked groups come first)
     const bf16 *xa = rows(j), *xb = rows(j + 16);
     f32x4 acc[2] = {};
+    if (j + 16 < k && pick[j + 16] >= 0) {  // two groups a wave
 #pragma unroll 8
-    for (int t = 0; t < D / 32; ++t) {
-      const bf16x8 qf = load8(qp + 32 * t);
-      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), qf, acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xb + 32 * t), qf, acc[1], 0, 0, 0);
+      for (int t = 0; t < D / 32; ++t) {
+        const bf16x8 qf = load8(qp + 32 * t);
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), qf, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xb + 32 * t), qf, acc[1], 0, 0, 0);
+      }
+    } else {
+#pragma unroll 8
+      for (int t = 0; t < D / 32; ++t)
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), load8(qp + 32 * t), acc[0], 0, 0, 0);
     }
     const int r = lane & 15;
 #pragma unroll
@@ -430,9 +441,11 @@ void run_stream_r(const TopkArgs& a) {
     once = true;
   }
   const int qtiles = (a.nq + NQ - 1) / NQ, ngr = (a.N + 15) / 16;
-  k1<<<(a.nwg + 7) / 8 * 8 * qtiles, 512, lds, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.nq, a.N, a.D, a.rows_per_wg, qtiles,
-                                         a.ws_v, a.ws_i, a.ws_v, ngr);
-  GAI_LAUNCH_CHECK();
+  if (K > 0 || ngr > a.k) {  // no group to leave out: no maxima
+    k1<<<(a.nwg + 7) / 8 * 8 * qtiles, 512, lds, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.nq, a.N, a.D, a.rows_per_wg,
+                                                         qtiles, a.ws_v, a.ws_i, a.ws_v, ngr);
+    GAI_LAUNCH_CHECK();
+  }
   if constexpr (K > 0)
     sim_topk_stage2<K><<<a.nq, 256, 0, a.st>>>(a.ws_v, a.ws_i, a.nwg, a.nq, a.k, a.out_v, a.out_i);
   else

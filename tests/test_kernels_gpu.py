@@ -490,7 +490,7 @@ def test_sim_topk_stream_large(cuda, nq):
 
 
 @pytest.mark.parametrize("nq,N,D,k,kind", [
-    (1, 9, 64, 9, "plain"), (2, 40, 384, 33, "plain"), (17, 16 * 1024, 96, 64, "plain"), (3, 16 * 1024 + 1, 384, 17, "plain"),
+    (1, 9, 64, 9, "plain"), (2, 40, 384, 33, "plain"), (300, 60, 1024, 16, "plain"), (3, 145, 64, 9, "plain"), (2, 640, 64, 40, "plain"), (17, 16 * 1024, 96, 64, "plain"), (3, 16 * 1024 + 1, 384, 17, "plain"),
     (130, 70_001, 128, 40, "plain"), (33, 300_000, 32, 64, "equal"), (70, 20_000, 64, 7, "plain"), (2, 400_003, 32, 64, "strided"), (5, 2000, 64, 12, "odd")])
 def test_sim_topk_long_lists(cuda, nq, N, D, k, kind):
     """k > 8 (group maxima + second pass): small whole numbers, so every sum is exact and the order among equal scores
