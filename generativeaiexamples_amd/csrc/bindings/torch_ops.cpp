@@ -14,6 +14,7 @@
 
 #include "gai_gemm_grouped.h"
 #include "gai_gemm_mid.h"
+#include "gai_gemm_slim.h"
 #include "gai_kernels.h"
 
 void gai_launch_error(const char* file, int line, const char* msg) {
@@ -1068,6 +1069,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("layernorm", &layernorm);
   m.def("rope_kv_write", &rope_kv_write);
   m.def("gemm_mid_rows", &gemm_mid_rows);
+  m.def("gemm_slim_nf", &gai_gemm_slim_nf);
   m.def("gemm", &gemm, pybind11::arg("A"), pybind11::arg("B"), pybind11::arg("C"), pybind11::arg("bias"),
         pybind11::arg("R"), pybind11::arg("epi"), pybind11::arg("force"), pybind11::arg("bfrag") = false);
   m.def("gemm_fp8", &gemm_fp8);

@@ -28,7 +28,9 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kStageBytes = 64 * 1024;     // activation columns of one stage, all rows
 constexpr int kPairK = kWaves * 64;        // k columns of one pair step of the workgroup: 2 x 32 per wave
-constexpr int kMaxPairs = 4096 / kPairK;   // every weight fragment of a wave's K share is in registers at once
+// the largest K: every weight fragment of a wave's K share is in registers at once; beyond 2560 only the forms that the rule
+// below takes
+constexpr int max_k(int mt, int nf) { return mt == 4 || nf == 2 ? 2560 : 4096; }
 
 template <int EPI, bool OUTF32>
 __device__ __forceinline__ void slim_store4(void* C, const bf16* bias, const bf16* R, int ldc, int m, int n, int M,
@@ -54,7 +56,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
   constexpr int KC = kStageBytes / (ROWS * 2);       // columns of a stage
   constexpr int CPR = KC / 8;                        // 16-B chunks of a staged row
   constexpr int P = KC / kPairK;                     // pair steps of a stage
-  constexpr int NST = kMaxPairs / P;                 // stages of the largest K
+  constexpr int kMaxPairs = max_k(MT, NF) / kPairK;
+  constexpr int NST = (kMaxPairs + P - 1) / P;       // stages of the largest K
   constexpr int DMA = kStageBytes / (64 * kWaves * 16);  // LDS-DMA instructions of a wave and stage
   extern __shared__ __attribute__((aligned(16))) char smem[];  // 2 stages; reused for the waves' partial tiles
   const int tid = threadIdx.x, lane = tid & 63;
@@ -121,7 +124,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
       const char* src = smem + (t & 1) * kStageBytes;
 #pragma unroll
       for (int j = 0; j < P; ++j) {
-        if (t * P + j < np) {
+        if (t * P + j < kMaxPairs && t * P + j < np) {
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             const int c = (j * kPairK + 64 * wid + 32 * u) / 8 + q;
@@ -215,16 +218,15 @@ int gai_gemm_slim_nf(int M, int N, int K, bool glu) {
     return 0;
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   const int nf = glu || (N / 16 > 256 && K > kStageBytes / (32 * mt)) ? 2 : 1;
-  if (K > 2560 && (mt == 4 || nf == 2)) return 0;
-  return nf;
+  return K <= max_k(mt, nf) ? nf : 0;
 }
 
 void gai_gemm_slim(const void* A, const void* W, void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
                    int epi, int out_f32, int nf, int psw, hipStream_t st) {
-  if (M < 1 || M > 64 || K < kPairK || K % kPairK || K > 4096 || N < 16 || N % 16 || (nf != 1 && nf != 2) ||
-      (epi_glu(epi) && (nf != 2 || N % 32)) || epi < 0 || (epi > EPI_BIAS_QUICKGELU && epi != EPI_GEGLU))
-    gai_launch_error(__FILE__, __LINE__, "gemm_slim: needs 1 <= M <= 64, K % 512 == 0, K <= 4096, N % 16 == 0");
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  if (M < 1 || M > 64 || K < kPairK || K % kPairK || K > max_k(mt, nf) || N < 16 || N % 16 || (nf != 1 && nf != 2) ||
+      (epi_glu(epi) && (nf != 2 || N % 32)) || epi < 0 || (epi > EPI_BIAS_QUICKGELU && epi != EPI_GEGLU))
+    gai_launch_error(__FILE__, __LINE__, "gemm_slim: needs 1 <= M <= 64, K % 512 == 0, K <= 4096 or 2560, N % 16 == 0");
 #define GAI_SLIM(MTV, NFV) \
   if (mt == MTV && nf == NFV) return launch_slim<MTV, NFV>(A, W, C, bias, R, M, N, K, ldc, epi, out_f32, psw, st);
   GAI_SLIM(1, 1)

@@ -50,12 +50,13 @@ def test_splitk_epilogues(cuda, act):
 @pytest.mark.parametrize("M,N,K,epi", [
     (1, 16, 512, "bias"), (16, 1040, 1024, "gelu"), (17, 64, 1536, "residual"), (31, 96, 2560, "swiglu"),
     (32, 1024, 4096, "bias_residual"), (33, 2064, 512, None), (64, 4096, 2560, "relu"), (64, 2048, 2048, "quick_gelu"),
-    (49, 3104, 1024, "geglu"), (5, 6160, 1024, None), (24, 5136, 1536, "bias")])
+    (49, 3104, 1024, "geglu"), (5, 6160, 1024, None), (24, 5136, 1536, "bias"), (64, 3264, 2560, "bias"), (33, 3232, 2560, "swiglu"),
+    (9, 2048, 4096, "gelu")])
 @pytest.mark.parametrize("frag,f32", [(False, False), (True, False), (False, True)])
 def test_one_launch_gemm(cuda, M, N, K, epi, frag, f32):
     """Narrow decode projections in one launch (all of K in a workgroup): row tiles 16 / 32 / 64 with ragged M, one and
-    two column fragments with a half-empty last pair, 1 to 8 activation stages with a short last one. Bound per element:
-    K fp32 products in any order, K 2^-24 sum |x w|, then what the epilogue's own steps can move, and one bf16 rounding."""
+    two column fragments with a half-empty last pair, 1 to 5 activation stages with a short last one; weights past 16 MiB
+    (64 x 4096 x 2560) keep the split kernels. Bound per element: K fp32 products in any order, K 2^-24 sum |x w|, then what the epilogue's own steps can move, and one bf16 rounding."""
     g = torch.Generator().manual_seed(M + N + K)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16)
     w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
@@ -66,6 +67,7 @@ def test_one_launch_gemm(cuda, M, N, K, epi, frag, f32):
     ncol = N // 2 if epi in ("swiglu", "geglu") else N
     out = torch.full((M, ncol), float("nan"), device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
     nat = ops.native()
+    assert (nat.gemm_slim_nf(M, N, K, epi in ("swiglu", "geglu")) > 0) == (N * K <= 8 << 20)
     ws = torch.empty(nat.gemm_splitk_ws_floats(M, N, K), device="cuda", dtype=torch.float32)
     nat.gemm_splitk(dev[0], dev[1], out, dev[2], dev[3], ops.EPI[epi] if epi else 0, ws, frag)
     y = x.double() @ w.double().t()
