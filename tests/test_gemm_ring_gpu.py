@@ -236,6 +236,40 @@ def test_mid_gemm_choice(cuda, M, N, K, act, frag, mid):
     assert ops.native().gemm_mid_rows(x, w, out, b, res, ops.EPI[act], frag) == (M if mid else 0)
 
 
+@pytest.mark.parametrize("plan", [8105, 8116, 8206, 12208, 0])  # 0: as chosen
+@pytest.mark.parametrize("M,N,K,act", [(65, 320, 4224, "bias_residual"), (193, 272, 2048, None), (187, 1024, 14336, "residual"),
+                                       (413, 1056, 2176, "swiglu"), (1000, 1024, 1024, "gelu"), (2047, 272, 3072, "relu")])
+def test_mid_gemm_many_parts(cuda, M, N, K, act, plan):
+    """More parts than one round of the sum takes (four): whole and partial later rounds, uneven parts, both layouts; and the
+    plan that is chosen. Repeated launches, also beside each other on two streams, give the same bits."""
+    if act == "swiglu" and plan // 100 % 10 == 1:
+        pytest.skip("a gated pair needs 128 columns")
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    w = (torch.randn(N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
+    b = torch.randn(N, device=cuda, dtype=torch.bfloat16) if act in ("gelu", "relu", "bias_residual") else None
+    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16) if act in ("residual", "bias_residual") else None
+    y = torch.full((M, N // 2 if act == "swiglu" else N), float("nan"), device=cuda, dtype=torch.bfloat16)
+    f, epi = ops.shuffle_fragments(w), ops.EPI[act]
+    ops.native().gemm(x, f, y, b, res, epi, plan, True)
+    y_ref = ref.linear(x.cpu(), w.cpu(), None if b is None else b.cpu(), None if res is None else res.cpu(),
+                       act if act in ("gelu", "relu", "swiglu") else None).float()
+    assert ((y.float().cpu() - y_ref).abs() <= 3e-2 + 2e-2 * y_ref.abs()).all()   # the bound of test_mid_gemm: roundings to bf16
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[torch.full_like(y, float("nan")) for _ in range(4)] for _ in streams]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    for i in range(4):
+        for s, o in zip(streams, outs):
+            with torch.cuda.stream(s):
+                ops.native().gemm(x, f, o[i], b, res, epi, plan, True)
+    torch.cuda.synchronize()
+    assert all(torch.equal(t, y) for o in outs for t in o)
+    if plan:  # (the rule may choose another plan for the other layout)
+        ops.native().gemm(x, w, outs[0][0], b, res, epi, plan, False)
+        assert torch.equal(outs[0][0], y)
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 1024, 4096), (192, 1024, 4096), (1536, 1024, 4096), (300, 2048, 5632)])
 def test_mid_gemm_captured_equals_eager(cuda, M, N, K):
     """A captured product with parts of K takes the eager one's plan, sums and bits, whatever runs between the replays or

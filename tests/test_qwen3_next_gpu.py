@@ -98,6 +98,29 @@ def test_gdn_prep_matches_torch(cuda, lens, Hk, Hv, dk, dv, dt):
     assert torch.allclose(cs.double(), kept, rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("Hv,dv,dt", [(4, 128, torch.bfloat16), (3, 48, torch.float32), (1, 16, torch.bfloat16)])
+def test_gdn_rows_wider_than_their_tensors(cuda, Hv, dv, dt):
+    """Projected rows and gates as columns of a wider buffer: the bits of contiguous ones; the gated norm against torch with
+    the same roundings (fp32 sums of up to 128 squares: one rounding of the type may fall the other way)."""
+    torch.manual_seed(Hv)
+    T, Hk, dk, eps = 70, 1, 64, 1e-6
+    cd, vd = 2 * Hk * dk + Hv * dv, Hv * dv
+    wide = torch.randn(T, 5 + cd + vd + 2 * Hv + 3, device=cuda).to(dt)
+    proj = wide[:, 5:5 + cd + vd + 2 * Hv]
+    cw, cs = torch.randn(cd, 4, device=cuda), torch.randn(2, 3, cd, device=cuda)
+    cu, slots = (torch.tensor(x, dtype=torch.int32, device=cuda) for x in ([0, 30, T], [1, 0]))
+    A_log, dt_bias = torch.randn(Hv, device=cuda), torch.randn(Hv, device=cuda)
+    for a, b in zip(*(ops.gdn_prep(p, cw, cs, cu, slots, A_log, dt_bias, Hk, dk, Hv, dv) for p in (proj, proj.contiguous()))):
+        assert torch.equal(a, b)
+    z, o, w = proj[:, cd:cd + vd], torch.randn(T, Hv, dv, device=cuda), torch.randn(dv, device=cuda).to(dt)
+    y = ops.gdn_out(o, z, w, eps)
+    assert torch.equal(y, ops.gdn_out(o, z.contiguous(), w, eps))
+    n = (o * torch.rsqrt(o.pow(2).mean(-1, keepdim=True) + eps)).to(dt)
+    want = (w * n).float() * torch.nn.functional.silu(z.float().view(T, Hv, dv))
+    tol = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -20
+    assert ((y.view(T, Hv, dv).float() - want).abs() <= tol * want.abs() + 1e-30).all()
+
+
 def _pair(cuda):
     cfg = Qwen3NextConfig.tiny()
     g = Qwen3NextModel(cfg, device=cuda).random_init(3)
