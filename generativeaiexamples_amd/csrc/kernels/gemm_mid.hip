@@ -263,22 +263,22 @@ bool parts_fit(int M, int N, int mt, int ng, int S) {
   return mid_tiles(M, N, mt, ng) * 8 <= kGaiMidTickets && part_bytes(M, N, mt, ng, S) < (1ull << 31);
 }
 
-// Modelled times in us, fitted to 1376 products of 65 to 2048 rows, N 256 to 32000, K 128 to 16384, every epilogue and both
-// weight layouts, each with the kernels below and with some 13 plans of this one (19 of 20 plans within 15 %, 9 of 10 of the
-// others). A product is taken where the model says 10 % less (25 % at K >= 8192): two of those taken are then slower than the
-// kernel replaced, by 4 %, and the choice as a whole is 1.6 % above the best one; of 719 products not used for the fit, 6
-// above 10 us measured 4 to 12 % slower. At equality 22 of the 1376 are slower, by up to 19 %; the first form of the model, without the bytes of the parts, the epilogues and the
-// rounds of short K, lost up to 54 % (1535 x 2176 x 384: 9.4 -> 14.4 us; with 150 MB of parts 1536 x 11264 x 2048: 90 -> 258).
+// Modelled times in us. This kernel: fitted to 7738 timings of 420 products (65 to 2048 rows, N 256 to 28672, K 256 to 14336, every
+// epilogue, both weight layouts, weights from HBM) with up to 33 plans each; 19 of 20 within 15 %, also of the products left out of the
+// fit. The kernels below: 1376 products, 9 of 10 within 15 %. Of those 420 the rule takes three in four, two of them up to 8 %
+// slower for it; its choice is 0.8 % (row-major) and 1.4 % (fragment order) above the best one. Without the bytes of the parts,
+// the epilogues and the rounds of short K, the model's first form lost up to 54 % (1535 x 2176 x 384: 9.4 -> 14.4 us; with
+// 150 MB of parts 1536 x 11264 x 2048: 90 -> 258).
 struct MidFit {
   double base, round, alone, full;  // launch; of a round of workgroups; of a 128-deep K step, few workgroups / full chip
-  double weights, row_major;        // GB/s / 1000 of the weights; a step's factor for row-major ones
+  double weights, few, row_major;   // GB/s / 1000 of the weights, the share of it with few workgroups; a row-major step's factor
   double part0, part1, parts;       // parts of K: once, each, GB/s / 1000 of the sums written and read
   double out, bias, gelu;           // GB/s / 1000 of residual and result; epilogues
 };
-constexpr MidFit kFit[3] = {{4.2, 0.4, 0.62, 0.66, 3.6, 1.30, 1.0, 0.73, 6.3, 2.5, 0.6, 0.9},    // 128 x 64
-                            {3.5, 2.4, 0.89, 0.97, 4.4, 1.39, 1.5, 0.85, 6.8, 3.0, 1.35, 1.8},   // 128 x 128
-                            {3.3, 3.6, 1.33, 1.36, 4.1, 1.22, 1.4, 1.13, 7.4, 3.3, 1.7, 2.8}};   // 192 x 128
-constexpr double kTicketFill = 1.6;  // a captured launch clears its tickets: counted always, the plan is the same
+constexpr MidFit kFit[3] = {{4.0, 0.0, 0.73, 0.68, 3.9, 0.32, 1.28, 0.55, 0.83, 5.1, 2.4, 0.45, 1.1},  // 128 x 64
+                            {2.6, 2.9, 0.99, 0.97, 4.1, 0.7, 1.35, 0.83, 1.0, 6.1, 2.7, 1.05, 2.0},   // 128 x 128
+                            {2.4, 4.4, 1.34, 1.36, 3.9, 0.7, 1.23, 0.8, 1.26, 6.7, 3.3, 1.9, 2.7}};   // 192 x 128
+constexpr double kTicketFill = 0.8;  // a captured launch clears its tickets (1.6 us): half of it counted always, the plan is the same
 
 // MB written and read by the epilogue; 0 none, 1 bias / residual, 2 GELU and the like
 double out_mb(int M, int N, int epi) {
@@ -294,8 +294,8 @@ double mid_cost(int M, int N, int K, int epi, int mt, int ng, int S, int bfrag) 
   const int items = mid_tiles(M, N, mt, ng) * S, steps = (K / kBK + S - 1) / S, G = mid_cus(), rounds = (items + G - 1) / G;
   const double fill = std::min(1.0, (double)items / G), step = (f.alone + (f.full - f.alone) * fill) * (bfrag ? 1.0 : f.row_major);
   const int ec = epi_class(epi);
-  return f.base + std::max(rounds * (f.round + steps * step), (double)N * K * 2 / 1e6 / f.weights) + out_mb(M, N, epi) / f.out +
-         (ec == 1 ? f.bias : ec == 2 ? f.gelu : 0.0) +
+  return f.base + std::max(rounds * (f.round + steps * step), (double)N * K * 2 / 1e6 / (f.weights * (f.few + (1 - f.few) * fill))) +
+         out_mb(M, N, epi) / f.out + (ec == 1 ? f.bias : ec == 2 ? f.gelu : 0.0) +
          (S > 1 ? f.part0 + f.part1 * S + 2 * part_bytes(M, N, mt, ng, S) / 1e6 / f.parts + kTicketFill : 0.0);
 }
 // the kernels of gemm_impl.h, by its own rules: skinny, stream-K, 256 x 256 tiles, 128 x 128 tiles
@@ -322,8 +322,12 @@ double other_cost(int M, int N, int K, int epi) {
                                              0.25 * std::min(1.0, wmb / 64);
   return 3.6 + (t1 + 2 * G - 1) / (2 * G) * (0.73 + kt * step) + out / 4.0 + (ec == 2 ? 10.1 : ec ? 7.0 : 0.0);
 }
+// A weight gives the same bits in either layout: which kernel, and into how many parts, is one choice for both; only the tile
+// is the layout's own (a sum's order does not depend on it). The parts are those of the smaller row-major + 2 x fragment-order
+// time: the large weights, where parts matter most, are stored in fragment order.
+constexpr double kFragShare = 2.0;
 // (the 256 x 256 kernels at K >= 8192 are up to a fifth faster than their model where the tiles divide the chip evenly)
-double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.25 : 1.1; }
+double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.2 : 1.05; }
 
 // the ordered form, fitted to 320 shapes of up to 3072 rows (19 of 20 within 15 %)
 double ordered_cost(int M, int N, int K, int mt, int bfrag) {
@@ -372,19 +376,27 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
   } else if (force >= 1000) {
     best = {force / 1000, glu ? 2 : force / 100 % 10, std::max(1, std::min(force % 100, K / kBK)), 0, 0.0};
   } else {
-    double bc = 1e30;
-    for (int v = glu ? 1 : 0; v < 3; ++v) {
-      const int mt = v == 2 ? 12 : 8, ng = v == 0 ? 1 : 2;
-      for (int S = 1; S <= std::min(16, std::max(1, K / kBK / 4)); ++S) {
-        if (S > 1 && !parts_fit(M, N, mt, ng, S)) break;
-        const double c = mid_cost(M, N, K, epi, mt, ng, S, bfrag);
-        if (c < bc) {
-          bc = c;
-          best = {mt, ng, S, 0, c};
+    double bc = 1e30, row = 1e30, frag = 1e30;
+    for (int S = 1; S <= std::min(16, std::max(1, K / kBK / 4)); ++S) {
+      GaiMidPlan at[2] = {{8, 2, S, 0, 1e30}, {8, 2, S, 0, 1e30}};  // row-major, fragment order: the best tile
+      for (int v = glu ? 1 : 0; v < 3; ++v) {
+        const int mt = v == 2 ? 12 : 8, ng = v == 0 ? 1 : 2;
+        if (S > 1 && !parts_fit(M, N, mt, ng, S)) continue;
+        for (int l = 0; l < 2; ++l) {
+          const double c = mid_cost(M, N, K, epi, mt, ng, S, l);
+          if (c < at[l].cost) at[l] = {mt, ng, S, 0, c};
         }
       }
+      const double c = at[0].cost + kFragShare * at[1].cost;
+      if (c < bc) {
+        bc = c;
+        row = at[0].cost;
+        frag = at[1].cost;
+        best = at[bfrag ? 1 : 0];
+      }
     }
-    if (force == 0 && bc * margin(M, K) >= other_cost(M, N, K, epi)) return false;
+    const double other = other_cost(M, N, K, epi);
+    if (force == 0 && (frag * margin(M, K) >= other || row * 1.03 >= other)) return false;
   }
   if (best.parts > 1 && !parts_fit(M, N, best.mt, best.ng, best.parts)) best.parts = 1;
   if (best.parts > 1) {

@@ -321,9 +321,10 @@ def test_mid_gemm_without_memory_for_its_parts(cuda):
             while True:
                 held.append(torch.empty(32 << 20, device=cuda, dtype=torch.uint8))
         ops.native().gemm(x, w, out, None, None, 0, 8116)   # 64 MB of partial sums
-        assert torch.equal(out, one)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+        held.clear()
+    assert torch.equal(out, one)   # (the comparison takes memory too)
     out.fill_(float("nan"))
     ops.native().gemm(x, w, out, None, None, 0, 8116)
     assert (out.float() - one.float()).abs().max() <= 2.0 ** -6 * one.float().abs().max()
