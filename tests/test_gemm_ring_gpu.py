@@ -265,9 +265,26 @@ def test_mid_gemm_many_parts(cuda, M, N, K, act, plan):
                 ops.native().gemm(x, f, o[i], b, res, epi, plan, True)
     torch.cuda.synchronize()
     assert all(torch.equal(t, y) for o in outs for t in o)
-    if plan:  # (the rule may choose another plan for the other layout)
-        ops.native().gemm(x, w, outs[0][0], b, res, epi, plan, False)
-        assert torch.equal(outs[0][0], y)
+    ops.native().gemm(x, w, outs[0][0], b, res, epi, plan, False)
+    assert torch.equal(outs[0][0], y)
+
+
+@pytest.mark.parametrize("M,N,K,act", [(187, 4096, 14336, "residual"), (300, 6144, 4096, None), (513, 4096, 4096, "residual"),
+                                       (1100, 2048, 4096, "swiglu"), (1536, 11264, 2048, "swiglu"), (128, 1024, 1024, "bias"),
+                                       (1400, 3072, 1024, "bias"), (513, 4096, 14336, "residual")])
+def test_mid_gemm_choice_is_one_for_both_layouts(cuda, M, N, K, act):
+    """Products where the best number of parts, or the best kernel, differs between the weight layouts: equal bits."""
+    torch.manual_seed(M)
+    x = torch.randn(M, K, device=cuda, dtype=torch.bfloat16)
+    w = (torch.randn(N, K, device=cuda) / math.sqrt(K)).to(torch.bfloat16)
+    b = torch.randn(N, device=cuda, dtype=torch.bfloat16) if act == "bias" else None
+    res = torch.randn(M, N, device=cuda, dtype=torch.bfloat16) if act == "residual" else None
+    f, epi = ops.shuffle_fragments(w), ops.EPI[act]
+    y, yf = (torch.empty(M, N // 2 if act == "swiglu" else N, device=cuda, dtype=torch.bfloat16) for _ in range(2))
+    assert ops.native().gemm_mid_rows(x, w, y, b, res, epi, False) == ops.native().gemm_mid_rows(x, f, y, b, res, epi, True)
+    ops.native().gemm(x, w, y, b, res, epi, 0, False)
+    ops.native().gemm(x, f, yf, b, res, epi, 0, True)
+    assert torch.equal(y, yf)
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 1024, 4096), (192, 1024, 4096), (1536, 1024, 4096), (300, 2048, 5632)])
