@@ -7,14 +7,15 @@
 //  * a workgroup takes 16 * MT rows x 64 * NG columns: 128 x 64 (two workgroups share a CU), 128 x 128 or, so that up to
 //    192 rows still fetch the weights once, 192 x 128;
 //  * the weights go straight to registers in operand layout, DB 128-deep K steps ahead (wave = 16 * NG columns x half of
-//    the K step: nothing is fetched twice, and in whole 128-byte lines); the rows of A, which sit in L2, pass through registers into LDS (two buffers, one
-//    barrier per step) and are read by all waves. All loads are ordinary ones, so their waits are counted. Both operands by
-//    DMA through a five-step LDS ring instead held 80 KB of weights per CU in flight and took 0.52 us a step, whatever the
-//    rest of the step looked like;
+//    the K step: nothing is fetched twice, and in whole 128-byte lines); the rows of A, which sit in L2, pass through registers
+//    into LDS (two buffers, one barrier per step) and are read by all waves. All loads are ordinary ones, so their waits are
+//    counted. Both operands by DMA through a five-step LDS ring instead held 80 KB of weights per CU in flight and took
+//    0.52 us a step, whatever the rest of the step looked like;
 //  * K is cut into S parts, so tile x part items fill the CUs;
-//  * measured on one card, weights from HBM, fragment order (row-major about 15 % slower), N x K: 187 rows 4096 x 14336
-//    200 -> 49 us, 4096 x 4096 66 -> 24 us, 6144 x 4096 57 -> 29 us, 28672 x 4096 (SwiGLU) 73 -> 61 us; 512 rows 67 -> 33,
-//    59 -> 41, 1024 x 4096 62 -> 19, 3072 x 1024 21 -> 11, 2048 x 5632 78 -> 28 us.
+//  * measured on one card, weights from HBM, fragment order (row-major about 15 % slower), N x K, against the kernels it
+//    replaced: 187 rows 4096 x 14336 200 -> 52 us, 4096 x 4096 67 -> 23, 6144 x 4096 58 -> 30, 28672 x 4096 (SwiGLU) 76 -> 62;
+//    512 rows 69 -> 31, 60 -> 40, 1024 x 4096 69 -> 19, 3072 x 1024 24 -> 11, 2048 x 5632 89 -> 27. The least of it: 512 rows
+//    4096 x 14336 82 -> 73, and row-major, for which the choice is the same, 84 -> 89;
 //  * MFMA operands swapped (rows = weights), so a lane ends with four consecutive columns of a row: 8-byte stores;
 //  * S > 1: every wave stores its fp32 share (write-through) and draws the (tile, wave) ticket; the one that draws the last
 //    sums the parts in part order - the same result whichever it is - and runs the epilogue. Nobody waits, and a wave that
@@ -263,9 +264,9 @@ bool parts_fit(int M, int N, int mt, int ng, int S) {
   return mid_tiles(M, N, mt, ng) * 8 <= kGaiMidTickets && part_bytes(M, N, mt, ng, S) < (1ull << 31);
 }
 
-// Modelled times in us. This kernel: fitted to 7738 timings of 420 products (65 to 2048 rows, N 256 to 28672, K 256 to 14336, every
-// epilogue, both weight layouts, weights from HBM) with up to 33 plans each; 19 of 20 within 15 %, also of the products left out of the
-// fit. The kernels below: 1376 products, 9 of 10 within 15 %. Of those 420 the rule takes three in four, two of them up to 8 %
+// Modelled times in us. This kernel: fitted to 7738 timings of 420 products (65 to 2048 rows, N 256 to 28672, K 256 to 14336,
+// every epilogue, both weight layouts, weights from HBM) with up to 33 plans each; 19 of 20 within 15 %, also of the products left
+// out of the fit. The kernels below: 1376 products, 9 of 10 within 15 %. Of those 420 the rule takes three in four, two of them up to 8 %
 // slower for it; its choice is 0.8 % (row-major) and 1.4 % (fragment order) above the best one. Without the bytes of the parts,
 // the epilogues and the rounds of short K, the model's first form lost up to 54 % (1535 x 2176 x 384: 9.4 -> 14.4 us; with
 // 150 MB of parts 1536 x 11264 x 2048: 90 -> 258).
@@ -326,7 +327,8 @@ double other_cost(int M, int N, int K, int epi) {
 // is the layout's own (a sum's order does not depend on it). The parts are those of the smaller row-major + 2 x fragment-order
 // time: the large weights, where parts matter most, are stored in fragment order.
 constexpr double kFragShare = 2.0;
-// (the 256 x 256 kernels at K >= 8192 are up to a fifth faster than their model where the tiles divide the chip evenly)
+// A product is taken where the model says 5 % less in fragment order and 3 % less row-major. (The 256 x 256 kernels at K >= 8192
+// are up to a fifth faster than their model where the tiles divide the chip evenly.)
 double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.2 : 1.05; }
 
 // the ordered form, fitted to 320 shapes of up to 3072 rows (19 of 20 within 15 %)
