@@ -6,25 +6,25 @@
 // are. So:
 //  * a workgroup takes 16 * MT rows x 64 * NG columns: 128 x 64 (two workgroups share a CU), 128 x 128 or, so that up to
 //    192 rows still fetch the weights once, 192 x 128;
-//  * the weights go straight to registers in operand layout, DB 128-deep K steps ahead (wave = 16 * NG columns x half of
-//    the K step: nothing is fetched twice, and in whole 128-byte lines); the rows of A, which sit in L2, pass through registers
-//    into LDS (two buffers, one barrier per step) and are read by all waves. All loads are ordinary ones, so their waits are
-//    counted. Both operands by DMA through a five-step LDS ring instead held 80 KB of weights per CU in flight and took
-//    0.52 us a step, whatever the rest of the step looked like;
+//  * the weights go straight to registers in operand layout (wave = 16 * NG columns x half of a 64-deep K step: nothing is
+//    fetched twice); the rows of A, which sit in L2, go to an LDS ring by DMA and are read by all waves. Loads return in
+//    order, so A is asked for as far ahead as the weights are (DB steps): with A a step or two ahead, waiting for it
+//    waited for weights that were asked for just before (187 rows, 28672 x 4096 SwiGLU 64.3 -> 56.0 us, 4096 x 14336 50.6 ->
+//    44.0, 6144 x 4096 30.7 -> 23.7, 4096 x 4096 23.3 -> 20.5; 1024 rows 4096 x 4096 41.4 -> 37.5). What is left: a CU holds
+//    about 32 KB of misses (a weight stream of 32 KB in flight per CU is as fast as one of 192 KB: 6.3 TB/s on the chip, 60 KB/us
+//    in one CU), and A's 24 KB a step share them, 0.75 us a step without any products. Four waves of 64 columns each (half the
+//    LDS reads) gave nothing: 57.5 us for the first of the products above;
 //  * K is cut into S parts, so tile x part items fill the CUs;
-//  * measured on one card, weights from HBM, fragment order (row-major about 15 % slower), N x K, against the kernels it
-//    replaced: 187 rows 4096 x 14336 200 -> 52 us, 4096 x 4096 67 -> 23, 6144 x 4096 58 -> 30, 28672 x 4096 (SwiGLU) 76 -> 62;
-//    512 rows 69 -> 31, 60 -> 40, 1024 x 4096 69 -> 19, 3072 x 1024 24 -> 11, 2048 x 5632 89 -> 27. The least of it: 512 rows
-//    4096 x 14336 82 -> 73, and row-major, for which the choice is the same, 84 -> 89;
+//  * measured on one card, weights from HBM, fragment order (row-major 10 - 40 % slower: its loads touch 16 lines each), N x K,
+//    against the kernels it replaced: 187 rows 4096 x 14336 200 -> 44 us, 4096 x 4096 67 -> 20, 6144 x 4096 58 -> 24, 28672 x
+//    4096 (SwiGLU) 76 -> 56; 512 rows 4096 x 14336 82 -> 74;
 //  * MFMA operands swapped (rows = weights), so a lane ends with four consecutive columns of a row: 8-byte stores;
 //  * S > 1: every wave stores its fp32 share (write-through) and draws the (tile, wave) ticket; the one that draws the last
 //    sums the parts in part order - the same result whichever it is - and runs the epilogue. Nobody waits, and a wave that
 //    sees all others done keeps its share in registers;
 //  * ORD, for the last rows of a large product (gai_gemm_mid_tail): a wave takes all of K for half the columns, one sum in
 //    the order of the 256 x 256 kernels, so equal rows give equal bits wherever they stand. 64 x 128 or 128 x 128 tiles:
-//    no weight is fetched twice in a workgroup, A is read from LDS twice as often as with k halves. 1953 rows, N 1024,
-//    residual, row-major | fragment order: K 1024 16.1 | 11.5 us (64 rows), K 4096 44.6 | 30.0 (k halves, 128 x 64 tiles
-//    14.8 | 12.5, 34.7 | 30.0; sharing a fetch between two row halves 18.4 | 13.6, 54.2 | 39.1).
+//    no weight is fetched twice in a workgroup, A is read from LDS twice as often as with k halves.
 #include "gai_common.h"
 #include "gai_epilogue.h"
 #include "gai_gemm_mid.h"
@@ -71,93 +71,109 @@ __device__ __forceinline__ void store4(void* C, const bf16* bias, const bf16* R,
   }
 }
 
+template <int MT>
+constexpr int mid_ring() { return MT == 12 ? 6 : 4; }  // K steps of A in LDS
+
 template <int MT, int NG, int EPI, bool OUTF32, bool ORD>
 __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B, void* C,
                                                           const bf16* __restrict__ bias, const bf16* R, int M, int N, int K,
                                                           int ldc, int bfrag, int S, float* ws, int* cnt) {
-  constexpr int BM = 16 * MT, BN = 64 * NG, NA = MT / 2, NF = MT / 2 * NG;
-  constexpr int FW = ORD ? NG / 2 : NG, KF = ORD ? 4 : 2, RW = ORD ? MT : MT / 2;  // a wave's columns / 16, k32 fragments of a
+  constexpr int BM = 16 * MT, BN = 64 * NG, NA = MT / 4, NF = MT / 2 * NG;
+  constexpr int FW = ORD ? NG / 2 : NG, KF = ORD ? 2 : 1, RW = ORD ? MT : MT / 2;  // a wave's columns / 16, k32 fragments of a
                                                                                    // step, rows / 16 that it stores
-  constexpr int DB = NG == 2 ? 3 : 4, U = NG == 2 ? 6 : 4;  // steps the weights are ahead; unrolled steps (even)
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // 2 x BM x 256 B; at the end the k halves' exchange
+  constexpr int RING = mid_ring<MT>(), DB = RING - 1, NB = FW * KF, PART = BM * 128;
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // RING x BM x 128 B; at the end the k halves' exchange
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tm_n = (M + BM - 1) / BM, tiles = tm_n * ((N + BN - 1) / BN);
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int part = id / tiles, tile = id - part * tiles;
   const int m0 = tile % tm_n * BM, n0 = tile / tm_n * BN;
-  const int nk = K / kBK, k0 = (int)((long long)nk * part / S), n = (int)((long long)nk * (part + 1) / S) - k0;
+  const int nk = K / kBK, k0 = (int)((long long)nk * part / S), n = 2 * ((int)((long long)nk * (part + 1) / S) - k0);
   const int g = ORD ? wid : wid & 3, h = ORD ? 0 : wid >> 2;  // column group, k half
 
-  const bf16* ap[NA];  // row tid / 16 (+ 32 per piece), 16-B piece tid & 15
-  int a_wr[NA];
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(A) + (size_t)m0 * K, (short)0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(B) + (size_t)n0 * K, (short)0, 0x7fffffff, 0x00020000);
+  int oa[3], ob[2];  // NA, FW of them
 #pragma unroll
   for (int q = 0; q < NA; ++q) {
-    const int row = q * 32 + (tid >> 4), c = tid & 15;
-    ap[q] = A + (size_t)min(m0 + row, M - 1) * K + (size_t)k0 * kBK + c * 8;
-    a_wr[q] = row * 256 + ((c ^ (row & 15)) << 4);
+    const int row = (q * 8 + wid) * 8 + (lane >> 3);
+    oa[q] = (min(m0 + row, M - 1) - m0) * K * 2 + k0 * (2 * kBK) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
-  const bf16* bp[FW];
 #pragma unroll
   for (int f = 0; f < FW; ++f) {
-    const int col = n0 + (g * FW + f) * 16;
-    bp[f] = bfrag ? B + ((size_t)min(col / 16, N / 16 - 1) * (K / 32) + 4 * (size_t)k0 + 2 * h) * 512 + lane * 8
-                  : B + (size_t)min(col + (lane & 15), N - 1) * K + (size_t)k0 * kBK + 64 * h + 8 * (lane >> 4);
+    const int col = (g * FW + f) * 16;
+    ob[f] = bfrag ? min(col, N - 16 - n0) * K * 2 + k0 * 4096 + h * 1024 + lane * 16
+                  : (min(n0 + col + (lane & 15), N - 1) - n0) * K * 2 + k0 * (2 * kBK) + h * 64 + 16 * (lane >> 4);
   }
-  const int bstep = bfrag ? 2048 : kBK, bhalf = bfrag ? 512 : 32;
-  bf16x8 ar[NA], br[DB][FW][KF];
+  const int bstep = bfrag ? 2048 : 128, bhalf = bfrag ? 1024 : 64;
+  bf16x8 br[DB][FW][KF];
   // past the end the last step is read again (from L2): the count of loads stays what the code says
-  auto load_a = [&](int t, bf16x8(&d)[NA]) {
+  auto load_a = [&](int t, int slot) {
+    const int so = min(t, n - 1) * 128;
+    char* d = smem + slot * PART + wid * 1024;
 #pragma unroll
-    for (int q = 0; q < NA; ++q) d[q] = load8(ap[q] + (size_t)min(t, n - 1) * kBK);
+    for (int q = 0; q < NA; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, GAI_LDS(d + q * 8192), 16, oa[q], so, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto load_b = [&](int t, bf16x8(&d)[FW][KF]) {
+    const int so = min(t, n - 1) * bstep;
 #pragma unroll
     for (int f = 0; f < FW; ++f)
 #pragma unroll
-      for (int e = 0; e < KF; ++e) d[f][e] = load8(bp[f] + (size_t)min(t, n - 1) * bstep + e * bhalf);
+      for (int e = 0; e < KF; ++e)
+        d[f][e] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rb, ob[f], so + e * bhalf, 0));
+    __builtin_amdgcn_sched_barrier(0);
   };
-  auto put_a = [&](int buf, const bf16x8(&d)[NA]) {
+  int a_rd[KF];  // + 2048 per 16 rows
 #pragma unroll
-    for (int q = 0; q < NA; ++q) *reinterpret_cast<bf16x8*>(smem + buf * (BM * 256) + a_wr[q]) = d[q];
-  };
-  int a_rd[KF];  // + 4096 per 16 rows
-#pragma unroll
-  for (int e = 0; e < KF; ++e) a_rd[e] = (lane & 15) * 256 + (((8 * h + 4 * e + (lane >> 4)) ^ (lane & 15)) << 4);
+  for (int e = 0; e < KF; ++e) a_rd[e] = (lane & 15) * 128 + (((4 * (h + e) + (lane >> 4)) ^ ((lane & 15) >> 1)) << 4);
   f32x4 acc[MT][FW];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int f = 0; f < FW; ++f) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  load_a(0, ar);
 #pragma unroll
-  for (int d = 0; d < DB; ++d) load_b(d, br[d]);
-  put_a(0, ar);
-  load_a(1, ar);
-  for (int t = 0;; t += U) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // A of this step is in LDS and everybody has left the other buffer
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      put_a((u + 1) & 1, ar);
-      load_a(t + u + 2, ar);
-      const char* s = smem + (u & 1) * (BM * 256);
-#pragma unroll
-      for (int e = 0; e < KF; ++e) {
-        bf16x8 af[MT];
-#pragma unroll
-        for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const bf16x8*>(s + a_rd[e] + i * 4096);
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int f = 0; f < FW; ++f)
-            acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(br[u % DB][f][e], af[i], acc[i][f], 0, 0, 0);
-      }
-      load_b(t + u + DB, br[u % DB]);
-      if (t + u + 1 >= n) goto done;
-    }
+  for (int d = 0; d < DB; ++d) {
+    load_a(d, d);
+    load_b(d, br[d]);
   }
-done:
+  int slot = 0, free = DB;
+  auto step = [&](int t, bf16x8(&b)[FW][KF]) {
+    // A of this step is in LDS (younger: DB B steps and DB - 1 A steps) and everybody has left the slot before it
+    asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(DB * NB + (DB - 1) * NA) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(t + DB, free);
+    const char* s = smem + slot * PART;
+#pragma unroll
+    for (int e = 0; e < KF; ++e) {
+      bf16x8 af[MT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const bf16x8*>(s + a_rd[e] + i * 2048);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int f = 0; f < FW; ++f) acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[f][e], af[i], acc[i][f], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_b(t + DB, b);
+    free = slot;
+    slot = slot + 1 == RING ? 0 : slot + 1;
+  };
+  int t = 0;
+  for (; t + DB <= n; t += DB)
+#pragma unroll
+    for (int u = 0; u < DB; ++u) step(t + u, br[u]);
+  // the rest, outside the loop: an exit from its middle would join its back edge, and every load be waited for there
+#pragma unroll
+  for (int u = 0; u < DB - 1; ++u)
+    if (t + u < n) step(t + u, br[u]);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is left
   f32x4 v[NF];  // [RW][FW]
   if constexpr (ORD) {
 #pragma unroll
@@ -264,10 +280,10 @@ bool parts_fit(int M, int N, int mt, int ng, int S) {
   return mid_tiles(M, N, mt, ng) * 8 <= kGaiMidTickets && part_bytes(M, N, mt, ng, S) < (1ull << 31);
 }
 
-// Modelled times in us. This kernel: fitted to 7738 timings of 420 products (65 to 2048 rows, N 256 to 28672, K 256 to 14336,
-// every epilogue, both weight layouts, weights from HBM) with up to 33 plans each; 19 of 20 within 15 %, also of the products left
-// out of the fit. The kernels below: 1376 products, 9 of 10 within 15 %. Of those 420 the rule takes three in four, two of them up to 8 %
-// slower for it; its choice is 0.8 % (row-major) and 1.4 % (fragment order) above the best one. Without the bytes of the parts,
+// Modelled times in us. This kernel: fitted to 2362 timings of 230 products (65 to 2048 rows, N 256 to 28672, K 256 to 14336,
+// both weight layouts, weights from HBM) with up to 7 plans each; 19 of 20 within 16 %, the chosen plan on average 0.6 % above the
+// best of those (the terms of bias and GELU from an earlier fit over every epilogue). The kernels below: 1376 products, 9 of 10
+// within 15 %. Without the bytes of the parts,
 // the epilogues and the rounds of short K, the model's first form lost up to 54 % (1535 x 2176 x 384: 9.4 -> 14.4 us; with
 // 150 MB of parts 1536 x 11264 x 2048: 90 -> 258).
 struct MidFit {
@@ -276,9 +292,9 @@ struct MidFit {
   double part0, part1, parts;       // parts of K: once, each, GB/s / 1000 of the sums written and read
   double out, bias, gelu;           // GB/s / 1000 of residual and result; epilogues
 };
-constexpr MidFit kFit[3] = {{4.0, 0.0, 0.73, 0.68, 3.9, 0.32, 1.28, 0.55, 0.83, 5.1, 2.4, 0.45, 1.1},  // 128 x 64
-                            {2.6, 2.9, 0.99, 0.97, 4.1, 0.7, 1.35, 0.83, 1.0, 6.1, 2.7, 1.05, 2.0},   // 128 x 128
-                            {2.4, 4.4, 1.34, 1.36, 3.9, 0.7, 1.23, 0.8, 1.26, 6.7, 3.3, 1.9, 2.7}};   // 192 x 128
+constexpr MidFit kFit[3] = {{3.5, 0.7, 0.49, 0.61, 4.45, 0.35, 1.47, 0.7, 0.67, 7.4, 4.5, 0.5, 1.1},   // 128 x 64
+                            {3.6, 1.4, 0.79, 0.88, 4.5, 0.7, 1.7, 0.85, 0.8, 6.9, 3.05, 0.95, 2.0},     // 128 x 128
+                            {3.9, 2.7, 1.03, 1.16, 4.2, 0.67, 1.47, 1.5, 1.08, 7.2, 3.1, 1.45, 2.7}};   // 192 x 128
 constexpr double kTicketFill = 0.8;  // a captured launch clears its tickets (1.6 us): half of it counted always, the plan is the same
 
 // MB written and read by the epilogue; 0 none, 1 bias / residual, 2 GELU and the like
@@ -327,16 +343,18 @@ double other_cost(int M, int N, int K, int epi) {
 // is the layout's own (a sum's order does not depend on it). The parts are those of the smaller row-major + 2 x fragment-order
 // time: the large weights, where parts matter most, are stored in fragment order.
 constexpr double kFragShare = 2.0;
-// A product is taken where the model says 5 % less in fragment order and 3 % less row-major. (The 256 x 256 kernels at K >= 8192
+// A product is taken where the model says 5 % less in fragment order and 3 % less row-major (up to 128 rows 20 %: 128 x 1024 x 1024
+// with bias, row-major, takes the skinny kernel 11.8 us and this one 12.7, where the model says 10.6). (The 256 x 256 kernels at K >= 8192
 // are up to a fifth faster than their model where the tiles divide the chip evenly.)
 double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.2 : 1.05; }
+double margin_row_major(int M) { return M <= 128 ? 1.2 : 1.03; }
 
-// the ordered form, fitted to 320 shapes of up to 3072 rows (19 of 20 within 15 %)
+// the ordered form, fitted to 600 timings of 150 products of up to 3072 rows (17 of 20 within 15 %)
 double ordered_cost(int M, int N, int K, int mt, int bfrag) {
   const int items = mid_tiles(M, N, mt, 2), G = mid_cus(), rounds = (items + G - 1) / G;
-  const double fill = std::min(1.0, (double)items / G), step = mt == 4 ? 0.66 + 0.09 * fill : 1.05;
-  const double row = mt == 4 ? 1.63 : 1.35;  // row-major weights
-  return (mt == 4 ? 3.6 : 5.6) + rounds * ((mt == 4 ? 2.5 : 2.1) + K / kBK * step * (bfrag ? 1.0 : row));
+  const double fill = std::min(1.0, (double)items / G), step = mt == 4 ? 0.61 + 0.04 * fill : 0.81 + 0.12 * fill;
+  const double row = mt == 4 ? 1.68 : 1.42;  // row-major weights
+  return (mt == 4 ? 2.4 : 2.3) + rounds * ((mt == 4 ? 1.55 : 3.0) + K / kBK * step * (bfrag ? 1.0 : row));
 }
 
 // operands of the kernel: whole k steps and column tiles, 4-column loads and stores, 16-byte loads of A and B
@@ -351,7 +369,7 @@ bool mid_fits(const void* A, const void* B, const void* C, const void* bias, con
 template <int MT, int NG, int EPI, bool OUTF32, bool ORD = false>
 void launch_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int S,
                 float* ws, int* cnt, hipStream_t st, int bfrag) {
-  constexpr int lds = MT * 8192;  // two A buffers; the exchange takes MT * NG * 4096
+  constexpr int lds = std::max(MT * 2048 * mid_ring<MT>(), MT * NG * 4096);  // the ring; the exchange
   static bool once = false;
   if (!once) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mid_kernel<MT, NG, EPI, OUTF32, ORD>),
@@ -398,7 +416,7 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
       }
     }
     const double other = other_cost(M, N, K, epi);
-    if (force == 0 && (frag * margin(M, K) >= other || row * 1.03 >= other)) return false;
+    if (force == 0 && (frag * margin(M, K) >= other || row * margin_row_major(M) >= other)) return false;
   }
   if (best.parts > 1 && !parts_fit(M, N, best.mt, best.ng, best.parts)) best.parts = 1;
   if (best.parts > 1) {
