@@ -292,7 +292,7 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, 
                  const Tensor& ctx_lens, Tensor& out, Tensor& ws_o, Tensor& ws_ml, double scale, int64_t split_keys,
                  int64_t max_splits, double k_scale, double v_scale, const c10::optional<Tensor>& split_cnt,
                  const c10::optional<Tensor>& qkv_part, int64_t part_ks, const c10::optional<Tensor>& positions,
-                 const c10::optional<Tensor>& cos_sin, const c10::optional<Tensor>& slots) {
+                 const c10::optional<Tensor>& cos_sin, const c10::optional<Tensor>& slots, bool queue) {
   check_bf16(q, "q");
   const int f8 = kv_cache_fp8(k_cache, v_cache);
   check_i32(block_tables, "block_tables");
@@ -334,10 +334,11 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, 
     fold.slots = slots->data_ptr<int>();
     fp = &fold;
   }
+  TORCH_CHECK(!queue || (cnt && split_cnt->numel() >= (int64_t)B * Hkv + kGaiDecodeQueueInts), "attn_decode: no room for the queues");
   gai_attn_decode(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr<int>(),
                   block_tables.size(1), ctx_lens.data_ptr<int>(), out.data_ptr(), ws_o.data_ptr<float>(),
                   ws_ml.data_ptr<float>(), B, Hq, Hkv, D, (float)scale, split_keys, max_splits, f8, (float)k_scale,
-                  (float)v_scale, cur_stream(), cnt, fp);
+                  (float)v_scale, cur_stream(), cnt, fp, queue);
 }
 
 int64_t gemm_qkv_partials(const Tensor& A, const Tensor& W, Tensor& ws, bool psw) {
@@ -1090,11 +1091,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_rows_per_tile", [](int64_t hq, int64_t hkv, int64_t d) { return gai_attn_prefill_rows_per_tile(hq, hkv, d); },
         py::arg("hq"), py::arg("hkv"), py::arg("d") = 128);
   m.def("attn_prefill_set_hl", [](int64_t hl) { gai_attn_prefill_set_hl((int)hl); });
+  m.attr("DECODE_QUEUE_INTS") = kGaiDecodeQueueInts;
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("scale"), py::arg("split_keys"),
         py::arg("max_splits"), py::arg("k_scale"), py::arg("v_scale"), py::arg("split_cnt") = py::none(),
         py::arg("qkv_part") = py::none(), py::arg("part_ks") = 0, py::arg("positions") = py::none(),
-        py::arg("cos_sin") = py::none(), py::arg("slots") = py::none());
+        py::arg("cos_sin") = py::none(), py::arg("slots") = py::none(), py::arg("queue") = false);
   m.def("sample", &sample, py::arg("logits"), py::arg("temperature"), py::arg("top_p"), py::arg("top_k"),
         py::arg("seeds"), py::arg("step"), py::arg("out"), py::arg("ws") = py::none());
   m.def("sample_ws_bytes", &sample_ws_bytes);

@@ -84,11 +84,13 @@ struct GaiQkvFold {
   const float* cos_sin = nullptr;
   const int* slots = nullptr;
 };
+// ints behind the B * Hkv tickets of split_cnt that queue = true counts its draws in: 0 before a launch and 0 again after it
+constexpr int kGaiDecodeQueueInts = 8 * 32;
 void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                      int max_blocks, const int* ctx_lens, void* out, float* ws_o, float* ws_ml, int B, int Hq,
                      int Hkv, int D, float scale, int split_keys, int max_splits, int kv_fp8, float k_scale,
                      float v_scale, hipStream_t st, int* split_cnt = nullptr,
-                     const GaiQkvFold* fold = nullptr);
+                     const GaiQkvFold* fold = nullptr, bool queue = false);
 // QKV partial slabs only (for GaiQkvFold): KS (2..8) when launched, 0 when the shape runs elsewhere.
 int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st);
 

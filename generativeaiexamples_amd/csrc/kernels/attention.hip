@@ -18,6 +18,7 @@
 // column, so K and V^T are read once per kv head with 16-B / 8-B loads straight to
 // VGPRs (memory-bound decode row of the glds-vs-register table); the 4 waves
 // combine through LDS, splits are merged by attn_decode_reduce.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <unordered_map>
@@ -755,6 +756,241 @@ __device__ __forceinline__ void merge_splits(const float* ws_o, const float* ws_
   }
 }
 
+// A wave step covers H halves of 32 keys (2 pages each). Per half: K rows for the QK^T MFMA (lane:
+// key row lane&15, 16 B of dims 32t + 8gq) and V^T columns for the PV MFMA.
+//  * V16 = false: S row m of MFMA i is key 16i + m; P^T's k order is then {4gq..4gq+3, 16+4gq..+3}
+//    and V^T is read as two 8-B pieces (one per page).
+//  * V16 = true: row m of MFMA i is key 8(m>>2) + 4i + (m&3), so lane group gq ends up holding the
+//    8 CONSECUTIVE keys 8gq..8gq+7 of P^T, and its V^T operand is one 16-B load (page gq>>1, keys
+//    8(gq&1)..+7): half the V load instructions.
+// Addresses of a chunk past the split are clamped to its last page (unconditional loads: a
+// data-dependent branch around them would force vmcnt(0) waits), and such keys are masked.
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+// physical blocks of a chunk's pages (scalar loads). The non-pipelined loop looks the NEXT chunk's blocks up
+// before issuing this chunk's K/V loads, so a K/V load never waits on a block-table round trip of its own.
+template <int H>
+struct DecBlk {
+  int b[H][2];
+};
+template <int H>
+__device__ __forceinline__ void dec_lookup(const int* bt, int kb, int last_page, int ctx, DecBlk<H>& o) {
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const int p0 = min(kb / kBS + 2 * h, last_page);
+    o.b[h][0] = bt[p0];
+    o.b[h][1] = (p0 + 1) * kBS < ctx ? bt[p0 + 1] : o.b[h][0];
+  }
+}
+// An fp8 K row is read 16 B at a time (8-B reads of 16 rows each end at 4.75 TB/s of a stream, 16-B ones at 6.4): lane group gq
+// then holds two 8-B pieces, 2gq and 2gq + 1 of the 64 dims. Two swaps put them where two MFMAs want them: x piece gq, y piece
+// 4 + gq. (Rows of 16 lanes, x | y: 0 2 4 6 | 1 3 5 7 -> 0 1 4 5 | 2 3 6 7 -> 0 1 2 3 | 4 5 6 7.)
+__device__ __forceinline__ void swap_pieces(unsigned& x, unsigned& y) {
+  const auto a = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(a[0], a[1], false, false);
+  x = b[0];
+  y = b[1];
+}
+template <int D, int H, bool V16, typename KV, bool NTL>
+struct DecChunk {
+  // fp8 caches: chunks hold the raw 8-byte pieces, converted to bf16 right before their MFMA
+  using Raw = typename std::conditional<sizeof(KV) == 1, uint2, bf16x8>::type;
+  Raw k[H][2][D / 32];
+  bf16x4_t vlo[H][V16 ? 1 : D / 16], vhi[H][V16 ? 1 : D / 16];
+  Raw v8[H][V16 ? D / 16 : 1];
+
+  __device__ __forceinline__ void load(const KV* kc, const KV* vc, int Hkv, int g, const DecBlk<H>& bl) {
+    const int lane = threadIdx.x & 63, gq = lane >> 4;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int blk0 = bl.b[h][0], blk1 = bl.b[h][1];
+      const size_t pb0 = ((size_t)blk0 * Hkv + g) * kBS * D, pb1 = ((size_t)blk1 * Hkv + g) * kBS * D;
+      if (V16) {
+        const int m = lane & 15;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int key = 8 * (m >> 2) + 4 * i + (m & 3);  // 0..31 inside the half
+          const KV* row = kc + (key < 16 ? pb0 : pb1) + (size_t)(key & 15) * D;
+          if constexpr (sizeof(KV) == 1) {
+#pragma unroll
+            for (int t = 0; t < D / 32; t += 2) {  // (as loaded; add() puts the pieces in their places)
+              const uint4 x = *reinterpret_cast<const uint4*>(row + 32 * t + 16 * gq);
+              k[h][i][t] = uint2{x.x, x.y};
+              k[h][i][t + 1] = uint2{x.z, x.w};
+            }
+          } else {
+            // K is read with the default policy even under NTL: one load instruction covers 16 key rows x 64 B, so
+            // each 128-B line is requested in two halves by consecutive instructions, and the second half then hits
+            // the line the first one allocated in L2 (B = 64, ctx 2535 graph replay 7.251 / 7.236 -> 7.149 /
+            // 7.169 ms per step, profiles/r6/decode/k_policy_ab); V^T loads cover whole lines and stay non-temporal
+#pragma unroll
+            for (int t = 0; t < D / 32; ++t) k[h][i][t] = *reinterpret_cast<const Raw*>(row + 32 * t + 8 * gq);
+          }
+        }
+        const size_t pbv = gq < 2 ? pb0 : pb1;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+          const Raw* vp = reinterpret_cast<const Raw*>(vc + pbv + (size_t)(16 * dt + (lane & 15)) * kBS + 8 * (gq & 1));
+          if constexpr (NTL) v8[h][dt] = __builtin_nontemporal_load(vp);
+          else v8[h][dt] = *vp;
+        }
+      } else if constexpr (sizeof(KV) == 2) {
+#pragma unroll
+        for (int t = 0; t < D / 32; ++t) {
+          k[h][0][t] = load8((const bf16*)kc + pb0 + (size_t)(lane & 15) * D + 32 * t + 8 * gq);
+          k[h][1][t] = load8((const bf16*)kc + pb1 + (size_t)(lane & 15) * D + 32 * t + 8 * gq);
+        }
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+          const size_t off = (size_t)(16 * dt + (lane & 15)) * kBS + 4 * gq;
+          vlo[h][dt] = *reinterpret_cast<const bf16x4_t*>((const bf16*)vc + pb0 + off);
+          vhi[h][dt] = *reinterpret_cast<const bf16x4_t*>((const bf16*)vc + pb1 + off);
+        }
+      }
+    }
+  }
+};
+// a wave's running attention over its chunks: O^T[d = 16dt + 4gq + r][q = lane&15], maximum and sum (log2 domain)
+template <int D>
+struct DecAcc {
+  f32x4 o[D / 16];
+  float m, l;
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m = kNeg;
+    l = 0.f;
+  }
+  template <int H, bool V16, typename KV, bool NTL>
+  __device__ __forceinline__ void add(int kb, int kend, const DecChunk<D, H, V16, KV, NTL>& c, const bf16x8* qf, float sl2,
+                                      float k_scale, float v_scale) {
+    const int gq = (threadIdx.x & 63) >> 4;
+    f32x4 s[H][2];
+    float mt = kNeg;
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        s[h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (sizeof(KV) == 1 && V16) {
+#pragma unroll
+          for (int t = 0; t < D / 32; t += 2) {
+            uint2 x = c.k[h][i][t], y = c.k[h][i][t + 1];
+            swap_pieces(x.x, y.x);
+            swap_pieces(x.y, y.y);
+            s[h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv_to_bf16(x, k_scale), qf[t], s[h][i], 0, 0, 0);
+            s[h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv_to_bf16(y, k_scale), qf[t + 1], s[h][i], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int t = 0; t < D / 32; ++t)
+            s[h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv_to_bf16(c.k[h][i][t], k_scale), qf[t], s[h][i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = kb + 32 * h + (V16 ? 8 * gq + 4 * i + r : 16 * i + 4 * gq + r);
+          const float x = key < kend ? s[h][i][r] * sl2 : kNeg;
+          s[h][i][r] = x;
+          mt = fmaxf(mt, x);
+        }
+      }
+    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float m_new = fmaxf(m, mt);
+    const float alpha = fexp2(m - m_new);
+    float rs = 0.f;
+    bf16x8 pf[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float pv = fexp2(s[h][i][r] - m_new);
+          rs += pv;
+          pf[h][4 * i + r] = (bf16)pv;
+        }
+    rs += __shfl_xor(rs, 16, 64);
+    rs += __shfl_xor(rs, 32, 64);
+    l = l * alpha + rs;
+    m = m_new;
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) {
+      o[dt] *= alpha;
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        bf16x8 vf;
+        if constexpr (V16) {
+          vf = kv_to_bf16(c.v8[h][dt], v_scale);
+        } else {
+          vf = bf16x8{c.vlo[h][dt][0], c.vlo[h][dt][1], c.vlo[h][dt][2], c.vlo[h][dt][3],
+                      c.vhi[h][dt][0], c.vhi[h][dt][1], c.vhi[h][dt][2], c.vhi[h][dt][3]};
+        }
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[h], o[dt], 0, 0, 0);
+      }
+    }
+  }
+};
+// QP prologue: the group's q heads from the split-K slabs (summed, rounded, rotated) into q_lds and on to qf; with `newest`
+// also the group's new key and value into the caches. Quarter-row items (4 + 4 rotation partners of one head).
+template <int D>
+__device__ __forceinline__ void dec_qp_prologue(const GaiQkvFold& fold, bf16 (*q_lds)[D], bf16x8* qf, bf16* kc, bf16* vc, int B,
+                                                int Hq, int Hkv, int seq, int g, bool newest) {
+  const int tid = threadIdx.x, gq = (tid & 63) >> 4, qi = tid & 15, ratio = Hq / Hkv;
+  constexpr int LPH = D / 8;
+  const int nh = ratio + (newest ? 2 : 0);
+  const size_t slab = (size_t)B * fold.n;
+  for (int it = tid; it < nh * LPH; it += 256) {
+    const int hh = it / LPH, i0 = (it % LPH) * 4;
+    const int habs = hh < ratio ? g * ratio + hh : hh == ratio ? Hq + g : Hq + Hkv + g;
+    const float* p1 = fold.part + (size_t)seq * fold.n + habs * D + i0;
+    float x[4] = {0.f, 0.f, 0.f, 0.f}, y[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < fold.ks; s0 += 4) {  // 4 slabs in flight; slab order from 0 (the split-K tails' rounding)
+      float4 a[4], b[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s0 + s < fold.ks) {
+          a[s] = *reinterpret_cast<const float4*>(p1 + (s0 + s) * slab);
+          b[s] = *reinterpret_cast<const float4*>(p1 + (s0 + s) * slab + D / 2);
+        }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s0 + s < fold.ks) {
+          x[0] += a[s].x; x[1] += a[s].y; x[2] += a[s].z; x[3] += a[s].w;
+          y[0] += b[s].x; y[1] += b[s].y; y[2] += b[s].z; y[3] += b[s].w;
+        }
+    }
+    bf16x4 x1, x2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x1[j] = (bf16)x[j];
+      x2[j] = (bf16)y[j];
+    }
+    if (hh < ratio) {
+      const int pp = fold.pos[seq];
+      const float4 c = *reinterpret_cast<const float4*>(fold.cos_sin + (size_t)pp * D + i0);
+      const float4 sn = *reinterpret_cast<const float4*>(fold.cos_sin + (size_t)pp * D + D / 2 + i0);
+      const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float u = (float)x1[j], w = (float)x2[j];
+        x1[j] = (bf16)(u * cc[j] - w * ss[j]);
+        x2[j] = (bf16)(w * cc[j] + u * ss[j]);
+      }
+      *reinterpret_cast<bf16x4*>(&q_lds[hh][i0]) = x1;
+      *reinterpret_cast<bf16x4*>(&q_lds[hh][i0 + D / 2]) = x2;
+    } else {
+      rope_kv_store<D, bf16>(x1, x2, seq, habs, i0, fold.pos, fold.cos_sin, fold.slots, nullptr,
+                             kc, vc, Hq, Hkv, 1, 1.f, 1.f);
+    }
+  }
+  if (newest) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the new key / value have landed before any wave reads them
+  __syncthreads();
+  const bool qv = qi < ratio;
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t)
+    qf[t] = qv ? *reinterpret_cast<const bf16x8*>(&q_lds[qi][32 * t + 8 * gq]) : bf16x8{};
+}
+
 // NTL: the V^T cache loads are non-temporal (each decode step streams the cache once; keeps it from evicting the
 // L2-resident Q / block tables / split partials)
 // Occupancy: unconstrained, the compiler takes 138 VGPRs + 32 AGPRs (2 workgroups per CU, 512 resident), and two
@@ -790,64 +1026,11 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const int qi = lane & 15;  // GQA head index inside the group (MFMA column)
 
   bf16x8 qf[D / 32];
-  // QP prologue (called after this wave's first K / V chunk is in flight, so its latency hides under the stream):
-  // quarter-row items (4 + 4 rotation partners of one head) of the group's ratio q heads, plus its k and v head in
-  // the split that holds key ctx - 1
+  // called after this wave's first K / V chunk is in flight, so its latency hides under the stream
   auto qp_prologue = [&]() {
-    constexpr int LPH = D / 8;
-    const int nh = ratio + (split == nsplit - 1 ? 2 : 0);
-    const size_t slab = (size_t)B * fold.n;
-    for (int it = tid; it < nh * LPH; it += 256) {
-      const int hh = it / LPH, i0 = (it % LPH) * 4;
-      const int habs = hh < ratio ? g * ratio + hh : hh == ratio ? Hq + g : Hq + Hkv + g;
-      const float* p1 = fold.part + (size_t)seq * fold.n + habs * D + i0;
-      float x[4] = {0.f, 0.f, 0.f, 0.f}, y[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int s0 = 0; s0 < fold.ks; s0 += 4) {  // 4 slabs in flight; slab order from 0 (the split-K tails' rounding)
-        float4 a[4], b[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          if (s0 + s < fold.ks) {
-            a[s] = *reinterpret_cast<const float4*>(p1 + (s0 + s) * slab);
-            b[s] = *reinterpret_cast<const float4*>(p1 + (s0 + s) * slab + D / 2);
-          }
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          if (s0 + s < fold.ks) {
-            x[0] += a[s].x; x[1] += a[s].y; x[2] += a[s].z; x[3] += a[s].w;
-            y[0] += b[s].x; y[1] += b[s].y; y[2] += b[s].z; y[3] += b[s].w;
-          }
-      }
-      bf16x4 x1, x2;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x1[j] = (bf16)x[j];
-        x2[j] = (bf16)y[j];
-      }
-      if (hh < ratio) {
-        const int pp = fold.pos[seq];
-        const float4 c = *reinterpret_cast<const float4*>(fold.cos_sin + (size_t)pp * D + i0);
-        const float4 sn = *reinterpret_cast<const float4*>(fold.cos_sin + (size_t)pp * D + D / 2 + i0);
-        const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float u = (float)x1[j], w = (float)x2[j];
-          x1[j] = (bf16)(u * cc[j] - w * ss[j]);
-          x2[j] = (bf16)(w * cc[j] + u * ss[j]);
-        }
-        *reinterpret_cast<bf16x4*>(&q_lds[hh][i0]) = x1;
-        *reinterpret_cast<bf16x4*>(&q_lds[hh][i0 + D / 2]) = x2;
-      } else {
-        rope_kv_store<D, bf16>(x1, x2, seq, habs, i0, fold.pos, fold.cos_sin, fold.slots, nullptr,
-                               const_cast<bf16*>(reinterpret_cast<const bf16*>(kc)),
-                               const_cast<bf16*>(reinterpret_cast<const bf16*>(vc)), Hq, Hkv, 1, 1.f, 1.f);
-      }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the new key / value have landed before any wave reads them
-    __syncthreads();
-    const bool qv = qi < ratio;
-#pragma unroll
-    for (int t = 0; t < D / 32; ++t)
-      qf[t] = qv ? *reinterpret_cast<const bf16x8*>(&q_lds[qi][32 * t + 8 * gq]) : bf16x8{};
+    if constexpr (QP)
+      dec_qp_prologue<D>(fold, q_lds, qf, const_cast<bf16*>(reinterpret_cast<const bf16*>(kc)),
+                         const_cast<bf16*>(reinterpret_cast<const bf16*>(vc)), B, Hq, Hkv, seq, g, split == nsplit - 1);
   };
   static_assert(!QP || !PIPE, "the folded QKV prologue runs in the non-pipelined loop");
   if constexpr (!QP) {
@@ -857,146 +1040,21 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     for (int t = 0; t < D / 32; ++t) qf[t] = qv ? load8(qp + 32 * t) : bf16x8{};
   }
 
-  f32x4 acc_o[D / 16];
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) acc_o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = kNeg, l_run = 0.f;
+  DecAcc<D> acc;
+  acc.clear();
   const float sl2 = scale * kLog2e;
 
-  // A wave step covers H halves of 32 keys (2 pages each). Per half: K rows for the QK^T MFMA (lane:
-  // key row lane&15, 16 B of dims 32t + 8gq) and V^T columns for the PV MFMA.
-  //  * V16 = false: S row m of MFMA i is key 16i + m; P^T's k order is then {4gq..4gq+3, 16+4gq..+3}
-  //    and V^T is read as two 8-B pieces (one per page).
-  //  * V16 = true: row m of MFMA i is key 8(m>>2) + 4i + (m&3), so lane group gq ends up holding the
-  //    8 CONSECUTIVE keys 8gq..8gq+7 of P^T, and its V^T operand is one 16-B load (page gq>>1, keys
-  //    8(gq&1)..+7): half the V load instructions.
-  // Addresses of a chunk past the split are clamped to its last page (unconditional loads: a
-  // data-dependent branch around them would force vmcnt(0) waits), and such keys are masked.
-  typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-  // fp8 caches: chunks hold the raw 8-byte pieces, converted to bf16 right before their MFMA
-  using Raw = typename std::conditional<sizeof(KV) == 1, uint2, bf16x8>::type;
-  struct Chunk {
-    Raw k[H][2][D / 32];
-    bf16x4_t vlo[H][V16 ? 1 : D / 16], vhi[H][V16 ? 1 : D / 16];
-    Raw v8[H][V16 ? D / 16 : 1];
-  };
+  using Chunk = DecChunk<D, H, V16, KV, NTL>;
+  using Blk = DecBlk<H>;
   const int last_page = (kend - 1) / kBS;
-  // physical blocks of a chunk's pages (scalar loads). The non-pipelined loop looks the NEXT chunk's blocks up
-  // before issuing this chunk's K/V loads, so a K/V load never waits on a block-table round trip of its own.
-  struct Blk {
-    int b[H][2];
-  };
-  auto lookup = [&](int kb, Blk& o) {
-#pragma unroll
-    for (int h = 0; h < H; ++h) {
-      const int p0 = min(kb / kBS + 2 * h, last_page);
-      o.b[h][0] = bt[p0];
-      o.b[h][1] = (p0 + 1) * kBS < ctx ? bt[p0 + 1] : o.b[h][0];
-    }
-  };
-  auto load_chunk_blk = [&](int kb, const Blk& bl, Chunk& c) {
-#pragma unroll
-    for (int h = 0; h < H; ++h) {
-      const int blk0 = bl.b[h][0], blk1 = bl.b[h][1];
-      const size_t pb0 = ((size_t)blk0 * Hkv + g) * kBS * D, pb1 = ((size_t)blk1 * Hkv + g) * kBS * D;
-      if (V16) {
-        const int m = lane & 15;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int key = 8 * (m >> 2) + 4 * i + (m & 3);  // 0..31 inside the half
-          const size_t pb = key < 16 ? pb0 : pb1;
-#pragma unroll
-          for (int t = 0; t < D / 32; ++t) {
-            const Raw* kp = reinterpret_cast<const Raw*>(kc + pb + (size_t)(key & 15) * D + 32 * t + 8 * gq);
-            // K is read with the default policy even under NTL: one load instruction covers 16 key rows x 64 B, so
-            // each 128-B line is requested in two halves by consecutive instructions, and the second half then hits
-            // the line the first one allocated in L2 (B = 64, ctx 2535 graph replay 7.251 / 7.236 -> 7.149 /
-            // 7.169 ms per step, profiles/r6/decode/k_policy_ab); V^T loads cover whole lines and stay non-temporal
-            c.k[h][i][t] = *kp;
-          }
-        }
-        const size_t pbv = gq < 2 ? pb0 : pb1;
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) {
-          const Raw* vp = reinterpret_cast<const Raw*>(vc + pbv + (size_t)(16 * dt + (lane & 15)) * kBS + 8 * (gq & 1));
-          if constexpr (NTL) c.v8[h][dt] = __builtin_nontemporal_load(vp);
-          else c.v8[h][dt] = *vp;
-        }
-      } else if constexpr (sizeof(KV) == 2) {
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t) {
-          c.k[h][0][t] = load8((const bf16*)kc + pb0 + (size_t)(lane & 15) * D + 32 * t + 8 * gq);
-          c.k[h][1][t] = load8((const bf16*)kc + pb1 + (size_t)(lane & 15) * D + 32 * t + 8 * gq);
-        }
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) {
-          const size_t off = (size_t)(16 * dt + (lane & 15)) * kBS + 4 * gq;
-          c.vlo[h][dt] = *reinterpret_cast<const bf16x4_t*>((const bf16*)vc + pb0 + off);
-          c.vhi[h][dt] = *reinterpret_cast<const bf16x4_t*>((const bf16*)vc + pb1 + off);
-        }
-      }
-    }
-  };
+  auto lookup = [&](int kb, Blk& o) { dec_lookup<H>(bt, kb, last_page, ctx, o); };
+  auto load_chunk_blk = [&](int, const Blk& bl, Chunk& c) { c.load(kc, vc, Hkv, g, bl); };
   auto load_chunk = [&](int kb, Chunk& c) {
     Blk bl;
     lookup(kb, bl);
-    load_chunk_blk(kb, bl, c);
+    c.load(kc, vc, Hkv, g, bl);
   };
-  auto compute_chunk = [&](int kb, const Chunk& c) {
-    f32x4 s[H][2];
-    float mt = kNeg;
-#pragma unroll
-    for (int h = 0; h < H; ++h)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        s[h][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t)
-          s[h][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv_to_bf16(c.k[h][i][t], k_scale), qf[t], s[h][i], 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kb + 32 * h + (V16 ? 8 * gq + 4 * i + r : 16 * i + 4 * gq + r);
-          const float x = key < kend ? s[h][i][r] * sl2 : kNeg;
-          s[h][i][r] = x;
-          mt = fmaxf(mt, x);
-        }
-      }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float m_new = fmaxf(m_run, mt);
-    const float alpha = fexp2(m_run - m_new);
-    float rs = 0.f;
-    bf16x8 pf[H];
-#pragma unroll
-    for (int h = 0; h < H; ++h)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float pv = fexp2(s[h][i][r] - m_new);
-          rs += pv;
-          pf[h][4 * i + r] = (bf16)pv;
-        }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * alpha + rs;
-    m_run = m_new;
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) {
-      acc_o[dt] *= alpha;
-#pragma unroll
-      for (int h = 0; h < H; ++h) {
-        bf16x8 vf;
-        if constexpr (V16) {
-          vf = kv_to_bf16(c.v8[h][dt], v_scale);
-        } else {
-          vf = bf16x8{c.vlo[h][dt][0], c.vlo[h][dt][1], c.vlo[h][dt][2], c.vlo[h][dt][3],
-                      c.vhi[h][dt][0], c.vhi[h][dt][1], c.vhi[h][dt][2], c.vhi[h][dt][3]};
-        }
-        acc_o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[h], acc_o[dt], 0, 0, 0);
-      }
-    }
-  };
+  auto compute_chunk = [&](int kb, const Chunk& c) { acc.add(kb, kend, c, qf, sl2, k_scale, v_scale); };
 
   constexpr int kStep = 128 * H;
   int kb = kstart + 32 * H * wid;
@@ -1049,13 +1107,13 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 
   // combine the 4 waves: acc_o lane layout O^T[d = 16dt + 4gq + r][q = lane&15]
   if (lane < 16) {
-    red_m[wid][lane] = m_run;
-    red_l[wid][lane] = l_run;
+    red_m[wid][lane] = acc.m;
+    red_l[wid][lane] = acc.l;
   }
 #pragma unroll
   for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red_o[wid][16 * dt + 4 * gq + r][qi] = acc_o[dt][r];
+    for (int r = 0; r < 4; ++r) red_o[wid][16 * dt + 4 * gq + r][qi] = acc.o[dt][r];
   __syncthreads();
   for (int e = tid; e < ratio * D; e += 256) {
     const int qq = e / D, d = e % D;
@@ -1102,6 +1160,194 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       out[((size_t)seq * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
     }
     if (tid == 0) __hip_atomic_store(cnt + seq * Hkv + g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The same parts of every context as attn_decode_kernel's (and the same bits), handed out longest first to the workgroups that are
+// resident: each begins with one and draws its next when it is about to finish, from the queue of its XCD (one counter for all,
+// drawn from 2048 times, took 2 - 4 us of a launch). There, of ragged contexts' parts the long ones may start last, and every part
+// starts anew with nothing in flight; here the next part's first chunk is on its way while the finished one is combined. One
+// card, 8 kv heads, graphs captured for 8192, there -> here, us: bf16, 64 sequences of 640 - 2663 keys 94.4 -> 87.7, of 40 - 700
+// 43.6 -> 33.4, 32 of 500 - 3000 57.8 -> 50.7, 23 of 1900 - 7900 92 -> 86.4; fp8 61 -> 56.8, 29.4 -> 26.0, 38.4 -> 34.0, 61.6 ->
+// 56.3. With no more parts than two a CU there is nothing to hand out (16 sequences 30.8 -> 31.7, 8 19.1 -> 20.3). Even cuts of
+// the whole batch's keys instead of each sequence's took 83, 30, 49 and 86 us, with other sums. Parts dealt beforehand, forth
+// and back, 93, 34, 54, 89. A second chunk in flight per wave changed nothing: what is left is the stream of 4-KB (2-KB) pages.
+constexpr int kQueueSeqs = 256;  // sequences that the ranking holds
+template <int D, typename KV, bool NTL, bool QP>
+__global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
+    const bf16* __restrict__ q, const KV* __restrict__ kc, const KV* __restrict__ vc, const int* __restrict__ block_tables,
+    int max_blocks, const int* __restrict__ ctx_lens, bf16* __restrict__ out, float* __restrict__ ws_o,
+    float* __restrict__ ws_ml, int B, int Hq, int Hkv, float scale, int max_splits, float k_scale, float v_scale,
+    int* __restrict__ cnt, GaiQkvFold fold) {
+  static_assert(!QP || sizeof(KV) == 2, "the folded QKV tail writes bf16 caches");
+  __shared__ __attribute__((aligned(16))) float red_o[4][D][16];
+  __shared__ float red_m[4][16], red_l[4][16];
+  __shared__ int s_last, s_next, s_total;
+  __shared__ int s_ctx[kQueueSeqs], s_parts[kQueueSeqs], s_seq[kQueueSeqs], s_first[kQueueSeqs];  // the last two by rank
+  __shared__ __attribute__((aligned(16))) bf16 q_lds[QP ? 16 : 1][QP ? D : 8];
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), gq = lane >> 4, qi = lane & 15;
+  const int ratio = Hq / Hkv;
+  const float sl2 = scale * kLog2e;
+  // sequences by falling length; the parts, one kv head after another, are numbered in that order
+  if (tid < B) {
+    const int ctx = max(ctx_lens[tid], 0);
+    s_ctx[tid] = ctx;
+    s_parts[tid] = (ctx + split_len(0, ctx, max_splits) - 1) / split_len(0, ctx, max_splits);
+  }
+  __syncthreads();
+  if (tid < B) {
+    const int ctx = s_ctx[tid];
+    int rank = 0, first = 0;
+    for (int j = 0; j < B; ++j) {
+      const bool before = s_ctx[j] > ctx || (s_ctx[j] == ctx && j < tid);
+      rank += before;
+      first += before ? s_parts[j] : 0;
+    }
+    s_seq[rank] = tid;
+    s_first[rank] = first * Hkv;
+    if (rank == B - 1) s_total = (first + s_parts[tid]) * Hkv;
+  }
+  __syncthreads();
+  const int total = __builtin_amdgcn_readfirstlane(s_total);
+  struct Part {
+    int seq, g, split, ctx, kstart, kend, nsplit;
+  };
+  auto find = [&](int item) {
+    int r = -1;  // the last rank that begins at or before item
+    for (int b0 = 0; b0 < B; b0 += 64) {
+      const int n = __popcll(__ballot(b0 + lane < B && s_first[min(b0 + lane, B - 1)] <= item));
+      r += n;
+      if (n < 64) break;
+    }
+    Part p;
+    r = __builtin_amdgcn_readfirstlane(r);
+    p.seq = __builtin_amdgcn_readfirstlane(s_seq[r]);
+    p.ctx = __builtin_amdgcn_readfirstlane(s_ctx[p.seq]);
+    const int i = item - __builtin_amdgcn_readfirstlane(s_first[r]);
+    p.split = i / Hkv;
+    p.g = i - p.split * Hkv;
+    const int len = split_len(0, p.ctx, max_splits);
+    p.nsplit = (p.ctx + len - 1) / len;
+    p.kstart = p.split * len;
+    p.kend = min(p.ctx, p.kstart + len);
+    return p;
+  };
+  // queue x: parts x, x + 8, ..; its workgroups (gridDim.x / 8) begin with the first ones and draw until nothing is left
+  const int x8 = blockIdx.x & 7, mine = (total - x8 + 7) / 8, G = gridDim.x / 8, draws = max(mine - G, 0) + G;
+  int* queue = cnt + B * Hkv + x8 * 32;  // 0 between launches
+  auto draw = [&]() { return __hip_atomic_fetch_add(queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto drew = [&](int n) {
+    if (n == draws - 1) __hip_atomic_store(queue, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  int item = blockIdx.x >> 3;
+  if (item >= mine) {
+    if (tid == 0) drew(draw());
+    return;
+  }
+
+  bf16x8 qf[D / 32];
+  DecAcc<D> acc;
+  DecBlk<1> nb;
+  DecChunk<D, 1, true, KV, NTL> c;
+  auto table = [&](const Part& p) { return block_tables + (size_t)p.seq * max_blocks; };
+  // The newest key is written by the prologue of the part that holds it: a first chunk with it is not asked for before.
+  auto early = [&](const Part& p, int kb) {
+    return kb < p.kend && !(QP && p.split == p.nsplit - 1 && kb <= p.ctx - 1 && p.ctx - 1 < kb + 32);
+  };
+  Part p = find(8 * item + x8);
+  int kb = p.kstart + 32 * wid;
+  dec_lookup<1>(table(p), kb, (p.kend - 1) / kBS, p.ctx, nb);
+  bool have = early(p, kb);
+  if (have) c.load(kc, vc, Hkv, p.g, nb);
+  for (;;) {
+    if constexpr (QP) {
+      dec_qp_prologue<D>(fold, q_lds, qf, const_cast<bf16*>(reinterpret_cast<const bf16*>(kc)),
+                         const_cast<bf16*>(reinterpret_cast<const bf16*>(vc)), B, Hq, Hkv, p.seq, p.g, p.split == p.nsplit - 1);
+    } else {
+      const bool qv = qi < ratio;
+      const bf16* qp = q + ((size_t)p.seq * Hq + p.g * ratio + (qv ? qi : 0)) * D + 8 * gq;
+#pragma unroll
+      for (int t = 0; t < D / 32; ++t) qf[t] = qv ? load8(qp + 32 * t) : bf16x8{};
+    }
+    acc.clear();
+    const int* bt = table(p);
+    const int last_page = (p.kend - 1) / kBS;
+    int drawn = 0;
+    if (!have && kb < p.kend) c.load(kc, vc, Hkv, p.g, nb);
+    while (kb < p.kend) {
+      const int next = kb + 128;
+      if (next < p.kend) dec_lookup<1>(bt, next, last_page, p.ctx, nb);
+      else if (tid == 0) drawn = draw();  // (wave 0 has keys of every part) under the last chunk's products
+      acc.add(kb, p.kend, c, qf, sl2, k_scale, v_scale);
+      if (next < p.kend) c.load(kc, vc, Hkv, p.g, nb);
+      kb = next;
+    }
+    // combine the 4 waves
+    __syncthreads();  // the previous part's sums have been read
+    if (tid == 0) {
+      s_next = G + drawn;
+      drew(drawn);
+    }
+    if (lane < 16) {
+      red_m[wid][lane] = acc.m;
+      red_l[wid][lane] = acc.l;
+    }
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red_o[wid][16 * dt + 4 * gq + r][qi] = acc.o[dt][r];
+    __syncthreads();
+    item = __builtin_amdgcn_readfirstlane(s_next);
+    const bool more = item < mine;
+    Part np = p;
+    if (more) {
+      np = find(8 * item + x8);
+      kb = np.kstart + 32 * wid;
+      dec_lookup<1>(table(np), kb, (np.kend - 1) / kBS, np.ctx, nb);
+      have = early(np, kb);
+      if (have) c.load(kc, vc, Hkv, np.g, nb);
+    }
+    for (int e = tid; e < ratio * D; e += 256) {
+      const int qq = e / D, d = e % D, hq = p.g * ratio + qq;
+      float M = kNeg, L = 0.f, O = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) M = fmaxf(M, red_m[w][qq]);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float f = fexp2(red_m[w][qq] - M);
+        L += red_l[w][qq] * f;
+        O += red_o[w][d][qq] * f;
+      }
+      if (p.nsplit == 1) {
+        out[((size_t)p.seq * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
+      } else {
+        const size_t i = ((size_t)p.split * B + p.seq) * Hq + hq;
+        st_sc1(ws_o + i * D + d, O);
+        if (d == 0) {
+          st_sc1(ws_ml + i * 2, M);
+          st_sc1(ws_ml + i * 2 + 1, L);
+        }
+      }
+    }
+    if (p.nsplit > 1) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's write-through partials have landed
+      __syncthreads();
+      if (tid == 0) s_last = __hip_atomic_fetch_add(cnt + p.seq * Hkv + p.g, 1, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT) == p.nsplit - 1;
+      __syncthreads();
+      if (s_last) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // no instruction: keeps the loads below the ticket
+        for (int e = tid; e < ratio * D; e += 256) {
+          const int qq = e / D, d = e % D, hq = p.g * ratio + qq;
+          float L, O;
+          merge_splits<true>(ws_o, ws_ml, B, Hq, D, p.seq, hq, d, p.nsplit, L, O);
+          out[((size_t)p.seq * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
+        }
+        if (tid == 0) __hip_atomic_store(cnt + p.seq * Hkv + p.g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (!more) return;
+    p = np;
   }
 }
 
@@ -1277,10 +1523,21 @@ int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D) {
   return 32 * (prefill_waves(D, ratio) / (hpw / prefill_hl(D, ratio)));
 }
 
+static int decode_cus() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus < 1)
+      gai_launch_error(__FILE__, __LINE__, "attn_decode: cannot query the CU count");
+    return cus;
+  }();
+  return n;
+}
+
 void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                      int max_blocks, const int* ctx_lens, void* out, float* ws_o, float* ws_ml, int B, int Hq,
                      int Hkv, int D, float scale, int split_keys, int max_splits, int kv_fp8, float k_scale,
-                     float v_scale, hipStream_t st, int* split_cnt, const GaiQkvFold* fold) {
+                     float v_scale, hipStream_t st, int* split_cnt, const GaiQkvFold* fold, bool queue) {
   if (B == 0) return;
   if (Hq / Hkv > 16) gai_launch_error(__FILE__, __LINE__, "attn_decode: GQA ratio > 16 unsupported");
   if (split_keys < 0 || split_keys % 128)
@@ -1296,6 +1553,22 @@ void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, co
   static const bool ntl = !(getenv("GAI_DECODE_NT") && atoi(getenv("GAI_DECODE_NT")) == 0);
   if (fold != nullptr && !(fuse && ntl && !kv_fp8 && D == 128 && fold->ks >= 1 && fold->ks <= 16))
     gai_launch_error(__FILE__, __LINE__, "attn_decode: the folded QKV tail needs the fused non-temporal bf16 kernel");
+  if (queue) {
+    if (!(fuse && D == 128 && split_keys == 0 && B <= kQueueSeqs && (kv_fp8 || ntl)))
+      gai_launch_error(__FILE__, __LINE__, "attn_decode: the queue is of the fused adaptive form of head_dim 128");
+    const GaiQkvFold f = fold ? *fold : GaiQkvFold{};
+    const int wgs = (std::min(3 * decode_cus(), B * Hkv * max_splits) + 7) & ~7;  // resident: up to 168 VGPRs, 41 KB of LDS
+#define GAI_QUEUE(KV, NT, QPF)                                                                                          \
+  attn_decode_queue_kernel<128, KV, NT, QPF><<<wgs, 256, 0, st>>>(                                                       \
+      (const bf16*)q, (const KV*)k_cache, (const KV*)v_cache, block_tables, max_blocks, ctx_lens, (bf16*)out, ws_o, ws_ml, B, \
+      Hq, Hkv, scale, max_splits, k_scale, v_scale, split_cnt, f)
+    if (fold) GAI_QUEUE(bf16, true, true);
+    else if (kv_fp8) GAI_QUEUE(fp8, false, false);
+    else GAI_QUEUE(bf16, true, false);
+#undef GAI_QUEUE
+    GAI_LAUNCH_CHECK();
+    return;
+  }
   if (fold != nullptr) {
     attn_decode_kernel<128, false, 1, true, bf16, true, true, true><<<grid, 256, 0, st>>>(
         (const bf16*)q, (const bf16*)k_cache, (const bf16*)v_cache, block_tables, max_blocks, ctx_lens, (bf16*)out,

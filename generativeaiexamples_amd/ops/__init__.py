@@ -553,6 +553,7 @@ class DecodeWorkspace:
     split can be chosen per call / per captured batch bucket (graph-capture safe)."""
 
     MIN_SPLIT = 128
+    QUEUE_INTS = 256  # kGaiDecodeQueueInts
 
     def __init__(self, max_batch: int, Hq: int, D: int, max_ctx: int, device, split_keys: int | None = None):
         self.fixed_split = split_keys
@@ -561,8 +562,9 @@ class DecodeWorkspace:
         self.o = torch.empty(self.max_splits * max_batch * Hq * D, dtype=torch.float32, device=device)
         self.ml = torch.empty(self.max_splits * max_batch * Hq * 2, dtype=torch.float32, device=device)
         # split tickets of the in-launch merge (one per (sequence, kv head) <= max_batch * Hq): zero at
-        # allocation, reset by each merge's last split
-        self.cnt = torch.zeros(max_batch * Hq, dtype=torch.int32, device=device)
+        # allocation, reset by each merge's last split; behind them the queues' counters,
+        # reset by their last draw
+        self.cnt = torch.zeros(max_batch * Hq + self.QUEUE_INTS, dtype=torch.int32, device=device)
 
     @property
     def split_keys(self) -> int:
@@ -607,6 +609,7 @@ _DECODE_MAX_SPLIT = int(os.environ.get("GAI_DECODE_MAX_SPLIT", "2048"))  # keys 
 # up to this many (sequence, kv head) pairs the split targets one resident wave of workgroups (512) instead of 1024
 _DECODE_ONE_WAVE_PAIRS = int(os.environ.get("GAI_DECODE_ONE_WAVE_PAIRS", "128"))
 _DECODE_ADAPTIVE = os.environ.get("GAI_DECODE_ADAPTIVE", "1") == "1"
+_DECODE_QUEUE = os.environ.get("GAI_DECODE_NT", "1") != "0" and os.environ.get("GAI_DECODE_VARIANT", "1") == "1"
 
 
 def attention_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, ws: DecodeWorkspace | None = None,
@@ -629,9 +632,14 @@ def attention_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, ws: Dec
     # adaptive (split_keys 0): the kernel cuts each sequence's ACTUAL context into nsplit equal parts, so graphs
     # captured for max_ctx balance their splits at every replay (GAI_DECODE_ADAPTIVE=0: fixed split_keys)
     f = qkv_fold if qkv_fold is not None else (None, 0, None, None, None)
+    adaptive = _DECODE_ADAPTIVE and ws.fixed_split is None
+    # more parts than two a CU: the same ones, handed out by the launch longest first (attention.hip has the times)
+    pairs = B * k_cache.shape[1]
+    queue = (adaptive and _DECODE_QUEUE and _ATTN_FUSE and D == 128 and nsplit > 1 and B <= 256 and pairs * nsplit > 512
+             and ws.cnt.numel() >= pairs + native().DECODE_QUEUE_INTS)
     native().attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, out, ws.o, ws.ml, scale,
-                         0 if (_DECODE_ADAPTIVE and ws.fixed_split is None) else split, nsplit, k_scale, v_scale,
-                         ws.cnt if _ATTN_FUSE else None, f[0], f[1], f[2], f[3], f[4])
+                         0 if adaptive else split, nsplit, k_scale, v_scale,
+                         ws.cnt if _ATTN_FUSE else None, f[0], f[1], f[2], f[3], f[4], queue)
     return out
 
 

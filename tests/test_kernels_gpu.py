@@ -261,6 +261,51 @@ def test_attention_decode_adaptive_splits(cuda, nsplit):
     _close(o_u, o_ref, 2e-2, 2e-2, "adaptive reduce")
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,nsplit,ctx", [
+    (32, 8, 2, [1]), (4, 4, 3, [257, 0, 128]), (16, 1, 2, [1, 127, 128, 129, 0, 0, 2049]),
+    (32, 8, 7, [2663, 31, 4097, 640, 1, 300, 2048, 255, 33, 96, 97, 1500]),
+    (64, 8, 33, [4200, 4096, 700, 700, 129]),             # a part per unit
+    (16, 4, 4, [(37 * i * i) % 701 for i in range(131)]),  # more parts than workgroups; equal lengths, empty sequences
+    (8, 8, 9, [8000, 1] * 100), (32, 8, 2, [0, 0, 0])])
+def test_attention_decode_queue(cuda, Hq, Hkv, nsplit, ctx, fp8):
+    """Parts handed out by the launch: the bits of the launch with a workgroup per part, whatever their number and order; rows of
+    sequences without keys are left alone; tickets and counters back at zero; graph replays the same."""
+    torch.manual_seed(len(ctx))
+    D, B = 128, len(ctx)
+    kc, vc, bt = _paged_setup([max(1, n) for n in ctx], Hkv, D, cuda, seed=4)
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    q = torch.randn(B, Hq, D, device=cuda, dtype=torch.bfloat16)
+    c, scale = torch.tensor(ctx, dtype=torch.int32, device=cuda), 1 / math.sqrt(D)
+    ws = ops.DecodeWorkspace(B, Hq, D, max(bt.shape[1] * 16, 128 * nsplit), cuda)
+    sk, sv = (0.5, 2.0) if fp8 else (1.0, 1.0)
+
+    def run(out, queue):
+        ops.native().attn_decode(q, kc, vc, bt, c, out, ws.o, ws.ml, scale, 0, nsplit, sk, sv, ws.cnt, queue=queue)
+
+    want, out = torch.full_like(q, 7.0), torch.full_like(q, 7.0)
+    run(want, False)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        run(out, True)
+    for i in range(6):
+        out.fill_(7.0)
+        run(out, True) if i % 2 else g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and int(ws.cnt.abs().sum()) == 0
+    live = c.cpu() > 0
+    assert (out.cpu()[~live] == 7.0).all()
+    if live.any() and B < 100:
+        k, v = (kc.float() * sk, vc.float() * sv) if fp8 else (kc, vc)
+        o_ref = ref.attention_decode(q.cpu()[live], k.cpu(), v.cpu(), bt.cpu()[live], c.cpu()[live], scale)
+        _close(out.cpu()[live], o_ref, 2e-2, 2e-2, "queue")     # test_attention_decode's bound: probabilities and result in bf16
+    with pytest.raises(RuntimeError):
+        ops.native().attn_decode(q, kc, vc, bt, c, out, ws.o, ws.ml, scale, 0, nsplit, sk, sv, ws.cnt[: B * Hkv], queue=True)
+
+
 def test_attention_decode_fused_merge_reuse(cuda):
     """In-launch split merge (ticket counters, last split combines): equal to the separate reduce launch, and
     the counters reset themselves - many back-to-back launches and graph replays on one workspace, with the
