@@ -9,9 +9,12 @@
 //   the lists of a workgroup are merged in LDS and the workgroups' lists by sim_topk_stage2;
 //   else only the largest score of every 16-row group is kept (sim_topk_stream<.., 0, ..>), and one workgroup per
 //   query picks the k best groups - which hold the k best rows - and scores their rows again (sim_topk_select).
-// us, lists / groups (first form of k > 8: a 64-entry list per lane): 1M x 1024, k = 4: 1 query 353 / 417, 300 queries
-// 1280 / 1314; k = 8: 64 queries 422 / 510, 300 queries 1375 / 1314, 100k x 384 and 100 queries 140 / 56; k = 40: 1 query
-// 1M x 1024 (18263) / 454, 100 queries 100k x 384 (20901) / 67, 300 queries 250k x 1024 (144700) / 509.
+// More than 64 queries (columns a multiple of 64, at least 256) take the groups from a tiled product instead (sim_group_max).
+// us, lists / groups (first form of k > 8: a 64-entry list per lane): 1M x 1024, k = 4, 1 query 353 / 417; k = 8, 64 queries 422 /
+// 510; k = 40, 1 query (18263) / 454. Lists / groups of the stream / of the tiled product, 300 queries: 250k x 1024, k = 4 414 / - /
+// 250, k = 8 - / 393 / 256, k = 40 (144700) / 470 / 330; 1M x 1024, k = 8 1375 / 1277 / 818; 100k x 384, k = 8 - / 92 / 85; 65
+// queries, 250k x 1024, k = 4 193 / 191 / 150. On small indexes the second pass costs more than the lists: 300 queries, 5000 x 1024,
+// k = 4 38 / 57 / 60; 30000 146 / 114 / 76.
 #include <algorithm>
 
 #include "gai_common.h"
@@ -227,6 +230,156 @@ __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ 
 }
 
 // ------------------------------------------------------------------------------------------------
+// Group maxima for many queries: a product with both operands staged in LDS. The stream above reads X again for every 64 queries, in
+// its operand layout (16 rows x 64 B a load: 37 KB/us in a CU, a quarter of what whole lines get), and a query fragment from LDS
+// for every MFMA. Here:
+//  * a workgroup takes 128 rows x 16 * QT queries (up to 320, so X is read once), waves 64 rows x half of the queries: 4 + QT / 2
+//    fragment reads for 2 * QT MFMAs of a 32-deep K step;
+//  * X and Q come by DMA, RING - 1 steps ahead and on into the workgroup's next tile of rows, the loads spread between the MFMAs;
+//    the next step's fragments are read meanwhile (one wave per SIMD, two register sets);
+//  * every output is one sum over K in order, the same bits as the stream's and the second pass's;
+//  * a group's maximum: of the four row tiles of a lane the transposed lane halves leave group 4w + (lane >> 4) in place.
+// 300 queries x 250007 rows x 1024: 370 -> 195 us (the matrix work alone 105; a CU's 32 KB of outstanding misses, shared by 8 KB of X
+// from HBM and 20 KB of Q from L2 a step, allow about 120).
+// ------------------------------------------------------------------------------------------------
+template <int QT>
+constexpr int tile_ring() { return QT >= 20 ? 5 : QT >= 16 ? 6 : QT >= 12 ? 7 : 8; }
+
+template <int QT>
+__global__ __launch_bounds__(256, 1) void sim_group_max(const bf16* __restrict__ Q, const bf16* __restrict__ X,
+                                                        const float* __restrict__ bias, int nq, int N, int D, int qblocks,
+                                                        float* __restrict__ gmax, int ngr) {
+  constexpr int RING = tile_ring<QT>(), QH = QT / 2, NL = (8 + QT) / 4, PART = (8 + QT) * 1024, NF = 4 + QH, NM = 4 * QH;
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // RING steps of 8 X and QT query fragments; two tiles' biases
+  float* bsm = reinterpret_cast<float*>(smem + RING * PART);
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wid >> 1, wq = wid & 1;
+  const int items = (N + 127) / 128 * qblocks, G = gridDim.x, nk = D / 32;
+  const int n = (items - (int)blockIdx.x + G - 1) / G;  // this workgroup's items: row tile, query block
+  if (n <= 0) return;
+  const int lrow = lane >> 2, lcol = ((lane & 3) ^ (lrow >> 2 & 3)) * 16;  // a load: 16 rows x 64 B, pieces swizzled by row
+  // prefetch position
+  __amdgpu_buffer_rsrc_t rx, rq, rb;
+  int ox[2], oq[5], ob;
+  int pit = 0, pt = 0;
+  auto aim = [&]() {
+    const int item = blockIdx.x + pit * G, r0 = item / qblocks * 128, q0 = item % qblocks * (16 * QT);
+    rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(X) + (size_t)r0 * D, (short)0, 0x7fffffff, 0x00020000);
+    rq = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(Q) + (size_t)q0 * D, (short)0, 0x7fffffff, 0x00020000);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) ox[q] = (min(r0 + (q * 4 + wid) * 16 + lrow, N - 1) - r0) * D * 2 + lcol;
+#pragma unroll
+    for (int q = 0; q < NL - 2; ++q) oq[q] = (min(q0 + (q * 4 + wid) * 16 + lrow, nq - 1) - q0) * D * 2 + lcol;
+    rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(bias) + r0, (short)0, 0x7fffffff, 0x00020000);
+    ob = (min(r0 + (wid & 1) * 64 + lane, N - 1) - r0) * 4;
+  };
+  auto load = [&](int q, int slot) {
+    char* d = smem + slot * PART + wid * 1024;
+    if (q < 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, GAI_LDS(d + q * 4096), 16, ox[q], pt * 64, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, GAI_LDS(d + q * 4096), 16, oq[q - 2], pt * 64, 0, 0);
+  };
+  auto load_bias = [&]() {  // with a tile's first step; an extra load only makes a counted wait stricter
+    if (pt == 0 && wid < 2) {
+      char* d = reinterpret_cast<char*>(bsm + (pit & 1) * 128 + wid * 64);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, GAI_LDS(d), 4, ob, 0, 0, 0);
+    }
+  };
+  auto next = [&]() {  // past the last item its last step is read again: the count of loads stays what the code says
+    if (pt + 1 < nk) ++pt;
+    else if (pit + 1 < n) {
+      ++pit;
+      pt = 0;
+      aim();
+    }
+  };
+  int rd[2];  // this wave's fragments: + 1024 each (16 rows x 64 B)
+  rd[0] = wr * 4096 + (lane & 15) * 64 + (((lane >> 4) ^ ((lane & 15) >> 2)) << 4);
+  rd[1] = (8 + wq * QH) * 1024 + (rd[0] - wr * 4096);
+  bf16x8 fr[2][NF];
+  f32x4 acc[4][QH];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < QH; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto fragment = [&](const char* s, int f) {
+    return *reinterpret_cast<const bf16x8*>(f < 4 ? s + rd[0] + f * 1024 : s + rd[1] + (f - 4) * 1024);
+  };
+  aim();
+#pragma unroll
+  for (int d = 0; d < RING; ++d) {
+    load_bias();
+#pragma unroll
+    for (int q = 0; q < NL; ++q) load(q, d);
+    __builtin_amdgcn_sched_barrier(0);
+    next();
+  }
+  asm volatile("s_waitcnt vmcnt(%c0)" ::"i"((RING - 1) * NL) : "memory");
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int f = 0; f < NF; ++f) fr[0][f] = fragment(smem, f);
+  int slot = 0;
+  auto step = [&](const bf16x8(&cur)[NF], bf16x8(&nxt)[NF]) {
+    const int ns = slot + 1 == RING ? 0 : slot + 1;
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this step's fragments in registers, its slot is free behind the barrier
+    asm volatile("s_waitcnt vmcnt(%c0)" ::"i"((RING - 2) * NL) : "memory");  // the next step's have landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    load_bias();
+    const char* s = smem + ns * PART;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      const int j = m / 4, i = m % 4;
+#pragma unroll
+      for (int f = m * NF / NM; f < (m + 1) * NF / NM; ++f) nxt[f] = fragment(s, f);
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[i], cur[4 + j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = m * NL / NM; q < (m + 1) * NL / NM; ++q) load(q, slot);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    next();
+    slot = ns;
+  };
+  auto finish = [&](int it) {
+    const int item = blockIdx.x + it * G, gr0 = item / qblocks * 8 + wr * 4, q0 = item % qblocks * (16 * QT) + wq * QH * 16;
+    f32x4 bv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      bv[i] = *reinterpret_cast<const f32x4*>(bsm + (it & 1) * 128 + wr * 64 + i * 16 + 4 * (lane >> 4));
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if ((gr0 + i) * 16 + 4 * (lane >> 4) + r >= N) bv[i][r] = -INFINITY;
+    }
+    const int g = gr0 + (lane >> 4);
+#pragma unroll
+    for (int j = 0; j < QH; ++j) {
+      float m[4];  // fmaxf passes NaN scores over
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        m[i] = fmaxf(fmaxf(fmaxf(-INFINITY, acc[i][j][0] + bv[i][0]), acc[i][j][1] + bv[i][1]),
+                     fmaxf(fmaxf(-INFINITY, acc[i][j][2] + bv[i][2]), acc[i][j][3] + bv[i][3]));
+      // lane groups 0 1 2 3 of m[0] m[1] m[2] m[3]: halves of 0 | 2 and 1 | 3, then quarters of all
+      const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[0]), __float_as_uint(m[2]), false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[1]), __float_as_uint(m[3]), false, false);
+      const float u = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1])), v = fmaxf(__uint_as_float(y[0]), __uint_as_float(y[1]));
+      const auto z = __builtin_amdgcn_permlane16_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+      const int q = q0 + 16 * j + (lane & 15);
+      if (q < nq && g < ngr) gmax[(size_t)q * ngr + g] = fmaxf(__uint_as_float(z[0]), __uint_as_float(z[1]));
+    }
+  };
+  for (int it = 0; it < n; ++it) {
+    clear();
+    for (int t = 0; t < nk; t += 2) {  // nk is even
+      step(fr[0], fr[1]);
+      step(fr[1], fr[0]);
+    }
+    finish(it);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is left
+}
+
+// ------------------------------------------------------------------------------------------------
 // k > 8, second pass: one workgroup per query. A key is (score, lowest row first) as one unsigned number, 0 = none.
 // The k groups with the largest maxima hold the k best rows: a row of another group has at least k rows before it, the
 // maxima of those groups. The same argument picks the groups: thread t's strided maximum over the group maxima, the k
@@ -430,6 +583,39 @@ struct TopkArgs {
   hipStream_t st;
 };
 
+template <int QT>
+void run_group_max(const TopkArgs& a, int qblocks) {
+  constexpr int lds = tile_ring<QT>() * (8 + QT) * 1024 + 1024;
+  static bool once = false;
+  if (!once) {
+    set_max_lds(sim_group_max<QT>, lds);
+    once = true;
+  }
+  const int items = (a.N + 127) / 128 * qblocks;
+  sim_group_max<QT><<<std::min(items, 256), 256, lds, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.nq, a.N, a.D, qblocks,
+                                                              a.ws_v, (a.N + 15) / 16);
+  GAI_LAUNCH_CHECK();
+}
+
+void run_select(const TopkArgs& a) {
+  sim_topk_select<<<a.nq, 1024, 0, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, (a.N + 15) / 16, a.N, a.D, a.k,
+                                           a.out_v, a.out_i);
+  GAI_LAUNCH_CHECK();
+}
+
+bool many_queries(const TopkArgs& a) {
+  if (a.nq <= 64 || a.D % 64 || a.D < 256 || (a.N + 15) / 16 <= a.k) return false;
+  auto off = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
+  if (off(a.Q) || off(a.X)) return false;
+  const int qblocks = (a.nq + 319) / 320, qt = ((a.nq + qblocks - 1) / qblocks + 63) / 64 * 4;
+  if (qt <= 8) run_group_max<8>(a, qblocks);
+  else if (qt <= 12) run_group_max<12>(a, qblocks);
+  else if (qt <= 16) run_group_max<16>(a, qblocks);
+  else run_group_max<20>(a, qblocks);
+  run_select(a);
+  return true;
+}
+
 template <int MT, int K, int RING>
 void run_stream_r(const TopkArgs& a) {
   constexpr int NQ = 16 * MT;
@@ -449,8 +635,7 @@ void run_stream_r(const TopkArgs& a) {
   if constexpr (K > 0)
     sim_topk_stage2<K><<<a.nq, 256, 0, a.st>>>(a.ws_v, a.ws_i, a.nwg, a.nq, a.k, a.out_v, a.out_i);
   else
-    sim_topk_select<<<a.nq, 1024, 0, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, ngr, a.N, a.D, a.k, a.out_v,
-                                             a.out_i);
+    return run_select(a);
   GAI_LAUNCH_CHECK();
 }
 
@@ -500,7 +685,10 @@ void gai_sim_topk(const void* Q, const void* X, const float* bias, int nq, int N
   if (nq == 0) return;
   if (D % 32) gai_launch_error(__FILE__, __LINE__, "sim_topk: D must be a multiple of 32");
   const TopkArgs a{Q, X, bias, nq, N, D, k, nwg, rows_per_wg, ws_v, ws_i, out_v, out_i, st};
-  if (!ws_i) return run_topk_k<0>(a);  // ws_v: the group maxima [nq][ceil(N / 16)]
+  if (!ws_i) {  // ws_v: the group maxima [nq][ceil(N / 16)]
+    if (!many_queries(a)) run_topk_k<0>(a);
+    return;
+  }
   switch (gai_topk_cap(k)) {
     case 4: return run_topk_k<4>(a);
     case 8: return run_topk_k<8>(a);

@@ -795,7 +795,8 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
     out_v = torch.empty(nq, k_eff, dtype=torch.float32, device=Q.device)
     out_i = torch.empty(nq, k_eff, dtype=torch.int64, device=Q.device)
     Q, cap = Q.contiguous(), topk_cap(k_eff)
-    if cap == 4 or (cap == 8 and nq <= 64):  # short lists in registers (topk.hip: both forms measured)
+    # short lists in registers (topk.hip has both forms' times); more than one tile of queries takes them on small indexes only
+    if cap <= 8 and (nq <= 64 or (cap == 4 and (n_rows < 16384 or D < 256 or D % 64))):
         ws_v = torch.empty(nwg * nq * cap, dtype=torch.float32, device=Q.device)
         ws_i = torch.empty(nwg * nq * cap, dtype=torch.int32, device=Q.device)
         native().sim_topk(Q, X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i)
