@@ -12,9 +12,9 @@
 // More than 64 queries (columns a multiple of 64, at least 256) take the groups from a tiled product instead (sim_group_max).
 // us, lists / groups (first form of k > 8: a 64-entry list per lane): 1M x 1024, k = 4, 1 query 353 / 417; k = 8, 64 queries 422 /
 // 510; k = 40, 1 query (18263) / 454. Lists / groups of the stream / of the tiled product, 300 queries: 250k x 1024, k = 4 414 / - /
-// 250, k = 8 - / 393 / 256, k = 40 (144700) / 470 / 330; 1M x 1024, k = 8 1375 / 1277 / 818; 100k x 384, k = 8 - / 92 / 85; 65
-// queries, 250k x 1024, k = 4 193 / 191 / 150. On small indexes the second pass costs more than the lists: 300 queries, 5000 x 1024,
-// k = 4 38 / 57 / 60; 30000 146 / 114 / 76.
+// 238, k = 8 - / 393 / 242, k = 40 (144700) / 470 / 298; 1M x 1024, k = 8 1375 / 1277 / 800; 100k x 384, k = 8 - / 94 / 77; 65
+// queries, 250k x 1024, k = 4 193 / 191 / 143. On small indexes the second pass costs more than the lists: 300 queries, 5000 x 1024,
+// k = 4 38 / 57 / 48; 30000 146 / 114 / 62.
 #include <algorithm>
 
 #include "gai_common.h"
@@ -384,8 +384,10 @@ __global__ __launch_bounds__(256, 1) void sim_group_max(const bf16* __restrict__
 // The k groups with the largest maxima hold the k best rows: a row of another group has at least k rows before it, the
 // maxima of those groups. The same argument picks the groups: thread t's strided maximum over the group maxima, the k
 // best of those 1024 threads, and of their entries the k best. The rows of the k groups (<= 1024) are scored again with
-// the stream's own instruction order and sorted. Bound by latency: 250 KB of maxima at 1M rows, k x 32 KB of X at
-// D = 1024, three 45-step selections across lanes; 300 queries run side by side on the chip.
+// the stream's own instruction order and sorted. Bound by the fetch of k x 32 KB of X at D = 1024 for every query (1.3 MB at k =
+// 40, through a CU's 32 KB of outstanding misses) and by latency: 250 KB of maxima at 1M rows, three 45-step selections across
+// lanes. Rows by DMA in whole lines instead of operand by operand: 300 queries of 250007 x 1024, k = 40 156 -> 119 us; of 5000 rows,
+// with the maxima, 124 -> 73.
 // With at most k groups (an index, or a filter's rows, of 16 k rows) all are taken: no stream, one selection. 300 queries, 60
 // rows of 1024, k = 16: 20 us, 89 with the stream and with second groups read for nothing (lists 57); 200 rows, k = 8: 48, 61
 // (lists 55).
@@ -437,13 +439,19 @@ __device__ __forceinline__ void top64(u64 x, u64* buf, u64* list) {
   __syncthreads();
 }
 
+constexpr int kSelectRows = 16 * 4096;
+
 __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__ Q, const bf16* __restrict__ X,
                                                         const float* __restrict__ bias, const float* __restrict__ gmax,
                                                         int ngr, int N, int D, int k, float* __restrict__ out_v,
                                                         int64_t* __restrict__ out_i) {
-  __shared__ u64 buf[1024], cand[1024], list[64];
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // 4 KB a wave of rows, the first 8 KB also keys; the query
+  u64* buf = reinterpret_cast<u64*>(smem);
+  bf16* qrow = reinterpret_cast<bf16*>(smem + kSelectRows);
+  __shared__ u64 cand[1024], list[64];
   __shared__ int pick[64], cnt;
-  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int e = tid; e < D / 8; e += 1024) store8(qrow + 8 * e, load8(Q + (size_t)q * D + 8 * e));
   const float* gm = gmax + (size_t)q * ngr;
   if (ngr > k) {  // else every group is taken, and gmax was not written
     u64 m = 0;
@@ -483,31 +491,83 @@ __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__
   if (tid < k) pick[tid] = ngr <= k ? (tid < ngr ? tid : -1) : list[tid] ? key_id(list[tid]) : -1;
   cand[tid] = 0;
   __syncthreads();
-  const bf16* qp = Q + (size_t)q * D + 8 * (lane >> 4);  // every column of the product is this query
-  auto rows = [&](int j) { return X + (size_t)min(16 * max(pick[min(j, k - 1)], 0) + (lane & 15), N - 1) * D + 8 * (lane >> 4); };
-  for (int j = wid; j < k && pick[j] >= 0; j += 32) {  // (the picked groups come first)
-    const bf16 *xa = rows(j), *xb = rows(j + 16);
-    f32x4 acc[2] = {};
-    if (j + 16 < k && pick[j + 16] >= 0) {  // two groups a wave
-#pragma unroll 8
-      for (int t = 0; t < D / 32; ++t) {
-        const bf16x8 qf = load8(qp + 32 * t);
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), qf, acc[0], 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xb + 32 * t), qf, acc[1], 0, 0, 0);
-      }
-    } else {
+  // group j's scores, this wave's, from the accumulator: every column of the product is this query
+  auto keep = [&](int j, const f32x4& acc) {
+    const int r = lane & 15, row = 16 * pick[j] + 4 * (lane >> 4) + r;
+    const float v = r == 0 ? acc[0] : r == 1 ? acc[1] : r == 2 ? acc[2] : acc[3];
+    if (r < 4 && row < N) cand[16 * j + 4 * (lane >> 4) + r] = make_key(v + bias[row], row);
+  };
+  if (D % 64) {
+    const bf16* qp = Q + (size_t)q * D + 8 * (lane >> 4);
+    for (int j = wid; j < k && pick[j] >= 0; j += 16) {  // (the picked groups come first)
+      const bf16* xa = X + (size_t)min(16 * pick[j] + (lane & 15), N - 1) * D + 8 * (lane >> 4);
+      f32x4 acc = {};
 #pragma unroll 8
       for (int t = 0; t < D / 32; ++t)
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), load8(qp + 32 * t), acc[0], 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xa + 32 * t), load8(qp + 32 * t), acc, 0, 0, 0);
+      keep(j, acc);
     }
-    const int r = lane & 15;
+  } else {
+    // rows by DMA in whole lines (16 rows x 64 B a load, as operands lie, come at a quarter of the rate), two 64-column pieces of
+    // 16 rows in flight per wave, on into its next group
+    int mine = 0;
+    while (wid + 16 * mine < k && pick[wid + 16 * mine] >= 0) ++mine;
+    mine = __builtin_amdgcn_readfirstlane(mine);
+    const int nc = D / 64, pieces = mine * nc;
+    char* own = reinterpret_cast<char*>(buf) + wid * 4096;
+    int pj = wid, pc = 0;  // next piece to ask for
+    int ox[2];
+    __amdgpu_buffer_rsrc_t rx;
+    auto aim = [&]() {
+      const int r0 = __builtin_amdgcn_readfirstlane(16 * pick[pj]);
+      rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(X) + (size_t)r0 * D, (short)0, 0x7fffffff, 0x00020000);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int jj = j + 16 * h;
-      if (jj >= k || pick[jj] < 0 || r >= 4) continue;
-      const int row = 16 * pick[jj] + 4 * (lane >> 4) + r;
-      const float v = r == 0 ? acc[h][0] : r == 1 ? acc[h][1] : r == 2 ? acc[h][2] : acc[h][3];
-      if (row < N) cand[16 * jj + 4 * (lane >> 4) + r] = make_key(v + bias[row], row);
+      for (int h = 0; h < 2; ++h) {
+        const int row = 8 * h + (lane >> 3);
+        ox[h] = (min(r0 + row, N - 1) - r0) * D * 2 + (((lane & 7) ^ (row >> 1)) << 4);
+      }
+    };
+    auto ask = [&](int slot) {  // past the last piece it is read again: the count of loads stays what the code says
+      char* d = own + slot * 2048;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, GAI_LDS(d + h * 1024), 16, ox[h], pc * 128, 0, 0);
+      if (pc + 1 < nc) ++pc;
+      else if (pj + 16 < wid + 16 * mine) {
+        pj += 16;
+        pc = 0;
+        aim();
+      }
+    };
+    if (mine > 0) {
+      aim();
+      ask(0);
+      ask(1);
+      const int rd = (lane & 15) * 128, sw = (lane & 15) >> 1, g = lane >> 4;
+      int j = wid, c = 0;
+      f32x4 acc = {};
+      for (int p = 0; p < pieces; ++p) {
+        const char* s = own + (p & 1) * 2048;
+        asm volatile("s_waitcnt vmcnt(2)" ::: "memory");  // the two loads of the next piece are younger
+        bf16x8 x[2], y[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          x[e] = *reinterpret_cast<const bf16x8*>(s + rd + (((4 * e + g) ^ sw) << 4));
+          y[e] = *reinterpret_cast<const bf16x8*>(qrow + 64 * c + 32 * e + 8 * g);
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this piece's slot is free
+        __builtin_amdgcn_sched_barrier(0);
+        ask(p & 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[e], y[e], acc, 0, 0, 0);
+        if (++c == nc) {
+          keep(j, acc);
+          acc = f32x4{0.f, 0.f, 0.f, 0.f};
+          c = 0;
+          j += 16;
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is left
     }
   }
   __syncthreads();
@@ -598,7 +658,12 @@ void run_group_max(const TopkArgs& a, int qblocks) {
 }
 
 void run_select(const TopkArgs& a) {
-  sim_topk_select<<<a.nq, 1024, 0, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, (a.N + 15) / 16, a.N, a.D, a.k,
+  static bool once = false;
+  if (!once) {
+    set_max_lds(sim_topk_select, 150 * 1024);  // (its own 9 KB are beside)
+    once = true;
+  }
+  sim_topk_select<<<a.nq, 1024, kSelectRows + a.D * 2, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, (a.N + 15) / 16, a.N, a.D, a.k,
                                            a.out_v, a.out_i);
   GAI_LAUNCH_CHECK();
 }
