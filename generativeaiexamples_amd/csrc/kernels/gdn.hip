@@ -9,6 +9,8 @@
 // contiguous across the workgroup), keeps its slice of the column in VGPRs between the read and the
 // write-back, and q / k live in LDS. The update is in place through `slots` (no gather / scatter copies), so the
 // launch is graph-capturable with the slot vector as a static input.
+#include <type_traits>
+
 #include "gai_common.h"
 #include "gai_kernels.h"
 
@@ -292,11 +294,258 @@ __global__ __launch_bounds__(256) void gdn_chunk_kernel(const float* __restrict_
   }
 }
 
-// The next chunk's rows are fetched while one is worked on: k in whole rows, through registers into LDS (it is read both
-// by rows and by columns), the rest straight in operand layout. Loaded by columns from memory, k made 64 loads a chunk, more
-// than the counter of outstanding loads holds, and every chunk waited for the latency of the next one's (5.9 us a chunk).
+// Of a chunk's products only k S, Ti x and k^T u are between one S and the next. Waves 0 - 3 make those, at the higher priority;
+// waves 4 - 7 make o of the chunk before meanwhile, q S and M u, and bring k into LDS (it is read both by rows and by columns). A SIMD's
+// matrix unit has 1.75 us of work a chunk (128 x 128, 16 value channels), its chain 1.1 us and the latencies of three barriers: four
+// waves that did one after the other took 4.5 us a chunk, these 3.0 (the chain by itself about 2.1). (Loaded by columns from memory, k made 64 loads a chunk,
+// more than the counter of outstanding loads holds: 5.9 us.)
 template <int DK>
-__global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
+__global__ __launch_bounds__(512, 1) void gdn_carry_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ To,
+    const float* __restrict__ Mo, const float* __restrict__ Fo, const int* __restrict__ chunks,
+    const int* __restrict__ chunk0, const int* __restrict__ slots, int Hk, int Hv, int DV, float* __restrict__ state,
+    float* __restrict__ out) {
+  constexpr int NT = DK / 16, ST = NT / 4;  // row tiles of S, of which each of four waves owns ST
+  constexpr int LK = DK + 4, KR = kC * DK / 1024;  // 16-byte pieces of a k chunk per thread of four waves
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  f32x4* Ss = reinterpret_cast<f32x4*>(sm);  // [3][NT * 64]: chunk i's at i % 3
+  f32x4* Rs = Ss + 3 * NT * 64;              // [4 * 64]
+  f32x4* Us = Rs + 4 * 64;                   // [2][4 * 64]
+  f32x4* Ud = Us + 8 * 64;                   // [4 * 64]
+  float* Ks = reinterpret_cast<float*>(Ud + 4 * 64);  // [2][64][LK]
+  const int tid = threadIdx.x & 255, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), lc = lane & 15,
+            lr = 4 * (lane >> 4);
+  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) == 0;
+  const int id = xcd_remap(blockIdx.x, gridDim.x), ns = DV / 16;  // the slices of a head share its rows in one XCD's L2
+  const int n = id % ns, h = id / ns % Hv, s = id / ns / Hv, hk = h / (Hv / Hk);
+  const int c0 = chunk0[s], nc = chunk0[s + 1] - c0;
+  if (nc <= 0) return;
+  // A chunk's rows through buffers that begin at its first row and end at its last one (past it: zeros; stores are dropped), so
+  // that a lane's offsets are the same for every chunk. The chunk's entry is read a chunk ahead of them: a scalar load
+  // and the address arithmetic of every load cost the chain 0.4 us a chunk.
+  struct Entry {
+    int t0, len;
+  };
+  auto entry = [&](int i) { return Entry{chunks[2 * (c0 + min(i, nc - 1))], chunks[2 * (c0 + min(i, nc - 1)) + 1]}; };
+  auto buffer = [&](const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, bytes, 0x00020000);
+  };
+  auto get4 = [&](const __amdgpu_buffer_rsrc_t& r, int off) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  };
+  if (chain) {
+    __builtin_amdgcn_s_setprio(3);
+    float* Sg = state + ((size_t)slots[s] * Hv + h) * DK * DV + 16 * n + lc;
+    f32x4 S[ST], kp[NT];
+#pragma unroll
+    for (int j = 0; j < ST; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[j][i] = Sg[(size_t)(16 * (ST * w + j) + lr + i) * DV];
+      Ss[(ST * w + j) * 64 + lane] = S[j];
+    }
+    struct Rows {  // this wave's 16 rows of Ti, v and the factors
+      f32x4 T[4], v, e0, ed, bt;
+      float eg;
+    };
+    int ov[4], oT[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ov[i] = ((16 * w + lr + i) * Hv * DV + lc) * 4;
+      oT[i] = ((16 * w + lc) * kC + 16 * min(i, w) + lr) * 4;
+    }
+    const int oF = (16 * w + lr) * 4;
+    auto fetch = [&](int c, const Entry& e, Rows& r) {  // past the chunk's end: beta is 0, so the row's write is
+      const size_t ch = (size_t)(c0 + c) * Hv + h;
+      const auto bv = buffer(v + ((size_t)e.t0 * Hv + h) * DV + 16 * n, (e.len - 1) * Hv * DV * 4 + 64);
+      const auto bT = buffer(To + ch * kC * kC, kC * kC * 4), bF = buffer(Fo + ch * kFac, kFac * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        r.v[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(bv, ov[i], 0, 0));
+        r.T[i] = get4(bT, oT[i]);
+      }
+      r.e0 = get4(bF, oF);
+      r.ed = get4(bF, oF + kC * 4);
+      r.bt = get4(bF, oF + 2 * kC * 4);
+      r.eg = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(bF, (kC - 1) * 4, 0, 0));
+    };
+    auto read_k = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) kp[j] = load4f(Ks + ((c & 1) * kC + 16 * w + lc) * LK + 16 * j + lr);
+    };
+    Entry ahead = entry(1);  // of the chunk after the one at work
+    auto step = [&](int c, const Rows& r, Rows& next) {
+      const float* Kb = Ks + (c & 1) * kC * LK;
+      const f32x4* Sb = Ss + c % 3 * NT * 64;
+      f32x4 p[2] = {}, u = {0.f, 0.f, 0.f, 0.f}, x, ud, kc[4][ST];
+      lds_barrier();  // S of this chunk is in LDS
+      if (c + 1 < nc) fetch(c + 1, ahead, next);
+      ahead = entry(c + 2);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) p[j & 1] = mfma4(kp[j], Sb[j * 64 + lane], p[j & 1]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = r.bt[i] * (r.v[i] - r.e0[i] * (p[0][i] + p[1][i]));
+      Rs[w * 64 + lane] = x;
+      lds_barrier();
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (m <= w) u = mfma4(r.T[m], Rs[m * 64 + lane], u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ud[i] = u[i] * r.ed[i];
+      Us[(c & 1) * 256 + w * 64 + lane] = u;
+      Ud[w * 64 + lane] = ud;
+#pragma unroll
+      for (int j = 0; j < ST; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[j][i] *= r.eg;
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) kc[m][j][i] = Kb[(16 * m + lr + i) * LK + 16 * (ST * w + j) + lc];
+      }
+      lds_barrier();  // u, and k of the next chunk
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const f32x4 um = Ud[m * 64 + lane];
+#pragma unroll
+        for (int j = 0; j < ST; ++j) S[j] = mfma4(kc[m][j], um, S[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < ST; ++j) Ss[((c + 1) % 3 * NT + ST * w + j) * 64 + lane] = S[j];
+      if (c + 1 < nc) read_k(c + 1);
+    };
+    Rows ra, rb;
+    fetch(0, entry(0), ra);
+    lds_barrier();  // k of the first chunk
+    read_k(0);
+    for (int c = 0; c < nc; c += 2) {
+      step(c, ra, rb);
+      if (c + 1 < nc) step(c + 1, rb, ra);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < ST; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Sg[(size_t)(16 * (ST * w + j) + lr + i) * DV] = S[j][i];
+  } else {
+    struct Rows {  // this wave's 16 rows of q, M and e^G
+      f32x4 Q[NT], M[4], e0;
+      Entry e;
+    };
+    f32x4 K[KR];
+    int ok[KR], oM[4], oo[4];
+#pragma unroll
+    for (int j = 0; j < KR; ++j) {
+      const int e = tid + 256 * j;
+      ok[j] = (e / (DK / 4) * Hk * DK + e % (DK / 4) * 4) * 4;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      oM[i] = ((16 * w + lc) * kC + 16 * min(i, w) + lr) * 4;
+      oo[i] = ((16 * w + lr + i) * Hv * DV + lc) * 4;
+    }
+    const int oq = ((16 * w + lc) * Hk * DK + lr) * 4, oF = (16 * w + lr) * 4;
+    auto fetch_k = [&](const Entry& e) {
+      const auto bk = buffer(k + ((size_t)e.t0 * Hk + hk) * DK, ((e.len - 1) * Hk + 1) * DK * 4);
+#pragma unroll
+      for (int j = 0; j < KR; ++j) K[j] = get4(bk, ok[j]);
+    };
+    auto stage_k = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < KR; ++j) {
+        const int e = tid + 256 * j;
+        *reinterpret_cast<f32x4*>(Ks + ((c & 1) * kC + e / (DK / 4)) * LK + e % (DK / 4) * 4) = K[j];
+      }
+    };
+    auto fetch = [&](int c, const Entry& e, Rows& r) {
+      const size_t ch = (size_t)(c0 + c) * Hv + h;
+      const auto bq = buffer(q + ((size_t)e.t0 * Hk + hk) * DK, ((e.len - 1) * Hk + 1) * DK * 4);
+      const auto bM = buffer(Mo + ch * kC * kC, kC * kC * 4);
+      r.e = e;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) r.Q[j] = get4(bq, oq + 64 * j);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r.M[i] = get4(bM, oM[i]);
+      r.e0 = get4(buffer(Fo + ch * kFac, kFac * 4), oF);
+    };
+    // operands are read ahead of the barrier that their products follow: those then run while the chain waits for its own
+    constexpr int HT = NT / 2;
+    f32x4 o[2], a[HT > 4 ? HT : 4];
+    auto read_s = [&](int c, int half) {
+#pragma unroll
+      for (int j = 0; j < HT; ++j) a[j] = Ss[(c % 3 * NT + half * HT + j) * 64 + lane];
+    };
+    auto q_s = [&](const Rows& r, auto half) {
+      constexpr int H = decltype(half)::value * HT;
+#pragma unroll
+      for (int j = 0; j < HT; ++j) o[(H + j) & 1] = mfma4(r.Q[H + j], a[j], o[(H + j) & 1]);
+    };
+    auto read_u = [&](int c) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) a[m] = Us[(c & 1) * 256 + m * 64 + lane];
+    };
+    auto rest = [&](const Rows& r) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[0][i] = r.e0[i] * (o[0][i] + o[1][i]);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (m <= w) o[0] = mfma4(r.M[m], a[m], o[0]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[0][i]),
+                                              buffer(out + ((size_t)r.e.t0 * Hv + h) * DV + 16 * n, (r.e.len - 1) * Hv * DV * 4 + 64),
+                                              oo[i], 0, 0);
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, 1>;
+    // while the others are at chunk c: o of chunk c - 1 (r), k of c + 1 into LDS, k of c + 2 and the rows of c on their way
+    Entry e0 = entry(0), e1 = entry(1), e2 = entry(2);  // of chunks c, c + 1, c + 2
+    auto step = [&](int c, const Rows& r, Rows& next) {
+      o[0] = o[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      lds_barrier();
+      if (c > 0) {
+        q_s(r, First{});
+        read_s(c - 1, 1);
+      }
+      fetch(c, e0, next);
+      e0 = e1;
+      e1 = e2;
+      e2 = entry(c + 3);
+      lds_barrier();
+      if (c > 0) {
+        q_s(r, Second{});
+        read_u(c - 1);
+      }
+      if (c + 1 < nc) {
+        stage_k(c + 1);
+        if (c + 2 < nc) fetch_k(e1);
+      }
+      lds_barrier();
+      if (c > 0) rest(r);
+      read_s(c, 0);
+    };
+    Rows ra, rb;
+    fetch_k(e0);
+    stage_k(0);
+    if (nc > 1) fetch_k(e1);
+    lds_barrier();
+    for (int c = 0; c < nc; c += 2) {
+      step(c, rb, ra);
+      if (c + 1 < nc) step(c + 1, ra, rb);
+    }
+    lds_barrier();
+    const Rows& r = nc & 1 ? ra : rb;
+    o[0] = o[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    q_s(r, First{});
+    read_s(nc - 1, 1);
+    q_s(r, Second{});
+    read_u(nc - 1);
+    rest(r);
+  }
+}
+
+// Key heads of 256: neither registers nor LDS for two chunks, and four waves do everything.
+template <int DK>
+__global__ __launch_bounds__(256, 1) void gdn_carry_wide_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ To,
     const float* __restrict__ Mo, const float* __restrict__ Fo, const int* __restrict__ chunks,
     const int* __restrict__ chunk0, const int* __restrict__ slots, int Hk, int Hv, int DV, float* __restrict__ state,
@@ -308,7 +557,7 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
   f32x4* Rs = Ss + 2 * NT * 64;              // [4 * 64] each
   f32x4* Us = Rs + 4 * 64;
   f32x4* Ud = Us + 4 * 64;
-  float* Ks = reinterpret_cast<float*>(Ud + 4 * 64);  // [2][64][LK], DK = 256: [64][LK]
+  float* Ks = reinterpret_cast<float*>(Ud + 4 * 64);  // [64][LK]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lc = lane & 15, lr = 4 * (lane >> 4);
   const int id = xcd_remap(blockIdx.x, gridDim.x), ns = DV / 16;  // the slices of a head share its rows in one XCD's L2
   const int n = id % ns, h = id / ns % Hv, s = id / ns / Hv, hk = h / (Hv / Hk);
@@ -352,17 +601,17 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
     r.bt = load4f(F + 2 * kC + 16 * w + lr);
     r.eg = F[kC - 1];
   };
-  auto stage = [&](int b, const Rows& r) {
+  auto stage = [&](const Rows& r) {
 #pragma unroll
     for (int j = 0; j < KR; ++j) {
       const int e = tid + 256 * j;
-      *reinterpret_cast<f32x4*>(Ks + (b * kC + e / (DK / 4)) * LK + e % (DK / 4) * 4) = r.K[j];
+      *reinterpret_cast<f32x4*>(Ks + e / (DK / 4) * LK + e % (DK / 4) * 4) = r.K[j];
     }
   };
   auto step = [&](int b, const Rows& r) {
     lds_barrier();  // S and k of this chunk are in LDS
     const f32x4* Sb = Ss + b * NT * 64;
-    const float* Kb = Ks + (DK <= 128 ? b * kC * LK : 0);
+    const float* Kb = Ks;
     f32x4 p[2] = {}, o[2] = {}, u = {0.f, 0.f, 0.f, 0.f}, x, ud;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
@@ -411,27 +660,12 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_kernel(
       if (t < r.len) out[((size_t)(r.t0 + t) * Hv + h) * DV + 16 * n + lc] = o[0][i];
     }
   };
-  if constexpr (DK <= 128) {
-    Rows ra, rb;
-    fetch(c0, ra);
-    stage(0, ra);
-    for (int c = c0; c < c1; c += 2) {
-      if (c + 1 < c1) fetch(c + 1, rb);
-      step(0, ra);
-      if (c + 1 >= c1) break;
-      stage(1, rb);
-      if (c + 2 < c1) fetch(c + 2, ra);
-      step(1, rb);
-      if (c + 2 < c1) stage(0, ra);
-    }
-  } else {  // neither registers nor LDS for two chunks
-    for (int c = c0; c < c1; ++c) {
-      Rows r;
-      fetch(c, r);
-      lds_barrier();  // the last chunk's k has been read
-      stage(0, r);
-      step((c - c0) & 1, r);
-    }
+  for (int c = c0; c < c1; ++c) {
+    Rows r;
+    fetch(c, r);
+    lds_barrier();  // the last chunk's k has been read
+    stage(r);
+    step((c - c0) & 1, r);
   }
 #pragma unroll
   for (int j = 0; j < ST; ++j)
@@ -485,7 +719,7 @@ void gai_gdn_prep(const void* proj, int ld, const float* cw, const float* cstate
   gai_launch_error(__FILE__, __LINE__, "gdn_prep: key head dim must be 64, 128 or 256");
 }
 
-// 6000 + 4095 tokens, 8 key / 16 value heads of 128 x 128: gdn_chunk 101 us, gdn_carry 437 us (94 chunks in a row at 4.7 us,
+// 6000 + 4095 tokens, 8 key / 16 value heads of 128 x 128: gdn_chunk 101 us, gdn_carry 290 us (94 chunks in a row at 3.0 us,
 // 256 workgroups), against 47 ms for the same rule as batched fp32 products and triangular solves chunk by chunk in torch;
 // error of o against float64 2.2e-7 - 3.4e-7 (torch 3.2e-7 - 1.1e-6).
 void gai_gdn_chunks(const float* q, const float* k, const float* v, const float* g, const float* beta, const int* chunks,
@@ -495,19 +729,21 @@ void gai_gdn_chunks(const float* q, const float* k, const float* v, const float*
 #define GAI_GDN(D)                                                                                                      \
   if (DK == D) {                                                                                                        \
     const int lds = (kC * (D + 4) + 2 * kC * (kC + 4)) * 4;                                                             \
-    const int lds2 = (2 * D / 16 + 12) * 64 * 16 + (D <= 128 ? 2 : 1) * kC * (D + 4) * 4;                               \
+    constexpr bool wide = D > 128;                                                                                      \
+    const int lds2 = ((wide ? 2 : 3) * D / 16 + (wide ? 12 : 16)) * 64 * 16 + (wide ? 1 : 2) * kC * (D + 4) * 4;         \
+    auto carry = wide ? gdn_carry_wide_kernel<256> : gdn_carry_kernel<wide ? 128 : D>;                                    \
     static bool once = false;                                                                                           \
     if (!once) {                                                                                                        \
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gdn_chunk_kernel<D>),                                     \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);                                       \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gdn_carry_kernel<D>),                                     \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(carry),                                                   \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds2);                                      \
       once = true;                                                                                                      \
     }                                                                                                                   \
     gdn_chunk_kernel<D><<<dim3(nc, Hv), 256, lds, st>>>(q, k, g, beta, chunks, Hk, Hv, Ti, M, F);                       \
     GAI_LAUNCH_CHECK();                                                                                                 \
-    gdn_carry_kernel<D><<<S * Hv * (DV / 16), 256, lds2, st>>>(q, k, v, Ti, M, F, chunks, chunk0, slots, Hk, Hv, DV,    \
-                                                               state, out);                                             \
+    carry<<<S * Hv * (DV / 16), wide ? 256 : 512, lds2, st>>>(q, k, v, Ti, M, F, chunks, chunk0, slots, Hk, Hv, DV,      \
+                                                              state, out);                                              \
     GAI_LAUNCH_CHECK();                                                                                                 \
     return;                                                                                                             \
   }
