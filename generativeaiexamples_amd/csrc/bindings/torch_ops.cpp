@@ -273,6 +273,22 @@ void attn_prefill(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
                    (float)k_scale, (float)v_scale, cur_stream(), (int)q.stride(0));
 }
 
+// self-attention over packed rows [T, 3 H 64]; tiles as attn_prefill's
+void attn_rows(const Tensor& qkv, const Tensor& tiles, const Tensor& cu_q, const Tensor& ctx_lens, Tensor& out, int64_t H,
+               double scale, bool causal) {
+  check_bf16(qkv, "qkv");
+  check_i32(tiles, "tiles");
+  check_i32(cu_q, "cu_q");
+  check_i32(ctx_lens, "ctx_lens");
+  check_bf16(out, "out");
+  TORCH_CHECK(qkv.dim() == 2 && qkv.is_contiguous() && H > 0 && qkv.size(1) == 3 * H * 64, "attn_rows: qkv [T, 3 H 64]");
+  TORCH_CHECK(out.is_contiguous() && out.numel() == qkv.size(0) * H * 64, "attn_rows: out [T, H 64]");
+  TORCH_CHECK(cu_q.numel() == ctx_lens.numel() + 1, "attn_rows: cu_q");
+  TORCH_CHECK(qkv.numel() * 2 < (int64_t)1 << 31, "attn_rows: rows beyond 32-bit offsets");
+  gai_attn_rows(qkv.data_ptr(), (int)qkv.size(1), tiles.data_ptr<int>(), tiles.numel() / 2, cu_q.data_ptr<int>(),
+                ctx_lens.data_ptr<int>(), out.data_ptr(), (int)H, (float)scale, causal ? 1 : 0, cur_stream());
+}
+
 void kv_pack(const Tensor& qkv, const Tensor& blk_tok, const Tensor& blk_n, Tensor& k_cache, Tensor& v_cache,
              int64_t Hq, int64_t Hkv, int64_t D) {
   check_bf16(qkv, "qkv");
@@ -1090,6 +1106,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_pack", &kv_pack);
   m.def("attn_prefill_rows_per_tile", [](int64_t hq, int64_t hkv, int64_t d) { return gai_attn_prefill_rows_per_tile(hq, hkv, d); },
         py::arg("hq"), py::arg("hkv"), py::arg("d") = 128);
+  m.def("attn_rows", &attn_rows);
   m.def("attn_prefill_set_hl", [](int64_t hl) { gai_attn_prefill_set_hl((int)hl); });
   m.attr("DECODE_QUEUE_INTS") = kGaiDecodeQueueInts;
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),

@@ -111,7 +111,11 @@ __device__ __forceinline__ bf16x8 kv_to_bf16(uint2 v, float s) { return fp8x8_to
 // LDS; the next K and V tiles are staged in two register sets during the iteration.
 // NWV = waves per workgroup: 4 (two workgroups per CU) or 8 (one; the row groups of two 4-wave workgroups share each
 // staged K / V^T tile, halving the tile loads and LDS writes per FLOP; head_dim 64 / 128, one head per wave)
-template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4>
+// ROWS: keys and values straight from the packed rows that q is in (self-attention of an encoder; kc / vc = the first row's key /
+// value of head 0, q_ld apart), instead of from pages that a kernel before has packed: 61 passages of e5-large 25 + 66 -> 68 us a
+// layer, a question 4.2 + 5.4 -> 5.3. V is turned on its way into LDS: a thread fetches two dims of eight keys, 4 B each
+// (whole lines across the wave), and writes two rows of the V^T image. head_dim 64, a kv head per q head.
+template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4, bool ROWS = false>
 __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) void attn_prefill_kernel(
     const bf16* __restrict__ q, const KV* __restrict__ kc, const KV* __restrict__ vc,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ tiles,
@@ -147,7 +151,8 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
   }
   const int seq = tiles[2 * bx], qs = tiles[2 * bx + 1];
   const int qbeg = cu_q[seq], qlen = cu_q[seq + 1] - qbeg;
-  const int ctx = ctx_lens[seq];
+  const int ctx = ROWS ? min(ctx_lens[seq], qlen) : ctx_lens[seq];
+  static_assert(!ROWS || (D == 64 && HPW == 1 && HL == 1 && !PIPE && NWV == 4 && sizeof(KV) == 2), "rows: encoder heads of 64");
   const int head = by * HPW + HL * (wid % WPR);  // first of this wave's HL heads
   const int g = (by * HPW) / (Hq / Hkv);
   const int r0 = qs + 32 * (wid / WPR);  // first q row (within the sequence) of this wave
@@ -236,6 +241,44 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
   };
   auto write_k = [&](int buf) { write_k_from(buf, stg); };
   auto write_v = [&](int buf) { write_v_from(buf, stg); };
+  // ROWS: tile kt's rows (past the context its last one: masked, and finite where the rows are)
+  const bf16 *rk = reinterpret_cast<const bf16*>(kc) + (size_t)qbeg * q_ld + g * D,
+             *rv = reinterpret_cast<const bf16*>(vc) + (size_t)qbeg * q_ld + g * D;
+  auto rows_k = [&](int kt, bf16x8(&dst)[2]) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int id = c * NTH + tid;
+      dst[c] = buf_load<bf16x8>(rk, (unsigned)(min(kt * 64 + id / 8, ctx - 1) * q_ld + id % 8 * 8) * 2);
+    }
+  };
+  auto rows_v = [&](int kt, bf16x8(&dst)[2]) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(rv), (short)0, 0x7fffffff, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const unsigned x = __builtin_amdgcn_raw_buffer_load_b32(
+          r, (unsigned)(min(kt * 64 + 8 * (tid >> 5) + e, ctx - 1) * q_ld + 2 * (tid & 31)) * 2, 0, 0);
+      const bf16x2 y = __builtin_bit_cast(bf16x2, x);
+      dst[e >> 2][2 * (e & 3)] = y[0];
+      dst[e >> 2][2 * (e & 3) + 1] = y[1];
+    }
+  };
+  auto write_rows_k = [&](int buf, const bf16x8(&src)[2]) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int id = c * NTH + tid;
+      *reinterpret_cast<bf16x8*>(smem + buf * Cfg::BUF + k_lds_off<D>(id / 8, id % 8)) = src[c];
+    }
+  };
+  auto write_rows_v = [&](int buf, const bf16x8(&src)[2]) {
+    char* sv = smem + buf * Cfg::BUF + Cfg::KBYTES;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bf16x4 x = {src[i][p], src[i][2 + p], src[i][4 + p], src[i][6 + p]};
+        *reinterpret_cast<bf16x4*>(sv + v_lds_off<D>(2 * (tid & 31) + p, 2 * (tid >> 5) + i)) = x;
+      }
+  };
 
   f32x16 acc_o[HL][D / 32];
   float m_run[HL], l_run[HL];
@@ -488,12 +531,20 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
   // one head per wave: +16 VGPRs)
   constexpr bool ESPLIT = HL == 1 && D <= 128;
   if (ntiles > 0) {
-    lookup(0);
-    load_half(kc);
-    write_k(0);
-    load_half(vc);
-    write_v(0);
-    lookup(1);
+    if constexpr (ROWS) {
+      Stage first[CH];
+      rows_k(0, stg);
+      rows_v(0, first);
+      write_rows_k(0, stg);
+      write_rows_v(0, first);
+    } else {
+      lookup(0);
+      load_half(kc);
+      write_k(0);
+      load_half(vc);
+      write_v(0);
+      lookup(1);
+    }
   }
   // Q fragments landed: without this wait the ntiles == 0 path reaches the loop header with the Q loads
   // pending, and hipcc's waitcnt pass then keeps vmcnt(7..0) in front of every tile's QK^T MFMAs, which
@@ -507,8 +558,13 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
     // latency cover; writing K right after QK^T left the K loads only the QK^T MFMAs to land in)
     Stage stv[ESPLIT ? CH : 1];
     if (more) {
-      load_half(kc);
-      if constexpr (ESPLIT) load_half_from(vc, nblk, stv);
+      if constexpr (ROWS) {
+        rows_k(kt + 1, stg);
+        rows_v(kt + 1, stv);
+      } else {
+        load_half(kc);
+        if constexpr (ESPLIT) load_half_from(vc, nblk, stv);
+      }
     }
     const char* sk = smem + cur * Cfg::BUF;
     const char* sv = sk + Cfg::KBYTES;
@@ -651,9 +707,12 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
     for (int j = 0; j < HL; ++j) l_run[j] = l_run[j] * alpha[j] + rs[j];  // per lane half (summed after the loop)
     // the next-but-one tile's page lookups (scalar loads) after the P.V reads: an SMEM load in flight makes every
     // LDS wait a full lgkmcnt(0) (the two return out of order)
-    lookup(kt + 2);  // pages past the context resolve to entry 0 (never read unmasked)
+    if constexpr (!ROWS) lookup(kt + 2);  // pages past the context resolve to entry 0 (never read unmasked)
     if (more) {
-      if constexpr (ESPLIT) {
+      if constexpr (ROWS) {
+        write_rows_k(cur ^ 1, stg);
+        write_rows_v(cur ^ 1, stv);
+      } else if constexpr (ESPLIT) {
         write_k(cur ^ 1);
         write_v_from(cur ^ 1, stv);
       } else {
@@ -1515,6 +1574,21 @@ void gai_attn_prefill(const void* q, const void* k_cache, const void* v_cache, c
   GAI_PF(256, 4)
 #undef GAI_PF
   gai_launch_error(__FILE__, __LINE__, "attn_prefill: unsupported head_dim");
+}
+
+// head_dim 64, one kv head per q head: rows [q | k | v] of H heads each, ld apart
+void gai_attn_rows(const void* qkv, int ld, const int* tiles, int ntiles, const int* cu_q, const int* ctx_lens, void* out, int H,
+                   float scale, int causal, hipStream_t st) {
+  if (ntiles == 0) return;
+  static const int prio_env = getenv("GAI_ATTN_PRIO") ? atoi(getenv("GAI_ATTN_PRIO")) : 2;
+  static const bool exact_max = getenv("GAI_ATTN_RESCALE_TH") && atoi(getenv("GAI_ATTN_RESCALE_TH")) == 0;
+  const bf16* q = (const bf16*)qkv;
+  auto kern = attn_prefill_kernel<64, 1, bf16, 1, false, 4, true>;
+  const int lds = 2 * PrefillCfg<64>::BUF;
+  set_max_lds(kern, lds);
+  kern<<<dim3(ntiles, H), 256, lds, st>>>(q, q + H * 64, q + 2 * H * 64, nullptr, 0, tiles, cu_q, ctx_lens, (bf16*)out, H, H, scale,
+                                          causal, nullptr, 1.f, 1.f, ((prio_env & 3) << 1) | (exact_max ? 8 : 0), ld);
+  GAI_LAUNCH_CHECK();
 }
 
 int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D) {

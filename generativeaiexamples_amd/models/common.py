@@ -140,16 +140,34 @@ class PackedAttention:
                     blk_n.append(min(BS, n - BS * i))
             self.pack = (torch.tensor(blk_tok, dtype=torch.int32).to(dev, non_blocking=True),
                          torch.tensor(blk_n, dtype=torch.int32).to(dev, non_blocking=True))
-        self.k_cache = torch.zeros(offs[-1] + 1, self.Hkv, BS, head_dim, device=dev, dtype=dtype)
-        self.v_cache = torch.zeros(offs[-1] + 1, self.Hkv, head_dim, BS, device=dev, dtype=dtype)
+        # heads of 64, one kv head each: the kernel reads keys and values from the QKV rows too (32-bit offsets into them), and
+        # the cache is made only if somebody asks for it
+        self.direct = (self.pack is not None and dev.type == "cuda" and head_dim == 64 and self.Hkv == num_heads
+                       and self.T * 3 * num_heads * 128 < 1 << 31)
+        self.pages = offs[-1] + 1
         self.q = torch.empty(self.T, self.H, head_dim, device=dev, dtype=dtype)
         # RoPE table [max_pos, hd] (decoder-based encoders, e.g. the Mistral reranker) or none
         self.rope = cos_sin is not None
         self.cs = cos_sin if self.rope else torch.zeros(1, head_dim, dtype=torch.float32, device=dev)
 
+    direct = False  # (subclasses that share pages between sequences)
+
+    def __getattr__(self, name):
+        from .. import ops
+        if name not in ("k_cache", "v_cache") or "pages" not in self.__dict__:
+            raise AttributeError(name)
+        page = (ops.BLOCK, self.hd) if name == "k_cache" else (self.hd, ops.BLOCK)
+        t = torch.zeros(self.pages, self.Hkv, *page, device=self.device, dtype=self.dtype)
+        setattr(self, name, t)
+        return t
+
     def __call__(self, qkv: torch.Tensor, scale: float, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """qkv [T, (H + 2 Hkv) * hd] -> attention output [T, H * hd]."""
         from .. import ops
+        if self.direct and qkv.is_contiguous():
+            o = torch.empty_like(self.q) if out is None else out.view(self.T, self.H, self.hd)
+            ops.native().attn_rows(qkv, self.tiles, self.cu_q, self.ctx, o, self.H, scale, self.causal)
+            return o.view(self.T, self.H * self.hd)
         if self.pack is not None:
             ops.kv_pack(qkv, self.pack[0], self.pack[1], self.k_cache, self.v_cache, self.H, self.Hkv, self.hd)
             q = qkv.view(self.T, self.H + 2 * self.Hkv, self.hd)[:, : self.H]

@@ -61,3 +61,24 @@ def test_gelu_epilogue_matches_exact_erf(cuda, M, N, K):
     ref = torch.nn.functional.gelu(x.float() @ w.float().t() + b.float())
     err = (y.float() - ref).abs().max().item()
     assert err <= 2e-2 * max(1.0, ref.abs().max().item()), err
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens,H,short", [([1], 1, 0), ([63, 64, 65, 1, 129], 2, 0), ([512, 7, 300, 128], 16, 0), ([96] * 5, 3, 41)])
+def test_rows_attention_equals_paged(cuda, lens, H, short, causal):
+    """Keys and values straight from the packed QKV rows: the bits of packing them into pages first; also where only the first
+    keys of each sequence count (padded batches)."""
+    torch.manual_seed(sum(lens))
+    D, T = 64, sum(lens)
+    qkv = torch.randn(T, 3 * H * D, device=cuda).to(torch.bfloat16)
+    a = PackedAttention(lens, H, D, cuda, causal=causal)
+    assert a.direct
+    if short and not causal:
+        a.ctx = (a.ctx - short).clamp_min(1)
+    out = torch.full((T, H * D), float("nan"), device=cuda, dtype=torch.bfloat16)
+    assert a(qkv, 0.2, out=out) is not None
+    ops.kv_pack(qkv, a.pack[0], a.pack[1], a.k_cache, a.v_cache, H, H, D)
+    want = torch.empty(T, H, D, device=cuda, dtype=torch.bfloat16)
+    ops.attention_prefill(qkv.view(T, 3 * H, D)[:, :H], a.k_cache, a.v_cache, a.block_tables, a.cu_q, a.ctx, 0.2, causal=causal,
+                          tiles=a.tiles, q_lens=lens, out=want)
+    assert torch.equal(out, want.view(T, H * D))
