@@ -21,16 +21,33 @@ constexpr int kWave = 64;
 
 #define GAI_LDS(p) ((__attribute__((address_space(3))) void*)(p))
 
+// Sum and maximum over a wave, in every lane; the whole wave has to be active. The butterfly over 32, 16, 8, 4, 2, 1 lanes
+// on VALU operands: half and row swaps, then DPP. After the step over 8 lanes a row of 16 holds equal values 8 apart, so a
+// rotation by 4 brings the partner of the step over 4. The pairs, and so every bit, are those of the same butterfly through
+// ds_bpermute, whose six LDS round trips (~100 clocks each, and four address instructions) these replace.
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+template <typename F>
+__device__ __forceinline__ float wave_butterfly(float v, F f) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(q[0]), __uint_as_float(q[1]));
+  v = f(v, dpp_f32<0x128>(v));   // row_ror:8
+  v = f(v, dpp_f32<0x124>(v));   // row_ror:4
+  v = f(v, dpp_f32<0x4E>(v));    // quad_perm [2, 3, 0, 1]
+  return f(v, dpp_f32<0xB1>(v));  // quad_perm [1, 0, 3, 2]
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_butterfly(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Reduce within aligned groups of `W` lanes (W power of two <= 64).
