@@ -77,8 +77,10 @@ __global__ __launch_bounds__(DK * 4) void gdn_decode_kernel(const float* __restr
 // ------------------------------------------------------------------------------------------------
 // Prompt portions. Inputs of the rule first (gdn_prep): causal depthwise convolution over four tokens + SiLU of the
 // projected q | k | v channels, unit q (x DK^-1/2) and k per key head, log decay and write strength per value head. A wave
-// owns one head's channels for RUN tokens, so the taps stay in registers and a row is read once; bound by the fp32 rows it
-// writes (10k tokens x 4096 channels: 250 MB, 100 us; as separate torch kernels 4.6 ms).
+// owns one head's channels for RUN tokens, so the taps stay in registers; all rows of the run are loaded before the first is
+// used, and a run inside one sequence takes a path without its branches. 10095 tokens x 4096 channels: 248 MB, 115 -> 78 us
+// (a load and a wait per row before), bound now by ~60 VALU instructions a channel (exponential and division at full
+// precision); as separate torch kernels 4.6 ms.
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(256) void gdn_prep_kernel(const TA* __restrict__ pr
                                                        float* __restrict__ q, float* __restrict__ k, float* __restrict__ v,
                                                        float* __restrict__ g, float* __restrict__ beta) {
   constexpr int CPL = DK / 64;  // channels per lane
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int t0 = blockIdx.x * RUN, kd = Hk * DK, vd = Hv * DV, cd = 2 * kd + vd;
   if (blockIdx.y == gridDim.y - 1) {  // gates
     for (int e = threadIdx.x; e < RUN * Hv; e += 256) {
@@ -105,16 +107,20 @@ __global__ __launch_bounds__(256) void gdn_prep_kernel(const TA* __restrict__ pr
   const int vec = blockIdx.y * 4 + wid, c0 = vec * DK + lane * CPL;
   if (c0 >= cd) return;
   const bool on_v = vec >= 2 * Hk;
-  float w[CPL][4], hist[3][CPL], x[RUN][CPL];
+  const bool full = (vec + 1) * DK <= cd;  // every lane's channels exist
+  int ci[CPL];                             // loads past the channels or the tokens read the last one: no branch parts them
 #pragma unroll
-  for (int i = 0; i < CPL; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) w[i][j] = c0 + i < cd ? cw[(size_t)(c0 + i) * 4 + j] : 0.f;
+  for (int i = 0; i < CPL; ++i) ci[i] = min(c0 + i, cd - 1);
+  float w[CPL][4];
+  TA x[RUN + 3][CPL];  // the taps' reach before the run, then the run
 #pragma unroll
   for (int r = 0; r < RUN; ++r)
 #pragma unroll
-    for (int i = 0; i < CPL; ++i)
-      x[r][i] = t0 + r < T && c0 + i < cd ? (float)proj[(size_t)(t0 + r) * ld + c0 + i] : 0.f;
+    for (int i = 0; i < CPL; ++i) x[r + 3][i] = proj[(size_t)min(t0 + r, T - 1) * ld + ci[i]];
+#pragma unroll
+  for (int i = 0; i < CPL; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[i][j] = cw[(size_t)ci[i] * 4 + j];
   int s = 0, hi = S;
   while (hi - s > 1) {
     const int mid = (s + hi) >> 1;
@@ -122,9 +128,47 @@ __global__ __launch_bounds__(256) void gdn_prep_kernel(const TA* __restrict__ pr
   }
   int first = cu[s], next = cu[s + 1];
   auto back = [&](int t, int i) -> float {  // channel i of row t, which may lie before its sequence's first
-    if (c0 + i >= cd) return 0.f;
-    return t >= first ? (float)proj[(size_t)t * ld + c0 + i] : cstate[((size_t)slots[s] * 3 + 3 + t - first) * cd + c0 + i];
+    return t >= first ? (float)proj[(size_t)t * ld + ci[i]] : cstate[((size_t)slots[s] * 3 + 3 + t - first) * cd + ci[i]];
   };
+  const float scale = vec < Hk ? 1.f / sqrtf((float)DK) : 1.f;
+  const int ldo = on_v ? vd : kd, oc = on_v ? c0 - 2 * kd : vec < Hk ? c0 : c0 - kd;
+  float* o = (on_v ? v : vec < Hk ? q : k) + oc;
+  auto row = [&](const float(&y0)[CPL], const float(&y1)[CPL], const float(&y2)[CPL], const float(&y3)[CPL], int t) {
+    float y[CPL], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+      const float a = fmaf(y3[i], w[i][3], fmaf(y2[i], w[i][2], fmaf(y1[i], w[i][1], y0[i] * w[i][0])));
+      y[i] = a / (1.f + expf(-a));
+      ss += y[i] * y[i];
+    }
+    if (!on_v) {
+      const float inv = rsqrtf(wave_sum(ss) + 1e-6f) * scale;
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) y[i] *= inv;
+    }
+#pragma unroll
+    for (int i = 0; i < CPL; ++i)
+      if (full || c0 + i < cd) o[(size_t)t * ldo + i] = y[i];
+  };
+  if (t0 - 3 >= first && t0 + RUN <= T && t0 + RUN <= next) {  // all of one sequence's rows
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) x[j][i] = proj[(size_t)(t0 - 3 + j) * ld + ci[i]];
+    float f[4][CPL];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) f[j][i] = (float)x[j][i];
+#pragma unroll
+    for (int r = 0; r < RUN; ++r) {
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) f[(r + 3) & 3][i] = (float)x[r + 3][i];
+      row(f[r & 3], f[(r + 1) & 3], f[(r + 2) & 3], f[(r + 3) & 3], t0 + r);
+    }
+    return;
+  }
+  float hist[3][CPL];
 #pragma unroll
   for (int j = 0; j < 3; ++j)
 #pragma unroll
@@ -142,25 +186,15 @@ __global__ __launch_bounds__(256) void gdn_prep_kernel(const TA* __restrict__ pr
 #pragma unroll
         for (int i = 0; i < CPL; ++i) hist[j][i] = back(t - 3 + j, i);
     }
-    float y[CPL], ss = 0.f;
+    float now[CPL];
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) now[i] = (float)x[r + 3][i];
+    row(hist[0], hist[1], hist[2], now, t);
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
-      const float a = fmaf(x[r][i], w[i][3], fmaf(hist[2][i], w[i][2], fmaf(hist[1][i], w[i][1], hist[0][i] * w[i][0])));
-      y[i] = a / (1.f + expf(-a));
-      ss += y[i] * y[i];
       hist[0][i] = hist[1][i];
       hist[1][i] = hist[2][i];
-      hist[2][i] = x[r][i];
-    }
-    if (!on_v) {
-      const float inv = rsqrtf(wave_sum(ss) + 1e-6f) * (vec < Hk ? 1.f / sqrtf((float)DK) : 1.f);
-      float* o = (vec < Hk ? q + (size_t)t * kd + c0 : k + (size_t)t * kd + c0 - kd);
-#pragma unroll
-      for (int i = 0; i < CPL; ++i) o[i] = y[i] * inv;
-    } else {
-#pragma unroll
-      for (int i = 0; i < CPL; ++i)
-        if (c0 + i < cd) v[(size_t)t * vd + c0 - 2 * kd + i] = y[i];
+      hist[2][i] = now[i];
     }
   }
 }
@@ -673,23 +707,60 @@ __global__ __launch_bounds__(256, 1) void gdn_carry_wide_kernel(
     for (int i = 0; i < 4; ++i) Sg[(size_t)(16 * (ST * w + j) + lr + i) * DV] = S[j][i];
 }
 
-// y = silu(z) * (w * norm(o)), one head per wave, with the roundings to the model's type of the published formulation
-// (after the norm, after the weight, at the end)
-template <typename TA>
+// y = silu(z) * (w * norm(o)), with the roundings to the model's type of the published formulation (after the norm, after
+// the weight, at the end). A wave takes R heads in a row, all of whose loads are in flight at once (10095 tokens x 16 heads
+// of 128: 165 MB, 67 -> 41 us; one head a wave waited for the row, the sum, the row again); NJ 0 reads heads of any width
+// twice.
+template <typename TA, int NJ, int R>
 __global__ __launch_bounds__(256) void gdn_out_kernel(const float* __restrict__ o, const TA* __restrict__ z, int ldz,
                                                       const TA* __restrict__ w, TA* __restrict__ y, int TH, int Hv, int DV,
                                                       float eps) {
-  const int lane = threadIdx.x & 63, th = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (th >= TH) return;
-  const float* orow = o + (size_t)th * DV;
-  float s = 0.f;
-  for (int i = lane; i < DV; i += 64) s += orow[i] * orow[i];
-  const float inv = rsqrtf(wave_sum(s) / DV + eps);
-  const TA* zr = z + (size_t)(th / Hv) * ldz + (size_t)(th % Hv) * DV;
-  for (int i = lane; i < DV; i += 64) {
-    const float zv = (float)zr[i];
-    const TA a = (TA)(orow[i] * inv), b = (TA)((float)w[i] * (float)a);
-    y[(size_t)th * DV + i] = (TA)((float)b * (zv / (1.f + expf(-zv))));
+  const int lane = threadIdx.x & 63;
+  const int th0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * R;
+  if constexpr (NJ == 0) {
+    if (th0 >= TH) return;
+    const float* orow = o + (size_t)th0 * DV;
+    float s = 0.f;
+    for (int i = lane; i < DV; i += 64) s += orow[i] * orow[i];
+    const float inv = rsqrtf(wave_sum(s) / DV + eps);
+    const TA* zr = z + (size_t)(th0 / Hv) * ldz + (size_t)(th0 % Hv) * DV;
+    for (int i = lane; i < DV; i += 64) {
+      const float zf = (float)zr[i];
+      const TA a = (TA)(orow[i] * inv), b = (TA)((float)w[i] * (float)a);
+      y[(size_t)th0 * DV + i] = (TA)((float)b * (zf / (1.f + expf(-zf))));
+    }
+    return;
+  }
+  constexpr int N = NJ ? NJ : 1;
+  float x[R][N], g[N];
+  TA zv[R][N];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int th = min(th0 + r, TH - 1);  // past the end: the last head's values, not written
+    const float* orow = o + (size_t)th * DV;
+    const TA* zr = z + (size_t)(th / Hv) * ldz + (size_t)(th % Hv) * DV;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {  // no branch parts the loads
+      const int i = min(lane + 64 * j, DV - 1);
+      x[r][j] = orow[i];
+      zv[r][j] = zr[i];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) g[j] = (float)w[min(lane + 64 * j, DV - 1)];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) s = lane + 64 * j < DV ? fmaf(x[r][j], x[r][j], s) : s;
+    const float inv = rsqrtf(wave_sum(s) / DV + eps);
+    if (th0 + r >= TH) return;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const float zf = (float)zv[r][j];
+      const TA a = (TA)(x[r][j] * inv), b = (TA)(g[j] * (float)a);
+      if (lane + 64 * j < DV) y[(size_t)(th0 + r) * DV + lane + 64 * j] = (TA)((float)b * (zf / (1.f + expf(-zf))));
+    }
   }
 }
 
@@ -758,10 +829,17 @@ void gai_gdn_out(const float* o, const void* z, int ldz, const void* w, void* y,
                  hipStream_t st) {
   const int TH = T * Hv;
   if (TH == 0) return;
-  if (dt)
-    gdn_out_kernel<float><<<(TH + 3) / 4, 256, 0, st>>>(o, (const float*)z, ldz, (const float*)w, (float*)y, TH, Hv, DV, eps);
-  else
-    gdn_out_kernel<bf16><<<(TH + 3) / 4, 256, 0, st>>>(o, (const bf16*)z, ldz, (const bf16*)w, (bf16*)y, TH, Hv, DV, eps);
+  // few heads (decode steps): one a wave, or the chip stays empty
+#define GAI_OUT(TA, NJ, R)                                                                                              \
+  gdn_out_kernel<TA, NJ, R><<<(TH + 4 * R - 1) / (4 * R), 256, 0, st>>>(o, (const TA*)z, ldz, (const TA*)w, (TA*)y, TH, Hv, \
+                                                                        DV, eps)
+#define GAI_OUT_N(TA)                                                                                                   \
+  if (DV <= 128) { if (TH > 8192) GAI_OUT(TA, 2, 4); else GAI_OUT(TA, 2, 1); }                                            \
+  else if (DV <= 256) GAI_OUT(TA, 4, 1);                                                                                \
+  else GAI_OUT(TA, 0, 1)
+  if (dt) { GAI_OUT_N(float); } else { GAI_OUT_N(bf16); }
+#undef GAI_OUT_N
+#undef GAI_OUT
   GAI_LAUNCH_CHECK();
 }
 

@@ -121,6 +121,41 @@ def test_gdn_rows_wider_than_their_tensors(cuda, Hv, dv, dt):
     assert ((y.view(T, Hv, dv).float() - want).abs() <= tol * want.abs() + 1e-30).all()
 
 
+@pytest.mark.parametrize("T,Hv,dv,dt", [(4097, 2, 128, torch.bfloat16), (2731, 3, 40, torch.float32), (3, 5, 129, torch.bfloat16),
+                                        (9, 1, 256, torch.float32), (2, 3, 300, torch.bfloat16)])
+def test_gdn_out_widths(cuda, T, Hv, dv, dt):
+    """Several heads a wave with a remainder, one head a wave, heads wider than the registers hold: against torch with the
+    same roundings (the order of up to 300 squares: one rounding of the type may fall the other way)."""
+    torch.manual_seed(dv)
+    o, w, z = torch.randn(T, Hv, dv, device=cuda), torch.randn(dv, device=cuda).to(dt), torch.randn(T, Hv * dv, device=cuda).to(dt)
+    y = ops.gdn_out(o, z, w, 1e-6)
+    n = (o * torch.rsqrt(o.pow(2).mean(-1, keepdim=True) + 1e-6)).to(dt)
+    want = (w * n).float() * torch.nn.functional.silu(z.float().view(T, Hv, dv))
+    tol = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -20
+    assert ((y.view(T, Hv, dv).float() - want).abs() <= tol * want.abs() + 1e-30).all()
+
+
+def test_gdn_prep_rows_do_not_depend_on_their_run(cuda):
+    """Rows that start, end or lie inside a run of tokens get the bits that they have one token a wave (short calls)."""
+    torch.manual_seed(2)
+    Hk, Hv, dk, dv, lens = 2, 3, 128, 40, [5, 0, 500, 11, 3, 24, 130]
+    T, cd = sum(lens), 2 * Hk * dk + Hv * dv
+    proj = torch.randn(T, cd + Hv * dv + 2 * Hv, device=cuda).to(torch.bfloat16)
+    cw, cs = torch.randn(cd, 4, device=cuda), torch.randn(len(lens), 3, cd, device=cuda)
+    A_log, dt_bias = torch.randn(Hv, device=cuda), torch.randn(Hv, device=cuda)
+    cu = torch.tensor([0] + lens).cumsum(0).to(cuda, torch.int32)
+    slots = torch.arange(len(lens), dtype=torch.int32, device=cuda)
+    many = ops.gdn_prep(proj, cw, cs, cu, slots, A_log, dt_bias, Hk, dk, Hv, dv)
+    at = 0
+    for s, n in enumerate(lens):
+        if n:
+            one = ops.gdn_prep(proj[at:at + n], cw, cs, torch.tensor([0, n], dtype=torch.int32, device=cuda), slots[s:s + 1],
+                               A_log, dt_bias, Hk, dk, Hv, dv)
+            for a, b in zip(many, one):
+                assert torch.equal(a[at:at + n], b)
+        at += n
+
+
 def _pair(cuda):
     cfg = Qwen3NextConfig.tiny()
     g = Qwen3NextModel(cfg, device=cuda).random_init(3)
