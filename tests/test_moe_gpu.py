@@ -177,6 +177,23 @@ def test_moe_dispatch_kernel_matches_stable_argsort(cuda, T, k, E):
     assert torch.equal(r.cpu().long(), order // k) and torch.equal(o.cpu().long(), want_offs)
 
 
+@pytest.mark.parametrize("T,k,E,div", [(257, 1, 1, 1), (128, 2, 512, 1), (129, 2, 513, 1), (512, 2, 512, 1), (4097, 2, 8, 1),
+                                       (1023, 8, 2048, 1), (16384, 2, 60, 1), (777, 3, 7, 9), (100, 2, 4, 16)])
+def test_moe_dispatch_edges(cuda, T, k, E, div):
+    """Waves with no rows, one row past a wave's run, one expert, the widest tables of either launch, buckets of ids: the plan
+    of a stable sort."""
+    g = torch.Generator().manual_seed(T + E)
+    ids = torch.randint(0, E * div, (T, k), generator=g, dtype=torch.int32)
+    n, flat = T * k, ids.reshape(-1).long() // div
+    order = torch.argsort(flat, stable=True)
+    new = lambda m: torch.full((m,), -7, dtype=torch.int32, device=cuda)  # noqa: E731
+    a_rows, a_pairs, offs, pos = new(n), new(n), new(E + 1), new(n).view(T, k)
+    ops.native().moe_dispatch_by(ids.to(cuda), E, div, a_rows, offs, pos, a_pairs)
+    assert torch.equal(a_pairs.cpu().long(), order) and torch.equal(a_rows.cpu().long(), order // k)
+    assert torch.equal(pos.cpu().long().reshape(-1)[order], torch.arange(n))
+    assert torch.equal(offs.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.int64), torch.bincount(flat, minlength=E).cumsum(0)]))
+
+
 @pytest.mark.parametrize("T,k,E,W", [(1, 2, 8, 2), (8, 2, 8, 2), (64, 2, 8, 4), (37, 2, 8, 8), (64, 2, 64, 4)])
 def test_ep_pack_and_combine_match_reference(cuda, T, k, E, W):
     """Native expert-parallel slab pack (counting-sorted by destination rank, expert ids in the row tails or a
