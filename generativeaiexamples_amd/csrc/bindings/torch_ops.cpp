@@ -72,6 +72,20 @@ void layernorm(const Tensor& x, const Tensor& w, const optional<Tensor>& b, doub
                 opt_ptr(b), out.data_ptr(), T, D, (float)eps, cur_stream());
 }
 
+// the product's own launches, then the norm that sums its slabs (shapes with gemm_slim_ks > 0)
+void linear_layernorm(const Tensor& A, const Tensor& W, const optional<Tensor>& bias, const Tensor& R, const Tensor& g,
+                      const optional<Tensor>& b, double eps, Tensor& out, Tensor& ws, bool psw) {
+  for (const Tensor* t : {&A, &W, &R, &g, static_cast<const Tensor*>(&out)}) check_bf16(*t, "linear_layernorm");
+  if (bias) check_bf16(*bias, "bias");
+  if (b) check_bf16(*b, "b");
+  const int64_t K = A.size(-1), M = A.numel() / K, N = g.numel(), ks = gai_gemm_slim_ks(M, N, K);
+  TORCH_CHECK(W.numel() == N * K && R.numel() == M * N && out.numel() == M * N && (!bias || bias->numel() == N) &&
+                  (!b || b->numel() == N), "linear_layernorm: sizes");
+  TORCH_CHECK(ks > 0 && ws.scalar_type() == at::kFloat && ws.numel() >= ks * M * N, "linear_layernorm: workspace");
+  gai_gemm_slim_layernorm(A.data_ptr(), W.data_ptr(), opt_ptr(bias), R.data_ptr(), g.data_ptr(), opt_ptr(b), out.data_ptr(),
+                          M, N, K, (float)eps, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
+}
+
 // KV caches are bf16, or 1-byte OCP e4m3fn (torch.float8_e4m3fn / uint8 storage) for the fp8 KV option
 int kv_cache_fp8(const Tensor& k, const Tensor& v) {
   check_dev(k, "k_cache");
@@ -1087,6 +1101,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_kv_write", &rope_kv_write);
   m.def("gemm_mid_rows", &gemm_mid_rows);
   m.def("gemm_slim_nf", &gai_gemm_slim_nf);
+  m.def("gemm_slim_ks", &gai_gemm_slim_ks);
+  m.def("linear_layernorm", &linear_layernorm);
   m.def("gemm", &gemm, pybind11::arg("A"), pybind11::arg("B"), pybind11::arg("C"), pybind11::arg("bias"),
         pybind11::arg("R"), pybind11::arg("epi"), pybind11::arg("force"), pybind11::arg("bfrag") = false);
   m.def("gemm_fp8", &gemm_fp8);

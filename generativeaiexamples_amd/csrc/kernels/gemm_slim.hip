@@ -26,6 +26,7 @@ using namespace gai;
 namespace {
 
 constexpr int kWaves = 8;
+constexpr int kMaxSlabs = 8;
 constexpr int kStageBytes = 64 * 1024;     // activation columns of one stage, all rows
 constexpr int kPairK = kWaves * 64;        // k columns of one pair step of the workgroup: 2 x 32 per wave
 // the largest K: every weight fragment of a wave's K share is in registers at once; beyond 2560 only the forms that the rule
@@ -51,7 +52,7 @@ template <int MT, int NF>
 __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* __restrict__ A,
                                                                    const bf16* __restrict__ W, void* C,
                                                                    const bf16* bias, const bf16* R, int M, int N, int K,
-                                                                   int ldc, int epi, int out_f32, int psw) {
+                                                                   int ld, int ldc, int epi, int out_f32, int psw) {
   constexpr int ROWS = 16 * MT;
   constexpr int KC = kStageBytes / (ROWS * 2);       // columns of a stage
   constexpr int CPR = KC / 8;                        // 16-B chunks of a staged row
@@ -63,6 +64,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * 16 * NF;
+  // slice blockIdx.y of a product cut over K: columns [y K, y K + K) of rows ld long, into slab y
+  const int k0 = blockIdx.y * K;
+  A += k0;
+  if (k0) C = (float*)C + (size_t)blockIdx.y * M * N;
   const int np = K / kPairK, nst = (np + P - 1) / P;
   const int r16 = lane & 15, q = lane >> 4;
 
@@ -72,8 +77,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
     const int n = min(n0 + 16 * f, N - 16);  // a fragment past N repeats the last one (not stored)
-    wp[f] = psw ? W + ((size_t)(n / 16) * (K / 32) + 2 * wid) * 512 + 8 * lane
-                : W + (size_t)(n + r16) * K + 64 * wid + 8 * q;
+    wp[f] = psw ? W + ((size_t)(n / 16) * (ld / 32) + k0 / 32 + 2 * wid) * 512 + 8 * lane
+                : W + (size_t)(n + r16) * ld + k0 + 64 * wid + 8 * q;
   }
 #pragma unroll
   for (int p = 0; p < kMaxPairs; ++p) {
@@ -101,7 +106,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
     for (int d = 0; d < DMA; ++d) {
       const int base = (d * kWaves + wid) * 64;
       const int i = base + lane, row = i / CPR, c = (i % CPR) ^ (row & 15);
-      const bf16* src = A + (size_t)min(row, M - 1) * K + min(t * KC + c * 8, K - 8);
+      const bf16* src = A + (size_t)min(row, M - 1) * ld + min(t * KC + c * 8, K - 8);
       __builtin_amdgcn_global_load_lds(src, GAI_LDS(dst + (size_t)base * 16), 16, 0, 0);
     }
   };
@@ -189,7 +194,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
 
 template <int MT, int NF>
 void launch_slim(const void* A, const void* W, void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
-                 int epi, int out_f32, int psw, hipStream_t st) {
+                 int epi, int out_f32, int psw, hipStream_t st, int ks = 1) {
   static bool once = false;
   if (!once) {
     hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_slim_kernel<MT, NF>),
@@ -197,10 +202,76 @@ void launch_slim(const void* A, const void* W, void* C, const void* bias, const 
     once = true;
   }
   constexpr int stage_k = kStageBytes / (32 * MT);
-  const size_t lds = (size_t)(K > stage_k ? 2 : 1) * kStageBytes;  // >= the partial tiles (8 MT NF KiB <= 64 KiB)
-  gemm_slim_kernel<MT, NF><<<(N + 16 * NF - 1) / (16 * NF), 64 * kWaves, lds, st>>>(
-      (const bf16*)A, (const bf16*)W, C, (const bf16*)bias, (const bf16*)R, M, N, K, ldc, epi, out_f32, psw);
+  const size_t lds = (size_t)(K / ks > stage_k ? 2 : 1) * kStageBytes;  // >= the partial tiles (8 MT NF KiB <= 64 KiB)
+  gemm_slim_kernel<MT, NF><<<dim3((N + 16 * NF - 1) / (16 * NF), ks), 64 * kWaves, lds, st>>>(
+      (const bf16*)A, (const bf16*)W, C, (const bf16*)bias, (const bf16*)R, M, N, K / ks, K, ldc, epi, out_f32, psw);
   GAI_LAUNCH_CHECK();
+}
+
+// out = LayerNorm(bf16(bf16(sum of the slabs + bias) + R)), the roundings of the product's residual epilogue; a wave a row,
+// every load of it in flight at once.
+template <int NCH>
+__global__ __launch_bounds__(64) void slabs_layernorm_kernel(const float* __restrict__ ws, int ks, int M, int N,
+                                                             const bf16* __restrict__ bias, const bf16* __restrict__ R,
+                                                             const bf16* __restrict__ g, const bf16* __restrict__ b,
+                                                             bf16* __restrict__ out, float eps) {
+  const int lane = threadIdx.x, row = blockIdx.x;
+  const size_t base = (size_t)row * N, slab = (size_t)M * N;
+  bf16x8 rv[NCH], bv[NCH], gv[NCH], lb[NCH];
+  float v[NCH][8];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int i = min((c * 64 + lane) * 8, N - 8);  // past the row: the last columns again, not counted
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[c][e] = 0.f;
+    rv[c] = load8(R + base + i);
+    gv[c] = load8(g + i);
+    bv[c] = bias ? load8(bias + i) : bf16x8{};
+    lb[c] = b ? load8(b + i) : bf16x8{};
+  }
+#pragma unroll
+  for (int k = 0; k < kMaxSlabs; ++k) {
+    if (k < ks) {
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        const float* p = ws + k * slab + base + min((c * 64 + lane) * 8, N - 8);
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[c][e] += lo[e];
+          v[c][4 + e] += hi[e];
+        }
+      }
+    }
+  }
+  float s = 0.f, q = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float y = bias ? v[c][e] + (float)bv[c][e] : v[c][e];
+      v[c][e] = (float)(bf16)((float)(bf16)y + (float)rv[c][e]);
+      s += (c * 64 + lane) * 8 < N ? v[c][e] : 0.f;
+    }
+  const float mean = wave_sum(s) / N;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float d = v[c][e] - mean;
+      q += (c * 64 + lane) * 8 < N ? d * d : 0.f;
+    }
+  const float inv = rsqrtf(wave_sum(q) / N + eps);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int i = (c * 64 + lane) * 8;
+    if (i < N) {
+      bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (bf16)((v[c][e] - mean) * inv * (float)gv[c][e] + (b ? (float)lb[c][e] : 0.f));
+      store8(out + base + i, o);
+    }
+  }
 }
 
 }  // namespace
@@ -236,4 +307,31 @@ void gai_gemm_slim(const void* A, const void* W, void* C, const void* bias, cons
   GAI_SLIM(4, 1)
   GAI_SLIM(4, 2)
 #undef GAI_SLIM
+}
+
+// Slices of K for a product whose rows a layer norm takes next (which sums the slabs): the most, up to 8, whose workgroups
+// fit the chip at once. One workgroup a 16 columns leaves most of it idle: N 1024, K 4096 has 64, each with 350 KB to fetch.
+int gai_gemm_slim_ks(int M, int N, int K) {
+  if (M < 1 || M > 64 || N < 16 || N % 16 || N > 2048 || K < 2 * kPairK || K % kPairK || (long long)N * K > (8 << 20)) return 0;
+  const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  for (int ks = kMaxSlabs; ks > 1; --ks)
+    if (K / kPairK % ks == 0 && N / 16 * ks <= 256 && K / ks <= max_k(mt, 1)) return ks;
+  return 0;
+}
+
+void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
+                             void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
+  const int ks = gai_gemm_slim_ks(M, N, K);
+  if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_slim_layernorm: the shape has no slices");
+  if (M <= 16) launch_slim<1, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
+  else if (M <= 32) launch_slim<2, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
+  else launch_slim<4, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
+#define GAI_SLN(NCH)                                                                                                     \
+  slabs_layernorm_kernel<NCH><<<M, 64, 0, st>>>(ws, ks, M, N, (const bf16*)bias, (const bf16*)R, (const bf16*)g,         \
+                                                (const bf16*)b, (bf16*)out, eps)
+  if (N <= 512) GAI_SLN(1);
+  else if (N <= 1024) GAI_SLN(2);
+  else GAI_SLN(4);
+#undef GAI_SLN
+  GAI_LAUNCH_CHECK();
 }

@@ -247,11 +247,9 @@ class BertModel:
             p = f"l{i}."
             qkv = ops.linear(h, w[p + "qkv"], bias=w[p + "qkv_b"])
             a = attn(qkv, self.scale, out=out)
-            x = ops.linear(a, w[p + "o"], bias=w[p + "o_b"], residual=h)
-            h = ops.layer_norm(x, w[p + "ln1_w"], w[p + "ln1_b"], c.ln_eps)
+            h = ops.linear_layer_norm(a, w[p + "o"], w[p + "o_b"], h, w[p + "ln1_w"], w[p + "ln1_b"], c.ln_eps)
             f = ops.linear(h, w[p + "up"], bias=w[p + "up_b"], act="gelu")
-            x = ops.linear(f, w[p + "down"], bias=w[p + "down_b"], residual=h)
-            h = ops.layer_norm(x, w[p + "ln2_w"], w[p + "ln2_b"], c.ln_eps)
+            h = ops.linear_layer_norm(f, w[p + "down"], w[p + "down_b"], h, w[p + "ln2_w"], w[p + "ln2_b"], c.ln_eps)
         return h
 
     def embed(self, ids, cu_seqlens, seq_lens) -> torch.Tensor:

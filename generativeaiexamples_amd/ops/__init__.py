@@ -153,6 +153,23 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     return out
 
 
+def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
+    """layer_norm(linear(x, w, bias, residual)). A short question's product leaves most of the chip idle with one workgroup a
+    column tile: its K is cut into slices (gemm_slim.hip) whose sums the norm adds up."""
+    if x.is_cuda and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.bfloat16:
+        K, N = x.shape[-1], w.shape[0]
+        M = x.numel() // K
+        ks = native().gemm_slim_ks(M, N, K) if M <= 64 else 0
+        if ks and residual.is_contiguous():
+            psw = decode_operand(w)
+            out = torch.empty_like(residual)
+            ws = torch.empty(ks, M, N, dtype=torch.float32, device=x.device)
+            native().linear_layernorm(x.contiguous(), w if psw is None else psw, bias, residual, ln_w, ln_b, eps, out, ws,
+                                      psw is not None)
+            return out
+    return layer_norm(linear(x, w, bias=bias, residual=residual), ln_w, ln_b, eps)
+
+
 def _fused_glu_ok(x, w, bias) -> bool:
     """The GEMMs take the GeGLU epilogue: bf16 operands on their tile grid, no bias."""
     return (x.is_cuda and isinstance(w, torch.Tensor) and bias is None and x.dtype == torch.bfloat16

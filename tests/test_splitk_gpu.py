@@ -303,3 +303,24 @@ def test_qkv_tail_graph_replays(cuda):
         torch.cuda.synchronize()
         for a, b in zip((q, kc, vc), want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("M,N,K,ks", [(1, 1024, 4096, 4), (27, 1024, 4096, 4), (33, 1024, 1024, 2), (64, 2048, 4096, 2),
+                                      (17, 384, 1536, 3), (16, 768, 3072, 3), (5, 16, 4096, 8), (31, 512, 2560, 5),
+                                      (40, 2048, 1536, 0), (65, 1024, 4096, 0)])
+@pytest.mark.parametrize("frag", [False, True])
+def test_product_in_slices_and_norm(cuda, M, N, K, ks, frag):
+    """LayerNorm(product + bias + residual) with K in slices, against float64; shapes without slices take the two ops. Error:
+    bf16 roundings of the product, of its sum with the residual and of the result (2^-9 each, the first two of values up to
+    ~6, divided by the row's deviation of ~1.4 and scaled by gains up to ~4)."""
+    torch.manual_seed(M + N)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, bias, r, g, b = bf(M, K), bf(N, K) * K ** -0.5, bf(N), bf(M, N), bf(N), bf(N)
+    assert (ops.native().gemm_slim_ks(M, N, K) if M <= 64 else 0) == ks
+    wn = w.clone()
+    if frag and ops.psw_qualifies(w):
+        assert ops.to_fragment_layout_(w)
+    y = ops.linear_layer_norm(x, w, bias, r, g, b, 1e-5)
+    v = x.double() @ wn.double().t() + bias.double() + r.double()
+    want = torch.nn.functional.layer_norm(v, (N,), g.double(), b.double(), 1e-5)
+    assert ((y.double() - want).abs() <= 2.0 ** -8 * (want.abs() + 8 * g.double().abs())).all()
