@@ -210,7 +210,7 @@ void launch_slim(const void* A, const void* W, void* C, const void* bias, const 
 
 // out = LayerNorm(bf16(bf16(sum of the slabs + bias) + R)), the roundings of the product's residual epilogue; a wave a row,
 // every load of it in flight at once.
-template <int NCH>
+template <int NCH, int KS>  // KS >= ks: slabs loaded, those past ks the last one again, not counted
 __global__ __launch_bounds__(64) void slabs_layernorm_kernel(const float* __restrict__ ws, int ks, int M, int N,
                                                              const bf16* __restrict__ bias, const bf16* __restrict__ R,
                                                              const bf16* __restrict__ g, const bf16* __restrict__ b,
@@ -230,20 +230,17 @@ __global__ __launch_bounds__(64) void slabs_layernorm_kernel(const float* __rest
     lb[c] = b ? load8(b + i) : bf16x8{};
   }
 #pragma unroll
-  for (int k = 0; k < kMaxSlabs; ++k) {
-    if (k < ks) {
+  for (int k = 0; k < KS; ++k)
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
-        const float* p = ws + k * slab + base + min((c * 64 + lane) * 8, N - 8);
-        const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
+    for (int c = 0; c < NCH; ++c) {
+      const float* p = ws + min(k, ks - 1) * slab + base + min((c * 64 + lane) * 8, N - 8);
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[c][e] += lo[e];
-          v[c][4 + e] += hi[e];
-        }
+      for (int e = 0; e < 4; ++e) {
+        v[c][e] += k < ks ? lo[e] : 0.f;
+        v[c][4 + e] += k < ks ? hi[e] : 0.f;
       }
     }
-  }
   float s = 0.f, q = 0.f;
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
@@ -326,12 +323,17 @@ void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, con
   if (M <= 16) launch_slim<1, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
   else if (M <= 32) launch_slim<2, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
   else launch_slim<4, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
-#define GAI_SLN(NCH)                                                                                                     \
-  slabs_layernorm_kernel<NCH><<<M, 64, 0, st>>>(ws, ks, M, N, (const bf16*)bias, (const bf16*)R, (const bf16*)g,         \
-                                                (const bf16*)b, (bf16*)out, eps)
-  if (N <= 512) GAI_SLN(1);
-  else if (N <= 1024) GAI_SLN(2);
-  else GAI_SLN(4);
+#define GAI_SLN(NCH, KS)                                                                                                 \
+  slabs_layernorm_kernel<NCH, KS><<<M, 64, 0, st>>>(ws, ks, M, N, (const bf16*)bias, (const bf16*)R, (const bf16*)g,     \
+                                                    (const bf16*)b, (bf16*)out, eps)
+#define GAI_SLN_K(NCH)                   \
+  if (ks <= 2) GAI_SLN(NCH, 2);          \
+  else if (ks <= 4) GAI_SLN(NCH, 4);     \
+  else GAI_SLN(NCH, kMaxSlabs)
+  if (N <= 512) { GAI_SLN_K(1); }
+  else if (N <= 1024) { GAI_SLN_K(2); }
+  else { GAI_SLN_K(4); }
+#undef GAI_SLN_K
 #undef GAI_SLN
   GAI_LAUNCH_CHECK();
 }
