@@ -23,36 +23,52 @@ __global__ __launch_bounds__(256) void embedding_kernel(const int* __restrict__ 
 
 // Pool each sequence of hidden [T, D] (varlen via cu_seqlens) into out [B, D] fp32.
 // mode 0 = masked mean, 1 = first token (CLS), 2 = last token. normalize -> v / ||v||.
-__global__ __launch_bounds__(256) void pool_kernel(const bf16* __restrict__ h, const int* __restrict__ cu,
-                                                   float* __restrict__ out, int D, int mode, int normalize) {
-  extern __shared__ float sh[];  // D floats + 16 scratch
-  float* acc = sh;
-  float* scratch = sh + D;
+// One workgroup a sequence, bound by what its CU fetches: 16-byte column units times as many row groups as 1024 threads
+// hold, eight rows of each in flight, the groups' sums added in LDS. 61 sequences of ~300 rows of 1024: one row group of 128
+// threads, a row at a time, took 142 us; now 20.
+constexpr int kPoolThreads = 1024;
+
+__global__ __launch_bounds__(kPoolThreads) void pool_kernel(const bf16* __restrict__ h, const int* __restrict__ cu,
+                                                            float* __restrict__ out, int D, int mode, int normalize) {
+  extern __shared__ float sh[];  // [groups][D] sums + 16 scratch
+  const int units = D / 8, cols = max(min(units, kPoolThreads), 1), groups = kPoolThreads / cols;
+  float* scratch = sh + groups * D;
   const int b = blockIdx.x;
   const int s0 = cu[b], s1 = cu[b + 1], n = s1 - s0;
-  for (int d = threadIdx.x; d < D; d += 256) acc[d] = 0.f;
-  __syncthreads();
   int r0 = s0, r1 = s1;
   if (mode == 1) r1 = min(s0 + 1, s1);
   if (mode == 2) r0 = max(s1 - 1, s0);
-  const int units = D / 8;
-  // each thread accumulates a fixed unit across rows
-  for (int u = threadIdx.x; u < units; u += 256) {
-    float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int r = r0; r < r1; ++r) {
-      const bf16x8 v = load8(h + (size_t)r * D + u * 8);
+  const int g = threadIdx.x / cols;
+  constexpr int U = 8;
+  if (g < groups) {
+    for (int u = threadIdx.x % cols; u < units; u += cols) {
+      float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      for (int r = r0 + g; r < r1; r += U * groups) {
+        bf16x8 v[U];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) a[j] += (float)v[j];
+        for (int i = 0; i < U; ++i) v[i] = load8(h + (size_t)min(r + i * groups, r1 - 1) * D + u * 8);
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+          if (r + i * groups < r1) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] += (float)v[i][j];
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sh[g * D + u * 8 + j] = a[j];
     }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[u * 8 + j] = a[j];
   }
   __syncthreads();
   const float div = (mode == 0 && n > 0) ? 1.f / n : 1.f;
   float ss = 0.f;
-  for (int d = threadIdx.x; d < D; d += 256) {
-    const float v = acc[d] * div;
-    acc[d] = v;
+  for (int d = threadIdx.x; d < D; d += kPoolThreads) {
+    float v = 0.f;
+    if (d < units * 8) {
+      v = sh[d];
+      for (int k = 1; k < groups; ++k) v += sh[k * D + d];
+      v *= div;
+    }
+    sh[d] = v;  // column d is this thread's alone
     ss += v * v;
   }
   float scale = 1.f;
@@ -60,7 +76,7 @@ __global__ __launch_bounds__(256) void pool_kernel(const bf16* __restrict__ h, c
     ss = block_sum(ss, scratch);
     scale = 1.f / fmaxf(sqrtf(ss), 1e-12f);
   }
-  for (int d = threadIdx.x; d < D; d += 256) out[(size_t)b * D + d] = acc[d] * scale;
+  for (int d = threadIdx.x; d < D; d += kPoolThreads) out[(size_t)b * D + d] = sh[d] * scale;
 }
 
 // MODE 0: y[t, i] = silu(x[t, i]) * x[t, I + i] (non-interleaved gate|up); 1: gelu_erf(x);
@@ -135,7 +151,8 @@ void gai_embedding(const int* ids, const void* table, void* out, int T, int D, i
 
 void gai_pool(const void* h, const int* cu, float* out, int B, int D, int mode, int normalize, hipStream_t st) {
   if (B == 0) return;
-  pool_kernel<<<B, 256, (D + 16) * sizeof(float), st>>>((const bf16*)h, cu, out, D, mode, normalize);
+  const int groups = D < 16 ? kPoolThreads : D < 8 * kPoolThreads ? kPoolThreads / (D / 8) : 1;
+  pool_kernel<<<B, kPoolThreads, (groups * D + 16) * sizeof(float), st>>>((const bf16*)h, cu, out, D, mode, normalize);
   GAI_LAUNCH_CHECK();
 }
 

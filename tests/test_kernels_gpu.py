@@ -615,6 +615,23 @@ def test_sim_topk_no_candidates(cuda):
     assert index.search_raw(X[:3], 0)[1].shape == (3, 0) and index.search(X[:3], 0) == [[], [], []]
 
 
+@pytest.mark.parametrize("D,lens", [(1024, [303, 1, 0, 65]), (384, [512, 7]), (64, [1000, 129, 128]), (8, [2000]), (8192, [3, 9]),
+                                    (8208, [2, 20])])
+@pytest.mark.parametrize("mode", ["mean", "cls", "last"])
+def test_pool_row_groups(cuda, D, lens, mode):
+    """More and fewer rows than the groups and their loads hold, one group, widths beyond it; fp32 sums of up to 2000 rows in
+    groups of at least two: error below 2000 * 2^-24 of the largest sum."""
+    torch.manual_seed(D)
+    h = torch.randn(sum(lens), D, device=cuda).to(torch.bfloat16)
+    cu = torch.tensor([0] + lens).cumsum(0).to(cuda, torch.int32)
+    got, at = ops.pool(h, cu, mode, False), 0
+    for b, n in enumerate(lens):
+        x = h[at:at + n].double()
+        want = torch.zeros(D, device=cuda).double() if n == 0 else x.mean(0) if mode == "mean" else x[0 if mode == "cls" else -1]
+        assert ((got[b].double() - want).abs() <= n * 2.0 ** -24 * (x.abs().sum(0) / max(n, 1) + 1e-30)).all()
+        at += n
+
+
 def test_embedding_pool_act(cuda):
     torch.manual_seed(10)
     table = torch.randn(1000, 256, device=cuda, dtype=torch.bfloat16)
