@@ -346,8 +346,10 @@ constexpr double kFragShare = 2.0;
 // A product is taken where the model says 5 % less in fragment order and 3 % less row-major (up to 128 rows 20 %: 128 x 1024 x 1024
 // with bias, row-major, takes the skinny kernel 11.8 us and this one 12.7, where the model says 10.6). (The 256 x 256 kernels at K >= 8192
 // are up to a fifth faster than their model where the tiles divide the chip evenly.)
+// At K >= 8192 the row-major form need only come within 5 %: N 4096, K 14336 with a residual, 400 - 512 rows, takes 61 - 74 us in
+// fragment order here and 79 - 81 on the 256 x 256 kernel, which row-major weights pay for with 88 - 102 instead of 78 - 80.
 double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.2 : 1.05; }
-double margin_row_major(int M) { return M <= 128 ? 1.2 : 1.03; }
+double margin_row_major(int M, int K) { return M <= 128 ? 1.2 : M >= 256 && K >= 8192 ? 0.955 : 1.03; }
 
 // the ordered form, fitted to 600 timings of 150 products of up to 3072 rows (17 of 20 within 15 %)
 double ordered_cost(int M, int N, int K, int mt, int bfrag) {
@@ -416,7 +418,7 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
       }
     }
     const double other = other_cost(M, N, K, epi);
-    if (force == 0 && (frag * margin(M, K) >= other || row * margin_row_major(M) >= other)) return false;
+    if (force == 0 && (frag * margin(M, K) >= other || row * margin_row_major(M, K) >= other)) return false;
   }
   if (best.parts > 1 && !parts_fit(M, N, best.mt, best.ng, best.parts)) best.parts = 1;
   if (best.parts > 1) {
