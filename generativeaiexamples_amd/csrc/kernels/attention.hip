@@ -112,7 +112,7 @@ __device__ __forceinline__ bf16x8 kv_to_bf16(uint2 v, float s) { return fp8x8_to
 // NWV = waves per workgroup: 4 (two workgroups per CU) or 8 (one; the row groups of two 4-wave workgroups share each
 // staged K / V^T tile, halving the tile loads and LDS writes per FLOP; head_dim 64 / 128, one head per wave)
 // ROWS: keys and values straight from the packed rows that q is in (self-attention of an encoder; kc / vc = the first row's key /
-// value of head 0, q_ld apart), instead of from pages that a kernel before has packed: 61 passages of e5-large 25 + 66 -> 68 us a
+// value of head 0, q_ld apart), instead of from pages that a kernel before has packed: 61 passages of e5-large 25 + 66 -> 62 us a
 // layer, a question 4.2 + 5.4 -> 5.3. V is turned on its way into LDS: a thread fetches two dims of eight keys, 4 B each
 // (whole lines across the wave), and writes two rows of the V^T image. head_dim 64, a kv head per q head.
 template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4, bool ROWS = false>

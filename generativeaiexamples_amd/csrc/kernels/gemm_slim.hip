@@ -307,7 +307,8 @@ void gai_gemm_slim(const void* A, const void* W, void* C, const void* bias, cons
 }
 
 // Slices of K for a product whose rows a layer norm takes next (which sums the slabs): the most, up to 8, whose workgroups
-// fit the chip at once. One workgroup a 16 columns leaves most of it idle: N 1024, K 4096 has 64, each with 350 KB to fetch.
+// fit the chip at once. One workgroup a 16 columns leaves most of it idle: N 1024, K 4096 has 64, each with 350 KB to fetch
+// (27 rows: 10.0 us and 3.9 of norm; in four slices 5.5 and 3.6; K 1024 4.1 + 3.9 and in two slices 4.0 + 3.6).
 int gai_gemm_slim_ks(int M, int N, int K) {
   if (M < 1 || M > 64 || N < 16 || N % 16 || N > 2048 || K < 2 * kPairK || K % kPairK || (long long)N * K > (8 << 20)) return 0;
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;

@@ -5,10 +5,11 @@ the HF sentence-transformers embedder (S11, ``utils.py:406-444``) and the Triton
 (S8), plus BERT-style cross-encoder rerankers (S3 analogue).
 
 Forward over a varlen batch (no padding): word+position+type embedding -> LayerNorm, then per
-layer: QKV GEMM(+bias) -> K/V scattered into a transient paged cache by the RoPE/KV kernel with
-rotation disabled -> bidirectional paged flash attention -> O GEMM with bias+residual fused ->
+layer: QKV GEMM(+bias) -> bidirectional flash attention straight from the packed QKV rows (or, where
+the rows do not fit that kernel, from transient pages) -> O GEMM with bias+residual fused ->
 LayerNorm (post-LN) -> FFN-up GEMM with bias+GELU fused -> FFN-down GEMM with bias+residual fused
--> LayerNorm. Pooling (mean / CLS) + L2-normalise in one kernel.
+-> LayerNorm; up to 64 tokens the O and down GEMMs leave K slices that the LayerNorm sums. Pooling
+(mean / CLS) + L2-normalise in one kernel.
 """
 from __future__ import annotations
 

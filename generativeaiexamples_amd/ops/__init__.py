@@ -160,7 +160,8 @@ def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
         K, N = x.shape[-1], w.shape[0]
         M = x.numel() // K
         ks = native().gemm_slim_ks(M, N, K) if M <= 64 else 0
-        if ks and residual.is_contiguous():
+        # 16-byte loads of rows and vectors that the two separate ops read singly
+        if ks and residual.is_contiguous() and not any(t.data_ptr() & 15 for t in (x, residual, bias, ln_w, ln_b) if t is not None):
             psw = decode_operand(w)
             out = torch.empty_like(residual)
             ws = torch.empty(ks, M, N, dtype=torch.float32, device=x.device)

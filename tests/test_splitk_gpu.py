@@ -324,3 +324,6 @@ def test_product_in_slices_and_norm(cuda, M, N, K, ks, frag):
     v = x.double() @ wn.double().t() + bias.double() + r.double()
     want = torch.nn.functional.layer_norm(v, (N,), g.double(), b.double(), 1e-5)
     assert ((y.double() - want).abs() <= 2.0 ** -8 * (want.abs() + 8 * g.double().abs())).all()
+    odd = torch.empty(M * N + 1, device=cuda, dtype=torch.bfloat16)[1:].view(M, N).copy_(r)  # not on 16 bytes: the two ops
+    z = ops.layer_norm(ops.linear(x, w, bias=bias, residual=odd), g, b, 1e-5)
+    assert torch.equal(ops.linear_layer_norm(x, w, bias, odd, g, b, 1e-5), z)
