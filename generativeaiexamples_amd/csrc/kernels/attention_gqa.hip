@@ -311,6 +311,13 @@ __global__ __launch_bounds__(64) void gqa_merge_kernel(GqaArgs a) {
     m = p0[lane * step + DV];
     l = p0[lane * step + DV + 1];
   }
+  // the first shares' values are on their way while the weights are worked out (past the last: the last again, not used):
+  // 384 rows of up to 10 shares 5.4 -> 4.8 us
+  constexpr int kAhead = 16;
+  const int c0v = min(4 * lane, DV - 4);
+  f32x4 x[kAhead];
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j) x[j] = *reinterpret_cast<const f32x4*>(p0 + max(min(j, used - 1), 0) * step + c0v);
   const float sk = a.sink ? a.sink[head] * kL2e : kOut;
   const float M = fmaxf(wave_max(m), sk);
   const float w = l > 0.f ? __builtin_amdgcn_exp2f(m - M) : 0.f;
@@ -320,8 +327,15 @@ __global__ __launch_bounds__(64) void gqa_merge_kernel(GqaArgs a) {
   bf16* o = a.out + (size_t)t * a.ldo + (size_t)head * DV;
   for (int c = 4 * lane; c < DV; c += 256) {
     f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
+    int j0 = 0;
+    if (c == c0v) {
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+        if (j < used) y += wgt[j] * x[j];
+      j0 = kAhead;
+    }
 #pragma unroll 8
-    for (int j = 0; j < used; ++j) y += wgt[j] * *reinterpret_cast<const f32x4*>(p0 + j * step + c);
+    for (int j = j0; j < used; ++j) y += wgt[j] * *reinterpret_cast<const f32x4*>(p0 + j * step + c);
     *reinterpret_cast<bf16x4*>(o + c) = bf16x4{(bf16)y[0], (bf16)y[1], (bf16)y[2], (bf16)y[3]};
   }
 }

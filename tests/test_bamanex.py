@@ -192,6 +192,23 @@ def test_parallel_add_norm_against_equations(device):
                             assert torch.allclose(got.cpu().double(), ref, atol=tol, rtol=tol), (T, D, dt, use, norms)
 
 
+@_GPU
+@pytest.mark.parametrize("D", [2044, 2048, 2052, 4096, 4100, 511, 513, 1025])
+def test_parallel_add_norm_kept_groups(D):
+    """Rows that fill the kept groups of each form, and one group more or fewer: against float64 (bf16 results, eight
+    significant bits: 2^-8; and the
+    fp32 sum of up to 4100 squares)."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    res, a, b, w1, w2 = rn(5, D), rn(5, D).bfloat16(), rn(5, D).bfloat16(), rn(D), rn(D)
+    want = res.double() + a.double() + b.double()
+    h1, h2 = ops.parallel_add_norm_f32(res, a=a, b=b, w1=w1, w2=w2, eps=1e-5, out_dtype=torch.bfloat16)
+    assert torch.allclose(res.double(), want, atol=1e-6, rtol=1e-6)
+    for h, w in ((h1, w1), (h2, w2)):
+        ref = O.unit_rms(want, 1e-5) * w.double()
+        assert ((h.double() - ref).abs() <= (2.0 ** -8 + 2e-6) * ref.abs()).all()
+
+
 @pytest.mark.parametrize("device,dtype", TARGETS)
 def test_rotation_unit_norm_and_cache_write(device, dtype):
     """Rotated halves at positions up to 10^5 with and without the unit norm, tokens in scattered slots and tokens that fill
