@@ -443,7 +443,7 @@ constexpr int kSelectRows = 16 * 4096;
 
 __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__ Q, const bf16* __restrict__ X,
                                                         const float* __restrict__ bias, const float* __restrict__ gmax,
-                                                        int ngr, int N, int D, int k, float* __restrict__ out_v,
+                                                        int ngr, int N, int D, int k, int dma, float* __restrict__ out_v,
                                                         int64_t* __restrict__ out_i) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // 4 KB a wave of rows, the first 8 KB also keys; the query
   u64* buf = reinterpret_cast<u64*>(smem);
@@ -451,7 +451,8 @@ __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__
   __shared__ u64 cand[1024], list[64];
   __shared__ int pick[64], cnt;
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  for (int e = tid; e < D / 8; e += 1024) store8(qrow + 8 * e, load8(Q + (size_t)q * D + 8 * e));
+  if (dma)
+    for (int e = tid; e < D / 8; e += 1024) store8(qrow + 8 * e, load8(Q + (size_t)q * D + 8 * e));
   const float* gm = gmax + (size_t)q * ngr;
   if (ngr > k) {  // else every group is taken, and gmax was not written
     u64 m = 0;
@@ -497,7 +498,7 @@ __global__ __launch_bounds__(1024) void sim_topk_select(const bf16* __restrict__
     const float v = r == 0 ? acc[0] : r == 1 ? acc[1] : r == 2 ? acc[2] : acc[3];
     if (r < 4 && row < N) cand[16 * j + 4 * (lane >> 4) + r] = make_key(v + bias[row], row);
   };
-  if (D % 64) {
+  if (!dma) {  // columns no multiple of 64, or rows off 16 bytes
     const bf16* qp = Q + (size_t)q * D + 8 * (lane >> 4);
     for (int j = wid; j < k && pick[j] >= 0; j += 16) {  // (the picked groups come first)
       const bf16* xa = X + (size_t)min(16 * pick[j] + (lane & 15), N - 1) * D + 8 * (lane >> 4);
@@ -657,21 +658,22 @@ void run_group_max(const TopkArgs& a, int qblocks) {
   GAI_LAUNCH_CHECK();
 }
 
+bool on16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 void run_select(const TopkArgs& a) {
   static bool once = false;
   if (!once) {
     set_max_lds(sim_topk_select, 150 * 1024);  // (its own 9 KB are beside)
     once = true;
   }
-  sim_topk_select<<<a.nq, 1024, kSelectRows + a.D * 2, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, (a.N + 15) / 16, a.N, a.D, a.k,
-                                           a.out_v, a.out_i);
+  const int dma = a.D % 64 == 0 && on16(a.X);  // 16-byte loads into LDS
+  sim_topk_select<<<a.nq, 1024, kSelectRows + a.D * 2, a.st>>>((const bf16*)a.Q, (const bf16*)a.X, a.bias, a.ws_v, (a.N + 15) / 16,
+                                                               a.N, a.D, a.k, dma, a.out_v, a.out_i);
   GAI_LAUNCH_CHECK();
 }
 
 bool many_queries(const TopkArgs& a) {
-  if (a.nq <= 64 || a.D % 64 || a.D < 256 || (a.N + 15) / 16 <= a.k) return false;
-  auto off = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
-  if (off(a.Q) || off(a.X)) return false;
+  if (a.nq <= 64 || a.D % 64 || a.D < 256 || (a.N + 15) / 16 <= a.k || !on16(a.Q) || !on16(a.X)) return false;
   const int qblocks = (a.nq + 319) / 320, qt = ((a.nq + qblocks - 1) / qblocks + 63) / 64 * 4;
   if (qt <= 8) run_group_max<8>(a, qblocks);
   else if (qt <= 12) run_group_max<12>(a, qblocks);

@@ -604,6 +604,23 @@ def test_sim_topk_many_queries(cuda, nq, N, D, k):
     assert torch.equal(v.isfinite(), fin)
 
 
+@pytest.mark.parametrize("nq,D,k", [(3, 64, 10), (70, 256, 10), (70, 256, 4), (2, 1024, 40)])
+@pytest.mark.parametrize("off", [2, 4])
+def test_sim_topk_rows_off_16_bytes(cuda, nq, D, k, off):
+    """Rows (and queries) that begin off a 16-byte line give the bits of the same rows on one: no 16-byte copies to LDS there."""
+    torch.manual_seed(nq)
+    N = 3000
+    base = torch.randn(N * D + off, device=cuda).bfloat16()
+    bq = torch.randn(nq * D + off, device=cuda).bfloat16()
+    X, Q = base[off:].view(N, D), bq[off:].view(nq, D)
+    assert X.data_ptr() % 16 and Q.data_ptr() % 16
+    bias = -0.5 * X.float().square().sum(-1)
+    want = ops.sim_topk(Q.clone(), X.clone(), bias, N, k)
+    for q, x in ((Q, X), (Q.clone(), X), (Q, X.clone())):
+        v, i = ops.sim_topk(q, x, bias, N, k)
+        assert torch.equal(v, want[0]) and torch.equal(i, want[1])
+
+
 def test_sim_topk_no_candidates(cuda):
     """k = 0 asks for nothing and gets empty lists, from the kernel's entry point and from the index."""
     from generativeaiexamples_amd.index.hbm_index import HBMIndex
