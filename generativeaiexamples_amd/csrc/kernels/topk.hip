@@ -658,6 +658,9 @@ void run_group_max(const TopkArgs& a, int qblocks) {
   GAI_LAUNCH_CHECK();
 }
 
+// an image of the queries of a tile fits LDS beside the bias rows
+bool tile_fits(const TopkArgs& a, int nq_tile) { return (size_t)nq_tile * a.D * 2 + (size_t)a.rows_per_wg * 4 <= 160 * 1024; }
+
 bool on16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 void run_select(const TopkArgs& a) {
@@ -720,12 +723,10 @@ void run_stream(const TopkArgs& a) {
 
 template <int K>
 void run_topk_k(const TopkArgs& a) {
-  // the largest query tile whose image fits LDS beside the bias rows
-  auto fits = [&](int nq_tile) { return (size_t)nq_tile * a.D * 2 + (size_t)a.rows_per_wg * 4 <= 160 * 1024; };
-  if (a.nq > 32 && fits(64)) return run_stream<4, K>(a);
-  if (a.nq > 16 && fits(32)) return run_stream<2, K>(a);
-  if (fits(16)) return run_stream<1, K>(a);
-  gai_launch_error(__FILE__, __LINE__, "sim_topk: dimension too large for the LDS query tile");
+  // the largest query tile that fits; 16 queries do (gai_sim_topk)
+  if (a.nq > 32 && tile_fits(a, 64)) return run_stream<4, K>(a);
+  if (a.nq > 16 && tile_fits(a, 32)) return run_stream<2, K>(a);
+  run_stream<1, K>(a);
 }
 
 }  // namespace
@@ -752,6 +753,8 @@ void gai_sim_topk(const void* Q, const void* X, const float* bias, int nq, int N
   if (nq == 0) return;
   if (D % 32) gai_launch_error(__FILE__, __LINE__, "sim_topk: D must be a multiple of 32");
   const TopkArgs a{Q, X, bias, nq, N, D, k, nwg, rows_per_wg, ws_v, ws_i, out_v, out_i, st};
+  // (the tiled product holds no such image, but what it takes must not depend on the number of queries)
+  if (!tile_fits(a, 16)) gai_launch_error(__FILE__, __LINE__, "sim_topk: dimension too large for the LDS query tile");
   if (!ws_i) {  // ws_v: the group maxima [nq][ceil(N / 16)]
     if (!many_queries(a)) run_topk_k<0>(a);
     return;

@@ -621,6 +621,14 @@ def test_sim_topk_rows_off_16_bytes(cuda, nq, D, k, off):
         assert torch.equal(v, want[0]) and torch.equal(i, want[1])
 
 
+@pytest.mark.parametrize("nq,k", [(1, 4), (64, 40), (65, 4), (65, 40)])
+def test_sim_topk_refuses_wide_rows(cuda, nq, k):
+    """Rows too wide for an LDS image of sixteen queries are an error whatever the number of queries."""
+    X = torch.zeros(20000, 5120 + 64, device=cuda, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="dimension too large"):
+        ops.sim_topk(X[:nq].contiguous(), X, torch.zeros(20000, device=cuda), 20000, k)
+
+
 def test_sim_topk_no_candidates(cuda):
     """k = 0 asks for nothing and gets empty lists, from the kernel's entry point and from the index."""
     from generativeaiexamples_amd.index.hbm_index import HBMIndex
