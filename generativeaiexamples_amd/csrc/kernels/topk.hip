@@ -1,20 +1,21 @@
-// Exact brute-force vector search: fused similarity GEMM + top-k (SURVEY K13, K14).
+// Exact brute-force vector search: fused similarity GEMM + top-k.
 //
 // scores[q, x] = Q[q] . X[x] + bias[x]  with bias = 0 (inner product / cosine on
 // normalised vectors), -0.5*|x|^2 (L2 ranking) or -inf (deleted row), so one
 // kernel serves IP / cosine / L2 and tombstones. The [nq, N] score matrix is
 // never materialised. Both paths stream X once per 64-query tile through
 // v_mfma_f32_16x16x32_bf16 (sim_topk_stream):
-//   short lists (k <= 4, or k <= 8 for one query tile): every lane keeps a sorted list of its best rows in registers;
-//   the lists of a workgroup are merged in LDS and the workgroups' lists by sim_topk_stage2;
+//   short lists (k <= 8 for one query tile; k <= 4 for more where the form below is slower or does not run): every lane
+//   keeps a sorted list of its best rows in registers; the lists of a workgroup are merged in LDS and the workgroups'
+//   lists by sim_topk_stage2;
 //   else only the largest score of every 16-row group is kept (sim_topk_stream<.., 0, ..>), and one workgroup per
 //   query picks the k best groups - which hold the k best rows - and scores their rows again (sim_topk_select).
-// More than 64 queries (columns a multiple of 64, at least 256) take the groups from a tiled product instead (sim_group_max).
+// More than 64 queries in one call (columns a multiple of 64, at least 256) take the groups from a tiled product instead
+// (sim_group_max). The caller's slices hold that many up to 8.4M rows.
 // us, lists / groups (first form of k > 8: a 64-entry list per lane): 1M x 1024, k = 4, 1 query 353 / 417; k = 8, 64 queries 422 /
-// 510; k = 40, 1 query (18263) / 454. Lists / groups of the stream / of the tiled product, 300 queries: 250k x 1024, k = 4 414 / - /
+// 510; k = 40, 1 query (18263) / 430. Lists / groups of the stream / of the tiled product, 300 queries: 250k x 1024, k = 4 414 / - /
 // 238, k = 8 - / 393 / 242, k = 40 (144700) / 470 / 298; 1M x 1024, k = 8 1375 / 1277 / 800; 100k x 384, k = 8 - / 94 / 77; 65
-// queries, 250k x 1024, k = 4 193 / 191 / 143. On small indexes the second pass costs more than the lists: 300 queries, 5000 x 1024,
-// k = 4 38 / 57 / 48; 30000 146 / 114 / 62.
+// queries, 250k x 1024, k = 4 193 / 191 / 143. (Where lists stay for k <= 4: ops.sim_topk.)
 #include <algorithm>
 
 #include "gai_common.h"

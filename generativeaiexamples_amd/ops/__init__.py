@@ -796,6 +796,30 @@ def topk_cap(k: int) -> int:
     return 4 if k <= 4 else 8 if k <= 8 else 16 if k <= 16 else 32 if k <= 32 else 64
 
 
+def _topk_slice(nq: int, n_rows: int) -> int:
+    """Queries whose group maxima are held at a time: 256 MB of maxima up to 16.8 M rows, past that those of one 64-query tile
+    (16 bytes a row: 1.6 GB at 100 M rows, beside 205 GB of index at 1024 columns)."""
+    return min(nq, max(64, _TOPK_MAXIMA // ((n_rows + 15) // 16) // 64 * 64))
+
+
+def _topk_lists(cap: int, nq: int, n_rows: int, D: int, aligned: bool = True) -> bool:
+    """Whether the best rows are kept as lists in registers (k <= 8) instead of group maxima and a second pass. One tile of
+    queries always; more of them only for k <= 4, where the tiled product of the maxima (topk.hip sim_group_max) does not run
+    or measured slower, us lists / maxima at k = 4:
+      * more queries than one slice of maxima holds (each slice reads the index again): 6M x 256, 130 queries 1227 / 1824, 300
+        1917 / 3066; above 8.4M rows a slice is one tile and the product never runs: 9M x 1024, 65 queries 5103 / 7620;
+      * up to 128 queries on half a million rows and more of a width that the stream likes: 1M x 384, 65 queries 1.06 times
+        the lists' time, 128 1.14; 4M x 256, 128 1.21; 1M x 768 1.01 - 1.04 (1M x 1024 0.86 - 0.96, 250k x 384 0.76 - 0.81);
+      * a small index, where more than 256 queries wait for the second pass: 300 queries, 2000 x 1024, 1.18; 5000 rows 1.21
+        (up to 256 queries 0.6 - 0.8 there, and from 10000 rows on 0.5 - 0.8)."""
+    if cap > 8 or nq <= 64:
+        return cap <= 8
+    if cap == 8:
+        return False
+    return (D < 256 or D % 64 != 0 or not aligned or n_rows < 16384 or nq > _topk_slice(nq, n_rows)
+            or (nq <= 128 and n_rows >= 1 << 19 and D < 1024 and D % 128 == 0))
+
+
 def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, k: int, ws=None):
     """Top-k of Q @ X[:n_rows]^T + bias (exact). Returns (scores fp32 [nq,k], ids int64 [nq,k])."""
     if k > 64:
@@ -813,17 +837,20 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
     out_v = torch.empty(nq, k_eff, dtype=torch.float32, device=Q.device)
     out_i = torch.empty(nq, k_eff, dtype=torch.int64, device=Q.device)
     Q, cap = Q.contiguous(), topk_cap(k_eff)
-    # short lists in registers (topk.hip has both forms' times); more than one tile of queries takes them on small indexes only
-    if cap <= 8 and (nq <= 64 or (cap == 4 and (n_rows < 16384 or D < 256 or D % 64))):
+    lists = _topk_lists(cap, nq, n_rows, D, not (Q.data_ptr() | X.data_ptr()) & 15)
+    step = _topk_slice(nq, n_rows)
+    if not lists:
+        try:
+            ws_v = torch.empty(max(1, step * ((n_rows + 15) // 16)), dtype=torch.float32, device=Q.device)
+        except torch.OutOfMemoryError:
+            if cap > 4:
+                raise
+            lists = True  # (a few MB)
+    if lists:
         ws_v = torch.empty(nwg * nq * cap, dtype=torch.float32, device=Q.device)
         ws_i = torch.empty(nwg * nq * cap, dtype=torch.int32, device=Q.device)
         native().sim_topk(Q, X, bias, n_rows, k_eff, ws_v, ws_i, nwg, rows_per_wg, out_v, out_i)
         return out_v, out_i
-    # the largest score of every 16 rows and query, in slices of queries: 256 MB of maxima at a time up to 16.8 M rows, past
-    # that those of one 64-query tile (16 bytes a row: 1.6 GB at 100 M rows, beside 205 GB of index at 1024 columns)
-    groups = (n_rows + 15) // 16
-    step = min(nq, max(64, _TOPK_MAXIMA // groups // 64 * 64))
-    ws_v = torch.empty(max(1, step * groups), dtype=torch.float32, device=Q.device)
     for s in range(0, nq, max(1, step)):
         e = min(nq, s + step)
         native().sim_topk(Q[s:e], X, bias, n_rows, k_eff, ws_v, None, nwg, rows_per_wg, out_v[s:e], out_i[s:e])

@@ -621,6 +621,54 @@ def test_sim_topk_rows_off_16_bytes(cuda, nq, D, k, off):
         assert torch.equal(v, want[0]) and torch.equal(i, want[1])
 
 
+@pytest.mark.parametrize("nq,N,D,k,room,lists", [
+    (65, 16384, 256, 4, 1 << 20, False), (300, 20000, 256, 4, 1250 * 320, False),
+    (300, 20000, 256, 4, 1250 * 256, True),     # two slices would read the index twice
+    (65, 20000, 256, 3, 1250 * 64, True),       # slices of one tile: the tiled product would not run
+    (300, 16383, 256, 4, 1 << 20, True), (65, 20000, 192, 4, 1 << 20, True), (65, 20000, 256, 8, 1000, False)])
+def test_sim_topk_form(cuda, monkeypatch, nq, N, D, k, room, lists):
+    """Short lists of more queries than a tile: which form answers, with maxima for one slice and for less, and the answer."""
+    torch.manual_seed(nq)
+    monkeypatch.setattr(ops, "_TOPK_MAXIMA", room)
+    X, Q = torch.randn(N, D, device=cuda).bfloat16(), torch.randn(nq, D, device=cuda).bfloat16()
+    nat, forms = ops.native(), []
+
+    class Spy:
+        def sim_topk(self, *a):
+            forms.append(a[6] is not None)
+            return nat.sim_topk(*a)
+
+    monkeypatch.setattr(ops, "native", Spy)
+    v, i = ops.sim_topk(Q, X, torch.zeros(N, device=cuda), N, k)
+    assert set(forms) == {lists}
+    s = Q.double() @ X.double().t()
+    # bf16 operands, fp32 sums of D products: D * 2^-24 of |q| |x| <= 2 D covers any order
+    tol = 2 * D * D * 2.0 ** -24
+    assert (v.double() - s.topk(k, dim=1).values).abs().max() <= tol
+    assert (torch.gather(s, 1, i) - v.double()).abs().max() <= tol
+    assert all(len(set(r)) == k for r in i.tolist())
+
+
+def test_sim_topk_without_room_for_maxima(cuda, monkeypatch):
+    """A card without memory for the group maxima answers k <= 4 from lists."""
+    torch.manual_seed(5)
+    X, Q = torch.randn(20000, 256, device=cuda).bfloat16(), torch.randn(70, 256, device=cuda).bfloat16()
+    bias = torch.zeros(20000, device=cuda)
+    want = ops.sim_topk(Q, X, bias, 20000, 4)
+    empty = torch.empty
+
+    def small(*a, **k):
+        if a[0] == 70 * 1250:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*a, **k)
+
+    monkeypatch.setattr(torch, "empty", small)
+    v, i = ops.sim_topk(Q, X, bias, 20000, 4)
+    assert torch.equal(v, want[0]) and torch.equal(i, want[1])
+    with pytest.raises(torch.OutOfMemoryError):
+        ops.sim_topk(Q, X, bias, 20000, 9)
+
+
 @pytest.mark.parametrize("nq,k", [(1, 4), (64, 40), (65, 4), (65, 40)])
 def test_sim_topk_refuses_wide_rows(cuda, nq, k):
     """Rows too wide for an LDS image of sixteen queries are an error whatever the number of queries."""
