@@ -965,12 +965,18 @@ def moe_router(x: torch.Tensor, W: torch.Tensor, E: int, k: int, eps: float = 0.
 _MOE_DISPATCH_MAX = int(os.environ.get("GAI_MOE_DISPATCH_MAX", "32768"))
 
 
+def _dispatch_native(ids, buckets: int) -> bool:
+    """The counting sort takes the plan. Past 2048 buckets, which it does not hold, more rows than a decode step's are sorted."""
+    n = ids.numel()
+    return ids.is_cuda and 0 < n <= _MOE_DISPATCH_MAX and (n <= 8192 or buckets <= 2048)
+
+
 def moe_dispatch(ids: torch.Tensor, num_experts: int):
     """Expert-sorted dispatch plan without host sync: (a_rows [T*k], offsets [E+1], pos [T,k]).
-    Up to _MOE_DISPATCH_MAX rows one single-workgroup counting-sort kernel builds it; larger steps keep the stable
-    argsort."""
+    Up to _MOE_DISPATCH_MAX rows one single-workgroup counting-sort kernel builds it (_dispatch_native); larger steps keep
+    the stable argsort."""
     T, k = ids.shape
-    if ids.is_cuda and 0 < T * k <= _MOE_DISPATCH_MAX:
+    if _dispatch_native(ids, num_experts):
         dev = ids.device
         a_rows = torch.empty(T * k, dtype=torch.int32, device=dev)
         offs = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
@@ -1032,7 +1038,7 @@ def ep_dispatch_plan(ids: torch.Tensor, world: int, e_local: int):
     """Expert-parallel send plan of the (token, choice) pairs: (offs [W+1], pos [T, k], a_pairs [T*k]) = the pairs
     counting-sorted by destination rank id // e_local (moe_dispatch's kernel with a bucket divisor), sync-free."""
     T, k = ids.shape
-    if ids.is_cuda and 0 < T * k <= _MOE_DISPATCH_MAX:
+    if _dispatch_native(ids, world):
         dev = ids.device
         a_rows = torch.empty(T * k, dtype=torch.int32, device=dev)
         a_pairs = torch.empty(T * k, dtype=torch.int32, device=dev)

@@ -194,6 +194,18 @@ def test_moe_dispatch_edges(cuda, T, k, E, div):
     assert torch.equal(offs.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.int64), torch.bincount(flat, minlength=E).cumsum(0)]))
 
 
+@pytest.mark.parametrize("T,E", [(4097, 2048), (4097, 2049), (16384, 5000)])
+def test_moe_dispatch_many_experts(cuda, T, E):
+    """More experts than the counting sort holds: long steps are still answered, and a decode step is still refused."""
+    ids = torch.randint(0, E, (T, 2), generator=torch.Generator().manual_seed(E), dtype=torch.int32)
+    rows, offs, pos = ops.moe_dispatch(ids.to(cuda), E)
+    want = ops.moe_dispatch(ids, E)
+    assert all(torch.equal(a.cpu(), b) for a, b in zip((rows, offs, pos), want))
+    if E > 2048:
+        with pytest.raises(RuntimeError, match="experts"):
+            ops.moe_dispatch(ids[:4096].to(cuda), E)
+
+
 @pytest.mark.parametrize("T,k,E,W", [(1, 2, 8, 2), (8, 2, 8, 2), (64, 2, 8, 4), (37, 2, 8, 8), (64, 2, 64, 4)])
 def test_ep_pack_and_combine_match_reference(cuda, T, k, E, W):
     """Native expert-parallel slab pack (counting-sorted by destination rank, expert ids in the row tails or a
