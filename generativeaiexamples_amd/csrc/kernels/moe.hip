@@ -529,6 +529,11 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16* __restrict
 // and a pass per distinct expert before); 16384 rows of 64 experts 61 -> 19 us with a ballot per bit.
 // div > 1 buckets id / div instead of id (expert parallelism: the destination rank of a global expert id);
 // a_pairs (optional) receives the flat pair index i of every sorted row next to its token i / k.
+// The short form, with a row a lane, counts and ranks in one pass and needs one barrier; as two passes and a scan over the workgroup
+// the plan of a decode step took 3.7 - 4.0 us instead of 2.5 - 2.9 (2 to 256 rows of 8 experts; 64 experts 3.9 - 4.1 and 2.6 - 2.9,
+// 128 experts 4.1 and 3.0 - 3.5). Every wave scans all experts: at 256 of them 4.0 - 5.7 and 4.4 - 6.2 us, past where it pays.
+constexpr int kRowALane = 192;  // most experts of the short form
+
 __global__ __launch_bounds__(1024) void moe_dispatch_kernel(const int* __restrict__ ids, int n, int k, int E,
                                                             int* __restrict__ a_rows, int* __restrict__ offs,
                                                             int* __restrict__ pos, int div, int* __restrict__ a_pairs) {
@@ -541,9 +546,56 @@ __global__ __launch_bounds__(1024) void moe_dispatch_kernel(const int* __restric
     const int id = ids[i];
     return min(max(div > 1 ? id / div : id, 0), E - 1);
   };
-  for (int x = lane; x < E; x += 64) mine[x] = 0;
   const int bits = 32 - __clz(E - 1);  // 0 for one expert
-  constexpr int U = 8;                 // loads in flight
+  auto alike = [&](int e) {  // the live lanes of this lane's expert, one ballot per bit of the id
+    unsigned long long same = __ballot(e >= 0);
+    for (int bit = 0; bit < bits; ++bit) {
+      const bool set = (e >> bit) & 1;
+      const unsigned long long m = __ballot(set);
+      same &= set ? m : ~m;
+    }
+    return same;
+  };
+  if (per == 64 && E <= kRowALane) {  // a row a lane: decode steps, one pass and one barrier
+    const int i = i0 + lane, e = i < i1 ? expert(i) : -1;
+    for (int x = lane; x < E; x += 64) mine[x] = 0;
+    const unsigned long long same = alike(e);
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own LDS row: zeros first
+    __builtin_amdgcn_wave_barrier();
+    if (e >= 0 && rank == 0) mine[e] = __popcll(same);
+    __syncthreads();
+    int r = 0, base = 0;
+    for (int x0 = 0; x0 < E; x0 += 64) {  // an expert a lane: every wave scans for itself
+      const int x = x0 + lane;
+      int tot = 0, at = base;
+      if (x < E)
+        for (int w = 0; w < nw; ++w) {
+          const int c = dsm[w * E + x];
+          at += w < wid ? c : 0;
+          tot += c;
+        }
+      int run = tot;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(run, o, 64);
+        if (lane >= o) run += up;
+      }
+      if (wid == 0 && x < E) offs[x] = base + run - tot;
+      const int to = __shfl(at + run - tot, e & 63, 64);
+      if (e >> 6 == x0 >> 6) r = to + rank;
+      base += __shfl(run, 63, 64);
+    }
+    if (tid == 0) offs[E] = base;
+    if (e >= 0) {
+      a_rows[r] = i / k;
+      if (a_pairs != nullptr) a_pairs[r] = i;
+      pos[i] = r;
+    }
+    return;
+  }
+  for (int x = lane; x < E; x += 64) mine[x] = 0;
+  constexpr int U = 8;  // loads in flight
   for (int b = i0; b < i1; b += 64 * U) {
     int e[U];
 #pragma unroll
@@ -591,13 +643,8 @@ __global__ __launch_bounds__(1024) void moe_dispatch_kernel(const int* __restric
     for (int u = 0; u < U; ++u) e[u] = b + 64 * u + lane < i1 ? expert(b + 64 * u + lane) : -1;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      unsigned long long same = __ballot(e[u] >= 0);  // the live lanes of this lane's expert, one ballot per bit of the id
-      if (same == 0) break;
-      for (int bit = 0; bit < bits; ++bit) {
-        const bool set = (e[u] >> bit) & 1;
-        const unsigned long long m = __ballot(set);
-        same &= set ? m : ~m;
-      }
+      if (__ballot(e[u] >= 0) == 0) break;
+      const unsigned long long same = alike(e[u]);
       const int rank = __popcll(same & ((1ull << lane) - 1ull)), count = __popcll(same);
       // the wave's own LDS row: reads before the last lane of each expert moves its cursor, both before the next 64 rows
       const int at = e[u] >= 0 ? mine[e[u]] : 0;
@@ -703,8 +750,8 @@ void gai_moe_dispatch(const int* ids, int n, int k, int E, int* a_rows, int* off
                       int div, int* a_pairs) {
   if (E < 1 || E > 2048) gai_launch_error(__FILE__, __LINE__, "moe_dispatch: 1 <= experts <= 2048");
   if (div < 1) gai_launch_error(__FILE__, __LINE__, "moe_dispatch: bucket divisor >= 1");
-  // sixteen waves where each has rows and their counts fit 32 KB of LDS
-  const int nw = n > 256 && E <= 512 ? 16 : 4;
+  // sixteen waves where each has rows and their counts fit 32 KB of LDS; one where it holds every row
+  const int nw = n > 256 && E <= 512 ? 16 : n <= 64 && E <= kRowALane ? 1 : 4;
   moe_dispatch_kernel<<<1, 64 * nw, (nw * E + nw) * sizeof(int), st>>>(ids, n, k, E, a_rows, offs, pos, div, a_pairs);
   GAI_LAUNCH_CHECK();
 }

@@ -178,9 +178,11 @@ def test_moe_dispatch_kernel_matches_stable_argsort(cuda, T, k, E):
 
 
 @pytest.mark.parametrize("T,k,E,div", [(257, 1, 1, 1), (128, 2, 512, 1), (129, 2, 513, 1), (512, 2, 512, 1), (4097, 2, 8, 1),
-                                       (1023, 8, 2048, 1), (16384, 2, 60, 1), (777, 3, 7, 9), (100, 2, 4, 16)])
+                                       (1023, 8, 2048, 1), (16384, 2, 60, 1), (777, 3, 7, 9), (100, 2, 4, 16),
+                                       (1, 1, 1, 1), (32, 2, 64, 1), (33, 2, 65, 1), (64, 4, 128, 3), (257, 1, 192, 1),
+                                       (512, 2, 192, 1), (64, 1, 192, 1), (64, 1, 193, 1), (1025, 1, 64, 1)])
 def test_moe_dispatch_edges(cuda, T, k, E, div):
-    """Waves with no rows, one row past a wave's run, one expert, the widest tables of either launch, buckets of ids: the plan
+    """A row a lane (one, four and sixteen waves) and the long form, waves with no rows, one row past a wave's run, one expert, the widest tables of either launch, buckets of ids: the plan
     of a stable sort."""
     g = torch.Generator().manual_seed(T + E)
     ids = torch.randint(0, E * div, (T, k), generator=g, dtype=torch.int32)
