@@ -6,6 +6,7 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -784,8 +785,8 @@ void pool(const Tensor& h, const Tensor& cu, Tensor& out, int64_t mode, bool nor
   check_bf16(h, "hidden");
   check_i32(cu, "cu_seqlens");
   check_f32(out, "out");
-  gai_pool(h.data_ptr(), cu.data_ptr<int>(), out.data_ptr<float>(), cu.numel() - 1, h.size(-1), mode,
-           normalize ? 1 : 0, cur_stream());
+  gai_pool(h.data_ptr(), cu.data_ptr<int>(), out.data_ptr<float>(), h.numel() / std::max<int64_t>(h.size(-1), 1),
+           cu.numel() - 1, h.size(-1), mode, normalize ? 1 : 0, cur_stream());
 }
 
 void silu_mul(const Tensor& x, Tensor& y) {

@@ -166,7 +166,7 @@ void gai_moe_scale_rows(const void* h, const int* pos, const float* w, void* out
 
 // misc.hip
 void gai_embedding(const int* ids, const void* table, void* out, int T, int D, int vstart, int vend, hipStream_t st);
-void gai_pool(const void* h, const int* cu, float* out, int B, int D, int mode, int normalize, hipStream_t st);
+void gai_pool(const void* h, const int* cu, float* out, int T, int B, int D, int mode, int normalize, hipStream_t st);
 void gai_silu_mul(const void* x, void* y, int T, int I, hipStream_t st);
 void gai_gelu(const void* x, void* y, int T, int I, hipStream_t st);
 void gai_gelu_tanh(const void* x, void* y, int T, int I, hipStream_t st);

@@ -689,7 +689,8 @@ def test_sim_topk_no_candidates(cuda):
 
 
 @pytest.mark.parametrize("D,lens", [(1024, [303, 1, 0, 65]), (384, [512, 7]), (64, [1000, 129, 128]), (8, [2000]), (8192, [3, 9]),
-                                    (8208, [2, 20])])
+                                    (8208, [2, 20]), (1024, [31, 1, 0, 20, 9]), (2048, [33, 2]), (64, [5, 2, 16]), (8, [3, 30]),
+                                    (4096, [1, 3, 17, 2] * 130)])  # the last five: 256 threads for means too
 @pytest.mark.parametrize("mode", ["mean", "cls", "last"])
 def test_pool_row_groups(cuda, D, lens, mode):
     """More and fewer rows than the groups and their loads hold, one group, widths beyond it; fp32 sums of up to 2000 rows in
