@@ -60,16 +60,92 @@ __global__ __launch_bounds__(256) void add_rmsnorm_f32_kernel(float* __restrict_
 }
 
 // One workgroup per row (as many threads as the row has groups of VEC channels, at most 256), the new sum kept in
-// registers between the passes (up to NQ groups per thread, at most 8; what is past them is re-read). Bound by latency: every load of the
-// kept groups, the norm weights too, is issued before the first is waited for (groups past the row read its last again),
-// 24 rows of 2048 6.6 -> 6.0 us (a round trip per group and another for the weights before).
-template <typename TA, int VEC, int NQ>
+// registers between the passes (up to kParRegs groups per thread; what is past them is re-read).
+constexpr int kParRegs = 8;
+
+template <typename TA, int VEC>
 __global__ __launch_bounds__(256) void parallel_add_norm_kernel(float* __restrict__ res, const TA* __restrict__ a, int lda,
                                                                 const float* __restrict__ sa, const TA* __restrict__ b,
                                                                 int ldb, const float* __restrict__ sb,
                                                                 const float* __restrict__ w1, TA* __restrict__ h1,
                                                                 const float* __restrict__ w2, TA* __restrict__ h2, int D,
                                                                 float eps) {
+  typedef TA vec __attribute__((ext_vector_type(VEC)));
+  typedef float fvec __attribute__((ext_vector_type(VEC)));
+  __shared__ float scratch[16];
+  const int row = blockIdx.x, tid = threadIdx.x, step = blockDim.x * VEC;
+  float* r = res + (size_t)row * D;
+  const TA* ar = a ? a + (size_t)row * lda : nullptr;
+  const TA* br = b ? b + (size_t)row * ldb : nullptr;
+  auto sum = [&](int i) {
+    fvec x = *reinterpret_cast<const fvec*>(r + i);
+    if (ar) {
+      const vec y = *reinterpret_cast<const vec*>(ar + i);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) x[e] = fmaf(sa ? sa[i + e] : 1.0f, (float)y[e], x[e]);
+    }
+    if (br) {
+      const vec y = *reinterpret_cast<const vec*>(br + i);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) x[e] = fmaf(sb ? sb[i + e] : 1.0f, (float)y[e], x[e]);
+    }
+    if (ar || br) *reinterpret_cast<fvec*>(r + i) = x;
+    return x;
+  };
+  fvec v[kParRegs];
+  float s = 0.f;
+#pragma unroll
+  for (int q = 0; q < kParRegs; ++q) {
+    const int i = tid * VEC + step * q;
+    if (i < D) {
+      v[q] = sum(i);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) s = fmaf(v[q][e], v[q][e], s);
+    }
+  }
+  for (int i = tid * VEC + step * kParRegs; i < D; i += step) {
+    const fvec x = sum(i);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) s = fmaf(x[e], x[e], s);
+  }
+  if (!h1 && !h2) return;
+  s = block_sum(s, scratch);
+  const float inv = 1.0f / sqrtf(s / D + eps);
+  auto put = [&](const fvec& x, int i, const float* w, TA* h) {
+    vec o;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o[e] = (TA)(x[e] * inv * w[i + e]);
+    *reinterpret_cast<vec*>(h + (size_t)row * D + i) = o;
+  };
+#pragma unroll
+  for (int q = 0; q < kParRegs; ++q) {
+    const int i = tid * VEC + step * q;
+    if (i < D) {
+      if (h1) put(v[q], i, w1, h1);
+      if (h2) put(v[q], i, w2, h2);
+    }
+  }
+  for (int i = tid * VEC + step * kParRegs; i < D; i += step) {
+    const fvec x = *reinterpret_cast<const fvec*>(r + i);
+    if (h1) put(x, i, w1, h1);
+    if (h2) put(x, i, w2, h2);
+  }
+}
+
+// The same for few rows (up to kAheadRows) of at most NQ groups a thread, bound by latency: every load of the groups, the norm weights
+// too, is issued before the first is waited for (groups past the row read its last again). It takes more registers, which cost more
+// rows a chip than a round trip does. Above -> here, us, bf16, two branches and two norms: 24 rows of 512 3.4 -> 3.1, of 1024 3.8 ->
+// 3.5, of 2048 4.8 -> 4.5; 256 rows of 2048 5.3 -> 5.1. One branch and one norm of 400 rows of 2048 4.4 -> 4.7, 2000 rows 7.8 -> 10.5;
+// four groups a thread 4.6 -> 4.8 (24 rows of 4096), eight 6.6 -> 7.5.
+constexpr int kAheadRows = 256;
+
+template <typename TA, int VEC, int NQ>
+__global__ __launch_bounds__(256) void parallel_add_norm_ahead_kernel(float* __restrict__ res, const TA* __restrict__ a, int lda,
+                                                                      const float* __restrict__ sa, const TA* __restrict__ b,
+                                                                      int ldb, const float* __restrict__ sb,
+                                                                      const float* __restrict__ w1, TA* __restrict__ h1,
+                                                                      const float* __restrict__ w2, TA* __restrict__ h2, int D,
+                                                                      float eps) {
   typedef TA vec __attribute__((ext_vector_type(VEC)));
   typedef float fvec __attribute__((ext_vector_type(VEC)));
   __shared__ float scratch[16];
@@ -698,18 +774,17 @@ void gai_parallel_add_norm_f32(float* res, const void* a, int lda, const float* 
   const bool four = D % 4 == 0 && (!a || lda % 4 == 0) && (!b || ldb % 4 == 0) && ((size_t)res & 15) == 0 &&
                     (((size_t)a | (size_t)b | (size_t)h1 | (size_t)h2) & mask) == 0;
   const int groups = four ? D / 4 : D, nt = groups >= 256 ? 256 : (groups + 63) / 64 * 64;
-#define GAI_PAN_Q(TA, VEC_, NQ)                                                                                        \
-  parallel_add_norm_kernel<TA, VEC_, NQ><<<T, nt, 0, st>>>(res, (const TA*)a, lda, sa, (const TA*)b, ldb, sb, w1,      \
-                                                           (TA*)h1, w2, (TA*)h2, D, eps)
+#define GAI_PAN_ARGS(TA) (res, (const TA*)a, lda, sa, (const TA*)b, ldb, sb, w1, (TA*)h1, w2, (TA*)h2, D, eps)
 #define GAI_PAN(TA, VEC_)                                                                                              \
   do {                                                                                                                 \
-    if (groups <= 2 * nt) GAI_PAN_Q(TA, VEC_, 2);                                                                      \
-    else if (groups <= 4 * nt) GAI_PAN_Q(TA, VEC_, 4);                                                                 \
-    else GAI_PAN_Q(TA, VEC_, 8);                                                                                       \
+    constexpr int most = VEC_ == 1 ? 8 : 2;                                                                            \
+    if (T > kAheadRows || groups > most * nt) parallel_add_norm_kernel<TA, VEC_><<<T, nt, 0, st>>> GAI_PAN_ARGS(TA);   \
+    else if (groups <= 2 * nt) parallel_add_norm_ahead_kernel<TA, VEC_, 2><<<T, nt, 0, st>>> GAI_PAN_ARGS(TA);         \
+    else parallel_add_norm_ahead_kernel<TA, VEC_, most><<<T, nt, 0, st>>> GAI_PAN_ARGS(TA);                            \
   } while (0)
   if (dt) { if (four) GAI_PAN(float, 4); else GAI_PAN(float, 1); }
   else { if (four) GAI_PAN(bf16, 4); else GAI_PAN(bf16, 1); }
 #undef GAI_PAN
-#undef GAI_PAN_Q
+#undef GAI_PAN_ARGS
   GAI_LAUNCH_CHECK();
 }

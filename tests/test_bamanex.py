@@ -209,6 +209,23 @@ def test_parallel_add_norm_kept_groups(D):
         assert ((h.double() - ref).abs() <= (2.0 ** -8 + 2e-6) * ref.abs()).all()
 
 
+@_GPU
+@pytest.mark.parametrize("D", [64, 513, 1000, 2048, 2050, 4096, 8196])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_parallel_add_norm_rows_alike(D, dt):
+    """A row has the same sums and norms whether it comes with few rows or with more than the form for few rows takes."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    res, a, b, w1, w2, sa = rn(257, D), rn(257, D).to(dt), rn(257, D).to(dt), rn(D), rn(D), rn(D)
+    kw = dict(w1=w1, w2=w2, sa=sa, eps=1e-5, out_dtype=dt)
+    few = res.clone()
+    parts = [ops.parallel_add_norm_f32(few[s:e], a=a[s:e], b=b[s:e], **kw) for s, e in ((0, 256), (256, 257))]
+    h = ops.parallel_add_norm_f32(res, a=a, b=b, **kw)
+    assert torch.equal(res, few)
+    for i in range(2):
+        assert torch.equal(h[i], torch.cat([p[i] for p in parts]))
+
+
 @pytest.mark.parametrize("device,dtype", TARGETS)
 def test_rotation_unit_norm_and_cache_write(device, dtype):
     """Rotated halves at positions up to 10^5 with and without the unit norm, tokens in scattered slots and tokens that fill
