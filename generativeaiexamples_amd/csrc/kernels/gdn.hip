@@ -577,9 +577,10 @@ __global__ __launch_bounds__(512, 1) void gdn_carry_kernel(
   }
 }
 
-// Key heads of 256: neither registers nor LDS for two chunks, and four waves do everything.
+// Four waves do everything, a chunk's rows are fetched when it begins: key heads of 256, for two chunks of which there are neither
+// registers nor LDS, and many short portions (the rule at the launch), where the next workgroup hides what the next chunk does not.
 template <int DK>
-__global__ __launch_bounds__(256, 1) void gdn_carry_wide_kernel(
+__global__ __launch_bounds__(256, 1) void gdn_carry_plain_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ To,
     const float* __restrict__ Mo, const float* __restrict__ Fo, const int* __restrict__ chunks,
     const int* __restrict__ chunk0, const int* __restrict__ slots, int Hk, int Hv, int DV, float* __restrict__ state,
@@ -793,6 +794,10 @@ void gai_gdn_prep(const void* proj, int ld, const float* cw, const float* cstate
 // 6000 + 4095 tokens, 8 key / 16 value heads of 128 x 128: gdn_chunk 101 us, gdn_carry 290 us (94 chunks in a row at 3.0 us,
 // 256 workgroups), against 47 ms for the same rule as batched fp32 products and triangular solves chunk by chunk in torch;
 // error of o against float64 2.2e-7 - 3.4e-7 (torch 3.2e-7 - 1.1e-6).
+// Key heads of 64 and many workgroups: two plain ones share a CU, which hides more than one of split roles does by itself. us with
+// gdn_chunk, split / plain, 16 heads of 64 x 128: 64 portions of 16 tokens 136 / 94, of 300 522 / 452, of 1000 1525 / 1379; 8
+// portions of one token (1024 workgroups) 25 / 21, 16 of 190 82 / 73. 8 heads of 64 x 64, 32 portions of 250 (1024 workgroups, four chunks
+// each) 70.0 / 71.3, 2 of 5000 217 / 314.
 void gai_gdn_chunks(const float* q, const float* k, const float* v, const float* g, const float* beta, const int* chunks,
                     const int* chunk0, const int* slots, int nc, int S, int Hk, int Hv, int DK, int DV, float* Ti, float* M,
                     float* F, float* state, float* out, hipStream_t st) {
@@ -800,21 +805,29 @@ void gai_gdn_chunks(const float* q, const float* k, const float* v, const float*
 #define GAI_GDN(D)                                                                                                      \
   if (DK == D) {                                                                                                        \
     const int lds = (kC * (D + 4) + 2 * kC * (kC + 4)) * 4;                                                             \
-    constexpr bool wide = D > 128;                                                                                      \
-    const int lds2 = ((wide ? 2 : 3) * D / 16 + (wide ? 12 : 16)) * 64 * 16 + (wide ? 1 : 2) * kC * (D + 4) * 4;         \
-    auto carry = wide ? gdn_carry_wide_kernel<256> : gdn_carry_kernel<wide ? 128 : D>;                                    \
+    const int wgs = S * Hv * (DV / 16);                                                                                 \
+    constexpr int lds_plain = (2 * D / 16 + 12) * 64 * 16 + kC * (D + 4) * 4;                                           \
+    constexpr int lds_split = (3 * D / 16 + 16) * 64 * 16 + 2 * kC * (D + 4) * 4;                                       \
+    constexpr int DP = D == 128 ? 64 : D, DS = D > 128 ? 128 : D; /* the widths that either kernel is reached with */   \
+    const bool plain = D > 128 || (D == 64 && (wgs >= 2048 || (wgs > 256 && nc < 4 * S)));                             \
     static bool once = false;                                                                                           \
     if (!once) {                                                                                                        \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gdn_chunk_kernel<D>),                                     \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);                                       \
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(carry),                                                   \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, lds2);                                      \
+      auto allow = [](const void* f, int bytes) {                                                                       \
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);                                \
+      };                                                                                                                \
+      allow(reinterpret_cast<const void*>(gdn_chunk_kernel<D>), lds);                                                   \
+      allow(reinterpret_cast<const void*>(gdn_carry_plain_kernel<DP>), lds_plain);                                       \
+      if (D <= 128) allow(reinterpret_cast<const void*>(gdn_carry_kernel<DS>), lds_split);                              \
       once = true;                                                                                                      \
     }                                                                                                                   \
     gdn_chunk_kernel<D><<<dim3(nc, Hv), 256, lds, st>>>(q, k, g, beta, chunks, Hk, Hv, Ti, M, F);                       \
     GAI_LAUNCH_CHECK();                                                                                                 \
-    carry<<<S * Hv * (DV / 16), wide ? 256 : 512, lds2, st>>>(q, k, v, Ti, M, F, chunks, chunk0, slots, Hk, Hv, DV,      \
-                                                              state, out);                                              \
+    if (plain)                                                                                                          \
+      gdn_carry_plain_kernel<DP><<<wgs, 256, lds_plain, st>>>(q, k, v, Ti, M, F, chunks, chunk0, slots, Hk, Hv, DV,      \
+                                                             state, out);                                               \
+    else                                                                                                                \
+      gdn_carry_kernel<DS><<<wgs, 512, lds_split, st>>>(q, k, v, Ti, M, F, chunks, chunk0, slots, Hk, Hv, DV, state,    \
+                                                        out);                                                           \
     GAI_LAUNCH_CHECK();                                                                                                 \
     return;                                                                                                             \
   }

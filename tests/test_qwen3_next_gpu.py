@@ -67,6 +67,33 @@ def test_gdn_chunks_against_float64(cuda, lens, Hk, Hv, dk, dv):
         assert (a.cpu().double() - b).norm() <= 4.8e-6 * b.norm()
 
 
+@pytest.mark.parametrize("lens,Hv,dv", [([1, 64, 0, 65, 130, 7] * 5, 8, 64), ([3, 200] * 32, 8, 64)])
+def test_gdn_chunks_many_portions(cuda, lens, Hv, dv):
+    """Many short portions of narrow heads, whose kernel differs from that of a few: the bits of every portion by itself."""
+    torch.manual_seed(len(lens))
+    T, S, Hk, dk = sum(lens), len(lens), 4, 64
+    q, k = (torch.nn.functional.normalize(torch.randn(T, Hk, dk, device=cuda), dim=-1) for _ in range(2))
+    v, g, beta = torch.randn(T, Hv, dv, device=cuda), -torch.rand(T, Hv, device=cuda), torch.rand(T, Hv, device=cuda)
+    state = torch.randn(S, Hv, dk, dv, device=cuda) * 0.1
+
+    def run(at, n, slots):
+        st, out = state.clone(), torch.full((sum(n), Hv, dv), float("nan"), device=cuda)
+        part = [t[at:at + sum(n)].contiguous() for t in (q, k, v, g, beta)]
+        chunks, chunk0 = ops.gdn_chunk_plan(n, cuda)
+        ops.gdn_chunks(*part, chunks, chunk0, torch.tensor(slots, dtype=torch.int32, device=cuda), st, out)
+        return out, st
+
+    out, st = run(0, lens, list(range(S)))
+    at = 0
+    for s, n in enumerate(lens):
+        if n:
+            o1, s1 = run(at, [n], [s])
+            assert torch.equal(out[at:at + n], o1) and torch.equal(st[s], s1[s])
+        else:
+            assert torch.equal(st[s], state[s])
+        at += n
+
+
 @pytest.mark.parametrize("lens,Hk,Hv,dk,dv,dt", [([1, 2, 5], 2, 4, 64, 64, torch.bfloat16), ([700, 1, 3, 0, 9], 1, 3, 128, 48, torch.bfloat16),
                                                  ([1] * 5, 2, 2, 256, 16, torch.float32)])
 def test_gdn_prep_matches_torch(cuda, lens, Hk, Hv, dk, dv, dt):
