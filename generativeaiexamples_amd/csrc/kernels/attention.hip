@@ -1226,11 +1226,14 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 // resident: each begins with one and draws its next when it is about to finish, from the queue of its XCD (one counter for all,
 // drawn from 2048 times, took 2 - 4 us of a launch). There, of ragged contexts' parts the long ones may start last, and every part
 // starts anew with nothing in flight; here the next part's first chunk is on its way while the finished one is combined. One
-// card, 8 kv heads, graphs captured for 8192, there -> here, us: bf16, 64 sequences of 640 - 2663 keys 94.4 -> 87.7, of 40 - 700
-// 43.6 -> 33.4, 32 of 500 - 3000 57.8 -> 50.7, 23 of 1900 - 7900 92 -> 86.4; fp8 61 -> 56.8, 29.4 -> 26.0, 38.4 -> 34.0, 61.6 ->
-// 56.3. With no more parts than two a CU there is nothing to hand out (16 sequences 30.8 -> 31.7, 8 19.1 -> 20.3). Even cuts of
-// the whole batch's keys instead of each sequence's took 83, 30, 49 and 86 us, with other sums. Parts dealt beforehand, forth
-// and back, 93, 34, 54, 89. A second chunk in flight per wave changed nothing: what is left is the stream of 4-KB (2-KB) pages.
+// card, 8 kv heads, graphs captured for 8192, there -> here, us: bf16, 64 sequences of 640 - 2663 keys 102 -> 90, of 40 - 700
+// 44.2 -> 31.4, 32 of 500 - 3000 59.3 -> 50.8, 23 of 1900 - 7900 98 -> 92; fp8 66.7 -> 55.2, 33.1 -> 23.9, 43.3 -> 33.5, 67.6 ->
+// 56.8. Where every part is resident at once (up to 64 sequences) the launch only spreads them evenly: 24 of 30 - 300 keys 10.8 -> 11.0,
+// of 30 - 100 7.4 -> 6.8, 64 of them 20.6 -> 8.8. Ranked and drawn from all the same, 13.2 and 8.9; ranked through LDS by a thread a
+// sequence, one after another, 1 us more at 24 sequences and 10 at 256. Equal contexts gain nothing (32 of 2600 - 2700 72.6 -> 74.6).
+// Even cuts of the whole batch's keys instead of each sequence's took 83, 30, 49 and 86 us where the parts here took 88, 33, 51 and 86,
+// with other sums. Parts dealt beforehand, forth and back, 93, 34, 54, 89. A second chunk in flight per wave changed nothing: what is
+// left is the stream of 4-KB (2-KB) pages.
 constexpr int kQueueSeqs = 256;  // sequences that the ranking holds
 template <int D, typename KV, bool NTL, bool QP>
 __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
@@ -1247,30 +1250,78 @@ __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), gq = lane >> 4, qi = lane & 15;
   const int ratio = Hq / Hkv;
   const float sl2 = scale * kLog2e;
-  // sequences by falling length; the parts, one kv head after another, are numbered in that order
-  if (tid < B) {
-    const int ctx = max(ctx_lens[tid], 0);
-    s_ctx[tid] = ctx;
-    s_parts[tid] = (ctx + split_len(0, ctx, max_splits) - 1) / split_len(0, ctx, max_splits);
-  }
-  __syncthreads();
-  if (tid < B) {
-    const int ctx = s_ctx[tid];
-    int rank = 0, first = 0;
-    for (int j = 0; j < B; ++j) {
-      const bool before = s_ctx[j] > ctx || (s_ctx[j] == ctx && j < tid);
-      rank += before;
-      first += before ? s_parts[j] : 0;
-    }
-    s_seq[rank] = tid;
-    s_first[rank] = first * Hkv;
-    if (rank == B - 1) s_total = (first + s_parts[tid]) * Hkv;
-  }
-  __syncthreads();
-  const int total = __builtin_amdgcn_readfirstlane(s_total);
   struct Part {
     int seq, g, split, ctx, kstart, kend, nsplit;
   };
+  auto part = [&](int seq, int ctx, int i) {  // part i of a sequence, one kv head after another
+    const int len = split_len(0, ctx, max_splits);
+    Part p;
+    p.seq = seq;
+    p.ctx = ctx;
+    p.split = i / Hkv;
+    p.g = i - p.split * Hkv;
+    p.nsplit = (ctx + len - 1) / len;
+    p.kstart = p.split * len;
+    p.kend = min(ctx, p.kstart + len);
+    return p;
+  };
+  auto parts_of = [&](int ctx) { return (ctx + split_len(0, ctx, max_splits) - 1) / split_len(0, ctx, max_splits); };
+  const int x8 = blockIdx.x & 7, G = gridDim.x / 8;
+  int item = blockIdx.x >> 3, total = 0;
+  Part p;
+  bool drawing = true;
+  if (B <= 64) {
+    // With no more parts than workgroups there is nothing to rank or draw (short contexts in a graph captured for long ones): every
+    // wave numbers the parts in the sequences' own order.
+    const int ctx = lane < B ? max(ctx_lens[lane], 0) : 0, n = lane < B ? parts_of(ctx) : 0;
+    int run = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(run, o, 64);
+      if (lane >= o) run += up;
+    }
+    total = __builtin_amdgcn_readlane(run, 63) * Hkv;
+    drawing = total > (int)gridDim.x;
+    if (!drawing) {
+      const int i = 8 * item + x8;
+      if (i >= total) return;
+      const int r = __popcll(__ballot(lane < B && (run - n) * Hkv <= i)) - 1;
+      p = part(r, __builtin_amdgcn_readlane(ctx, r), i - __builtin_amdgcn_readlane(run - n, r) * Hkv);
+    }
+  }
+  if (drawing) {
+    // Sequences by falling length; the parts are numbered in that order. Every wave compares all sequences, one a lane, with a quarter
+    // of them, held a lane each and read from there.
+    for (int i = tid; i < kQueueSeqs; i += 256) s_seq[i] = 0;
+    const int quarter = (B + 3) / 4, j0 = wid * quarter, nj = min(quarter, B - j0);
+    int key = 0, val = 0;  // longer first, then as given; one sequence and its parts (B * max_splits < 2^22)
+    if (lane < nj) {
+      const int j = j0 + lane, ctx = max(ctx_lens[j], 0), n = parts_of(ctx);
+      s_ctx[j] = ctx;
+      s_parts[j] = n;
+      s_first[j] = key = min(ctx, (1 << 23) - 1) << 8 | (255 - j);
+      val = n << 9 | 1;
+    }
+    __syncthreads();
+    for (int i0 = 0; i0 < B; i0 += 64) {
+      const int i = min(i0 + lane, B - 1), mine = s_first[i];
+      int sum = 0;
+      for (int j = 0; j < nj; ++j)
+        sum += __builtin_amdgcn_readlane(key, j) > mine ? __builtin_amdgcn_readlane(val, j) : 0;
+      if (i0 + lane < B && sum) atomicAdd(&s_seq[i], sum);
+    }
+    __syncthreads();
+    const int before = tid < B ? s_seq[tid] : 0;
+    __syncthreads();
+    if (tid < B) {
+      const int rank = before & 511, first = before >> 9;
+      s_seq[rank] = tid;
+      s_first[rank] = first * Hkv;
+      if (rank == B - 1) s_total = (first + s_parts[tid]) * Hkv;
+    }
+    __syncthreads();
+    total = __builtin_amdgcn_readfirstlane(s_total);
+  }
   auto find = [&](int item) {
     int r = -1;  // the last rank that begins at or before item
     for (int b0 = 0; b0 < B; b0 += 64) {
@@ -1278,31 +1329,22 @@ __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
       r += n;
       if (n < 64) break;
     }
-    Part p;
     r = __builtin_amdgcn_readfirstlane(r);
-    p.seq = __builtin_amdgcn_readfirstlane(s_seq[r]);
-    p.ctx = __builtin_amdgcn_readfirstlane(s_ctx[p.seq]);
-    const int i = item - __builtin_amdgcn_readfirstlane(s_first[r]);
-    p.split = i / Hkv;
-    p.g = i - p.split * Hkv;
-    const int len = split_len(0, p.ctx, max_splits);
-    p.nsplit = (p.ctx + len - 1) / len;
-    p.kstart = p.split * len;
-    p.kend = min(p.ctx, p.kstart + len);
-    return p;
+    const int seq = __builtin_amdgcn_readfirstlane(s_seq[r]);
+    return part(seq, __builtin_amdgcn_readfirstlane(s_ctx[seq]), item - __builtin_amdgcn_readfirstlane(s_first[r]));
   };
-  // queue x: parts x, x + 8, ..; its workgroups (gridDim.x / 8) begin with the first ones and draw until nothing is left
-  const int x8 = blockIdx.x & 7, mine = (total - x8 + 7) / 8, G = gridDim.x / 8, draws = max(mine - G, 0) + G;
+  // queue x: parts x, x + 8, ..; its workgroups (gridDim.x / 8) begin with the first ones and draw until nothing is left, mine times in
+  // all; with no more parts than workgroups nobody draws
+  const int mine = (total - x8 + 7) / 8;
+  const bool ranked = drawing;
+  drawing = mine > G;
   int* queue = cnt + B * Hkv + x8 * 32;  // 0 between launches
   auto draw = [&]() { return __hip_atomic_fetch_add(queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
   auto drew = [&](int n) {
-    if (n == draws - 1) __hip_atomic_store(queue, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (n == mine - 1) __hip_atomic_store(queue, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  int item = blockIdx.x >> 3;
-  if (item >= mine) {
-    if (tid == 0) drew(draw());
-    return;
-  }
+  if (item >= mine) return;
+  if (ranked) p = find(8 * item + x8);
 
   bf16x8 qf[D / 32];
   DecAcc<D> acc;
@@ -1313,7 +1355,6 @@ __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
   auto early = [&](const Part& p, int kb) {
     return kb < p.kend && !(QP && p.split == p.nsplit - 1 && kb <= p.ctx - 1 && p.ctx - 1 < kb + 32);
   };
-  Part p = find(8 * item + x8);
   int kb = p.kstart + 32 * wid;
   dec_lookup<1>(table(p), kb, (p.kend - 1) / kBS, p.ctx, nb);
   bool have = early(p, kb);
@@ -1336,14 +1377,14 @@ __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
     while (kb < p.kend) {
       const int next = kb + 128;
       if (next < p.kend) dec_lookup<1>(bt, next, last_page, p.ctx, nb);
-      else if (tid == 0) drawn = draw();  // (wave 0 has keys of every part) under the last chunk's products
+      else if (drawing && tid == 0) drawn = draw();  // (wave 0 has keys of every part) under the last chunk's products
       acc.add(kb, p.kend, c, qf, sl2, k_scale, v_scale);
       if (next < p.kend) c.load(kc, vc, Hkv, p.g, nb);
       kb = next;
     }
     // combine the 4 waves
     __syncthreads();  // the previous part's sums have been read
-    if (tid == 0) {
+    if (drawing && tid == 0) {
       s_next = G + drawn;
       drew(drawn);
     }
@@ -1356,7 +1397,7 @@ __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) red_o[wid][16 * dt + 4 * gq + r][qi] = acc.o[dt][r];
     __syncthreads();
-    item = __builtin_amdgcn_readfirstlane(s_next);
+    item = drawing ? __builtin_amdgcn_readfirstlane(s_next) : mine;
     const bool more = item < mine;
     Part np = p;
     if (more) {
@@ -1628,7 +1669,7 @@ void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, co
   if (fold != nullptr && !(fuse && ntl && !kv_fp8 && D == 128 && fold->ks >= 1 && fold->ks <= 16))
     gai_launch_error(__FILE__, __LINE__, "attn_decode: the folded QKV tail needs the fused non-temporal bf16 kernel");
   if (queue) {
-    if (!(fuse && D == 128 && split_keys == 0 && B <= kQueueSeqs && (kv_fp8 || ntl)))
+    if (!(fuse && D == 128 && split_keys == 0 && B <= kQueueSeqs && (long long)B * max_splits < 1 << 22 && (kv_fp8 || ntl)))
       gai_launch_error(__FILE__, __LINE__, "attn_decode: the queue is of the fused adaptive form of head_dim 128");
     const GaiQkvFold f = fold ? *fold : GaiQkvFold{};
     const int wgs = (std::min(3 * decode_cus(), B * Hkv * max_splits) + 7) & ~7;  // resident: up to 168 VGPRs, 41 KB of LDS

@@ -630,6 +630,16 @@ _DECODE_ADAPTIVE = os.environ.get("GAI_DECODE_ADAPTIVE", "1") == "1"
 _DECODE_QUEUE = os.environ.get("GAI_DECODE_NT", "1") != "0" and os.environ.get("GAI_DECODE_VARIANT", "1") == "1"
 
 
+def _decode_queue(B: int, Hkv: int, nsplit: int) -> bool:
+    """More parts than two a CU: the same ones, handed out by the launch longest first (attention.hip has the times). With
+    few kv heads, as a tensor-parallel rank has, there are many sequences to rank, and the launch with a workgroup per part is
+    the faster one (8 / 1 heads, 80 sequences of 2600 - 2700 keys 35.8 us a launch, 41.6 with queues; 16 / 2, 80 of 30 - 100 7.8
+    and 10.0) unless the number of parts is a multiple of eight: there a part's number chooses its XCD, and short contexts leave most of
+    them idle (16 / 2, 64 of 30 - 100 13.4 and 7.1, of 500 - 3000 39.8 and 35.7)."""
+    return (nsplit > 1 and B <= 256 and B * Hkv * nsplit > 512 and B * nsplit < 1 << 22
+            and (Hkv >= 4 or (nsplit % 8 == 0 and B <= 128)))
+
+
 def attention_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, ws: DecodeWorkspace | None = None,
                      max_ctx: int | None = None, out=None, k_scale=1.0, v_scale=1.0, qkv_fold=None):
     """qkv_fold = (slabs, ks, positions, cos_sin, slots) from :func:`qkv_fold_partials`: q is computed inside the
@@ -651,9 +661,8 @@ def attention_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, ws: Dec
     # captured for max_ctx balance their splits at every replay (GAI_DECODE_ADAPTIVE=0: fixed split_keys)
     f = qkv_fold if qkv_fold is not None else (None, 0, None, None, None)
     adaptive = _DECODE_ADAPTIVE and ws.fixed_split is None
-    # more parts than two a CU: the same ones, handed out by the launch longest first (attention.hip has the times)
     pairs = B * k_cache.shape[1]
-    queue = (adaptive and _DECODE_QUEUE and _ATTN_FUSE and D == 128 and nsplit > 1 and B <= 256 and pairs * nsplit > 512
+    queue = (adaptive and _DECODE_QUEUE and _ATTN_FUSE and D == 128 and _decode_queue(B, k_cache.shape[1], nsplit)
              and ws.cnt.numel() >= pairs + native().DECODE_QUEUE_INTS)
     native().attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, out, ws.o, ws.ml, scale,
                          0 if adaptive else split, nsplit, k_scale, v_scale,

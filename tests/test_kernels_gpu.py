@@ -267,7 +267,9 @@ def test_attention_decode_adaptive_splits(cuda, nsplit):
     (32, 8, 7, [2663, 31, 4097, 640, 1, 300, 2048, 255, 33, 96, 97, 1500]),
     (64, 8, 33, [4200, 4096, 700, 700, 129]),             # a part per unit
     (16, 4, 4, [(37 * i * i) % 701 for i in range(131)]),  # more parts than workgroups; equal lengths, empty sequences
-    (8, 8, 9, [8000, 1] * 100), (32, 8, 2, [0, 0, 0])])
+    (8, 8, 9, [8000, 1] * 100), (32, 8, 2, [0, 0, 0]),
+    (32, 8, 8, [2663 - 97 * i for i in range(24)]), (8, 4, 4, [513] * 63 + [0]), (8, 4, 4, [513] * 64 + [0]),  # ranked, one wave's worth or more
+    (8, 4, 2, [(91 * i) % 300 for i in range(256)]), (8, 4, 3, [0] * 60 + [300] * 4), (4, 4, 3, [60] * 70)])  # all resident
 def test_attention_decode_queue(cuda, Hq, Hkv, nsplit, ctx, fp8):
     """Parts handed out by the launch: the bits of the launch with a workgroup per part, whatever their number and order; rows of
     sequences without keys are left alone; tickets and counters back at zero; graph replays the same."""
