@@ -9,6 +9,7 @@
 from __future__ import annotations
 
 import os
+import re
 from typing import Optional, Sequence
 
 import numpy as np
@@ -627,7 +628,18 @@ _DECODE_MAX_SPLIT = int(os.environ.get("GAI_DECODE_MAX_SPLIT", "2048"))  # keys 
 # up to this many (sequence, kv head) pairs the split targets one resident wave of workgroups (512) instead of 1024
 _DECODE_ONE_WAVE_PAIRS = int(os.environ.get("GAI_DECODE_ONE_WAVE_PAIRS", "128"))
 _DECODE_ADAPTIVE = os.environ.get("GAI_DECODE_ADAPTIVE", "1") == "1"
-_DECODE_QUEUE = os.environ.get("GAI_DECODE_NT", "1") != "0" and os.environ.get("GAI_DECODE_VARIANT", "1") == "1"
+
+
+def _decode_default() -> bool:
+    """The launcher's switches GAI_DECODE_NT and GAI_DECODE_VARIANT leave the default kernel, read as it reads them (atoi: the
+    leading number, or 0)."""
+    def atoi(name):
+        m = re.match(r"[ \t\n\v\f\r]*([+-]?[0-9]+)", os.environ.get(name, "1"))
+        return int(m[1]) if m else 0
+    return atoi("GAI_DECODE_NT") != 0 and atoi("GAI_DECODE_VARIANT") == 1
+
+
+_DECODE_QUEUE = _decode_default()
 
 
 def _decode_queue(B: int, Hkv: int, nsplit: int) -> bool:
@@ -674,8 +686,7 @@ def attention_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, ws: Dec
 # partial slabs, and attention_decode sums them, applies RoPE and writes the new key / value itself - one launch per
 # layer fewer than the split-K RoPE / KV-write tail (GAI_QKV_FOLD=0: the tail kernel). Needs the default fused,
 # non-temporal bf16 decode kernel.
-_QKV_FOLD = (os.environ.get("GAI_QKV_FOLD", "1") == "1" and os.environ.get("GAI_DECODE_NT", "1") != "0"
-             and os.environ.get("GAI_DECODE_VARIANT", "1") == "1")
+_QKV_FOLD = os.environ.get("GAI_QKV_FOLD", "1") == "1" and _decode_default()
 
 
 def qkv_fold_partials(x: torch.Tensor, w, bias, k_cache, head_dim: int, ws: "DecodeWorkspace | None", k_scale=1.0,
