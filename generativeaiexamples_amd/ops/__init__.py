@@ -572,7 +572,6 @@ class DecodeWorkspace:
     split can be chosen per call / per captured batch bucket (graph-capture safe)."""
 
     MIN_SPLIT = 128
-    QUEUE_INTS = 256  # kGaiDecodeQueueInts
 
     def __init__(self, max_batch: int, Hq: int, D: int, max_ctx: int, device, split_keys: int | None = None):
         self.fixed_split = split_keys
@@ -581,9 +580,9 @@ class DecodeWorkspace:
         self.o = torch.empty(self.max_splits * max_batch * Hq * D, dtype=torch.float32, device=device)
         self.ml = torch.empty(self.max_splits * max_batch * Hq * 2, dtype=torch.float32, device=device)
         # split tickets of the in-launch merge (one per (sequence, kv head) <= max_batch * Hq): zero at
-        # allocation, reset by each merge's last split; behind them the queues' counters,
-        # reset by their last draw
-        self.cnt = torch.zeros(max_batch * Hq + self.QUEUE_INTS, dtype=torch.int32, device=device)
+        # allocation, reset by each merge's last split; behind them the queues' counters, reset by their last draw
+        queues = native().DECODE_QUEUE_INTS if torch.device(device).type == "cuda" else 0
+        self.cnt = torch.zeros(max_batch * Hq + queues, dtype=torch.int32, device=device)
 
     @property
     def split_keys(self) -> int:

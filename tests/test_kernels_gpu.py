@@ -308,6 +308,27 @@ def test_attention_decode_queue(cuda, Hq, Hkv, nsplit, ctx, fp8):
         ops.native().attn_decode(q, kc, vc, bt, c, out, ws.o, ws.ml, scale, 0, nsplit, sk, sv, ws.cnt[: B * Hkv], queue=True)
 
 
+def test_decode_workspace_holds_the_queues(cuda, monkeypatch):
+    """A workspace has room for whatever the launch asks for its queues, also behind a ticket for every sequence and q head."""
+    nat = ops.native()
+
+    class Larger:
+        DECODE_QUEUE_INTS = nat.DECODE_QUEUE_INTS + 64
+
+        def __getattr__(self, name):
+            return getattr(nat, name)
+
+    monkeypatch.setattr(ops, "native", Larger)
+    B, H, D = 70, 8, 128
+    kc, vc, bt = _paged_setup([600] * B, H, D, cuda, seed=1)
+    ws, took = ops.DecodeWorkspace(B, H, D, 1024, cuda), []
+    attn = nat.attn_decode
+    monkeypatch.setattr(Larger, "attn_decode", lambda self, *a: took.append(a[-1]) or attn(*a), raising=False)
+    q = torch.randn(B, H, D, device=cuda, dtype=torch.bfloat16)
+    ops.attention_decode(q, kc, vc, bt, torch.full((B,), 600, dtype=torch.int32, device=cuda), 0.1, ws=ws, max_ctx=1024)
+    assert took == [True] and ops.DecodeWorkspace(B, H, D, 1024, "cpu").cnt.numel() == B * H
+
+
 def test_attention_decode_fused_merge_reuse(cuda):
     """In-launch split merge (ticket counters, last split combines): equal to the separate reduce launch, and
     the counters reset themselves - many back-to-back launches and graph replays on one workspace, with the
