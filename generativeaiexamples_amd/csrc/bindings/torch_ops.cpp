@@ -298,6 +298,7 @@ void attn_rows(const Tensor& qkv, const Tensor& tiles, const Tensor& cu_q, const
   check_bf16(out, "out");
   TORCH_CHECK(qkv.dim() == 2 && qkv.is_contiguous() && H > 0 && qkv.size(1) == 3 * H * 64, "attn_rows: qkv [T, 3 H 64]");
   TORCH_CHECK(out.is_contiguous() && out.numel() == qkv.size(0) * H * 64, "attn_rows: out [T, H 64]");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0, "attn_rows: qkv on 16 bytes");
   TORCH_CHECK(cu_q.numel() == ctx_lens.numel() + 1, "attn_rows: cu_q");
   TORCH_CHECK(qkv.numel() * 2 < (int64_t)1 << 31, "attn_rows: rows beyond 32-bit offsets");
   gai_attn_rows(qkv.data_ptr(), (int)qkv.size(1), tiles.data_ptr<int>(), tiles.numel() / 2, cu_q.data_ptr<int>(),

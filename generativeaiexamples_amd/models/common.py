@@ -164,7 +164,7 @@ class PackedAttention:
     def __call__(self, qkv: torch.Tensor, scale: float, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """qkv [T, (H + 2 Hkv) * hd] -> attention output [T, H * hd]."""
         from .. import ops
-        if self.direct and qkv.is_contiguous():
+        if self.direct and qkv.is_contiguous() and not qkv.data_ptr() & 15:  # (16-byte buffer loads)
             o = torch.empty_like(self.q) if out is None else out.view(self.T, self.H, self.hd)
             ops.native().attn_rows(qkv, self.tiles, self.cu_q, self.ctx, o, self.H, scale, self.causal)
             return o.view(self.T, self.H * self.hd)

@@ -82,3 +82,18 @@ def test_rows_attention_equals_paged(cuda, lens, H, short, causal):
     ops.attention_prefill(qkv.view(T, 3 * H, D)[:, :H], a.k_cache, a.v_cache, a.block_tables, a.cu_q, a.ctx, 0.2, causal=causal,
                           tiles=a.tiles, q_lens=lens, out=want)
     assert torch.equal(out, want.view(T, H * D))
+
+
+@pytest.mark.parametrize("off", [2, 4])
+def test_rows_off_16_bytes_take_the_pages(cuda, off):
+    """QKV rows that begin off a 16-byte line: the bits of the same rows on one, and no call of the kernel that reads them by
+    16-byte buffer loads, which refuses them."""
+    torch.manual_seed(off)
+    lens, H = [70, 1, 33], 2
+    T = sum(lens)
+    qkv = torch.randn(T * 3 * H * 64 + off, device=cuda).to(torch.bfloat16)[off:].view(T, 3 * H * 64)
+    assert qkv.data_ptr() % 16
+    a = PackedAttention(lens, H, 64, cuda)
+    assert a.direct and torch.equal(a(qkv, 0.2), a(qkv.clone(), 0.2))
+    with pytest.raises(RuntimeError, match="16 bytes"):
+        ops.native().attn_rows(qkv, a.tiles, a.cu_q, a.ctx, torch.empty(T, H * 64, device=cuda, dtype=torch.bfloat16), H, 0.2, False)
