@@ -160,10 +160,10 @@ def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
     if x.is_cuda and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.bfloat16:
         K, N = x.shape[-1], w.shape[0]
         M = x.numel() // K
-        ks = native().gemm_slim_ks(M, N, K) if M <= 64 else 0
+        psw = decode_operand(w)
+        ks = native().gemm_slim_ks(M, N, K) if M <= 64 and (psw is not None or (_SPLITK and _GEMM_FORCE == 0)) else 0
         # 16-byte loads of rows and vectors that the two separate ops read singly
         if ks and residual.is_contiguous() and not any(t.data_ptr() & 15 for t in (x, residual, bias, ln_w, ln_b) if t is not None):
-            psw = decode_operand(w)
             out = torch.empty_like(residual)
             ws = torch.empty(ks, M, N, dtype=torch.float32, device=x.device)
             native().linear_layernorm(x.contiguous(), w if psw is None else psw, bias, residual, ln_w, ln_b, eps, out, ws,

@@ -327,3 +327,16 @@ def test_product_in_slices_and_norm(cuda, M, N, K, ks, frag):
     odd = torch.empty(M * N + 1, device=cuda, dtype=torch.bfloat16)[1:].view(M, N).copy_(r)  # not on 16 bytes: the two ops
     z = ops.layer_norm(ops.linear(x, w, bias=bias, residual=odd), g, b, 1e-5)
     assert torch.equal(ops.linear_layer_norm(x, w, bias, odd, g, b, 1e-5), z)
+
+
+@pytest.mark.parametrize("name,value", [("_SPLITK", False), ("_GEMM_FORCE", 2)])
+def test_linear_layer_norm_under_the_gemm_switches(cuda, monkeypatch, name, value):
+    """A forced GEMM kernel, or the decode GEMMs switched off, hold for the product before a layer norm too."""
+    torch.manual_seed(0)
+    x, r = torch.randn(20, 1024, device=cuda).bfloat16(), torch.randn(20, 1024, device=cuda).bfloat16()
+    w = (torch.randn(1024, 1024, device=cuda) / 32).bfloat16()
+    g, b = torch.randn(1024, device=cuda).bfloat16(), torch.randn(1024, device=cuda).bfloat16()
+    monkeypatch.setattr(ops, name, value)
+    want = ops.layer_norm(ops.linear(x, w, bias=b, residual=r), g, b, 1e-5)
+    monkeypatch.setattr(ops.native(), "linear_layernorm", None)
+    assert torch.equal(ops.linear_layer_norm(x, w, b, r, g, b, 1e-5), want)
