@@ -164,7 +164,7 @@ def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
         ks = native().gemm_slim_ks(M, N, K) if M <= 64 and (psw is not None or (_SPLITK and _GEMM_FORCE == 0)) else 0
         # 16-byte loads of rows and vectors that the two separate ops read singly
         if ks and residual.is_contiguous() and not any(t.data_ptr() & 15 for t in (x, residual, bias, ln_w, ln_b) if t is not None):
-            out = torch.empty_like(residual)
+            out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
             ws = torch.empty(ks, M, N, dtype=torch.float32, device=x.device)
             native().linear_layernorm(x.contiguous(), w if psw is None else psw, bias, residual, ln_w, ln_b, eps, out, ws,
                                       psw is not None)

@@ -340,3 +340,12 @@ def test_linear_layer_norm_under_the_gemm_switches(cuda, monkeypatch, name, valu
     want = ops.layer_norm(ops.linear(x, w, bias=b, residual=r), g, b, 1e-5)
     monkeypatch.setattr(ops.native(), "linear_layernorm", None)
     assert torch.equal(ops.linear_layer_norm(x, w, b, r, g, b, 1e-5), want)
+
+
+@pytest.mark.parametrize("M", [20, 70])
+def test_linear_layer_norm_has_the_rows_shape(cuda, M):
+    """The result has the shape of the product's rows, whatever that of the residual's, on either side of the K slices' reach."""
+    torch.manual_seed(1)
+    x, r = torch.randn(2, M // 2, 1024, device=cuda).bfloat16(), torch.randn(M, 1024, device=cuda).bfloat16()
+    w, g = (torch.randn(1024, 1024, device=cuda) / 32).bfloat16(), torch.randn(1024, device=cuda).bfloat16()
+    assert ops.linear_layer_norm(x, w, None, r, g, None, 1e-5).shape == (2, M // 2, 1024)
