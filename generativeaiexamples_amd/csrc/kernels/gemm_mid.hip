@@ -6,18 +6,22 @@
 // are. So:
 //  * a workgroup takes 16 * MT rows x 64 * NG columns: 128 x 64 (two workgroups share a CU), 128 x 128 or, so that up to
 //    192 rows still fetch the weights once, 192 x 128;
-//  * the weights go straight to registers in operand layout (wave = 16 * NG columns x half of a 64-deep K step: nothing is
-//    fetched twice); the rows of A, which sit in L2, go to an LDS ring by DMA and are read by all waves. Loads return in
-//    order, so A is asked for as far ahead as the weights are (DB steps): with A a step or two ahead, waiting for it
+//  * weights in fragment order go straight to registers in operand layout (wave = 16 * NG columns x half of a 64-deep K step:
+//    nothing is fetched twice); the rows of A, which sit in L2, go to an LDS ring by DMA and are read by all waves. Loads return
+//    in order, so A is asked for as far ahead as the weights are (DB steps): with A a step or two ahead, waiting for it
 //    waited for weights that were asked for just before (187 rows, 28672 x 4096 SwiGLU 64.3 -> 56.0 us, 4096 x 14336 50.6 ->
 //    44.0, 6144 x 4096 30.7 -> 23.7, 4096 x 4096 23.3 -> 20.5; 1024 rows 4096 x 4096 41.4 -> 37.5). What is left: a CU holds
 //    about 32 KB of misses (a weight stream of 32 KB in flight per CU is as fast as one of 192 KB: 6.3 TB/s on the chip, 60 KB/us
 //    in one CU), and A's 24 KB a step share them, 0.75 us a step without any products. Four waves of 64 columns each (half the
 //    LDS reads) gave nothing: 57.5 us for the first of the products above;
+//  * row-major weights go through LDS beside A, by the same DMA in whole lines: in operand layout a load touches 16 lines for 64 bytes
+//    of each. Row-major, one way -> the other, us: 187 rows 4096 x 14336 61 -> 47, 28672 x 4096 (SwiGLU) 75 -> 65, 448 rows 97 ->
+//    70 and 6144 x 4096 52 -> 36, 512 rows 1024 x 1024 10.5 -> 8.6; the last rows of 18337 x 1024 x 1024 (ORD) 47.5 -> 43.7 in
+//    all. Sums are the layout's own in neither: equal bits;
 //  * K is cut into S parts, so tile x part items fill the CUs;
-//  * measured on one card, weights from HBM, fragment order (row-major 10 - 40 % slower: its loads touch 16 lines each), N x K,
-//    against the kernels it replaced: 187 rows 4096 x 14336 200 -> 44 us, 4096 x 4096 67 -> 20, 6144 x 4096 58 -> 24, 28672 x
-//    4096 (SwiGLU) 76 -> 56; 512 rows 4096 x 14336 82 -> 74;
+//  * measured on one card, weights from HBM, fragment order (row-major: half of 240 products within 7 % of it, nineteen in twenty
+//    within 21 %), N x K, against the kernels it replaced: 187 rows 4096 x 14336 200 -> 44 us, 4096 x 4096 67 -> 20, 6144 x 4096
+//    58 -> 24, 28672 x 4096 (SwiGLU) 76 -> 56; 512 rows 4096 x 14336 82 -> 74;
 //  * MFMA operands swapped (rows = weights), so a lane ends with four consecutive columns of a row: 8-byte stores;
 //  * S > 1: every wave stores its fp32 share (write-through) and draws the (tile, wave) ticket; the one that draws the last
 //    sums the parts in part order - the same result whichever it is - and runs the epilogue. Nobody waits, and a wave that
@@ -71,18 +75,22 @@ __device__ __forceinline__ void store4(void* C, const bf16* bias, const bf16* R,
   }
 }
 
-template <int MT>
-constexpr int mid_ring() { return MT == 12 ? 6 : 4; }  // K steps of A in LDS
+// K steps in LDS: A's, and row-major weights with them (two workgroups of 128 x 64 tiles share a CU)
+template <int MT, int NG, bool FRAG>
+constexpr int mid_ring() { return FRAG ? (MT == 12 ? 6 : 4) : MT == 12 ? 4 : NG == 1 ? 3 : 5; }
+template <int MT, int NG, bool FRAG>
+constexpr int mid_step() { return MT * 2048 + (FRAG ? 0 : NG * 8192); }  // bytes of one
 
-template <int MT, int NG, int EPI, bool OUTF32, bool ORD>
+template <int MT, int NG, int EPI, bool OUTF32, bool ORD, bool FRAG>
 __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B, void* C,
                                                           const bf16* __restrict__ bias, const bf16* R, int M, int N, int K,
-                                                          int ldc, int bfrag, int S, float* ws, int* cnt) {
+                                                          int ldc, int S, float* ws, int* cnt) {
   constexpr int BM = 16 * MT, BN = 64 * NG, NA = MT / 4, NF = MT / 2 * NG;
   constexpr int FW = ORD ? NG / 2 : NG, KF = ORD ? 2 : 1, RW = ORD ? MT : MT / 2;  // a wave's columns / 16, k32 fragments of a
                                                                                    // step, rows / 16 that it stores
-  constexpr int RING = mid_ring<MT>(), DB = RING - 1, NB = FW * KF, PART = BM * 128;
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // RING x BM x 128 B; at the end the k halves' exchange
+  constexpr int RING = mid_ring<MT, NG, FRAG>(), DB = RING - 1, NB = FW * KF, PART = mid_step<MT, NG, FRAG>();
+  constexpr int YOUNGER = FRAG ? DB * NB + (DB - 1) * NA : (DB - 1) * (NA + NG);  // loads after those of a step's LDS
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // RING x (BM [+ BN]) x 128 B; at the end the k halves' exchange
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tm_n = (M + BM - 1) / BM, tiles = tm_n * ((N + BN - 1) / BN);
   const int id = xcd_remap(blockIdx.x, gridDim.x);
@@ -95,36 +103,40 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
       __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(A) + (size_t)m0 * K, (short)0, 0x7fffffff, 0x00020000);
   const __amdgpu_buffer_rsrc_t rb =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(B) + (size_t)n0 * K, (short)0, 0x7fffffff, 0x00020000);
-  int oa[3], ob[2];  // NA, FW of them
+  // a DMA load: 8 rows x 128 B, the pieces of a row swizzled
+  auto dma_row = [&](int q) { return (q * 8 + wid) * 8 + (lane >> 3); };
+  auto dma_col = [&](int row) { return k0 * (2 * kBK) + (((lane & 7) ^ ((row >> 1) & 7)) << 4); };
+  int oa[3], ob[2];  // NA, FW (NG) of them
 #pragma unroll
-  for (int q = 0; q < NA; ++q) {
-    const int row = (q * 8 + wid) * 8 + (lane >> 3);
-    oa[q] = (min(m0 + row, M - 1) - m0) * K * 2 + k0 * (2 * kBK) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
-  }
+  for (int q = 0; q < NA; ++q) oa[q] = (min(m0 + dma_row(q), M - 1) - m0) * K * 2 + dma_col(dma_row(q));
+  if constexpr (FRAG) {
 #pragma unroll
-  for (int f = 0; f < FW; ++f) {
-    const int col = (g * FW + f) * 16;
-    ob[f] = bfrag ? min(col, N - 16 - n0) * K * 2 + k0 * 4096 + h * 1024 + lane * 16
-                  : (min(n0 + col + (lane & 15), N - 1) - n0) * K * 2 + k0 * (2 * kBK) + h * 64 + 16 * (lane >> 4);
+    for (int f = 0; f < FW; ++f) ob[f] = min((g * FW + f) * 16, N - 16 - n0) * K * 2 + k0 * 4096 + h * 1024 + lane * 16;
+  } else {
+#pragma unroll
+    for (int q = 0; q < NG; ++q) ob[q] = (min(n0 + dma_row(q), N - 1) - n0) * K * 2 + dma_col(dma_row(q));
   }
-  const int bstep = bfrag ? 2048 : 128, bhalf = bfrag ? 1024 : 64;
-  bf16x8 br[DB][FW][KF];
+  bf16x8 br[FRAG ? DB : 1][FW][KF];
   // past the end the last step is read again (from L2): the count of loads stays what the code says
-  auto load_a = [&](int t, int slot) {
+  auto load_lds = [&](int t, int slot) {
     const int so = min(t, n - 1) * 128;
     char* d = smem + slot * PART + wid * 1024;
 #pragma unroll
     for (int q = 0; q < NA; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, GAI_LDS(d + q * 8192), 16, oa[q], so, 0, 0);
+    if constexpr (!FRAG)
+#pragma unroll
+      for (int q = 0; q < NG; ++q)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, GAI_LDS(d + BM * 128 + q * 8192), 16, ob[q], so, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto load_b = [&](int t, bf16x8(&d)[FW][KF]) {
-    const int so = min(t, n - 1) * bstep;
+    const int so = min(t, n - 1) * 2048;
 #pragma unroll
     for (int f = 0; f < FW; ++f)
 #pragma unroll
       for (int e = 0; e < KF; ++e)
-        d[f][e] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rb, ob[f], so + e * bhalf, 0));
+        d[f][e] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rb, ob[f], so + e * 1024, 0));
     __builtin_amdgcn_sched_barrier(0);
   };
   int a_rd[KF];  // + 2048 per 16 rows
@@ -138,17 +150,22 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
 
 #pragma unroll
   for (int d = 0; d < DB; ++d) {
-    load_a(d, d);
-    load_b(d, br[d]);
+    load_lds(d, d);
+    if constexpr (FRAG) load_b(d, br[d]);
   }
   int slot = 0, free = DB;
   auto step = [&](int t, bf16x8(&b)[FW][KF]) {
-    // A of this step is in LDS (younger: DB B steps and DB - 1 A steps) and everybody has left the slot before it
-    asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(DB * NB + (DB - 1) * NA) : "memory");
+    // this step's rows are in LDS and everybody has left the slot before it
+    asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(YOUNGER) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    load_a(t + DB, free);
+    load_lds(t + DB, free);
     const char* s = smem + slot * PART;
+    if constexpr (!FRAG)
+#pragma unroll
+      for (int f = 0; f < FW; ++f)
+#pragma unroll
+        for (int e = 0; e < KF; ++e) b[f][e] = *reinterpret_cast<const bf16x8*>(s + BM * 128 + a_rd[e] + (g * FW + f) * 2048);
 #pragma unroll
     for (int e = 0; e < KF; ++e) {
       bf16x8 af[MT];
@@ -161,18 +178,18 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
         for (int f = 0; f < FW; ++f) acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[f][e], af[i], acc[i][f], 0, 0, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    load_b(t + DB, b);
+    if constexpr (FRAG) load_b(t + DB, b);
     free = slot;
     slot = slot + 1 == RING ? 0 : slot + 1;
   };
   int t = 0;
   for (; t + DB <= n; t += DB)
 #pragma unroll
-    for (int u = 0; u < DB; ++u) step(t + u, br[u]);
+    for (int u = 0; u < DB; ++u) step(t + u, br[FRAG ? u : 0]);
   // the rest, outside the loop: an exit from its middle would join its back edge, and every load be waited for there
 #pragma unroll
   for (int u = 0; u < DB - 1; ++u)
-    if (t + u < n) step(t + u, br[u]);
+    if (t + u < n) step(t + u, br[FRAG ? u : 0]);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is left
   f32x4 v[NF];  // [RW][FW]
   if constexpr (ORD) {
@@ -368,20 +385,27 @@ bool mid_fits(const void* A, const void* B, const void* C, const void* bias, con
   return !(off(A, 16) || off(B, 16) || off(C, out_f32 ? 16 : 8) || off(bias, 8) || off(R, 8));
 }
 
-template <int MT, int NG, int EPI, bool OUTF32, bool ORD = false>
-void launch_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int S,
-                float* ws, int* cnt, hipStream_t st, int bfrag) {
-  constexpr int lds = std::max(MT * 2048 * mid_ring<MT>(), MT * NG * 4096);  // the ring; the exchange
+template <int MT, int NG, int EPI, bool OUTF32, bool ORD, bool FRAG>
+void launch_mid_order(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int S,
+                      float* ws, int* cnt, hipStream_t st) {
+  constexpr int lds = std::max(mid_step<MT, NG, FRAG>() * mid_ring<MT, NG, FRAG>(), MT * NG * 4096);  // the ring; the exchange
+  auto kern = gemm_mid_kernel<MT, NG, EPI, OUTF32, ORD, FRAG>;
   static bool once = false;
   if (!once) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mid_kernel<MT, NG, EPI, OUTF32, ORD>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       gai_launch_error(__FILE__, __LINE__, "gemm_mid: LDS size");
     once = true;
   }
-  gemm_mid_kernel<MT, NG, EPI, OUTF32, ORD><<<mid_tiles(M, N, MT, NG) * S, 512, lds, st>>>(
-      (const bf16*)A, (const bf16*)B, C, (const bf16*)bias, (const bf16*)R, M, N, K, ldc, bfrag, S, ws, cnt);
+  kern<<<mid_tiles(M, N, MT, NG) * S, 512, lds, st>>>((const bf16*)A, (const bf16*)B, C, (const bf16*)bias, (const bf16*)R, M, N, K,
+                                                      ldc, S, ws, cnt);
   GAI_LAUNCH_CHECK();
+}
+
+template <int MT, int NG, int EPI, bool OUTF32, bool ORD = false>
+void launch_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int S,
+                float* ws, int* cnt, hipStream_t st, int bfrag) {
+  if (bfrag) launch_mid_order<MT, NG, EPI, OUTF32, ORD, true>(A, B, C, bias, R, M, N, K, ldc, S, ws, cnt, st);
+  else launch_mid_order<MT, NG, EPI, OUTF32, ORD, false>(A, B, C, bias, R, M, N, K, ldc, S, ws, cnt, st);
 }
 
 }  // namespace
