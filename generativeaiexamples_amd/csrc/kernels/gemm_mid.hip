@@ -305,7 +305,8 @@ bool parts_fit(int M, int N, int mt, int ng, int S) {
 // 150 MB of parts 1536 x 11264 x 2048: 90 -> 258).
 struct MidFit {
   double base, round, alone, full;  // launch; of a round of workgroups; of a 128-deep K step, few workgroups / full chip
-  double weights, few, row_major;   // GB/s / 1000 of the weights, the share of it with few workgroups; a row-major step's factor
+  double weights, few, row_major;   // GB/s / 1000 of the weights, the share of it with few workgroups; the factor of a row-major step whose
+                                    // loads were in operand layout
   double part0, part1, parts;       // parts of K: once, each, GB/s / 1000 of the sums written and read
   double out, bias, gelu;           // GB/s / 1000 of residual and result; epilogues
 };
@@ -323,12 +324,13 @@ int epi_class(int epi) {
   return epi == EPI_NONE || epi_glu(epi) ? 0 : epi == EPI_BIAS_GELU || epi == EPI_BIAS_QUICKGELU ? 2 : 1;
 }
 
-double mid_cost(int M, int N, int K, int epi, int mt, int ng, int S, int bfrag) {
+// step: of a layout's K step against one of fragment order
+double mid_cost(int M, int N, int K, int epi, int mt, int ng, int S, double step) {
   const MidFit& f = kFit[mt == 12 ? 2 : ng - 1];
   const int items = mid_tiles(M, N, mt, ng) * S, steps = (K / kBK + S - 1) / S, G = mid_cus(), rounds = (items + G - 1) / G;
-  const double fill = std::min(1.0, (double)items / G), step = (f.alone + (f.full - f.alone) * fill) * (bfrag ? 1.0 : f.row_major);
+  const double fill = std::min(1.0, (double)items / G);
   const int ec = epi_class(epi);
-  return f.base + std::max(rounds * (f.round + steps * step), (double)N * K * 2 / 1e6 / (f.weights * (f.few + (1 - f.few) * fill))) +
+  return f.base + std::max(rounds * (f.round + steps * (f.alone + (f.full - f.alone) * fill) * step), (double)N * K * 2 / 1e6 / (f.weights * (f.few + (1 - f.few) * fill))) +
          out_mb(M, N, epi) / f.out + (ec == 1 ? f.bias : ec == 2 ? f.gelu : 0.0) +
          (S > 1 ? f.part0 + f.part1 * S + 2 * part_bytes(M, N, mt, ng, S) / 1e6 / f.parts + kTicketFill : 0.0);
 }
@@ -358,21 +360,29 @@ double other_cost(int M, int N, int K, int epi) {
 }
 // A weight gives the same bits in either layout: which kernel, and into how many parts, is one choice for both; only the tile
 // is the layout's own (a sum's order does not depend on it). The parts are those of the smaller row-major + 2 x fragment-order
-// time: the large weights, where parts matter most, are stored in fragment order.
+// time: the large weights, where parts matter most, are stored in fragment order. (The row-major times of that sum are of the
+// loads in operand layout: parts, and with them every bit, stay where they were.)
 constexpr double kFragShare = 2.0;
-// A product is taken where the model says 5 % less in fragment order and 3 % less row-major (up to 128 rows 20 %: 128 x 1024 x 1024
-// with bias, row-major, takes the skinny kernel 11.8 us and this one 12.7, where the model says 10.6). (The 256 x 256 kernels at K >= 8192
-// are up to a fifth faster than their model where the tiles divide the chip evenly.)
-// At K >= 8192 the row-major form need only come within 5 %: N 4096, K 14336 with a residual, 400 - 512 rows, takes 61 - 74 us in
-// fragment order here and 79 - 81 on the 256 x 256 kernel, which row-major weights pay for with 88 - 102 instead of 78 - 80.
+constexpr double kRowStep[3] = {1.14, 1.12, 1.1};  // a row-major step by DMA against one of fragment order: 128 x 64, 128, 192 x 128
+// A product is taken where the model says so much less time than the kernels it replaces take, in both layouts. Deep K leaves the model
+// of the 256 x 256 kernels up to a fifth too slow where the tiles divide the chip evenly. Of 1210 products in one layout (30 weights,
+// 22 numbers of rows from 65 to 2048), timed with every plan and on the other kernels, the chosen way is on average 2.6 % above the best;
+// with row-major steps at 1.47 - 1.7, and a row-major margin that made up for it at deep K, 3.6 %: 1536 rows 2048 x 2048, fragment
+// order, 31.7 us instead of 21.1, 128 rows of a gated 5632 x 2048 22.7 instead of 16.3. The margins up to 128 rows and past 1024
+// leave 128 x 1024 x 1024 with bias (11.2 us, 8.6 here) and 1536 rows of a gated 11264 x 2048 (94, 86) on the other kernels.
 double margin(int M, int K) { return M >= 256 && K >= 8192 ? 1.2 : 1.05; }
-double margin_row_major(int M, int K) { return M <= 128 ? 1.2 : M >= 256 && K >= 8192 ? 0.955 : 1.03; }
+double margin_row_major(int M, int K, bool glu) {
+  if (M <= 128) return glu ? 1.05 : 1.28;
+  return M >= 256 && K >= 8192 ? 1.27 : M <= 1024 ? 1.1 : 1.21;
+}
 
 // the ordered form, fitted to 600 timings of 150 products of up to 3072 rows (17 of 20 within 15 %)
 double ordered_cost(int M, int N, int K, int mt, int bfrag) {
   const int items = mid_tiles(M, N, mt, 2), G = mid_cus(), rounds = (items + G - 1) / G;
   const double fill = std::min(1.0, (double)items / G), step = mt == 4 ? 0.61 + 0.04 * fill : 0.81 + 0.12 * fill;
-  const double row = mt == 4 ? 1.68 : 1.42;  // row-major weights
+  // row-major weights, as with loads in operand layout: by DMA a step is 1.02 - 1.29 of one in fragment order, but with that the rows of
+  // 6000 x 4096 x 4096 were split too (164 -> 178 us)
+  const double row = mt == 4 ? 1.68 : 1.42;
   return (mt == 4 ? 2.4 : 2.3) + rounds * ((mt == 4 ? 1.55 : 3.0) + K / kBK * step * (bfrag ? 1.0 : row));
 }
 
@@ -425,15 +435,17 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
     double bc = 1e30, row = 1e30, frag = 1e30;
     for (int S = 1; S <= std::min(16, std::max(1, K / kBK / 4)); ++S) {
       GaiMidPlan at[2] = {{8, 2, S, 0, 1e30}, {8, 2, S, 0, 1e30}};  // row-major, fragment order: the best tile
+      double operand = 1e30;
       for (int v = glu ? 1 : 0; v < 3; ++v) {
         const int mt = v == 2 ? 12 : 8, ng = v == 0 ? 1 : 2;
         if (S > 1 && !parts_fit(M, N, mt, ng, S)) continue;
+        operand = std::min(operand, mid_cost(M, N, K, epi, mt, ng, S, kFit[v].row_major));
         for (int l = 0; l < 2; ++l) {
-          const double c = mid_cost(M, N, K, epi, mt, ng, S, l);
+          const double c = mid_cost(M, N, K, epi, mt, ng, S, l ? 1.0 : kRowStep[v]);
           if (c < at[l].cost) at[l] = {mt, ng, S, 0, c};
         }
       }
-      const double c = at[0].cost + kFragShare * at[1].cost;
+      const double c = operand + kFragShare * at[1].cost;
       if (c < bc) {
         bc = c;
         row = at[0].cost;
@@ -442,7 +454,7 @@ bool gai_gemm_mid_plan(const void* A, const void* B, const void* C, const void* 
       }
     }
     const double other = other_cost(M, N, K, epi);
-    if (force == 0 && (frag * margin(M, K) >= other || row * margin_row_major(M, K) >= other)) return false;
+    if (force == 0 && (frag * margin(M, K) >= other || row * margin_row_major(M, K, glu) >= other)) return false;
   }
   if (best.parts > 1 && !parts_fit(M, N, best.mt, best.ng, best.parts)) best.parts = 1;
   if (best.parts > 1) {

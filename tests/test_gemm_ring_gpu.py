@@ -236,6 +236,21 @@ def test_mid_gemm_choice(cuda, M, N, K, act, frag, mid):
     assert ops.native().gemm_mid_rows(x, w, out, b, res, ops.EPI[act], frag) == (M if mid else 0)
 
 
+@pytest.mark.parametrize("M,N,K,act,mid", [
+    (1536, 2048, 2048, None, True), (2048, 2048, 2048, None, True), (100, 5632, 2048, "swiglu", True), (128, 5632, 2048, "swiglu", True),
+    (400, 8192, 8192, "residual", True), (448, 4096, 14336, "residual", True), (768, 4096, 14336, "residual", True),
+    (1536, 4096, 14336, "residual", True), (150, 28672, 4096, "swiglu", True), (512, 6144, 4096, None, True),
+    (1024, 4096, 11008, "residual", False), (2048, 2048, 16384, None, False), (512, 14336, 4096, None, False)])
+@pytest.mark.parametrize("frag", [False, True])
+def test_mid_gemm_choice_near_the_line(cuda, M, N, K, act, mid, frag):
+    """Products that a margin or the row-major steps' share decide, timed on both kernels in both layouts: one choice for both,
+    and not the slower one in either."""
+    x, w = (torch.empty(n, K, device=cuda, dtype=torch.bfloat16) for n in (M, N))
+    out = torch.empty(M, N // 2 if act == "swiglu" else N, device=cuda, dtype=torch.bfloat16)
+    res = out if act == "residual" else None
+    assert ops.native().gemm_mid_rows(x, w, out, None, res, ops.EPI[act], frag) == (M if mid else 0)
+
+
 @pytest.mark.parametrize("plan", [8105, 8116, 8206, 12208, 0])  # 0: as chosen
 @pytest.mark.parametrize("M,N,K,act", [(65, 320, 4224, "bias_residual"), (193, 272, 2048, None), (187, 1024, 14336, "residual"),
                                        (413, 1056, 2176, "swiglu"), (1000, 1024, 1024, "gelu"), (2047, 272, 3072, "relu")])
