@@ -840,7 +840,9 @@ def _topk_lists(cap: int, nq: int, n_rows: int, D: int, aligned: bool = True) ->
 
 
 def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, k: int, ws=None):
-    """Top-k of Q @ X[:n_rows]^T + bias (exact). Returns (scores fp32 [nq,k], ids int64 [nq,k])."""
+    """Top-k of Q @ X[:n_rows]^T + bias (exact). Returns (scores fp32 [nq,k], ids int64 [nq,k]). Which of several rows of
+    equal score are returned, and in what order, depends on the form that answers, and so on k, the index and the number of
+    queries: the group form (_topk_lists False) returns the lowest rows first, the lists do not."""
     if k > 64:
         raise ValueError("sim_topk supports k <= 64")
     k_eff = min(k, n_rows)

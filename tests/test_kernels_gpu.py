@@ -619,6 +619,11 @@ def test_sim_topk_many_queries(cuda, nq, N, D, k):
         assert torch.equal(v, torch.cat([p[0] for p in parts])) and torch.equal(i, torch.cat([p[1] for p in parts]))
     else:     # the best k of the longer lists: the same scores (equal ones may swap rows)
         assert torch.equal(v, torch.cat([p[0] for p in parts])[:, :k])
+    if N > k:     # every query's rows are different ones, and have the scores that stand beside them
+        got = v.isfinite()
+        assert ((i[:, :, None] == i[:, None, :]) & got[:, :, None] & got[:, None, :]).sum() == got.sum()
+        own = torch.gather(Q.double() @ X.double().t() + bias.double(), 1, i.clamp_min(0))
+        assert ((v.double() - own).abs()[got] <= 1e-5 * D ** 0.5 * 8).all()
     s = Q.double() @ X.double().t() + bias.double()
     s[:, N // 2] = float("-inf")
     want = torch.topk(s.masked_fill(s.isnan(), float("-inf")), k, dim=-1)[0]

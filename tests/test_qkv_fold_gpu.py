@@ -78,6 +78,44 @@ def test_qkv_fold_matches_unfused_and_reference(cuda, B, Hq, Hkv, K, psw):
     assert err < 3e-2, err
 
 
+@pytest.mark.parametrize("Hq,Hkv,nsplit,ctx", [
+    (32, 8, 8, [1 + 32 * (i % 4) + 128 * (3 + 7 * i % 17) for i in range(48)]),   # drawn parts; the newest key first in a wave's chunk
+    (32, 8, 8, [1, 33, 65, 97, 128, 129, 32, 64, 96, 160, 1025, 2657] * 2),       # and ranked or all resident
+    (16, 1, 5, [31 + 37 * i for i in range(70)]), (8, 4, 4, [2000] * 66)])
+def test_qkv_fold_queue_equals_a_workgroup_per_part(cuda, Hq, Hkv, nsplit, ctx):
+    """The folded tail in the launch that hands parts out: the outputs, the caches with the new key and value in them, and the
+    tickets of the launch with a workgroup per part, eagerly and in graph replays."""
+    torch.manual_seed(len(ctx) + Hq)
+    D, B, ks = 128, len(ctx), 3
+    nb = max(ctx) // 16 + 2
+    part = torch.randn(ks, B, (Hq + 2 * Hkv) * D, device=cuda)
+    bt = torch.randperm(B * nb, device=cuda).to(torch.int32).view(B, nb)
+    c = torch.tensor(ctx, dtype=torch.int32, device=cuda)
+    pos = c - 1
+    slots = (bt.gather(1, (pos // 16).long().view(-1, 1)).view(-1) * 16 + pos % 16).to(torch.int32)
+    cs = ops.rope_cos_sin(4096, D, 500000.0).to(cuda)
+    kc0 = torch.randn(B * nb, Hkv, 16, D, device=cuda, dtype=torch.bfloat16)
+    vc0 = torch.randn(B * nb, Hkv, D, 16, device=cuda, dtype=torch.bfloat16)
+    ws, q = ops.DecodeWorkspace(B, Hq, D, 128 * max(nsplit, nb // 8 + 1), cuda), torch.empty(B, Hq, D, device=cuda, dtype=torch.bfloat16)
+    kc, vc, out = kc0.clone(), vc0.clone(), torch.full_like(q, 7.0)
+
+    def run(queue):
+        ops.native().attn_decode(q, kc, vc, bt, c, out, ws.o, ws.ml, D ** -0.5, 0, nsplit, 1.0, 1.0, ws.cnt, part, ks, pos, cs, slots,
+                                 queue)
+
+    run(False)
+    want = out.clone(), kc.clone(), vc.clone()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(g, stream=s):
+        run(True)
+    for i in range(6):
+        kc.copy_(kc0), vc.copy_(vc0), out.fill_(7.0)
+        run(True) if i % 2 else g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip((out, kc, vc), want)) and int(ws.cnt.abs().sum()) == 0
+
+
 def test_qkv_fold_in_graph_replay(cuda, monkeypatch):
     """The folded path in the engine, eager and inside captured multi-step decode graphs: every greedy token is the
     fp32 reference argmax of its prefix up to a bf16 near-tie."""
