@@ -7,7 +7,9 @@
 //    is waited for;
 //  * the activations go through LDS in two 64 KiB stages (LDS-DMA, 16-B chunks XOR-swizzled: conflict-free b128 reads),
 //    since fragments read straight from global memory (16 rows x 64 B a load) cost about 2 us per 64 KiB of them;
-//  * the waves' sums meet in LDS, in wave order, and the epilogue runs there: no fp32 partials, no second launch.
+//  * the waves' sums meet in LDS, in wave order, and the epilogue runs there: no fp32 partials, no second launch. (A product
+//    whose rows a layer norm takes next is the exception: K in slices, fp32 sums of which the norm's launch adds up,
+//    gai_gemm_slim_layernorm.)
 // MI355X, weights cold, row-major | fragment order, us, against split-K + reduce (two launches; the gap of about 1 us
 // between them not counted):
 //   M 32, N 3072, K 1024   5.3 | 4.9   was  10.4 |  8.3        M 32, N 2048, K 2048   7.4 | 6.6   was 10.5 |  8.4

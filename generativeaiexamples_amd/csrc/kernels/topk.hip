@@ -385,10 +385,12 @@ __global__ __launch_bounds__(256, 1) void sim_group_max(const bf16* __restrict__
 // The k groups with the largest maxima hold the k best rows: a row of another group has at least k rows before it, the
 // maxima of those groups. The same argument picks the groups: thread t's strided maximum over the group maxima, the k
 // best of those 1024 threads, and of their entries the k best. The rows of the k groups (<= 1024) are scored again with
-// the stream's own instruction order and sorted. Bound by the fetch of k x 32 KB of X at D = 1024 for every query (1.3 MB at k =
-// 40, through a CU's 32 KB of outstanding misses) and by latency: 250 KB of maxima at 1M rows, three 45-step selections across
-// lanes. Rows by DMA in whole lines instead of operand by operand: 300 queries of 250007 x 1024, k = 40 156 -> 119 us; of 5000 rows,
-// with the maxima, 124 -> 73.
+// the stream's own instruction order and sorted. 300 queries of 250007 rows, k = 40: 46 us at 64 columns, 56 at 256, 119 at 1024
+// (k = 10 60, k = 64 162; 1M rows 178). What the columns add is the fetch of k x 32 KB of X for every query, 1.3 MB and
+// for 44 of the CUs twice that, at the 60 KB/us of a CU alone 44 us of it; the 46 are the maxima and three selections, each 45
+// exchanges of 64-bit keys across lanes through LDS. Rows by DMA in whole lines instead of operand by operand: k = 40 156 -> 119 us; of
+// 5000 rows, with the maxima, 124 -> 73. One to 64 queries run it too, none slower for that form (1M x 1024, k = 40, with the
+// stream: 1 query 444 -> 430, 64 540 -> 519).
 // With at most k groups (an index, or a filter's rows, of 16 k rows) all are taken: no stream, one selection. 300 queries, 60
 // rows of 1024, k = 16: 20 us, 89 with the stream and with second groups read for nothing (lists 57); 200 rows, k = 8: 48, 61
 // (lists 55).

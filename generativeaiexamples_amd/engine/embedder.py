@@ -79,7 +79,7 @@ class Embedder:
             g = torch.cuda.CUDAGraph()
             with hip_graph_capture(g, s):
                 out = m.embed_padded(ids, lens, attn, B, L)
-            # the graph reads and writes attn's buffers (KV scratch, index tensors) by address: keep them alive
+            # the graph reads and writes attn's buffers (index tensors, pages where it has any) by address: keep them alive
             self._graphs[key] = (g, ids, lens, out, attn)
         return self._graphs[key]
 

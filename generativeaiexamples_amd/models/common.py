@@ -87,10 +87,11 @@ def quantize_linear_weights_fp8(w: dict, keys) -> int:
 class PackedAttention:
     """Self- (or cross-) attention over a packed varlen batch for encoders (BERT/E5, CLIP, ViT).
 
-    The paged flash-attention kernels read K/V from a paged cache, so an encoder forward allocates
-    one *transient* cache for the whole batch (sequence b owns blocks [off_b, off_b + ceil(n_b/16)));
-    every layer scatters its K/V into it with the RoPE/KV kernel (rotation off) and runs the
-    bidirectional (or causal) prefill kernel. All index tensors are built once per forward.
+    Self-attention without RoPE, bf16 heads of 64 with a kv head each: one kernel reads queries, keys and values straight
+    from the packed QKV rows. Anything else goes through the paged kernels: a *transient* cache for the whole batch
+    (sequence b owns blocks [off_b, off_b + ceil(n_b/16))), made when the first layer asks for it, into which every
+    layer packs its K/V (``pack``) or scatters them with the RoPE/KV kernel before the bidirectional (or causal) prefill
+    kernel. All index tensors are built once per forward.
     ``kv_lens`` (cross-attention) gives the key length per sequence when it differs from the query.
     """
 
