@@ -842,12 +842,14 @@ void gai_gdn_out(const float* o, const void* z, int ldz, const void* w, void* y,
                  hipStream_t st) {
   const int TH = T * Hv;
   if (TH == 0) return;
-  // few heads (decode steps): one a wave, or the chip stays empty
+  // One head a wave where few heads leave the chip empty, four where their loads in flight pay. us a launch, one | four a wave, heads
+  // of 128: 2048 heads 2.6 | 3.9, 10240 4.5 | 5.1, 16384 6.0 | 6.1, 32768 9.6 | 9.5, 65536 18.7 | 17.7, 192000 49.5 | 42.4; of 64:
+  // 8192 3.4 | 3.7, 16384 4.9 | 5.0, 32768 7.9 | 7.3.
 #define GAI_OUT(TA, NJ, R)                                                                                              \
   gdn_out_kernel<TA, NJ, R><<<(TH + 4 * R - 1) / (4 * R), 256, 0, st>>>(o, (const TA*)z, ldz, (const TA*)w, (TA*)y, TH, Hv, \
                                                                         DV, eps)
 #define GAI_OUT_N(TA)                                                                                                   \
-  if (DV <= 128) { if (TH > 8192) GAI_OUT(TA, 2, 4); else GAI_OUT(TA, 2, 1); }                                            \
+  if (DV <= 128) { if (TH > 16384) GAI_OUT(TA, 2, 4); else GAI_OUT(TA, 2, 1); }                                            \
   else if (DV <= 256) GAI_OUT(TA, 4, 1);                                                                                \
   else GAI_OUT(TA, 0, 1)
   if (dt) { GAI_OUT_N(float); } else { GAI_OUT_N(bf16); }

@@ -151,7 +151,7 @@ def test_gdn_rows_wider_than_their_tensors(cuda, Hv, dv, dt):
 @pytest.mark.parametrize("T,Hv,dv,dt", [(4097, 2, 128, torch.bfloat16), (2731, 3, 40, torch.float32), (3, 5, 129, torch.bfloat16),
                                         (9, 1, 256, torch.float32), (2, 3, 300, torch.bfloat16)])
 def test_gdn_out_widths(cuda, T, Hv, dv, dt):
-    """Several heads a wave with a remainder, one head a wave, heads wider than the registers hold: against torch with the
+    """One head a wave, with a remainder, heads wider than the registers hold: against torch with the
     same roundings (the order of up to 300 squares: one rounding of the type may fall the other way)."""
     torch.manual_seed(dv)
     o, w, z = torch.randn(T, Hv, dv, device=cuda), torch.randn(dv, device=cuda).to(dt), torch.randn(T, Hv * dv, device=cuda).to(dt)
@@ -160,6 +160,18 @@ def test_gdn_out_widths(cuda, T, Hv, dv, dt):
     want = (w * n).float() * torch.nn.functional.silu(z.float().view(T, Hv, dv))
     tol = 2.0 ** -7 if dt == torch.bfloat16 else 2.0 ** -20
     assert ((y.view(T, Hv, dv).float() - want).abs() <= tol * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("T,Hv,dv,dt", [(8193, 2, 128, torch.bfloat16), (5463, 3, 40, torch.float32), (16385, 1, 65, torch.bfloat16)])
+def test_gdn_out_many_heads_equal_few(cuda, T, Hv, dv, dt):
+    """More than 16384 heads run four a wave, with a remainder here: the bits of two calls of one head a wave, which
+    test_gdn_out_widths holds against torch."""
+    torch.manual_seed(T)
+    o, w, z = torch.randn(T, Hv, dv, device=cuda), torch.randn(dv, device=cuda).to(dt), torch.randn(T, Hv * dv, device=cuda).to(dt)
+    h = T // 2
+    assert h * Hv <= 16384 < T * Hv and (T - h) * Hv <= 16384 and T * Hv % 4
+    y = ops.gdn_out(o, z, w, 1e-6)
+    assert torch.equal(y, torch.cat([ops.gdn_out(o[:h], z[:h], w, 1e-6), ops.gdn_out(o[h:], z[h:], w, 1e-6)]))
 
 
 def test_gdn_prep_rows_do_not_depend_on_their_run(cuda):
