@@ -646,7 +646,8 @@ def _decode_queue(B: int, Hkv: int, nsplit: int) -> bool:
     few kv heads, as a tensor-parallel rank has, there are many sequences to rank, and the launch with a workgroup per part is
     the faster one (8 / 1 heads, 80 sequences of 2600 - 2700 keys 35.8 us a launch, 41.6 with queues; 16 / 2, 80 of 30 - 100 7.8
     and 10.0) unless the number of parts is a multiple of eight: there a part's number chooses its XCD, and short contexts leave most of
-    them idle (16 / 2, 64 of 30 - 100 13.4 and 7.1, of 500 - 3000 39.8 and 35.7)."""
+    them idle (16 / 2, 64 of 30 - 100 13.4 and 7.1, of 500 - 3000 39.8 and 35.7). Heads of 128 alone have
+    the queues: they were measured for no other width, and those keep a workgroup per part."""
     return (nsplit > 1 and B <= 256 and B * Hkv * nsplit > 512 and B * nsplit < 1 << 22
             and (Hkv >= 4 or (nsplit % 8 == 0 and B <= 128)))
 
