@@ -466,9 +466,9 @@ void token_mask(Tensor& logits, const Tensor& rows, const Tensor& mask) {
                  reinterpret_cast<const uint32_t*>(mask.data_ptr<int>()), W, cur_stream());
 }
 
-// ws_i none: the group form, ws_v holds a maximum per query and 16 rows; else both hold a list per query and row range
+// ws_i none: the group form, ws_v holds a maximum per query and group_rows rows; else both hold a list per query and row range
 void sim_topk(const Tensor& Q, const Tensor& X, const Tensor& bias, int64_t n_rows, int64_t k, Tensor& ws_v,
-              const optional<Tensor>& ws_i, int64_t nwg, int64_t rows_per_wg, Tensor& out_v, Tensor& out_i) {
+              const optional<Tensor>& ws_i, int64_t nwg, int64_t rows_per_wg, Tensor& out_v, Tensor& out_i, int64_t group_rows) {
   check_bf16(Q, "Q");
   check_bf16(X, "X");
   check_f32(bias, "bias");
@@ -480,14 +480,15 @@ void sim_topk(const Tensor& Q, const Tensor& X, const Tensor& bias, int64_t n_ro
   TORCH_CHECK(X.size(1) == D, "sim_topk: dim mismatch");
   TORCH_CHECK(n_rows <= X.size(0) && n_rows <= bias.numel(), "sim_topk: n_rows exceeds storage");
   TORCH_CHECK(rows_per_wg % 128 == 0, "sim_topk: rows_per_wg must be a multiple of 128");
+  TORCH_CHECK(group_rows == 4 || group_rows == 16, "sim_topk: groups of 4 or 16 rows");
   const int cap = gai_topk_cap(k);
   TORCH_CHECK(n_rows >= 1 && k >= 1 && k <= 64 && nwg * rows_per_wg >= n_rows, "sim_topk: rows or k out of range");
   TORCH_CHECK(out_v.numel() >= nq * k && out_i.numel() >= nq * k && out_i.scalar_type() == at::kLong, "sim_topk: outputs");
   TORCH_CHECK(ws_i ? cap <= 8 && ws_v.numel() >= nwg * nq * cap && ws_i->numel() >= nwg * nq * cap
-                   : ws_v.numel() >= nq * ((n_rows + 15) / 16),
+                   : ws_v.numel() >= (int64_t)nq * gai_topk_places(group_rows, n_rows),
               "sim_topk: workspace too small");
   gai_sim_topk(Q.data_ptr(), X.data_ptr(), bias.data_ptr<float>(), nq, n_rows, D, k, ws_v.data_ptr<float>(),
-               ws_i ? ws_i->data_ptr<int>() : nullptr, nwg, rows_per_wg, out_v.data_ptr<float>(), out_i.data_ptr<int64_t>(),
+               ws_i ? ws_i->data_ptr<int>() : nullptr, nwg, rows_per_wg, group_rows, out_v.data_ptr<float>(), out_i.data_ptr<int64_t>(),
                cur_stream());
 }
 
@@ -1139,7 +1140,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tp_stats", &sample_tp_stats);
   m.def("apply_penalties", &apply_penalties);
   m.def("token_mask", &token_mask);
-  m.def("sim_topk", &sim_topk);
+  m.def("sim_topk", &sim_topk, py::arg("Q"), py::arg("X"), py::arg("bias"), py::arg("n_rows"), py::arg("k"), py::arg("ws_v"),
+        py::arg("ws_i"), py::arg("nwg"), py::arg("rows_per_wg"), py::arg("out_v"), py::arg("out_i"), py::arg("group_rows") = 16);
   m.def("topk_merge", [](const Tensor& vals, const Tensor& idx, int64_t k, Tensor& out_v, Tensor& out_i) {
     check_f32(vals, "vals");
     check_i32(idx, "idx");

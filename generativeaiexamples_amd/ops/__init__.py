@@ -840,6 +840,16 @@ def _topk_lists(cap: int, nq: int, n_rows: int, D: int, aligned: bool = True) ->
             or (nq <= 128 and n_rows >= 1 << 19 and D < 1024 and D % 128 == 0))
 
 
+def _topk_group_rows(nq: int, n_rows: int, D: int, k: int) -> int:
+    """Rows of a group of the group form, 16 or 4: what a query fetches again is k groups, what it reads first a maximum per group.
+    Groups of 4 where that fetch is long (k x D; us 16 / 4, 250007 x 1024, 300 queries: k = 10 228 / 232, 20 243 / 238, 40 285 / 250) and
+    the index is not much longer; the stream of up to 64 queries also pays for four times the stores (250007 x 1024: 1 query,
+    k = 40 121 / 114, 64 queries, k = 20 120 / 126; 1M, 1, k = 40 386 / 392). The maxima of all queries are held at once."""
+    if k * D < 16384 or n_rows <= 16 * k or n_rows > (16384 if nq > 64 else 8192) * k:
+        return 16
+    return 4 if nq * ((n_rows + 31) // 32 * 8) <= _TOPK_MAXIMA else 16
+
+
 def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, k: int, ws=None):
     """Top-k of Q @ X[:n_rows]^T + bias (exact). Returns (scores fp32 [nq,k], ids int64 [nq,k]). Which of several rows of
     equal score are returned, and in what order, depends on the form that answers, and so on k, the index and the number of
@@ -860,6 +870,14 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
     out_i = torch.empty(nq, k_eff, dtype=torch.int64, device=Q.device)
     Q, cap = Q.contiguous(), topk_cap(k_eff)
     lists = _topk_lists(cap, nq, n_rows, D, not (Q.data_ptr() | X.data_ptr()) & 15)
+    if not lists and _topk_group_rows(nq, n_rows, D, k_eff) == 4:
+        try:
+            ws_v = torch.empty(nq * ((n_rows + 31) // 32 * 8), dtype=torch.float32, device=Q.device)
+        except torch.OutOfMemoryError:
+            pass  # (maxima of 16 rows are a quarter of that)
+        else:
+            native().sim_topk(Q, X, bias, n_rows, k_eff, ws_v, None, nwg, rows_per_wg, out_v, out_i, 4)
+            return out_v, out_i
     step = _topk_slice(nq, n_rows)
     if not lists:
         try:

@@ -632,6 +632,46 @@ def test_sim_topk_many_queries(cuda, nq, N, D, k):
     assert torch.equal(v.isfinite(), fin)
 
 
+@pytest.mark.parametrize("nq,N,D,k,off", [
+    (1, 33, 64, 2, 0), (3, 641, 192, 40, 0), (2, 1025, 96, 64, 0), (17, 4100, 320, 9, 0), (5, 70_001, 64, 64, 0), (40, 12_345, 1024, 17, 4),
+    (64, 262_165, 32, 33, 0), (65, 100, 256, 6, 0), (70, 20_003, 320, 40, 0), (130, 5_021, 384, 64, 0), (200, 9_999, 448, 12, 2),
+    (300, 40_007, 256, 50, 0)])
+def test_sim_topk_groups_of_four(cuda, monkeypatch, nq, N, D, k, off):
+    """Maxima of 4 rows give the lists of maxima of 16 rows, bit for bit, in either first pass and with rows off 16 bytes: whole
+    numbers with many equal scores (lowest rows first), then random rows with deleted, infinite and NaN ones among them."""
+    g = torch.Generator(device=cuda).manual_seed(N)
+    for whole in (True, False):
+        make = (lambda *s: torch.randint(-2, 3, s, device=cuda, generator=g)) if whole else (
+            lambda *s: torch.randn(*s, device=cuda, generator=g))
+        base = make(N * D + off).bfloat16()
+        X, Q = base[off:].view(N, D), make(nq, D).bfloat16()
+        bias = torch.zeros(N, device=cuda)
+        bias[::7] = float("-inf")
+        if not whole:
+            X[N // 2], X[N // 3, 0] = float("nan"), float("inf")
+            bias[N - 1] = 50.0
+        got = []
+        for rows in (16, 4):
+            monkeypatch.setattr(ops, "_topk_group_rows", lambda *a, r=rows: r)
+            monkeypatch.setattr(ops, "_topk_lists", lambda *a: False)
+            got.append(ops.sim_topk(Q, X, bias, N, k))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+        if whole:
+            vr, ir = torch.sort(Q.float() @ X.float().t() + bias, dim=-1, descending=True, stable=True)
+            vr, ir = vr[:, :k], ir[:, :k]
+            assert torch.equal(got[1][0], vr)
+            assert torch.equal(got[1][1], torch.where(vr == float("-inf"), torch.full_like(ir, -1), ir))
+
+
+def test_sim_topk_group_rows():
+    """Which groups, on either side of each line of the rule."""
+    rows = ops._topk_group_rows
+    assert rows(300, 250_007, 1024, 40) == 4 and rows(300, 250_007, 1024, 10) == 16      # long fetch
+    assert rows(300, 640, 1024, 40) == 16 and rows(300, 641, 1024, 40) == 4              # every group is taken
+    assert rows(65, 16384 * 16, 1024, 16) == 4 and rows(64, 16384 * 16, 1024, 16) == 16  # the stream's stores
+    assert rows(300, 250_000, 1024, 40) == 4 and rows(1100, 250_000, 1024, 40) == 16     # all maxima at once
+
+
 @pytest.mark.parametrize("nq,D,k", [(3, 64, 10), (70, 256, 10), (70, 256, 4), (2, 1024, 40)])
 @pytest.mark.parametrize("off", [2, 4])
 def test_sim_topk_rows_off_16_bytes(cuda, nq, D, k, off):
