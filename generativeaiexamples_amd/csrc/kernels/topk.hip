@@ -275,14 +275,16 @@ __global__ __launch_bounds__(512) void sim_topk_stream(const bf16* __restrict__ 
 // Group maxima for many queries: a product with both operands staged in LDS. The stream above reads X again for every 64 queries, in
 // its operand layout (16 rows x 64 B a load: 37 KB/us in a CU, a quarter of what whole lines get), and a query fragment from LDS
 // for every MFMA. Here:
-//  * a workgroup takes 128 rows x 16 * QT queries (up to 320, so X is read once), waves 64 rows x half of the queries: 4 + QT / 2
-//    fragment reads for 2 * QT MFMAs of a 32-deep K step;
-//  * X and Q come by DMA, RING - 1 steps ahead and on into the workgroup's next tile of rows, the loads spread between the MFMAs;
-//    the next step's fragments are read meanwhile (one wave per SIMD, two register sets);
+//  * a workgroup takes 32 * RF rows x 16 * QT queries (up to 320, so X is read once), waves half of the rows x half of the queries:
+//    RF + QT / 2 fragment reads for RF * QT / 2 MFMAs of a 32-deep K step;
+//  * X and Q come by DMA, RING - 2 steps ahead and on into the workgroup's next tile of rows, the loads spread between the MFMAs; the
+//    next step's rows are read meanwhile, query fragments three ahead (one wave per SIMD);
 //  * every output is one sum over K in order, the same bits as the stream's and the second pass's;
-//  * a group's maximum: of the four row tiles of a lane the transposed lane halves leave group 4w + (lane >> 4) in place.
-// 300 queries x 250007 rows x 1024: 370 -> 195 us (the matrix work alone 105; a CU's 32 KB of outstanding misses, shared by 8 KB of X
-// from HBM and 20 KB of Q from L2 a step, allow about 120).
+//  * maxima of 4 rows are stored as the lanes hold them; of 16: of the four row tiles of a lane the transposed lane halves leave group
+//    4w + (lane >> 4) in place.
+// 300 queries x 250007 rows x 1024: 370 -> 189 us with tiles of 128 rows. The matrix work alone is 105 and everything but the loads 119;
+// the loads alone take 178: 28 KB a step at 40 KB/us a CU, 8 of X from HBM and 20 of Q from L2 that share 32 KB of outstanding misses
+// (whole lines instead of 16 rows x 64 B a load: 200). Taller tiles load less Q for the same rows, see group_max.
 // ------------------------------------------------------------------------------------------------
 template <int QT, int RF>
 constexpr int tile_ring() { return 158 / (2 * RF + QT) < 8 ? 158 / (2 * RF + QT) : 8; }
@@ -827,13 +829,20 @@ void run_select_r(const TopkArgs& a) {
 }
 void run_select(const TopkArgs& a) { a.gr == 4 ? run_select_r<4>(a) : run_select_r<16>(a); }
 
+// Rows of a tile: 128, or more where the last round of tiles over the 256 CUs does not cost what that saves. A tile of 192 rows x 320
+// queries takes 1.34 times one of 128 (1M x 1024, 300 queries, k = 4: 815 -> 745 us; 170000, k = 40: 185 -> 173; but 200000 in 5 rounds
+// for 7: 209 -> 206, 120000 x 768 in 3 for 4: 89 -> 93), one of 256 x 192 or 256 queries 1.77 times (250007 x 1024, 192 queries:
+// 165 -> 150, 256: 191 -> 174; 70000, 250 queries, 2 rounds for 3: 66.7 -> 72.1). 256 rows x 320 queries do not fit the registers;
+// up to 128 queries X bounds both.
 template <int GR>
 void group_max(const TopkArgs& a) {
   const int qblocks = (a.nq + 319) / 320, qt = ((a.nq + qblocks - 1) / qblocks + 63) / 64 * 4;
+  auto rounds = [&](int rows) { return ((a.N + rows - 1) / rows * qblocks + 255) / 256; };
+  const bool by192 = rounds(192) * 136 < rounds(128) * 100, by256 = rounds(256) * 178 < rounds(128) * 100;
   if (qt <= 8) run_group_max<8, 4, GR>(a, qblocks);
-  else if (qt <= 12) run_group_max<12, 4, GR>(a, qblocks);
-  else if (qt <= 16) run_group_max<16, 4, GR>(a, qblocks);
-  else run_group_max<20, 4, GR>(a, qblocks);
+  else if (qt <= 12) by256 ? run_group_max<12, 8, GR>(a, qblocks) : run_group_max<12, 4, GR>(a, qblocks);
+  else if (qt <= 16) by256 ? run_group_max<16, 8, GR>(a, qblocks) : run_group_max<16, 4, GR>(a, qblocks);
+  else by192 ? run_group_max<20, 6, GR>(a, qblocks) : run_group_max<20, 4, GR>(a, qblocks);
 }
 
 bool many_queries(const TopkArgs& a) {

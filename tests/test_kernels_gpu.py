@@ -663,6 +663,24 @@ def test_sim_topk_groups_of_four(cuda, monkeypatch, nq, N, D, k, off):
             assert torch.equal(got[1][1], torch.where(vr == float("-inf"), torch.full_like(ir, -1), ir))
 
 
+@pytest.mark.parametrize("nq,N,D,k", [(300, 33_001, 256, 5), (257, 49_152, 320, 40), (319, 33_000, 1024, 9), (190, 33_001, 256, 12),
+                                      (256, 65_535, 320, 64), (193, 40_000, 768, 20)])
+def test_sim_topk_tall_tiles(cuda, nq, N, D, k):
+    """Tiles of 192 and of 256 rows (a round of them over the chip where two of 128 rows would go): the lists of the same queries 64 at
+    a time, bit for bit, partial tiles of rows and queries, deleted and NaN rows among them."""
+    g = torch.Generator(device=cuda).manual_seed(nq)
+    X = torch.randn(N, D, device=cuda, generator=g).to(torch.bfloat16)
+    Q = torch.randn(nq, D, device=cuda, generator=g).to(torch.bfloat16)
+    bias = torch.randn(N, device=cuda, generator=g)
+    bias[::7] = float("-inf")
+    bias[N - 1] = 5.0 * D ** 0.5
+    X[N // 2] = float("nan")
+    v, i = ops.sim_topk(Q, X, bias, N, k)
+    parts = [ops.sim_topk(Q[s:s + 64], X, bias, N, max(k, 9)) for s in range(0, nq, 64)]
+    assert torch.equal(v, torch.cat([p[0] for p in parts])[:, :k])
+    assert torch.equal(i, torch.cat([p[1] for p in parts])[:, :k])
+
+
 def test_sim_topk_group_rows():
     """Which groups, on either side of each line of the rule."""
     rows = ops._topk_group_rows
