@@ -492,6 +492,14 @@ void sim_topk(const Tensor& Q, const Tensor& X, const Tensor& bias, int64_t n_ro
                cur_stream());
 }
 
+void l2_relevance(const Tensor& q, const Tensor& s, Tensor& out) {
+  check_f32(q, "q");
+  check_f32(s, "s");
+  check_f32(out, "out");
+  TORCH_CHECK(q.dim() == 2 && s.dim() == 2 && s.size(0) == q.size(0) && out.sizes() == s.sizes(), "l2_relevance: shapes");
+  gai_l2_relevance(q.data_ptr<float>(), s.data_ptr<float>(), q.size(0), q.size(1), s.size(1), out.data_ptr<float>(), cur_stream());
+}
+
 void moe_route(const Tensor& logits, int64_t k, bool renorm, Tensor& ids, Tensor& w, bool sigmoid,
                const optional<Tensor>& bias, double eps) {
   TORCH_CHECK(logits.is_cuda() && logits.scalar_type() == at::kFloat && logits.dim() == 2 &&
@@ -1140,6 +1148,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tp_stats", &sample_tp_stats);
   m.def("apply_penalties", &apply_penalties);
   m.def("token_mask", &token_mask);
+  m.def("l2_relevance", &l2_relevance);
   m.def("sim_topk", &sim_topk, py::arg("Q"), py::arg("X"), py::arg("bias"), py::arg("n_rows"), py::arg("k"), py::arg("ws_v"),
         py::arg("ws_i"), py::arg("nwg"), py::arg("rows_per_wg"), py::arg("out_v"), py::arg("out_i"), py::arg("group_rows") = 16);
   m.def("topk_merge", [](const Tensor& vals, const Tensor& idx, int64_t k, Tensor& out_v, Tensor& out_i) {

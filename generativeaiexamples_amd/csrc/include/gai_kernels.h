@@ -113,6 +113,7 @@ void gai_apply_penalties(float* logits, int B, long ld, const int* tok_ids, cons
 
 // topk.hip
 int gai_topk_cap(int k);
+void gai_l2_relevance(const float* q, const float* s, int nq, int D, int k, float* out, hipStream_t st);
 int gai_topk_places(int group_rows, int N);  // group maxima of a query
 // Streaming-SDR DSP (dsp.hip): complex64 FIR with zero initial state, FM discriminator, polyphase rational resampler
 void gai_dsp_fir_complex(const void* x, const float* taps, int n, int ntaps, void* y, hipStream_t st);

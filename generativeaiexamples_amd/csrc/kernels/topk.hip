@@ -895,6 +895,23 @@ void run_topk_k(const TopkArgs& a) {
   run_stream<1, K>(a);
 }
 
+// Relevance of euclidean search, 1 - sqrt(max(|q|^2 - 2 s, 0)) / sqrt(2) of the scores s = q . x - |x|^2 / 2: a wave a query, its row in
+// one pass. Bound by its launch (300 queries x 1024, k = 40: 1.2 MB); as torch operations it was eight launches, 20 us.
+__global__ __launch_bounds__(64) void l2_relevance_kernel(const float* __restrict__ q, const float* __restrict__ s, int D, int k,
+                                                          float* __restrict__ out) {
+  const int lane = threadIdx.x;
+  const float* row = q + (size_t)blockIdx.x * D;
+  float sum = 0.f;
+#pragma unroll 4
+  for (int i = lane; i < D; i += 64) sum += row[i] * row[i];
+  const float qq = wave_sum(sum);
+  for (int j = lane; j < k; j += 64) {
+    float d2 = qq - 2.f * s[(size_t)blockIdx.x * k + j];
+    d2 = d2 < 0.f ? 0.f : d2;  // (NaN stays)
+    out[(size_t)blockIdx.x * k + j] = 1.f - sqrtf(d2) / 1.41421356f;
+  }
+}
+
 }  // namespace
 
 // Cross-list merge (the sharded index's W shard lists per query): stage 2 alone over ws [nlists][nq][cap].
@@ -915,6 +932,12 @@ void gai_topk_merge(const float* vals, const int* idx, int nlists, int nq, int c
 int gai_topk_places(int group_rows, int N) { return places(group_rows, N); }
 
 int gai_topk_cap(int k) { return k <= 4 ? 4 : k <= 8 ? 8 : k <= 16 ? 16 : k <= 32 ? 32 : 64; }
+
+void gai_l2_relevance(const float* q, const float* s, int nq, int D, int k, float* out, hipStream_t st) {
+  if (nq == 0 || k == 0) return;
+  l2_relevance_kernel<<<nq, 64, 0, st>>>(q, s, D, k, out);
+  GAI_LAUNCH_CHECK();
+}
 
 void gai_sim_topk(const void* Q, const void* X, const float* bias, int nq, int N, int D, int k, float* ws_v,
                   int* ws_i, int nwg, int rows_per_wg, int group_rows, float* out_v, int64_t* out_i, hipStream_t st) {

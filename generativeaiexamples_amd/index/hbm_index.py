@@ -221,9 +221,7 @@ class HBMIndex:
     # ------------------------------------------------------------------ query
     def _relevance(self, raw: torch.Tensor, q: torch.Tensor) -> torch.Tensor:
         if self.metric == "l2":
-            # raw = q.x - |x|^2/2  ->  d^2 = |q|^2 - 2 raw
-            d2 = (q.float().pow(2).sum(-1, keepdim=True) - 2 * raw).clamp_min(0)
-            return 1.0 - d2.sqrt() / math.sqrt(2.0)
+            return ops.l2_relevance(q, raw)
         return raw
 
     def search_raw(self, queries: torch.Tensor, k: int):

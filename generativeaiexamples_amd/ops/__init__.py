@@ -897,6 +897,16 @@ def sim_topk(Q: torch.Tensor, X: torch.Tensor, bias: torch.Tensor, n_rows: int, 
     return out_v, out_i
 
 
+def l2_relevance(q: torch.Tensor, raw: torch.Tensor) -> torch.Tensor:
+    """Scores q . x - |x|^2 / 2 of euclidean search, fp32 [nq, k], and the fp32 queries [nq, D] -> 1 - |q - x| / sqrt(2)."""
+    if not q.is_cuda or (torch.is_grad_enabled() and (q.requires_grad or raw.requires_grad)):
+        return ref.l2_relevance(q, raw)
+    q, raw = q.float().contiguous(), raw.float().contiguous()
+    out = torch.empty_like(raw)
+    native().l2_relevance(q, raw, out)
+    return out
+
+
 def topk_merge(vals: torch.Tensor, k: int):
     """Merge W descending-sorted candidate lists per query: vals [W, Q, n] fp32 -> (top values [Q, k], positions
     [Q, k] int64 into the flattened [W * n] candidates of the query, w * n + j). On the GPU: the similarity top-k's

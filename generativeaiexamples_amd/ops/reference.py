@@ -256,6 +256,11 @@ def apply_penalties(logits, tok_ids, tok_cnt, n, freq, pres, rep):
     return logits
 
 
+def l2_relevance(q, raw):
+    d2 = (q.float().pow(2).sum(-1, keepdim=True) - 2 * raw).clamp_min(0)
+    return 1.0 - d2.sqrt() / math.sqrt(2.0)
+
+
 def sim_topk(Q, X, bias, n_rows, k):
     s = Q.float() @ X[:n_rows].float().t() + bias[:n_rows].float()
     k = min(k, n_rows)

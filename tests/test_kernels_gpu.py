@@ -681,6 +681,29 @@ def test_sim_topk_tall_tiles(cuda, nq, N, D, k):
     assert torch.equal(i, torch.cat([p[1] for p in parts])[:, :k])
 
 
+@pytest.mark.parametrize("nq,D,k", [(1, 32, 1), (3, 100, 4), (70, 1024, 64), (300, 384, 65), (2, 8, 130), (4, 64, 0), (0, 64, 4)])
+def test_l2_relevance(cuda, nq, D, k):
+    """1 - |q - x| / sqrt(2) from the scores, against 64 bits: the kernel rounds |q|^2 at most D / 64 + 6 times on the way to a sum, so
+    d^2 is off by e <= (D / 64 + 8) 2^-24 |q|^2 + 2^-22 |score| and the distance by at most min(e / d, sqrt(e)). Rows at the query itself,
+    absent rows (-inf), NaN and strided queries among them."""
+    g = torch.Generator(device=cuda).manual_seed(nq + D)
+    q = torch.randn(nq, 2 * D, device=cuda, generator=g)[:, ::2]
+    raw = torch.randn(nq, k, device=cuda, generator=g) - 0.3 * D
+    if nq and k:
+        raw[0, 0] = 0.5 * q[0].square().sum()
+        raw[nq - 1, k - 1] = float("-inf")
+        raw[nq // 2, k // 2] = float("nan")
+    got = ops.l2_relevance(q, raw)
+    qq = q.double().square().sum(-1, keepdim=True)
+    d2 = (qq - 2 * raw.double()).clamp_min(0)
+    want = 1 - d2.sqrt() / 2 ** 0.5
+    e = (D / 64 + 8) * 2.0 ** -24 * qq + 2.0 ** -22 * raw.double().abs()
+    tol = torch.minimum(e / d2.sqrt(), e.sqrt()) + 2.0 ** -22 * (1 + d2.sqrt())
+    fin = want.isfinite()
+    assert got.shape == (nq, k) and ((got.double() - want).abs() <= tol)[fin].all()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+
+
 def test_sim_topk_group_rows():
     """Which groups, on either side of each line of the rule."""
     rows = ops._topk_group_rows
