@@ -73,6 +73,24 @@ void layernorm(const Tensor& x, const Tensor& w, const optional<Tensor>& b, doub
                 opt_ptr(b), out.data_ptr(), T, D, (float)eps, cur_stream());
 }
 
+void embed_layernorm(const Tensor& ids, const Tensor& pos, const Tensor& word, const Tensor& ptab, const Tensor& type, const Tensor& w,
+                     const Tensor& b, double eps, Tensor& out) {
+  check_i32(ids, "ids");
+  check_i32(pos, "positions");
+  check_bf16(word, "word");
+  check_bf16(ptab, "position table");
+  check_bf16(type, "type row");
+  check_bf16(w, "w");
+  check_bf16(b, "b");
+  check_bf16(out, "out");
+  const int T = ids.numel(), D = word.size(1);
+  TORCH_CHECK(D % 8 == 0 && D <= 2048 && ptab.size(1) == D && type.numel() == D && w.numel() == D && b.numel() == D,
+              "embed_layernorm: bad hidden size");
+  TORCH_CHECK(pos.numel() == T && out.numel() == (int64_t)T * D, "embed_layernorm: a position and a row per id");
+  gai_embed_layernorm(ids.data_ptr<int>(), pos.data_ptr<int>(), word.data_ptr(), ptab.data_ptr(), type.data_ptr(), w.data_ptr(),
+                      b.data_ptr(), out.data_ptr(), T, D, word.size(0), (float)eps, cur_stream());
+}
+
 // the product's own launches, then the norm that sums its slabs (shapes with gemm_slim_ks > 0)
 void linear_layernorm(const Tensor& A, const Tensor& W, const optional<Tensor>& bias, const Tensor& R, const Tensor& g,
                       const optional<Tensor>& b, double eps, Tensor& out, Tensor& ws, bool psw) {
@@ -791,11 +809,15 @@ void decode_advance(const Tensor& toks, Tensor& ids, Tensor& pos, Tensor& ctx, T
                      cur_stream());
 }
 
-void pool(const Tensor& h, const Tensor& cu, Tensor& out, int64_t mode, bool normalize) {
+void pool(const Tensor& h, const Tensor& cu, Tensor& out, int64_t mode, bool normalize, const optional<Tensor>& lens) {
   check_bf16(h, "hidden");
   check_i32(cu, "cu_seqlens");
   check_f32(out, "out");
-  gai_pool(h.data_ptr(), cu.data_ptr<int>(), out.data_ptr<float>(), h.numel() / std::max<int64_t>(h.size(-1), 1),
+  if (lens) {
+    check_i32(*lens, "lens");
+    TORCH_CHECK(lens->numel() == cu.numel() - 1, "pool: one length a sequence");
+  }
+  gai_pool(h.data_ptr(), cu.data_ptr<int>(), lens ? lens->data_ptr<int>() : nullptr, out.data_ptr<float>(), h.numel() / std::max<int64_t>(h.size(-1), 1),
            cu.numel() - 1, h.size(-1), mode, normalize ? 1 : 0, cur_stream());
 }
 
@@ -1108,6 +1130,7 @@ void gai_bind_seq_ops(pybind11::module_& m);  // seq_ops.cpp
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "gfx950 (MI355X) HIP kernels for generativeaiexamples_amd";
   m.def("rmsnorm", &rmsnorm);
+  m.def("embed_layernorm", &embed_layernorm);
   m.def("layernorm", &layernorm);
   m.def("rope_kv_write", &rope_kv_write);
   m.def("gemm_mid_rows", &gemm_mid_rows);
@@ -1217,7 +1240,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("Hkv"), pybind11::arg("frag") = false);
   m.def("embedding", &embedding);
   m.def("decode_advance", &decode_advance);
-  m.def("pool", &pool);
+  m.def("pool", &pool, py::arg("h"), py::arg("cu"), py::arg("out"), py::arg("mode"), py::arg("normalize"),
+        py::arg("lens") = py::none());
   m.def("silu_mul", &silu_mul);
   m.def("gelu", &gelu);
   m.def("gelu_tanh", &gelu_tanh);

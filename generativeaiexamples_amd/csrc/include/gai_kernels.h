@@ -9,6 +9,8 @@ void gai_launch_error(const char* file, int line, const char* msg);
 // norm.hip
 void gai_rmsnorm(const void* x, const void* residual_in, void* residual_out, const void* w, void* out, int T, int D,
                  float eps, hipStream_t st);
+void gai_embed_layernorm(const int* ids, const int* pos, const void* word, const void* ptab, const void* type, const void* w,
+                         const void* b, void* out, int T, int D, int vocab, float eps, hipStream_t st);
 void gai_layernorm(const void* x, const void* residual_in, void* residual_out, const void* w, const void* b,
                    void* out, int T, int D, float eps, hipStream_t st);
 
@@ -168,7 +170,7 @@ void gai_moe_scale_rows(const void* h, const int* pos, const float* w, void* out
 
 // misc.hip
 void gai_embedding(const int* ids, const void* table, void* out, int T, int D, int vstart, int vend, hipStream_t st);
-void gai_pool(const void* h, const int* cu, float* out, int T, int B, int D, int mode, int normalize, hipStream_t st);
+void gai_pool(const void* h, const int* cu, const int* lens, float* out, int T, int B, int D, int mode, int normalize, hipStream_t st);
 void gai_silu_mul(const void* x, void* y, int T, int I, hipStream_t st);
 void gai_gelu(const void* x, void* y, int T, int I, hipStream_t st);
 void gai_gelu_tanh(const void* x, void* y, int T, int I, hipStream_t st);

@@ -22,17 +22,18 @@ __global__ __launch_bounds__(256) void embedding_kernel(const int* __restrict__ 
 }
 
 // Pool each sequence of hidden [T, D] (varlen via cu_seqlens) into out [B, D] fp32.
-// mode 0 = masked mean, 1 = first token (CLS), 2 = last token. normalize -> v / ||v||.
+// mode 0 = masked mean, 1 = first token (CLS), 2 = last token. normalize -> v / ||v||. With lens, sequence b is the first lens[b] of its
+// rows (padded batches; the first and last token of an empty one is its first row).
 // One workgroup a sequence, bound by what its CU fetches: 16-byte column units times as many row groups as the threads
 // hold, eight rows of each in flight, the groups' sums added in LDS. 61 sequences of ~300 rows of 1024: one row group of 128
 // threads, a row at a time, took 142 us; with 1024 threads 20.
 template <int kPoolThreads>
 __global__ __launch_bounds__(kPoolThreads) void pool_kernel(const bf16* __restrict__ h, const int* __restrict__ cu,
-                                                            float* __restrict__ out, int D, int mode, int normalize) {
+                                                            const int* __restrict__ lens, float* __restrict__ out, int D, int mode, int normalize) {
   extern __shared__ float sh[];  // [groups][D] sums + 16 scratch
   const int units = D / 8, cols = max(min(units, kPoolThreads), 1);
   const int b = blockIdx.x;
-  const int s0 = cu[b], s1 = cu[b + 1], n = s1 - s0;
+  const int s0 = cu[b], s1 = lens ? min(s0 + max(lens[b], mode == 0 ? 0 : 1), cu[b + 1]) : cu[b + 1], n = s1 - s0;
   int r0 = s0, r1 = s1;
   if (mode == 1) r1 = min(s0 + 1, s1);
   if (mode == 2) r0 = max(s1 - 1, s0);
@@ -155,20 +156,20 @@ void gai_embedding(const int* ids, const void* table, void* out, int T, int D, i
 }
 
 template <int NT>
-static void launch_pool(const void* h, const int* cu, float* out, int B, int D, int mode, int normalize, hipStream_t st) {
+static void launch_pool(const void* h, const int* cu, const int* lens, float* out, int B, int D, int mode, int normalize, hipStream_t st) {
   const int groups = D < 16 ? NT : D < 8 * NT ? NT / (D / 8) : 1;
-  pool_kernel<NT><<<B, NT, (groups * D + 16) * sizeof(float), st>>>((const bf16*)h, cu, out, D, mode, normalize);
+  pool_kernel<NT><<<B, NT, (groups * D + 16) * sizeof(float), st>>>((const bf16*)h, cu, lens, out, D, mode, normalize);
   GAI_LAUNCH_CHECK();
 }
 
 // T rows in B sequences. 256 threads where 1024 wait for each other over little: one row a sequence (1024 columns, 64 sequences 3.9 -> 3.2 us,
 // 1024 sequences 9.3 -> 4.1) or short ones (1024 x 8 rows of 1024 columns 10.5 -> 5.6). Wide rows fill 1024 threads by themselves (4096
 // columns, 64 x 20 rows 8.7 -> 6.1) unless there are more sequences than the chip holds such workgroups (1024 x 1 row 12.3 -> 8.9).
-void gai_pool(const void* h, const int* cu, float* out, int T, int B, int D, int mode, int normalize, hipStream_t st) {
+void gai_pool(const void* h, const int* cu, const int* lens, float* out, int T, int B, int D, int mode, int normalize, hipStream_t st) {
   if (B == 0) return;
   const bool narrow = D <= 2048;
-  if ((narrow || B > 512) && (mode != 0 || T / (narrow ? 32 : 16) < B)) launch_pool<256>(h, cu, out, B, D, mode, normalize, st);
-  else launch_pool<1024>(h, cu, out, B, D, mode, normalize, st);
+  if ((narrow || B > 512) && (mode != 0 || T / (narrow ? 32 : 16) < B)) launch_pool<256>(h, cu, lens, out, B, D, mode, normalize, st);
+  else launch_pool<1024>(h, cu, lens, out, B, D, mode, normalize, st);
 }
 
 void gai_silu_mul(const void* x, void* y, int T, int I, hipStream_t st) {

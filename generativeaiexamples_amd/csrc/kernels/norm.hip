@@ -95,6 +95,68 @@ __global__ __launch_bounds__(256) void norm_kernel(const bf16* __restrict__ x, c
   }
 }
 
+// An encoder's first norm: LayerNorm(bf16(bf16(word + position) + type)), the roundings of three additions of bf16 rows, each row read
+// once. As a gather, two additions, another gather and the norm it was five launches and eleven passes over the rows: 9240 tokens of 1024
+// columns 84 -> 19 us, 32 tokens 13 -> 4. Ids outside the table take a row of zeros.
+template <int NCH>
+__global__ __launch_bounds__(256) void embed_layernorm_kernel(const int* __restrict__ ids, const int* __restrict__ pos,
+                                                              const bf16* __restrict__ word, const bf16* __restrict__ ptab,
+                                                              const bf16* __restrict__ type, const bf16* __restrict__ w,
+                                                              const bf16* __restrict__ b, bf16* __restrict__ out, int T, int D, int vocab,
+                                                              float eps) {
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= T) return;
+  const int id = ids[row];
+  const bool known = id >= 0 && id < vocab;
+  const bf16 *wr = word + (size_t)(known ? id : 0) * D, *pr = ptab + (size_t)pos[row] * D;
+  bf16x8 xa[NCH], pa[NCH], ta[NCH], ga[NCH], ba[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int idx = (c * 64 + lane) * 8;
+    if (idx < D) {
+      xa[c] = known ? load8(wr + idx) : bf16x8{};
+      pa[c] = load8(pr + idx);
+      ta[c] = load8(type + idx);
+      ga[c] = load8(w + idx);
+      ba[c] = load8(b + idx);
+    }
+  }
+  float s = 0.f, q = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    if ((c * 64 + lane) * 8 < D) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        xa[c][j] = (bf16)((float)(bf16)((float)xa[c][j] + (float)pa[c][j]) + (float)ta[c][j]);
+        s += (float)xa[c][j];
+      }
+    }
+  }
+  const float mean = wave_sum(s) / D;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    if ((c * 64 + lane) * 8 < D) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float d = (float)xa[c][j] - mean;
+        q += d * d;
+      }
+    }
+  }
+  const float inv = rsqrtf(wave_sum(q) / D + eps);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int idx = (c * 64 + lane) * 8;
+    if (idx < D) {
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (bf16)(((float)xa[c][j] - mean) * inv * (float)ga[c][j] + (float)ba[c][j]);
+      store8(out + (size_t)row * D + idx, o);
+    }
+  }
+}
+
 template <bool LN>
 void dispatch_norm(const void* x, const void* rin, void* rout, const void* w, const void* b, void* out, int T,
                    int D, float eps, hipStream_t st) {
@@ -118,6 +180,24 @@ void dispatch_norm(const void* x, const void* rin, void* rout, const void* w, co
 }
 
 }  // namespace
+
+void gai_embed_layernorm(const int* ids, const int* pos, const void* word, const void* ptab, const void* type, const void* w,
+                         const void* b, void* out, int T, int D, int vocab, float eps, hipStream_t st) {
+  if (T == 0) return;
+  const int nch = (D + 511) / 512;
+#define GAI_EMB_CASE(N)                                                                                                       \
+  if (nch <= N) {                                                                                                            \
+    embed_layernorm_kernel<N><<<(T + 3) / 4, 256, 0, st>>>(ids, pos, (const bf16*)word, (const bf16*)ptab, (const bf16*)type, \
+                                                           (const bf16*)w, (const bf16*)b, (bf16*)out, T, D, vocab, eps);    \
+    GAI_LAUNCH_CHECK();                                                                                                      \
+    return;                                                                                                                  \
+  }
+  GAI_EMB_CASE(1)
+  GAI_EMB_CASE(2)
+  GAI_EMB_CASE(4)
+#undef GAI_EMB_CASE
+  gai_launch_error(__FILE__, __LINE__, "embed_layernorm: hidden size > 2048 unsupported");
+}
 
 void gai_rmsnorm(const void* x, const void* residual_in, void* residual_out, const void* w, void* out, int T, int D,
                  float eps, hipStream_t st) {

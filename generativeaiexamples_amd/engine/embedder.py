@@ -67,8 +67,9 @@ class Embedder:
 
             m, dev = self.model, self.model.device
             c = m.cfg
-            ids = torch.zeros(B * L, dtype=torch.int32, device=dev)
-            lens = torch.full((B,), L, dtype=torch.int32, device=dev)
+            inp = torch.zeros(B * L + B, dtype=torch.int32, device=dev)  # ids and lengths: one copy fills both
+            ids, lens = inp[:B * L], inp[B * L:]
+            lens.fill_(L)
             attn = PackedAttention([L] * B, c.num_heads, c.head_dim_padded, dev, m.dtype)
             attn.ctx = lens  # the key count per sequence IS the real length (keys past it are masked)
             s = torch.cuda.Stream(device=dev)
@@ -80,7 +81,7 @@ class Embedder:
             with hip_graph_capture(g, s):
                 out = m.embed_padded(ids, lens, attn, B, L)
             # the graph reads and writes attn's buffers (index tensors, pages where it has any) by address: keep them alive
-            self._graphs[key] = (g, ids, lens, out, attn)
+            self._graphs[key] = (g, inp, out, attn)
         return self._graphs[key]
 
     def capture_graphs(self, max_batch: int = 64, max_len: int = 128) -> int:
@@ -101,14 +102,13 @@ class Embedder:
         L = next((x for x in self.GRAPH_L if x >= longest), None)
         if B is None or L is None:
             return None
-        g, ids, lens, out, _ = self._graph_for(B, L)
-        flat = torch.zeros(B, L, dtype=torch.int32)
-        ln = torch.ones(B, dtype=torch.int32)
+        g, inp, out, _ = self._graph_for(B, L)
+        host = torch.zeros(B * L + B, dtype=torch.int32)
+        host[B * L:] = 1
         for i, x in enumerate(seqs):
-            flat[i, :len(x)] = torch.tensor(x, dtype=torch.int32)
-            ln[i] = len(x)
-        ids.copy_(flat.view(-1), non_blocking=True)
-        lens.copy_(ln, non_blocking=True)
+            host[i * L:i * L + len(x)] = torch.tensor(x, dtype=torch.int32)
+            host[B * L + i] = len(x)
+        inp.copy_(host, non_blocking=True)
         g.replay()
         return out[:n].clone()
 

@@ -239,10 +239,13 @@ class BertModel:
         dev = ids.device
         attn = attn if attn is not None else PackedAttention(seq_lens, H, hp, dev, self.dtype)
         pos = attn.positions  # restart at 0 for every sequence
-        h = ops.embedding(ids, w["word"])
-        h = h + w["pos"][pos.long()]
-        h = h + (w["type"][0] if type_ids is None else w["type"][type_ids.long()])
-        h = ops.layer_norm(h, w["emb_ln_w"], w["emb_ln_b"], c.ln_eps)
+        if max(attn.q_lens, default=0) > w["pos"].shape[0]:
+            raise IndexError(f"a sequence of {max(attn.q_lens)} tokens, the encoder has {w['pos'].shape[0]} positions")
+        if type_ids is None:
+            h = ops.embed_layer_norm(ids, pos, w["word"], w["pos"], w["type"][0], w["emb_ln_w"], w["emb_ln_b"], c.ln_eps)
+        else:
+            h = ops.embedding(ids, w["word"]) + w["pos"][pos.long()] + w["type"][type_ids.long()]
+            h = ops.layer_norm(h, w["emb_ln_w"], w["emb_ln_b"], c.ln_eps)
         out = torch.empty(T, H * hp, device=dev, dtype=self.dtype)
         for i in range(c.num_layers):
             p = f"l{i}."
@@ -264,18 +267,8 @@ class BertModel:
         ``attn`` built for q_lens = [L] * B whose ``ctx`` tensor holds ``lens``: every query row attends to the
         real keys of its sequence only (the kernel masks keys >= ctx), so real rows equal the packed forward;
         pooling runs over the real rows. All shapes are fixed: capturable once per (B, L) bucket."""
-        c = self.cfg
-        h = self.encode_hidden(ids, attn.cu_q, [L] * B, attn=attn).view(B, L, -1).float()
-        if c.pooling == "cls":
-            o = h[:, 0]
-        elif c.pooling == "last":
-            o = h[torch.arange(B, device=h.device), (lens.long() - 1).clamp_min(0)]
-        else:
-            m = (torch.arange(L, device=h.device)[None, :] < lens[:, None]).float()
-            o = (h * m[..., None]).sum(1) / lens.clamp_min(1)[:, None].float()
-        if c.normalize:
-            o = torch.nn.functional.normalize(o, dim=-1, eps=1e-12)
-        return o
+        h = self.encode_hidden(ids, attn.cu_q, [L] * B, attn=attn)
+        return ops.pool(h, attn.cu_q, self.cfg.pooling, self.cfg.normalize, lens)
 
     def score(self, ids, cu_seqlens, seq_lens, type_ids=None) -> torch.Tensor:
         """Cross-encoder relevance logits [B] (CLS -> dense+tanh -> classifier)."""

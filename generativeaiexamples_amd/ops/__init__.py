@@ -942,6 +942,18 @@ def embedding(ids, table, vstart: int = 0, vend: int | None = None, out=None):
     return out
 
 
+def embed_layer_norm(ids, pos, word, ptab, type_row, w, b, eps):
+    """LayerNorm(word[ids] + ptab[pos] + type_row), each sum rounded to the tables' dtype; positions must lie in ``ptab`` (not looked
+    at here: they are on the device), ids outside ``word`` take a row of zeros."""
+    ok = (ids.is_cuda and word.shape[1] % 8 == 0 and word.shape[1] <= 2048 and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+          and not t.data_ptr() & 15 for t in (word, ptab, type_row, w, b)) and pos.dtype == torch.int32)
+    if not ok:
+        return layer_norm(embedding(ids, word) + ptab[pos.long()] + type_row, w, b, eps)
+    out = torch.empty(ids.numel(), word.shape[1], dtype=word.dtype, device=ids.device)
+    native().embed_layernorm(ids.int().contiguous(), pos.contiguous(), word, ptab, type_row, w, b, eps, out)
+    return out
+
+
 def decode_advance(toks, ids, pos, ctx, slots, block_tables, n_valid):
     """In-place multi-step decode update for rows < n_valid[0]: ids <- toks, pos += 1, ctx = pos + 1,
     slots from block_tables (int32 tensors; graph-capturable: the row count is read on device)."""
@@ -1189,11 +1201,12 @@ def moe_combine(Y, pos, w, residual=None, ids=None, n_real: int = 0, identity=No
 POOL_MODES = {"mean": 0, "cls": 1, "last": 2}
 
 
-def pool(h, cu_seqlens, mode: str = "mean", normalize: bool = True):
+def pool(h, cu_seqlens, mode: str = "mean", normalize: bool = True, lens=None):
+    """Sentence vectors of packed rows; ``lens`` [B] int32: sequence b is the first lens[b] of its rows (padded batches)."""
     if not h.is_cuda:
-        return ref.pool(h, cu_seqlens, mode, normalize)
+        return ref.pool(h, cu_seqlens, mode, normalize, lens)
     out = torch.empty(cu_seqlens.numel() - 1, h.shape[-1], dtype=torch.float32, device=h.device)
-    native().pool(h, cu_seqlens, out, POOL_MODES[mode], normalize)
+    native().pool(h, cu_seqlens, out, POOL_MODES[mode], normalize, lens)
     return out
 
 

@@ -384,14 +384,22 @@ def decode_advance(toks, ids, pos, ctx, slots, bt, n_valid, block):
     slots[:n] = (bt[rows, p // block].long() * block + p % block).to(slots.dtype)
 
 
-def pool(h, cu_seqlens, mode="mean", normalize=True):
+def embed_layer_norm(ids, pos, word, ptab, type_row, w, b, eps):
+    h = embedding(ids, word) + ptab[pos.long()]
+    return layer_norm(h + type_row, w, b, eps, None)
+
+
+def pool(h, cu_seqlens, mode="mean", normalize=True, lens=None):
     cu = cu_seqlens.tolist()
+    n = None if lens is None else lens.tolist()
     outs = []
     for b in range(len(cu) - 1):
         s, e = cu[b], cu[b + 1]
+        if n is not None:
+            e = min(e, s + max(n[b], 0 if mode == "mean" else 1))
         x = h[s:e].float()
         if mode == "mean":
-            v = x.mean(0)
+            v = x.sum(0) / max(e - s, 1) if n is not None else x.mean(0)
         elif mode == "cls":
             v = x[0]
         else:

@@ -797,6 +797,38 @@ def test_sim_topk_no_candidates(cuda):
     assert index.search_raw(X[:3], 0)[1].shape == (3, 0) and index.search(X[:3], 0) == [[], [], []]
 
 
+@pytest.mark.parametrize("T,D", [(1, 8), (5, 64), (33, 512), (3, 520), (300, 1024), (9, 1032), (7, 2048), (4, 2056), (0, 64)])
+def test_embed_layer_norm(cuda, T, D):
+    """The rows of separate gathers, additions and norm, bit for bit: ids outside the table (a row of zeros), the last position; past
+    2048 columns those operations themselves run."""
+    g = torch.Generator(device=cuda).manual_seed(T + D)
+    word, ptab, typ, w, b = (torch.randn(*n, device=cuda, generator=g).bfloat16() for n in ((97, D), (31, D), (2, D), (D,), (D,)))
+    ids = torch.randint(-1, 99, (T,), device=cuda, generator=g, dtype=torch.int32)
+    pos = torch.randint(0, 31, (T,), device=cuda, generator=g, dtype=torch.int32)
+    if T:
+        pos[T - 1], ids[0] = 30, 96
+    want = ops.layer_norm(ops.embedding(ids, word) + ptab[pos.long()] + typ[1], w, b, 1e-12)
+    assert torch.equal(ops.embed_layer_norm(ids, pos, word, ptab, typ[1], w, b, 1e-12), want)
+
+
+@pytest.mark.parametrize("mode", ["mean", "cls", "last"])
+@pytest.mark.parametrize("L,lens,D", [(32, [23], 1024), (5, [5, 0, 1, 3], 64), (128, [128, 7, 0] * 30, 384), (9, [2, 9], 4096)])
+def test_pool_padded(cuda, mode, L, lens, D):
+    """The first lens[b] rows of each L: what the rows alone give, whatever stands in the padding (NaN here)."""
+    torch.manual_seed(L)
+    h = torch.randn(len(lens), L, D, device=cuda).bfloat16()
+    for i, n in enumerate(lens):
+        h[i, max(n, 1):] = float("nan")
+        if n == 0 and mode == "mean":
+            h[i] = float("nan")
+    cu = torch.arange(len(lens) + 1, device=cuda, dtype=torch.int32) * L
+    ln = torch.tensor(lens, device=cuda, dtype=torch.int32)
+    for normalize in (False, True):
+        got = ops.pool(h.view(-1, D), cu, mode, normalize, ln)
+        want = ref.pool(h.view(-1, D).cpu(), cu.cpu(), mode, normalize, ln.cpu())
+        _close(got, want, 1e-5, 1e-5, "padded pool")
+
+
 @pytest.mark.parametrize("D,lens", [(1024, [303, 1, 0, 65]), (384, [512, 7]), (64, [1000, 129, 128]), (8, [2000]), (8192, [3, 9]),
                                     (8208, [2, 20]), (1024, [31, 1, 0, 20, 9]), (2048, [33, 2]), (64, [5, 2, 16]), (8, [3, 30]),
                                     (4096, [1, 3, 17, 2] * 130)])  # the last five: 256 threads for means too
