@@ -43,6 +43,8 @@ class Embedder:
                  max_batch_tokens: int = 65536, query_prefix: str = "query: ", passage_prefix: str = "passage: ",
                  model_name: str | None = None):
         self.model, self.tok = model, tokenizer
+        if hasattr(model, "fragment_weights_"):
+            model.fragment_weights_()  # a service's weights are final: the layout that its products read fastest
         self.max_len = min(max_len or model.cfg.max_position, model.cfg.max_position)
         self.max_batch_tokens = max_batch_tokens
         self.prefix = {"query": query_prefix, "passage": passage_prefix}
@@ -253,6 +255,8 @@ class Reranker:
                  max_batch_tokens: int = 65536, model_name: str | None = None):
         assert model.cfg.num_labels > 0, "reranker needs a cross-encoder head (num_labels > 0)"
         self.model, self.tok = model, tokenizer
+        if hasattr(model, "fragment_weights_"):
+            model.fragment_weights_()  # a service's weights are final: the layout that its products read fastest
         self.max_len = min(max_len or model.cfg.max_position, model.cfg.max_position)
         self.max_batch_tokens = max_batch_tokens
         self.name = model_name or model.cfg.name

@@ -34,6 +34,7 @@ import torch
 import torch.distributed as dist
 import torch.nn.functional as F
 
+from .. import ops
 from .ddp import GradBucketer
 
 log = logging.getLogger(__name__)
@@ -115,7 +116,7 @@ class EmbedFineTuner:
         dev = self.model.device
         self.device = dev
         # fp32 master copies of every weight (the serving model keeps its bf16 tensors)
-        self.w = {k: t.detach().float().clone().requires_grad_(True) for k, t in self.model.w.items()
+        self.w = {k: ops.natural_weight(t).detach().float().clone().requires_grad_(True) for k, t in self.model.w.items()
                   if not k.startswith("cls_")}
         self.params = list(self.w.values())
         self.opt = torch.optim.AdamW(self.params, lr=cfg.lr, weight_decay=cfg.weight_decay)
@@ -226,7 +227,7 @@ class EmbedFineTuner:
     def sync_to_model(self):
         """Copy the fp32 master weights into the serving model (bf16), ready for /v1/embeddings."""
         for k, t in self.w.items():
-            self.model.w[k].copy_(t.to(self.model.w[k].dtype))
+            self.model.put_weight(k, t)
 
     def save(self):
         from safetensors.torch import save_file

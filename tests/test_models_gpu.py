@@ -204,6 +204,35 @@ def test_query_embed_graph_matches_packed(cuda):
     assert bool((cos > 0.999).all()), cos
 
 
+@pytest.mark.parametrize("hidden,heads,ff", [(1024, 16, 4096), (512, 8, 1024), (512, 16, 2048), (384, 12, 1536)])
+def test_encoder_fragment_weights(cuda, hidden, heads, ff):
+    """A service's weights in fragment order give the row-major model's bits, from one token to large products (heads padded, and
+    projections off the layout's grid, among them); checkpoints come out and go in row-major."""
+    cfg = BertConfig(vocab_size=2048, hidden_size=hidden, intermediate_size=ff, num_layers=2, num_heads=heads)
+    m = BertModel(cfg, device=cuda).random_init(7)
+    state = m.export_hf_state()
+    row = BertModel(cfg, device=cuda).load_hf_state(state)
+    emb = Embedder(m, bert_byte_tokenizer(cfg.vocab_size))
+    assert ops.is_frag(m.w["l1.down"]) and ops.is_frag(m.w["l0.qkv"]) == (hidden % 512 == 0) and not ops.is_frag(row.w["l1.down"])
+    after = m.export_hf_state()
+    assert all(torch.equal(after[k], state[k]) for k in state)
+
+    def same():
+        for lens in ([1], [23], [64, 1], [60, 5], [300, 17], [512] * 9, [33] * 70):
+            ids = torch.randint(3, 2048, (sum(lens),), device=cuda, dtype=torch.int32)
+            cu = torch.tensor([0] + lens, device=cuda).cumsum(0).int()
+            assert torch.equal(m.embed(ids, cu, lens), row.embed(ids, cu, lens))
+
+    same()
+    state = BertModel(cfg, device=cuda).random_init(8).export_hf_state()
+    m.load_hf_state(state), row.load_hf_state(state)
+    same()
+    m.random_init(9), row.random_init(9)
+    same()
+    Embedder(m, emb.tok)    # a second service on the same model
+    same()
+
+
 @pytest.mark.parametrize("L", [40, 100])
 def test_query_embed_graph_e5_large_batch64(cuda, L):
     """The headline's query encoder (e5-large-v2 shape) through the graph path at batch 64."""
