@@ -642,6 +642,50 @@ void parallel_add_norm_f32(Tensor& res, const optional<Tensor>& a, const optiona
                             h2 ? h2->data_ptr() : nullptr, T, D, (float)eps, dt, cur_stream());
 }
 
+// a / b: bf16 rows [T, D], or fp32 K slices [k, T, D] of a product (+ a bias)
+void slabs_add_norm_f32(Tensor& res, const optional<Tensor>& a, const optional<Tensor>& a_bias, const optional<Tensor>& sa,
+                        const optional<Tensor>& b, const optional<Tensor>& b_bias, const optional<Tensor>& sb,
+                        const optional<Tensor>& w1, const optional<Tensor>& h1, const optional<Tensor>& w2, const optional<Tensor>& h2,
+                        double eps) {
+  float* r = f32w(res, "res");
+  TORCH_CHECK(res.dim() == 2, "slabs_add_norm_f32: res [T, D]");
+  const int T = res.size(0), D = res.size(1);
+  auto on = [](const Tensor& t, int bytes) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0; };
+  TORCH_CHECK(on(res, 16), "slabs_add_norm_f32: res on 16 bytes");
+  struct Branch {
+    const float* slabs = nullptr;
+    const void *rows = nullptr, *bias = nullptr;
+    int ks = 0, ld = 0;
+  };
+  auto branch = [&](const optional<Tensor>& x, const optional<Tensor>& bias, const char* name) {
+    Branch o;
+    if (!x) return o;
+    if (x->dim() == 3) {
+      o.slabs = f32(*x, name);
+      o.ks = x->size(0);
+      TORCH_CHECK(o.ks > 0 && x->size(1) == T && x->size(2) == D && on(*x, 16), "slabs_add_norm_f32: ", name, " [k, T, D] on 16 bytes");
+    } else {
+      TORCH_CHECK(act_dt(*x, name) == 0 && x->dim() == 2 && x->size(0) == T && x->size(1) == D, "slabs_add_norm_f32: ", name, " [T, D]");
+      o.rows = x->data_ptr();
+      o.ld = row_stride(*x, name);
+      TORCH_CHECK(o.ld % 4 == 0 && on(*x, 8) && !bias, "slabs_add_norm_f32: rows on 8 bytes, without a bias");
+    }
+    if (bias) {
+      TORCH_CHECK(act_dt(*bias, "bias") == 0 && bias->numel() == D && bias->is_contiguous() && on(*bias, 8), "slabs_add_norm_f32: bias");
+      o.bias = bias->data_ptr();
+    }
+    return o;
+  };
+  const Branch A = branch(a, a_bias, "a"), B = branch(b, b_bias, "b");
+  for (const auto* x : {&sa, &sb, &w1, &w2})
+    if (*x) TORCH_CHECK((*x)->numel() == D, "slabs_add_norm_f32: one scale / weight per channel");
+  for (const auto* x : {&h1, &h2})
+    if (*x) TORCH_CHECK(act_dt(**x, "h") == 0 && (*x)->is_contiguous() && (*x)->numel() == res.numel() && on(**x, 8), "slabs_add_norm_f32: outputs");
+  gai_slabs_add_norm_f32(r, A.slabs, A.ks, A.bias, A.rows, A.ld, sa ? f32(*sa, "sa") : nullptr, B.slabs, B.ks, B.bias, B.rows, B.ld,
+                         sb ? f32(*sb, "sb") : nullptr, w1 ? f32(*w1, "w1") : nullptr, h1 ? h1->data_ptr() : nullptr,
+                         w2 ? f32(*w2, "w2") : nullptr, h2 ? h2->data_ptr() : nullptr, T, D, (float)eps, cur_stream());
+}
+
 void latent_norm_write(const Tensor& dq, const Tensor& wq, const Tensor& dkv, const Tensor& wkv, const Tensor& slots,
                        Tensor& q_out, Tensor& k_cache, Tensor& v_cache, double eps) {
   const int dt = act_dt(dq, "dq");
@@ -786,6 +830,7 @@ void gai_bind_seq_ops(pybind11::module_& m) {
   m.def("gqa_attention_ws_floats", &gqa_attention_ws_floats);
   m.def("rotary_half_kv_write", &rotary_half_kv_write);
   m.def("parallel_add_norm_f32", &parallel_add_norm_f32);
+  m.def("slabs_add_norm_f32", &slabs_add_norm_f32);
   m.def("latent_norm_write", &latent_norm_write);
   m.def("hyper_connect", &hyper_connect);
   m.def("head_linear", &head_linear);

@@ -403,6 +403,17 @@ int64_t gemm_qkv_partials(const Tensor& A, const Tensor& W, Tensor& ws, bool psw
   return gai_gemm_qkv_partials(A.data_ptr(), W.data_ptr(), M, N, K, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
 }
 
+void gemm_partials(const Tensor& A, const Tensor& W, Tensor& ws, bool psw) {
+  check_bf16(A, "A");
+  check_bf16(W, "W");
+  check_f32(ws, "ws");
+  TORCH_CHECK(A.dim() == 2 && A.is_contiguous() && W.dim() == 2 && W.size(1) == A.size(1) && W.is_contiguous(), "gemm_partials: A, W");
+  const int M = A.size(0), K = A.size(1), N = W.size(0), ks = gai_gemm_partials_ks(M, N, K);
+  TORCH_CHECK(ks > 0 && ws.numel() >= (int64_t)ks * M * N, "gemm_partials: workspace");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(A.data_ptr()) & 15) == 0, "gemm_partials: rows on 16 bytes");
+  gai_gemm_partials(A.data_ptr(), W.data_ptr(), M, N, K, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
+}
+
 void sample(const Tensor& logits, const Tensor& temperature, const Tensor& top_p, const Tensor& top_k,
             const Tensor& seeds, int64_t step, Tensor& out, const c10::optional<Tensor>& ws) {
   check_f32(logits, "logits");
@@ -1231,6 +1242,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ep_combine", &ep_combine);
   m.def("custom_all_to_all", &custom_all_to_all);
   m.def("gemm_qkv_partials", &gemm_qkv_partials);
+  m.def("gemm_partials", &gemm_partials);
+  m.def("gemm_partials_ks", [](int64_t M, int64_t N, int64_t K) { return gai_gemm_partials_ks(M, N, K); });
   m.def("gemv", &gemv, pybind11::arg("x"), pybind11::arg("gamma"), pybind11::arg("eps"), pybind11::arg("W"),
         pybind11::arg("epi"), pybind11::arg("out"), pybind11::arg("res"), pybind11::arg("frag") = false,
         pybind11::arg("swi") = pybind11::none(), pybind11::arg("ks") = 1);

@@ -95,6 +95,8 @@ void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, co
                      int Hkv, int D, float scale, int split_keys, int max_splits, int kv_fp8, float k_scale,
                      float v_scale, hipStream_t st, int* split_cnt = nullptr,
                      const GaiQkvFold* fold = nullptr, bool queue = false);
+int gai_gemm_partials_ks(int M, int N, int K);
+void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st);
 // QKV partial slabs only (for GaiQkvFold): KS (2..8) when launched, 0 when the shape runs elsewhere.
 int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st);
 
@@ -305,6 +307,10 @@ void gai_rotary_half_kv_write(const void* q, int ldq, const void* k, int ldk, co
 void gai_parallel_add_norm_f32(float* res, const void* a, int lda, const float* sa, const void* b, int ldb, const float* sb,
                                const float* w1, void* h1, const float* w2, void* h2, int T, int D, float eps, int dt,
                                hipStream_t st);
+// the same with bf16 rows, a branch being rows or K slices [k][T][D] (+ bias) of its product; D <= 2048
+void gai_slabs_add_norm_f32(float* res, const float* a_slabs, int ka, const void* a_bias, const void* a, int lda, const float* sa,
+                            const float* b_slabs, int kb, const void* b_bias, const void* b, int ldb, const float* sb, const float* w1,
+                            void* h1, const float* w2, void* h2, int T, int D, float eps, hipStream_t st);
 // sigmoid-mode decode steps: number of key splits (1: none); part must hold splits * T * H * DV floats
 int gai_sigmoid_attention_splits(int T, int S, int H);
 // recurrent.hip

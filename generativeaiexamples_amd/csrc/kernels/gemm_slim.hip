@@ -319,13 +319,19 @@ int gai_gemm_slim_ks(int M, int N, int K) {
   return 0;
 }
 
-void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
-                             void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
+// those slices, [ks][M][N]
+void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, float* ws, int psw, hipStream_t st) {
   const int ks = gai_gemm_slim_ks(M, N, K);
-  if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_slim_layernorm: the shape has no slices");
+  if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_slim_partials: the shape has no slices");
   if (M <= 16) launch_slim<1, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
   else if (M <= 32) launch_slim<2, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
   else launch_slim<4, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
+}
+
+void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
+                             void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
+  const int ks = gai_gemm_slim_ks(M, N, K);
+  gai_gemm_slim_partials(A, W, M, N, K, ws, psw, st);
 #define GAI_SLN(NCH, KS)                                                                                                 \
   slabs_layernorm_kernel<NCH, KS><<<M, 64, 0, st>>>(ws, ks, M, N, (const bf16*)bias, (const bf16*)R, (const bf16*)g,     \
                                                     (const bf16*)b, (bf16*)out, eps)

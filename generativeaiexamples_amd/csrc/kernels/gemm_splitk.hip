@@ -928,6 +928,21 @@ int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, flo
   return KS;
 }
 
+// The K slices of a product, fp32 [ks][M][N], for a kernel that adds them up itself; ks from gai_gemm_partials_ks (0: the product has none).
+int gai_gemm_partials_ks(int M, int N, int K) {
+  if (M < 1 || M > 64 || N % 16 || K % 512 || gai_gemm_dec2_ok(M, N, K, EPI_NONE)) return 0;  // single-pass kernel owns it
+  if (gai_gemm_slim_nf(M, N, K, false)) return gai_gemm_slim_ks(M, N, K);
+  const int ks2 = gai_gemm_dec2_partials_ks(M, N, K), ks = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
+  return ks < 2 ? 0 : ks;
+}
+
+void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st) {
+  const int ks = gai_gemm_partials_ks(M, N, K);
+  if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_partials: the product has no slices");
+  if (gai_gemm_slim_nf(M, N, K, false)) gai_gemm_slim_partials(A, B, M, N, K, ws, psw, st);
+  else if (!gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw)) launch_partials(A, B, M, N, K, ks, ws, psw, st);
+}
+
 void gai_gemm_splitk(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K,
                      int ldc, int epi, int out_f32, float* ws, int psw, hipStream_t st) {
   if (psw && N % 16) gai_launch_error(__FILE__, __LINE__, "gemm_splitk: pre-shuffled weights need N % 16 == 0");

@@ -279,7 +279,7 @@ class BamanexModel(HybridDecoderBase):
                                      w[x + "inv_freq"], self.cfg.rms_eps)
         att = ops.window_attention(q, kc, vc, seq["bt"], seq["cu"], seq["ctx"], H, G, dk, dv, float(m["scale"]),
                                    window=m["window"], sink=w[x + "sink"], gate=proj[:, c:c + H])
-        return ops.linear(att, w[x + "o"], w[x + "o.b"])
+        return ops.linear_partial(att, w[x + "o"], w[x + "o.b"])
 
     def _dense(self, h, p):
         w, F_ = self.w, self.w[p + "down"].shape[1]
@@ -288,7 +288,7 @@ class BamanexModel(HybridDecoderBase):
         else:
             gu = ops.linear(h, w[p + "in"])
             mid = ops.act_mul(gu[:, :F_], gu[:, F_:], "gelu_tanh", self.dtype)
-        return ops.linear(mid, w[p + "down"])
+        return ops.linear_partial(mid, w[p + "down"])
 
     def _shared(self, h, p, limit):
         """Shared expert -> (output, its gate logit per token): one fused gate | up | sg projection."""

@@ -154,6 +154,34 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     return out
 
 
+class Partial:
+    """A product whose K slices are not added up yet: fp32 [slices, rows, columns] and the bias that their sum takes
+    (linear_partial). parallel_add_norm_f32 takes it in place of the rows."""
+
+    __slots__ = ("slabs", "bias")
+
+    def __init__(self, slabs: torch.Tensor, bias: Optional[torch.Tensor] = None):
+        self.slabs, self.bias = slabs, bias
+
+    def index_select(self, dim: int, idx: torch.Tensor) -> "Partial":
+        assert dim == 0
+        return Partial(self.slabs.index_select(1, idx), self.bias)
+
+
+def linear_partial(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
+    """linear(x, w, bias) for parallel_add_norm_f32: its K slices (a Partial) where a decode-sized product on the GPU has some,
+    which saves the launch that adds them, else the rows."""
+    if (x.is_cuda and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
+            and 1 <= x.shape[0] <= 64 and w.shape[0] <= 2048 and not (x.data_ptr() & 15 or (bias is not None and bias.data_ptr() & 7))):
+        psw, nat = decode_operand(w), native()
+        ks = nat.gemm_partials_ks(x.shape[0], *w.shape) if psw is not None or (_SPLITK and _GEMM_FORCE == 0) else 0
+        if ks:
+            ws = torch.empty(ks, x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+            nat.gemm_partials(x, w if psw is None else psw, ws, psw is not None)
+            return Partial(ws, bias)
+    return linear(x, w, bias)
+
+
 def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
     """layer_norm(linear(x, w, bias, residual)). A short question's product leaves most of the chip idle with one workgroup a
     column tile: its K is cut into slices (gemm_slim.hip) whose sums the norm adds up."""
@@ -1780,10 +1808,15 @@ def mlstm(q, k, v, ig, fg, ib, fb, cap: float, gate, norm_w, S, n, m, cu, slots,
 def parallel_add_norm_f32(res, a=None, sa=None, b=None, sb=None, w1=None, w2=None, eps: float = 1e-6, out_dtype=None):
     """The pass between two parallel layers: fp32 ``res`` (in place) += sa * a + sb * b - the two branch outputs times
     their per-channel scales (fp32 [D]; None: one) - and the next layer's two norms of the new sum, rmsnorm(res) * w1 and
-    rmsnorm(res) * w2 in out_dtype (None where no weight is given). One read of the stream, one set of statistics."""
+    rmsnorm(res) * w2 in out_dtype (None where no weight is given). One read of the stream, one set of statistics. A branch
+    may be a Partial (linear_partial; bf16, at most 2048 channels)."""
     if not res.is_cuda:
         return ref.parallel_add_norm_f32(res, a, sa, b, sb, w1, w2, eps, out_dtype)
     h1, h2 = (torch.empty(res.shape, dtype=out_dtype, device=res.device) if w is not None else None for w in (w1, w2))
+    if isinstance(a, Partial) or isinstance(b, Partial):
+        rows = [(x.slabs, x.bias) if isinstance(x, Partial) else (x, None) for x in (a, b)]
+        native().slabs_add_norm_f32(res, *rows[0], sa, *rows[1], sb, w1, h1, w2, h2, float(eps))
+        return h1, h2
     native().parallel_add_norm_f32(res, a, sa, b, sb, w1, h1, w2, h2, float(eps))
     return h1, h2
 

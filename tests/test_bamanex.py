@@ -209,6 +209,49 @@ def test_parallel_add_norm_kept_groups(D):
         assert ((h.double() - ref).abs() <= (2.0 ** -8 + 2e-6) * ref.abs()).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D,K", [(1, 512, 512), (24, 2048, 5632), (24, 2048, 2048), (64, 2048, 11264), (17, 1040, 4096), (3, 16, 1024),
+                                   (33, 1024, 5120), (65, 2048, 2048), (5, 2064, 5632)])
+def test_branches_as_k_slices(cuda, T, D, K):
+    """A branch handed over as its product's K slices: the rows that adding them in order and rounding once gives (the stream's bits),
+    normed alike up to the order of the squares' sum, in either branch, beside rows or alone, with and without bias and scale. Past 64
+    rows or 2048 channels, and where a product is one pass, linear_partial gives rows."""
+    g = torch.Generator(device=cuda).manual_seed(T + D + K)
+    rn = lambda *s: torch.randn(*s, device=cuda, generator=g)  # noqa: E731
+    x, w, bias = rn(T, K).bfloat16(), (rn(D, K) * K ** -0.5).bfloat16(), rn(D).bfloat16()
+    other, res, sa, sb, w1, w2 = rn(T, D).bfloat16(), rn(T, D), rn(D), rn(D), rn(D), rn(D)
+    for frag in (False, True):
+        wt = w.clone()
+        if frag and not ops.to_fragment_layout_(wt):
+            continue
+        for b in (None, bias):
+            p = ops.linear_partial(x, wt, b)
+            want = ops.linear(x, wt, b)
+            if not isinstance(p, ops.Partial):
+                assert torch.equal(p, want)
+                continue
+            assert T <= 64 and D <= 2048
+            rows = torch.zeros(T, D, device=cuda)
+            for s in p.slabs:
+                rows = rows + s
+            rows = (rows if b is None else rows + b.float()).bfloat16()
+            exact = x.double() @ w.double().t() + (0 if b is None else b.double())
+            # K products of unit normals and weights of K^-1/2: fp32 sums, then one rounding to bf16
+            assert ((rows.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 2.0 ** -18 * K ** 0.5).all()
+            for kw, kr in ((dict(a=p, sa=sa), dict(a=rows, sa=sa)), (dict(a=other, sa=sa, b=p, sb=sb), dict(a=other, sa=sa, b=rows, sb=sb)),
+                           (dict(a=p, b=ops.Partial(p.slabs.flip(0).contiguous()[:1])), dict(a=rows, b=p.slabs[-1].bfloat16()))):
+                r1, r2 = res.clone(), res.clone()
+                h = ops.parallel_add_norm_f32(r1, **kw, w1=w1, w2=w2, eps=1e-5, out_dtype=torch.bfloat16)
+                k = ops.parallel_add_norm_f32(r2, **kr, w1=w1, w2=w2, eps=1e-5, out_dtype=torch.bfloat16)
+                assert torch.equal(r1, r2)
+                for y, z in zip(h, k):    # one bf16 step where the two sums of squares round apart
+                    assert ((y.float() - z.float()).abs() <= 2.0 ** -7 * z.float().abs()).all()
+                r1 = res.clone()
+                assert ops.parallel_add_norm_f32(r1, **kw) == (None, None) and torch.equal(r1, r2)
+            few = p.index_select(0, torch.tensor([T - 1, 0], device=cuda))
+            assert torch.equal(few.slabs, p.slabs[:, [T - 1, 0]])
+
+
 @_GPU
 @pytest.mark.parametrize("D", [64, 513, 1000, 2048, 2050, 4096, 8196])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
