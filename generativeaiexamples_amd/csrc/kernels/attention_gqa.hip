@@ -252,19 +252,39 @@ __global__ __launch_bounds__(64) void gqa_split_kernel(GqaArgs a) {
 #pragma unroll
   for (int i = 0; i < DV / 32; ++i) acc[i] = f32x16{};
   const int kr = key_perm(qi), lp = p_last >> 4;
-  for (int kb = kb0; kb <= kb1; kb += 32) {
-    const int pg[2] = {bt[kb >> 4], bt[min((kb >> 4) + 1, lp)]};
-    const bf16* kp = a.kc + (((size_t)(kr < 16 ? pg[0] : pg[1]) * a.G + g) * 16 + (kr & 15)) * DK + 8 * hb;
-    bf16x8 kf[DK / 16], vf[2][DV / 32];  // the values of the block are on their way while it is scored
+  // A wave's share is a chain of blocks, each of which waited for memory. A block's keys (and the pages of the one after) are on their way
+  // while the one before is used, its values while it is scored; keys and values of both, 128 channels: 28.5 us where this takes 27.1
+  // (64 streams). Up to 192 + 128 channels: wider heads' keys do not fit the registers twice (192: 26.9 -> 27.1 us, 256: 36 -> 54) and are
+  // asked for with the block's values. Us, chain -> ahead, with the merge: 24 streams of 1000 keys (16 heads of 128 on 4) 20.1 -> 16.6, 64
+  // of 1024 27.2 -> 27.1, 64 of 8000 198 -> 182, 16 x 4 tokens of 2000 53.6 -> 39.1, 8 of 30000 99.5 -> 89.5.
+  constexpr bool AHEAD = DK + DV <= 320;
+  bf16x8 kf[AHEAD ? 2 : 1][DK / 16], vf[2][DV / 32];
+  int pg[2][2];
+  auto pages = [&](int n, int u) {
+    const int p = (kb0 >> 4) + 2 * n;
+    pg[u][0] = bt[min(p, lp)];
+    pg[u][1] = bt[min(p + 1, lp)];
+  };
+  auto keys = [&](int u) {
+    const bf16* kp = a.kc + (((size_t)(kr < 16 ? pg[u][0] : pg[u][1]) * a.G + g) * 16 + (kr & 15)) * DK + 8 * hb;
 #pragma unroll
-    for (int i = 0; i < DK / 16; ++i) kf[i] = load8(kp + 16 * i);
+    for (int i = 0; i < DK / 16; ++i) kf[AHEAD ? u : 0][i] = load8(kp + 16 * i);
+  };
+  const int nb = (kb1 - kb0) / 32 + 1;
+  auto use = [&](int n, int u) __attribute__((always_inline)) {
+    const int kb = kb0 + 32 * n;
+    if (!AHEAD) keys(u);
 #pragma unroll
     for (int k2 = 0; k2 < 2; ++k2)
 #pragma unroll
-      for (int i = 0; i < DV / 32; ++i) vf[k2][i] = load8(a.vc + (((size_t)pg[k2] * a.G + g) * DV + qi) * 16 + 8 * hb + 32 * i * 16);
+      for (int i = 0; i < DV / 32; ++i) vf[k2][i] = load8(a.vc + (((size_t)pg[u][k2] * a.G + g) * DV + qi) * 16 + 8 * hb + 32 * i * 16);
+    if (n + 1 < nb) {
+      if (AHEAD) keys(u ^ 1);
+      pages(n + 2, u);
+    }
     f32x16 sc = f32x16{};
 #pragma unroll
-    for (int i = 0; i < DK / 16; ++i) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], sc, 0, 0, 0);
+    for (int i = 0; i < DK / 16; ++i) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[AHEAD ? u : 0][i], qf[i], sc, 0, 0, 0);
     soft_block(sc, a.scale2, kb + 31 > p_first || kb < lo_last, kb, pos, lo, hb, m, l, acc);
 #pragma unroll
     for (int k2 = 0; k2 < 2; ++k2) {
@@ -276,6 +296,13 @@ __global__ __launch_bounds__(64) void gqa_split_kernel(GqaArgs a) {
         acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k2][i], pl, acc[i], 0, 0, 0);
       }
     }
+  };
+  pages(0, 0);
+  pages(1, 1);
+  if (AHEAD) keys(0);
+  for (int n = 0; n < nb; n += 2) {
+    use(n, 0);
+    if (n + 1 < nb) use(n + 1, 1);
   }
   l = half_sum(l);
   if (!mine) return;

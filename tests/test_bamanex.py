@@ -576,6 +576,30 @@ def test_grouped_attention_bf16_against_reference(dk, dv, H, G, window):
         assert e.max() < 1e-2, (ctx, float(e.max()), int(e.argmax()))
 
 
+@_GPU
+@pytest.mark.parametrize("dk,dv,H,G", [(128, 128, 8, 2), (32, 32, 4, 1), (160, 160, 4, 2), (192, 128, 3, 1), (192, 192, 2, 1), (256, 256, 4, 2)])
+@pytest.mark.parametrize("window", [0, 2500])
+def test_grouped_attention_long_shares(dk, dv, H, G, window):
+    """Single-token steps whose waves walk shares of one to five key blocks, the last of them partly past the sequence, against the fp32
+    reference of the same op (the tolerance of the test above)."""
+    g = torch.Generator().manual_seed(dk)
+    rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    ctx = [4097, 3100, 2049, 33, 1, 4640]
+    S, nb = len(ctx), [(c + B - 1) // B for c in ctx]
+    perm = torch.randperm(sum(nb), generator=g).tolist()
+    bt = torch.zeros(S, max(nb), dtype=torch.int32)
+    for s in range(S):
+        bt[s, :nb[s]] = torch.tensor(perm[sum(nb[:s]):sum(nb[:s + 1])], dtype=torch.int32)
+    kc, vc = rn(sum(nb), G, B, dk).to(torch.bfloat16), rn(sum(nb), G, dv, B).to(torch.bfloat16)
+    q, sink = (rn(S, H * dk) * 2 * dk ** -0.5).to(torch.bfloat16), rn(H) * 2
+    args = (bt, torch.arange(S + 1, dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32))
+    want = ops.window_attention(q.float(), kc.float(), vc.float(), *args, H, G, dk, dv, 0.9, window=window, sink=sink)
+    got = ops.window_attention(q.cuda(), kc.cuda(), vc.cuda(), *[a.cuda() for a in args], H, G, dk, dv, 0.9, window=window,
+                               sink=sink.cuda()).float().cpu()
+    e = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert e.max() < 1e-2, (float(e.max()), int(e.argmax()))
+
+
 @pytest.mark.parametrize("device,dtype", FP32_TARGETS)
 def test_window_edge_in_model(device, dtype):
     """One attention layer with nearly even weights: changing the token at the window's last position moves the logits,
