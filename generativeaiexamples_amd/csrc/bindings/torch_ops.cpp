@@ -1229,6 +1229,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                     (int)down, (int)offset, (int)y.numel(), (float)gain, y.data_ptr<float>(), cur_stream());
   });
   m.def("moe_route", &moe_route);
+  m.def("moe_router_rows_ok", [](int64_t D, int64_t E) { return gai_moe_router_rows_ok(D, E) != 0; });
   m.def("moe_router", &moe_router);
   m.def("moe_scale_rows", &moe_scale_rows);
   m.def("moe_gemm_large", &moe_gemm_large);

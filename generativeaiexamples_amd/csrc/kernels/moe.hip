@@ -84,6 +84,81 @@ __global__ void moe_route_kernel(const float* __restrict__ logits, int T, int E,
   }
 }
 
+// Prompt-sized steps of up to 16 experts, bf16: router product, softmax and top-k in one launch. A workgroup takes 16 tokens, its eight
+// waves a share of D each, on matrix cores (products of bf16 are exact, sums fp32; the shares are added in order), then a thread a token
+// does what moe_route_kernel does. Bound by the latency of one read of the rows: a wave has 16 steps of them in flight, which is all of
+// its share at 4096. 3389 tokens x 4096, 8 experts: as the upcast of rows and weights, an fp32 library product and moe_route_kernel four
+// launches, 40 us; here 12.7, about half of it the rows, 16 x 64 bytes a load.
+__global__ __launch_bounds__(512) void moe_router_rows_kernel(const bf16* __restrict__ x, int ldx, const bf16* __restrict__ W, int T,
+                                                              int D, int E, int k, float eps, int* __restrict__ ids,
+                                                              float* __restrict__ w) {
+  constexpr int WAVES = 8, U = 16;
+  __shared__ float part[WAVES][16][17];
+  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4, t0 = blockIdx.x * 16;
+  const bf16* xp = x + (size_t)min(t0 + r16, T - 1) * ldx + 8 * q;
+  const bf16* wp = W + (size_t)min(r16, E - 1) * D + 8 * q;
+  const int nk = D / 32, per = (nk + WAVES - 1) / WAVES, s1 = min(nk, (wid + 1) * per);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int s = wid * per;
+  for (; s + U <= s1; s += U) {
+    bf16x8 a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      a[u] = load8(xp + 32 * (s + u));
+      b[u] = load8(wp + 32 * (s + u));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
+  }
+  for (; s < s1; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(xp + 32 * s), load8(wp + 32 * s), acc, 0, 0, 0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) part[wid][4 * q + r][r16] = acc[r];  // [token][expert]
+  __syncthreads();
+  const int t = t0 + threadIdx.x;
+  if (threadIdx.x >= 16 || t >= T) return;
+  float z[16], mx = -INFINITY, sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    z[e] = e < E ? 0.f : -INFINITY;
+    if (e < E)
+#pragma unroll
+      for (int i = 0; i < WAVES; ++i) z[e] += part[i][threadIdx.x][e];
+    mx = fmaxf(mx, z[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 16; ++e)
+    if (e < E) {
+      z[e] = __expf(z[e] - mx);
+      sum += z[e];
+    }
+  float tot = eps;
+  uint32_t taken = 0;
+  int id[16];
+  float p[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {  // the largest not taken, the lower id of equal ones
+    if (j >= k) break;
+    float best = -1.f;
+    int at = 0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (e < E && !(taken >> e & 1) && z[e] / sum > best) {
+        best = z[e] / sum;
+        at = e;
+      }
+    taken |= 1u << at;
+    id[j] = at;
+    p[j] = best < 0.f ? NAN : best;  // no score compares: NaN logits
+    tot += p[j];
+  }
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (j < k) {
+      ids[(size_t)t * k + j] = id[j];
+      w[(size_t)t * k + j] = p[j] / tot;
+    }
+}
+
 // Decode-sized steps: router product, softmax and top-k of a token in one workgroup (logits and scores stay in LDS). The
 // waves deal the experts out and dot them in fp32; wave 0 normalises and picks k times the largest score (the lower id wins
 // a tie); weights = chosen scores / (their sum + eps).
@@ -764,6 +839,8 @@ void gai_moe_route(const float* logits, int T, int E, int k, int renorm, int* id
   GAI_LAUNCH_CHECK();
 }
 
+int gai_moe_router_rows_ok(int D, int E) { return E <= 16 && D % 32 == 0; }
+
 // dt: x / W 0 bf16, 1 fp32
 void gai_moe_router(const void* x, int ldx, const void* W, int T, int D, int E, int k, float eps, int* ids, float* w, int dt,
                     hipStream_t st) {
@@ -772,6 +849,11 @@ void gai_moe_router(const void* x, int ldx, const void* W, int T, int D, int E, 
     gai_launch_error(__FILE__, __LINE__, "moe_router: 1 <= top-k <= min(16, experts), experts <= 4096");
   const int wide = dt ? 4 : 8;
   const bool ok = D % wide == 0 && ldx % wide == 0 && (((size_t)x | (size_t)W) & 15) == 0;
+  if (T > 64 && !dt && gai_moe_router_rows_ok(D, E) && ok) {
+    moe_router_rows_kernel<<<(T + 15) / 16, 512, 0, st>>>((const bf16*)x, ldx, (const bf16*)W, T, D, E, k, eps, ids, w);
+    GAI_LAUNCH_CHECK();
+    return;
+  }
   const size_t lds = E * sizeof(float);
 #define GAI_MR(TA, VEC_) moe_router_kernel<TA, VEC_><<<T, 256, lds, st>>>((const TA*)x, ldx, (const TA*)W, D, E, k, eps, ids, w)
   if (dt) { if (ok) GAI_MR(float, 4); else GAI_MR(float, 1); }

@@ -138,8 +138,7 @@ class MixtralModel(LlamaModel):
     def moe_mlp(self, x: torch.Tensor, layer: int, residual: torch.Tensor | None) -> torch.Tensor:
         c, w, p = self.cfg, self.w, f"l{layer}."
         T = x.shape[0]
-        logits = ops.linear(x, w[p + "router"], out_dtype=torch.float32)
-        ids, wts = ops.moe_route(logits, c.top_k, True)
+        ids, wts = ops.moe_router(x, w[p + "router"], c.num_experts, c.top_k)
         k = c.top_k
         if self.ep_group is not None:
             return self._moe_ep(x, ids, wts, w[p + "w13"], w[p + "w2"], residual)
@@ -167,7 +166,7 @@ class MixtralModel(LlamaModel):
         128x128 grouped kernel at Mixtral widths: all experts in one launch from _GROUPED_MIN_ROWS rows an expert on, else
         one launch each, which reads the expert row ranges on the host: one sync per layer, prefill only (decode steps
         keep the graph-capturable grouped path)."""
-        xs = x.index_select(0, a_rows.long())
+        xs = ops.embedding(a_rows, x) if x.dtype == torch.bfloat16 else x.index_select(0, a_rows.long())
         if rows >= _GROUPED_MIN_ROWS * w13.shape[0] and x.dtype == w13.dtype == torch.bfloat16 and ops._GEMM_FORCE == 0:
             h1 = ops.moe_gemm_large(xs, w13, offs, swiglu=True)
             y = None if h1 is None else ops.moe_gemm_large(h1, w2, offs)
@@ -243,28 +242,34 @@ class MixtralModel(LlamaModel):
         q = torch.empty(T, self.hq, hd, device=res.device, dtype=self.dtype)
         attn = torch.empty_like(q)
         h = None
+        # prompts on one GPU: the O product and the experts' sum add the residual themselves, the norms only read it
+        res_epi = res.is_cuda and ctx.tp_size == 1 and self.ep_group is None and self.e_local == c.num_experts and T > 64
         for i in range(c.num_layers):
             p = f"l{i}."
             x = ops.rms_norm(res, w[p + "attn_norm"], c.rms_eps) if h is None else \
                 ops.rms_norm(h, w[p + "attn_norm"], c.rms_eps, residual=res)
-            qkv = ops.linear(x, w[p + "qkv"])
             kc, vc = kv.layer(i)
-            ops.rope_kv_write(qkv, fb.positions, self.cos_sin, fb.slots, q, kc, vc, self.hq, self.hkv, hd, True)
+            ops.linear_rope_kv(x, w[p + "qkv"], None, fb.positions, self.cos_sin, fb.slots, q, kc, vc, self.hq, self.hkv, hd)
             if P > 0:
                 ops.attention_prefill(q[:P], kc, vc, fb.prefill_block_tables, fb.cu_q, fb.prefill_ctx, self.scale,
                                       True, tiles=fb.prefill_tiles, q_lens=fb.prefill_qlen, out=attn[:P])
             if T > P:
                 ops.attention_decode(q[P:], kc, vc, fb.decode_block_tables, fb.decode_ctx, self.scale, ws=decode_ws,
                                      max_ctx=fb.max_decode_ctx, out=attn[P:])
+            if res_epi:
+                ops.linear(attn.view(T, -1), w[p + "o"], residual=res, out=res)
+                x = ops.rms_norm(res, w[p + "mlp_norm"], c.rms_eps)
+                res = self.moe_mlp(x, i, res)
+                continue
             h = ops.linear(attn.view(T, -1), w[p + "o"])
             ctx.tp_all_reduce(h)
             x = ops.rms_norm(h, w[p + "mlp_norm"], c.rms_eps, residual=res)
             h = self.moe_mlp(x, i, None)
             ctx.tp_all_reduce(h)
         if fb.sample_rows is not None:
-            h = h.index_select(0, fb.sample_rows)
+            h = h.index_select(0, fb.sample_rows) if h is not None else None
             res = res.index_select(0, fb.sample_rows)
-        x = ops.rms_norm(h, w["norm"], c.rms_eps, residual=res)
+        x = ops.rms_norm(res, w["norm"], c.rms_eps) if h is None else ops.rms_norm(h, w["norm"], c.rms_eps, residual=res)
         logits = ops.linear(x, w["lm_head"], out_dtype=torch.float32)
         if fb.tp_local_logits and ctx.tp_size > 1:
             return logits

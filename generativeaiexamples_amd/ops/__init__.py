@@ -1039,10 +1039,11 @@ def moe_route(logits: torch.Tensor, k: int, renorm: bool = True, score: str = "s
 
 def moe_router(x: torch.Tensor, W: torch.Tensor, E: int, k: int, eps: float = 0.0):
     """Router product, softmax scores over the E experts and the k largest -> (expert ids int32 [T, k], weights fp32 [T, k]
-    = chosen scores / (their sum + eps)). W [>= E, D] (rows past E: padding). One launch per decode-sized step, the router
-    GEMM and moe_route otherwise; logits are fp32 either way."""
+    = chosen scores / (their sum + eps)). W [>= E, D] (rows past E: padding). One launch for decode-sized steps, and for any
+    with up to 16 experts in bf16; the router GEMM and moe_route otherwise. Logits are fp32 either way."""
     T = x.shape[0]
-    if not x.is_cuda or T > 64:
+    if not x.is_cuda or (T > 64 and not (x.dtype == W.dtype == torch.bfloat16 and native().moe_router_rows_ok(x.shape[1], E)
+                                         and x.stride(1) == 1 and x.stride(0) % 8 == 0 and not (x.data_ptr() | W.data_ptr()) & 15)):
         return moe_route(linear(x, W, out_dtype=torch.float32)[:, :E], k, eps=eps)
     ids = torch.empty(T, k, dtype=torch.int32, device=x.device)
     w = torch.empty(T, k, dtype=torch.float32, device=x.device)

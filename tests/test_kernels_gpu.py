@@ -797,6 +797,30 @@ def test_sim_topk_no_candidates(cuda):
     assert index.search_raw(X[:3], 0)[1].shape == (3, 0) and index.search(X[:3], 0) == [[], [], []]
 
 
+@pytest.mark.parametrize("T,D,E,k", [(65, 32, 1, 1), (80, 96, 5, 5), (200, 4096, 8, 2), (1003, 1056, 16, 4), (97, 64, 3, 2), (66, 2080, 16, 16)])
+def test_moe_router_rows(cuda, T, D, E, k):
+    """Prompt-sized router against 64 bits: the same experts wherever two scores are further apart than the sums' error, softmax
+    weights, equal logits in the order of their ids; W with padding rows, rows of a wider buffer, NaN rows stay NaN."""
+    g = torch.Generator(device=cuda).manual_seed(T)
+    W = torch.randn(E + 3, D, device=cuda, generator=g).bfloat16()
+    x = (torch.randn(T, D + 8, device=cuda, generator=g) * D ** -0.5).bfloat16()[:, :D]
+    x[3] = 0
+    x[T - 1, D - 1] = float("nan")
+    for W_ in (W, W[:E].contiguous()):
+        ids, w = ops.moe_router(x, W_, E, k, 1e-9)
+        z = x.double() @ W_[:E].double().t()
+        err = D * 2.0 ** -24 * (x.double().abs() @ W_[:E].double().abs().t()).max(-1).values    # any order of the sum
+        p = z.softmax(-1)
+        want, order = torch.sort(p, dim=-1, descending=True, stable=True)
+        got = torch.gather(p, 1, ids.long())
+        ok = torch.arange(T, device=cuda) < T - 1
+        tol = (4 * err + 1e-6)[:, None]     # exp: relative error of the logit's; division and the hardware exponential 1e-6
+        assert ((got - want[:, :k]).abs() <= tol * want[:, :k] + 1e-9)[ok].all()
+        assert ((w.double() - got / (got.sum(-1, keepdim=True) + 1e-9)).abs() <= 2 * tol + 1e-7)[ok].all()
+        assert all(len(set(r)) == k for r in ids[:-1].tolist()) and ids[3].tolist() == list(range(k))
+        assert w[T - 1].isnan().all()
+
+
 @pytest.mark.parametrize("T,D", [(1, 8), (5, 64), (33, 512), (3, 520), (300, 1024), (9, 1032), (7, 2048), (4, 2056), (0, 64)])
 def test_embed_layer_norm(cuda, T, D):
     """The rows of separate gathers, additions and norm, bit for bit: ids outside the table (a row of zeros), the last position; past
