@@ -134,6 +134,28 @@ void rope_kv_write(const Tensor& qkv, const Tensor& pos, const Tensor& cos_sin, 
                     (float)k_scale, (float)v_scale, cur_stream());
 }
 
+// the same with an RMS norm of every q and k head in front of the rotation; bf16 pages
+void norm_rope_kv_write(const Tensor& qkv, const Tensor& wq, const Tensor& wk, double eps, const Tensor& pos, const Tensor& cos_sin,
+                        const Tensor& slots, Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t Hq, int64_t Hkv, int64_t D) {
+  for (const Tensor* t : {&qkv, &wq, &wk, static_cast<const Tensor*>(&q_out)}) {
+    check_bf16(*t, "norm_rope_kv_write");
+    TORCH_CHECK((reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0, "norm_rope_kv_write: rows on 16 bytes");
+  }
+  check_i32(pos, "positions");
+  check_f32(cos_sin, "cos_sin");
+  check_i32(slots, "slot_mapping");
+  const int T = qkv.size(0);
+  TORCH_CHECK(!kv_cache_fp8(k_cache, v_cache) && k_cache.is_contiguous() && v_cache.is_contiguous() && gai_rope_kv_norm_ok(D) &&
+                  ((reinterpret_cast<uintptr_t>(k_cache.data_ptr()) | reinterpret_cast<uintptr_t>(v_cache.data_ptr())) & 15) == 0,
+              "norm_rope_kv_write: bf16 pages on 16 bytes, heads of 64, 128 or 256");
+  TORCH_CHECK(qkv.dim() == 2 && qkv.is_contiguous() && qkv.size(1) == (Hq + 2 * Hkv) * D && q_out.numel() == T * Hq * D &&
+                  wq.numel() == D && wk.numel() == D && pos.numel() >= T && slots.numel() >= T && cos_sin.size(-1) == D,
+              "norm_rope_kv_write: shapes");
+  TORCH_CHECK(k_cache.size(-2) == 16 && k_cache.size(-1) == D && v_cache.size(-1) == 16, "bad kv cache layout");
+  gai_rope_kv_rows(qkv.data_ptr(), pos.data_ptr<int>(), cos_sin.data_ptr<float>(), slots.data_ptr<int>(), q_out.data_ptr(),
+                   k_cache.data_ptr(), v_cache.data_ptr(), T, Hq, Hkv, D, 1, wq.data_ptr(), wk.data_ptr(), (float)eps, cur_stream());
+}
+
 // QKV projection fused with RoPE + KV write: split-K path for decode (M <= 64), the prefill GEMM's
 // epilogue for M >= 1024. False: nothing launched, the caller runs linear + rope_kv_write.
 bool gemm_rope_kv(const Tensor& A, const Tensor& B, const optional<Tensor>& bias, const Tensor& pos,
@@ -1144,6 +1166,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_layernorm", &embed_layernorm);
   m.def("layernorm", &layernorm);
   m.def("rope_kv_write", &rope_kv_write);
+  m.def("norm_rope_kv_write", &norm_rope_kv_write);
+  m.def("rope_kv_norm_ok", [](int64_t D) { return gai_rope_kv_norm_ok(D) != 0; });
   m.def("gemm_mid_rows", &gemm_mid_rows);
   m.def("gemm_slim_nf", &gai_gemm_slim_nf);
   m.def("gemm_slim_ks", &gai_gemm_slim_ks);

@@ -21,6 +21,9 @@ void gai_layernorm(const void* x, const void* residual_in, void* residual_out, c
 // row count of page b (rows past blk_n are zeroed).
 void gai_kv_pack(const void* qkv, int ld, int koff, int voff, const int* blk_tok, const int* blk_n, int nblk,
                  void* k_cache, void* v_cache, int Hkv, int D, hipStream_t st);
+int gai_rope_kv_norm_ok(int D);
+void gai_rope_kv_rows(const void* qkv, const int* pos, const float* cos_sin, const int* slots, void* q_out, void* k_cache, void* v_cache,
+                      int T, int Hq, int Hkv, int D, int rope, const void* wq, const void* wk, float eps, hipStream_t st);
 void gai_rope_kv_write(const void* qkv, const int* pos, const float* cos_sin, const int* slots, void* q_out,
                        void* k_cache, void* v_cache, int T, int Hq, int Hkv, int D, int rope, int kv_fp8,
                        float k_scale, float v_scale, hipStream_t st);

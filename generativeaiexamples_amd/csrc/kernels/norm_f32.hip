@@ -600,6 +600,7 @@ __global__ __launch_bounds__(256) void act_mul_kernel(const TI* __restrict__ a, 
     else if (act == 1) y = fmaxf(x, 0.f) * fmaxf(x, 0.f);
     else if (act == 2) y = cap * tanhf(x / cap);
     else if (act == 3) y = 0.5f * x * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
+    else if (act == 5) y = 1.0f / (1.0f + expf(-x));
     else {  // clamped gated activation of (a, b) with limit cap
       const float g = fminf(x, cap), u = fminf(fmaxf((float)xb.v[i], -cap), cap);
       y = g / (1.0f + expf(-kGluSlope * g)) * (u + 1.0f);
@@ -741,8 +742,8 @@ void gai_add_dyt_f32(float* res, const void* delta, int ldd, const float* extra,
 void gai_act_mul(const void* a, int lda, const void* b, int ldb, void* out, int T, int C, int act, float cap, int dt_in,
                  int dt_out, hipStream_t st) {
   if (T == 0 || C == 0) return;
-  if (act < 0 || act > 4)
-    gai_launch_error(__FILE__, __LINE__, "act_mul: act 0 (silu), 1 (squared ReLU), 2 (tanh cap), 3 (tanh GELU) or 4 (clamped gate)");
+  if (act < 0 || act > 5)
+    gai_launch_error(__FILE__, __LINE__, "act_mul: act 0 (silu), 1 (squared ReLU), 2 (tanh cap), 3 (tanh GELU), 4 (clamped gate) or 5 (sigmoid)");
   if ((act == 2 || act == 4) && !(cap > 0.f)) gai_launch_error(__FILE__, __LINE__, "act_mul: the cap / limit must be positive");
   if (act == 4 && !b) gai_launch_error(__FILE__, __LINE__, "act_mul: the clamped gated activation takes two operands");
   // four elements per thread where rows, strides and base addresses allow aligned vector accesses

@@ -39,6 +39,116 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(const bf16* __restrict__ q
   rope_kv_store<D>(x1, x2, t, h, i0, pos, cos_sin, slots, q_out, k_cache, v_cache, Hq, Hkv, rope, inv_ks, inv_vs);
 }
 
+// The same for a prompt's tokens and bf16 pages, with an optional RMS norm of every q and k head (weights wq / wk, rounded to bf16 before
+// the rotation). Bound by one read and one write of the rows; what kept it from that was V^T, whose elements went out two bytes at a time,
+// 32 bytes apart (a page row is one channel of 16 tokens). Here a workgroup takes TOK tokens and either four heads of q and k - 16-byte
+// loads and stores, all four heads' rows in flight, the token's angles read once for them - or one head of v, turned in LDS: eight tokens
+// that fill half a page row go out as 16 bytes, others a token's neighbours side by side. Us, before | here: 10095 tokens of 16 + 4 + 4
+// heads of 128 49.7 | 30.7, 3389 of 32 + 8 + 8 34.8 | 21.0, 999 14.8 | 7.6, 187 4.3 | 3.8, 66 to 100 alike; 3000 of 3 x 16 of 64 27.8 | 10.3. With
+// the norm, which was copies of the heads, two norm launches and copies back, 10095 tokens 147 | 27.3 (under the profiler).
+template <int D>
+constexpr int rows_tokens() { return 256 / (D / 16) / 8 * 8; }
+constexpr int kHeadsAWg = 4;
+
+template <int D, bool NORM>
+__global__ __launch_bounds__(256) void rope_kv_rows_kernel(const bf16* __restrict__ qkv, const int* __restrict__ pos,
+                                                           const float* __restrict__ cos_sin, const int* __restrict__ slots,
+                                                           bf16* __restrict__ q_out, bf16* __restrict__ k_cache,
+                                                           bf16* __restrict__ v_cache, int T, int Hq, int Hkv, int rope,
+                                                           const bf16* __restrict__ wq, const bf16* __restrict__ wk, float eps) {
+  constexpr int LP = D / 16, TOK = rows_tokens<D>(), GROUPS = TOK / 8;
+  __shared__ __attribute__((aligned(16))) bf16 vs[TOK][D + 8];
+  __shared__ int whole[GROUPS];
+  const int tid = threadIdx.x, t0 = blockIdx.x * TOK, H = Hq + 2 * Hkv, qk = (Hq + Hkv + kHeadsAWg - 1) / kHeadsAWg;
+  if ((int)blockIdx.y < qk) {
+    const int t = t0 + tid / LP, i0 = tid % LP * 8;
+    if (tid >= TOK * LP || t >= T) return;
+    const int h0 = blockIdx.y * kHeadsAWg, hn = min(kHeadsAWg, Hq + Hkv - h0), slot = slots[t];
+    const bf16* src = qkv + ((size_t)t * H + h0) * D + i0;
+    bf16x8 x[kHeadsAWg][2];
+#pragma unroll
+    for (int j = 0; j < kHeadsAWg; ++j)
+      if (j < hn) {
+        x[j][0] = load8(src + j * D);
+        x[j][1] = load8(src + j * D + D / 2);
+      }
+    float c[8], s[8];
+    if (rope) {
+      const float* cs = cos_sin + (size_t)pos[t] * D + i0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        c[e] = cs[e];
+        s[e] = cs[e + D / 2];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kHeadsAWg; ++j) {
+      if (j >= hn) break;
+      const int h = h0 + j;
+      if constexpr (NORM) {
+        float ss = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ss += (float)x[j][u][e] * (float)x[j][u][e];
+#pragma unroll
+        for (int d = 1; d < LP; d <<= 1) ss += __shfl_xor(ss, d, 64);
+        const float inv = rsqrtf(ss / D + eps);
+        const bf16* w = (h < Hq ? wq : wk) + i0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const bf16x8 g = load8(w + u * (D / 2));
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[j][u][e] = (bf16)((float)x[j][u][e] * inv * (float)g[e]);
+        }
+      }
+      if (rope) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float a = (float)x[j][0][e], b = (float)x[j][1][e];
+          x[j][0][e] = (bf16)(a * c[e] - b * s[e]);
+          x[j][1][e] = (bf16)(b * c[e] + a * s[e]);
+        }
+      }
+      bf16* dst;
+      if (h < Hq) dst = q_out + ((size_t)t * Hq + h) * D + i0;
+      else if (slot >= 0) dst = k_cache + (((size_t)(slot / kKvBlock) * Hkv + h - Hq) * kKvBlock + slot % kKvBlock) * D + i0;
+      else continue;
+      store8(dst, x[j][0]);
+      store8(dst + D / 2, x[j][1]);
+    }
+    return;
+  }
+  const int g = blockIdx.y - qk;
+  for (int p = tid; p < TOK * (D / 8); p += 256) {
+    const int r = p / (D / 8), col = p % (D / 8) * 8;
+    *reinterpret_cast<bf16x8*>(&vs[r][col]) = load8(qkv + ((size_t)min(t0 + r, T - 1) * H + Hq + Hkv + g) * D + col);
+  }
+  if (tid < GROUPS) {  // eight tokens side by side in one half of a page
+    const int t = t0 + 8 * tid;
+    int ok = t + 7 < T && slots[min(t, T - 1)] >= 0 && slots[min(t, T - 1)] % 8 == 0;
+    for (int i = 1; i < 8; ++i) ok &= slots[min(t + i, T - 1)] == slots[min(t, T - 1)] + i;
+    whole[tid] = ok;
+  }
+  __syncthreads();
+  for (int e = tid; e < D * GROUPS; e += 256) {
+    const int p = e % GROUPS, d = e / GROUPS;
+    if (!whole[p]) continue;
+    const int slot = slots[t0 + 8 * p];
+    bf16x8 o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = vs[8 * p + i][d];
+    store8(v_cache + (((size_t)(slot / kKvBlock) * Hkv + g) * D + d) * kKvBlock + slot % kKvBlock, o);
+  }
+  for (int p = 0; p < GROUPS; ++p) {
+    if (whole[p]) continue;
+    const int t = t0 + 8 * p + (tid & 7), slot = t < T ? slots[t] : -1;
+    if (slot < 0) continue;
+    bf16* dst = v_cache + ((size_t)(slot / kKvBlock) * Hkv + g) * D * kKvBlock + slot % kKvBlock;
+    for (int d = tid >> 3; d < D; d += 32) dst[(size_t)d * kKvBlock] = vs[8 * p + (tid & 7)][d];
+  }
+}
+
 // Encoder self-attention (no RoPE, K / V straight from the packed QKV rows): one workgroup per (transient page, kv
 // head) writes the page's K image [16][D] and V^T image [D][16] whole, with 16-B stores; V is transposed through LDS.
 // Replaces rope_kv_kernel's per-(token, head) scatter for encoders, whose V^T half is 2-B stores 32 B apart and which
@@ -99,10 +209,38 @@ void gai_kv_pack(const void* qkv, int ld, int koff, int voff, const int* blk_tok
   gai_launch_error(__FILE__, __LINE__, "kv_pack: head_dim must be 64, 96, 128 or 256");
 }
 
+namespace {
+constexpr int kRowsFrom = 65;  // decode-sized steps: four times the workgroups
+}
+
+int gai_rope_kv_norm_ok(int D) { return D == 64 || D == 128 || D == 256; }
+
+// wq / wk: weights of the norms of q and k heads (both or none; bf16 pages, gai_rope_kv_norm_ok)
+void gai_rope_kv_rows(const void* qkv, const int* pos, const float* cos_sin, const int* slots, void* q_out, void* k_cache, void* v_cache,
+                      int T, int Hq, int Hkv, int D, int rope, const void* wq, const void* wk, float eps, hipStream_t st) {
+  if (T == 0) return;
+  if ((wq == nullptr) != (wk == nullptr) || (wq && !gai_rope_kv_norm_ok(D)))
+    gai_launch_error(__FILE__, __LINE__, "rope_kv: head norms need both weights and head_dim 64, 128 or 256");
+#define GAI_ROWS(DD, N)                                                                                                              \
+  rope_kv_rows_kernel<DD, N><<<dim3((T + rows_tokens<DD>() - 1) / rows_tokens<DD>(), (Hq + Hkv + kHeadsAWg - 1) / kHeadsAWg + Hkv), \
+                               256, 0, st>>>((const bf16*)qkv, pos, cos_sin, slots, (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, T, \
+                                             Hq, Hkv, rope, (const bf16*)wq, (const bf16*)wk, eps)
+  if (D == 64) { if (wq) GAI_ROWS(64, true); else GAI_ROWS(64, false); }
+  else if (D == 96) GAI_ROWS(96, false);
+  else if (D == 128) { if (wq) GAI_ROWS(128, true); else GAI_ROWS(128, false); }
+  else if (D == 256) { if (wq) GAI_ROWS(256, true); else GAI_ROWS(256, false); }
+  else gai_launch_error(__FILE__, __LINE__, "rope_kv: head_dim must be 64, 96, 128 or 256");
+#undef GAI_ROWS
+  GAI_LAUNCH_CHECK();
+}
+
 void gai_rope_kv_write(const void* qkv, const int* pos, const float* cos_sin, const int* slots, void* q_out,
                        void* k_cache, void* v_cache, int T, int Hq, int Hkv, int D, int rope, int kv_fp8,
                        float k_scale, float v_scale, hipStream_t st) {
   if (T == 0) return;
+  const bool on16 = (((size_t)qkv | (size_t)q_out | (size_t)k_cache | (size_t)v_cache) & 15) == 0;
+  if (T >= kRowsFrom && !kv_fp8 && on16 && D % 32 == 0 && D <= 256)
+    return gai_rope_kv_rows(qkv, pos, cos_sin, slots, q_out, k_cache, v_cache, T, Hq, Hkv, D, rope, nullptr, nullptr, 0.f, st);
   const long items = (long)T * (Hq + 2 * Hkv);
   const float iks = 1.f / k_scale, ivs = 1.f / v_scale;
 #define GAI_ROPE_CASE(DD)                                                                                   \

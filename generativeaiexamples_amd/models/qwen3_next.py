@@ -428,21 +428,18 @@ class Qwen3NextModel:
         hd = c.head_dim
         qkv = ops.linear(x, w[p + "qkv"])
         gate = ops.linear(x, w[p + "gate"])
-        q3 = qkv.view(T, self.hq + 2 * self.hkv, hd)
-        for sl, key in ((slice(0, self.hq), "q_norm"), (slice(self.hq, self.hq + self.hkv), "k_norm")):
-            q3[:, sl] = ops.rms_norm(q3[:, sl].reshape(-1, hd), w[p + key], c.rms_eps).view(T, -1, hd)
         q = torch.empty(T, self.hq, hd, device=x.device, dtype=self.dtype)
         attn = torch.empty_like(q)
         kc, vc = kv.layer(self.kv_index[i])
-        ops.rope_kv_write(qkv, fb.positions, self.cos_sin, fb.slots, q, kc, vc, self.hq, self.hkv, hd, True)
+        ops.norm_rope_kv_write(qkv, w[p + "q_norm"], w[p + "k_norm"], c.rms_eps, fb.positions, self.cos_sin, fb.slots, q, kc, vc,
+                               self.hq, self.hkv, hd)
         if P > 0:
             ops.attention_prefill(q[:P], kc, vc, fb.prefill_block_tables, fb.cu_q, fb.prefill_ctx, self.scale, True,
                                   tiles=fb.prefill_tiles, q_lens=fb.prefill_qlen, out=attn[:P])
         if T > P:
             ops.attention_decode(q[P:], kc, vc, fb.decode_block_tables, fb.decode_ctx, self.scale, ws=decode_ws,
                                  max_ctx=fb.max_decode_ctx, out=attn[P:])
-        a = attn.view(T, -1) * torch.sigmoid(gate)
-        return ops.linear(a, w[p + "o"])
+        return ops.linear(ops.act_mul(gate, attn.view(T, -1), "sigmoid"), w[p + "o"])
 
     @property
     def _gdn_kernels(self) -> bool:

@@ -519,6 +519,20 @@ def rope_kv_write(qkv, positions, cos_sin, slots, q_out, k_cache, v_cache, Hq, H
                            v_scale)
 
 
+def norm_rope_kv_write(qkv, wq, wk, eps, positions, cos_sin, slots, q_out, k_cache, v_cache, Hq: int, Hkv: int, D: int):
+    """rope_kv_write of heads that an RMS norm over their own D channels (weights wq, wk [D]) goes in front of; ``qkv`` may be
+    overwritten. One launch with bf16 pages and heads of 64, 128 or 256."""
+    if (qkv.is_cuda and qkv.dtype == k_cache.dtype == v_cache.dtype == wq.dtype == wk.dtype == torch.bfloat16 and qkv.is_contiguous()
+            and native().rope_kv_norm_ok(D) and not any(t.data_ptr() & 15 for t in (qkv, wq, wk, q_out, k_cache, v_cache))):
+        native().norm_rope_kv_write(qkv, wq, wk, float(eps), positions, cos_sin, slots, q_out, k_cache, v_cache, Hq, Hkv, D)
+        return
+    T = qkv.shape[0]
+    q3 = qkv.view(T, Hq + 2 * Hkv, D)
+    for sl, w in ((slice(0, Hq), wq), (slice(Hq, Hq + Hkv), wk)):
+        q3[:, sl] = rms_norm(q3[:, sl].reshape(-1, D).contiguous(), w, eps).view(T, -1, D)
+    rope_kv_write(qkv, positions, cos_sin, slots, q_out, k_cache, v_cache, Hq, Hkv, D, True)
+
+
 def kv_pack(qkv, blk_tok, blk_n, k_cache, v_cache, Hq: int, Hkv: int, D: int) -> None:
     """Encoder self-attention K / V (no RoPE) from the packed QKV rows [T, (Hq + 2 Hkv) D] into the pages of a transient
     paged cache: page b holds tokens blk_tok[b] .. + blk_n[b] (K [16][D], V^T [D][16]; rows past blk_n zeroed)."""
@@ -1620,12 +1634,12 @@ def add_dyt_f32(res: torch.Tensor, delta: Optional[torch.Tensor], extra: Optiona
     return out
 
 
-_ACT_MUL = {"silu": 0, "relu2": 1, "tanh_cap": 2, "gelu_tanh": 3, "clamp_glu": 4}
+_ACT_MUL = {"silu": 0, "relu2": 1, "tanh_cap": 2, "gelu_tanh": 3, "clamp_glu": 4, "sigmoid": 5}
 
 
 def act_mul(a: torch.Tensor, b: Optional[torch.Tensor] = None, act: str = "silu", out_dtype=None, cap: float = 0.0):
     """act(a) (* b) element by element in fp32: "silu", "relu2" (squared ReLU), "tanh_cap" (cap * tanh(a / cap)),
-    "gelu_tanh"; "clamp_glu": the clamped gated activation min(a, cap) * sigmoid(1.702 min(a, cap)) * (clamp(b, +-cap)
+    "gelu_tanh", "sigmoid"; "clamp_glu": the clamped gated activation min(a, cap) * sigmoid(1.702 min(a, cap)) * (clamp(b, +-cap)
     + 1). a / b may be column slices of wider rows; the result is contiguous in out_dtype (default: a's)."""
     if act not in _ACT_MUL:
         raise ValueError(f"act_mul: unknown activation {act!r}")

@@ -791,7 +791,7 @@ def add_dyt_f32(res, delta, extra, alpha, w, b, out_dtype):
 
 
 def act_mul(a, b, act, out_dtype, cap=0.0):
-    """act(a) (* b): "silu", "relu2" (squared ReLU), "tanh_cap" (cap tanh(a / cap)), "gelu_tanh", or "clamp_glu" (the
+    """act(a) (* b): "silu", "relu2" (squared ReLU), "tanh_cap" (cap tanh(a / cap)), "gelu_tanh", "sigmoid", or "clamp_glu" (the
     clamped gated activation of a, b with limit cap), in fp32."""
     x = a.float()
     if act == "clamp_glu":
@@ -802,6 +802,8 @@ def act_mul(a, b, act, out_dtype, cap=0.0):
         y = F.silu(x)
     elif act == "relu2":
         y = torch.relu(x) ** 2
+    elif act == "sigmoid":
+        y = torch.sigmoid(x)
     else:
         y = float(cap) * torch.tanh(x / float(cap))
     if b is not None:

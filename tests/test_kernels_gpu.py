@@ -797,6 +797,61 @@ def test_sim_topk_no_candidates(cuda):
     assert index.search_raw(X[:3], 0)[1].shape == (3, 0) and index.search(X[:3], 0) == [[], [], []]
 
 
+def _scattered(lens, g, skip=()):
+    """Packed prompts' positions and slots on shuffled pages; tokens of `skip` have no slot."""
+    pages = torch.randperm(sum(-(-n // 16) for n in lens), device="cuda", generator=g)
+    pos, slots, at = [], [], 0
+    for n in lens:
+        p = torch.arange(n, device="cuda")
+        pos.append(p)
+        slots.append(pages[at:at + -(-n // 16)].repeat_interleave(16)[:n] * 16 + p % 16)
+        at += -(-n // 16)
+    slots = torch.cat(slots)
+    slots[list(skip)] = -1
+    return torch.cat(pos).int(), slots.int(), pages.numel()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,lens,skip", [(128, 32, 8, [187], ()), (128, 16, 4, [100, 33, 7, 1, 300], (5, 150)), (64, 3, 2, [65], (64,)),
+                                                (256, 5, 1, [16, 16, 40], ()), (96, 7, 3, [41, 90], (0,)), (128, 0, 3, [70], ()),
+                                                (64, 9, 1, [1] * 80, (8, 9))])
+def test_rope_kv_rows(cuda, D, Hq, Hkv, lens, skip):
+    """Prompt-sized rotation and cache write: the bits of the same tokens 64 at a time (the kernel of decode-sized steps), nothing
+    written for tokens without a slot, with and without the rotation; with head norms the separate norm's rows up to a bf16 step."""
+    g = torch.Generator(device=cuda).manual_seed(sum(lens))
+    pos, slots, n = _scattered(lens, g, skip)
+    T = pos.numel()
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device=cuda, generator=g).bfloat16()
+    cs = torch.randn(512, D, device=cuda, generator=g)
+
+    def run(step, rope=True, norm=None):
+        q = torch.full((T, Hq, D), 7.0, device=cuda, dtype=torch.bfloat16)
+        kc, vc = torch.full((n, Hkv, 16, D), 7.0, device=cuda).bfloat16(), torch.full((n, Hkv, D, 16), 7.0, device=cuda).bfloat16()
+        for a in range(0, T, step):
+            b = min(T, a + step)
+            args = (pos[a:b].contiguous(), cs, slots[a:b].contiguous(), q[a:b], kc, vc, Hq, Hkv, D)
+            if norm:
+                ops.norm_rope_kv_write(qkv[a:b].clone(), *norm, 1e-6, *args)
+            else:
+                ops.rope_kv_write(qkv[a:b], *args, rope)
+        return q, kc, vc
+
+    for rope in (True, False):
+        for got, want in zip(run(T, rope), run(64, rope)):
+            assert torch.equal(got, want)
+    if not ops.native().rope_kv_norm_ok(D) or Hq == 0:
+        return
+    w = [1 + 0.1 * torch.randn(D, device=cuda, generator=g).bfloat16() for _ in range(2)]
+    q3 = qkv.view(T, -1, D).clone()
+    q3[:, :Hq] = ops.rms_norm(q3[:, :Hq].reshape(-1, D).contiguous(), w[0], 1e-6).view(T, -1, D)
+    q3[:, Hq:Hq + Hkv] = ops.rms_norm(q3[:, Hq:Hq + Hkv].reshape(-1, D).contiguous(), w[1], 1e-6).view(T, -1, D)
+    got = run(T, norm=w)
+    assert all(torch.equal(x, y) for x, y in zip(got, run(7, norm=w)))     # a token's rows do not depend on the others
+    qkv = q3.view(T, -1)
+    for x, y in zip(got, run(64)):      # a normed element may round the other way: a bf16 step of it, times |cos| + |sin|
+        assert ((x.float() - y.float()).abs() <= 2.0 ** -7 * 2 * (cs.abs().max() * q3.float().abs().max())).all()
+        assert ((x.float() - y.float()).norm() <= 2.0 ** -9 * y.float().norm())
+
+
 @pytest.mark.parametrize("T,D,E,k", [(65, 32, 1, 1), (80, 96, 5, 5), (200, 4096, 8, 2), (1003, 1056, 16, 4), (97, 64, 3, 2), (66, 2080, 16, 16)])
 def test_moe_router_rows(cuda, T, D, E, k):
     """Prompt-sized router against 64 bits: the same experts wherever two scores are further apart than the sums' error, softmax
