@@ -235,20 +235,20 @@ __global__ __launch_bounds__(256) void gdn_chunk_kernel(const float* __restrict_
   constexpr int LK = DK + 4, LC = kC + 4;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   float* Ks = sm;            // [64][LK]
-  float* Ls = Ks + kC * LK;  // [64][LC]
-  float* Ti = Ls + kC * LC;  // [64][LC]
+  float* Ti = Ks;            // [64][LC] once k is used up; blocks above the diagonal are not kept
+  float* Ls = Ks + kC * (LK > LC ? LK : LC);  // [64][LC]
   __shared__ double Gs[kC];
   __shared__ float Bs[kC];
   const int c = blockIdx.x, h = blockIdx.y, hk = h / (Hv / Hk);
   const int t0 = chunks[2 * c], len = chunks[2 * c + 1];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lc = lane & 15, lr = 4 * (lane >> 4);
+  const int tid = threadIdx.x, lane = tid & 63, lc = lane & 15, lr = 4 * (lane >> 4);
+  const int w = ((tid >> 6) + c + h) & 3;  // this wave's block of 16 rows: block 3 has four tiles, block 0 one
   for (int e = tid; e < kC * DK / 4; e += 256) {
     const int r = e / (DK / 4), col = e % (DK / 4) * 4;
     *reinterpret_cast<f32x4*>(Ks + r * LK + col) =
         r < len ? load4f(k + ((size_t)(t0 + r) * Hk + hk) * DK + col) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int e = tid; e < kC * LC; e += 256) Ti[e] = 0.f;
-  if (w == 0) {  // running sum of the log decay
+  if (tid < 64) {  // running sum of the log decay
     double x = lane < len ? (double)g[(size_t)(t0 + lane) * Hv + h] : 0.;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_kernel(const float* __restrict_
   float* Tc = To + ((size_t)c * Hv + h) * kC * kC;
   for (int e = tid; e < kC * kC / 4; e += 256) {
     const int r = e / (kC / 4), col = e % (kC / 4) * 4;
-    *reinterpret_cast<f32x4*>(Tc + r * kC + col) = load4f(Ti + r * LC + col);
+    *reinterpret_cast<f32x4*>(Tc + r * kC + col) = col / 16 <= r / 16 ? load4f(Ti + r * LC + col) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
 }
 
@@ -791,7 +791,8 @@ void gai_gdn_prep(const void* proj, int ld, const float* cw, const float* cstate
   gai_launch_error(__FILE__, __LINE__, "gdn_prep: key head dim must be 64, 128 or 256");
 }
 
-// 6000 + 4095 tokens, 8 key / 16 value heads of 128 x 128: gdn_chunk 101 us, gdn_carry 290 us (94 chunks in a row at 3.0 us,
+// 6000 + 4095 tokens, 8 key / 16 value heads of 128 x 128: gdn_chunk 90 us (two workgroups a CU, the inverse beside k in LDS, and the
+// block of four tiles always on one SIMD: 101; its bytes alone 45), gdn_carry 290 us (94 chunks in a row at 3.0 us,
 // 256 workgroups), against 47 ms for the same rule as batched fp32 products and triangular solves chunk by chunk in torch;
 // error of o against float64 2.2e-7 - 3.4e-7 (torch 3.2e-7 - 1.1e-6).
 // Key heads of 64 and many workgroups: two plain ones share a CU, which hides more than one of split roles does by itself. us with
@@ -804,7 +805,7 @@ void gai_gdn_chunks(const float* q, const float* k, const float* v, const float*
   if (nc == 0) return;
 #define GAI_GDN(D)                                                                                                      \
   if (DK == D) {                                                                                                        \
-    const int lds = (kC * (D + 4) + 2 * kC * (kC + 4)) * 4;                                                             \
+    const int lds = (kC * (D + 4) + kC * (kC + 4)) * 4;                                                                 \
     const int wgs = S * Hv * (DV / 16);                                                                                 \
     constexpr int lds_plain = (2 * D / 16 + 12) * 64 * 16 + kC * (D + 4) * 4;                                           \
     constexpr int lds_split = (3 * D / 16 + 16) * 64 * 16 + 2 * kC * (D + 4) * 4;                                       \
