@@ -107,14 +107,13 @@ __global__ __launch_bounds__(64 * WPG) void gemm_splitk_kernel(const bf16* __res
   const int cpr = KL / 8;  // 16-B chunks per staged row (multiple of 64)
   constexpr int ROWS = 16 * MB;
 
-  // ---- stage the activation slice: chunk p -> row p / cpr, physical chunk pc, logical pc ^ (row & 15)
-  const int chunks = ROWS * cpr;  // multiple of 256 (cpr % 64 == 0, ROWS % 16 == 0)
-  for (int base = wid * 64; base < chunks; base += 64 * WPG) {
-    const int p = base + lane;
-    const int row = p / cpr, pc = p % cpr, c = pc ^ (row & 15);
-    const bf16* src = A + (size_t)min(row, M - 1) * K + k0 + c * 8;
-    __builtin_amdgcn_global_load_lds(src, GAI_LDS(smem + (size_t)base * 16), 16, 0, 0);
-  }
+  // ---- stage the activation slice, a row's 64 chunks a load: physical chunk pc of a row holds logical pc ^ (row & 15)
+  const int chunks = ROWS * cpr;  // cpr % 64 == 0
+  for (int b = 0; b < cpr; b += 64)
+    for (int row = wid; row < ROWS; row += WPG) {
+      const bf16* src = A + (size_t)min(row, M - 1) * K + k0 + (b + (lane ^ (row & 15))) * 8;
+      __builtin_amdgcn_global_load_lds(src, GAI_LDS(smem + ((size_t)row * cpr + b) * 16), 16, 0, 0);
+    }
 
   // ---- weight stream of this wave: rows n0 + 16*wid + (lane & 15)
   // PSW: W is pre-shuffled into MFMA fragments (psw_offset): one k32 step of a 16-row tile is 1 KiB
@@ -594,6 +593,17 @@ bool splitk_ntw() {
   return on;
 }
 
+// Waves (of 16 columns) that share a staged slice: eight, or six where that leaves the busiest CU fewer columns. A CU draws weights at
+// 25 - 30 KB/us whatever the others do, so 192 workgroups of eight take what 256 of six take three quarters of. A wave's sums do not
+// depend on it. us, eight | six, fragment order: N 6144, K 4096 at M 64 16.0 | 13.4, at M 23 13.3 | 11.4, at M 8 11.9 | 10.4 (and 17.1, 14.1
+// and 12.1 with the slice's rows and columns divided out a 16-byte piece at a time).
+int waves_per_wg(int N, int KS) {
+  const int v = splitk_wpg();
+  if (v != 8) return v;
+  auto busiest = [&](int w) { return ((N + 16 * w - 1) / (16 * w) * KS + 255) / 256 * w; };
+  return busiest(6) < busiest(8) ? 6 : 8;
+}
+
 void launch_partials(const void* A, const void* B, int M, int N, int K, int KS, float* ws, int psw, hipStream_t st) {
   const int MB = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   if (!use_legacy(N, K)) {
@@ -604,7 +614,7 @@ void launch_partials(const void* A, const void* B, int M, int N, int K, int KS, 
   }
   const int KL = K / KS;
   const size_t lds = (size_t)16 * MB * KL * 2;
-  const int wpg = splitk_wpg();
+  const int wpg = waves_per_wg(N, KS);
   dim3 grid((N + 16 * wpg - 1) / (16 * wpg), KS);
 #define GAI_SK1(MBV, WPGV)                                                                                       \
   {                                                                                                              \
@@ -632,6 +642,7 @@ void launch_partials(const void* A, const void* B, int M, int N, int K, int KS, 
 #define GAI_SK(MBV)                   \
   case MBV:                           \
     if (wpg == 4) GAI_SK1(MBV, 4)     \
+    else if (wpg == 6) GAI_SK1(MBV, 6) \
     else GAI_SK1(MBV, 8)              \
     break;
   switch (MB) {

@@ -797,6 +797,23 @@ def test_sim_topk_no_candidates(cuda):
     assert index.search_raw(X[:3], 0)[1].shape == (3, 0) and index.search(X[:3], 0) == [[], [], []]
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 6144, 4096), (23, 6080, 4096), (7, 6144, 4096), (33, 5120, 3072), (1, 3072, 2048), (16, 2064, 1024),
+                                   (64, 4096, 4096)])
+@pytest.mark.parametrize("frag", [True, False])
+def test_splitk_slices(cuda, M, N, K, frag):
+    """K slices of decode-sized products with six and with eight waves a workgroup, the last of them partly past the columns: every
+    slice against 64 bits (sums of exact bf16 products in fp32: K / ks roundings of at most the absolute sum)."""
+    g = torch.Generator(device=cuda).manual_seed(N + M)
+    x, w = (torch.randn(n, K, device=cuda, generator=g).bfloat16() for n in (M, N))
+    ws = torch.full((ops.native().gemm_splitk_ws_floats(M, N, K),), float("nan"), device=cuda)
+    ks = ops.native().gemm_qkv_partials(x, ops.shuffle_fragments(w) if frag else w, ws, frag)
+    assert ks >= 2
+    for i, part in enumerate(ws[:ks * M * N].view(ks, M, N)):
+        a, b = (t[:, i * K // ks:(i + 1) * K // ks].double() for t in (x, w))
+        tol = K // ks * 2.0 ** -24 * (a.abs() @ b.abs().t())
+        assert ((part.double() - a @ b.t()).abs() <= tol).all()
+
+
 def _scattered(lens, g, skip=()):
     """Packed prompts' positions and slots on shuffled pages; tokens of `skip` have no slot."""
     pages = torch.randperm(sum(-(-n // 16) for n in lens), device="cuda", generator=g)
