@@ -115,7 +115,8 @@ __device__ __forceinline__ bf16x8 kv_to_bf16(uint2 v, float s) { return fp8x8_to
 // value of head 0, q_ld apart), instead of from pages that a kernel before has packed: 61 passages of e5-large 25 + 66 -> 62 us a
 // layer, a question 4.2 + 5.4 -> 5.3. V is turned on its way into LDS: a thread fetches two dims of eight keys, 4 B each
 // (whole lines across the wave), and writes two rows of the V^T image. head_dim 64, a kv head per q head.
-template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4, bool ROWS = false>
+// HALF: a workgroup takes one of the two 32-row halves of a tile of the list (few tiles: see prefill_launch)
+template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4, bool ROWS = false, bool HALF = false>
 __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) void attn_prefill_kernel(
     const bf16* __restrict__ q, const KV* __restrict__ kc, const KV* __restrict__ vc,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ tiles,
@@ -149,8 +150,11 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
     bx = L / gridDim.y;
     by = L % gridDim.y;
   }
-  const int seq = tiles[2 * bx], qs = tiles[2 * bx + 1];
+  static_assert(!HALF || RPW == 1, "half tiles: one row group a workgroup");
+  const int tb = HALF ? bx >> 1 : bx;
+  const int seq = tiles[2 * tb], qs = tiles[2 * tb + 1] + (HALF ? 32 * (bx & 1) : 0);
   const int qbeg = cu_q[seq], qlen = cu_q[seq + 1] - qbeg;
+  if (HALF && qs >= qlen) return;
   const int ctx = ROWS ? min(ctx_lens[seq], qlen) : ctx_lens[seq];
   static_assert(!ROWS || (D == 64 && HPW == 1 && HL == 1 && !PIPE && NWV == 4 && sizeof(KV) == 2), "rows: encoder heads of 64");
   const int head = by * HPW + HL * (wid % WPR);  // first of this wave's HL heads
@@ -1505,6 +1509,17 @@ int prefill_waves(int D, int ratio) {
   return env == 8 && (D == 64 || D == 128) && ratio >= 4 && prefill_hl(D, ratio) == 1 && pipe != 1 ? 8 : 4;
 }
 
+int decode_cus() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus < 1)
+      gai_launch_error(__FILE__, __LINE__, "attention: cannot query the CU count");
+    return cus;
+  }();
+  return n;
+}
+
 template <int DD, int HP, typename KV>
 void prefill_launch(const void* q, const void* k_cache, const void* v_cache, const int* block_tables, int max_blocks,
                     const int* tiles, int ntiles, const int* cu_q, const int* ctx_lens, void* out, int Hq, int Hkv,
@@ -1512,6 +1527,23 @@ void prefill_launch(const void* q, const void* k_cache, const void* v_cache, con
                     hipStream_t st) {
   const int lds = 2 * PrefillCfg<DD>::BUF;
   if constexpr (DD == 64 || DD == 128) {
+    // Few tiles: 32 of their 64 rows to a workgroup. A tile is a chain of key tiles, and one wave a SIMD goes down it in 1.6 us
+    // a key tile, two in 2.0; halves also even out the causal lengths. Up to three halves a CU (two are resident): 32 / 8 heads
+    // of 128, a prompt of 17, 66, 187, 600, 1024 tokens 7.1, 10.3, 14.2, 24.9, 38.1 -> 5.9, 6.8, 10.1, 19.7, 30.2 us, 1496 50.6 ->
+    // 44.4, 2000 66.4 -> 60.8, 3000 99.6 -> 93.3; 16 / 4 heads 3000 87.7 -> 75.4. Beyond, the key tiles fetched once for 64 rows
+    // count too: 4000 145.5 | 149.2, 4095 + 6000 (16 / 4) 238.5 | 241.2, 6 x 2300 306 | 301. Equal bits: a row's key tiles and
+    // their order are the same.
+    if constexpr (HP == 4) {
+      if (nwv == 8 && 2 * ntiles * (Hq / HP) <= 3 * decode_cus()) {
+        auto kern = attn_prefill_kernel<DD, HP, KV, 1, false, 4, false, true>;
+        set_max_lds(kern, lds);
+        kern<<<dim3(2 * ntiles, Hq / HP), 256, lds, st>>>((const bf16*)q, (const KV*)k_cache, (const KV*)v_cache, block_tables,
+                                                          max_blocks, tiles, cu_q, ctx_lens, (bf16*)out, Hq, Hkv, scale, causal,
+                                                          lse, k_scale, v_scale, xcd, q_ld);
+        GAI_LAUNCH_CHECK();
+        return;
+      }
+    }
     if (nwv == 8) {  // the staggered loop keeps three tile slots
       auto kern = attn_prefill_kernel<DD, HP, KV, 1, false, 8>;
       set_max_lds(kern, 3 * PrefillCfg<DD>::BUF);
@@ -1636,17 +1668,6 @@ int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D) {
   const int ratio = Hq / Hkv;
   const int hpw = ratio >= 4 ? 4 : ratio >= 2 ? 2 : 1;
   return 32 * (prefill_waves(D, ratio) / (hpw / prefill_hl(D, ratio)));
-}
-
-static int decode_cus() {
-  static const int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus < 1)
-      gai_launch_error(__FILE__, __LINE__, "attn_decode: cannot query the CU count");
-    return cus;
-  }();
-  return n;
 }
 
 void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,

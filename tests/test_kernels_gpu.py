@@ -135,6 +135,27 @@ def test_attention_prefill(cuda, D, Hq, Hkv, causal):
     _close(o, o_ref, 2e-2, 2e-2, "prefill")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv", [(128, 32, 8), (64, 16, 2), (128, 16, 1)])
+def test_attention_prefill_half_tiles(cuda, D, Hq, Hkv):
+    """Few tiles go to the 4-wave kernel in halves of 32 rows, many whole to the 8-wave one: sequences of one short half, one
+    row into the second, whole tiles, chunks over a prefix. A row's sums are the same in both, so the bits are."""
+    torch.manual_seed(19)
+    ctx = [1, 32, 33, 64, 65, 200, 131]
+    qlen = [1, 32, 33, 64, 65, 17, 64]
+    times = 3 * 256 // (2 * Hkv * (Hq // Hkv // 4)) // len(ctx) + 1  # sequences enough for whole tiles
+    kc, vc, bt = _paged_setup(ctx, Hkv, D, cuda, seed=7)
+    q = torch.randn(sum(qlen), Hq, D, device=cuda, dtype=torch.bfloat16)
+    out = []
+    for n in (1, times):
+        cu = torch.tensor([0] + list(torch.tensor(qlen * n).cumsum(0)), dtype=torch.int32)
+        out.append(ops.attention_prefill(q.repeat(n, 1, 1), kc, vc, bt.repeat(n, 1), cu.to(cuda), torch.tensor(ctx * n, dtype=torch.int32, device=cuda),
+                                         D ** -0.5, True, q_lens=qlen * n))
+    assert torch.equal(out[0], out[1][:len(q)]) and torch.equal(out[0], out[1][-len(q):])
+    cu = torch.tensor([0] + list(torch.tensor(qlen).cumsum(0)), dtype=torch.int32)
+    want = ref.attention_prefill(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), cu, torch.tensor(ctx, dtype=torch.int32), D ** -0.5, True)
+    _close(out[0], want, 2e-2, 2e-2, "half tiles")
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (16, 16)])
 def test_attention_prefill_running_max_jumps(cuda, Hq, Hkv):
     """Score scales that jump by far more than the deferred-max threshold between key tiles (keys 64-255 scaled x8,
