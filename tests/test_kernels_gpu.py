@@ -156,6 +156,16 @@ def test_attention_prefill_half_tiles(cuda, D, Hq, Hkv):
     _close(out[0], want, 2e-2, 2e-2, "half tiles")
 
 
+@pytest.mark.parametrize("D", [256, 4096, 8192])
+def test_norm_one_wave_rows(cuda, D):
+    """A wave a workgroup up to 512 rows, four beyond: the same row, the same bits."""
+    torch.manual_seed(20)
+    x, w, b = torch.randn(513, D, device=cuda).bfloat16(), torch.randn(D, device=cuda).bfloat16(), torch.randn(D, device=cuda).bfloat16()
+    four, one = ops.layer_norm(x, w, b, 1e-5), torch.cat([ops.layer_norm(x[:512].clone(), w, b, 1e-5), ops.layer_norm(x[512:].clone(), w, b, 1e-5)])
+    assert torch.equal(four, one)
+    assert torch.equal(ops.rms_norm(x, w, 1e-5)[:512], ops.rms_norm(x[:512].clone(), w, 1e-5))
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (16, 16)])
 def test_attention_prefill_running_max_jumps(cuda, Hq, Hkv):
     """Score scales that jump by far more than the deferred-max threshold between key tiles (keys 64-255 scaled x8,
