@@ -13,7 +13,8 @@
 //    44.0, 6144 x 4096 30.7 -> 23.7, 4096 x 4096 23.3 -> 20.5; 1024 rows 4096 x 4096 41.4 -> 37.5). What is left: a CU holds
 //    about 32 KB of misses (a weight stream of 32 KB in flight per CU is as fast as one of 192 KB: 6.3 TB/s on the chip, 60 KB/us
 //    in one CU), and A's 24 KB a step share them, 0.75 us a step without any products. Four waves of 64 columns each (half the
-//    LDS reads) gave nothing: 57.5 us for the first of the products above;
+//    LDS reads) gave nothing: 57.5 us for the first of the products above; nor did 192 x 64 tiles, which pad 187 rows less but fetch A twice
+//    as often: 4096 x 14336 47.8 | 48.6;
 //  * row-major weights go through LDS beside A, by the same DMA in whole lines: in operand layout a load touches 16 lines for 64 bytes
 //    of each. Row-major, one way -> the other, us: 187 rows 4096 x 14336 61 -> 47, 28672 x 4096 (SwiGLU) 75 -> 65, 448 rows 97 ->
 //    70 and 6144 x 4096 52 -> 36, 512 rows 1024 x 1024 10.5 -> 8.6; the last rows of 18337 x 1024 x 1024 (ORD) 47.5 -> 43.7 in
@@ -43,14 +44,15 @@ namespace {
 constexpr int kBK = 128;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
+constexpr bool epi_bias(int e) {
+  return e == EPI_BIAS || e == EPI_BIAS_GELU || e == EPI_BIAS_RESIDUAL || e == EPI_BIAS_RELU || e == EPI_BIAS_QUICKGELU;
+}
+constexpr bool epi_res(int e) { return e == EPI_RESIDUAL || e == EPI_BIAS_RESIDUAL; }
+
 template <int EPI, bool OUTF32>
-__device__ __forceinline__ void store4(void* C, const bf16* bias, const bf16* R, int ldc, int m, int n, f32x4 v) {
+__device__ __forceinline__ void store4(void* C, bf16x4 b, bf16x4 x, int ldc, int m, int n, f32x4 v) {
   const size_t o = (size_t)m * ldc + n;
-  constexpr bool kBias = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU || EPI == EPI_BIAS_RESIDUAL || EPI == EPI_BIAS_RELU ||
-                         EPI == EPI_BIAS_QUICKGELU;
-  constexpr bool kRes = EPI == EPI_RESIDUAL || EPI == EPI_BIAS_RESIDUAL;
-  if constexpr (kBias) {
-    const bf16x4 b = *reinterpret_cast<const bf16x4*>(bias + n);
+  if constexpr (epi_bias(EPI)) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] += (float)b[r];
   }
@@ -60,8 +62,7 @@ __device__ __forceinline__ void store4(void* C, const bf16* bias, const bf16* R,
     if constexpr (EPI == EPI_BIAS_RELU) v[r] = fmaxf(v[r], 0.f);
     if constexpr (EPI == EPI_BIAS_QUICKGELU) v[r] = quick_gelu(v[r]);
   }
-  if constexpr (kRes) {
-    const bf16x4 x = *reinterpret_cast<const bf16x4*>(R + o);
+  if constexpr (epi_res(EPI)) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = (OUTF32 ? v[r] : (float)(bf16)v[r]) + (float)x[r];
   }
@@ -191,6 +192,20 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
   for (int u = 0; u < DB - 1; ++u)
     if (t + u < n) step(t + u, br[FRAG ? u : 0]);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is left
+  // the epilogue's operands, under way while the sums are exchanged (a wave that another one finishes for has asked in vain):
+  // 187 rows with a residual, a graph's launches: 4096 x 14336 46.4 -> 45.6 us, 4096 x 4096 22.1 -> 21.5, 1024 x 4096 16.2 -> 15.3
+  bf16x4 rb4[epi_bias(EPI) ? FW : 1], rx[epi_res(EPI) ? RW : 1][epi_res(EPI) ? FW : 1];
+  if constexpr (epi_bias(EPI) || epi_res(EPI)) {
+#pragma unroll
+    for (int f = 0; f < FW; ++f) {
+      const int nn = min(n0 + (g * FW + f) * 16, N - 16) + 4 * (lane >> 4);
+      if constexpr (epi_bias(EPI)) rb4[f] = *reinterpret_cast<const bf16x4*>(bias + nn);
+      if constexpr (epi_res(EPI))
+#pragma unroll
+        for (int i = 0; i < RW; ++i)
+          rx[i][f] = *reinterpret_cast<const bf16x4*>(R + (size_t)min(m0 + 16 * (h * RW + i) + (lane & 15), M - 1) * ldc + nn);
+    }
+  }
   f32x4 v[NF];  // [RW][FW]
   if constexpr (ORD) {
 #pragma unroll
@@ -266,11 +281,12 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
       f32x4 y;
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[r] = glu_act<EPI>(v[i * NG][r], v[i * NG + NG - 1][r]);
-      store4<EPI_NONE, OUTF32>(C, nullptr, nullptr, ldc, m, nn / 2 + 4 * (lane >> 4), y);
+      store4<EPI_NONE, OUTF32>(C, bf16x4{}, bf16x4{}, ldc, m, nn / 2 + 4 * (lane >> 4), y);
     } else {
 #pragma unroll
       for (int f = 0; f < FW; ++f)
-        if (nn + 16 * f < N) store4<EPI, OUTF32>(C, bias, R, ldc, m, nn + 16 * f + 4 * (lane >> 4), v[i * FW + f]);
+        if (nn + 16 * f < N) store4<EPI, OUTF32>(C, rb4[epi_bias(EPI) ? f : 0], rx[epi_res(EPI) ? i : 0][epi_res(EPI) ? f : 0], ldc, m,
+                               nn + 16 * f + 4 * (lane >> 4), v[i * FW + f]);
     }
   }
 }
