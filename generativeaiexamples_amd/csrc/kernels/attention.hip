@@ -114,10 +114,10 @@ __device__ __forceinline__ bf16x8 kv_to_bf16(uint2 v, float s) { return fp8x8_to
 // ROWS: keys and values straight from the packed rows that q is in (self-attention of an encoder; kc / vc = the first row's key /
 // value of head 0, q_ld apart), instead of from pages that a kernel before has packed: 61 passages of e5-large 25 + 66 -> 62 us a
 // layer, a question 4.2 + 5.4 -> 5.3. V is turned on its way into LDS: a thread fetches two dims of eight keys, 4 B each
-// (whole lines across the wave), and writes two rows of the V^T image. head_dim 64, a kv head per q head.
+// (whole lines across the wave), and writes two rows of the V^T image. head_dim 64, a kv head per q head. 2: in 128 registers.
 // HALF: a workgroup takes one of the two 32-row halves of a tile of the list (few tiles: see prefill_launch)
-template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4, bool ROWS = false, bool HALF = false>
-__global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) void attn_prefill_kernel(
+template <int D, int HPW, typename KV, int HL = 1, bool PIPE = false, int NWV = 4, int ROWS = 0, bool HALF = false>
+__global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : ROWS == 2 ? 4 : 2) void attn_prefill_kernel(
     const bf16* __restrict__ q, const KV* __restrict__ kc, const KV* __restrict__ vc,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ tiles,
     const int* __restrict__ cu_q, const int* __restrict__ ctx_lens, bf16* __restrict__ out, int Hq, int Hkv,
@@ -162,6 +162,7 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
   const int r0 = qs + 32 * (wid / WPR);  // first q row (within the sequence) of this wave
   const int qrow = r0 + (lane & 31);
   const int qpos = ctx - qlen + qrow;  // absolute position of this lane's query
+  const int klim = (causal ? min(ctx, qpos + 1) : ctx) - 4 * h;  // keys below it (+ 4 h) are seen
   const int* bt = block_tables + (size_t)seq * max_blocks;
 
   // rows covered by the whole workgroup -> number of key tiles
@@ -245,22 +246,31 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
   };
   auto write_k = [&](int buf) { write_k_from(buf, stg); };
   auto write_v = [&](int buf) { write_v_from(buf, stg); };
-  // ROWS: tile kt's rows (past the context its last one: masked, and finite where the rows are)
+  // ROWS: tile kt's rows, from a buffer that begins at its first one and ends with the context: beyond it zeros (masked), and a
+  // lane's offsets are the same for every tile. Clamped rows took ten multiplications at a quarter of the rate and twenty more
+  // instructions of a tile's 240: those 61 passages 68.9 -> 66.2 us, one of 32 tokens 4.13 -> 3.82
   const bf16 *rk = reinterpret_cast<const bf16*>(kc) + (size_t)qbeg * q_ld + g * D,
              *rv = reinterpret_cast<const bf16*>(vc) + (size_t)qbeg * q_ld + g * D;
+  auto rows_at = [&](const bf16* p, int kt) {
+    const int left = ctx - 64 * kt;  // > 0: tiles that are asked for
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(p) + (size_t)(64 * kt) * q_ld, (short)0, ((left - 1) * q_ld + D) * 2,
+                                             0x00020000);
+  };
+  const int ork = (tid / 8 * q_ld + tid % 8 * 8) * 2, orv = (8 * (tid >> 5) * q_ld + 2 * (tid & 31)) * 2;
   auto rows_k = [&](int kt, bf16x8(&dst)[2]) {
+    const __amdgpu_buffer_rsrc_t r = rows_at(rk, kt);
+    int o = ork;
+    if constexpr (ROWS == 2) asm volatile("" : "+v"(o));  // addresses made anew for each tile, not kept: eight registers
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int id = c * NTH + tid;
-      dst[c] = buf_load<bf16x8>(rk, (unsigned)(min(kt * 64 + id / 8, ctx - 1) * q_ld + id % 8 * 8) * 2);
-    }
+    for (int c = 0; c < 2; ++c) dst[c] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, o + c * NTH / 8 * q_ld * 2, 0, 0));
   };
   auto rows_v = [&](int kt, bf16x8(&dst)[2]) {
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(rv), (short)0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r = rows_at(rv, kt);
+    int o = orv;
+    if constexpr (ROWS == 2) asm volatile("" : "+v"(o));
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const unsigned x = __builtin_amdgcn_raw_buffer_load_b32(
-          r, (unsigned)(min(kt * 64 + 8 * (tid >> 5) + e, ctx - 1) * q_ld + 2 * (tid & 31)) * 2, 0, 0);
+      const unsigned x = __builtin_amdgcn_raw_buffer_load_b32(r, o + e * q_ld * 2, 0, 0);
       const bf16x2 y = __builtin_bit_cast(bf16x2, x);
       dst[e >> 2][2 * (e & 3)] = y[0];
       dst[e >> 2][2 * (e & 3) + 1] = y[1];
@@ -352,8 +362,7 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
         for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int key = kt * 64 + 32 * sub + (r & 3) + 8 * (r >> 2) + 4 * h;
-            const bool ok = key < ctx && (!causal || key <= qpos);
+            const bool ok = 32 * sub + (r & 3) + 8 * (r >> 2) < klim - kt * 64;
             const float x = ok ? sc[sub][r] : kNeg;
             sc[sub][r] = x;
             mt = fmaxf(mt, x);
@@ -450,8 +459,7 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
         for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int key = kt * 64 + 32 * sub + (r & 3) + 8 * (r >> 2) + 4 * h;
-            const bool ok = key < ctx && (!causal || key <= qpos);
+            const bool ok = 32 * sub + (r & 3) + 8 * (r >> 2) < klim - kt * 64;
             const float x = ok ? sc[sub][r] : kNeg;
             sc[sub][r] = x;
             mt = fmaxf(mt, x);
@@ -580,7 +588,7 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
     for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
       for (int j = 0; j < HL; ++j) s[j][sub] = f32x16{};
-    if constexpr (QL && D <= 128) {
+    if constexpr (QL && D <= 128 && ROWS != 2) {
       // The first 32-key half's D / 16 K fragments are read together, the second half's one per first-half MFMA:
       // no MFMA waits on its own LDS round trip (left to the compiler, one fragment register was re-used and
       // every QK^T MFMA waited lgkmcnt(0) behind its read)
@@ -652,8 +660,7 @@ __global__ __launch_bounds__(64 * NWV, (D > 128 || HL > 1 || NWV == 8) ? 1 : 2) 
       for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = kt * 64 + 32 * sub + (r & 3) + 8 * (r >> 2) + 4 * h;
-          const bool ok = key < ctx && (!causal || key <= qpos);
+          const bool ok = 32 * sub + (r & 3) + 8 * (r >> 2) < klim - kt * 64;
 #pragma unroll
           for (int j = 0; j < HL; ++j) {
             const float x = ok ? s[j][sub][r] : kNeg;
@@ -1535,7 +1542,7 @@ void prefill_launch(const void* q, const void* k_cache, const void* v_cache, con
     // their order are the same.
     if constexpr (HP == 4) {
       if (nwv == 8 && 2 * ntiles * (Hq / HP) <= 3 * decode_cus()) {
-        auto kern = attn_prefill_kernel<DD, HP, KV, 1, false, 4, false, true>;
+        auto kern = attn_prefill_kernel<DD, HP, KV, 1, false, 4, 0, true>;
         set_max_lds(kern, lds);
         kern<<<dim3(2 * ntiles, Hq / HP), 256, lds, st>>>((const bf16*)q, (const KV*)k_cache, (const KV*)v_cache, block_tables,
                                                           max_blocks, tiles, cu_q, ctx_lens, (bf16*)out, Hq, Hkv, scale, causal,
@@ -1656,9 +1663,13 @@ void gai_attn_rows(const void* qkv, int ld, const int* tiles, int ntiles, const 
   static const int prio_env = getenv("GAI_ATTN_PRIO") ? atoi(getenv("GAI_ATTN_PRIO")) : 2;
   static const bool exact_max = getenv("GAI_ATTN_RESCALE_TH") && atoi(getenv("GAI_ATTN_RESCALE_TH")) == 0;
   const bf16* q = (const bf16*)qkv;
-  auto kern = attn_prefill_kernel<64, 1, bf16, 1, false, 4, true>;
   const int lds = 2 * PrefillCfg<64>::BUF;
-  set_max_lds(kern, lds);
+  // Past three workgroups a CU (143 registers) the kernel in 128, of which four are resident: 16 heads, us, three | four: 61
+  // passages of 117 - 512 tokens 66.2 | 64.6, 16 of 512 36.9 | 32.3, 64 of 30 8.5 | 7.6; one of 32 3.82 | 3.94, one of 300 8.85 | 9.26
+  const bool dense = ntiles * H > 3 * decode_cus();
+  auto kern = dense ? attn_prefill_kernel<64, 1, bf16, 1, false, 4, 2> : attn_prefill_kernel<64, 1, bf16, 1, false, 4, 1>;
+  set_max_lds(attn_prefill_kernel<64, 1, bf16, 1, false, 4, 1>, lds);
+  set_max_lds(attn_prefill_kernel<64, 1, bf16, 1, false, 4, 2>, lds);
   kern<<<dim3(ntiles, H), 256, lds, st>>>(q, q + H * 64, q + 2 * H * 64, nullptr, 0, tiles, cu_q, ctx_lens, (bf16*)out, H, H, scale,
                                           causal, nullptr, 1.f, 1.f, ((prio_env & 3) << 1) | (exact_max ? 8 : 0), ld);
   GAI_LAUNCH_CHECK();

@@ -156,6 +156,26 @@ def test_attention_prefill_half_tiles(cuda, D, Hq, Hkv):
     _close(out[0], want, 2e-2, 2e-2, "half tiles")
 
 
+@pytest.mark.parametrize("lens", [[1, 64, 65, 63], [128, 129, 200], [512, 17]])
+def test_attention_rows_many(cuda, lens):
+    """Past three workgroups a CU the form in fewer registers: the bits of the other one, whose rows fp32 attention bounds (P and
+    the result are rounded to bf16: 2^-8 of the largest value, as the other attention tests). The last sequence ends the buffer."""
+    torch.manual_seed(23)
+    H, out = 16, []
+    qkv = torch.randn(sum(lens), 3 * H * 64, device=cuda, dtype=torch.bfloat16)
+    for n in (1, 3 * 256 // (H * len(lens)) + 2):
+        cu = torch.tensor([0] + list(torch.tensor(lens * n).cumsum(0)), dtype=torch.int32, device=cuda)
+        o = torch.empty(sum(lens) * n, H, 64, device=cuda, dtype=torch.bfloat16)
+        ops.native().attn_rows(qkv.repeat(n, 1), ops.build_prefill_tiles(lens * n, H, H, cuda, head_dim=64), cu,
+                               torch.tensor(lens * n, dtype=torch.int32, device=cuda), o, H, 0.125, False)
+        out.append(o)
+    assert torch.equal(out[0], out[1][:len(qkv)]) and torch.equal(out[0], out[1][-len(qkv):])
+    q, k, v = qkv.float().cpu().view(-1, 3, H, 64).unbind(1)
+    want = torch.cat([torch.nn.functional.scaled_dot_product_attention(*(x[a:a + n].transpose(0, 1) for x in (q, k, v)), scale=0.125).transpose(0, 1)
+                      for a, n in zip([0] + list(torch.tensor(lens).cumsum(0)), lens)])
+    _close(out[0], want, 2e-2, 2e-2, "rows")
+
+
 @pytest.mark.parametrize("D", [256, 4096, 8192])
 def test_norm_one_wave_rows(cuda, D):
     """A wave a workgroup up to 512 rows, four beyond: the same row, the same bits."""
