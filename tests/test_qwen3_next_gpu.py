@@ -233,3 +233,43 @@ def test_qwen3_next_graph_decode_equals_eager(cuda):
             assert eng.stats["graph_steps"] > 0
     assert res[0] == res[1]
     assert not g.slot_of
+
+
+def test_qwen3_next_fragment_weights(cuda):
+    """Weights loaded into fragment order: once, again and drawn anew they are the row-major ones reordered, and prompts from a
+    token to many rows get the row-major model's bits."""
+    pytest.importorskip("transformers")
+    from transformers.models.qwen3_next import Qwen3NextConfig as HFConfig, Qwen3NextForCausalLM
+
+    cfg = Qwen3NextConfig.tiny(hidden_size=512, num_heads=8, intermediate_size=512, num_experts=0, linear_num_value_heads=8)
+    hc = HFConfig(vocab_size=512, hidden_size=512, intermediate_size=512, num_hidden_layers=4, num_attention_heads=8, num_key_value_heads=2,
+                  head_dim=64, linear_num_key_heads=2, linear_num_value_heads=8, linear_key_head_dim=64, linear_value_head_dim=64,
+                  num_experts=0, max_position_embeddings=2048, tie_word_embeddings=False, bos_token_id=1, eos_token_id=2)
+    g, row = Qwen3NextModel(cfg, device=cuda), Qwen3NextModel(cfg, device="cpu")
+
+    def rows():
+        m = Qwen3NextModel(cfg, device=cuda)
+        for k in m.w:
+            m.w[k].copy_(ops.natural_weight(g.w[k]))
+        return m
+
+    for seed in (1, 2):
+        torch.manual_seed(seed)
+        sd = Qwen3NextForCausalLM(hc).state_dict()
+        g.load_hf_state(sd), row.load_hf_state(sd)
+        assert ops.is_frag(g.w["l0.out"]) and ops.is_frag(g.w["l3.o"]) and ops.is_frag(g.w["lm_head"]) and not ops.is_frag(g.w["embed"])
+        for k in row.w:
+            assert torch.equal(ops.natural_weight(g.w[k]).cpu(), row.w[k]), k
+    a = rows()
+    g.random_init(5), a.random_init(5)
+    assert all(torch.equal(ops.natural_weight(g.w[k]), ops.natural_weight(a.w[k])) for k in a.w)
+    a = rows()
+    assert not any(ops.is_frag(t) for t in a.w.values())
+    for n in (1, 9, 90, 700):
+        got = []
+        for m in (g, a):
+            eng = LLMEngine(m, small_byte_tokenizer(512), EngineConfig(num_blocks=64, max_model_len=1024, use_graphs=False))
+            eng.add_request([3 + i % 400 for i in range(n)], SamplingParams(temperature=0.0, max_tokens=1))
+            fb, _ = eng._make_batch(eng.sched.schedule())
+            got.append(m.forward(fb, eng.kv, eng.decode_ws))
+        assert torch.equal(*got), n
