@@ -345,6 +345,33 @@ void attn_rows(const Tensor& qkv, const Tensor& tiles, const Tensor& cu_q, const
                 ctx_lens.data_ptr<int>(), out.data_ptr(), (int)H, (float)scale, causal ? 1 : 0, cur_stream());
 }
 
+// layer_norm(attention over packed rows . W^T + bias + R): sequences of up to 64 rows, W [N, H 64] row-major or in fragment order
+void attn_rows_layernorm(const Tensor& qkv, const Tensor& cu_q, const Tensor& ctx_lens, const Tensor& W, const optional<Tensor>& bias,
+                         const Tensor& R, const Tensor& g, const optional<Tensor>& b, double eps, Tensor& out, Tensor& ws, int64_t H,
+                         double scale, int64_t longest, bool frag) {
+  for (const Tensor* t : {&qkv, &W, &R, &g, static_cast<const Tensor*>(&out)}) check_bf16(*t, "attn_rows_layernorm");
+  if (bias) check_bf16(*bias, "bias");
+  if (b) check_bf16(*b, "b");
+  check_i32(cu_q, "cu_q");
+  check_i32(ctx_lens, "ctx_lens");
+  const int64_t M = qkv.size(0), N = g.numel();
+  const int64_t hg = H > 0 ? gai_attn_rows_heads(H, longest) : 0;
+  TORCH_CHECK(hg > 0 && H / hg <= 8 && N % 64 == 0 && N <= 2048 && M <= 64, "attn_rows_layernorm: shape");
+  TORCH_CHECK(qkv.dim() == 2 && qkv.is_contiguous() && qkv.size(1) == 3 * H * 64, "attn_rows_layernorm: qkv [T, 3 H 64]");
+  TORCH_CHECK(W.is_contiguous() && W.numel() == N * H * 64 && R.is_contiguous() && R.numel() == M * N && out.is_contiguous() &&
+                  out.numel() == M * N && (!bias || bias->numel() == N) && (!b || b->numel() == N),
+              "attn_rows_layernorm: sizes");
+  TORCH_CHECK(cu_q.numel() == ctx_lens.numel() + 1, "attn_rows_layernorm: cu_q");
+  TORCH_CHECK(ws.scalar_type() == at::kFloat && ws.numel() >= H / hg * M * N, "attn_rows_layernorm: workspace");
+  for (const Tensor* t : {&qkv, &W, &R, &g, static_cast<const Tensor*>(&out), static_cast<const Tensor*>(&ws)})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "attn_rows_layernorm: operands on 16 bytes");
+  if (M == 0) return;
+  gai_attn_rows_slabs(qkv.data_ptr(), (int)qkv.size(1), cu_q.data_ptr<int>(), ctx_lens.data_ptr<int>(), ctx_lens.numel(), longest,
+                      W.data_ptr(), ws.data_ptr<float>(), M, N, H, (float)scale, frag ? 1 : 0, cur_stream());
+  gai_slabs_layernorm(ws.data_ptr<float>(), H / hg, opt_ptr(bias), R.data_ptr(), g.data_ptr(), opt_ptr(b), out.data_ptr(), M, N, (float)eps,
+                      cur_stream());
+}
+
 void kv_pack(const Tensor& qkv, const Tensor& blk_tok, const Tensor& blk_n, Tensor& k_cache, Tensor& v_cache,
              int64_t Hq, int64_t Hkv, int64_t D) {
   check_bf16(qkv, "qkv");
@@ -1192,6 +1219,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_rows_per_tile", [](int64_t hq, int64_t hkv, int64_t d) { return gai_attn_prefill_rows_per_tile(hq, hkv, d); },
         py::arg("hq"), py::arg("hkv"), py::arg("d") = 128);
   m.def("attn_rows", &attn_rows);
+  m.def("attn_rows_layernorm", &attn_rows_layernorm);
   m.def("attn_prefill_set_hl", [](int64_t hl) { gai_attn_prefill_set_hl((int)hl); });
   m.attr("DECODE_QUEUE_INTS") = kGaiDecodeQueueInts;
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),

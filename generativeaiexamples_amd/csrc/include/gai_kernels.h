@@ -78,6 +78,11 @@ void gai_attn_prefill(const void* q, const void* k_cache, const void* v_cache, c
                       float v_scale, hipStream_t st, int q_ld = 0);
 void gai_attn_rows(const void* qkv, int ld, const int* tiles, int ntiles, const int* cu_q, const int* ctx_lens, void* out, int H,
                    float scale, int causal, hipStream_t st);
+int gai_attn_rows_heads(int H, int longest);
+void gai_attn_rows_slabs(const void* qkv, int ld, const int* cu_q, const int* ctx_lens, int seqs, int longest, const void* W, float* ws, int M,
+                         int N, int H, float scale, int frag, hipStream_t st);
+void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* R, const void* g, const void* b, void* out, int M, int N,
+                         float eps, hipStream_t st);
 int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D = 128);
 void gai_attn_prefill_set_hl(int hl);
 // Decode QKV tail folded into the decode-attention launch: the split-K QKV partial slabs part[ks][B][n] (n = (Hq +

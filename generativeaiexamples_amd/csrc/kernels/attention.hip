@@ -1675,6 +1675,148 @@ void gai_attn_rows(const void* qkv, int ld, const int* tiles, int ntiles, const 
   GAI_LAUNCH_CHECK();
 }
 
+namespace {
+// Attention of up to 64 rows and its output projection in one launch: a workgroup takes HG heads of a sequence and 64 columns of the
+// projection, whose K slices the heads are, and leaves their sums in slab blockIdx.y for the norm that follows. Up to 64 rows both
+// launches are latency (the projection's 2 MB are a slice of 16 KB a workgroup, on its way while the heads attend), and every
+// workgroup of a head group attends anew, which takes it what one workgroup of attn_prefill_kernel takes. Up to eight sequences
+// (attention_layer_norm_ok): with the norm, 1024 x 1024, us, three launches | two: 16 rows 9.6 | 7.6, 32 9.8 | 8.0, 64 10.9 | 10.3,
+// four sequences of 16 10.7 | 8.0, eight of 8 10.7 | 8.6, but 64 of one row 12.8 | 21.3 (every sequence reads the slices again).
+// A wave takes 32 rows of a head: four heads of up to 32 rows, two of up to 64. The attention's sums are attn_prefill_kernel's.
+template <int HG>
+__global__ __launch_bounds__(256) void attn_rows_slabs_kernel(const bf16* __restrict__ qkv, int ld, const int* __restrict__ cu_q,
+                                                              const int* __restrict__ ctx_lens, const bf16* __restrict__ W,
+                                                              float* __restrict__ ws, int M, int N, int H, float scale, int frag) {
+  using Cfg = PrefillCfg<64>;
+  constexpr int RW = 4 / HG, KS = 2 * HG, OS = HG * 128 + 16;  // waves a head, k32 steps, bytes of a row of the heads' results
+  __shared__ __attribute__((aligned(16))) char sv[HG * Cfg::VBYTES], so[32 * RW * OS];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5;
+  const int hp = blockIdx.y, seq = blockIdx.z, nt = blockIdx.x * 4 + w;  // this wave's 16 columns
+  const int qbeg = cu_q[seq], qlen = min(cu_q[seq + 1] - qbeg, 32 * RW);
+  if (qlen <= 0) return;
+  const int ctx = max(min(ctx_lens[seq], qlen), 0);
+  bf16x8 wf[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+    wf[k] = load8(frag ? W + ((size_t)nt * (2 * H) + KS * hp + k) * 512 + lane * 8
+                       : W + (size_t)(nt * 16 + (lane & 15)) * (H * 64) + (KS * hp + k) * 32 + (lane >> 4) * 8);
+  auto rows = [&](int which, int head, int n) {  // n rows of a head, zeros beyond
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(qkv) + (size_t)qbeg * ld + (which * H + head) * 64, (short)0,
+                                             n > 0 ? ((n - 1) * ld + 64) * 2 : 0, 0x00020000);
+  };
+  // values: two dims of eight keys an item, two items a thread
+  unsigned vr[2][8];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const auto rv = rows(2, HG * hp + (HG == 2 ? j : 2 * j + (w >> 1)), ctx);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      vr[j][e] = __builtin_amdgcn_raw_buffer_load_b32(rv, ((8 * ((tid >> 5) & (4 * RW - 1)) + e) * ld + 2 * (tid & 31)) * 2, 0, 0);
+  }
+  const int head = w / RW, r0 = 32 * (w % RW);  // this wave's head of the group and its 32 rows
+  bf16x8 qf[4], kf[RW][4];
+  {
+    const auto rq = rows(0, HG * hp + head, qlen), rk = rows(1, HG * hp + head, ctx);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      qf[t] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rq, ((r0 + (lane & 31)) * ld + 16 * t + 8 * h) * 2, 0, 0));
+#pragma unroll
+      for (int sub = 0; sub < RW; ++sub)
+        kf[sub][t] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rk, ((32 * sub + (lane & 31)) * ld + 16 * t + 8 * h) * 2, 0, 0));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load is on its way
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        bf16x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = __builtin_bit_cast(bf16x2, vr[j][4 * i + e])[p];
+        *reinterpret_cast<bf16x4*>(sv + (HG == 2 ? j : 2 * j + (w >> 1)) * Cfg::VBYTES +
+                                   v_lds_off<64>(2 * (tid & 31) + p, 2 * ((tid >> 5) & (4 * RW - 1)) + i)) = x;
+      }
+  f32x16 s[2] = {f32x16{}, f32x16{}}, o[2] = {f32x16{}, f32x16{}};
+  float l = 0.f;
+  bf16x8 pf[2 * RW] = {};
+  if (r0 < qlen && ctx > 0) {  // (without a key, the difference of two -1e30 is a rounding of any size)
+#pragma unroll
+    for (int sub = 0; sub < RW; ++sub)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[sub][t], qf[t], s[sub], 0, 0, 0);
+    float m = kNeg;
+    const float sl2 = scale * kLog2e;
+#pragma unroll
+    for (int sub = 0; sub < RW; ++sub)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[sub][r] = 32 * sub + (r & 3) + 8 * (r >> 2) < ctx - 4 * h ? s[sub][r] : kNeg;
+        m = fmaxf(m, s[sub][r]);
+      }
+    m = max_halves(m) * sl2;
+#pragma unroll
+    for (int st = 0; st < 2 * RW; ++st)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float p = fexp2(fmaf(s[st >> 1][8 * (st & 1) + e], sl2, -m));
+        l += p;
+        pf[st][e] = (bf16)p;
+      }
+  }
+  __syncthreads();
+  if (r0 < qlen) {
+#pragma unroll
+    for (int st = 0; st < 2 * RW; ++st)
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) {
+        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(sv + head * Cfg::VBYTES + v_lds_off<64>(32 * dt + (lane & 31), 4 * st + h));
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[st], o[dt], 0, 0, 0);
+      }
+    l = sum_halves(l);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        bf16x4 x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = (bf16)(o[dt][4 * c + r] * inv);
+        *reinterpret_cast<bf16x4*>(so + (r0 + (lane & 31)) * OS + (head * 64 + 32 * dt + 8 * c + 4 * h) * 2) = x;
+      }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2 * RW; ++i) {
+    if (16 * i >= qlen) break;
+    const int row = 16 * i + (lane & 15);
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[k], *reinterpret_cast<const bf16x8*>(so + row * OS + k * 64 + (lane >> 4) * 16), a, 0, 0, 0);
+    if (row < qlen) *reinterpret_cast<f32x4*>(ws + ((size_t)hp * M + qbeg + row) * N + nt * 16 + 4 * (lane >> 4)) = a;
+  }
+}
+}  // namespace
+
+// Heads a workgroup: slabs of the projection = H / that
+int gai_attn_rows_heads(int H, int longest) { return H % 4 == 0 && longest <= 32 ? 4 : H % 2 == 0 && longest <= 64 ? 2 : 0; }
+
+// ws: that many slabs of [M][N]; W row-major or in fragment order (the same bits), N % 64 == 0, no sequence longer than `longest`
+void gai_attn_rows_slabs(const void* qkv, int ld, const int* cu_q, const int* ctx_lens, int seqs, int longest, const void* W, float* ws, int M,
+                         int N, int H, float scale, int frag, hipStream_t st) {
+  if (seqs == 0) return;
+  const int hg = gai_attn_rows_heads(H, longest);
+  if (!hg) gai_launch_error(__FILE__, __LINE__, "attn_rows_slabs: shape");
+  const dim3 grid(N / 64, H / hg, seqs);
+  if (hg == 4)
+    attn_rows_slabs_kernel<4><<<grid, 256, 0, st>>>((const bf16*)qkv, ld, cu_q, ctx_lens, (const bf16*)W, ws, M, N, H, scale, frag);
+  else
+    attn_rows_slabs_kernel<2><<<grid, 256, 0, st>>>((const bf16*)qkv, ld, cu_q, ctx_lens, (const bf16*)W, ws, M, N, H, scale, frag);
+  GAI_LAUNCH_CHECK();
+}
+
 int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D) {
   const int ratio = Hq / Hkv;
   const int hpw = ratio >= 4 ? 4 : ratio >= 2 ? 2 : 1;

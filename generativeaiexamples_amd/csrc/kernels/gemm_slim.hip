@@ -328,10 +328,9 @@ void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, f
   else launch_slim<4, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
 }
 
-void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
-                             void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
-  const int ks = gai_gemm_slim_ks(M, N, K);
-  gai_gemm_slim_partials(A, W, M, N, K, ws, psw, st);
+void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* R, const void* g, const void* b, void* out, int M, int N,
+                         float eps, hipStream_t st) {
+  if (ks < 1 || ks > kMaxSlabs || N > 2048 || N % 8) gai_launch_error(__FILE__, __LINE__, "slabs_layernorm: shape");
 #define GAI_SLN(NCH, KS)                                                                                                 \
   slabs_layernorm_kernel<NCH, KS><<<M, 64, 0, st>>>(ws, ks, M, N, (const bf16*)bias, (const bf16*)R, (const bf16*)g,     \
                                                     (const bf16*)b, (bf16*)out, eps)
@@ -345,4 +344,10 @@ void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, con
 #undef GAI_SLN_K
 #undef GAI_SLN
   GAI_LAUNCH_CHECK();
+}
+
+void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
+                             void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
+  gai_gemm_slim_partials(A, W, M, N, K, ws, psw, st);
+  gai_slabs_layernorm(ws, gai_gemm_slim_ks(M, N, K), bias, R, g, b, out, M, N, eps, st);
 }

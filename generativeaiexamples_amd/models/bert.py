@@ -269,8 +269,12 @@ class BertModel:
         for i in range(c.num_layers):
             p = f"l{i}."
             qkv = ops.linear(h, w[p + "qkv"], bias=w[p + "qkv_b"])
-            a = attn(qkv, self.scale, out=out)
-            h = ops.linear_layer_norm(a, w[p + "o"], w[p + "o_b"], h, w[p + "ln1_w"], w[p + "ln1_b"], c.ln_eps)
+            rest = w[p + "o_b"], h, w[p + "ln1_w"], w[p + "ln1_b"]
+            if attn.direct and not attn.causal and ops.attention_layer_norm_ok(qkv, H, attn.q_lens, w[p + "o"], rest):
+                h = ops.attention_linear_layer_norm(qkv, attn.cu_q, attn.ctx, attn.q_lens, H, self.scale, w[p + "o"], *rest, c.ln_eps)
+            else:
+                a = attn(qkv, self.scale, out=out)
+                h = ops.linear_layer_norm(a, w[p + "o"], w[p + "o_b"], h, w[p + "ln1_w"], w[p + "ln1_b"], c.ln_eps)
             f = ops.linear(h, w[p + "up"], bias=w[p + "up_b"], act="gelu")
             h = ops.linear_layer_norm(f, w[p + "down"], w[p + "down_b"], h, w[p + "ln2_w"], w[p + "ln2_b"], c.ln_eps)
         return h

@@ -200,6 +200,28 @@ def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
     return layer_norm(linear(x, w, bias=bias, residual=residual), ln_w, ln_b, eps)
 
 
+def attention_layer_norm_ok(qkv, heads, q_lens, w, rest) -> bool:
+    """attention_linear_layer_norm takes these rows: a few short questions (figures at attn_rows_slabs_kernel), all of it and of
+    ``rest`` (the residual and vectors) on 16 bytes; the switches of linear_layer_norm hold."""
+    return (qkv.is_cuda and qkv.dtype == torch.bfloat16 and isinstance(w, torch.Tensor) and w.dtype == torch.bfloat16
+            and 0 < qkv.shape[0] <= 64 and len(q_lens) <= 8 and heads % 2 == 0 and heads <= 16 and w.shape[1] == heads * 64
+            and w.shape[0] % 64 == 0 and w.shape[0] <= 2048
+            and (decode_operand(w) is not None or (_SPLITK and _GEMM_FORCE == 0))
+            and all(t is None or t.is_contiguous() and not t.data_ptr() & 15 for t in (qkv, w, decode_operand(w), *rest)))
+
+
+def attention_linear_layer_norm(qkv, cu_q, ctx_lens, q_lens, heads, scale, w, bias, residual, ln_w, ln_b, eps):
+    """layer_norm(linear(self-attention of the packed rows, w, bias, residual)) where attention_layer_norm_ok: the projection's K
+    slices come from the launch that attends."""
+    T, N = qkv.shape[0], w.shape[0]
+    out = torch.empty(T, N, dtype=qkv.dtype, device=qkv.device)
+    ws = torch.empty(heads // 2, T, N, dtype=torch.float32, device=qkv.device)
+    psw = decode_operand(w)
+    native().attn_rows_layernorm(qkv, cu_q, ctx_lens, w if psw is None else psw, bias, residual, ln_w, ln_b, eps, out, ws, heads, scale,
+                                 max(q_lens), psw is not None)
+    return out
+
+
 def _fused_glu_ok(x, w, bias) -> bool:
     """The GEMMs take the GeGLU epilogue: bf16 operands on their tile grid, no bias."""
     return (x.is_cuda and isinstance(w, torch.Tensor) and bias is None and x.dtype == torch.bfloat16

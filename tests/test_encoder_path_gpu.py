@@ -97,3 +97,26 @@ def test_rows_off_16_bytes_take_the_pages(cuda, off):
     assert a.direct and torch.equal(a(qkv, 0.2), a(qkv.clone(), 0.2))
     with pytest.raises(RuntimeError, match="16 bytes"):
         ops.native().attn_rows(qkv, a.tiles, a.cu_q, a.ctx, torch.empty(T, H * 64, device=cuda, dtype=torch.bfloat16), H, 0.2, False)
+
+
+@pytest.mark.parametrize("H,lens", [(16, [1]), (16, [31, 32, 1]), (16, [33, 17]), (16, [64]), (8, [32, 32]), (8, [5, 0, 40]), (16, [8] * 8)])
+def test_attention_layer_norm_short(cuda, H, lens):
+    """Attention, projection and norm of a few short sequences in two launches against the three: the attention has the same
+    bits, the projection's fp32 sums another order, so a rounding of its bf16 result may fall the other way (2^-8 of it, a
+    value of the norm then moves by as much of a standard deviation). Keys past ctx are masked, a sequence without any gives 0."""
+    torch.manual_seed(29)
+    D, T = H * 64, sum(lens)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    W, b, g, lb, res, qkv = bf(D, D) * D ** -0.5, bf(D), bf(D), bf(D), bf(T, D), bf(T, 3 * D)
+    row = W.clone()
+    assert ops.to_fragment_layout_(W)
+    a = PackedAttention(lens, H, 64, cuda)
+    assert ops.attention_layer_norm_ok(qkv, H, a.q_lens, W, (res, b, g, lb))
+    for short in (0, 3):
+        a.ctx.copy_(torch.tensor([max(n - short, 0) for n in lens], dtype=torch.int32))
+        want = ops.linear_layer_norm(a(qkv, 0.125), W, b, res, g, lb, 1e-5).float()
+        got = ops.attention_linear_layer_norm(qkv, a.cu_q, a.ctx, a.q_lens, H, 0.125, W, b, res, g, lb, 1e-5).float()
+        other = ops.attention_linear_layer_norm(qkv, a.cu_q, a.ctx, a.q_lens, H, 0.125, row, b, res, g, lb, 1e-5)
+        assert torch.equal(other.float(), got)  # row-major: the same bits
+        assert ((got - want).abs() <= 2 ** -6 * (1 + want.abs())).all() and (got != want).float().mean() < 0.01
+    assert not ops.attention_layer_norm_ok(qkv, H, [1] * 9, W, ()) and not ops.attention_layer_norm_ok(bf(65, 3 * D), H, [65], W, ())
