@@ -595,7 +595,7 @@ bool splitk_ntw() {
 
 // Waves (of 16 columns) that share a staged slice: eight, or six where that leaves the busiest CU fewer columns. A CU draws weights at
 // 25 - 30 KB/us whatever the others do, so 192 workgroups of eight take what 256 of six take three quarters of. A wave's sums do not
-// depend on it. us, eight | six, fragment order: N 6144, K 4096 at M 64 16.0 | 13.4, at M 23 13.3 | 11.4, at M 8 11.9 | 10.4 (and 17.1, 14.1
+// depend on it. us, eight | six, fragment order: N 6144, K 4096 at M 64 16.5 | 13.4, at M 23 14.5 | 11.4, at M 8 11.9 | 10.4 (and 17.1, 14.1
 // and 12.1 with the slice's rows and columns divided out a 16-byte piece at a time).
 int waves_per_wg(int N, int KS) {
   const int v = splitk_wpg();

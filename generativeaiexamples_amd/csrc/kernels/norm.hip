@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void norm_kernel(const bf16* __restrict__ x, c
 
 // An encoder's first norm: LayerNorm(bf16(bf16(word + position) + type)), the roundings of three additions of bf16 rows, each row read
 // once. As a gather, two additions, another gather and the norm it was five launches and eleven passes over the rows: 9240 tokens of 1024
-// columns 84 -> 19 us, 32 tokens 13 -> 4. Ids outside the table take a row of zeros.
+// columns 50 -> 11.4 us, 18480 74 -> 17, 32 tokens 13 -> 3.4. Ids outside the table take a row of zeros.
 template <int NCH>
 __global__ __launch_bounds__(256) void embed_layernorm_kernel(const int* __restrict__ ids, const int* __restrict__ pos,
                                                               const bf16* __restrict__ word, const bf16* __restrict__ ptab,

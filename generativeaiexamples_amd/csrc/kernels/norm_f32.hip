@@ -770,8 +770,8 @@ namespace {
 // The pass between two parallel layers whose products left K slices (gai_gemm_partials): it adds the slices of a branch up, in order and
 // rounded to bf16 as the product's own reduction does, instead of a launch of its own that writes rows for this one to read. A workgroup
 // a row, four channels a thread, every load (16 slices of each branch) in flight before the first is used; bound by that round trip.
-// 24 rows of 2048, slices of 2 and 11: reduction + norm 4.6 + 6.2 us, here 6.5; the product in front of the first branch 6.1 -> 4.9 in two
-// slices.
+// 24 rows of 2048, slices of 2 and 11: reduction + norm 4.6 + 6.2 us under the profiler, here 7.7; the product in front of the first branch
+// 6.1 -> 4.8 in two slices.
 struct SlabBranch {
   const float* slabs;  // [ks][T][D], or null:
   const bf16* rows;    // rows ld apart, or null: no branch

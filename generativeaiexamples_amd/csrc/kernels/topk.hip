@@ -455,7 +455,7 @@ __global__ __launch_bounds__(256, 1) void sim_group_max(const bf16* __restrict__
 // the stream's own instruction order and sorted. Bound by the fetch of k groups' rows for every query (1.3 MB at k = 40, 1024 columns and
 // 16 rows, for 44 of 300 queries on a CU that has another; a CU alone draws 60 KB/us) and by the latency of the maxima and of three
 // selections of 45 exchanges. 300 queries of 250007 rows of 1024, k = 40: 119 us with keys exchanged through LDS and maxima loaded
-// one after the other, 98 with exchanges on VALU operands and four loads ahead, 62 with groups of 4 rows (a quarter of the fetch, four
+// one after the other, 98 with exchanges on VALU operands and four loads ahead, 56 with groups of 4 rows (a quarter of the fetch, four
 // times the maxima). Whole calls, groups of 16 | 4: 30000 rows, 250 queries, k = 50 87 | 49; 5000 rows, 300, k = 40 77 | 57; 60000, 16,
 // k = 50 49 | 42; but 1M, 1, k = 40 386 | 392 and 100000 x 384, 300, k = 10 68 | 72. Rows by DMA in whole lines instead of operand by
 // operand: k = 40 156 -> 119 us.
@@ -896,7 +896,7 @@ void run_topk_k(const TopkArgs& a) {
 }
 
 // Relevance of euclidean search, 1 - sqrt(max(|q|^2 - 2 s, 0)) / sqrt(2) of the scores s = q . x - |x|^2 / 2: a wave a query, its row in
-// one pass. Bound by its launch (300 queries x 1024, k = 40: 1.2 MB); as torch operations it was eight launches, 20 us.
+// one pass. Bound by its launch (300 queries x 1024, k = 40: 1.2 MB): 2.9 us in a graph; as torch operations it was eight launches, 17.4.
 __global__ __launch_bounds__(64) void l2_relevance_kernel(const float* __restrict__ q, const float* __restrict__ s, int D, int k,
                                                           float* __restrict__ out) {
   const int lane = threadIdx.x;

@@ -8,7 +8,8 @@ Forward over a varlen batch (no padding): word+position+type embedding -> LayerN
 layer: QKV GEMM(+bias) -> bidirectional flash attention straight from the packed QKV rows (or, where
 the rows do not fit that kernel, from transient pages) -> O GEMM with bias+residual fused ->
 LayerNorm (post-LN) -> FFN-up GEMM with bias+GELU fused -> FFN-down GEMM with bias+residual fused
--> LayerNorm; up to 64 tokens the O and down GEMMs leave K slices that the LayerNorm sums. Pooling
+-> LayerNorm; up to 64 tokens the O and down GEMMs leave K slices that the LayerNorm sums (up to eight short
+sequences O's slices come from the launch that attends). Pooling
 (mean / CLS) + L2-normalise in one kernel.
 """
 from __future__ import annotations
