@@ -213,6 +213,10 @@ __global__ __launch_bounds__(256) void moe_router_kernel(const TA* __restrict__ 
         id = oi;
       }
     }
+    if (b < 0.f) {  // no score compares: NaN logits; expert 0 without a weight, as the other routers have it
+      b = NAN;
+      id = 0;
+    }
     if ((id & 63) == lane) score[id] = -2.f;   // taken
     tot += b;
     if (lane == j) {

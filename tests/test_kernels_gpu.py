@@ -944,6 +944,23 @@ def test_moe_router_rows(cuda, T, D, E, k):
         assert w[T - 1].isnan().all()
 
 
+@pytest.mark.parametrize("T,D,E,k", [(1, 4096, 8, 2), (64, 64, 16, 4), (5, 96, 5, 5), (7, 2048, 64, 8), (3, 40, 130, 16), (65, 64, 8, 2), (70, 64, 40, 3)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_moe_router_without_scores(cuda, T, D, E, k, bad):
+    """A row whose scores are NaN gets expert 0 and NaN weights from every router, an id in range; the rows beside it what they get alone."""
+    g = torch.Generator(device=cuda).manual_seed(E)
+    W = torch.randn(E, D, device=cuda, generator=g).bfloat16()
+    x = (torch.randn(T, D, device=cuda, generator=g) * D ** -0.5).bfloat16()
+    want, wts = ops.moe_router(x, W, E, k)
+    x[T // 2] = bad
+    ids, w = ops.moe_router(x, W, E, k)
+    rest = torch.arange(T, device=cuda) != T // 2
+    assert (ids[T // 2] == 0).all() and w[T // 2].isnan().all()
+    assert torch.equal(ids[rest], want[rest]) and torch.equal(w[rest], wts[rest])
+    ids, w = ops.moe_route(x.float() @ W.float().t(), k)
+    assert (ids[T // 2] == 0).all() and w[T // 2].isnan().all()
+
+
 @pytest.mark.parametrize("T,D", [(1, 8), (5, 64), (33, 512), (3, 520), (300, 1024), (9, 1032), (7, 2048), (4, 2056), (0, 64)])
 def test_embed_layer_norm(cuda, T, D):
     """The rows of separate gathers, additions and norm, bit for bit: ids outside the table (a row of zeros), the last position; past
