@@ -41,13 +41,17 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(const bf16* __restrict__ q
 
 // The same for a prompt's tokens and bf16 pages, with an optional RMS norm of every q and k head (weights wq / wk, rounded to bf16 before
 // the rotation). Bound by one read and one write of the rows; what kept it from that was V^T, whose elements went out two bytes at a time,
-// 32 bytes apart (a page row is one channel of 16 tokens). Here a workgroup takes TOK tokens and either four heads of q and k - 16-byte
-// loads and stores, all four heads' rows in flight, the token's angles read once for them - or one head of v, turned in LDS: eight tokens
-// that fill half a page row go out as 16 bytes, others a token's neighbours side by side. Us, before | here: 10095 tokens of 16 + 4 + 4
-// heads of 128 49.7 | 30.7, 3389 of 32 + 8 + 8 34.8 | 21.0, 999 14.8 | 7.6, 187 4.3 | 3.8, 66 to 100 alike; 3000 of 3 x 16 of 64 27.8 | 10.3. With
-// the norm, which was copies of the heads, two norm launches and copies back, 10095 tokens 147 | 27.3 (under the profiler).
+// 32 bytes apart (a page row is one channel of 16 tokens). Here a workgroup takes four heads of q and k of TOK tokens - 16-byte loads and stores,
+// all four heads' rows in flight, the token's angles read once for them - or one head of v of half as many, 16 bytes a thread, turned in LDS:
+// eight tokens that fill half a page row go out as 16 bytes, others (a prompt that begins anywhere in the packed rows, tokens in pages of
+// their own) a token's neighbours side by side, all at once: one after the other they took 400 tokens in pages of their own to 7.2 us for 6.3.
+// Us, rope_kv_kernel | here | here, prompts that begin off a half page: 10095 tokens of 16 + 4 + 4 heads of 128 39.4 | 24.2 | 25.5, 3389 of 32 + 8 + 8
+// 28.9 | 14.5 | 15.5, 999 12.1 | 5.2 | 5.8, 187 4.1 | 3.2 | 3.2; 3000 of 3 x 16 of 64 22.8 | 7.3 | 8.9. With the norm, which was copies of the heads, two
+// norm launches and copies back, 10095 tokens 119 | 23.9.
 template <int D>
-constexpr int rows_tokens() { return 256 / (D / 16) / 8 * 8; }
+constexpr int value_tokens() { return 256 / (D / 8) / 8 * 8; }  // 16 bytes a thread
+template <int D>
+constexpr int rows_tokens() { return 2 * value_tokens<D>(); }
 constexpr int kHeadsAWg = 4;
 
 template <int D, bool NORM>
@@ -56,12 +60,11 @@ __global__ __launch_bounds__(256) void rope_kv_rows_kernel(const bf16* __restric
                                                            bf16* __restrict__ q_out, bf16* __restrict__ k_cache,
                                                            bf16* __restrict__ v_cache, int T, int Hq, int Hkv, int rope,
                                                            const bf16* __restrict__ wq, const bf16* __restrict__ wk, float eps) {
-  constexpr int LP = D / 16, TOK = rows_tokens<D>(), GROUPS = TOK / 8;
-  __shared__ __attribute__((aligned(16))) bf16 vs[TOK][D + 8];
-  __shared__ int whole[GROUPS];
-  const int tid = threadIdx.x, t0 = blockIdx.x * TOK, H = Hq + 2 * Hkv, qk = (Hq + Hkv + kHeadsAWg - 1) / kHeadsAWg;
+  constexpr int LP = D / 16, TOK = rows_tokens<D>(), LV = D / 8, TV = value_tokens<D>();
+  __shared__ __attribute__((aligned(16))) bf16 vs[TV][D + 8];
+  const int tid = threadIdx.x, H = Hq + 2 * Hkv, qk = (Hq + Hkv + kHeadsAWg - 1) / kHeadsAWg;
   if ((int)blockIdx.y < qk) {
-    const int t = t0 + tid / LP, i0 = tid % LP * 8;
+    const int t = blockIdx.x * TOK + tid / LP, i0 = tid % LP * 8;
     if (tid >= TOK * LP || t >= T) return;
     const int h0 = blockIdx.y * kHeadsAWg, hn = min(kHeadsAWg, Hq + Hkv - h0), slot = slots[t];
     const bf16* src = qkv + ((size_t)t * H + h0) * D + i0;
@@ -119,33 +122,29 @@ __global__ __launch_bounds__(256) void rope_kv_rows_kernel(const bf16* __restric
     }
     return;
   }
-  const int g = blockIdx.y - qk;
-  for (int p = tid; p < TOK * (D / 8); p += 256) {
-    const int r = p / (D / 8), col = p % (D / 8) * 8;
-    *reinterpret_cast<bf16x8*>(&vs[r][col]) = load8(qkv + ((size_t)min(t0 + r, T - 1) * H + Hq + Hkv + g) * D + col);
-  }
-  if (tid < GROUPS) {  // eight tokens side by side in one half of a page
-    const int t = t0 + 8 * tid;
-    int ok = t + 7 < T && slots[min(t, T - 1)] >= 0 && slots[min(t, T - 1)] % 8 == 0;
-    for (int i = 1; i < 8; ++i) ok &= slots[min(t + i, T - 1)] == slots[min(t, T - 1)] + i;
-    whole[tid] = ok;
-  }
+  // an eight of tokens: rows r & ~7 on, D threads, j the one of them
+  const int y = blockIdx.y - qk, g = y >> 1, r = tid / LV, col = tid % LV * 8, t = (2 * blockIdx.x + (y & 1)) * TV + r;
+  const int r8 = r & ~7, tg = t - (r & 7), j = tid - r8 * LV, tj = tg + (j & 7);
+  const bf16x8 x = load8(qkv + ((size_t)min(t, T - 1) * H + Hq + Hkv + g) * D + col);
+  const int slot = slots[min(tj, T - 1)];
+  int s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s[i] = slots[min(tg + i, T - 1)];
+  if (r < TV) *reinterpret_cast<bf16x8*>(&vs[r][col]) = x;
   __syncthreads();
-  for (int e = tid; e < D * GROUPS; e += 256) {
-    const int p = e % GROUPS, d = e / GROUPS;
-    if (!whole[p]) continue;
-    const int slot = slots[t0 + 8 * p];
+  if (r >= TV) return;
+  bool whole = tg + 7 < T && s[0] >= 0 && s[0] % 8 == 0;  // side by side in one half of a page
+#pragma unroll
+  for (int i = 1; i < 8; ++i) whole &= s[i] == s[0] + i;
+  if (whole) {  // a channel a thread
     bf16x8 o;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = vs[8 * p + i][d];
-    store8(v_cache + (((size_t)(slot / kKvBlock) * Hkv + g) * D + d) * kKvBlock + slot % kKvBlock, o);
-  }
-  for (int p = 0; p < GROUPS; ++p) {
-    if (whole[p]) continue;
-    const int t = t0 + 8 * p + (tid & 7), slot = t < T ? slots[t] : -1;
-    if (slot < 0) continue;
+    for (int i = 0; i < 8; ++i) o[i] = vs[r8 + i][j];
+    store8(v_cache + (((size_t)(s[0] / kKvBlock) * Hkv + g) * D + j) * kKvBlock + s[0] % kKvBlock, o);
+  } else if (tj < T && slot >= 0) {  // eight channels of a token, its neighbours' beside them
     bf16* dst = v_cache + ((size_t)(slot / kKvBlock) * Hkv + g) * D * kKvBlock + slot % kKvBlock;
-    for (int d = tid >> 3; d < D; d += 32) dst[(size_t)d * kKvBlock] = vs[8 * p + (tid & 7)][d];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[(j / 8 + i * LV) * kKvBlock] = vs[r8 + (j & 7)][j / 8 + i * LV];
   }
 }
 
@@ -209,9 +208,12 @@ void gai_kv_pack(const void* qkv, int ld, int koff, int voff, const int* blk_tok
   gai_launch_error(__FILE__, __LINE__, "kv_pack: head_dim must be 64, 96, 128 or 256");
 }
 
-namespace {
-constexpr int kRowsFrom = 65;  // decode-sized steps: four times the workgroups
-}
+// Steps that take rope_kv_rows_kernel. Decode-sized and small ones are a launch and one chain of loads, and rope_kv_kernel has four times the
+// workgroups for that; what it pays for is values (two bytes a store), about four times a query's elements. Us, that kernel | this one, tokens
+// in order / each in a page of its own: 65 x (32 + 8 + 8) x 128 3.25 | 3.01 / 3.31 | 3.51, 100 of those 3.47 | 3.02 / 3.64 | 3.71; 65 x (16 + 16 + 16) x 128
+// 3.81 | 2.95 / 4.11 | 3.75; (16 + 4 + 4) x 128, 100 2.90 | 2.97 / 2.94 | 3.26, 187 3.41 | 3.05 / 3.55 | 3.54; (8 + 1 + 1) x 256, 187 3.01 | 3.08 / 2.93 | 3.32,
+// 400 3.35 | 3.26 / 3.54 | 3.78; (14 + 2 + 2) x 64, 400 3.01 | 3.02 / 3.04 | 3.27, 1000 3.73 | 3.17.
+static bool rope_rows(int T, int Hq, int Hkv, int D) { return T > 64 && (long)T * (Hq + 4 * Hkv) * D >= 9 << 16; }
 
 int gai_rope_kv_norm_ok(int D) { return D == 64 || D == 128 || D == 256; }
 
@@ -222,7 +224,7 @@ void gai_rope_kv_rows(const void* qkv, const int* pos, const float* cos_sin, con
   if ((wq == nullptr) != (wk == nullptr) || (wq && !gai_rope_kv_norm_ok(D)))
     gai_launch_error(__FILE__, __LINE__, "rope_kv: head norms need both weights and head_dim 64, 128 or 256");
 #define GAI_ROWS(DD, N)                                                                                                              \
-  rope_kv_rows_kernel<DD, N><<<dim3((T + rows_tokens<DD>() - 1) / rows_tokens<DD>(), (Hq + Hkv + kHeadsAWg - 1) / kHeadsAWg + Hkv), \
+  rope_kv_rows_kernel<DD, N><<<dim3((T + rows_tokens<DD>() - 1) / rows_tokens<DD>(), (Hq + Hkv + kHeadsAWg - 1) / kHeadsAWg + 2 * Hkv), \
                                256, 0, st>>>((const bf16*)qkv, pos, cos_sin, slots, (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, T, \
                                              Hq, Hkv, rope, (const bf16*)wq, (const bf16*)wk, eps)
   if (D == 64) { if (wq) GAI_ROWS(64, true); else GAI_ROWS(64, false); }
@@ -239,7 +241,7 @@ void gai_rope_kv_write(const void* qkv, const int* pos, const float* cos_sin, co
                        float k_scale, float v_scale, hipStream_t st) {
   if (T == 0) return;
   const bool on16 = (((size_t)qkv | (size_t)q_out | (size_t)k_cache | (size_t)v_cache) & 15) == 0;
-  if (T >= kRowsFrom && !kv_fp8 && on16 && D % 32 == 0 && D <= 256)
+  if (rope_rows(T, Hq, Hkv, D) && !kv_fp8 && on16 && D % 32 == 0 && D <= 256)
     return gai_rope_kv_rows(qkv, pos, cos_sin, slots, q_out, k_cache, v_cache, T, Hq, Hkv, D, rope, nullptr, nullptr, 0.f, st);
   const long items = (long)T * (Hq + 2 * Hkv);
   const float iks = 1.f / k_scale, ivs = 1.f / v_scale;

@@ -920,6 +920,33 @@ def test_rope_kv_rows(cuda, D, Hq, Hkv, lens, skip):
         assert ((x.float() - y.float()).norm() <= 2.0 ** -9 * y.float().norm())
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,lens,shift", [(128, 32, 8, [72], 0), (128, 32, 8, [5, 80, 1, 9, 40], 0), (128, 16, 4, [1] * 144, 0), (64, 3, 2, [838], 5),
+                                                 (64, 12, 12, [17, 137], 0), (256, 5, 1, [253, 11], 0), (96, 7, 3, [204, 120], 0), (96, 0, 3, [512], 7)])
+def test_rope_kv_rows_from(cuda, D, Hq, Hkv, lens, shift):
+    """Steps at the line from which the kernel for many rows runs, and a token below it: the bits of 64 tokens at a time. Prompts that begin
+    anywhere in the packed rows or in their pages, tokens in pages of their own or in none, a last eight that the rows end in."""
+    g = torch.Generator(device=cuda).manual_seed(sum(lens) + D)
+    pos, slots, n = _scattered([x + shift for x in lens], g, ())
+    pos, slots = pos[shift:], slots[shift:]
+    slots[40::211] = -1
+    H = Hq + 2 * Hkv
+    line = -(-(9 << 16) // ((Hq + 4 * Hkv) * D))
+    cs = torch.randn(2048, D, device=cuda, generator=g)
+    for T in sorted({min(line - 1, pos.numel()), min(line, pos.numel()), pos.numel()}):
+        qkv = torch.randn(T, H * D, device=cuda, generator=g).bfloat16()
+
+        def run(step):
+            q = torch.full((T, Hq, D), 7.0, device=cuda, dtype=torch.bfloat16)
+            kc, vc = torch.full((n, Hkv, 16, D), 7.0, device=cuda).bfloat16(), torch.full((n, Hkv, D, 16), 7.0, device=cuda).bfloat16()
+            for a in range(0, T, step):
+                b = min(T, a + step)
+                ops.rope_kv_write(qkv[a:b], pos[a:b].contiguous(), cs, slots[a:b].contiguous(), q[a:b], kc, vc, Hq, Hkv, D)
+            return q, kc, vc
+
+        for got, want in zip(run(T), run(64)):
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("T,D,E,k", [(65, 32, 1, 1), (80, 96, 5, 5), (200, 4096, 8, 2), (1003, 1056, 16, 4), (97, 64, 3, 2), (66, 2080, 16, 16)])
 def test_moe_router_rows(cuda, T, D, E, k):
     """Prompt-sized router against 64 bits: the same experts wherever two scores are further apart than the sums' error, softmax
