@@ -1296,6 +1296,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("custom_all_to_all", &custom_all_to_all);
   m.def("gemm_qkv_partials", &gemm_qkv_partials);
   m.def("gemm_partials", &gemm_partials);
+  m.def("gemm_splitk_waves", [](int64_t N, int64_t KS) { return gai_gemm_splitk_waves(N, KS); });
   m.def("gemm_partials_ks", [](int64_t M, int64_t N, int64_t K) { return gai_gemm_partials_ks(M, N, K); });
   m.def("gemv", &gemv, pybind11::arg("x"), pybind11::arg("gamma"), pybind11::arg("eps"), pybind11::arg("W"),
         pybind11::arg("epi"), pybind11::arg("out"), pybind11::arg("res"), pybind11::arg("frag") = false,

@@ -104,6 +104,7 @@ void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, co
                      float v_scale, hipStream_t st, int* split_cnt = nullptr,
                      const GaiQkvFold* fold = nullptr, bool queue = false);
 int gai_gemm_partials_ks(int M, int N, int K);
+int gai_gemm_splitk_waves(int N, int KS);  // of a workgroup of the split-K products that stage their slice
 void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st);
 // QKV partial slabs only (for GaiQkvFold): KS (2..8) when launched, 0 when the shape runs elsewhere.
 int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st);

@@ -474,10 +474,12 @@ namespace {
 
 // Waves per workgroup of the slice-staging kernel: every workgroup stages its activation K-slice once,
 // so 8 waves (128 columns) halve the activation bytes per weight byte of 4 waves (64 columns).
-int splitk_wpg() {
-  static const int v = getenv("GAI_SPLITK_WPG") ? atoi(getenv("GAI_SPLITK_WPG")) : 8;
-  return v == 4 ? 4 : 8;
+// GAI_SPLITK_WPG asks for 4, or (any other value) 8, for every shape.
+int asked_wpg() {
+  static const int v = getenv("GAI_SPLITK_WPG") ? (atoi(getenv("GAI_SPLITK_WPG")) == 4 ? 4 : 8) : 0;
+  return v;
 }
+int splitk_wpg() { return asked_wpg() ? asked_wpg() : 8; }
 
 // Legacy (whole-slice staging) K-split: the grid reaches ~2 workgroups per CU while the slice fits LDS.
 int legacy_ks(int M, int N, int K) {
@@ -598,8 +600,7 @@ bool splitk_ntw() {
 // depend on it. us, eight | six, fragment order: N 6144, K 4096 at M 64 16.5 | 13.4, at M 23 14.5 | 11.4, at M 8 11.9 | 10.4 (and 17.1, 14.1
 // and 12.1 with the slice's rows and columns divided out a 16-byte piece at a time).
 int waves_per_wg(int N, int KS) {
-  const int v = splitk_wpg();
-  if (v != 8) return v;
+  if (asked_wpg()) return asked_wpg();
   auto busiest = [&](int w) { return ((N + 16 * w - 1) / (16 * w) * KS + 255) / 256 * w; };
   return busiest(6) < busiest(8) ? 6 : 8;
 }
@@ -938,6 +939,8 @@ int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, flo
     launch_partials(A, B, M, N, K, KS, ws, psw, st);
   return KS;
 }
+
+int gai_gemm_splitk_waves(int N, int KS) { return waves_per_wg(N, KS); }
 
 // The K slices of a product, fp32 [ks][M][N], for a kernel that adds them up itself; ks from gai_gemm_partials_ks (0: the product has none).
 int gai_gemm_partials_ks(int M, int N, int K) {

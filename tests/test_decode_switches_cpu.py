@@ -1,5 +1,9 @@
-"""The environment switches of the decode attention, read in Python and by the launcher: both have to choose the same kernel."""
+"""The environment switches of the decode kernels: of the attention, read in Python and by the launcher (both have to choose the same
+kernel), and of the split-K products."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -16,3 +20,16 @@ def test_default_kernel_as_the_launcher_reads_it(monkeypatch, nt, variant):
     atoi = ctypes.CDLL(None).atoi
     want = (nt is None or atoi(nt.encode()) != 0) and (variant is None or atoi(variant.encode()) == 1)
     assert ops._decode_default() == want
+
+
+@pytest.mark.skipif(not ops.native_available(), reason="the kernels are not built")
+@pytest.mark.parametrize("asked,want", [(None, [6, 8, 6]), ("8", [8, 8, 8]), ("4", [4, 4, 4]), ("6", [8, 8, 8])])
+def test_split_k_waves_as_asked(asked, want):
+    """GAI_SPLITK_WPG is what every shape gets, also where the rule would choose six waves. (Read once a process.)"""
+    env = {k: v for k, v in os.environ.items() if k != "GAI_SPLITK_WPG"}
+    if asked is not None:
+        env["GAI_SPLITK_WPG"] = asked
+    code = "from generativeaiexamples_amd import ops; print([ops.native().gemm_splitk_waves(*s) for s in ((6144, 4), (4096, 8), (128, 2))])"
+    p = subprocess.run([sys.executable, "-c", code], env=env, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0 and p.stdout.split("\n")[0] == str(want), p.stdout + p.stderr
