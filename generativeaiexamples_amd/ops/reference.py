@@ -384,11 +384,6 @@ def decode_advance(toks, ids, pos, ctx, slots, bt, n_valid, block):
     slots[:n] = (bt[rows, p // block].long() * block + p % block).to(slots.dtype)
 
 
-def embed_layer_norm(ids, pos, word, ptab, type_row, w, b, eps):
-    h = embedding(ids, word) + ptab[pos.long()]
-    return layer_norm(h + type_row, w, b, eps, None)
-
-
 def pool(h, cu_seqlens, mode="mean", normalize=True, lens=None):
     cu = cu_seqlens.tolist()
     n = None if lens is None else lens.tolist()

@@ -210,12 +210,14 @@ def test_parallel_add_norm_kept_groups(D):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,D,K", [(1, 512, 512), (24, 2048, 5632), (24, 2048, 2048), (64, 2048, 11264), (17, 1040, 4096), (3, 16, 1024),
-                                   (33, 1024, 5120), (65, 2048, 2048), (5, 2064, 5632)])
-def test_branches_as_k_slices(cuda, T, D, K):
+@pytest.mark.parametrize("T,D,K,form", [(1, 512, 512, "rows"), (24, 2048, 5632, "split"), (24, 2048, 2048, "cut"), (64, 2048, 11264, "split"),
+                                        (17, 1040, 4096, "cut"), (3, 16, 1024, "cut"), (33, 1024, 5120, "split"), (65, 2048, 2048, "rows"),
+                                        (5, 2064, 5632, "rows")])
+def test_branches_as_k_slices(cuda, T, D, K, form):
     """A branch handed over as its product's K slices: the rows that adding them in order and rounding once gives (the stream's bits),
-    normed alike up to the order of the squares' sum, in either branch, beside rows or alone, with and without bias and scale. Past 64
-    rows or 2048 channels, and where a product is one pass, linear_partial gives rows."""
+    normed alike up to the order of the squares' sum, in either branch, beside rows or alone, with and without bias and scale. "split": the
+    product has these slices by itself, and gives these bits; "cut": it is one pass over K, which is cut here; "rows" (more than 64, or 2048
+    channels, or too little K): the product."""
     g = torch.Generator(device=cuda).manual_seed(T + D + K)
     rn = lambda *s: torch.randn(*s, device=cuda, generator=g)  # noqa: E731
     x, w, bias = rn(T, K).bfloat16(), (rn(D, K) * K ** -0.5).bfloat16(), rn(D).bfloat16()
@@ -227,14 +229,15 @@ def test_branches_as_k_slices(cuda, T, D, K):
         for b in (None, bias):
             p = ops.linear_partial(x, wt, b)
             want = ops.linear(x, wt, b)
-            if not isinstance(p, ops.Partial):
+            assert isinstance(p, ops.Partial) == (form != "rows")
+            if form == "rows":
                 assert torch.equal(p, want)
                 continue
-            assert T <= 64 and D <= 2048
             rows = torch.zeros(T, D, device=cuda)
             for s in p.slabs:
                 rows = rows + s
             rows = (rows if b is None else rows + b.float()).bfloat16()
+            assert len(p.slabs) > 1 and (form == "cut" or torch.equal(rows, want))
             exact = x.double() @ w.double().t() + (0 if b is None else b.double())
             # K products of unit normals and weights of K^-1/2: fp32 sums, then one rounding to bf16
             assert ((rows.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 2.0 ** -18 * K ** 0.5).all()
