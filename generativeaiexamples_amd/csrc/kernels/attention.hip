@@ -1538,8 +1538,10 @@ void prefill_launch(const void* q, const void* k_cache, const void* v_cache, con
     // a key tile, two in 2.0; halves also even out the causal lengths. Up to three halves a CU (two are resident): 32 / 8 heads
     // of 128, a prompt of 17, 66, 187, 600, 1024 tokens 7.1, 10.3, 14.2, 24.9, 38.1 -> 5.9, 6.8, 10.1, 19.7, 30.2 us, 1496 50.6 ->
     // 44.4, 2000 66.4 -> 60.8, 3000 99.6 -> 93.3; 16 / 4 heads 3000 87.7 -> 75.4. Beyond, the key tiles fetched once for 64 rows
-    // count too: 4000 145.5 | 149.2, 4095 + 6000 (16 / 4) 238.5 | 241.2, 6 x 2300 306 | 301. Equal bits: a row's key tiles and
-    // their order are the same.
+    // count too: 4000 145.5 | 149.2, 4095 + 6000 (16 / 4) 238.5 | 241.2, 6 x 2300 306 | 301. Chunks over a prefix, whose keys both halves
+    // fetch: 64 rows behind 2000 63.9 -> 49.5, behind 30000 784 -> 634, 1024 behind 8000 248 -> 209. Heads of 64 and fp8 pages alike (0.71 -
+    // 0.91 of whole tiles); nothing at the upper end: 32 / 8 heads of 64, 1500 tokens 34.2 | 34.0, 64 / 8 of 128, 1024 behind 8000 300 | 301. Equal
+    // bits: a row's key tiles and their order are the same.
     if constexpr (HP == 4) {
       if (nwv == 8 && 2 * ntiles * (Hq / HP) <= 3 * decode_cus()) {
         auto kern = attn_prefill_kernel<DD, HP, KV, 1, false, 4, 0, true>;

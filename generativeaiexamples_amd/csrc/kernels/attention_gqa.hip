@@ -256,7 +256,8 @@ __global__ __launch_bounds__(64) void gqa_split_kernel(GqaArgs a) {
   // while the one before is used, its values while it is scored; keys and values of both, 128 channels: 28.5 us where this takes 27.1
   // (64 streams). Up to 192 + 128 channels: wider heads' keys do not fit the registers twice (192: 26.9 -> 27.1 us, 256: 36 -> 54) and are
   // asked for with the block's values. Us, chain -> ahead, with the merge: 24 streams of 1000 keys (16 heads of 128 on 4) 20.1 -> 16.6, 64
-  // of 1024 27.2 -> 27.1, 64 of 8000 198 -> 182, 16 x 4 tokens of 2000 53.6 -> 39.1, 8 of 30000 99.5 -> 89.5.
+  // of 1024 27.2 -> 27.1, 64 of 8000 198 -> 182, 16 x 4 tokens of 2000 53.6 -> 39.1, 8 of 30000 99.5 -> 89.5. A share of few blocks has little to
+  // gain: 64 of 200 keys on 8 heads 16.7 -> 17.1; heads of 256 (pages ahead only) 24 of 1000 15.7 -> 16.2, 64 of 3000 78.2 -> 77.9, one of 30000 78 -> 57.
   constexpr bool AHEAD = DK + DV <= 320;
   bf16x8 kf[AHEAD ? 2 : 1][DK / 16], vf[2][DV / 32];
   int pg[2][2];

@@ -597,8 +597,9 @@ bool splitk_ntw() {
 
 // Waves (of 16 columns) that share a staged slice: eight, or six where that leaves the busiest CU fewer columns. A CU draws weights at
 // 25 - 30 KB/us whatever the others do, so 192 workgroups of eight take what 256 of six take three quarters of. A wave's sums do not
-// depend on it. us, eight | six, fragment order: N 6144, K 4096 at M 64 16.5 | 13.4, at M 23 14.5 | 11.4, at M 8 11.9 | 10.4 (and 17.1, 14.1
-// and 12.1 with the slice's rows and columns divided out a 16-byte piece at a time).
+// depend on it. us, eight | six, with their sum, weights from HBM: N 6144, K 4096 in fragment order at M 64 20.1 | 17.4, at M 23 16.3 | 13.6, at
+// M 8 14.1 | 12.6, row-major 19.5 | 18.4, 16.0 | 15.0, 15.5 | 14.6; 5120 and 4608 x 4096 0.87 - 0.90 of eight at every M, 3072 x 3072 0.93 - 0.99, 2560 and
+// 1024 x 4096 0.93 - 1.00, with rotation and cache write 3072 x 2048 0.90 - 0.96 and 1152 x 1024 0.94 - 0.96.
 int waves_per_wg(int N, int KS) {
   if (asked_wpg()) return asked_wpg();
   auto busiest = [&](int w) { return ((N + 16 * w - 1) / (16 * w) * KS + 255) / 256 * w; };

@@ -86,9 +86,11 @@ __global__ void moe_route_kernel(const float* __restrict__ logits, int T, int E,
 
 // Prompt-sized steps of up to 16 experts, bf16: router product, softmax and top-k in one launch. A workgroup takes 16 tokens, its eight
 // waves a share of D each, on matrix cores (products of bf16 are exact, sums fp32; the shares are added in order), then a thread a token
-// does what moe_route_kernel does. Bound by the latency of one read of the rows: a wave has 16 steps of them in flight, which is all of
-// its share at 4096. 3389 tokens x 4096, 8 experts: as the upcast of rows and weights, an fp32 library product and moe_route_kernel four
-// launches, 40 us; here 12.7, about half of it the rows, 16 x 64 bytes a load.
+// does what moe_route_kernel does. Bound by the latency of one read of the rows: from D 4096 on a wave has 16 steps of them in flight, which
+// is all of its share there; narrower rows go through the loop behind them. As the upcast of rows and
+// weights, an fp32 library product and moe_route_kernel it was four launches. 8 experts, us, those | here: D 4096, 65 tokens 22.3 | 10.4, 1024
+// 33.3 | 11.0, 3389 40.2 | 11.4, 8192 64.7 | 17.6 (about half of it the rows, 16 x 64 bytes a load); D 2048, 65 20.3 | 7.6, 3389 34.8 | 9.1; D 512, 65
+// 23.0 | 5.6. 4 or 16 experts and D to 8192 alike: 0.22 - 0.55 of the four.
 __global__ __launch_bounds__(512) void moe_router_rows_kernel(const bf16* __restrict__ x, int ldx, const bf16* __restrict__ W, int T,
                                                               int D, int E, int k, float eps, int* __restrict__ ids,
                                                               float* __restrict__ w) {

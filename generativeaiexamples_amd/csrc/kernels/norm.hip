@@ -160,8 +160,9 @@ __global__ __launch_bounds__(256) void embed_layernorm_kernel(const int* __restr
 template <bool LN>
 void dispatch_norm(const void* x, const void* rin, void* rout, const void* w, const void* b, void* out, int T,
                    int D, float eps, hipStream_t st) {
-  // Up to two rows a CU a workgroup is one wave: a CU draws 25 - 30 KB/us, and four rows of 4096 are 32 KB. Rows of 4096, RMS:
-  // 17 of them 4.66 -> 4.11 us, 187 5.33 -> 4.63, 400 5.57 -> 5.12; 1024 rows of 8192 four 11.4, one 11.9
+  // Up to two rows a CU a workgroup is one wave: a CU draws 25 - 30 KB/us, and four rows of 4096 are 32 KB. Us, four waves | one, RMS:
+  // rows of 4096, 32 of them 4.8 | 4.3, 256 5.1 | 4.5, 512 5.7 | 5.35; of 8192, 512 9.3 | 8.9; of 1024, 32 2.50 | 2.29, 512 2.64 | 2.62; of 384, 8 2.29 | 2.35,
+  // 512 2.32 | 2.30. LayerNorm of 4096, 32 6.0 | 5.2; of 1024, 512 2.99 | 3.00. 1024 rows of 8192, RMS, 11.4 | 11.9
   const int wv = T <= 512 ? 1 : 4;
   const dim3 grid((T + wv - 1) / wv), block(64 * wv);
   const int nch = (D + 511) / 512;

@@ -935,16 +935,16 @@ def test_rope_kv_rows_from(cuda, D, Hq, Hkv, lens, shift):
     for T in sorted({min(line - 1, pos.numel()), min(line, pos.numel()), pos.numel()}):
         qkv = torch.randn(T, H * D, device=cuda, generator=g).bfloat16()
 
-        def run(step):
+        def run(step, rope):
             q = torch.full((T, Hq, D), 7.0, device=cuda, dtype=torch.bfloat16)
             kc, vc = torch.full((n, Hkv, 16, D), 7.0, device=cuda).bfloat16(), torch.full((n, Hkv, D, 16), 7.0, device=cuda).bfloat16()
             for a in range(0, T, step):
                 b = min(T, a + step)
-                ops.rope_kv_write(qkv[a:b], pos[a:b].contiguous(), cs, slots[a:b].contiguous(), q[a:b], kc, vc, Hq, Hkv, D)
+                ops.rope_kv_write(qkv[a:b], pos[a:b].contiguous(), cs, slots[a:b].contiguous(), q[a:b], kc, vc, Hq, Hkv, D, rope)
             return q, kc, vc
 
-        for got, want in zip(run(T), run(64)):
-            assert torch.equal(got, want)
+        for rope in (True, False):
+            assert all(torch.equal(x, y) for x, y in zip(run(T, rope), run(64, rope)))
 
 
 @pytest.mark.parametrize("T,D,E,k", [(65, 32, 1, 1), (80, 96, 5, 5), (200, 4096, 8, 2), (1003, 1056, 16, 4), (97, 64, 3, 2), (66, 2080, 16, 16)])
