@@ -1078,8 +1078,9 @@ def moe_router(x: torch.Tensor, W: torch.Tensor, E: int, k: int, eps: float = 0.
     = chosen scores / (their sum + eps)). W [>= E, D] (rows past E: padding). One launch for decode-sized steps, and for any
     with up to 16 experts in bf16; the router GEMM and moe_route otherwise. Logits are fp32 either way."""
     T = x.shape[0]
-    if not x.is_cuda or (T > 64 and not (x.dtype == W.dtype == torch.bfloat16 and native().moe_router_rows_ok(x.shape[1], E)
-                                         and x.stride(1) == 1 and x.stride(0) % 8 == 0 and not (x.data_ptr() | W.data_ptr()) & 15)):
+    if not x.is_cuda or is_frag(W) or (T > 64 and not (
+            x.dtype == W.dtype == torch.bfloat16 and native().moe_router_rows_ok(x.shape[1], E) and W.is_contiguous()
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and not (x.data_ptr() | W.data_ptr()) & 15)):
         return moe_route(linear(x, W, out_dtype=torch.float32)[:, :E], k, eps=eps)
     ids = torch.empty(T, k, dtype=torch.int32, device=x.device)
     w = torch.empty(T, k, dtype=torch.float32, device=x.device)

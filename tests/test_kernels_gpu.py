@@ -988,6 +988,23 @@ def test_moe_router_without_scores(cuda, T, D, E, k, bad):
     assert (ids[T // 2] == 0).all() and w[T // 2].isnan().all()
 
 
+@pytest.mark.parametrize("T", [5, 64, 65, 200])
+def test_moe_router_weight_layouts(cuda, T):
+    """Router weights in fragment order, or (past 64 rows) rows of a wider buffer: the row-major ones' experts. (512 exact products of unit
+    normals and weights of 512^-1/2, summed in fp32: scores to far less than 2^-10.)"""
+    torch.manual_seed(T)
+    W, x = (torch.randn(64, 512, device=cuda) * 512 ** -0.5).bfloat16(), torch.randn(T, 512, device=cuda).bfloat16()
+    p = (x.double() @ W[:9].double().t()).softmax(-1)
+    wide = torch.empty(9, 520, device=cuda, dtype=torch.bfloat16)[:, :512].copy_(W[:9])
+    frag = W.clone()
+    assert ops.to_fragment_layout_(frag)
+    for w in (W, frag) + ((wide,) if T > 64 else ()):
+        ids, wts = ops.moe_router(x, w, 9, 2)
+        got = torch.gather(p, 1, ids.long())
+        assert ((got - p.topk(2).values).abs() <= 2.0 ** -10).all()
+        assert ((wts.double() - got / got.sum(-1, keepdim=True)).abs() <= 2.0 ** -10).all()
+
+
 @pytest.mark.parametrize("T,D", [(1, 8), (5, 64), (33, 512), (3, 520), (300, 1024), (9, 1032), (7, 2048), (4, 2056), (0, 64)])
 def test_embed_layer_norm(cuda, T, D):
     """The rows of separate gathers, additions and norm, bit for bit: ids outside the table (a row of zeros), the last position; past
