@@ -1268,11 +1268,11 @@ POOL_MODES = {"mean": 0, "cls": 1, "last": 2}
 
 
 def pool(h, cu_seqlens, mode: str = "mean", normalize: bool = True, lens=None):
-    """Sentence vectors of packed rows; ``lens`` [B] int32: sequence b is the first lens[b] of its rows (padded batches)."""
+    """Sentence vectors of packed rows; ``lens`` [B], whole numbers: sequence b is the first lens[b] of its rows (padded batches)."""
     if not h.is_cuda:
         return ref.pool(h, cu_seqlens, mode, normalize, lens)
     out = torch.empty(cu_seqlens.numel() - 1, h.shape[-1], dtype=torch.float32, device=h.device)
-    native().pool(h, cu_seqlens, out, POOL_MODES[mode], normalize, lens)
+    native().pool(h, cu_seqlens, out, POOL_MODES[mode], normalize, None if lens is None else lens.int().contiguous())
     return out
 
 

@@ -1035,6 +1035,8 @@ def test_pool_padded(cuda, mode, L, lens, D):
         got = ops.pool(h.view(-1, D), cu, mode, normalize, ln)
         want = ref.pool(h.view(-1, D).cpu(), cu.cpu(), mode, normalize, ln.cpu())
         _close(got, want, 1e-5, 1e-5, "padded pool")
+        for other in (ln.long(), torch.stack([ln, ln], 1)[:, 0]):
+            assert torch.equal(ops.pool(h.view(-1, D), cu, mode, normalize, other), got)
 
 
 @pytest.mark.parametrize("D,lens", [(1024, [303, 1, 0, 65]), (384, [512, 7]), (64, [1000, 129, 128]), (8, [2000]), (8192, [3, 9]),
