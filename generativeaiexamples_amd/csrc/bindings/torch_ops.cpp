@@ -286,6 +286,45 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
            (int)force, cur_stream(), bfrag ? 1 : 0);
 }
 
+// The parts of a product of 65 to 640 rows as slabs, and the norm that adds them: rms (g; res += the product, in place) or
+// layer (g, b; res is only read). False, and nothing launched, where the product has no such plan, an operand is not on 16 bytes
+// or there is no memory for the slabs.
+bool slabs_plan(int64_t M, int64_t N, int64_t K, bool layer, GaiMidPlan* plan) {
+  return layer ? gai_slabs_layernorm_ok(1, N) && gai_gemm_mid_slabs_plan(M, N, K, 8, plan) : N >= 2048 && gai_gemm_mid_slabs_plan(M, N, K, 16, plan);
+}
+
+bool linear_slabs_norm(const Tensor& A, const Tensor& W, const optional<Tensor>& bias, Tensor& res, const Tensor& g,
+                       const optional<Tensor>& b, bool layer, double eps, Tensor& out, bool bfrag) {
+  for (const Tensor* t : {&A, &W, &g, static_cast<const Tensor*>(&res), static_cast<const Tensor*>(&out)}) check_bf16(*t, "linear_slabs_norm");
+  if (bias) check_bf16(*bias, "bias");
+  if (b) check_bf16(*b, "b");
+  const int64_t K = A.size(-1), M = A.numel() / K, N = W.size(0);
+  TORCH_CHECK(W.dim() == 2 && W.size(1) == K && res.numel() == M * N && out.numel() == M * N && g.numel() == N &&
+                  (!bias || bias->numel() == N) && (!b || b->numel() == N), "linear_slabs_norm: sizes");
+  GaiMidPlan plan;
+  if (!slabs_plan(M, N, K, layer, &plan)) return false;
+  uintptr_t at = 0;
+  for (const Tensor* t : {&A, &W, &g, static_cast<const Tensor*>(&res), static_cast<const Tensor*>(&out)})
+    at |= reinterpret_cast<uintptr_t>(t->data_ptr());
+  if (bias) at |= reinterpret_cast<uintptr_t>(bias->data_ptr());
+  if (b) at |= reinterpret_cast<uintptr_t>(b->data_ptr());
+  if (at & 15) return false;
+  Tensor ws;
+  try {
+    ws = at::empty({plan.parts, M, N}, A.options().dtype(at::kFloat));
+  } catch (const c10::OutOfMemoryError&) {
+    return false;
+  }
+  gai_gemm_mid_slabs(A.data_ptr(), W.data_ptr(), M, N, K, plan, ws.data_ptr<float>(), cur_stream(), bfrag ? 1 : 0);
+  if (layer)
+    gai_slabs_layernorm(ws.data_ptr<float>(), plan.parts, opt_ptr(bias), res.data_ptr(), g.data_ptr(), opt_ptr(b), out.data_ptr(), M, N,
+                        (float)eps, cur_stream());
+  else
+    gai_slabs_add_rmsnorm(ws.data_ptr<float>(), plan.parts, opt_ptr(bias), res.data_ptr(), g.data_ptr(), out.data_ptr(), M, N,
+                          (float)eps, cur_stream());
+  return true;
+}
+
 // rows at the end of gemm's product that the mid-size kernel computes (all, some or none), for the tests of that rule
 int64_t gemm_mid_rows(const Tensor& A, const Tensor& B, const Tensor& C, const optional<Tensor>& bias,
                       const optional<Tensor>& R, int64_t epi, bool bfrag) {
@@ -1199,6 +1238,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_slim_nf", &gai_gemm_slim_nf);
   m.def("gemm_slim_ks", &gai_gemm_slim_ks);
   m.def("linear_layernorm", &linear_layernorm);
+  m.def("linear_slabs_norm", &linear_slabs_norm);
+  m.def("gemm_slabs_parts", [](int64_t M, int64_t N, int64_t K, bool layer) {
+    GaiMidPlan plan;
+    return slabs_plan(M, N, K, layer, &plan) ? plan.parts : 0;
+  });
   m.def("gemm", &gemm, pybind11::arg("A"), pybind11::arg("B"), pybind11::arg("C"), pybind11::arg("bias"),
         pybind11::arg("R"), pybind11::arg("epi"), pybind11::arg("force"), pybind11::arg("bfrag") = false);
   m.def("gemm_fp8", &gemm_fp8);

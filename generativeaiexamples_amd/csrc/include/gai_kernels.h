@@ -81,6 +81,7 @@ void gai_attn_rows(const void* qkv, int ld, const int* tiles, int ntiles, const 
 int gai_attn_rows_heads(int H, int longest);
 void gai_attn_rows_slabs(const void* qkv, int ld, const int* cu_q, const int* ctx_lens, int seqs, int longest, const void* W, float* ws, int M,
                          int N, int H, float scale, int frag, hipStream_t st);
+bool gai_slabs_layernorm_ok(int ks, int N);
 void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* R, const void* g, const void* b, void* out, int M, int N,
                          float eps, hipStream_t st);
 int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D = 128);
@@ -223,6 +224,14 @@ void gai_ipc_free(void* p);
 void gai_ipc_get_handle(void* p, char* handle64);
 void* gai_ipc_open(const char* handle64);
 void gai_ipc_close(void* p);
+
+// the sums of fp32 slabs [KS][M][N] of a product (+ bias), rounded to bf16, with what follows it: res += them, out = rmsnorm(res) * g
+// (N % 8 == 0, N <= 8192); rotation and the write of queries and cached rows (0: not this head size)
+void gai_slabs_add_rmsnorm(const float* ws, int KS, const void* bias, void* res, const void* g, void* out, int M, int N, float eps,
+                           hipStream_t st);
+int gai_slabs_rope_kv(const float* ws, int KS, const void* bias, const int* pos, const float* cos_sin, const int* slots, void* q_out,
+                      void* k_cache, void* v_cache, int M, int Hq, int Hkv, int D, int kv_fp8, float k_scale, float v_scale,
+                      hipStream_t st);
 
 // gemm_splitk.hip fused decode tail (TP = 1): res = bf16(bf16(A.W^T + bias) + res); out = rmsnorm(res) * g
 int gai_gemm_splitk_fusable_norm(int M, int N, int K);

@@ -230,6 +230,19 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_kernel(const bf16* __restrict
       v[e] = h ? y + v[e] : v[e] + y;  // first half + second half
     }
   }
+  if constexpr (!ORD && EPI == EPI_NONE && !OUTF32) {
+    if (ws && !cnt) {  // slabs [part][M][N] for the launch that adds them
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const int m = m0 + 16 * (h * RW + i) + (lane & 15);
+        float* d = ws + ((size_t)part * M + m) * N + n0 + g * FW * 16 + 4 * (lane >> 4);
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+          if (m < M && n0 + (g * FW + f) * 16 < N) *reinterpret_cast<f32x4*>(d + 16 * f) = v[i * FW + f];
+      }
+      return;
+    }
+  }
   if (!ORD && S > 1) {
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(ws, (short)0, 0x7fffffff, 0x00020000);
     auto woff = [&](int p, int e) {
@@ -503,6 +516,59 @@ int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* b
   const double round = 6.0 + K / 64 * 1.42 + (R ? 9.0 : 0.0);
   const double saved = round - plan->cost * 1.15 - 3.0;
   return saved > 0.05 * round * ((tiles + G - 1) / G) ? m2 : 0;
+}
+
+// Where a norm follows, its launch can add the parts: the last workgroup of a tile no longer reads all of them by itself (a CU
+// takes in 40 - 60 KB/us: eight parts of 192 x 128 are 15 us), so more parts pay, and K is cut where the rows of A would be fetched for
+// few columns. Product and norm, fragment order, us, before | here: 187 rows 4096 x 14336 49.5 | 40.6, 4096 x 4096 25.5 | 21.6, 256 rows 54.2 | 47.0
+// and 26.2 | 22.4, 96 rows 38.6 | 31.6 and 21.8 | 17.2, 640 rows 97.0 | 94.2 and 45.6 | 40.7.
+// The model: 3336 timings of 200 products (65 to 640 rows, N 2048 to 8192, K 2048 to 14336), nine in ten within 13 %; over the 156 that
+// the rule takes product and norm are on average 15 % faster, one is slower (400 x 2048 x 2048: 15.9 -> 18.4). At 1000 rows the slabs' bytes
+// cost more than the sums did (46.4 | 48.2, 126.9 | 131.2).
+namespace {
+struct SlabFit {
+  double base, alone, full, weights, few, slabs, round;  // as MidFit; slabs: GB/s / 1000 written; round: each past the first
+};
+constexpr SlabFit kSlabFit[3] = {{2.9, 0.54, 0.64, 4.66, 0.31, 2.8, 0.43}, {4.7, 0.77, 1.0, 5.75, 0.39, 4.24, 2.97}, {6.8, 1.0, 1.23, 4.65, 1.0, 4.0, 5.25}};
+constexpr double kSlabRead = 0.141, kSlabRows = 0.78e-6;  // the norm: us a MB of slabs, an element of the rows past 256
+constexpr double kSlabMargin = 0.95;
+
+double slabs_cost(int M, int N, int K, int v, int S) {
+  const SlabFit& f = kSlabFit[v];
+  const int items = mid_tiles(M, N, v == 2 ? 12 : 8, v == 0 ? 1 : 2) * S, G = mid_cus(), rounds = (items + G - 1) / G;
+  const int steps = (K / kBK + S - 1) / S;
+  const double fill = std::min(1.0, (double)items / G), mb = (double)S * M * N * 4 / 1e6;
+  return f.base + std::max(rounds * steps * (f.alone + (f.full - f.alone) * fill), (double)N * K * 2 / 1e6 / (f.weights * (f.few + (1 - f.few) * fill))) +
+         mb / f.slabs + f.round * (rounds - 1) + kSlabRead * mb + kSlabRows * std::max(0, M - 256) * N;
+}
+}  // namespace
+
+bool gai_gemm_mid_slabs_plan(int M, int N, int K, int most, GaiMidPlan* plan) {
+  if (M <= 64 || M > 640 || N < 256 || N > 8192 || N % 16 || K % kBK || (long long)N * K * 2 >= 1ll << 31) return false;
+  double one = 1e30, more = 1e30;
+  for (int v = 0; v < 3; ++v)
+    for (int S = 1; S <= std::min(most, 16) && K / kBK / S >= 3; ++S) {
+      if ((long long)S * M * N * 4 >= 1ll << 31) break;
+      const double c = slabs_cost(M, N, K, v, S);
+      if (S == 1) {
+        one = std::min(one, c);
+      } else if (c < more) {
+        more = c;
+        *plan = {v == 2 ? 12 : 8, v == 0 ? 1 : 2, S, 0, c};
+      }
+    }
+  return more < kSlabMargin * one;
+}
+
+void gai_gemm_mid_slabs(const void* A, const void* B, int M, int N, int K, const GaiMidPlan& p, float* ws, hipStream_t st, int bfrag) {
+#define GAI_MID_SLABS(MT, NG)   \
+  if (p.mt == MT && p.ng == NG) \
+    return launch_mid<MT, NG, EPI_NONE, false>(A, B, nullptr, nullptr, nullptr, M, N, K, N, p.parts, ws, nullptr, st, bfrag);
+  GAI_MID_SLABS(8, 1)
+  GAI_MID_SLABS(8, 2)
+  GAI_MID_SLABS(12, 2)
+#undef GAI_MID_SLABS
+  gai_launch_error(__FILE__, __LINE__, "gemm_mid: no kernel for this plan");
 }
 
 void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K, int ldc, int epi,

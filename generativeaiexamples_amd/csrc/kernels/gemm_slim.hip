@@ -328,9 +328,11 @@ void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, f
   else launch_slim<4, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
 }
 
+bool gai_slabs_layernorm_ok(int ks, int N) { return ks >= 1 && ks <= kMaxSlabs && N <= 2048 && N % 8 == 0; }
+
 void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* R, const void* g, const void* b, void* out, int M, int N,
                          float eps, hipStream_t st) {
-  if (ks < 1 || ks > kMaxSlabs || N > 2048 || N % 8) gai_launch_error(__FILE__, __LINE__, "slabs_layernorm: shape");
+  if (!gai_slabs_layernorm_ok(ks, N)) gai_launch_error(__FILE__, __LINE__, "slabs_layernorm: shape");
 #define GAI_SLN(NCH, KS)                                                                                                 \
   slabs_layernorm_kernel<NCH, KS><<<M, 64, 0, st>>>(ws, ks, M, N, (const bf16*)bias, (const bf16*)R, (const bf16*)g,     \
                                                     (const bf16*)b, (bf16*)out, eps)

@@ -756,22 +756,8 @@ int gai_gemm_splitk_fusable_norm(int M, int N, int K) {
   return M >= 1 && M <= 64 && N % 8 == 0 && N <= 256 * 8 * 4 && gai_gemm_splitk_ks(M, N, K) > 1;
 }
 
-void gai_gemm_splitk_add_rmsnorm(const void* A, const void* B, const void* bias, void* res, const void* g, void* out,
-                                 int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
-  if (M == 0) return;
-  if (!gai_gemm_splitk_fusable_norm(M, N, K)) gai_launch_error(__FILE__, __LINE__, "gemm_splitk_add_rmsnorm: shape");
-  if (gai_gemm_dec2_ok(M, N, K, bias ? EPI_BIAS : EPI_NONE)) {
-    // decode GEMM into a bf16 scratch h (the workspace), then the residual-add RMSNorm kernel:
-    // res = bf16(h + res), out = rmsnorm(res) * g - the same roundings as the fused tail
-    bf16* h = reinterpret_cast<bf16*>(ws);
-    gai_gemm_dec2(A, B, h, bias, nullptr, M, N, K, N, bias ? EPI_BIAS : EPI_NONE, 0, st, psw);
-    gai_rmsnorm(h, res, res, g, out, M, N, eps, st);
-    return;
-  }
-  // deep K (down): LDS-staged decode kernel writing K-split slabs
-  const int ks2 = gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw);
-  const int KS = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
-  if (!ks2) launch_partials(A, B, M, N, K, KS, ws, psw, st);
+void gai_slabs_add_rmsnorm(const float* ws, int KS, const void* bias, void* res, const void* g, void* out, int M, int N, float eps,
+                           hipStream_t st) {
   if (N <= 4096 && N % 4 == 0 && getenv("GAI_NORM_TAIL_256") == nullptr) {
 #define GAI_W4(KC)                                                                                              \
     splitk_add_rmsnorm_w4_kernel<KC><<<M, 1024, 0, st>>>(ws, KS, M, N, (const bf16*)bias, (bf16*)res,          \
@@ -794,6 +780,25 @@ void gai_gemm_splitk_add_rmsnorm(const void* A, const void* B, const void* bias,
   GAI_FN(3)
   GAI_FN(4)
 #undef GAI_FN
+}
+
+void gai_gemm_splitk_add_rmsnorm(const void* A, const void* B, const void* bias, void* res, const void* g, void* out,
+                                 int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
+  if (M == 0) return;
+  if (!gai_gemm_splitk_fusable_norm(M, N, K)) gai_launch_error(__FILE__, __LINE__, "gemm_splitk_add_rmsnorm: shape");
+  if (gai_gemm_dec2_ok(M, N, K, bias ? EPI_BIAS : EPI_NONE)) {
+    // decode GEMM into a bf16 scratch h (the workspace), then the residual-add RMSNorm kernel:
+    // res = bf16(h + res), out = rmsnorm(res) * g - the same roundings as the fused tail
+    bf16* h = reinterpret_cast<bf16*>(ws);
+    gai_gemm_dec2(A, B, h, bias, nullptr, M, N, K, N, bias ? EPI_BIAS : EPI_NONE, 0, st, psw);
+    gai_rmsnorm(h, res, res, g, out, M, N, eps, st);
+    return;
+  }
+  // deep K (down): LDS-staged decode kernel writing K-split slabs
+  const int ks2 = gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw);
+  const int KS = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
+  if (!ks2) launch_partials(A, B, M, N, K, KS, ws, psw, st);
+  gai_slabs_add_rmsnorm(ws, KS, bias, res, g, out, M, N, eps, st);
 }
 
 namespace {
@@ -872,27 +877,10 @@ bool launch_rope_tail(const void* A, const void* B, int M, int N, int K, float* 
 
 }  // namespace
 
-int gai_gemm_splitk_rope_kv(const void* A, const void* B, const void* bias, const int* pos, const float* cos_sin,
-                            const int* slots, void* q_out, void* k_cache, void* v_cache, int M, int Hq, int Hkv,
-                            int D, int kv_fp8, float k_scale, float v_scale, float* ws, int psw, hipStream_t st,
-                            int K, int* tail_cnt) {
+int gai_slabs_rope_kv(const float* ws, int KS, const void* bias, const int* pos, const float* cos_sin, const int* slots, void* q_out,
+                      void* k_cache, void* v_cache, int M, int Hq, int Hkv, int D, int kv_fp8, float k_scale, float v_scale,
+                      hipStream_t st) {
   const int N = (Hq + 2 * Hkv) * D;
-  if (M < 1 || M > 64 || (D != 64 && D != 128 && D != 256) || N % 16) return 0;
-  if (gai_gemm_dec2_ok(M, N, K, bias ? EPI_BIAS : EPI_NONE)) return 0;  // single-pass kernel owns it
-  const int ks2 = gai_gemm_dec2_partials_ks(M, N, K);
-  if (tail_cnt != nullptr && D == 128 && !ks2) {
-    const RopeTail t{tail_cnt, (const bf16*)bias, pos, cos_sin, slots, (bf16*)q_out, k_cache, v_cache, Hq, Hkv,
-                     1.f / k_scale, 1.f / v_scale};
-    if (kv_fp8 ? launch_rope_tail<fp8>(A, B, M, N, K, ws, psw, t, st)
-               : launch_rope_tail<bf16>(A, B, M, N, K, ws, psw, t, st))
-      return 1;
-  }
-  const int KS = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
-  if (KS <= 1) return 0;
-  if (ks2)
-    gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw);
-  else
-    launch_partials(A, B, M, N, K, KS, ws, psw, st);
   const long items = (long)M * (Hq + 2 * Hkv);
   const float iks = 1.f / k_scale, ivs = 1.f / v_scale;
 #define GAI_SRK(DD)                                                                                               \
@@ -923,6 +911,30 @@ int gai_gemm_splitk_rope_kv(const void* A, const void* B, const void* bias, cons
   GAI_SRK(256)
 #undef GAI_SRK
   return 0;
+}
+
+int gai_gemm_splitk_rope_kv(const void* A, const void* B, const void* bias, const int* pos, const float* cos_sin,
+                            const int* slots, void* q_out, void* k_cache, void* v_cache, int M, int Hq, int Hkv,
+                            int D, int kv_fp8, float k_scale, float v_scale, float* ws, int psw, hipStream_t st,
+                            int K, int* tail_cnt) {
+  const int N = (Hq + 2 * Hkv) * D;
+  if (M < 1 || M > 64 || (D != 64 && D != 128 && D != 256) || N % 16) return 0;
+  if (gai_gemm_dec2_ok(M, N, K, bias ? EPI_BIAS : EPI_NONE)) return 0;  // single-pass kernel owns it
+  const int ks2 = gai_gemm_dec2_partials_ks(M, N, K);
+  if (tail_cnt != nullptr && D == 128 && !ks2) {
+    const RopeTail t{tail_cnt, (const bf16*)bias, pos, cos_sin, slots, (bf16*)q_out, k_cache, v_cache, Hq, Hkv,
+                     1.f / k_scale, 1.f / v_scale};
+    if (kv_fp8 ? launch_rope_tail<fp8>(A, B, M, N, K, ws, psw, t, st)
+               : launch_rope_tail<bf16>(A, B, M, N, K, ws, psw, t, st))
+      return 1;
+  }
+  const int KS = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
+  if (KS <= 1) return 0;
+  if (ks2)
+    gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw);
+  else
+    launch_partials(A, B, M, N, K, KS, ws, psw, st);
+  return gai_slabs_rope_kv(ws, KS, bias, pos, cos_sin, slots, q_out, k_cache, v_cache, M, Hq, Hkv, D, kv_fp8, k_scale, v_scale, st);
 }
 
 int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st) {

@@ -638,6 +638,8 @@ class LlamaModel:
         # one fewer [T, d] read and write per norm (a 16K-token chunk: 134 MB each)
         res_epi = (res.is_cuda and ctx.tp_size == 1 and not fuse and not self.lora_names
                    and os.environ.get("GAI_RES_EPI", "1") == "1")
+        # up to a few hundred rows the parts of K that such a product is cut into are added in the norm's launch
+        fuse = fuse or (res_epi and c.norm != "layernorm" and os.environ.get("GAI_FUSE_NORM", "1") == "1")
         for i in range(c.num_layers):
             p = f"l{i}."
             if xn is not None:

@@ -257,8 +257,7 @@ class MixtralModel(LlamaModel):
                 ops.attention_decode(q[P:], kc, vc, fb.decode_block_tables, fb.decode_ctx, self.scale, ws=decode_ws,
                                      max_ctx=fb.max_decode_ctx, out=attn[P:])
             if res_epi:
-                ops.linear(attn.view(T, -1), w[p + "o"], residual=res, out=res)
-                x = ops.rms_norm(res, w[p + "mlp_norm"], c.rms_eps)
+                x = ops.linear_add_rmsnorm(attn.view(T, -1), w[p + "o"], res, w[p + "mlp_norm"], c.rms_eps)
                 res = self.moe_mlp(x, i, res)
                 continue
             h = ops.linear(attn.view(T, -1), w[p + "o"])

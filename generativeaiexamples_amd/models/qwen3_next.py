@@ -440,6 +440,7 @@ class Qwen3NextModel:
         extra["decode_slots"][n:].fill_(self.pad_slot)
 
     # ------------------------------------------------------------------ blocks
+    # a mixer returns its rows and the weight of its output projection, which the next norm's operation applies
     def _full_attention(self, x, i, fb, kv, decode_ws, T, P):
         c, w, p = self.cfg, self.w, f"l{i}."
         hd = c.head_dim
@@ -456,7 +457,7 @@ class Qwen3NextModel:
         if T > P:
             ops.attention_decode(q[P:], kc, vc, fb.decode_block_tables, fb.decode_ctx, self.scale, ws=decode_ws,
                                  max_ctx=fb.max_decode_ctx, out=attn[P:])
-        return ops.linear(ops.act_mul(gate, attn.view(T, -1), "sigmoid"), w[p + "o"])
+        return ops.act_mul(gate, attn.view(T, -1), "sigmoid"), w[p + "o"]
 
     @property
     def _gdn_kernels(self) -> bool:
@@ -481,7 +482,7 @@ class Qwen3NextModel:
                            extra["slots"][: len(fb.prefill_qlen)], ss, core[:P])
         if T > P:
             ops.native().gdn_decode(q[P:], k[P:], v[P:], g[P:], beta[P:], ss, extra["decode_slots"][: T - P], core[P:])
-        return ops.linear(ops.gdn_out(core, proj[:, cd:cd + vd], w[p + "gnorm"], c.rms_eps), w[p + "out"])
+        return ops.gdn_out(core, proj[:, cd:cd + vd], w[p + "gnorm"], c.rms_eps), w[p + "out"]
 
     def _linear_attention(self, x, i, fb, T, P):
         c, w, p = self.cfg, self.w, f"l{i}."
@@ -544,12 +545,12 @@ class Qwen3NextModel:
         y = core * torch.rsqrt(core.pow(2).mean(-1, keepdim=True) + c.rms_eps)
         y = w[p + "gnorm"] * y.to(self.dtype)
         y = (y.float() * F.silu(z.view(T, Hv, dv).float())).to(self.dtype)
-        return ops.linear(y.view(T, vd), w[p + "out"])
+        return y.view(T, vd), w[p + "out"]
 
     def _mlp(self, x, i):
         c, w, p = self.cfg, self.w, f"l{i}."
         if not c.is_moe(i):
-            return ops.linear(ops.linear(x, w[p + "gate_up"], act="swiglu"), w[p + "down"])
+            return ops.linear(x, w[p + "gate_up"], act="swiglu"), w[p + "down"]
         T, E, k = x.shape[0], c.num_experts, c.top_k
         logits = ops.linear(x, w[p + "router"], out_dtype=torch.float32)
         ids, wts = ops.moe_route(logits[:, :E].contiguous(), k, c.norm_topk_prob)
@@ -558,7 +559,7 @@ class Qwen3NextModel:
         y = ops.moe_gemm(h1, None, w[p + "w2"], offs, T * k, swiglu=False)
         moe = ops.moe_combine(y, pos, wts, None)
         sh = ops.linear(ops.linear(x, w[p + "sh_gate_up"], act="swiglu"), w[p + "sh_down"])
-        return (moe.float() + torch.sigmoid(logits[:, E:E + 1]) * sh.float()).to(self.dtype)
+        return (moe.float() + torch.sigmoid(logits[:, E:E + 1]) * sh.float()).to(self.dtype), None
 
     def forward(self, fb: ForwardBatch, kv, decode_ws=None) -> torch.Tensor:
         """Returns fp32 logits [len(sample_rows), vocab]."""
@@ -569,19 +570,20 @@ class Qwen3NextModel:
         if fb.extra is None:  # direct forward without the engine hook
             self.prepare_batch(fb)
         res = ops.embedding(fb.token_ids, w["embed"], 0, c.vocab_size)
-        h = None
+        x = ops.rms_norm(res, w["l0.attn_norm"], c.rms_eps)
         for i in range(c.num_layers):
             p = f"l{i}."
-            x = ops.rms_norm(res, w[p + "attn_norm"], c.rms_eps) if h is None else \
-                ops.rms_norm(h, w[p + "attn_norm"], c.rms_eps, residual=res)
             if c.layer_types[i] == "full_attention":
-                h = self._full_attention(x, i, fb, kv, decode_ws, T, P)
+                a, wo = self._full_attention(x, i, fb, kv, decode_ws, T, P)
             else:
-                h = self._linear_attention(x, i, fb, T, P)
-            x = ops.rms_norm(h, w[p + "mlp_norm"], c.rms_eps, residual=res)
-            h = self._mlp(x, i)
-        if fb.sample_rows is not None:
-            h = h.index_select(0, fb.sample_rows)
-            res = res.index_select(0, fb.sample_rows)
-        x = ops.rms_norm(h, w["norm"], c.rms_eps, residual=res)
+                a, wo = self._linear_attention(x, i, fb, T, P)
+            x = ops.linear_add_rmsnorm(a, wo, res, w[p + "mlp_norm"], c.rms_eps)
+            a, wo = self._mlp(x, i)
+            last = i + 1 == c.num_layers
+            if last and fb.sample_rows is not None:
+                a, wo = a if wo is None else ops.linear(a, wo), None
+                a = a.index_select(0, fb.sample_rows)
+                res = res.index_select(0, fb.sample_rows)
+            nxt = w["norm" if last else f"l{i + 1}.attn_norm"]
+            x = ops.rms_norm(a, nxt, c.rms_eps, residual=res) if wo is None else ops.linear_add_rmsnorm(a, wo, res, nxt, c.rms_eps)
         return ops.linear(x, w["lm_head"], out_dtype=torch.float32)[:, : c.vocab_size]

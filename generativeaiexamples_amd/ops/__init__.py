@@ -197,7 +197,23 @@ def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
             native().linear_layernorm(x.contiguous(), w if psw is None else psw, bias, residual, ln_w, ln_b, eps, out, ws,
                                       psw is not None)
             return out
+        out = _slabs_norm(x, w, bias, residual, ln_w, ln_b, True, eps)
+        if out is not None:
+            return out
     return layer_norm(linear(x, w, bias=bias, residual=residual), ln_w, ln_b, eps)
+
+
+def _slabs_norm(x, w, bias, residual, norm_w, norm_b, layer: bool, eps):
+    """The norm of 65 to 640 rows of linear(x, w, bias) + residual whose parts of K the norm's own launch adds (rms: the residual is
+    updated in place), or None where gemm_mid.hip has no plan for that."""
+    K, N = x.shape[-1], w.shape[0]
+    M = x.numel() // K
+    if not (64 < M <= 640 and w.dtype == x.dtype == residual.dtype == torch.bfloat16 and _SPLITK and _GEMM_FORCE == 0
+            and residual.is_contiguous() and w.is_contiguous()):
+        return None
+    out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    ok = native().linear_slabs_norm(x.contiguous(), w, bias, residual, norm_w, norm_b, layer, eps, out, is_frag(w))
+    return out if ok else None
 
 
 def attention_layer_norm_ok(qkv, heads, q_lens, w, rest) -> bool:
@@ -250,10 +266,10 @@ _SPLITK = os.environ.get("GAI_SPLITK", "1") == "1"
 
 def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, norm_w: torch.Tensor, eps: float,
                        bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Decode tail of a row-parallel projection at TP = 1: ``residual += x @ w^T (+ bias)`` (bf16 rounding
-    as the unfused pair) and return ``rmsnorm(residual) * norm_w``. For decode-sized M the split-K
-    partials are reduced, added and normalised in ONE kernel (no separate reduce / norm launches);
-    otherwise ``linear`` + ``rms_norm``."""
+    """Tail of a row-parallel projection at TP = 1: ``residual += x @ w^T (+ bias)`` (bf16 rounding
+    as the unfused pair) and return ``rmsnorm(residual) * norm_w``. For decode-sized M, and up to a few hundred rows,
+    the parts of K are reduced, added and normalised in ONE kernel (no separate reduce / norm launches); longer prompts
+    add the residual in the product's epilogue."""
     K = x.shape[-1]
     M, N = x.numel() // K, w.shape[0]
     if (x.is_cuda and not isinstance(w, Fp8Weight) and _SPLITK and _GEMM_FORCE == 0 and M <= 64
@@ -264,6 +280,12 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
         out = torch.empty_like(residual)
         nat.gemm_splitk_add_rmsnorm(x.reshape(M, K).contiguous(), w if psw is None else psw, bias, residual,
                                     norm_w, out, eps, ws, psw is not None)
+        return out
+    if x.is_cuda and M > 64 and residual.is_contiguous():
+        out = _slabs_norm(x, w, bias, residual, norm_w, None, False, eps) if isinstance(w, torch.Tensor) else None
+        if out is None:
+            linear(x, w, bias, residual=residual, out=residual)
+            out = rms_norm(residual, norm_w, eps)
         return out
     return rms_norm(linear(x, w, bias), norm_w, eps, residual=residual)
 

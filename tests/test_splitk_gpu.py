@@ -329,6 +329,50 @@ def test_product_in_slices_and_norm(cuda, M, N, K, ks, frag):
     assert torch.equal(ops.linear_layer_norm(x, w, bias, odd, g, b, 1e-5), z)
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(65, 2048, 1536, True), (96, 4096, 4096, True), (187, 4096, 14336, True), (193, 3088, 4096, True),
+                                         (640, 4096, 4096, True), (640, 8192, 2048, False), (641, 4096, 4096, False), (200, 2032, 4096, False)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_parts_added_by_the_rms_norm(cuda, M, N, K, parts, bias):
+    """residual += product; rms norm, the parts of K added in the norm's launch, in both layouts of the weight and for a residual off
+    16 bytes, against float64. Error: half a unit of bf16, at most 2^-8 of the value, for the product p, for its sum v with the
+    residual and for the result; 2^-10 of it for the root mean square of thousands of such v and the fp32 sums."""
+    torch.manual_seed(M + N)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, b, r, g = bf(M, K), bf(N, K) * K ** -0.5, bf(N) if bias else None, bf(M, N), bf(N)
+    assert (ops.native().gemm_slabs_parts(M, N, K, False) > 1) == parts
+    p = x.double() @ w.double().t() + (b.double() if bias else 0)
+    v = p + r.double()
+    inv = torch.rsqrt(v.square().mean(-1, keepdim=True) + 1e-5)
+    want, off = v * inv * g.double(), 2.0 ** -8 * 1.01 * (p.abs() + v.abs()) + 1e-4
+    odd = torch.empty(M * N + 1, device=cuda, dtype=torch.bfloat16)[1:].view(M, N).copy_(r)
+    wf = w.clone()
+    assert ops.to_fragment_layout_(wf)
+    seen = []
+    for wt, res in ((w, r.clone()), (wf, r.clone()), (wf, odd)):
+        y = ops.linear_add_rmsnorm(x, wt, res, g, 1e-5, bias=b)
+        assert ((res.double() - v).abs() <= off).all()
+        assert ((y.double() - want).abs() <= 1.01 * off * inv * g.double().abs() + (2.0 ** -8 + 2.0 ** -10) * want.abs()).all()
+        seen.append((res, y))
+    assert torch.equal(seen[0][0], seen[1][0]) and torch.equal(seen[0][1], seen[1][1])
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 1024, 1024), (187, 1024, 4096), (320, 768, 3072), (500, 384, 1536), (300, 2048, 4096), (640, 1024, 4096)])
+def test_parts_added_by_the_layer_norm(cuda, M, N, K):
+    """The same before a layer norm (error as in test_product_in_slices_and_norm), and rows with nothing beside them."""
+    torch.manual_seed(M + N)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, bias, r, g, b = bf(M, K), bf(N, K) * K ** -0.5, bf(N), bf(M, N), bf(N), bf(N)
+    assert ops.native().gemm_slabs_parts(M, N, K, True) > 1
+    wf = w.clone()
+    assert ops.to_fragment_layout_(wf)
+    for bi, lb in ((bias, b), (None, None)):
+        y = ops.linear_layer_norm(x, wf, bi, r, g, lb, 1e-5)
+        v = x.double() @ w.double().t() + (bias.double() if bi is not None else 0) + r.double()
+        want = torch.nn.functional.layer_norm(v, (N,), g.double(), None if lb is None else lb.double(), 1e-5)
+        assert ((y.double() - want).abs() <= 2.0 ** -8 * (want.abs() + 8 * g.double().abs())).all()
+        assert torch.equal(y, ops.linear_layer_norm(x, w, bi, r, g, lb, 1e-5))
+
+
 @pytest.mark.parametrize("name,value", [("_SPLITK", False), ("_GEMM_FORCE", 2)])
 def test_linear_layer_norm_under_the_gemm_switches(cuda, monkeypatch, name, value):
     """A forced GEMM kernel, or the decode GEMMs switched off, hold for the product before a layer norm too."""
