@@ -640,6 +640,9 @@ class LlamaModel:
                    and os.environ.get("GAI_RES_EPI", "1") == "1")
         # up to a few hundred rows the parts of K that such a product is cut into are added in the norm's launch
         fuse = fuse or (res_epi and c.norm != "layernorm" and os.environ.get("GAI_FUSE_NORM", "1") == "1")
+        # the last layer's projections run over the sampled rows only (its attention has written the cache by then): a layer less
+        # but for QKV and attention. 14643 rows of six prompts 163.3 -> 159.1 ms
+        few = fb.sample_rows is not None and fb.sample_rows.numel() > 0 and ctx.tp_size == 1 and not self.lora_names
         for i in range(c.num_layers):
             p = f"l{i}."
             if xn is not None:
@@ -670,6 +673,9 @@ class LlamaModel:
                 ops.attention_decode(q[P:], kc, vc, fb.decode_block_tables, fb.decode_ctx, self.scale, ws=decode_ws,
                                      max_ctx=fb.max_decode_ctx, out=attn[P:], k_scale=ks, v_scale=vs, qkv_fold=fold)
             a2 = attn.view(T, -1)
+            last = i + 1 == c.num_layers
+            if last and few:  # nothing reads the other rows past the last layer's cache
+                a2, res = a2.index_select(0, fb.sample_rows), res.index_select(0, fb.sample_rows)
             if fuse:
                 x = ops.linear_add_rmsnorm(a2, w[p + "o"], res, w[p + "mlp_norm"], c.rms_eps, bias=w.get(p + "o_b"))
             elif overlap:  # TP prefill: each row chunk's all-reduce overlaps the next chunk's GEMM
@@ -689,8 +695,7 @@ class LlamaModel:
                 g = self._lora(ops.linear(x, w[p + "fc"], bias=w.get(p + "fc_b"), act="gelu_tanh"), x, i, "fc", fb)
             else:
                 g = ops.linear(x, w[p + "gate_up"], act=c.mlp)
-            last = i + 1 == c.num_layers
-            if fuse and not (last and fb.sample_rows is not None):
+            if fuse and (few or not (last and fb.sample_rows is not None)):
                 nxt = "norm" if last else f"l{i + 1}.attn_norm"
                 xn = ops.linear_add_rmsnorm(g, w[p + "down"], res, w[nxt], c.rms_eps, bias=w.get(p + "down_b"))
                 h = None
@@ -712,7 +717,7 @@ class LlamaModel:
             if fb.tp_local_logits and ctx.tp_size > 1:
                 return logits
             return ctx.tp_all_gather_last(logits)[:, : c.vocab_size]
-        if fb.sample_rows is not None:
+        if fb.sample_rows is not None and not few:
             h = h.index_select(0, fb.sample_rows) if h is not None else None
             res = res.index_select(0, fb.sample_rows)
         x = self._norm(res, "norm") if h is None else self._norm(h, "norm", residual=res)

@@ -244,6 +244,7 @@ class MixtralModel(LlamaModel):
         h = None
         # prompts on one GPU: the O product and the experts' sum add the residual themselves, the norms only read it
         res_epi = res.is_cuda and ctx.tp_size == 1 and self.ep_group is None and self.e_local == c.num_experts and T > 64
+        few = fb.sample_rows is not None and fb.sample_rows.numel() > 0 and ctx.tp_size == 1 and self.ep_group is None
         for i in range(c.num_layers):
             p = f"l{i}."
             x = ops.rms_norm(res, w[p + "attn_norm"], c.rms_eps) if h is None else \
@@ -256,16 +257,19 @@ class MixtralModel(LlamaModel):
             if T > P:
                 ops.attention_decode(q[P:], kc, vc, fb.decode_block_tables, fb.decode_ctx, self.scale, ws=decode_ws,
                                      max_ctx=fb.max_decode_ctx, out=attn[P:])
+            a2 = attn.view(T, -1)
+            if few and i + 1 == c.num_layers:  # as LlamaModel.forward
+                a2, res, res_epi = a2.index_select(0, fb.sample_rows), res.index_select(0, fb.sample_rows), False
             if res_epi:
-                x = ops.linear_add_rmsnorm(attn.view(T, -1), w[p + "o"], res, w[p + "mlp_norm"], c.rms_eps)
+                x = ops.linear_add_rmsnorm(a2, w[p + "o"], res, w[p + "mlp_norm"], c.rms_eps)
                 res = self.moe_mlp(x, i, res)
                 continue
-            h = ops.linear(attn.view(T, -1), w[p + "o"])
+            h = ops.linear(a2, w[p + "o"])
             ctx.tp_all_reduce(h)
             x = ops.rms_norm(h, w[p + "mlp_norm"], c.rms_eps, residual=res)
             h = self.moe_mlp(x, i, None)
             ctx.tp_all_reduce(h)
-        if fb.sample_rows is not None:
+        if fb.sample_rows is not None and not few:
             h = h.index_select(0, fb.sample_rows) if h is not None else None
             res = res.index_select(0, fb.sample_rows)
         x = ops.rms_norm(res, w["norm"], c.rms_eps) if h is None else ops.rms_norm(h, w["norm"], c.rms_eps, residual=res)

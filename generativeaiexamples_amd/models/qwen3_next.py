@@ -571,19 +571,21 @@ class Qwen3NextModel:
             self.prepare_batch(fb)
         res = ops.embedding(fb.token_ids, w["embed"], 0, c.vocab_size)
         x = ops.rms_norm(res, w["l0.attn_norm"], c.rms_eps)
+        # the last layer's projections run over the sampled rows only: two prompts of 10095 rows in six layers 7465 -> 6885 us
+        few = fb.sample_rows is not None and fb.sample_rows.numel() > 0
         for i in range(c.num_layers):
             p = f"l{i}."
             if c.layer_types[i] == "full_attention":
                 a, wo = self._full_attention(x, i, fb, kv, decode_ws, T, P)
             else:
                 a, wo = self._linear_attention(x, i, fb, T, P)
+            last = i + 1 == c.num_layers
+            if last and few:  # nothing reads the other rows past the last layer's cache and state
+                a, res = a.index_select(0, fb.sample_rows), res.index_select(0, fb.sample_rows)
             x = ops.linear_add_rmsnorm(a, wo, res, w[p + "mlp_norm"], c.rms_eps)
             a, wo = self._mlp(x, i)
-            last = i + 1 == c.num_layers
-            if last and fb.sample_rows is not None:
-                a, wo = a if wo is None else ops.linear(a, wo), None
-                a = a.index_select(0, fb.sample_rows)
-                res = res.index_select(0, fb.sample_rows)
+            if last and fb.sample_rows is not None and not few:
+                a, res = a[:0], res[:0]
             nxt = w["norm" if last else f"l{i + 1}.attn_norm"]
             x = ops.rms_norm(a, nxt, c.rms_eps, residual=res) if wo is None else ops.linear_add_rmsnorm(a, wo, res, nxt, c.rms_eps)
         return ops.linear(x, w["lm_head"], out_dtype=torch.float32)[:, : c.vocab_size]
