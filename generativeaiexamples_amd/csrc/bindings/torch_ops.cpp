@@ -325,6 +325,20 @@ bool linear_slabs_norm(const Tensor& A, const Tensor& W, const optional<Tensor>&
   return true;
 }
 
+// (GeGLU(A1 . W1^T), A2 . W2^T + bias) of the same number of rows, weights in fragment order, in one launch
+void gemm_dec2_pair(const Tensor& A1, const Tensor& W1, Tensor& C1, const Tensor& A2, const Tensor& W2, const Tensor& bias, Tensor& C2) {
+  for (const Tensor* t : {&A1, &W1, &A2, &W2, &bias, static_cast<const Tensor*>(&C1), static_cast<const Tensor*>(&C2)}) {
+    check_bf16(*t, "gemm_dec2_pair");
+    TORCH_CHECK(t->is_contiguous() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "gemm_dec2_pair: whole operands on 16 bytes");
+  }
+  const int64_t M = A1.size(0), K = A1.size(-1), N1 = W1.size(0), N2 = W2.size(0);
+  TORCH_CHECK(A1.dim() == 2 && A2.dim() == 2 && A2.size(0) == M && A2.size(1) == K && W1.size(1) == K && W2.size(1) == K &&
+                  C1.numel() == M * (N1 / 2) && C2.numel() == M * N2 && bias.numel() == N2, "gemm_dec2_pair: sizes");
+  TORCH_CHECK(gai_gemm_dec2_pair_ok(M, N1, N2, K), "gemm_dec2_pair: shape");
+  gai_gemm_dec2_pair(A1.data_ptr(), W1.data_ptr(), C1.data_ptr(), N1, A2.data_ptr(), W2.data_ptr(), bias.data_ptr(), C2.data_ptr(), N2, M, K,
+                     cur_stream());
+}
+
 // rows at the end of gemm's product that the mid-size kernel computes (all, some or none), for the tests of that rule
 int64_t gemm_mid_rows(const Tensor& A, const Tensor& B, const Tensor& C, const optional<Tensor>& bias,
                       const optional<Tensor>& R, int64_t epi, bool bfrag) {
@@ -1238,6 +1252,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_slim_nf", &gai_gemm_slim_nf);
   m.def("gemm_slim_ks", &gai_gemm_slim_ks);
   m.def("linear_layernorm", &linear_layernorm);
+  m.def("gemm_dec2_pair", &gemm_dec2_pair);
+  m.def("gemm_dec2_pair_ok", [](int64_t M, int64_t N1, int64_t N2, int64_t K) { return gai_gemm_dec2_pair_ok(M, N1, N2, K) != 0; });
   m.def("linear_slabs_norm", &linear_slabs_norm);
   m.def("gemm_slabs_parts", [](int64_t M, int64_t N, int64_t K, bool layer) {
     GaiMidPlan plan;

@@ -105,6 +105,10 @@ void gai_attn_decode(const void* q, const void* k_cache, const void* v_cache, co
                      float v_scale, hipStream_t st, int* split_cnt = nullptr,
                      const GaiQkvFold* fold = nullptr, bool queue = false);
 int gai_gemm_partials_ks(int M, int N, int K);
+// gemm_decode.hip: GeGLU(A1 . W1^T) [M, N1 / 2] and A2 . W2^T + bias [M, N2] in one launch, M <= 64, weights in fragment order
+int gai_gemm_dec2_pair_ok(int M, int N1, int N2, int K);
+void gai_gemm_dec2_pair(const void* A1, const void* W1, void* C1, int N1, const void* A2, const void* W2, const void* bias, void* C2, int N2,
+                        int M, int K, hipStream_t st);
 int gai_gemm_splitk_waves(int N, int KS);  // of a workgroup of the split-K products that stage their slice
 void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st);
 // QKV partial slabs only (for GaiQkvFold): KS (2..8) when launched, 0 when the shape runs elsewhere.

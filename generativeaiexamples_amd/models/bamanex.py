@@ -268,10 +268,10 @@ class BamanexModel(HybridDecoderBase):
         return self.load_state(random_state(self.cfg, seed))
 
     # ------------------------------------------------------------------ branches
-    def _attention(self, h, i, run, fb, kv, seq):
+    def _attention(self, h, proj, i, run, fb, kv, seq):
         m, w, x = self.cfg.layers[i]["mixer"], self.w, f"l{i}.mix."
         H, G, dk, dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
-        proj = ops.linear(h, w[x + "in"], w[x + "in.b"])
+        proj = ops.linear(h, w[x + "in"], w[x + "in.b"]) if proj is None else proj
         a, b = H * dk, (H + G) * dk
         c = b + G * dv
         kc, vc = kv.layer(self.kv_index[run])
@@ -281,11 +281,9 @@ class BamanexModel(HybridDecoderBase):
                                    window=m["window"], sink=w[x + "sink"], gate=proj[:, c:c + H])
         return ops.linear_partial(att, w[x + "o"], w[x + "o.b"])
 
-    def _dense(self, h, p):
+    def _dense(self, h, mid, p):
         w, F_ = self.w, self.w[p + "down"].shape[1]
-        if self.dtype == torch.bfloat16:   # gate / up rows interleaved: the activation is the GEMM's epilogue
-            mid = ops.linear(h, w[p + "in"], act="geglu")
-        else:
+        if mid is None:
             gu = ops.linear(h, w[p + "in"])
             mid = ops.act_mul(gu[:, :F_], gu[:, F_:], "gelu_tanh", self.dtype)
         return ops.linear_partial(mid, w[p + "down"])
@@ -324,10 +322,15 @@ class BamanexModel(HybridDecoderBase):
         for i, t in self.runs:
             p, ml = f"l{i}.", c.layers[i]["mlp"]
             h1, h2 = ops.parallel_add_norm_f32(res, a, s1, b, s2, w[p + "norm1"], w.get(p + "norm2"), eps, dt)
-            a, s1 = self._attention(h1, i, (i, t), fb, kv, seq), w[p + "ls1"]
+            # gate / up rows of a bf16 dense branch are interleaved: the activation is the product's epilogue. It is ready with the
+            # attention's projection, which shares its launch in a decode step
+            proj = mid = None
+            if dt == torch.bfloat16 and ml is not None and ml["kind"] == "dense":
+                mid, proj = ops.linear_pair(h2, w[p + "mlp.in"], h1, w[p + "mix.in"], w[p + "mix.in.b"])
+            a, s1 = self._attention(h1, proj, i, (i, t), fb, kv, seq), w[p + "ls1"]
             b = s2 = None
             if ml is not None:
-                b = self._moe(h2, ml, p + "mlp.") if ml["kind"] == "moe" else self._dense(h2, p + "mlp.")
+                b = self._moe(h2, ml, p + "mlp.") if ml["kind"] == "moe" else self._dense(h2, mid, p + "mlp.")
                 s2 = w[p + "ls2"]
             if self.capture_residuals is not None:
                 ops.parallel_add_norm_f32(res, a, s1, b, s2)

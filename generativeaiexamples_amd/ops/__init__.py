@@ -182,6 +182,20 @@ def linear_partial(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor
     return linear(x, w, bias)
 
 
+def linear_pair(x1, w1, x2, w2, b2):
+    """(linear(x1, w1, act="geglu"), linear(x2, w2, b2)) of decode-sized rows that are ready together: one launch where both weights are in
+    fragment order and the shapes fit it."""
+    if (x1.is_cuda and x1.dim() == x2.dim() == 2 and x1.shape == x2.shape and 1 <= x1.shape[0] <= 64 and _SPLITK and _GEMM_FORCE == 0
+            and all(isinstance(t, torch.Tensor) and t.dtype == torch.bfloat16 and t.is_contiguous() and not t.data_ptr() & 15
+                    for t in (x1, w1, x2, w2, b2)) and is_frag(w1) and is_frag(w2)
+            and native().gemm_dec2_pair_ok(x1.shape[0], w1.shape[0], w2.shape[0], x1.shape[1])):
+        y1 = torch.empty(x1.shape[0], w1.shape[0] // 2, dtype=x1.dtype, device=x1.device)
+        y2 = torch.empty(x1.shape[0], w2.shape[0], dtype=x1.dtype, device=x1.device)
+        native().gemm_dec2_pair(x1, w1, y1, x2, w2, b2, y2)
+        return y1, y2
+    return linear(x1, w1, act="geglu"), linear(x2, w2, b2)
+
+
 def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
     """layer_norm(linear(x, w, bias, residual)). A short question's product leaves most of the chip idle with one workgroup a
     column tile: its K is cut into slices (gemm_slim.hip) whose sums the norm adds up."""

@@ -329,6 +329,24 @@ def test_product_in_slices_and_norm(cuda, M, N, K, ks, frag):
     assert torch.equal(ops.linear_layer_norm(x, w, bias, odd, g, b, 1e-5), z)
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N1,N2,K,one", [(11264, 3088, 2048, True), (1120, 1040, 2048, True), (1056, 1072, 6144, True), (1024, 1024, 1088, False)])
+def test_pair_of_products(cuda, M, N1, N2, K, one):
+    """A gated product and one with a bias in one launch (one) or two, against float64: bf16 roundings of the result (2^-8 of it) and fp32 sums,
+    the gate by approximate exponential and reciprocal (2^-20)."""
+    torch.manual_seed(M + N1)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x1, x2, w1, w2, b = bf(M, K), bf(M, K), bf(N1, K) * K ** -0.5, bf(N2, K) * K ** -0.5, bf(N2)
+    gu = (x1.double() @ w1.double().t()).view(M, N1 // 32, 2, 16)
+    want1 = (torch.nn.functional.gelu(gu[:, :, 0], approximate="tanh") * gu[:, :, 1]).reshape(M, -1)
+    want2 = x2.double() @ w2.double().t() + b.double()
+    assert (ops.to_fragment_layout_(w1) and ops.to_fragment_layout_(w2)) or not one
+    assert ops.native().gemm_dec2_pair_ok(M, N1, N2, K) == one
+    y1, y2 = ops.linear_pair(x1, w1, x2, w2, b)
+    for y, want in ((y1, want1), (y2, want2)):
+        assert ((y.double() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 2e-5).all()
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(65, 2048, 1536, True), (96, 4096, 4096, True), (187, 4096, 14336, True), (193, 3088, 4096, True),
                                          (640, 4096, 4096, True), (640, 8192, 2048, False), (641, 4096, 4096, False), (200, 2032, 4096, False)])
 @pytest.mark.parametrize("bias", [False, True])
