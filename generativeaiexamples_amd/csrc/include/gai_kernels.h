@@ -323,6 +323,9 @@ void gai_rotary_kv_write(const void* q, int ldq, const void* k, int ldk, const v
                          const int* slots, void* q_out, void* k_cache, void* v_cache, int T, int H, int G, int DK, int DV,
                          int ROT, float base, int dt_in, int dt, hipStream_t st);
 // rotate-half positions (inv_freq: fp64 [half]), unit RMS norm per head (unit_eps >= 0), cache write
+int gai_gemm_partials_rotary(const void* A, const void* B, int M, int N, int K, float* ws, const void* q, int ldq, const void* k, int ldk,
+                             const void* v, int ldv, const int* positions, const int* slots, void* q_out, void* k_cache, void* v_cache, int T,
+                             int H, int G, int DK, int DV, const double* inv_freq, int half, float unit_eps, hipStream_t st);
 void gai_rotary_half_kv_write(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const int* positions,
                               const int* slots, void* q_out, void* k_cache, void* v_cache, int T, int H, int G, int DK,
                               int DV, const double* inv_freq, int half, float unit_eps, int dt, hipStream_t st);

@@ -52,6 +52,7 @@
 // kernel further down.
 #include "gai_common.h"
 #include "gai_kernels.h"
+#include "gai_rotary.h"
 
 using namespace gai;
 
@@ -350,101 +351,10 @@ __global__ __launch_bounds__(256) void rotary_kv_write_kernel(const TI* __restri
   }
 }
 
-// Workgroups 0 .. T - 1: q and k heads of one token, `lph` lanes (a power of two) per head with NJ groups of VEC channels
-// each, so a wave holds 64 / lph heads; the others: v of VT tokens, a thread per channel, so that tokens filling a whole page
-// store its V^T row at once.
-constexpr int kHalfRegs = 8;
-
 template <typename TA, int VEC, int NJ, int VT>
-__global__ __launch_bounds__(256) void rotary_half_kv_write_kernel(
-    const TA* __restrict__ q, int ldq, const TA* __restrict__ k, int ldk, const TA* __restrict__ v, int ldv,
-    const int* __restrict__ positions, const int* __restrict__ slots, TA* __restrict__ q_out, TA* __restrict__ k_cache,
-    TA* __restrict__ v_cache, int T, int H, int G, int DK, int DV, const double* __restrict__ inv_freq, int half,
-    float unit_eps, int lph) {
-  const int tid = threadIdx.x;
-  if ((int)blockIdx.x >= T) {
-    const int t0 = ((int)blockIdx.x - T) * VT, n = min(VT, T - t0), NV = G * DV, s0 = slots[t0];
-    const bool page = VT == 16 && n == 16 && (s0 & 15) == 0 && __all(slots[t0 + (tid & 15)] == s0 + (tid & 15));
-    for (int i = tid; i < NV; i += 256) {
-      const int g = i / DV, c = i - g * DV;
-      const TA* src = v + (size_t)t0 * ldv + i;
-      if (page) {
-        TA* dst = v_cache + (((size_t)(s0 >> 4) * G + g) * DV + c) * 16;
-        __attribute__((aligned(16))) TA x[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) x[j] = src[(size_t)j * ldv];
-#pragma unroll
-        for (int j = 0; j < (int)sizeof(TA); ++j)
-          reinterpret_cast<uint4*>(dst)[j] = reinterpret_cast<const uint4*>(x)[j];
-      } else {
-        for (int j = 0; j < n; ++j) {
-          const int s = slots[t0 + j];
-          v_cache[(((size_t)(s >> 4) * G + g) * DV + c) * 16 + (s & 15)] = src[(size_t)j * ldv];
-        }
-      }
-    }
-    return;
-  }
-  extern __shared__ float cs[];  // cos[half] | sin[half]
-  const int t = blockIdx.x, lane = tid & (lph - 1);
-  const double pos = (double)positions[t];
-  for (int i = tid; i < half; i += 256) {
-    const double a = pos * inv_freq[i];
-    const double r = a - 6.283185307179586476925 * rint(a * 0.15915494309189533577);
-    float sn, c;
-    sincosf((float)r, &sn, &c);
-    cs[i] = c;
-    cs[half + i] = sn;
-  }
-  __syncthreads();
-  const int slot = slots[t], off = slot & 15;
-  const size_t page = slot >> 4;
-  typedef TA vec __attribute__((ext_vector_type(VEC)));
-  for (int hh = tid / lph; hh < H + G; hh += 256 / lph) {  // q heads, then k heads: uniform over the head's lanes
-    const bool isq = hh < H;
-    const int g = isq ? hh : hh - H;
-    const TA* src = isq ? q + (size_t)t * ldq + (size_t)g * DK : k + (size_t)t * ldk + (size_t)g * DK;
-    TA* dst = isq ? q_out + ((size_t)t * H + g) * DK : k_cache + ((page * G + g) * 16 + off) * DK;
-    float y[NJ][VEC];
-    float ss = 0.f;
-#pragma unroll
-    for (int r = 0; r < NJ; ++r) {
-      const int i = (lane + lph * r) * VEC;
-      if (i < DK) {
-        const vec x = *reinterpret_cast<const vec*>(src + i);
-        if (i < 2 * half) {   // VEC divides half: the group has one partner group
-          const bool up = i >= half;
-          const vec p = *reinterpret_cast<const vec*>(src + (up ? i - half : i + half));
-          const int f = up ? i - half : i;
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) {
-            const float c = cs[f + e], sn = cs[half + f + e];
-            y[r][e] = up ? (float)x[e] * c + (float)p[e] * sn : (float)x[e] * c - (float)p[e] * sn;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) y[r][e] = (float)x[e];
-        }
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) ss += y[r][e] * y[r][e];
-      }
-    }
-    float inv = 1.0f;
-    if (unit_eps >= 0.f) {
-      for (int o = lph >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-      inv = 1.0f / sqrtf(ss / DK + unit_eps);
-    }
-#pragma unroll
-    for (int r = 0; r < NJ; ++r) {
-      const int i = (lane + lph * r) * VEC;
-      if (i < DK) {
-        vec o;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) o[e] = (TA)(y[r][e] * inv);
-        *reinterpret_cast<vec*>(dst + i) = o;
-      }
-    }
-  }
+__global__ __launch_bounds__(256) void rotary_half_kv_write_kernel(RotaryHalf<TA> a) {
+  extern __shared__ float cs[];
+  rotary_half_body<TA, VEC, NJ, VT>(a, blockIdx.x, cs);
 }
 
 constexpr int kMaxVChunks = 8;  // DV <= 512
@@ -891,8 +801,8 @@ void gai_rotary_half_kv_write(const void* q, int ldq, const void* k, int ldk, co
   const int grid = T + (tiles ? (T + 15) / 16 : T);
 #define GAI_RH(TA, VEC_, NJ_, VT_)                                                                                   \
   rotary_half_kv_write_kernel<TA, VEC_, NJ_, VT_><<<grid, 256, lds, st>>>(                                           \
-      (const TA*)q, ldq, (const TA*)k, ldk, (const TA*)v, ldv, positions, slots, (TA*)q_out, (TA*)k_cache, (TA*)v_cache, \
-      T, H, G, DK, DV, inv_freq, half, unit_eps, NJ_ == 1 ? per : 64)
+      RotaryHalf<TA>{(const TA*)q, ldq, (const TA*)k, ldk, (const TA*)v, ldv, positions, slots, (TA*)q_out, (TA*)k_cache, \
+                     (TA*)v_cache, T, H, G, DK, DV, inv_freq, half, unit_eps, NJ_ == 1 ? per : 64})
 #define GAI_RH2(TA, VEC_, NJ_) if (tiles) GAI_RH(TA, VEC_, NJ_, 16); else GAI_RH(TA, VEC_, NJ_, 1)
   if (dt) { if (one) { GAI_RH2(float, 4, 1); } else if (two) { GAI_RH2(float, 2, kHalfRegs); } else { GAI_RH2(float, 1, kHalfRegs); } }
   else { if (one) { GAI_RH2(bf16, 8, 1); } else if (two) { GAI_RH2(bf16, 2, kHalfRegs); } else { GAI_RH2(bf16, 1, kHalfRegs); } }

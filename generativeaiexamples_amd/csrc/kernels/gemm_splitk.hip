@@ -20,6 +20,7 @@
 #include "gai_gemm_slim.h"
 #include "gai_kernels.h"
 #include "gai_rope.h"
+#include "gai_rotary.h"
 
 using namespace gai;
 
@@ -237,17 +238,15 @@ constexpr int kLdsRow = 68;  // fp32 row stride of the reduction tiles
 template <int MB>
 constexpr int dec_lds_bytes() { return 4 * 16 * MB * kLdsRow * 4; }
 
+// workgroup (bx, ks of KS)
 template <int MB, int EPI, bool OUTF32, bool PSW>
-__global__ __launch_bounds__(256, 2) void gemm_dec_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
-                                                          float* __restrict__ part, void* __restrict__ C,
-                                                          const bf16* __restrict__ bias, const bf16* R, int M, int N,
-                                                          int K, int KW, int ldc) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+__device__ __forceinline__ void dec_body(const bf16* __restrict__ A, const bf16* __restrict__ W, float* __restrict__ part,
+                                         void* __restrict__ C, const bf16* __restrict__ bias, const bf16* R, int M, int N, int K, int KW,
+                                         int ldc, char* smem, int bx, int ks, int KS) {
   constexpr int ROWS = 16 * MB;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * 64;
-  const int ks = blockIdx.y, KS = gridDim.y;
+  const int n0 = bx * 64;
   const int kbeg = (ks * 4 + wid) * KW;  // this wave's K range [kbeg, kbeg + KW)
   const int nsteps = KW / 32;
   const int kq = 8 * (lane >> 4);
@@ -375,6 +374,28 @@ __global__ __launch_bounds__(256, 2) void gemm_dec_kernel(const bf16* __restrict
         if (n0 + 16 * q + c < N) store_out<EPI, OUTF32>(C, bias, R, ldc, m, n0 + 16 * q + c, v[c]);
     }
   }
+}
+
+template <int MB, int EPI, bool OUTF32, bool PSW>
+__global__ __launch_bounds__(256, 2) void gemm_dec_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                          float* __restrict__ part, void* __restrict__ C,
+                                                          const bf16* __restrict__ bias, const bf16* R, int M, int N,
+                                                          int K, int KW, int ldc) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  dec_body<MB, EPI, OUTF32, PSW>(A, W, part, C, bias, R, M, N, K, KW, ldc, smem, blockIdx.x, blockIdx.y, gridDim.y);
+}
+
+// The K slices of a product beside the rotation of a step's heads and its cache write (workgroups below `rot`), which wait for nothing of
+// each other in a layer of parallel branches. 24 rows: product 10.0 us, rotation 5.2 by itself, 10.7 together; a step of the 2k hybrid stack,
+// 24 streams 389 -> 361 us, one 299 -> 274, 64 540 -> 500.
+template <int MB>
+__global__ __launch_bounds__(256, 2) void gemm_dec_rotary_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                                 float* __restrict__ part, int M, int N, int K, int KW, int KS,
+                                                                 RotaryHalf<bf16> r, int rot) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if ((int)blockIdx.x < rot) return rotary_half_body<bf16, 8, 1, 1>(r, blockIdx.x, reinterpret_cast<float*>(smem));
+  const int i = blockIdx.x - rot, tiles = (N + 63) / 64;
+  dec_body<MB, EPI_NONE, true, true>(A, W, part, nullptr, nullptr, nullptr, M, N, K, KW, 0, smem, i % tiles, i / tiles, KS);
 }
 
 // Sum the KS fp32 partial slabs (stride floats apart) of W consecutive values at p, slab 0 first (the
@@ -968,6 +989,34 @@ void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float*
   if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_partials: the product has no slices");
   if (gai_gemm_slim_nf(M, N, K, false)) gai_gemm_slim_partials(A, B, M, N, K, ws, psw, st);
   else if (!gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw)) launch_partials(A, B, M, N, K, ks, ws, psw, st);
+}
+
+// gai_gemm_partials of a weight in fragment order beside gai_rotary_half_kv_write of T bf16 rows; 0: not these, nothing launched
+int gai_gemm_partials_rotary(const void* A, const void* B, int M, int N, int K, float* ws, const void* q, int ldq, const void* k, int ldk,
+                             const void* v, int ldv, const int* positions, const int* slots, void* q_out, void* k_cache, void* v_cache, int T,
+                             int H, int G, int DK, int DV, const double* inv_freq, int half, float unit_eps, hipStream_t st) {
+  const int ks = gai_gemm_partials_ks(M, N, K), per = DK / 8;
+  if (ks == 0 || gai_gemm_slim_nf(M, N, K, false) || gai_gemm_dec2_partials_ks(M, N, K) || use_legacy(N, K)) return 0;
+  const bool on8 = DK % 8 == 0 && half % 8 == 0 && ldq % 8 == 0 && ldk % 8 == 0 &&
+                   (((size_t)q | (size_t)k | (size_t)q_out | (size_t)k_cache) & 15) == 0;
+  if (T < 1 || T > 64 || half < 0 || 2 * half > DK || !on8 || per > 64 || (per & (per - 1))) return 0;
+  const RotaryHalf<bf16> r{(const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, positions, slots, (bf16*)q_out, (bf16*)k_cache,
+                           (bf16*)v_cache, T, H, G, DK, DV, inv_freq, half, unit_eps, per};
+#define GAI_DR(MB)                                                                                                                     \
+  {                                                                                                                                    \
+    static bool once = false;                                                                                                          \
+    if (!once) {                                                                                                                       \
+      hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_dec_rotary_kernel<MB>), hipFuncAttributeMaxDynamicSharedMemorySize,       \
+                          dec_lds_bytes<MB>());                                                                                        \
+      once = true;                                                                                                                     \
+    }                                                                                                                                  \
+    gemm_dec_rotary_kernel<MB><<<2 * T + (N + 63) / 64 * ks, 256, dec_lds_bytes<MB>(), st>>>((const bf16*)A, (const bf16*)B, ws, M, N, K, \
+                                                                                            K / (4 * ks), ks, r, 2 * T);               \
+  }
+  if (M <= 16) GAI_DR(1) else if (M <= 32) GAI_DR(2) else GAI_DR(4)
+#undef GAI_DR
+  GAI_LAUNCH_CHECK();
+  return 1;
 }
 
 void gai_gemm_splitk(const void* A, const void* B, void* C, const void* bias, const void* R, int M, int N, int K,

@@ -268,7 +268,7 @@ class BamanexModel(HybridDecoderBase):
         return self.load_state(random_state(self.cfg, seed))
 
     # ------------------------------------------------------------------ branches
-    def _attention(self, h, proj, i, run, fb, kv, seq):
+    def _attention(self, h, proj, i, run, fb, kv, seq, beside=None):
         m, w, x = self.cfg.layers[i]["mixer"], self.w, f"l{i}.mix."
         H, G, dk, dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
         proj = ops.linear(h, w[x + "in"], w[x + "in.b"]) if proj is None else proj
@@ -276,7 +276,7 @@ class BamanexModel(HybridDecoderBase):
         c = b + G * dv
         kc, vc = kv.layer(self.kv_index[run])
         q = ops.rotary_half_kv_write(proj[:, :a], proj[:, a:b], proj[:, b:c], fb.positions, fb.slots, kc, vc, H, G, dk, dv,
-                                     w[x + "inv_freq"], self.cfg.rms_eps)
+                                     w[x + "inv_freq"], self.cfg.rms_eps, beside=beside)
         att = ops.window_attention(q, kc, vc, seq["bt"], seq["cu"], seq["ctx"], H, G, dk, dv, float(m["scale"]),
                                    window=m["window"], sink=w[x + "sink"], gate=proj[:, c:c + H])
         return ops.linear_partial(att, w[x + "o"], w[x + "o.b"])
@@ -324,13 +324,14 @@ class BamanexModel(HybridDecoderBase):
             h1, h2 = ops.parallel_add_norm_f32(res, a, s1, b, s2, w[p + "norm1"], w.get(p + "norm2"), eps, dt)
             # gate / up rows of a bf16 dense branch are interleaved: the activation is the product's epilogue. It is ready with the
             # attention's projection, which shares its launch in a decode step
-            proj = mid = None
+            proj = mid = b = s2 = None
             if dt == torch.bfloat16 and ml is not None and ml["kind"] == "dense":
                 mid, proj = ops.linear_pair(h2, w[p + "mlp.in"], h1, w[p + "mix.in"], w[p + "mix.in.b"])
-            a, s1 = self._attention(h1, proj, i, (i, t), fb, kv, seq), w[p + "ls1"]
-            b = s2 = None
+                b = ops.linear_partial_later(mid, w[p + "mlp.down"])
+            a, s1 = self._attention(h1, proj, i, (i, t), fb, kv, seq, beside=b), w[p + "ls1"]
             if ml is not None:
-                b = self._moe(h2, ml, p + "mlp.") if ml["kind"] == "moe" else self._dense(h2, mid, p + "mlp.")
+                if b is None:
+                    b = self._moe(h2, ml, p + "mlp.") if ml["kind"] == "moe" else self._dense(h2, mid, p + "mlp.")
                 s2 = w[p + "ls2"]
             if self.capture_residuals is not None:
                 ops.parallel_add_norm_f32(res, a, s1, b, s2)

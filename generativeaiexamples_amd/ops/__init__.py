@@ -158,17 +158,23 @@ class Partial:
     """A product whose K slices are not added up yet: fp32 [slices, rows, columns] and the bias that their sum takes
     (linear_partial). parallel_add_norm_f32 takes it in place of the rows."""
 
-    __slots__ = ("slabs", "bias")
+    __slots__ = ("slabs", "bias", "operands")
 
-    def __init__(self, slabs: torch.Tensor, bias: Optional[torch.Tensor] = None):
-        self.slabs, self.bias = slabs, bias
+    def __init__(self, slabs: torch.Tensor, bias: Optional[torch.Tensor] = None, operands=None):
+        self.slabs, self.bias, self.operands = slabs, bias, operands  # operands: of slabs that another launch still makes
 
     def index_select(self, dim: int, idx: torch.Tensor) -> "Partial":
         assert dim == 0
         return Partial(self.slabs.index_select(1, idx), self.bias)
 
 
-def linear_partial(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
+def linear_partial_later(x: torch.Tensor, w: torch.Tensor) -> Optional[Partial]:
+    """linear_partial(x, w) whose slices rotary_half_kv_write(beside=) makes; None where that takes no slices of this product."""
+    p = linear_partial(x, w, launch=False) if is_frag(w) and x.is_cuda else None
+    return p if isinstance(p, Partial) else None
+
+
+def linear_partial(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, launch: bool = True):
     """linear(x, w, bias) for parallel_add_norm_f32: its K slices (a Partial) where a decode-sized product on the GPU has some,
     which saves the launch that adds them, else the rows."""
     if (x.is_cuda and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()
@@ -177,9 +183,11 @@ def linear_partial(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor
         ks = nat.gemm_partials_ks(x.shape[0], *w.shape) if psw is not None or (_SPLITK and _GEMM_FORCE == 0) else 0
         if ks:
             ws = torch.empty(ks, x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+            if not launch:
+                return Partial(ws, bias, (x, w))
             nat.gemm_partials(x, w if psw is None else psw, ws, psw is not None)
             return Partial(ws, bias)
-    return linear(x, w, bias)
+    return linear(x, w, bias) if launch else None
 
 
 def linear_pair(x1, w1, x2, w2, b2):
@@ -1896,17 +1904,18 @@ def parallel_add_norm_f32(res, a=None, sa=None, b=None, sb=None, w1=None, w2=Non
 
 
 def rotary_half_kv_write(q, k, v, positions, slots, k_cache, v_cache, H: int, G: int, DK: int, DV: int, inv_freq,
-                         unit_eps: Optional[float] = None):
+                         unit_eps: Optional[float] = None, beside: Optional[Partial] = None):
     """Rotation in the rotate-half layout: the channel pairs (i, i + n), i < n = len(inv_freq), of every q and k head
     turned by position * inv_freq[i] (inv_freq: fp64 [n], see rope_inv_freq; angles formed and reduced in fp64; channels
     past 2 n pass unchanged); with unit_eps, every q and k head is then divided by its root mean square (eps inside the
     root, no weight). k and v go into their cache slots; returns q [T, H * DK]. q / k / v may be column slices of one
-    projection."""
+    projection. beside: a linear_partial_later, whose slices are made too, in the same launch where they can be."""
     if 2 * inv_freq.numel() > DK:
         raise ValueError("rotary_half_kv_write: more rotated channels than a head has")
     if not q.is_cuda:
         return ref.rotary_half_kv_write(q, k, v, positions, slots, k_cache, v_cache, H, G, DK, DV, inv_freq, unit_eps)
     q_out = torch.empty(q.shape[0], H * DK, dtype=k_cache.dtype, device=q.device)
     native().rotary_half_kv_write(q, k, v, positions, slots, q_out, k_cache, v_cache, H, G, DK, DV, inv_freq,
-                                  -1.0 if unit_eps is None else float(unit_eps))
+                                  -1.0 if unit_eps is None else float(unit_eps),
+                                  *((None, None, None) if beside is None else (*beside.operands, beside.slabs)))
     return q_out

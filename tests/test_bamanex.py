@@ -721,3 +721,29 @@ def test_config_errors():
     with pytest.raises(ValueError):
         ops.rotary_half_kv_write(*[torch.zeros(1, 4)] * 3, torch.zeros(1), torch.zeros(1), None, None, 1, 1, 4, 4,
                                  torch.zeros(3, dtype=torch.float64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,G,D,n", [(1, 16, 4, 128, 32), (16, 16, 4, 128, 32), (17, 8, 8, 64, 32), (33, 4, 2, 256, 40), (64, 16, 4, 128, 0)])
+@pytest.mark.parametrize("N,K", [(2048, 5632), (1040, 6144)])
+def test_rotation_beside_a_product(cuda, T, H, G, D, n, N, K):
+    """The rotation and cache write in the launch of a product's K slices: the bits of both by themselves. A head size that the shared
+    launch does not take (96) and a row-major weight run one after the other."""
+    torch.manual_seed(T + D)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    for d in (D, 96):
+        qkv, x, w = bf(T, (H + 2 * G) * d), bf(T, K), bf(N, K)
+        pos = torch.randint(0, 4000, (T,), device=cuda, dtype=torch.int32)
+        slots = torch.randperm(8 * 16, device=cuda)[:T].to(torch.int32)
+        freq = ops.rope_inv_freq(2 * n, 10000.0, None).to(cuda) if n else torch.zeros(0, dtype=torch.float64, device=cuda)
+        want = ops.linear_partial(x, w)
+        assert ops.linear_partial_later(x, w) is None   # row-major
+        assert ops.to_fragment_layout_(w)
+        outs = []
+        for beside in (None, ops.linear_partial_later(x, w)):
+            kc, vc = torch.zeros(8, G, 16, d, device=cuda, dtype=torch.bfloat16), torch.zeros(8, G, d, 16, device=cuda, dtype=torch.bfloat16)
+            q = ops.rotary_half_kv_write(qkv[:, :H * d], qkv[:, H * d:(H + G) * d], qkv[:, (H + G) * d:], pos, slots, kc, vc, H, G, d, d,
+                                         freq, 1e-6, beside=beside)
+            outs.append((q, kc, vc))
+        assert all(torch.equal(a, b) for a, b in zip(*outs))
+        assert torch.equal(beside.slabs, want.slabs)
