@@ -487,9 +487,12 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, 
     fp = &fold;
   }
   TORCH_CHECK(!queue || (cnt && split_cnt->numel() >= (int64_t)B * Hkv + kGaiDecodeQueueInts), "attn_decode: no room for the queues");
+  // the merge reads the partials in 8-byte pairs
+  const auto pairs = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 8 ? at::empty_like(t) : t; };
+  const Tensor po = pairs(ws_o), pml = pairs(ws_ml);
   gai_attn_decode(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr<int>(),
-                  block_tables.size(1), ctx_lens.data_ptr<int>(), out.data_ptr(), ws_o.data_ptr<float>(),
-                  ws_ml.data_ptr<float>(), B, Hq, Hkv, D, (float)scale, split_keys, max_splits, f8, (float)k_scale,
+                  block_tables.size(1), ctx_lens.data_ptr<int>(), out.data_ptr(), po.data_ptr<float>(),
+                  pml.data_ptr<float>(), B, Hq, Hkv, D, (float)scale, split_keys, max_splits, f8, (float)k_scale,
                   (float)v_scale, cur_stream(), cnt, fp, queue);
 }
 

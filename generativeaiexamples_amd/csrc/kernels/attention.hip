@@ -780,7 +780,7 @@ __device__ __forceinline__ float ld_sc1(const float* p) {
 }
 // Merge the flash-decoding partials (O, max, sum) of ns splits for one (sequence, q head, dim): groups of
 // kMergeGroup splits, every load of a group issued before its math, running-max rescale between groups. The
-// separate reduce launch and the in-launch merge (SC1: write-through partials read with sc1 loads) share it,
+// separate reduce launch and the in-launch merge (write-through partials read with sc1 loads) take the same steps,
 // so both round identically.
 constexpr int kMergeGroup = 8;
 
@@ -793,7 +793,74 @@ __device__ __forceinline__ int split_len(int split_keys, int ctx, int max_splits
   const int per = (ctx + max_splits - 1) / max_splits;
   return max(128, (per + 127) / 128 * 128);
 }
-template <bool SC1>
+template <int N>
+struct MergeGroups {  // N groups of splits of neighbouring dims, and their running sums
+  float m[N * kMergeGroup], l[N * kMergeGroup];
+  float2 o[N * kMergeGroup];
+  float M = kNeg, L = 0.f, O0 = 0.f, O1 = 0.f;
+  __device__ __forceinline__ void add(int j0, int s0, int ns) {
+    float Mn = M;
+#pragma unroll
+    for (int j = 0; j < kMergeGroup; ++j) Mn = s0 + j < ns ? fmaxf(Mn, m[j0 + j]) : Mn;
+    if (s0 > 0) {
+      const float a = fexp2(M - Mn);
+      L *= a;
+      O0 *= a;
+      O1 *= a;
+    }
+#pragma unroll
+    for (int j = 0; j < kMergeGroup; ++j) {
+      const float f = s0 + j < ns ? fexp2(m[j0 + j] - Mn) : 0.f;
+      L = fmaf(l[j0 + j], f, L);
+      O0 = fmaf(o[j0 + j].x, f, O0);
+      O1 = fmaf(o[j0 + j].y, f, O1);
+    }
+    M = Mn;
+  }
+};
+// The last workgroup's merge of a (sequence, kv head): a thread takes two neighbouring dims, and up to 8 N splits' partials are on
+// their way at once (a round trip past this XCD's L2 is over a microsecond; a dim and a group at a time, 20 splits took six of them: one
+// sequence of 2531 keys 12.3 -> 10.1 us, 23 of 1900 - 7900 on 8-bit pages 55.5 -> 53.7).
+template <int N>
+__device__ __forceinline__ void merge_and_store(const float* ws_o, const float* ws_ml, int B, int Hq, int D, int seq, int h0, int heads,
+                                                int ns, bf16* out) {
+  const auto ld2 = [](const float* p) {
+    const unsigned long long x = __hip_atomic_load((__attribute__((address_space(1))) unsigned long long*)p, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+    return float2{__uint_as_float((unsigned)x), __uint_as_float((unsigned)(x >> 32))};
+  };
+  for (int e = 2 * threadIdx.x; e < heads * D; e += 512) {
+    const int hq = h0 + e / D, d = e % D;
+    MergeGroups<N> g;
+    auto load = [&](int j0, int s0) {
+#pragma unroll
+      for (int j = 0; j < kMergeGroup; ++j) {
+        const size_t i = ((size_t)min(s0 + j, ns - 1) * B + seq) * Hq + hq;
+        const float2 ml = ld2(ws_ml + i * 2);
+        g.m[j0 + j] = ml.x;
+        g.l[j0 + j] = ml.y;
+        g.o[j0 + j] = ld2(ws_o + i * D + d);
+      }
+    };
+    int s0 = 0;
+    if constexpr (N > 1) {
+      for (; ns - s0 > kMergeGroup; s0 += N * kMergeGroup) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) load(n * kMergeGroup, s0 + n * kMergeGroup);
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+          if (s0 + n * kMergeGroup < ns) g.add(n * kMergeGroup, s0 + n * kMergeGroup, ns);
+      }
+    }
+    for (; s0 < ns; s0 += kMergeGroup) {
+      load(0, s0);
+      g.add(0, s0, ns);
+    }
+    bf16* y = out + ((size_t)seq * Hq + hq) * D + d;
+    y[0] = (bf16)(g.L > 0.f ? g.O0 / g.L : 0.f);
+    y[1] = (bf16)(g.L > 0.f ? g.O1 / g.L : 0.f);
+  }
+}
 __device__ __forceinline__ void merge_splits(const float* ws_o, const float* ws_ml, int B, int Hq, int D, int seq,
                                              int hq, int d, int ns, float& L, float& O) {
   float M = kNeg;
@@ -804,9 +871,9 @@ __device__ __forceinline__ void merge_splits(const float* ws_o, const float* ws_
 #pragma unroll
     for (int j = 0; j < kMergeGroup; ++j) {
       const size_t i = ((size_t)min(s0 + j, ns - 1) * B + seq) * Hq + hq;
-      m[j] = SC1 ? ld_sc1(ws_ml + i * 2) : ws_ml[i * 2];
-      l[j] = SC1 ? ld_sc1(ws_ml + i * 2 + 1) : ws_ml[i * 2 + 1];
-      o[j] = SC1 ? ld_sc1(ws_o + i * D + d) : ws_o[i * D + d];
+      m[j] = ws_ml[i * 2];
+      l[j] = ws_ml[i * 2 + 1];
+      o[j] = ws_o[i * D + d];
     }
     float Mn = M;
 #pragma unroll
@@ -819,8 +886,8 @@ __device__ __forceinline__ void merge_splits(const float* ws_o, const float* ws_
 #pragma unroll
     for (int j = 0; j < kMergeGroup; ++j) {
       const float f = s0 + j < ns ? fexp2(m[j] - Mn) : 0.f;
-      L += l[j] * f;
-      O += o[j] * f;
+      L = fmaf(l[j], f, L);
+      O = fmaf(o[j], f, O);
     }
     M = Mn;
   }
@@ -1223,12 +1290,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     __syncthreads();
     if (!s_last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // no instruction: keeps the loads below the ticket
-    for (int e = tid; e < ratio * D; e += 256) {
-      const int qq = e / D, d = e % D, hq = g * ratio + qq;
-      float L, O;
-      merge_splits<true>(ws_o, ws_ml, B, Hq, D, seq, hq, d, nsplit, L, O);
-      out[((size_t)seq * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
-    }
+    merge_and_store<(D >= 128 ? 3 : 1)>(ws_o, ws_ml, B, Hq, D, seq, g * ratio, ratio, nsplit, out);
     if (tid == 0) __hip_atomic_store(cnt + seq * Hkv + g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -1448,12 +1510,7 @@ __global__ __launch_bounds__(256, 3) void attn_decode_queue_kernel(
       __syncthreads();
       if (s_last) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // no instruction: keeps the loads below the ticket
-        for (int e = tid; e < ratio * D; e += 256) {
-          const int qq = e / D, d = e % D, hq = p.g * ratio + qq;
-          float L, O;
-          merge_splits<true>(ws_o, ws_ml, B, Hq, D, p.seq, hq, d, p.nsplit, L, O);
-          out[((size_t)p.seq * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
-        }
+        merge_and_store<1>(ws_o, ws_ml, B, Hq, D, p.seq, p.g * ratio, ratio, p.nsplit, out);
         if (tid == 0) __hip_atomic_store(cnt + p.seq * Hkv + p.g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
@@ -1472,7 +1529,7 @@ __global__ void attn_decode_reduce_kernel(const float* __restrict__ ws_o, const 
   const int ns = (ctx + split_keys - 1) / split_keys;
   if (ns <= 1) return;
   float L, O;
-  merge_splits<false>(ws_o, ws_ml, B, Hq, D, seq, hq, d, ns, L, O);
+  merge_splits(ws_o, ws_ml, B, Hq, D, seq, hq, d, ns, L, O);
   out[((size_t)seq * Hq + hq) * D + d] = (bf16)(L > 0.f ? O / L : 0.f);
 }
 

@@ -116,6 +116,27 @@ def test_qkv_fold_queue_equals_a_workgroup_per_part(cuda, Hq, Hkv, nsplit, ctx):
         assert all(torch.equal(a, b) for a, b in zip((out, kc, vc), want)) and int(ws.cnt.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("D,Hq,Hkv", [(128, 32, 8), (128, 16, 1), (128, 3, 3), (64, 6, 2), (256, 4, 4)])
+@pytest.mark.parametrize("f8", [False, True])
+def test_merge_in_the_launch_equals_the_reduce_launch(cuda, D, Hq, Hkv, f8):
+    """1 to 65 parts: groups of eight that arrive three at a time, and those left over, against the merge in a launch of its own."""
+    torch.manual_seed(D + Hq)
+    ctx = [128 * n - 3 * i for i, n in enumerate((1, 2, 7, 8, 9, 16, 17, 24, 25, 32, 33, 48, 49, 65))]
+    B, nb, nsplit = len(ctx), max(ctx) // 16 + 2, 65
+    q = torch.randn(B, Hq, D, device=cuda, dtype=torch.bfloat16)
+    bt = torch.randperm(B * nb, device=cuda).to(torch.int32).view(B, nb)
+    c = torch.tensor(ctx, dtype=torch.int32, device=cuda)
+    dt = torch.float8_e4m3fn if f8 else torch.bfloat16
+    kc = torch.randn(B * nb, Hkv, 16, D, device=cuda).to(dt)
+    vc = torch.randn(B * nb, Hkv, D, 16, device=cuda).to(dt)
+    ws = ops.DecodeWorkspace(B, Hq, D, 128 * nsplit, cuda)
+    out = [torch.full_like(q, 7.0) for _ in range(2)]
+    for o, cnt in zip(out, (ws.cnt, None)):
+        ops.native().attn_decode(q, kc, vc, bt, c, o, ws.o, ws.ml, D ** -0.5, 128, nsplit, 1.0, 1.0, cnt, None, 0, None, None, None, False)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1]) and int(ws.cnt.abs().sum()) == 0
+
+
 def test_qkv_fold_in_graph_replay(cuda, monkeypatch):
     """The folded path in the engine, eager and inside captured multi-step decode graphs: every greedy token is the
     fp32 reference argmax of its prefix up to a bf16 near-tie."""
