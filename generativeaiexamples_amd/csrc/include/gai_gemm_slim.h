@@ -10,6 +10,8 @@ void gai_gemm_slim(const void* A, const void* W, void* C, const void* bias, cons
                    int epi, int out_f32, int nf, int psw, hipStream_t st);
 // out = LayerNorm(A . W^T + bias + R) with K in gai_gemm_slim_ks slices (0: not for this shape); ws: slices x M x N floats
 int gai_gemm_slim_ks(int M, int N, int K);
-void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, float* ws, int psw, hipStream_t st);
+// slices, longer ones first, of a product whose K is deeper than that (0: not for this shape)
+int gai_gemm_slim_few_ks(int M, int N, int K);
+void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, int ks, float* ws, int psw, hipStream_t st);
 void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
                              void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st);

@@ -121,3 +121,7 @@ __device__ __forceinline__ void rotary_half_body(const RotaryHalf<TA>& a, int wg
 }
 
 }  // namespace gai
+
+// gemm_slim.hip: the slices of gai_gemm_slim_few_ks (A . W^T, W in fragment order) beside the rotation of up to 64 rows (heads by 8s)
+void gai_gemm_slim_partials_rotary(const void* A, const void* W, int M, int N, int K, float* ws, const gai::RotaryHalf<gai::bf16>& r,
+                                   hipStream_t st);

@@ -22,6 +22,7 @@
 #include "gai_epilogue.h"
 #include "gai_gemm_slim.h"
 #include "gai_kernels.h"
+#include "gai_rotary.h"
 
 using namespace gai;
 
@@ -31,9 +32,19 @@ constexpr int kWaves = 8;
 constexpr int kMaxSlabs = 8;
 constexpr int kStageBytes = 64 * 1024;     // activation columns of one stage, all rows
 constexpr int kPairK = kWaves * 64;        // k columns of one pair step of the workgroup: 2 x 32 per wave
-// the largest K: every weight fragment of a wave's K share is in registers at once; beyond 2560 only the forms that the rule
-// below takes
+// the largest K of a slice: every weight fragment of a wave's share is in registers at once; beyond 2560 only the forms that the rules
+// below take
 constexpr int max_k(int mt, int nf) { return mt == 4 || nf == 2 ? 2560 : 4096; }
+
+// a product's slices in 512s of K: `each`, the first `longer` of them one more. (Divided on the host: in the kernel it cost every launch of an
+// embedded question 0.06 us.)
+struct Slices {
+  int each, longer;
+  Slices(int K, int slices) : each(K / kPairK / slices), longer(K / kPairK % slices) {}
+  __device__ __forceinline__ int begin(int y) const { return each * y + min(y, longer); }
+  __device__ __forceinline__ int size(int y) const { return each + (y < longer); }
+};
+int slice_k(int K, int slices) { return (K + slices * kPairK - 1) / (slices * kPairK) * kPairK; }  // the longest
 
 template <int EPI, bool OUTF32>
 __device__ __forceinline__ void slim_store4(void* C, const bf16* bias, const bf16* R, int ldc, int m, int n, int M,
@@ -50,27 +61,25 @@ __device__ __forceinline__ void slim_store(void* C, const bf16* bias, const bf16
   else slim_store4<EPI, false>(C, bias, R, ldc, m, n, M, v);
 }
 
-template <int MT, int NF>
-__global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* __restrict__ A,
-                                                                   const bf16* __restrict__ W, void* C,
-                                                                   const bf16* bias, const bf16* R, int M, int N, int K,
-                                                                   int ld, int ldc, int epi, int out_f32, int psw) {
+// K: all of it; slice y of it into slab y of C
+template <int MT, int NF, int STAGE, int MAXK>
+__device__ __forceinline__ void slim_body(const bf16* __restrict__ A, const bf16* __restrict__ W, void* C, const bf16* bias,
+                                          const bf16* R, int M, int N, int K, int y, Slices slices, int ldc, int epi, int out_f32, int psw,
+                                          int bx, char* smem) {
   constexpr int ROWS = 16 * MT;
-  constexpr int KC = kStageBytes / (ROWS * 2);       // columns of a stage
+  constexpr int KC = STAGE / (ROWS * 2);       // columns of a stage
   constexpr int CPR = KC / 8;                        // 16-B chunks of a staged row
   constexpr int P = KC / kPairK;                     // pair steps of a stage
-  constexpr int kMaxPairs = max_k(MT, NF) / kPairK;
+  constexpr int kMaxPairs = MAXK / kPairK;
   constexpr int NST = (kMaxPairs + P - 1) / P;       // stages of the largest K
-  constexpr int DMA = kStageBytes / (64 * kWaves * 16);  // LDS-DMA instructions of a wave and stage
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // 2 stages; reused for the waves' partial tiles
+  constexpr int DMA = STAGE / (64 * kWaves * 16);  // LDS-DMA instructions of a wave and stage
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * 16 * NF;
-  // slice blockIdx.y of a product cut over K: columns [y K, y K + K) of rows ld long, into slab y
-  const int k0 = blockIdx.y * K;
+  const int n0 = bx * 16 * NF;
+  const int ld = K, k0 = slices.begin(y) * kPairK, np = slices.size(y), nst = (np + P - 1) / P;
+  K = np * kPairK;
   A += k0;
-  if (k0) C = (float*)C + (size_t)blockIdx.y * M * N;
-  const int np = K / kPairK, nst = (np + P - 1) / P;
+  if (y) C = (float*)C + (size_t)y * M * N;
   const int r16 = lane & 15, q = lane >> 4;
 
   // ---- every weight fragment of this wave: pair p covers k = p * 512 + 64 wid + {0, 32}
@@ -103,7 +112,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
 
   // ---- activation stage t into slot t & 1: chunk i -> row i / CPR, physical chunk i % CPR = logical ^ (row & 15)
   auto stage = [&](int t) {
-    char* dst = smem + (t & 1) * kStageBytes;
+    char* dst = smem + (t & 1) * STAGE;
 #pragma unroll
     for (int d = 0; d < DMA; ++d) {
       const int base = (d * kWaves + wid) * 64;
@@ -128,7 +137,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
       if (t + 1 < nst) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      const char* src = smem + (t & 1) * kStageBytes;
+      const char* src = smem + (t & 1) * STAGE;
 #pragma unroll
       for (int j = 0; j < P; ++j) {
         if (t * P + j < kMaxPairs && t * P + j < np) {
@@ -194,6 +203,32 @@ __global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* _
   }
 }
 
+// smem: 2 stages; reused for the waves' partial tiles
+template <int MT, int NF>
+__global__ __launch_bounds__(64 * kWaves, 1) void gemm_slim_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, void* C,
+                                                                   const bf16* bias, const bf16* R, int M, int N, int K,
+                                                                   Slices slices, int ldc, int epi, int out_f32, int psw) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  slim_body<MT, NF, kStageBytes, max_k(MT, NF)>(A, W, C, bias, R, M, N, K, blockIdx.y, slices, ldc, epi, out_f32, psw, blockIdx.x, smem);
+}
+
+// The K slices of a product beside the rotation of a step's heads and its cache write (workgroups below `rot`). Two workgroups share a
+// CU, stages of half the size: with one, the last slices waited for the rotations to end (24 rows, 2048 x 5632: 10.9 -> 9.9 us, 11.3 in
+// eleven slices of the streaming kernel; a step of the 2k hybrid stack, 24 streams 363 -> 354 us, one 274 -> 264)
+constexpr int kBesideStage = kStageBytes / 2, kBesideK = 3072;
+template <int MT>
+__global__ __launch_bounds__(64 * kWaves, 4) void gemm_slim_rotary_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                                          float* __restrict__ part, int M, int N, int K, Slices slices,
+                                                                          RotaryHalf<bf16> r, int rot) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int i = (int)blockIdx.x - rot, tiles = N / 16;
+  if (i < 0) {
+    if (threadIdx.x < 256) rotary_half_body<bf16, 8, 1, 1>(r, blockIdx.x, reinterpret_cast<float*>(smem));
+    return;  // (a barrier counts the waves that are left)
+  }
+  slim_body<MT, 1, kBesideStage, kBesideK>(A, W, part, nullptr, nullptr, M, N, K, i / tiles, slices, N, EPI_NONE, 1, 1, i % tiles, smem);
+}
+
 template <int MT, int NF>
 void launch_slim(const void* A, const void* W, void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
                  int epi, int out_f32, int psw, hipStream_t st, int ks = 1) {
@@ -204,9 +239,9 @@ void launch_slim(const void* A, const void* W, void* C, const void* bias, const 
     once = true;
   }
   constexpr int stage_k = kStageBytes / (32 * MT);
-  const size_t lds = (size_t)(K / ks > stage_k ? 2 : 1) * kStageBytes;  // >= the partial tiles (8 MT NF KiB <= 64 KiB)
+  const size_t lds = (size_t)(slice_k(K, ks) > stage_k ? 2 : 1) * kStageBytes;  // >= the partial tiles (8 MT NF KiB <= 64 KiB)
   gemm_slim_kernel<MT, NF><<<dim3((N + 16 * NF - 1) / (16 * NF), ks), 64 * kWaves, lds, st>>>(
-      (const bf16*)A, (const bf16*)W, C, (const bf16*)bias, (const bf16*)R, M, N, K / ks, K, ldc, epi, out_f32, psw);
+      (const bf16*)A, (const bf16*)W, C, (const bf16*)bias, (const bf16*)R, M, N, K, Slices(K, ks), ldc, epi, out_f32, psw);
   GAI_LAUNCH_CHECK();
 }
 
@@ -319,13 +354,43 @@ int gai_gemm_slim_ks(int M, int N, int K) {
   return 0;
 }
 
+// Slices of a deeper product of up to 32 rows for a norm that adds them: the fewest that fit a workgroup's registers (two share a CU where
+// a rotation is beside them), where all fit the chip at once; the first ones are longer by 512 where K does not divide. Which products
+// take them: gemm_splitk.hip
+int gai_gemm_slim_few_ks(int M, int N, int K) {
+  if (M < 1 || M > 32 || N < 16 || N % 16 || N > 2048 || K < kPairK || K % kPairK || gai_gemm_slim_nf(M, N, K, false)) return 0;
+  for (int ks = 2; ks <= kMaxSlabs && N / 16 * ks <= 256; ++ks)
+    if (slice_k(K, ks) <= kBesideK) return ks;
+  return 0;
+}
+
 // those slices, [ks][M][N]
-void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, float* ws, int psw, hipStream_t st) {
-  const int ks = gai_gemm_slim_ks(M, N, K);
+void gai_gemm_slim_partials(const void* A, const void* W, int M, int N, int K, int ks, float* ws, int psw, hipStream_t st) {
   if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_slim_partials: the shape has no slices");
   if (M <= 16) launch_slim<1, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
   else if (M <= 32) launch_slim<2, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
   else launch_slim<4, 1>(A, W, ws, nullptr, nullptr, M, N, K, N, EPI_NONE, 1, psw, st, ks);
+}
+
+// gai_gemm_slim_few_ks of a weight in fragment order beside the rotation r (T rows, a head's channels by 8s)
+void gai_gemm_slim_partials_rotary(const void* A, const void* W, int M, int N, int K, float* ws, const RotaryHalf<bf16>& r,
+                                   hipStream_t st) {
+  const int ks = gai_gemm_slim_few_ks(M, N, K), rot = 2 * r.T;
+  if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_slim_partials_rotary: the shape has no slices");
+#define GAI_SR(MT)                                                                                                                       \
+  {                                                                                                                                      \
+    static bool once = false;                                                                                                            \
+    if (!once) {                                                                                                                         \
+      hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_slim_rotary_kernel<MT>), hipFuncAttributeMaxDynamicSharedMemorySize,        \
+                          2 * kBesideStage);                                                                                             \
+      once = true;                                                                                                                       \
+    }                                                                                                                                    \
+    gemm_slim_rotary_kernel<MT><<<rot + N / 16 * ks, 64 * kWaves, 2 * kBesideStage, st>>>((const bf16*)A, (const bf16*)W, ws, M, N, K,     \
+                                                                                         Slices(K, ks), r, rot);                         \
+  }
+  if (M <= 16) GAI_SR(1) else GAI_SR(2)
+#undef GAI_SR
+  GAI_LAUNCH_CHECK();
 }
 
 bool gai_slabs_layernorm_ok(int ks, int N) { return ks >= 1 && ks <= kMaxSlabs && N <= 2048 && N % 8 == 0; }
@@ -350,6 +415,7 @@ void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* 
 
 void gai_gemm_slim_layernorm(const void* A, const void* W, const void* bias, const void* R, const void* g, const void* b,
                              void* out, int M, int N, int K, float eps, float* ws, int psw, hipStream_t st) {
-  gai_gemm_slim_partials(A, W, M, N, K, ws, psw, st);
-  gai_slabs_layernorm(ws, gai_gemm_slim_ks(M, N, K), bias, R, g, b, out, M, N, eps, st);
+  const int ks = gai_gemm_slim_ks(M, N, K);
+  gai_gemm_slim_partials(A, W, M, N, K, ks, ws, psw, st);
+  gai_slabs_layernorm(ws, ks, bias, R, g, b, out, M, N, eps, st);
 }

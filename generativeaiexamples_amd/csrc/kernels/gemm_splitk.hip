@@ -531,9 +531,12 @@ int legacy_ks(int M, int N, int K) {
 // register-streamed kernel wins on the wide (gate_up, lm_head: 1.1-1.3x) and deep (down: 1.1-1.4x)
 // projections; the LDS-staged one stays ahead on the square K = 4096 ones (QKV, O) by 2-10 %.
 // GAI_SPLITK_V = 1 / 2 forces the legacy / streamed variant.
-bool use_legacy(int N, int K) {
+int asked_variant() {
   static const int v = getenv("GAI_SPLITK_V") ? atoi(getenv("GAI_SPLITK_V")) : 0;
-  if (v) return v == 1;
+  return v;
+}
+bool use_legacy(int N, int K) {
+  if (asked_variant()) return asked_variant() == 1;
   return K % kKAlign == 0 && K <= 4096 && N <= 8192;
 }
 
@@ -551,9 +554,23 @@ int stream_ks(int N, int K) {
   return units;
 }
 
+// Up to 32 rows whose streamed slices are more workgroups than CUs (K / 512 is what they come in: 11 of 5632) take a few uneven ones of
+// gemm_slim.hip. Product and the hybrid norm that adds the slices, 24 rows, fragment order | row-major, us: 2048 x 4608 16.0 | 19.8 -> 13.3 |
+// 14.2, 2048 x 5632 16.4 | 20.2 -> 13.9 | 15.1, 1024 x 5632 13.6 | 15.2 -> 11.8 | 13.2, one row of that 11.1 | 12.7 -> 9.7 | 11.3. Where they
+// fit one round the stream is faster: 2048 x 6144 in eight 13.4 (13.9 in two), 1024 x 8192 in sixteen 11.9 (13.2). Past 32 rows the
+// rotations beside them (two a row) take the CUs that the slices would.
+int slim_few(int M, int N, int K) {
+  if (asked_variant() || use_legacy(N, K) || gai_gemm_slim_nf(M, N, K, false) || gai_gemm_dec2_partials_ks(M, N, K)) return 0;
+  return (N + 63) / 64 * stream_ks(N, K) > 256 ? gai_gemm_slim_few_ks(M, N, K) : 0;
+}
+
 }  // namespace
 
-int gai_gemm_splitk_ks(int M, int N, int K) { return use_legacy(N, K) ? legacy_ks(M, N, K) : stream_ks(N, K); }
+int gai_gemm_splitk_ks(int M, int N, int K) {
+  if (use_legacy(N, K)) return legacy_ks(M, N, K);
+  const int few = slim_few(M, N, K);
+  return few ? few : stream_ks(N, K);
+}
 
 size_t gai_gemm_splitk_ws_bytes(int M, int N, int K) {
   const int KS = max(gai_gemm_splitk_ks(M, N, K), gai_gemm_dec2_partials_ks(M, N, K));
@@ -630,6 +647,7 @@ int waves_per_wg(int N, int KS) {
 void launch_partials(const void* A, const void* B, int M, int N, int K, int KS, float* ws, int psw, hipStream_t st) {
   const int MB = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   if (!use_legacy(N, K)) {
+    if (slim_few(M, N, K)) return gai_gemm_slim_partials(A, B, M, N, K, KS, ws, psw, st);
     if (MB == 1) launch_stream<1, EPI_NONE, true>(A, B, nullptr, nullptr, nullptr, M, N, K, 0, KS, ws, psw, st);
     else if (MB == 2) launch_stream<2, EPI_NONE, true>(A, B, nullptr, nullptr, nullptr, M, N, K, 0, KS, ws, psw, st);
     else launch_stream<4, EPI_NONE, true>(A, B, nullptr, nullptr, nullptr, M, N, K, 0, KS, ws, psw, st);
@@ -987,7 +1005,7 @@ int gai_gemm_partials_ks(int M, int N, int K) {
 void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st) {
   const int ks = gai_gemm_partials_ks(M, N, K);
   if (ks == 0) gai_launch_error(__FILE__, __LINE__, "gemm_partials: the product has no slices");
-  if (gai_gemm_slim_nf(M, N, K, false)) gai_gemm_slim_partials(A, B, M, N, K, ws, psw, st);
+  if (gai_gemm_slim_nf(M, N, K, false)) gai_gemm_slim_partials(A, B, M, N, K, ks, ws, psw, st);
   else if (!gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw)) launch_partials(A, B, M, N, K, ks, ws, psw, st);
 }
 
@@ -996,12 +1014,17 @@ int gai_gemm_partials_rotary(const void* A, const void* B, int M, int N, int K, 
                              const void* v, int ldv, const int* positions, const int* slots, void* q_out, void* k_cache, void* v_cache, int T,
                              int H, int G, int DK, int DV, const double* inv_freq, int half, float unit_eps, hipStream_t st) {
   const int ks = gai_gemm_partials_ks(M, N, K), per = DK / 8;
-  if (ks == 0 || gai_gemm_slim_nf(M, N, K, false) || gai_gemm_dec2_partials_ks(M, N, K) || use_legacy(N, K)) return 0;
+  const bool few = slim_few(M, N, K) > 0;
+  if (ks == 0 || gai_gemm_slim_nf(M, N, K, false) || (!few && (gai_gemm_dec2_partials_ks(M, N, K) || use_legacy(N, K)))) return 0;
   const bool on8 = DK % 8 == 0 && half % 8 == 0 && ldq % 8 == 0 && ldk % 8 == 0 &&
                    (((size_t)q | (size_t)k | (size_t)q_out | (size_t)k_cache) & 15) == 0;
   if (T < 1 || T > 64 || half < 0 || 2 * half > DK || !on8 || per > 64 || (per & (per - 1))) return 0;
   const RotaryHalf<bf16> r{(const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, positions, slots, (bf16*)q_out, (bf16*)k_cache,
                            (bf16*)v_cache, T, H, G, DK, DV, inv_freq, half, unit_eps, per};
+  if (few) {
+    gai_gemm_slim_partials_rotary(A, B, M, N, K, ws, r, st);
+    return 1;
+  }
 #define GAI_DR(MB)                                                                                                                     \
   {                                                                                                                                    \
     static bool once = false;                                                                                                          \

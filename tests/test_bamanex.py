@@ -212,7 +212,8 @@ def test_parallel_add_norm_kept_groups(D):
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,D,K,form", [(1, 512, 512, "rows"), (24, 2048, 5632, "split"), (24, 2048, 2048, "cut"), (64, 2048, 11264, "split"),
                                         (17, 1040, 4096, "cut"), (3, 16, 1024, "cut"), (33, 1024, 5120, "split"), (65, 2048, 2048, "rows"),
-                                        (5, 2064, 5632, "rows")])
+                                        (5, 2064, 5632, "rows"), (1, 2048, 4608, "split"), (16, 1024, 5632, "split"), (32, 1040, 5120, "split"),
+                                        (9, 2048, 6656, "split")])
 def test_branches_as_k_slices(cuda, T, D, K, form):
     """A branch handed over as its product's K slices: the rows that adding them in order and rounding once gives (the stream's bits),
     normed alike up to the order of the squares' sum, in either branch, beside rows or alone, with and without bias and scale. "split": the
