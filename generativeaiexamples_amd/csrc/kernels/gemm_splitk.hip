@@ -387,7 +387,7 @@ __global__ __launch_bounds__(256, 2) void gemm_dec_kernel(const bf16* __restrict
 
 // The K slices of a product beside the rotation of a step's heads and its cache write (workgroups below `rot`), which wait for nothing of
 // each other in a layer of parallel branches. 24 rows: product 10.0 us, rotation 5.2 by itself, 10.7 together; a step of the 2k hybrid stack,
-// 24 streams 389 -> 361 us, one 299 -> 274, 64 540 -> 500.
+// 24 streams 389 -> 361 us, one 299 -> 274, 64 540 -> 500. (Up to 32 rows of such a product share gemm_slim.hip's launch now: slim_few.)
 template <int MB>
 __global__ __launch_bounds__(256, 2) void gemm_dec_rotary_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
                                                                  float* __restrict__ part, int M, int N, int K, int KW, int KS,

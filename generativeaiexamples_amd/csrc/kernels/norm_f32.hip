@@ -771,8 +771,8 @@ namespace {
 // rounded to bf16, instead of a launch of its own that writes rows for this one to read (the bits of the reduction of a product that is
 // split over K by itself; the narrow ones that are one pass over K are cut for this). A workgroup a row, four channels a thread (so 2048
 // channels, with 512 threads), every load (16 slices of each branch) in flight before the first is used; bound by that round trip.
-// 24 rows of 2048, slices of 2 and 11: reduction + norm 4.6 + 6.2 us under the profiler, here 7.7; the product in front of the first branch
-// 6.1 -> 4.8 in two slices.
+// 24 rows of 2048, slices of 2 and 11: reduction + norm 4.6 + 6.2 us under the profiler, here 7.7 (of 2 and 2 6.6; with the branches' scales
+// among the loads 6.4, a hybrid step 353.3 -> 350.6); the product in front of the first branch 6.1 -> 4.8 in two slices.
 struct SlabBranch {
   const float* slabs;  // [ks][T][D], or null:
   const bf16* rows;    // rows ld apart, or null: no branch
@@ -790,9 +790,12 @@ __global__ __launch_bounds__(512) void slabs_add_norm_kernel(float* __restrict__
   const int row = blockIdx.x, own = threadIdx.x * 4, i = min(own, D - 4);  // threads past the row read its last again
   const size_t slab = (size_t)T * D, at = (size_t)row * D + i;
   f32x4 x = *reinterpret_cast<const f32x4*>(res + at);
-  f32x4 sa[kSlabsAhead], sb[kSlabsAhead], g1 = {}, g2 = {};
+  f32x4 sa[kSlabsAhead], sb[kSlabsAhead], ca = {1.f, 1.f, 1.f, 1.f}, cb = ca, g1 = {}, g2 = {};
   bf16x4 ya = {}, yb = {}, ba = {}, bb = {};
-  auto ahead = [&](const SlabBranch& r, f32x4(&s)[kSlabsAhead], bf16x4& y, bf16x4& bias) {
+  auto ahead = [&](const SlabBranch& r, f32x4(&s)[kSlabsAhead], bf16x4& y, bf16x4& bias, f32x4& c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (r.scale) c[e] = r.scale[i + e];
     if (r.slabs) {
 #pragma unroll
       for (int k = 0; k < kSlabsAhead; ++k)
@@ -802,14 +805,14 @@ __global__ __launch_bounds__(512) void slabs_add_norm_kernel(float* __restrict__
       y = *reinterpret_cast<const bf16x4*>(r.rows + (size_t)row * r.ld + i);
     }
   };
-  ahead(a, sa, ya, ba);
-  ahead(b, sb, yb, bb);
+  ahead(a, sa, ya, ba, ca);
+  ahead(b, sb, yb, bb, cb);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {  // norm weights may lie on 4 bytes
     if (h1) g1[e] = w1[i + e];
     if (h2) g2[e] = w2[i + e];
   }
-  auto add = [&](const SlabBranch& r, const f32x4(&s)[kSlabsAhead], bf16x4 y, const bf16x4& bias) {
+  auto add = [&](const SlabBranch& r, const f32x4(&s)[kSlabsAhead], bf16x4 y, const bf16x4& bias, const f32x4& c) {
     if (!r.slabs && !r.rows) return;
     if (r.slabs) {
       f32x4 v = {};
@@ -821,10 +824,10 @@ __global__ __launch_bounds__(512) void slabs_add_norm_kernel(float* __restrict__
       for (int e = 0; e < 4; ++e) y[e] = (bf16)(r.bias ? v[e] + (float)bias[e] : v[e]);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = fmaf(r.scale ? r.scale[i + e] : 1.0f, (float)y[e], x[e]);
+    for (int e = 0; e < 4; ++e) x[e] = fmaf(c[e], (float)y[e], x[e]);
   };
-  add(a, sa, ya, ba);
-  add(b, sb, yb, bb);
+  add(a, sa, ya, ba, ca);
+  add(b, sb, yb, bb, cb);
   if (own < D) *reinterpret_cast<f32x4*>(res + at) = x;
   if (!h1 && !h2) return;
   const float s = own < D ? x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3] : 0.f;
