@@ -554,7 +554,7 @@ int stream_ks(int N, int K) {
   return units;
 }
 
-// Up to 32 rows whose streamed slices are more workgroups than CUs (K / 512 is what they come in: 11 of 5632) take a few uneven ones of
+// Up to 32 rows whose streamed slices are more workgroups than CUs (their number divides K / 128: 11 of 5632) take a few uneven ones of
 // gemm_slim.hip. Product and the hybrid norm that adds the slices, 24 rows, fragment order | row-major, us: 2048 x 4608 16.0 | 19.8 -> 13.3 |
 // 14.2, 2048 x 5632 16.4 | 20.2 -> 13.9 | 15.1, 1024 x 5632 13.6 | 15.2 -> 11.8 | 13.2, one row of that 11.1 | 12.7 -> 9.7 | 11.3. Where they
 // fit one round the stream is faster: 2048 x 6144 in eight 13.4 (13.9 in two), 1024 x 8192 in sixteen 11.9 (13.2). Past 32 rows the
