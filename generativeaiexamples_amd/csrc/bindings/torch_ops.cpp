@@ -290,7 +290,8 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
 // layer (g, b; res is only read). False, and nothing launched, where the product has no such plan, an operand is not on 16 bytes
 // or there is no memory for the slabs.
 bool slabs_plan(int64_t M, int64_t N, int64_t K, bool layer, GaiMidPlan* plan) {
-  return layer ? gai_slabs_layernorm_ok(1, N) && gai_gemm_mid_slabs_plan(M, N, K, 8, plan) : N >= 2048 && gai_gemm_mid_slabs_plan(M, N, K, 16, plan);
+  return layer ? gai_slabs_layernorm_ok(1, N) && gai_gemm_mid_slabs_plan(M, N, K, 8, true, plan)
+               : N >= 2048 && gai_gemm_mid_slabs_plan(M, N, K, 16, false, plan);
 }
 
 bool linear_slabs_norm(const Tensor& A, const Tensor& W, const optional<Tensor>& bias, Tensor& res, const Tensor& g,

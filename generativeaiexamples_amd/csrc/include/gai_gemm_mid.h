@@ -23,9 +23,9 @@ void gai_gemm_mid(const void* A, const void* B, void* C, const void* bias, const
 // round of tiles (0: none), with the same sums; *plan is for those rows
 int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* bias, const void* R, int M, int N, int K, int ldc,
                       int epi, int out_f32, int bfrag, GaiMidPlan* plan);
-// The same kernel's parts as fp32 slabs [parts][M][N] for a launch that adds them with what follows (a norm): false where the parts
-// with their own sum, or one part, are expected to be faster. The plan is one for both layouts of the weight, rows on 16 bytes.
-// most: the parts that launch takes.
-bool gai_gemm_mid_slabs_plan(int M, int N, int K, int most, GaiMidPlan* plan);
+// The same kernel's parts as fp32 slabs [parts][M][N] for a launch that adds them with what follows (a layer or rms norm): false where the
+// product with its own sums and residual, and the norm, are expected to be faster. The plan is one for both layouts of the weight, rows
+// on 16 bytes. most: the parts that launch takes.
+bool gai_gemm_mid_slabs_plan(int M, int N, int K, int most, bool layer, GaiMidPlan* plan);
 void gai_gemm_mid_slabs(const void* A, const void* B, int M, int N, int K, const GaiMidPlan& plan, float* ws, hipStream_t st,
                         int bfrag);

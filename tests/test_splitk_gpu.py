@@ -374,6 +374,15 @@ def test_parts_added_by_the_rms_norm(cuda, M, N, K, parts, bias):
     assert torch.equal(seen[0][0], seen[1][0]) and torch.equal(seen[0][1], seen[1][1])
 
 
+@pytest.mark.parametrize("M,N,K,layer,taken", [(385, 2048, 1024, False, False), (513, 4096, 3072, False, False), (400, 2048, 2048, False, True),
+                                               (500, 2048, 3072, False, True), (513, 4096, 4096, False, True), (385, 1536, 768, True, False),
+                                               (513, 1536, 1024, True, False), (65, 2048, 3072, True, False), (65, 2048, 1024, True, True),
+                                               (385, 768, 1536, True, True)])
+def test_slabs_where_they_are_the_faster_way(cuda, M, N, K, layer, taken):
+    """Both sides of the line (timed at gai_gemm_mid_slabs_plan): products whose own sums and a norm after them take less are left to those."""
+    assert (ops.native().gemm_slabs_parts(M, N, K, layer) > 1) == taken
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 1024, 1024), (187, 1024, 4096), (320, 768, 3072), (500, 384, 1536), (300, 2048, 4096), (640, 1024, 4096)])
 def test_parts_added_by_the_layer_norm(cuda, M, N, K):
     """The same before a layer norm (error as in test_product_in_slices_and_norm), and rows with nothing beside them."""
