@@ -82,6 +82,7 @@ int gai_attn_rows_heads(int H, int longest);
 void gai_attn_rows_slabs(const void* qkv, int ld, const int* cu_q, const int* ctx_lens, int seqs, int longest, const void* W, float* ws, int M,
                          int N, int H, float scale, int frag, hipStream_t st);
 bool gai_slabs_layernorm_ok(int ks, int N);
+int gai_slabs_layernorm_reads(int ks, int N);
 void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* R, const void* g, const void* b, void* out, int M, int N,
                          float eps, hipStream_t st);
 int gai_attn_prefill_rows_per_tile(int Hq, int Hkv, int D = 128);

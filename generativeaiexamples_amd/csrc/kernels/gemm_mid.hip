@@ -524,12 +524,14 @@ int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* b
 // and 26.2 | 22.4, 96 rows 38.6 | 31.6 and 21.8 | 17.2, 640 rows 97.0 | 94.2 and 45.6 | 40.7.
 // The model: 3336 timings of 200 products (65 to 640 rows, N 2048 to 8192, K 2048 to 14336), nine in ten within 13 %, and for the choice
 // product and norm together, here and as they would run without slabs (the plan of the product that adds its own residual, or the kernels
-// past this one), fitted to both ways of 1888 products (N 2048 to 8192 before a rms norm, 256 to 2048 before a layer norm, both layouts),
-// nine in ten within 10 %. A layer norm's wave reads a row's slabs by itself, so wide rows in many parts cost it most. Of 1888 the rule
-// takes 1722: before a rms norm 0.85 of the time on average, before a layer norm 0.79; the slowest, us: 160 rows 5120 x 14336 53.5 | 54.3 (row-major
-// 55.2 | 56.9), 8192 x 14336 89.8 | 70.7 (72.9 | 74.3). Without the comparison 385 x 2048 x 1024 took 13.1 instead of 12.3, before a layer norm 385 x 1536 x
-// 768 12.5 instead of 11.2 and 65 x 2048 x 3072 18.3 instead of 17.1; past 512 rows two short parts fill the pipeline too often (513 x 4096 x
-// 3072 31.9 instead of 30.3). At 1000 rows the slabs' bytes cost more than the sums did (46.4 | 48.2, 126.9 | 131.2).
+// past this one), fitted to both ways of 2588 products (N 2048 to 8192 before a rms norm, 256 to 2048 before a layer norm, both layouts),
+// nine in ten within 10 %. A layer norm's wave reads a row's slabs by itself, so wide rows in many parts cost it most. The rule takes 2262
+// of these: before a rms norm 0.85 of the time on average, before a layer norm 0.80; the slowest, us: 160 rows 5120 x 14336 53.5 | 54.3 (row-major
+// 55.2 | 56.9), 8192 x 14336 89.8 | 70.7 (72.9 | 74.3); of 700 others that it takes six are more than 1 % slower in fragment order, 417 x 1536 x 1280
+// before a layer norm 13.1 | 13.8 the most, and 142 x 7328 x 12288 60.6 | 62.8 (62.5 | 69.0). Without the comparison 385 x 2048 x 1024 took 13.1 instead of 12.3, before a layer norm 385 x 1536 x
+// 768 12.5 instead of 11.2, 65 x 2048 x 3072 18.3 instead of 17.1 and 212 x 1088 x 1920 15.8 instead of 14.5; past 512 rows two short parts
+// fill the pipeline too often (513 x 4096 x 3072 31.9 instead of 30.3). At 1000 rows the slabs' bytes cost more than the sums did (46.4 |
+// 48.2, 126.9 | 131.2).
 namespace {
 struct SlabFit {
   double base, alone, full, weights, few, slabs, round;  // as MidFit; slabs: GB/s / 1000 written; round: each past the first
@@ -537,13 +539,14 @@ struct SlabFit {
 constexpr SlabFit kSlabFit[3] = {{2.9, 0.54, 0.64, 4.66, 0.31, 2.8, 0.43}, {4.7, 0.77, 1.0, 5.75, 0.39, 4.24, 2.97}, {6.8, 1.0, 1.23, 4.65, 1.0, 4.0, 5.25}};
 constexpr double kSlabRead = 0.141, kSlabRows = 0.78e-6;  // the norm: us a MB of slabs, an element of the rows past 256
 constexpr double kSlabMargin = 0.95;
-// product and norm, us: base + slope x modelled product + row x (columns x parts) + elem x (elements x parts), against the same without
-// slabs; least: what has to be saved at least
+// product and norm, us: base + slope x modelled product + read x the norm's reads of slabs one after another + elem x (elements x parts), against
+// the same without slabs; least: what has to be saved at least
 struct SlabNormFit {
-  double base, slope, row, elem, was_base, was_slope, was_elem, least;
+  double base, slope, read, elem, was_base, was_slope, was_elem, least;
 };
-constexpr SlabNormFit kSlabRms = {4.1, 0.92, 0.0, 0.25e-6, 2.7, 0.97, 1.8e-6, 1.4}, kSlabLayer = {3.0, 0.93, 4.5e-4, 0.275e-6, 1.4, 1.01, 2.45e-6, 0.8};
-constexpr double kSlabShare = 0.94;
+constexpr SlabNormFit kSlabRms = {4.31, 0.911, 2.05, 0.192e-6, 2.55, 0.974, 1.975e-6, 1.4};
+constexpr SlabNormFit kSlabLayer = {2.76, 0.93, 0.194, 0.349e-6, 1.41, 1.021, 2.354e-6, 0.8};
+constexpr double kSlabShare = 0.95;
 
 double slabs_cost(int M, int N, int K, int v, int S) {
   const SlabFit& f = kSlabFit[v];
@@ -574,7 +577,8 @@ bool gai_gemm_mid_slabs_plan(int M, int N, int K, int most, bool layer, GaiMidPl
   GaiMidPlan was;
   const double product = gai_gemm_mid_plan(nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, N, epi, 0, 0, 1, &was) ? was.cost : other_cost(M, N, K, epi);
   const SlabNormFit& f = layer ? kSlabLayer : kSlabRms;
-  const double now = f.base + f.slope * more + plan->parts * (f.row * N + f.elem * M * N);
+  const int reads = layer ? gai_slabs_layernorm_reads(plan->parts, N) : N > 4096;  // (a rms norm of wider rows has fewer waves a row)
+  const double now = f.base + f.slope * more + f.read * reads + f.elem * M * N * plan->parts;
   const double then = f.was_base + f.was_slope * product + f.was_elem * M * N;
   return now < kSlabShare * then && then - now > f.least;
 }

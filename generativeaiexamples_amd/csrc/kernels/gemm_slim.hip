@@ -395,6 +395,9 @@ void gai_gemm_slim_partials_rotary(const void* A, const void* W, int M, int N, i
 
 bool gai_slabs_layernorm_ok(int ks, int N) { return ks >= 1 && ks <= kMaxSlabs && N <= 2048 && N % 8 == 0; }
 
+// the 16-byte pairs of a slab's row that a lane of it asks for: chunks of 512 columns, times the slabs that its kernel is built for
+int gai_slabs_layernorm_reads(int ks, int N) { return (N <= 512 ? 1 : N <= 1024 ? 2 : 4) * (ks <= 2 ? 2 : ks <= 4 ? 4 : kMaxSlabs); }
+
 void gai_slabs_layernorm(const float* ws, int ks, const void* bias, const void* R, const void* g, const void* b, void* out, int M, int N,
                          float eps, hipStream_t st) {
   if (!gai_slabs_layernorm_ok(ks, N)) gai_launch_error(__FILE__, __LINE__, "slabs_layernorm: shape");

@@ -377,7 +377,7 @@ def test_parts_added_by_the_rms_norm(cuda, M, N, K, parts, bias):
 @pytest.mark.parametrize("M,N,K,layer,taken", [(385, 2048, 1024, False, False), (513, 4096, 3072, False, False), (400, 2048, 2048, False, True),
                                                (500, 2048, 3072, False, True), (513, 4096, 4096, False, True), (385, 1536, 768, True, False),
                                                (513, 1536, 1024, True, False), (65, 2048, 3072, True, False), (65, 2048, 1024, True, True),
-                                               (385, 768, 1536, True, True)])
+                                               (385, 768, 1536, True, True), (212, 1088, 1920, True, False), (364, 1040, 4352, True, False)])
 def test_slabs_where_they_are_the_faster_way(cuda, M, N, K, layer, taken):
     """Both sides of the line (timed at gai_gemm_mid_slabs_plan): products whose own sums and a norm after them take less are left to those."""
     assert (ops.native().gemm_slabs_parts(M, N, K, layer) > 1) == taken
