@@ -376,9 +376,18 @@ bool dec2_shape_ok(int NT, int K) {
   return (KW / 32) % L == 0;
 }
 
+bool dec2_off() {
+  static const bool off = getenv("GAI_DEC2") && atoi(getenv("GAI_DEC2")) == 0;
+  return off;
+}
+int dec2_asked_nt() {
+  static const int nt = getenv("GAI_DEC2_NT") ? atoi(getenv("GAI_DEC2_NT")) : 0;
+  return nt;
+}
+
 template <int MB>
 int dec2_pick_nt(int N, int K, bool swiglu) {
-  static const int force = getenv("GAI_DEC2_NT") ? atoi(getenv("GAI_DEC2_NT")) : 0;
+  const int force = dec2_asked_nt();
   // 64: measured on MI355X (profiles/r2/dec2_minwg_sweep.txt) the widest tile wins on the wide shapes
   // (gate_up+SwiGLU at M = 64: 54.9 us with 224 workgroups vs 66.4 us with 448): every workgroup re-stages
   // the whole activation K range, so fewer, wider workgroups move fewer bytes through the load path
@@ -422,8 +431,7 @@ int gai_gemm_dec2_ok(int M, int N, int K, int epi) {
   static const int min_n = getenv("GAI_DEC2_MINN") ? atoi(getenv("GAI_DEC2_MINN")) : 16384;
   const bool shallow_shard = N >= 8192 && K <= 4096 && !getenv("GAI_DEC2_MINN");
   if (M < 1 || M > 64 || N % 16 || (N < min_n && !shallow_shard) || (epi_glu(epi) && N % 32)) return 0;
-  static const bool off = getenv("GAI_DEC2") && atoi(getenv("GAI_DEC2")) == 0;
-  if (off) return 0;
+  if (dec2_off()) return 0;
   const bool sw = epi_glu(epi);
   if (M <= 16) return dec2_pick_nt<1>(N, K, sw) > 0;
   if (M <= 32) return dec2_pick_nt<2>(N, K, sw) > 0;
@@ -445,6 +453,7 @@ bool gai_gemm_dec2(const void* A, const void* W, void* C, const void* bias, cons
 
 // GeGLU(A1 . W1^T) and A2 . W2^T + bias of M rows in one launch, weights in fragment order; 0: not for this shape, nothing launched.
 int gai_gemm_dec2_pair_ok(int M, int N1, int N2, int K) {
+  if (dec2_off() || (dec2_asked_nt() && dec2_asked_nt() != 4)) return 0;
   if (M < 1 || M > 64 || N1 % 32 || N2 % 16 || N1 < 16 || N2 < 16 || K % 256) return 0;
   return M <= 16 ? dec2_shape_ok<1>(4, K) : M <= 32 ? dec2_shape_ok<2>(4, K) : dec2_shape_ok<4>(4, K);
 }
@@ -519,9 +528,8 @@ int dec2_part_run(const void* A, const void* W, int M, int N, int K, float* ws, 
 int dec2_part_dispatch(const void* A, const void* W, int M, int N, int K, float* ws, hipStream_t st, bool launch,
                        bool psw = false) {
   static const int min_k = getenv("GAI_DEC2_PART_MINK") ? atoi(getenv("GAI_DEC2_PART_MINK")) : 8192;
-  static const bool off = getenv("GAI_DEC2") && atoi(getenv("GAI_DEC2")) == 0;
   // M <= 16: the register-streamed split-K kernel is faster (down at M = 1: 30 vs 34 us)
-  if (off || M <= 16 || M > 64 || N % 16 || K < min_k) return 0;
+  if (dec2_off() || M <= 16 || M > 64 || N % 16 || K < min_k) return 0;
   if (psw) return M <= 32 ? dec2_part_run<2, true>(A, W, M, N, K, ws, st, launch)
                           : dec2_part_run<4, true>(A, W, M, N, K, ws, st, launch);
   if (M <= 32) return dec2_part_run<2, false>(A, W, M, N, K, ws, st, launch);

@@ -1,5 +1,5 @@
 """The environment switches of the decode kernels: of the attention, read in Python and by the launcher (both have to choose the same
-kernel), and of the split-K products."""
+kernel), and of the decode products."""
 import ctypes
 import os
 import subprocess
@@ -30,6 +30,19 @@ def test_split_k_waves_as_asked(asked, want):
     if asked is not None:
         env["GAI_SPLITK_WPG"] = asked
     code = "from generativeaiexamples_amd import ops; print([ops.native().gemm_splitk_waves(*s) for s in ((6144, 4), (4096, 8), (128, 2))])"
+    p = subprocess.run([sys.executable, "-c", code], env=env, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0 and p.stdout.split("\n")[0] == str(want), p.stdout + p.stderr
+
+
+@pytest.mark.skipif(not ops.native_available(), reason="the kernels are not built")
+@pytest.mark.parametrize("switch,value,want", [(None, None, 1), ("GAI_DEC2", "0", 0), ("GAI_DEC2", "1", 1), ("GAI_DEC2_NT", "8", 0), ("GAI_DEC2_NT", "4", 1)])
+def test_pair_of_products_as_asked(switch, value, want):
+    """Two products in one launch of the LDS-staged kernel: off with it, and where column tiles of another width are asked for."""
+    env = {k: v for k, v in os.environ.items() if not k.startswith("GAI_DEC2")}
+    if switch is not None:
+        env[switch] = value
+    code = "from generativeaiexamples_amd import ops; print(int(ops.native().gemm_dec2_pair_ok(24, 11264, 3088, 2048)))"
     p = subprocess.run([sys.executable, "-c", code], env=env, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                        capture_output=True, text=True, timeout=300)
     assert p.returncode == 0 and p.stdout.split("\n")[0] == str(want), p.stdout + p.stderr
