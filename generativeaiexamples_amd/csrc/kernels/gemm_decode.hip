@@ -451,10 +451,19 @@ bool gai_gemm_dec2(const void* A, const void* W, void* C, const void* bias, cons
   return dec2_run<4, false>(A, W, C, bias, R, M, N, K, ldc, epi, out_f32, st);
 }
 
-// GeGLU(A1 . W1^T) and A2 . W2^T + bias of M rows in one launch, weights in fragment order; 0: not for this shape, nothing launched.
+// GeGLU(A1 . W1^T) and A2 . W2^T + bias of M rows in one launch, weights in fragment order; 0: not for this shape, or the two launches are
+// faster. Its column tiles are 64 wide whatever the shape. Timed against the two at 2046 shapes (M 1 to 64, N1 1024 to 28672, N2 512 to 8192, K
+// 512 to 6144, captured, weights from HBM): while every workgroup has a CU it takes 0.44 - 0.99 of their time, but for few tiles of a
+// deep product, which leave CUs idle that slices of K would use (24 rows, 1024 + 1024 columns, K 6144 17.7 us in two, 21.4 in one; K 4096 up
+// to 64 tiles 0.85 - 1.04). With a few more tiles than CUs some CUs do twice the work (14336 + 3088, K 2048 20.1 -> 21.5, 4096 35.4 -> 39.6);
+// from 336 on to two each it is ahead again (18432 + 6144, K 2048 0.72 - 0.78), at more than 32 rows of a deep product too rarely: the
+// gated product by itself takes 128 columns a workgroup there (28672 + 512, K 4096, 64 rows 50.9 -> 52.7), and past two each it is slower
+// still (28672 + 6144, K 4096, 64 rows 59.8 -> 71.0). K up to 1024: 0.54 - 0.99 at any width. Over the shapes taken 0.74 on average.
 int gai_gemm_dec2_pair_ok(int M, int N1, int N2, int K) {
   if (dec2_off() || (dec2_asked_nt() && dec2_asked_nt() != 4)) return 0;
   if (M < 1 || M > 64 || N1 % 32 || N2 % 16 || N1 < 16 || N2 < 16 || K % 256) return 0;
+  const int tiles = (N1 + 63) / 64 + (N2 + 63) / 64;
+  if (tiles <= 256 ? K >= 4096 && tiles <= 64 : K > 1024 && (tiles < 336 || tiles > 512 || (K > 3072 && M > 32))) return 0;
   return M <= 16 ? dec2_shape_ok<1>(4, K) : M <= 32 ? dec2_shape_ok<2>(4, K) : dec2_shape_ok<4>(4, K);
 }
 void gai_gemm_dec2_pair(const void* A1, const void* W1, void* C1, int N1, const void* A2, const void* W2, const void* bias, void* C2, int N2,

@@ -330,9 +330,10 @@ def test_product_in_slices_and_norm(cuda, M, N, K, ks, frag):
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
-@pytest.mark.parametrize("N1,N2,K,one", [(11264, 3088, 2048, True), (1120, 1040, 2048, True), (1056, 1072, 6144, True), (1024, 1024, 1088, False)])
+@pytest.mark.parametrize("N1,N2,K,one", [(11264, 3088, 2048, 64), (1120, 1040, 2048, 64), (1056, 1072, 6144, 0), (4128, 1072, 6144, 64), (1024, 1024, 1088, 0),
+                                       (14336, 3088, 2048, 0), (18432, 4112, 2048, 64), (18432, 6144, 4096, 32), (28672, 6144, 3072, 0)])
 def test_pair_of_products(cuda, M, N1, N2, K, one):
-    """A gated product and one with a bias in one launch (one) or two, against float64: bf16 roundings of the result (2^-8 of it) and fp32 sums,
+    """A gated product and one with a bias in one launch (up to ``one`` rows) or two, against float64: bf16 roundings of the result (2^-8 of it) and fp32 sums,
     the gate by approximate exponential and reciprocal (2^-20)."""
     torch.manual_seed(M + N1)
     bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
@@ -340,8 +341,8 @@ def test_pair_of_products(cuda, M, N1, N2, K, one):
     gu = (x1.double() @ w1.double().t()).view(M, N1 // 32, 2, 16)
     want1 = (torch.nn.functional.gelu(gu[:, :, 0], approximate="tanh") * gu[:, :, 1]).reshape(M, -1)
     want2 = x2.double() @ w2.double().t() + b.double()
-    assert (ops.to_fragment_layout_(w1) and ops.to_fragment_layout_(w2)) or not one
-    assert ops.native().gemm_dec2_pair_ok(M, N1, N2, K) == one
+    assert (ops.to_fragment_layout_(w1) and ops.to_fragment_layout_(w2)) or K % 256
+    assert ops.native().gemm_dec2_pair_ok(M, N1, N2, K) == (M <= one)
     y1, y2 = ops.linear_pair(x1, w1, x2, w2, b)
     for y, want in ((y1, want1), (y2, want2)):
         assert ((y.double() - want).abs() <= 2.0 ** -8 * 1.01 * want.abs() + 2e-5).all()
