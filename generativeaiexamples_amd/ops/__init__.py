@@ -205,9 +205,9 @@ def linear_pair(x1, w1, x2, w2, b2):
 
 
 def linear_layer_norm(x, w, bias, residual, ln_w, ln_b, eps):
-    """layer_norm(linear(x, w, bias, residual)). A short question's product leaves most of the chip idle with one workgroup a
+    """layer_norm(linear(x, w, bias, residual)); residual may be None. A short question's product leaves most of the chip idle with one workgroup a
     column tile: its K is cut into slices (gemm_slim.hip) whose sums the norm adds up."""
-    if x.is_cuda and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.bfloat16:
+    if residual is not None and x.is_cuda and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.bfloat16:
         K, N = x.shape[-1], w.shape[0]
         M = x.numel() // K
         psw = decode_operand(w)

@@ -401,6 +401,16 @@ def test_parts_added_by_the_layer_norm(cuda, M, N, K):
         assert torch.equal(y, ops.linear_layer_norm(x, w, bi, r, g, lb, 1e-5))
 
 
+@pytest.mark.parametrize("M", [1, 27, 64, 65, 300, 640, 641])
+def test_linear_layer_norm_without_a_residual(cuda, M):
+    """Nothing to add: the product's norm, as from the two operations."""
+    torch.manual_seed(M)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, b, g = bf(M, 1024), bf(1024, 1024) / 32, bf(1024), bf(1024)
+    want = ops.layer_norm(ops.linear(x, w, b), g, b, 1e-5)
+    assert torch.equal(ops.linear_layer_norm(x, w, b, None, g, b, 1e-5), want)
+
+
 @pytest.mark.parametrize("name,value", [("_SPLITK", False), ("_GEMM_FORCE", 2)])
 def test_linear_layer_norm_under_the_gemm_switches(cuda, monkeypatch, name, value):
     """A forced GEMM kernel, or the decode GEMMs switched off, hold for the product before a layer norm too."""
