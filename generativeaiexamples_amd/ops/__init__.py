@@ -305,10 +305,11 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
         return out
     if x.is_cuda and M > 64 and residual.is_contiguous():
         out = _slabs_norm(x, w, bias, residual, norm_w, None, False, eps) if isinstance(w, torch.Tensor) else None
-        if out is None:
+        if out is None and residual.shape == (*x.shape[:-1], N):
             linear(x, w, bias, residual=residual, out=residual)
             out = rms_norm(residual, norm_w, eps)
-        return out
+        if out is not None:
+            return out
     return rms_norm(linear(x, w, bias), norm_w, eps, residual=residual)
 
 

@@ -411,6 +411,24 @@ def test_linear_layer_norm_without_a_residual(cuda, M):
     assert torch.equal(ops.linear_layer_norm(x, w, b, None, g, b, 1e-5), want)
 
 
+@pytest.mark.parametrize("N,K", [(2048, 2048), (1024, 1024), (2048, 1000), (2056, 2048)])
+def test_residual_of_another_shape(cuda, N, K):
+    """A stream [3, 100, N] beside rows [300, K]: the result has the rows' shape whatever kernels take the product (parts and norm; the
+    product, then the norm; operands off the tile grid), the bits of the product and a norm that adds the residual where that ran."""
+    torch.manual_seed(N + K)
+    x, w = torch.randn(300, K, device=cuda).bfloat16(), (torch.randn(N, K, device=cuda) * K ** -0.5).bfloat16()
+    g, r = torch.randn(N, device=cuda).bfloat16(), torch.randn(3, 100, N, device=cuda).bfloat16()
+    res, want_res = r.clone(), r.clone()
+    want = ops.rms_norm(ops.linear(x, w), g, 1e-5, residual=want_res)
+    y = ops.linear_add_rmsnorm(x, w, res, g, 1e-5)
+    assert y.shape == want.shape == (300, N) and res.shape == r.shape
+    if ops.native().gemm_slabs_parts(300, N, K, False):  # sums in another order: a bf16 step of the product, and of the result
+        assert ((res.float() - want_res.float()).abs() <= 2.0 ** -7 * ((want_res - r).float().abs() + want_res.float().abs()) + 1e-4).all()
+        assert ((y.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm())
+    else:
+        assert torch.equal(res, want_res) and torch.equal(y, want)
+
+
 @pytest.mark.parametrize("name,value", [("_SPLITK", False), ("_GEMM_FORCE", 2)])
 def test_linear_layer_norm_under_the_gemm_switches(cuda, monkeypatch, name, value):
     """A forced GEMM kernel, or the decode GEMMs switched off, hold for the product before a layer norm too."""
