@@ -287,8 +287,8 @@ void gemm(const Tensor& A, const Tensor& B, Tensor& C, const optional<Tensor>& b
 }
 
 // The parts of a product of 65 to 640 rows as slabs, and the norm that adds them: rms (g; res += the product, in place) or
-// layer (g, b; res is only read). False, and nothing launched, where the product has no such plan, an operand is not on 16 bytes
-// or there is no memory for the slabs.
+// layer (g, b; res is only read). False, and nothing launched, where the product has no such plan, an operand is not on 16 bytes or not
+// bf16 of its size, or there is no memory for the slabs.
 bool slabs_plan(int64_t M, int64_t N, int64_t K, bool layer, GaiMidPlan* plan) {
   return layer ? gai_slabs_layernorm_ok(1, N) && gai_gemm_mid_slabs_plan(M, N, K, 8, true, plan)
                : N >= 2048 && gai_gemm_mid_slabs_plan(M, N, K, 16, false, plan);
@@ -296,12 +296,14 @@ bool slabs_plan(int64_t M, int64_t N, int64_t K, bool layer, GaiMidPlan* plan) {
 
 bool linear_slabs_norm(const Tensor& A, const Tensor& W, const optional<Tensor>& bias, Tensor& res, const Tensor& g,
                        const optional<Tensor>& b, bool layer, double eps, Tensor& out, bool bfrag) {
-  for (const Tensor* t : {&A, &W, &g, static_cast<const Tensor*>(&res), static_cast<const Tensor*>(&out)}) check_bf16(*t, "linear_slabs_norm");
-  if (bias) check_bf16(*bias, "bias");
-  if (b) check_bf16(*b, "b");
+  check_bf16(A, "A");
+  check_bf16(W, "W");
+  check_bf16(out, "out");
   const int64_t K = A.size(-1), M = A.numel() / K, N = W.size(0);
-  TORCH_CHECK(W.dim() == 2 && W.size(1) == K && res.numel() == M * N && out.numel() == M * N && g.numel() == N &&
-                  (!bias || bias->numel() == N) && (!b || b->numel() == N), "linear_slabs_norm: sizes");
+  TORCH_CHECK(W.dim() == 2 && W.size(1) == K && out.numel() == M * N, "linear_slabs_norm: sizes");
+  // what the product and the norm make of other vectors and residuals is theirs to say
+  auto fits = [](const Tensor& t, int64_t n) { return t.is_cuda() && t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.numel() == n; };
+  if (!fits(res, M * N) || !fits(g, N) || (bias && !fits(*bias, N)) || (b && !fits(*b, N))) return false;
   GaiMidPlan plan;
   if (!slabs_plan(M, N, K, layer, &plan)) return false;
   uintptr_t at = 0;

@@ -429,6 +429,21 @@ def test_residual_of_another_shape(cuda, N, K):
         assert torch.equal(res, want_res) and torch.equal(y, want)
 
 
+@pytest.mark.parametrize("layer", [False, True])
+def test_longer_bias_before_a_norm(cuda, layer):
+    """A bias padded past the product's columns: the first N are taken, as by the product alone."""
+    torch.manual_seed(2)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, b, r, g = bf(200, 2048), bf(2048, 2048) / 45, bf(2064), bf(200, 2048), bf(2048)
+    assert ops.native().gemm_slabs_parts(200, 2048, 2048, layer) > 1
+    if layer:
+        assert torch.equal(ops.linear_layer_norm(x, w, b, r, g, g, 1e-5), ops.layer_norm(ops.linear(x, w, b, residual=r), g, g, 1e-5))
+    else:
+        res, want_res = r.clone(), r.clone()
+        want = ops.rms_norm(ops.linear(x, w, b), g, 1e-5, residual=want_res)
+        assert torch.equal(ops.linear_add_rmsnorm(x, w, res, g, 1e-5, bias=b), want) and torch.equal(res, want_res)
+
+
 @pytest.mark.parametrize("name,value", [("_SPLITK", False), ("_GEMM_FORCE", 2)])
 def test_linear_layer_norm_under_the_gemm_switches(cuda, monkeypatch, name, value):
     """A forced GEMM kernel, or the decode GEMMs switched off, hold for the product before a layer norm too."""
