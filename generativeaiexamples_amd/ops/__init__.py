@@ -286,6 +286,12 @@ def _vendor_linear(x, w, bias, residual, act, out_dtype, out):
 _SPLITK = os.environ.get("GAI_SPLITK", "1") == "1"
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Contiguous b may share memory with a (which is read until the last workgroup of a product that writes b is done)."""
+    return a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr() and not (
+        a.is_contiguous() and (a.data_ptr() + a.nbytes <= b.data_ptr() or b.data_ptr() + b.nbytes <= a.data_ptr()))
+
+
 def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, norm_w: torch.Tensor, eps: float,
                        bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Tail of a row-parallel projection at TP = 1: ``residual += x @ w^T (+ bias)`` (bf16 rounding
@@ -305,7 +311,7 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
         return out
     if x.is_cuda and M > 64 and residual.is_contiguous():
         out = _slabs_norm(x, w, bias, residual, norm_w, None, False, eps) if isinstance(w, torch.Tensor) else None
-        if out is None and residual.shape == (*x.shape[:-1], N):
+        if out is None and residual.shape == (*x.shape[:-1], N) and not _overlap(x, residual):
             linear(x, w, bias, residual=residual, out=residual)
             out = rms_norm(residual, norm_w, eps)
         if out is not None:

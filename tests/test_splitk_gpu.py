@@ -429,6 +429,18 @@ def test_residual_of_another_shape(cuda, N, K):
         assert torch.equal(res, want_res) and torch.equal(y, want)
 
 
+@pytest.mark.parametrize("M,N", [(70, 1024), (300, 2048), (1500, 1024)])
+def test_rows_that_are_the_stream(cuda, M, N):
+    """The stream itself as the product's rows: no product writes over rows that it still reads."""
+    torch.manual_seed(M)
+    w, g = (torch.randn(N, N, device=cuda) * N ** -0.5).bfloat16(), torch.randn(N, device=cuda).bfloat16()
+    r = torch.randn(M, N, device=cuda).bfloat16()
+    apart, res = r.clone(), r.clone()
+    want = ops.linear_add_rmsnorm(r, w, apart, g, 1e-5)
+    y = ops.linear_add_rmsnorm(res, w, res, g, 1e-5)
+    assert torch.equal(res, apart) and torch.equal(y, want)
+
+
 @pytest.mark.parametrize("layer", [False, True])
 def test_longer_bias_before_a_norm(cuda, layer):
     """A bias padded past the product's columns: the first N are taken, as by the product alone."""
