@@ -45,6 +45,8 @@ void check_f32(const Tensor& t, const char* name) {
   check_dev(t, name);
   TORCH_CHECK(t.scalar_type() == at::kFloat, name, " must be float32");
 }
+// rows as the decode products stage them, by loads of 16 bytes straight into LDS: the same memory, or a copy where it is off 16 bytes
+Tensor rows16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) & 15 ? t.clone() : t; }
 const void* opt_ptr(const optional<Tensor>& t) { return t.has_value() ? t->data_ptr() : nullptr; }
 
 void rmsnorm(const Tensor& x, const Tensor& w, double eps, Tensor& out, const optional<Tensor>& residual_in,
@@ -189,7 +191,7 @@ bool gemm_rope_kv(const Tensor& A, const Tensor& B, const optional<Tensor>& bias
     TORCH_CHECK(tail_cnt->numel() >= (N + 127) / 128, "gemm_rope_kv: tail_cnt too small");
     cnt = tail_cnt->data_ptr<int>();
   }
-  return gai_gemm_splitk_rope_kv(A.data_ptr(), B.data_ptr(), opt_ptr(bias), pos.data_ptr<int>(),
+  return gai_gemm_splitk_rope_kv(rows16(A).data_ptr(), B.data_ptr(), opt_ptr(bias), pos.data_ptr<int>(),
                                  cos_sin.data_ptr<float>(), slots.data_ptr<int>(), q_out.data_ptr(),
                                  k_cache.data_ptr(), v_cache.data_ptr(), M, Hq, Hkv, D, f8, (float)k_scale,
                                  (float)v_scale, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream(), K, cnt) != 0;
@@ -508,7 +510,7 @@ int64_t gemm_qkv_partials(const Tensor& A, const Tensor& W, Tensor& ws, bool psw
   const int N = W.size(0);  // the fragment-shuffled copy keeps the [N, K] shape
   TORCH_CHECK(W.dim() == 2 && W.size(1) == K && W.is_contiguous(), "gemm_qkv_partials: W [N, K]");
   TORCH_CHECK(ws.numel() >= (int64_t)gai_gemm_splitk_ws_bytes(M, N, K) / 4, "gemm_qkv_partials: workspace");
-  return gai_gemm_qkv_partials(A.data_ptr(), W.data_ptr(), M, N, K, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
+  return gai_gemm_qkv_partials(rows16(A).data_ptr(), W.data_ptr(), M, N, K, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
 }
 
 void gemm_partials(const Tensor& A, const Tensor& W, Tensor& ws, bool psw) {
@@ -734,7 +736,7 @@ void gemm_splitk(const Tensor& A, const Tensor& B, Tensor& C, const optional<Ten
     check_bf16(*R, "residual");
     TORCH_CHECK(R->numel() == (int64_t)M * N, "gemm_splitk: residual has wrong size");
   }
-  gai_gemm_splitk(A.data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi,
+  gai_gemm_splitk(rows16(A).data_ptr(), B.data_ptr(), C.data_ptr(), opt_ptr(bias), opt_ptr(R), M, N, K, ldc, (int)epi,
                   f32 ? 1 : 0, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
 }
 
@@ -1216,7 +1218,7 @@ void gemm_splitk_add_rmsnorm(const Tensor& A, const Tensor& B, const optional<Te
   TORCH_CHECK(ws.scalar_type() == at::kFloat && (size_t)ws.numel() * 4 >= gai_gemm_splitk_ws_bytes(M, N, K),
               "gemm_splitk_add_rmsnorm: workspace too small");
   if (bias) check_bf16(*bias, "bias");
-  gai_gemm_splitk_add_rmsnorm(A.data_ptr(), B.data_ptr(), opt_ptr(bias), res.data_ptr(), g.data_ptr(),
+  gai_gemm_splitk_add_rmsnorm(rows16(A).data_ptr(), B.data_ptr(), opt_ptr(bias), res.data_ptr(), g.data_ptr(),
                               out.data_ptr(), M, N, K, (float)eps, ws.data_ptr<float>(), psw ? 1 : 0, cur_stream());
 }
 

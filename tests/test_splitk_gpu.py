@@ -429,6 +429,22 @@ def test_residual_of_another_shape(cuda, N, K):
         assert torch.equal(res, want_res) and torch.equal(y, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 1024, 5632), (9, 1024, 7168), (24, 1024, 1024), (24, 6144, 4096), (3, 18432, 2048), (24, 4096, 14336), (40, 1024, 5632)])
+@pytest.mark.parametrize("off", [1, 4])
+@pytest.mark.parametrize("frag", [False, True])
+def test_rows_off_16_bytes(cuda, M, N, K, off, frag):
+    """Decode products of rows 2 or 8 bytes past a multiple of 16, by every kernel of them: the bits of the same rows on 16 bytes."""
+    torch.manual_seed(M + K)
+    x, w = torch.randn(M, K, device=cuda).bfloat16(), (torch.randn(N, K, device=cuda) * K ** -0.5).bfloat16()
+    odd = torch.empty(M * K + off, device=cuda, dtype=torch.bfloat16)[off:].view(M, K).copy_(x)
+    assert odd.data_ptr() & 15 and odd.is_contiguous() and (not frag or ops.to_fragment_layout_(w))
+    assert torch.equal(ops.linear(odd, w), ops.linear(x, w))
+    if N <= 8192:
+        g, r = torch.randn(N, device=cuda).bfloat16(), torch.randn(M, N, device=cuda).bfloat16()
+        a, b = r.clone(), r.clone()
+        assert torch.equal(ops.linear_add_rmsnorm(odd, w, a, g, 1e-5), ops.linear_add_rmsnorm(x, w, b, g, 1e-5)) and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("M,N", [(70, 1024), (300, 2048), (1500, 1024)])
 def test_rows_that_are_the_stream(cuda, M, N):
     """The stream itself as the product's rows: no product writes over rows that it still reads."""
