@@ -163,13 +163,20 @@ class Partial:
     def __init__(self, slabs: torch.Tensor, bias: Optional[torch.Tensor] = None, operands=None):
         self.slabs, self.bias, self.operands = slabs, bias, operands  # operands: of slabs that another launch still makes
 
+    def made(self) -> "Partial":
+        if self.operands is not None:
+            raise RuntimeError("the slices of this product are still to be made: rotary_half_kv_write(beside=)")
+        return self
+
     def index_select(self, dim: int, idx: torch.Tensor) -> "Partial":
         assert dim == 0
+        self.made()
         return Partial(self.slabs.index_select(1, idx), self.bias)
 
 
 def linear_partial_later(x: torch.Tensor, w: torch.Tensor) -> Optional[Partial]:
-    """linear_partial(x, w) whose slices rotary_half_kv_write(beside=) makes; None where that takes no slices of this product."""
+    """linear_partial(x, w) whose slices rotary_half_kv_write(beside=) makes, without which it is of no use; None where that takes no slices
+    of this product."""
     p = linear_partial(x, w, launch=False) if is_frag(w) and x.is_cuda else None
     return p if isinstance(p, Partial) else None
 
@@ -1899,6 +1906,9 @@ def parallel_add_norm_f32(res, a=None, sa=None, b=None, sb=None, w1=None, w2=Non
     their per-channel scales (fp32 [D]; None: one) - and the next layer's two norms of the new sum, rmsnorm(res) * w1 and
     rmsnorm(res) * w2 in out_dtype (None where no weight is given). One read of the stream, one set of statistics. A branch
     may be a Partial (linear_partial; bf16, at most 2048 channels)."""
+    for x in (a, b):
+        if isinstance(x, Partial):
+            x.made()
     if not res.is_cuda:
         return ref.parallel_add_norm_f32(res, a, sa, b, sb, w1, w2, eps, out_dtype)
     h1, h2 = (torch.empty(res.shape, dtype=out_dtype, device=res.device) if w is not None else None for w in (w1, w2))
@@ -1919,10 +1929,14 @@ def rotary_half_kv_write(q, k, v, positions, slots, k_cache, v_cache, H: int, G:
     projection. beside: a linear_partial_later, whose slices are made too, in the same launch where they can be."""
     if 2 * inv_freq.numel() > DK:
         raise ValueError("rotary_half_kv_write: more rotated channels than a head has")
+    if beside is not None and beside.operands is None:
+        raise RuntimeError("rotary_half_kv_write: the slices beside it are made")
     if not q.is_cuda:
         return ref.rotary_half_kv_write(q, k, v, positions, slots, k_cache, v_cache, H, G, DK, DV, inv_freq, unit_eps)
     q_out = torch.empty(q.shape[0], H * DK, dtype=k_cache.dtype, device=q.device)
     native().rotary_half_kv_write(q, k, v, positions, slots, q_out, k_cache, v_cache, H, G, DK, DV, inv_freq,
                                   -1.0 if unit_eps is None else float(unit_eps),
                                   *((None, None, None) if beside is None else (*beside.operands, beside.slabs)))
+    if beside is not None:
+        beside.operands = None
     return q_out

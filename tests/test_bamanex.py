@@ -748,3 +748,31 @@ def test_rotation_beside_a_product(cuda, T, H, G, D, n, N, K):
             outs.append((q, kc, vc))
         assert all(torch.equal(a, b) for a, b in zip(*outs))
         assert torch.equal(beside.slabs, want.slabs)
+
+
+def test_slices_still_to_be_made():
+    """A product whose slices a later launch makes: nothing reads them before, nothing makes them twice."""
+    t = torch.zeros(2, 3, 8)
+    later, there = ops.Partial(t, None, (t, t)), ops.Partial(t)
+    assert there.index_select(0, torch.tensor([1])).slabs.shape == (2, 1, 8)
+    with pytest.raises(RuntimeError):
+        later.index_select(0, torch.tensor([1]))
+    for a, b in ((later, None), (None, later), (there, later)):
+        with pytest.raises(RuntimeError):
+            ops.parallel_add_norm_f32(torch.zeros(3, 8), a, None, b)
+    with pytest.raises(RuntimeError):
+        ops.rotary_half_kv_write(*[torch.zeros(1, 4)] * 3, torch.zeros(1), torch.zeros(1), None, None, 1, 1, 4, 4,
+                                 torch.zeros(2, dtype=torch.float64), beside=there)
+
+
+@pytest.mark.gpu
+def test_slices_made_beside_the_rotation(cuda):
+    x, w = torch.zeros(3, 5632, device=cuda).bfloat16(), torch.zeros(2048, 5632, device=cuda).bfloat16()
+    assert ops.to_fragment_layout_(w)
+    p, qkv = ops.linear_partial_later(x, w), torch.zeros(3, 3 * 64, device=cuda).bfloat16()
+    at = torch.arange(3, device=cuda, dtype=torch.int32)
+    kc, vc = torch.zeros(1, 1, 16, 64, device=cuda).bfloat16(), torch.zeros(1, 1, 64, 16, device=cuda).bfloat16()
+    freq, q = torch.ones(32, dtype=torch.float64, device=cuda), torch.empty(3, 64, device=cuda).bfloat16()
+    rows = (qkv[:, :64], qkv[:, 64:128], qkv[:, 128:], at, at)
+    ops.rotary_half_kv_write(*rows, kc, vc, 1, 1, 64, 64, freq, beside=p)
+    assert p.made() is p and not p.slabs.any()
