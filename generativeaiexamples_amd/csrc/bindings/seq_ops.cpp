@@ -609,11 +609,12 @@ void rotary_half_kv_write(const Tensor& q, const Tensor& k, const Tensor& v, con
   TORCH_CHECK(inv_freq.is_cuda() && inv_freq.scalar_type() == at::kDouble && inv_freq.is_contiguous() &&
                   2 * inv_freq.numel() <= DK, "rotary_half_kv_write: fp64 frequencies of at most half a head's channels");
   if (A) {  // the K slices of A . W^T (fragment order) into ws, in the same launch where it has them
+    TORCH_CHECK(W && ws, "rotary_half_kv_write: rows of a product beside it without its weight or slices");
     for (const Tensor* t : {&*A, &*W})
       TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->dim() == 2 && t->is_contiguous() &&
                       reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "rotary_half_kv_write: bf16 product beside it, on 16 bytes");
     const int64_t M = A->size(0), K = A->size(1), N = W->size(0), ks = gai_gemm_partials_ks(M, N, K);
-    TORCH_CHECK(W->size(1) == K && ks > 0 && ws && ws->is_cuda() && ws->scalar_type() == at::kFloat && ws->is_contiguous() &&
+    TORCH_CHECK(W->size(1) == K && ks > 0 && ws->is_cuda() && ws->scalar_type() == at::kFloat && ws->is_contiguous() &&
                     ws->numel() >= ks * M * N, "rotary_half_kv_write: slices of the product beside it");
     if (dt == 0 && gai_gemm_partials_rotary(A->data_ptr(), W->data_ptr(), M, N, K, ws->data_ptr<float>(), q.data_ptr(), row_stride(q, "q"),
                                             k.data_ptr(), row_stride(k, "k"), v.data_ptr(), row_stride(v, "v"), i32(positions, "positions"),

@@ -776,3 +776,6 @@ def test_slices_made_beside_the_rotation(cuda):
     rows = (qkv[:, :64], qkv[:, 64:128], qkv[:, 128:], at, at)
     ops.rotary_half_kv_write(*rows, kc, vc, 1, 1, 64, 64, freq, beside=p)
     assert p.made() is p and not p.slabs.any()
+    for w_, ws in ((None, p.slabs), (w, None)):
+        with pytest.raises(RuntimeError, match="without its weight or slices"):
+            ops.native().rotary_half_kv_write(*rows, q, kc, vc, 1, 1, 64, 64, freq, -1.0, x, w_, ws)
