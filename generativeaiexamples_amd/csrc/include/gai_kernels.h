@@ -230,13 +230,9 @@ void gai_ipc_get_handle(void* p, char* handle64);
 void* gai_ipc_open(const char* handle64);
 void gai_ipc_close(void* p);
 
-// the sums of fp32 slabs [KS][M][N] of a product (+ bias), rounded to bf16, with what follows it: res += them, out = rmsnorm(res) * g
-// (N % 8 == 0, N <= 8192); rotation and the write of queries and cached rows (0: not this head size)
+// res += the sums of fp32 slabs [KS][M][N] of a product (+ bias), rounded to bf16; out = rmsnorm(res) * g (N % 8 == 0, N <= 8192)
 void gai_slabs_add_rmsnorm(const float* ws, int KS, const void* bias, void* res, const void* g, void* out, int M, int N, float eps,
                            hipStream_t st);
-int gai_slabs_rope_kv(const float* ws, int KS, const void* bias, const int* pos, const float* cos_sin, const int* slots, void* q_out,
-                      void* k_cache, void* v_cache, int M, int Hq, int Hkv, int D, int kv_fp8, float k_scale, float v_scale,
-                      hipStream_t st);
 
 // gemm_splitk.hip fused decode tail (TP = 1): res = bf16(bf16(A.W^T + bias) + res); out = rmsnorm(res) * g
 int gai_gemm_splitk_fusable_norm(int M, int N, int K);
@@ -323,10 +319,12 @@ void gai_mlstm(const void* q, int ldq, const void* k, int ldk, const void* v, in
 void gai_rotary_kv_write(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const int* positions,
                          const int* slots, void* q_out, void* k_cache, void* v_cache, int T, int H, int G, int DK, int DV,
                          int ROT, float base, int dt_in, int dt, hipStream_t st);
-// rotate-half positions (inv_freq: fp64 [half]), unit RMS norm per head (unit_eps >= 0), cache write
+// gemm_splitk.hip: gai_gemm_partials of a weight in fragment order, and gai_rotary_half_kv_write of T bf16 rows, in one launch; 0: not for
+// these, nothing launched
 int gai_gemm_partials_rotary(const void* A, const void* B, int M, int N, int K, float* ws, const void* q, int ldq, const void* k, int ldk,
                              const void* v, int ldv, const int* positions, const int* slots, void* q_out, void* k_cache, void* v_cache, int T,
                              int H, int G, int DK, int DV, const double* inv_freq, int half, float unit_eps, hipStream_t st);
+// rotate-half positions (inv_freq: fp64 [half]), unit RMS norm per head (unit_eps >= 0), cache write
 void gai_rotary_half_kv_write(const void* q, int ldq, const void* k, int ldk, const void* v, int ldv, const int* positions,
                               const int* slots, void* q_out, void* k_cache, void* v_cache, int T, int H, int G, int DK,
                               int DV, const double* inv_freq, int half, float unit_eps, int dt, hipStream_t st);

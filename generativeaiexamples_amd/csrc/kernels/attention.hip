@@ -775,9 +775,6 @@ typedef __attribute__((address_space(1))) unsigned gu32_t;
 __device__ __forceinline__ void st_sc1(float* p, float v) {
   __hip_atomic_store((gu32_t*)p, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ float ld_sc1(const float* p) {
-  return __uint_as_float(__hip_atomic_load((gu32_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
 // Merge the flash-decoding partials (O, max, sum) of ns splits for one (sequence, q head, dim): groups of
 // kMergeGroup splits, every load of a group issued before its math, running-max rescale between groups. The
 // separate reduce launch and the in-launch merge (write-through partials read with sc1 loads) take the same steps,

@@ -558,7 +558,10 @@ int stream_ks(int N, int K) {
 // gemm_slim.hip. Product and the hybrid norm that adds the slices, 24 rows, fragment order | row-major, us: 2048 x 4608 16.0 | 19.8 -> 13.3 |
 // 14.2, 2048 x 5632 16.4 | 20.2 -> 13.9 | 15.1, 1024 x 5632 13.6 | 15.2 -> 11.8 | 13.2, one row of that 11.1 | 12.7 -> 9.7 | 11.3. Where they
 // fit one round the stream is faster: 2048 x 6144 in eight 13.4 (13.9 in two), 1024 x 8192 in sixteen 11.9 (13.2). Past 32 rows the
-// rotations beside them (two a row) take the CUs that the slices would.
+// rotations beside them (two a row) take the CUs that the slices would. Few columns gain as well, though their slices are a few dozen workgroups
+// (the stream's were many slabs of little each): at 695 shapes that the rule takes, N 64 to 2048, K 4608 to 22528, 1 to 32 rows, weights
+// from HBM, product and sum are 0.72 of the stream's on average, with a rms norm 0.71, with the hybrid norm 0.57, none above 0.95. 24 rows
+// with the rms norm, us: 256 x 8704 13.6 -> 9.2 (48 workgroups), 512 x 4608 11.0 -> 8.8, 768 x 5632 10.8 -> 9.2; 16 of 1280 x 8192 12.9 -> 9.8 (three slices, 16).
 int slim_few(int M, int N, int K) {
   if (asked_variant() || use_legacy(N, K) || gai_gemm_slim_nf(M, N, K, false) || gai_gemm_dec2_partials_ks(M, N, K)) return 0;
   return (N + 63) / 64 * stream_ks(N, K) > 256 ? gai_gemm_slim_few_ks(M, N, K) : 0;
@@ -914,9 +917,8 @@ bool launch_rope_tail(const void* A, const void* B, int M, int N, int K, float* 
   return false;
 }
 
-}  // namespace
-
-int gai_slabs_rope_kv(const float* ws, int KS, const void* bias, const int* pos, const float* cos_sin, const int* slots, void* q_out,
+// rotation, queries and cached rows of the slabs' sums; 0: not this head size
+int slabs_rope_kv(const float* ws, int KS, const void* bias, const int* pos, const float* cos_sin, const int* slots, void* q_out,
                       void* k_cache, void* v_cache, int M, int Hq, int Hkv, int D, int kv_fp8, float k_scale, float v_scale,
                       hipStream_t st) {
   const int N = (Hq + 2 * Hkv) * D;
@@ -952,6 +954,8 @@ int gai_slabs_rope_kv(const float* ws, int KS, const void* bias, const int* pos,
   return 0;
 }
 
+}  // namespace
+
 int gai_gemm_splitk_rope_kv(const void* A, const void* B, const void* bias, const int* pos, const float* cos_sin,
                             const int* slots, void* q_out, void* k_cache, void* v_cache, int M, int Hq, int Hkv,
                             int D, int kv_fp8, float k_scale, float v_scale, float* ws, int psw, hipStream_t st,
@@ -973,7 +977,7 @@ int gai_gemm_splitk_rope_kv(const void* A, const void* B, const void* bias, cons
     gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw);
   else
     launch_partials(A, B, M, N, K, KS, ws, psw, st);
-  return gai_slabs_rope_kv(ws, KS, bias, pos, cos_sin, slots, q_out, k_cache, v_cache, M, Hq, Hkv, D, kv_fp8, k_scale, v_scale, st);
+  return slabs_rope_kv(ws, KS, bias, pos, cos_sin, slots, q_out, k_cache, v_cache, M, Hq, Hkv, D, kv_fp8, k_scale, v_scale, st);
 }
 
 int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, float* ws, int psw, hipStream_t st) {
@@ -981,8 +985,8 @@ int gai_gemm_qkv_partials(const void* A, const void* B, int M, int N, int K, flo
   if (gai_gemm_dec2_ok(M, N, K, EPI_NONE)) return 0;  // single-pass kernel owns it
   const int ks2 = gai_gemm_dec2_partials_ks(M, N, K);
   const int KS = ks2 ? ks2 : gai_gemm_splitk_ks(M, N, K);
-  // up to 16 slabs: the TP = 8 shard of Llama-3-70B (N 1280, K 8192) takes 16 K-slices to reach 192 workgroups;
-  // GAI_QKV_FOLD_MAXKS = 8 restores the round-5 limit (A/B)
+  // up to 16 slabs: 64 rows of the TP = 8 shard of Llama-3-70B (N 1280, K 8192) take 16 K-slices (up to 32 rows three: slim_few);
+  // GAI_QKV_FOLD_MAXKS lowers the limit
   static const int max_ks = getenv("GAI_QKV_FOLD_MAXKS") ? atoi(getenv("GAI_QKV_FOLD_MAXKS")) : 16;
   if (KS < 2 || KS > max_ks) return 0;
   if (ks2)
@@ -1009,7 +1013,6 @@ void gai_gemm_partials(const void* A, const void* B, int M, int N, int K, float*
   else if (!gai_gemm_dec2_partials(A, B, M, N, K, ws, st, psw)) launch_partials(A, B, M, N, K, ks, ws, psw, st);
 }
 
-// gai_gemm_partials of a weight in fragment order beside gai_rotary_half_kv_write of T bf16 rows; 0: not these, nothing launched
 int gai_gemm_partials_rotary(const void* A, const void* B, int M, int N, int K, float* ws, const void* q, int ldq, const void* k, int ldk,
                              const void* v, int ldv, const int* positions, const int* slots, void* q_out, void* k_cache, void* v_cache, int T,
                              int H, int G, int DK, int DV, const double* inv_freq, int half, float unit_eps, hipStream_t st) {
