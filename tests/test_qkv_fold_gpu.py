@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,K", [(7, 32, 8, 4096), (64, 32, 8, 4096),
-                                         (64, 8, 1, 8192)])  # last: a Llama-3-70B TP = 8 shard, 16 K-slices
+                                         (64, 8, 1, 8192), (7, 8, 1, 8192), (32, 8, 1, 8192)])  # a Llama-3-70B TP = 8 shard: 64 rows
+# in 16 K slices, up to 32 in three of unequal length
 @pytest.mark.parametrize("psw", [True, False])
 def test_qkv_fold_matches_unfused_and_reference(cuda, B, Hq, Hkv, K, psw):
     torch.manual_seed(B + 100 * psw + K)

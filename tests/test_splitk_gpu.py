@@ -429,6 +429,41 @@ def test_residual_of_another_shape(cuda, N, K):
         assert torch.equal(res, want_res) and torch.equal(y, want)
 
 
+@pytest.mark.parametrize("M,N,K,ks", [(1, 1024, 5632, 2), (9, 1024, 7168, 3), (32, 512, 17408, 6), (17, 256, 8704, 3), (16, 1280, 8192, 3), (5, 144, 18944, 7)])
+def test_deep_products_in_uneven_slices(cuda, M, N, K, ks):
+    """Up to 32 rows of a deep product in slices that differ by 512, the first ones longer, under every epilogue that adds them and before a
+    rms norm, against float64: a bf16 rounding of each result (2^-8 of it; the activations as elsewhere by approximate functions, 2^-10 more)
+    and fp32 sums of K products of unit normals and weights of K^-1/2."""
+    torch.manual_seed(M + K)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, b, r, g = bf(M, K), bf(N, K) * K ** -0.5, bf(N), bf(M, N), bf(N)
+    assert ops.native().gemm_partials_ks(M, N, K) == ks and (K // 512) % ks  # unequal
+    wf = w.clone()
+    assert ops.to_fragment_layout_(wf)
+    p = x.double() @ w.double().t()
+    gelu = torch.nn.functional.gelu
+    cases = [(dict(out_dtype=torch.float32), p, 0), (dict(), p, 2.0 ** -8), (dict(bias=b), p + b.double(), 2.0 ** -8),
+             (dict(bias=b, act="gelu"), gelu(p + b.double()), 2.0 ** -8 + 2.0 ** -10), (dict(bias=b, act="relu"), (p + b.double()).relu(), 2.0 ** -8)]
+    if N % 32 == 0:
+        gu = p.view(M, N // 32, 2, 16)
+        cases.append((dict(act="swiglu"), (torch.nn.functional.silu(gu[:, :, 0]) * gu[:, :, 1]).reshape(M, -1), 2.0 ** -8 + 2.0 ** -10))
+    sums = 2.0 ** -18 * K ** 0.5
+    for kw, want, rel in cases:
+        y = ops.linear(x, w, **kw)
+        assert ((y.double() - want).abs() <= rel * want.abs() + sums).all()
+        assert torch.equal(y, ops.linear(x, wf, **kw))
+    # the product is rounded before the residual is added
+    v, off = p + r.double(), 2.0 ** -8 * 1.01 * (p.abs() + (p + r.double()).abs()) + sums
+    assert ((ops.linear(x, w, residual=r).double() - v).abs() <= off).all()
+    inv = torch.rsqrt(v.square().mean(-1, keepdim=True) + 1e-5)
+    want = v * inv * g.double()
+    for wt in (w, wf):
+        res = r.clone()
+        y = ops.linear_add_rmsnorm(x, wt, res, g, 1e-5)
+        assert ((res.double() - v).abs() <= off).all()
+        assert ((y.double() - want).abs() <= 1.01 * off * inv * g.double().abs() + (2.0 ** -8 + 2.0 ** -8) * want.abs()).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 1024, 5632), (9, 1024, 7168), (24, 1024, 1024), (24, 6144, 4096), (3, 18432, 2048), (24, 4096, 14336), (40, 1024, 5632)])
 @pytest.mark.parametrize("off", [1, 4])
 @pytest.mark.parametrize("frag", [False, True])
