@@ -794,7 +794,13 @@ __global__ __launch_bounds__(1024) void splitk_add_rmsnorm_w4_kernel(const float
 
 }  // namespace
 
+// A small shallow product is done in one launch with all of K (gemm_slim.hip) before its slices would be written: with the norm that adds the
+// residual as a launch of its own, us, slices and norm -> product and norm, 1 row | 32 | 64, fragment order: 1024 x 1024 6.2 -> 5.5 | 7.5 -> 6.1 | 8.8 -> 7.0,
+// 512 x 1024 6.3 -> 5.0 | 7.2 -> 5.5 | 8.4 -> 6.4, 2048 x 1024 6.6 -> 6.7 | 7.8 -> 7.7 | 9.2 -> 8.5 (row-major 8.1 -> 7.6 | 9.3 -> 8.5 | 10.8 -> 9.4), 1536 x 1536
+// 7.0 -> 6.5 | 8.0 -> 7.9 | 9.7 -> 8.9. Past that the slices are ahead: 2560 x 1024 6.9 | 8.1 | 9.6 against 7.9 | 8.8 | 9.9, 2048 x 1536 6.9 | 8.3 | 9.8
+// against 7.5 | 8.5 | 9.8, 1024 x 2048 within 5 % either way, 2048 x 2048 6.9 | 8.1 | 9.8 against 7.6 | 9.4 | 11.2.
 int gai_gemm_splitk_fusable_norm(int M, int N, int K) {
+  if (K <= 1536 && (long long)N * K <= 1536 * 1536 && gai_gemm_slim_nf(M, N, K, false)) return 0;
   return M >= 1 && M <= 64 && N % 8 == 0 && N <= 256 * 8 * 4 && gai_gemm_splitk_ks(M, N, K) > 1;
 }
 

@@ -429,6 +429,25 @@ def test_residual_of_another_shape(cuda, N, K):
         assert torch.equal(res, want_res) and torch.equal(y, want)
 
 
+@pytest.mark.parametrize("M", [1, 17, 64])
+@pytest.mark.parametrize("N,K,slices", [(1024, 1024, False), (2048, 1024, False), (1536, 1536, False), (16, 1536, False), (2320, 1024, True), (1552, 1536, True),
+                                        (1024, 2048, True), (1024, 1152, True)])
+def test_small_products_before_a_norm(cuda, M, N, K, slices):
+    """Both sides of the line below which the product is one launch and the norm another: there, the bits of those two."""
+    torch.manual_seed(M + N)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, r, g = bf(M, K), bf(N, K) * K ** -0.5, bf(M, N), bf(N)
+    assert ops.native().gemm_splitk_fusable_norm(M, N, K) == slices
+    res, want_res = r.clone(), r.clone()
+    want = ops.rms_norm(ops.linear(x, w), g, 1e-5, residual=want_res)
+    y = ops.linear_add_rmsnorm(x, w, res, g, 1e-5)
+    if not slices:
+        assert torch.equal(res, want_res) and torch.equal(y, want)
+    # sums in another order: the product, its sum with the residual and the result each a bf16 step apart
+    assert ((res.float() - want_res.float()).abs() <= 2.0 ** -7 * ((want_res - r).float().abs() + want_res.float().abs()) + 1e-4).all()
+    assert (y.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
 @pytest.mark.parametrize("M,N,K,ks", [(1, 1024, 5632, 2), (9, 1024, 7168, 3), (32, 512, 17408, 6), (17, 256, 8704, 3), (16, 1280, 8192, 3), (5, 144, 18944, 7)])
 def test_deep_products_in_uneven_slices(cuda, M, N, K, ks):
     """Up to 32 rows of a deep product in slices that differ by 512, the first ones longer, under every epilogue that adds them and before a
