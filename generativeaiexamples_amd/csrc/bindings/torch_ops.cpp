@@ -1263,6 +1263,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_dec2_pair", &gemm_dec2_pair);
   m.def("gemm_dec2_pair_ok", [](int64_t M, int64_t N1, int64_t N2, int64_t K) { return gai_gemm_dec2_pair_ok(M, N1, N2, K) != 0; });
   m.def("linear_slabs_norm", &linear_slabs_norm);
+  m.def("gemm_residual_apart", [](int64_t M, int64_t N, int64_t K) { return gai_gemm_residual_apart(M, N, K); });
   m.def("gemm_slabs_parts", [](int64_t M, int64_t N, int64_t K, bool layer) {
     GaiMidPlan plan;
     return slabs_plan(M, N, K, layer, &plan) ? plan.parts : 0;

@@ -29,3 +29,5 @@ int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* b
 bool gai_gemm_mid_slabs_plan(int M, int N, int K, int most, bool layer, GaiMidPlan* plan);
 void gai_gemm_mid_slabs(const void* A, const void* B, int M, int N, int K, const GaiMidPlan& plan, float* ws, hipStream_t st,
                         int bfrag);
+// a residual in front of a norm is faster added by the norm than by the product's epilogue
+bool gai_gemm_residual_apart(int M, int N, int K);

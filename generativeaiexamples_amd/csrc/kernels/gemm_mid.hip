@@ -583,6 +583,19 @@ bool gai_gemm_mid_slabs_plan(int M, int N, int K, int most, bool layer, GaiMidPl
   return now < kSlabShare * then && then - now > f.least;
 }
 
+// res += product; rms norm: in the product's epilogue, or (apart) by the norm, which then reads the product and the stream and writes the stream
+// as well, at the copy's 4.8 TB/s. The kernels of 128 x 128 tiles ask for the residual when their sums are done, 8 - 10 us in all, and a tile of the
+// others hides it or has enough rounds to. Both timed at 2286 products of 65 to 14643 rows (N 512 to 8192, K 512 to 14336, both layouts): apart
+// at 420 of them, where the epilogue took 1.21 of the time on average and nowhere less than 0.99 (2100 rows 2048 x 4096 63.8 | 70.4 us, 4100 x 1024 x 1024
+// 26.1 | 36.5); at the others it takes 0.954, and 10 % more at worst (641 x 1024 x 8192).
+bool gai_gemm_residual_apart(int M, int N, int K) {
+  auto product = [&](int epi) {
+    GaiMidPlan p;
+    return gai_gemm_mid_plan(nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, N, epi, 0, 0, 1, &p) ? p.cost : other_cost(M, N, K, epi);
+  };
+  return product(EPI_RESIDUAL) > product(EPI_NONE) + (double)M * N * 4 / 4.8e6 + 1.0;
+}
+
 void gai_gemm_mid_slabs(const void* A, const void* B, int M, int N, int K, const GaiMidPlan& p, float* ws, hipStream_t st, int bfrag) {
 #define GAI_MID_SLABS(MT, NG)   \
   if (p.mt == MT && p.ng == NG) \

@@ -293,6 +293,15 @@ def _vendor_linear(x, w, bias, residual, act, out_dtype, out):
 _SPLITK = os.environ.get("GAI_SPLITK", "1") == "1"
 
 
+def _residual_in_product(x, w, M: int, N: int, K: int) -> bool:
+    """A product of more than 64 rows in front of a rms norm adds the residual itself. 8-bit products: up to 1024 rows of at least 4096
+    columns (641 x 4096 x 1024 26.3 us with the norm adding it, 25.2 so; 2100 rows of it 46.0 | 49.4, 14643 x 4096 x 4096 392 | 441, 1300 x 1024 x 4096 36.8
+    | 39.9). The library's products have no epilogue."""
+    if isinstance(w, Fp8Weight):
+        return N >= 4096 and M <= 1024
+    return x.dtype == w.dtype == torch.bfloat16 and K % 64 == 0 and N % 16 == 0 and not native().gemm_residual_apart(M, N, K)
+
+
 def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Contiguous b may share memory with a (which is read until the last workgroup of a product that writes b is done)."""
     return a.untyped_storage().data_ptr() == b.untyped_storage().data_ptr() and not (
@@ -304,7 +313,7 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
     """Tail of a row-parallel projection at TP = 1: ``residual += x @ w^T (+ bias)`` (bf16 rounding
     as the unfused pair) and return ``rmsnorm(residual) * norm_w``. For decode-sized M, and up to a few hundred rows,
     the parts of K are reduced, added and normalised in ONE kernel (no separate reduce / norm launches); longer prompts
-    add the residual in the product's epilogue."""
+    add the residual in the product's epilogue or in the norm."""
     K = x.shape[-1]
     M, N = x.numel() // K, w.shape[0]
     if (x.is_cuda and not isinstance(w, Fp8Weight) and _SPLITK and _GEMM_FORCE == 0 and M <= 64
@@ -318,7 +327,7 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
         return out
     if x.is_cuda and M > 64 and residual.is_contiguous():
         out = _slabs_norm(x, w, bias, residual, norm_w, None, False, eps) if isinstance(w, torch.Tensor) else None
-        if out is None and residual.shape == (*x.shape[:-1], N) and not _overlap(x, residual):
+        if out is None and residual.shape == (*x.shape[:-1], N) and not _overlap(x, residual) and _residual_in_product(x, w, M, N, K):
             linear(x, w, bias, residual=residual, out=residual)
             out = rms_norm(residual, norm_w, eps)
         if out is not None:

@@ -411,6 +411,24 @@ def test_linear_layer_norm_without_a_residual(cuda, M):
     assert torch.equal(ops.linear_layer_norm(x, w, b, None, g, b, 1e-5), want)
 
 
+@pytest.mark.parametrize("M,N,K,apart", [(2100, 1024, 1024, True), (4100, 512, 1024, True), (1300, 4096, 1024, True), (128, 1024, 1024, True), (8192, 1024, 1024, False),
+                                         (2048, 4096, 1024, False), (641, 2048, 2048, False)])
+def test_residual_in_the_product_or_the_norm(cuda, M, N, K, apart):
+    """Both sides of the line between a residual added by the product's epilogue and by the norm (apart: the bits of the two operations)."""
+    torch.manual_seed(M + N)
+    bf = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)  # noqa: E731
+    x, w, r, g = bf(M, K), bf(N, K) * K ** -0.5, bf(M, N), bf(N)
+    assert ops.native().gemm_residual_apart(M, N, K) == apart and ops._residual_in_product(x, w, M, N, K) != apart
+    res, want_res = r.clone(), r.clone()
+    want = ops.rms_norm(ops.linear(x, w), g, 1e-5, residual=want_res)
+    y = ops.linear_add_rmsnorm(x, w, res, g, 1e-5)
+    if apart:
+        assert torch.equal(res, want_res) and torch.equal(y, want)
+    # the product, its sum with the residual and the result may each be a bf16 step apart
+    assert ((res.float() - want_res.float()).abs() <= 2.0 ** -7 * ((want_res - r).float().abs() + want_res.float().abs()) + 1e-4).all()
+    assert (y.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
 @pytest.mark.parametrize("N,K", [(2048, 2048), (1024, 1024), (2048, 1000), (2056, 2048)])
 def test_residual_of_another_shape(cuda, N, K):
     """A stream [3, 100, N] beside rows [300, K]: the result has the rows' shape whatever kernels take the product (parts and norm; the
