@@ -525,8 +525,8 @@ int gai_gemm_mid_tail(const void* A, const void* B, const void* C, const void* b
 // The model: 3336 timings of 200 products (65 to 640 rows, N 2048 to 8192, K 2048 to 14336), nine in ten within 13 %, and for the choice
 // product and norm together, here and as they would run without slabs (the plan of the product that adds its own residual, or the kernels
 // past this one), fitted to both ways of 2588 products (N 2048 to 8192 before a rms norm, 256 to 2048 before a layer norm, both layouts),
-// nine in ten within 10 %. A layer norm's wave reads a row's slabs by itself, so wide rows in many parts cost it most. The rule takes 2262
-// of these: before a rms norm 0.85 of the time on average, before a layer norm 0.80; the slowest, us: 160 rows 5120 x 14336 53.5 | 54.3 (row-major
+// nine in ten within 10 %. A layer norm's wave reads a row's slabs by itself, so wide rows in many parts cost it most. The rule takes 2265
+// of these: before a rms norm 0.84 of the time on average, before a layer norm 0.79; the slowest, us: 160 rows 5120 x 14336 53.5 | 54.3 (row-major
 // 55.2 | 56.9), 8192 x 14336 89.8 | 70.7 (72.9 | 74.3); of 700 others that it takes six are more than 1 % slower in fragment order, 417 x 1536 x 1280
 // before a layer norm 13.1 | 13.8 the most, and 142 x 7328 x 12288 60.6 | 62.8 (62.5 | 69.0). Without the comparison 385 x 2048 x 1024 took 13.1 instead of 12.3, before a layer norm 385 x 1536 x
 // 768 12.5 instead of 11.2, 65 x 2048 x 3072 18.3 instead of 17.1 and 212 x 1088 x 1920 15.8 instead of 14.5; past 512 rows two short parts
